@@ -17,7 +17,7 @@ from typing import Optional, Tuple
 
 import torch
 
-from . import _lib
+from . import _ext, _lib
 
 _DT = {torch.float32: _lib.VIG_F32, torch.bfloat16: _lib.VIG_BF16}
 
@@ -61,6 +61,11 @@ def gla_bidir_forward(q, k, v, g_fwd, g_bwd=None, scale: float = -1, out_scale: 
     have a channel whose gates sum below about -8 over 64 tokens.
     Differentiable: when autograd is recording and an input requires grad, the backward runs vig_gla_bidir_bwd.
     """
+    calls = _ext.calls() if out is None else None
+    if calls is not None:  # one native call for contiguous GPU tensors of a built shape; None: not of that kind
+        o = calls.gla(q, k, v, g_fwd, g_bwd, scale, out_scale, 2 if exact else 1 if strong_gates else 0)
+        if o is not None:
+            return o
     tensors = (q, k, v, g_fwd) + ((g_bwd,) if g_bwd is not None else ())
     if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
         if out is not None:
@@ -258,6 +263,17 @@ def _split_bid_gates(q, g):
     return g[:B], g[B:]
 
 
+def _bid_gla(q, k, v, g, scale):
+    """The bidirectional op on packed gates [2B,H,L,Dk], directions averaged."""
+    calls = _ext.calls()
+    if calls is not None:
+        o = calls.bid_gla(q, k, v, g, scale, 0.5)
+        if o is not None:
+            return o
+    gf, gb = _split_bid_gates(q, g)
+    return gla_bidir_forward(q, k, v, gf, gb, scale, 0.5)
+
+
 def gla_causal_state_forward(q, k, v, g, initial_state=None, output_final_state: bool = False, scale: float = -1,
                              exact: bool = False):
     """The causal op with a state carried in and / or out: (o, final_state or None).
@@ -364,8 +380,7 @@ def batch_bid_fused_chunk_gla(q, k, v, g, scale: int = -1, initial_state=None, o
     """q,k,v [B,H,L,D]; g [2B,H,L,Dk] = cat(fwd gates, bwd gates), both in natural order; o=(o_f+o_b)/2."""
     if initial_state is not None or output_final_state:
         raise NotImplementedError("bidirectional GLA takes no initial/final state")
-    gf, gb = _split_bid_gates(q, g)
-    return gla_bidir_forward(q, k, v, gf, gb, scale, 0.5), None
+    return _bid_gla(q, k, v, g, scale), None
 
 
 def bid_fused_recurrent_gla(q, k, v, gk=None, gv=None, scale: int = -1, initial_state=None,
@@ -380,8 +395,7 @@ def bid_fused_recurrent_gla(q, k, v, gk=None, gv=None, scale: int = -1, initial_
         raise NotImplementedError("causal=False on the merged op is unused by ViG and not built")
     if gk is None:
         gk = torch.zeros((2 * q.shape[0],) + tuple(q.shape[1:]), dtype=q.dtype, device=q.device)
-    gf, gb = _split_bid_gates(q, gk)
-    return gla_bidir_forward(q, k, v, gf, gb, scale, 0.5), None
+    return _bid_gla(q, k, v, gk, scale), None
 
 
 # ---------------------------------------------------------------------------
@@ -560,11 +574,16 @@ def gla_bidir_locality_gate(q, k, v, g_fwd, g_bwd, weight: torch.Tensor, hw, sca
     Shapes the one-kernel form is built for (bf16, Dk in {32,64}, Dv=64, L=h*w<=256) never write the ungated
     output to memory; every other shape makes the two calls.  Inference only.
     """
+    h, w = hw
+    calls = _ext.calls()
+    if calls is not None:
+        y = calls.gla_gate(q, k, v, g_fwd, g_bwd, weight, h, w, scale, out_scale)
+        if y is not None:
+            return y
     lib = _lib.load()
     _check_cuda(q, k, v, g_fwd, g_bwd, weight)
     B, H, L, Dk = q.shape
     Dv = v.shape[-1]
-    h, w = hw
     if L != h * w:
         raise ValueError("L must equal h*w")
     if scale == -1 or scale is None:
