@@ -22,7 +22,7 @@ def test_calls_match_ctypes(monkeypatch, B, H, L, Dk, Dv, dtype):
     w = make_locality_weight(H * Dv, seed=7).cuda()
 
     def everything():
-        out = [vig_amd.gla_bidir_locality_gate(q, k, v, gf, gb, w, (1, L))]
+        out = [vig_amd.gla_bidir_locality_gate(q, k, v, gf, gb, w, (L, 1))]
         for f, x in ((lambda *a: vig_amd.batch_bid_fused_chunk_gla(*a)[0], (q, k, v, g)), (ops.gla_bidir_forward, (q, k, v, gf, gb)),
                      (ops.gla_bidir_forward, (q, k, v, gf)), (lambda *a: ops.gla_bidir_forward(*a, exact=True), (q, k, v, gf, gb))):
             leaves = [t.clone().requires_grad_() for t in x]

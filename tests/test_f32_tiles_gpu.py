@@ -1,0 +1,40 @@
+"""fp32 tensors on the matrix cores (gla_f32.hip) against the fp64 oracle, and no less precise than the token-recurrent
+fp32 kernel on the same inputs: edges of tiles and segments, one or two directions, gates that leave the tile form's range."""
+import numpy as np
+import pytest
+import torch
+
+import vig_amd
+from vig_amd.synthetic import make_gla_inputs
+
+from .util import announce, f64, oracle_bidir
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(1, 1, 1, 64), (2, 2, 32, 32), (1, 2, 33, 64), (2, 3, 224, 64), (1, 2, 225, 32), (1, 2, 449, 64), (1, 1, 1100, 32)]
+
+
+@pytest.mark.parametrize("gate_scale", [1 / 16, 1.0, 40.0])  # in range; some tiles beyond it; every tile beyond it
+@pytest.mark.parametrize("B,H,L,Dk", SHAPES)
+def test_forward(B, H, L, Dk, gate_scale):
+    announce(f"fp32 forward on the matrix cores B{B} H{H} L={L} Dk={Dk} gates x {gate_scale}")
+    t = make_gla_inputs(B, H, L, Dk, 64, seed=900 + L, dtype=torch.float32, gate_scale=gate_scale)
+    for args in (t, (*t[:4], None)):
+        want = oracle_bidir(*args)
+        x = [a.cuda() if a is not None else None for a in args]
+        err = lambda o: np.linalg.norm(f64(o) - want) / np.linalg.norm(want)
+        mine, serial = err(vig_amd.gla_bidir_forward(*x)), err(vig_amd.gla_bidir_forward(*x, exact=True))
+        print(f"  relative error {mine:.2e}, token-recurrent {serial:.2e}", flush=True)
+        assert mine <= max(2 * serial, 3e-7)
+
+
+def test_forward_magnitudes_and_infinite_gates():
+    """Inputs beyond the tile form's magnitude bound, and gates of -inf, take the serial form."""
+    announce("fp32 forward, large magnitudes and gates of -inf")
+    q, k, v, gf, gb = make_gla_inputs(1, 2, 300, 64, 64, seed=5, dtype=torch.float32)
+    q[0, 0, 3] *= 1e14
+    gf[0, 1, 40:60:7] = -float("inf")
+    want = oracle_bidir(q, k, v, gf, gb)
+    got = f64(vig_amd.gla_bidir_forward(*(t.cuda() for t in (q, k, v, gf, gb))))
+    for h in range(2):
+        assert np.abs(got[0, h] - want[0, h]).max() <= 1e-5 * np.abs(want[0, h]).max()

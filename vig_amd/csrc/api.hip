@@ -123,6 +123,7 @@ static size_t padded_workspace(int B, int H, int L) {
 static size_t fwd_workspace_exact(int B, int H, int L, int Dk, int Dv, int io_dtype, int gate_dtype, bool bidir) {
   if (io_dtype == VIG_BF16 && gate_dtype == VIG_BF16 && (Dk == 64 || Dk == 32) && Dv == 64)
     return vig::gla_mfma_workspace(B, H, L, Dk, Dv);
+  if (io_dtype == VIG_F32 && gate_dtype == VIG_F32) return vig::gla_f32_workspace(B, H, L, Dk, Dv);
   if (padded_shape(L, Dk, Dv, io_dtype, gate_dtype, bidir)) return padded_workspace(B, H, L);
   return bidir ? vig::gla_recurrent_workspace(B, H, L, Dv, io_dtype) : 0;
 }
@@ -143,6 +144,9 @@ size_t vig_gla_bidir_fwd_workspace(int B, int H, int L, int Dk, int Dv, int io_d
   }
   if (io_dtype == VIG_BF16) {
     const size_t m = vig::gla_mfma_workspace(B, H, L, Dk, Dv);
+    if (m > need) need = m;
+  } else {
+    const size_t m = vig::gla_f32_workspace(B, H, L, Dk, Dv);
     if (m > need) need = m;
   }
   return need;
@@ -184,6 +188,11 @@ static int gla_bidir_fwd(const void* q, const void* k, const void* v, const void
     e = vig::launch_gla_mfma(b);
     if (e) return e;
     return vig::launch_pad_channels(op, o, rows, 64, 32, st);
+  }
+  // fp32 on the matrix cores; a caller that brought no room for a long sequence's states gets the recurrent kernel
+  if (vig::gla_f32_supported(a)) {
+    const size_t n = vig::gla_f32_workspace(B, H, L, Dk, Dv);
+    if (n == 0 || (workspace && workspace_bytes >= n)) return vig::launch_gla_f32(a);
   }
   const size_t need = g_bwd ? vig::gla_recurrent_workspace(B, H, L, Dv, io_dtype) : 0;
   if (need > workspace_bytes) return VIG_ENOSPC;
@@ -310,7 +319,8 @@ int vig_gla_bidir_fwd_noalloc(const void* q, const void* k, const void* v, const
   if (B <= 0 || H <= 0 || L <= 0) return VIG_EINVAL;
   if (!dtype_ok(io_dtype) || !dtype_ok(gate_dtype)) return VIG_ENOTSUP;
   // what the dispatched path of vig_gla_bidir_fwd needs; shapes whose need exceeds the array are refused, not shrunk
-  const size_t need = fwd_workspace_exact(B, H, L, Dk, Dv, io_dtype, gate_dtype, g_bwd != nullptr);
+  size_t need = fwd_workspace_exact(B, H, L, Dk, Dv, io_dtype, gate_dtype, g_bwd != nullptr);
+  if (io_dtype == VIG_F32 && need > kScratchBytes) need = 0;  // (fp32 tensors: the recurrent kernel keeps its state in registers)
   if (need > kScratchBytes) return VIG_ENOSPC;
   void* ws = nullptr;
   if (need > 0) {

@@ -1003,6 +1003,12 @@ __global__ __launch_bounds__(256) void gla_segment_scan_kernel(float* state_ws, 
   }
 }
 
+int launch_gla_segment_scan(float* slots, int nseq, int nseg, int ndir, int ng, hipStream_t stream) {
+  hipLaunchKernelGGL(gla_segment_scan_kernel, dim3(64 * 64 / 256, nseq * ndir), dim3(256), 0, stream, slots, nseq, nseg, ndir,
+                     ng, (const float*)nullptr, (float*)nullptr, (float*)nullptr);
+  return hipGetLastError() == hipSuccess ? 0 : -5;
+}
+
 // tiles: the segments of the tile-pair output pass (whole 32-token tiles) instead of this kernel's own
 static Geometry make_geometry(int nseq, int L, bool tiles = false) {
   Geometry g{};

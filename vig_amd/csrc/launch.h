@@ -56,6 +56,16 @@ inline int gla_tile_segment_tiles(int L) { return ((L + gla_tile_segments(L) - 1
 // segment| (one per block of the scan), for consumers that read the states as fp16.
 constexpr int kGlaScanMaxima = 16;
 
+// fp32 tensors and gates on the matrix cores (operands in three bf16 pieces): segments of up to seven 32-token tiles, as
+// the tile-pair kernel cuts them.
+inline int gla_f32_segments(int L) { return gla_tile_segments(L); }
+inline int gla_f32_segment_tiles(int L) { return gla_tile_segment_tiles(L); }
+bool gla_f32_supported(const GlaArgs& a);
+size_t gla_f32_workspace(int B, int H, int L, int Dk, int Dv);
+int launch_gla_f32(const GlaArgs& a);
+// chains the slots of a state pass in place (gla_segment_scan_kernel, no state in or out)
+int launch_gla_segment_scan(float* slots, int nseq, int nseg, int ndir, int ng, hipStream_t stream);
+
 // fp32-arithmetic token-recurrent path (any supported dtype combination).
 int launch_gla_recurrent(const GlaArgs& a);
 size_t gla_recurrent_workspace(int B, int H, int L, int Dv, int io_dtype);
