@@ -5,6 +5,7 @@ import pytest
 import torch
 
 import vig_amd
+from oracle import gla_oracle as O
 from vig_amd.synthetic import make_gla_inputs
 
 from .util import announce, f64, oracle_bidir
@@ -38,3 +39,24 @@ def test_forward_magnitudes_and_infinite_gates():
     got = f64(vig_amd.gla_bidir_forward(*(t.cuda() for t in (q, k, v, gf, gb))))
     for h in range(2):
         assert np.abs(got[0, h] - want[0, h]).max() <= 1e-5 * np.abs(want[0, h]).max()
+
+
+@pytest.mark.parametrize("gate_scale", [1 / 16, 1.0])  # in range; beyond it (flagged for the recurrent kernel)
+@pytest.mark.parametrize("B,H,L,Dk", [(1, 1, 2, 64), (2, 2, 33, 32), (2, 3, 196, 32), (1, 2, 224, 64), (1, 2, 225, 64),
+                                      (1, 2, 256, 32), (1, 2, 449, 64), (1, 1, 700, 32)])
+def test_backward(B, H, L, Dk, gate_scale):
+    announce(f"fp32 backward on the matrix cores B{B} H{H} L={L} Dk={Dk} gates x {gate_scale}")
+    t = make_gla_inputs(B, H, L, Dk, 64, seed=950 + L, dtype=torch.float32, gate_scale=gate_scale)
+    d_o = torch.randn(t[2].shape, generator=torch.Generator().manual_seed(4))
+    for args in (t, (*t[:4], None)):
+        want = O.bidir_gla_backward(*(f64(a) if a is not None else None for a in args), f64(d_o), out_scale=0.5)
+        x = [a.cuda() if a is not None else None for a in (*args, d_o)]
+        mine = vig_amd.gla_bidir_backward(*x, out_scale=0.5)
+        serial = vig_amd.gla_bidir_backward(*x, out_scale=0.5, exact=True)
+        for name, a, b, w in zip(("dq", "dk", "dv", "dg_fwd", "dg_bwd"), mine, serial, want):
+            if w is None:
+                assert a is None
+                continue
+            err = lambda y: np.linalg.norm(f64(y) - w) / np.linalg.norm(w)
+            assert err(a) <= max(2 * err(b), 4e-7), (name, err(a), err(b))
+

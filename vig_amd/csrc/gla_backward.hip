@@ -270,6 +270,7 @@ static size_t flags_end(int B, int H, int L, int Dk, int Dv, int bidir) {
 }
 size_t gla_backward_workspace(int B, int H, int L, int Dk, int Dv, int bidir) {
   const size_t seg = gla_backward_mfma_workspace(B, H, L, Dk, Dv);
+
   if (seg == 0) return recurrent_floats(B, H, L, Dk, Dv, bidir) * sizeof(float) + (size_t)B * H * sizeof(int);
   return flags_end(B, H, L, Dk, Dv, bidir) + seg;
 }
@@ -287,6 +288,20 @@ int launch_gla_backward(const void* q, const void* k, const void* v, const void*
                                             H, L, Dk, scale * out_scale, stream);
     if (rc != 0) return rc;
     a.only_flagged = flags;  // slabs with gates beyond the matrix-core kernel's range
+  }
+  if (!exact && gla_backward_f32_supported(B, H, L, Dk, Dv, io_dtype, gate_dtype, g_bwd != nullptr)) {
+    // the states of a long sequence lie in the segment workspace (two 16.6 KB slots per set and 224 tokens; 149 KB are there
+    // per 256), of 225 to 256 tokens in the recurrent kernel's scratch, which runs after everything has read them
+    int* flags = reinterpret_cast<int*>((float*)workspace + recurrent_floats(B, H, L, Dk, Dv, g_bwd != nullptr));
+    const bool behind = L > 256;
+    const size_t room = behind ? gla_backward_mfma_workspace(B, H, L, Dk, Dv)
+                               : recurrent_floats(B, H, L, Dk, Dv, g_bwd != nullptr) * sizeof(float);
+    if (gla_backward_f32_states(B, H, L) > room) return -28;
+    float* states = behind ? (float*)((char*)workspace + flags_end(B, H, L, Dk, Dv, g_bwd != nullptr)) : (float*)workspace;
+    const int rc = launch_gla_backward_f32(q, k, v, g_fwd, g_bwd, d_o, dq, dk, dv, dg_fwd, dg_bwd, flags, states, B, H, L,
+                                           Dk, scale * out_scale, stream);
+    if (rc != 0) return rc;
+    a.only_flagged = flags;
   }
   if (io_dtype == 0) return gate_dtype == 0 ? launch_bwd_d<float, float>(a) : launch_bwd_d<float, uint16_t>(a);
   return gate_dtype == 0 ? launch_bwd_d<uint16_t, float>(a) : launch_bwd_d<uint16_t, uint16_t>(a);

@@ -307,12 +307,14 @@ template <int NG>
 __global__ __launch_bounds__(256, 2) void gla_f32_state_kernel(const float* __restrict__ k0, const float* __restrict__ v0,
                                                                const float* __restrict__ q1, const float* __restrict__ do1,
                                                                const float* __restrict__ gf, const float* __restrict__ gb,
-                                                               float* __restrict__ ws, int L, int NT, int nseg) {
+                                                               float* __restrict__ ws, int* __restrict__ flags, int L, int NT,
+                                                               int nseg) {
   constexpr int DK = 16 * NG, NP = NG / 2;
   const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
   const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int dir = w >> 1, pv = w & 1;
   const bool grad = blockIdx.z != 0;
+  if (flags && blockIdx.y == 0 && !grad && threadIdx.x == 0) flags[blockIdx.x] = 0;
   const float* kk = grad ? q1 : k0;
   const float* vv = grad ? do1 : v0;
   const float* gg = (dir == 0) != grad ? gf : gb;
@@ -434,13 +436,26 @@ static int launch_f32_t(const GlaArgs& a, const F32Geo& geo, int dev) {
   if (geo.states) {
     hipLaunchKernelGGL((gla_f32_state_kernel<NG>), dim3(a.B * a.H, geo.nseg), dim3(BIDIR ? 256 : 128), 0, a.stream,
                        (const float*)a.k, (const float*)a.v, nullptr, nullptr, (const float*)a.g_fwd, (const float*)a.g_bwd,
-                       (float*)a.workspace, a.L, geo.NT, geo.nseg);
+                       (float*)a.workspace, (int*)nullptr, a.L, geo.NT, geo.nseg);
     const int rc = launch_gla_segment_scan((float*)a.workspace, a.B * a.H, geo.nseg, BIDIR ? 2 : 1, NG, a.stream);
     if (rc) return rc;
   }
   hipLaunchKernelGGL((gla_f32_kernel<NG, BIDIR>), dim3(a.B * a.H, geo.nseg), dim3(64 * geo.NT), lay.total, a.stream,
                      (const float*)a.q, (const float*)a.k, (const float*)a.v, (const float*)a.g_fwd, (const float*)a.g_bwd,
                      (float*)a.o, geo, a.scale * a.out_scale);
+  return hipGetLastError() == hipSuccess ? 0 : -5;
+}
+
+int launch_gla_f32_states(int NG, const float* k, const float* v, const float* q, const float* d_o, const float* gf,
+                          const float* gb, float* slots, int* flags, int nseq, int L, int NT, int nseg, hipStream_t stream) {
+  // (a causal call has no reverse gates: its second direction's slots are computed with the forward ones and not read)
+  const float* g2 = gb ? gb : gf;
+  if (NG == 4)
+    hipLaunchKernelGGL((gla_f32_state_kernel<4>), dim3(nseq, nseg, 2), dim3(256), 0, stream, k, v, q, d_o, gf, g2, slots, flags, L, NT,
+                       nseg);
+  else
+    hipLaunchKernelGGL((gla_f32_state_kernel<2>), dim3(nseq, nseg, 2), dim3(256), 0, stream, k, v, q, d_o, gf, g2, slots, flags, L, NT,
+                       nseg);
   return hipGetLastError() == hipSuccess ? 0 : -5;
 }
 

@@ -63,6 +63,17 @@ inline int gla_f32_segment_tiles(int L) { return gla_tile_segment_tiles(L); }
 bool gla_f32_supported(const GlaArgs& a);
 size_t gla_f32_workspace(int B, int H, int L, int Dk, int Dv);
 int launch_gla_f32(const GlaArgs& a);
+// both sets of segment contributions of an fp32 backward: the states (k, v) and, behind them, the gradient states (q, d_o)
+// (flags, one int per sequence, are cleared on the way)
+int launch_gla_f32_states(int NG, const float* k, const float* v, const float* q, const float* d_o, const float* gf,
+                          const float* gb, float* slots, int* flags, int nseq, int L, int NT, int nseg, hipStream_t stream);
+// fp32 backward on the matrix cores; one flag per sequence marks what it left to the recurrent kernel; states:
+// gla_backward_f32_states() bytes
+bool gla_backward_f32_supported(int B, int H, int L, int Dk, int Dv, int io_dtype, int gate_dtype, bool bidir);
+size_t gla_backward_f32_states(int B, int H, int L);
+int launch_gla_backward_f32(const void* q, const void* k, const void* v, const void* gf, const void* gb, const void* d_o,
+                            void* dq, void* dk, void* dv, void* dgf, void* dgb, int* flags, float* states, int B, int H, int L,
+                            int Dk, float s, hipStream_t stream);
 // chains the slots of a state pass in place (gla_segment_scan_kernel, no state in or out)
 int launch_gla_segment_scan(float* slots, int nseq, int nseg, int ndir, int ng, hipStream_t stream);
 
