@@ -494,6 +494,17 @@ int vig_locality_blend_linear_fwd(const void* o, const void* local, const void* 
 int vig_patch_conv_fwd(const void* x, const void* w_packed, void* y, int B, int Cin, int H, int W, int KH, int KW,
                        int stride, int padding, int Cout, int io_dtype, void* stream);
 
+/*
+ * Weight and bias gradients of a linear layer over bf16 rows (what autograd derives for the nn.Linear layers of the block):
+ *   dweight [N, K] (fp32) = sum over rows of dy[row, n] * x[row, k];  dbias [N] (fp32) = sum over rows of dy[row, n],
+ * fp32 accumulation in a fixed order.  dy rows are dy_row_stride elements apart, x rows x_row_stride (multiples of 8, 16-byte
+ * aligned bases: either may be a column block of a wider tensor); N % 8 == 0, K % 8 == 0; dbias NULL: not wanted.
+ * `workspace` holds vig_linear_bwd_weight_workspace(rows, N, K) bytes of partial sums.
+ */
+size_t vig_linear_bwd_weight_workspace(long long rows, int N, int K);
+int vig_linear_bwd_weight(const void* dy, long long dy_row_stride, const void* x, long long x_row_stride, float* dweight,
+                          float* dbias, void* workspace, size_t workspace_bytes, long long rows, int N, int K, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -62,6 +62,9 @@ SIGNATURES = {
     "vig_swiglu_bwd": (_c_int, [_c_void_p] * 3 + [_c_longlong, _c_int, _c_int, _c_void_p]),
     "vig_rmsnorm_bwd_workspace": (_c_size_t, [_c_longlong, _c_int]),
     "vig_rmsnorm_bwd": (_c_int, [_c_void_p] * 7 + [_c_size_t, _c_longlong, _c_int, _c_float, _c_int, _c_void_p]),
+    "vig_linear_bwd_weight_workspace": (_c_size_t, [_c_longlong, _c_int, _c_int]),
+    "vig_linear_bwd_weight": (_c_int, [_c_void_p, _c_longlong, _c_void_p, _c_longlong] + [_c_void_p] * 3 +
+                              [_c_size_t, _c_longlong, _c_int, _c_int, _c_void_p]),
     "vig_swiglu_fwd": (_c_int, [_c_void_p, _c_void_p, ctypes.c_longlong, _c_int, _c_int, _c_void_p]),
 }
 

@@ -59,6 +59,10 @@ int launch_gla_backward(const void* q, const void* k, const void* v, const void*
                         int B, int H, int L, int Dk, int Dv, float scale, float out_scale, int io_dtype,
                         int gate_dtype, bool exact, hipStream_t stream);
 size_t gla_backward_workspace(int B, int H, int L, int Dk, int Dv, int bidir);
+bool linear_wgrad_supported(long long T, int N, int K);
+size_t linear_wgrad_workspace(long long T, int N, int K);
+int launch_linear_wgrad(const void* dy, long long ldy, const void* x, long long ldx, long long T, int N, int K, float* dw,
+                        float* db, void* workspace, hipStream_t stream);
 }  // namespace vig
 
 static bool dtype_ok(int d) { return d == VIG_F32 || d == VIG_BF16; }
@@ -643,6 +647,21 @@ int vig_gla_bidir_bwd_exact(const void* q, const void* k, const void* v, const v
                             float out_scale, int io_dtype, int gate_dtype, void* stream) {
   return gla_bidir_bwd(q, k, v, g_fwd, g_bwd, d_o, dq, dk, dv, dg_fwd, dg_bwd, workspace, workspace_bytes, B, H, L, Dk,
                        Dv, scale, out_scale, io_dtype, gate_dtype, true, stream);
+}
+
+size_t vig_linear_bwd_weight_workspace(long long rows, int N, int K) {
+  return vig::linear_wgrad_supported(rows, N, K) ? vig::linear_wgrad_workspace(rows, N, K) : 0;
+}
+
+int vig_linear_bwd_weight(const void* dy, long long dy_row_stride, const void* x, long long x_row_stride, float* dweight,
+                          float* dbias, void* workspace, size_t workspace_bytes, long long rows, int N, int K, void* stream) {
+  if (!dy || !x || !dweight || rows <= 0 || N <= 0 || K <= 0 || dy_row_stride < N || x_row_stride < K) return VIG_EINVAL;
+  if (!vig::linear_wgrad_supported(rows, N, K)) return VIG_ENOTSUP;
+  if (!strided_rows_ok(dy, dy_row_stride, VIG_BF16) || !strided_rows_ok(x, x_row_stride, VIG_BF16) ||
+      !aligned16(dweight, workspace) || (dbias && reinterpret_cast<uintptr_t>(dbias) % 4))
+    return VIG_EINVAL;
+  if (!workspace || workspace_bytes < vig::linear_wgrad_workspace(rows, N, K)) return VIG_ENOSPC;
+  return vig::launch_linear_wgrad(dy, dy_row_stride, x, x_row_stride, rows, N, K, dweight, dbias, workspace, (hipStream_t)stream);
 }
 
 }  // extern "C"

@@ -89,4 +89,21 @@ __device__ __forceinline__ float logsigmoidf_(float x) {
   return fminf(x, 0.f) - 0.6931471805599453f * __builtin_amdgcn_logf(1.f + exp_fast(-fabsf(x)));
 }
 
+// 16 bytes per lane from memory straight into LDS: lane i lands 16 i bytes behind lds_base (wave-uniform byte offset in the
+// workgroup's LDS).  In assembly, because the compiler answers the builtin of this load with waits of its own in front of
+// every later LDS read it cannot tell apart from the destination, down to vmcnt(0), which also drains the stores and the
+// loads of stages further ahead.  The caller waits (wait_vmem), counting what it has issued since.  (m0 is reserved, so it
+// cannot be named as changed: no kernel mixes this with the builtin.)
+__device__ __forceinline__ void load_to_lds16(const void* p, uint32_t lds_base) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_base), "v"(p) : "memory");
+}
+// at most N vector memory operations (loads and stores, in the order of issue) still out
+template <int N>
+__device__ __forceinline__ void wait_vmem() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"i"(N) : "memory");
+}
+__device__ __forceinline__ uint32_t lds_offset(const void* p) {
+  return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p;
+}
+
 }  // namespace vig

@@ -23,6 +23,11 @@ namespace {
 
 constexpr int kLinWaves = 8;
 
+// This wave's LDS writes done, then the barrier, and nothing else: global requests and stores issued before it stay in
+// flight.  (A fence would drain them: the compiler counts loads that land in LDS as LDS writes.  Whoever reads what
+// such a load brings waits for it by itself.)
+__device__ __forceinline__ void tile_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
 template <int KS>
 __global__ __launch_bounds__(64 * kLinWaves) void linear_swiglu_kernel(const uint16_t* __restrict__ A,
                                                                        const uint16_t* __restrict__ W,
@@ -58,16 +63,16 @@ __global__ __launch_bounds__(64 * kLinWaves) void linear_swiglu_kernel(const uin
   // the wave's base, so a wave loads whole token rows (the first K/8 lanes, one 16-byte chunk each) to the rows' padded
   // places.  Token rows past the end are not requested: their rows of the buffer keep old data, and their products
   // are never stored.
-  typedef __attribute__((address_space(3))) void* lds_ptr_t;
+  const uint32_t lds0 = lds_offset(buf);
+  const int uwave = __builtin_amdgcn_readfirstlane(wave);
   auto fetch = [&](int tile, int which) {
     if (tile >= ntiles_t) return;
-    char* base = reinterpret_cast<char*>(buf + which * (32 * kRow));
+    const uint32_t base = lds0 + which * (32 * kRow * 2);
 #pragma unroll
     for (int i = 0; i < kPer; ++i) {
-      const int row = i * kLinWaves + wave;
+      const int row = i * kLinWaves + uwave;
       if (lane < kCols && tile * 32 + row < T)
-        __builtin_amdgcn_global_load_lds(A + (size_t)tile * (32 * K) + (size_t)row * K + lane * 8,
-                                         (lds_ptr_t)(base + row * (kRow * 2)), 16, 0, 0);
+        load_to_lds16(A + (size_t)tile * (32 * K) + (size_t)row * K + lane * 8, base + row * (kRow * 2));
     }
   };
   f32x16_t g, u;
@@ -117,10 +122,15 @@ __global__ __launch_bounds__(64 * kLinWaves) void linear_swiglu_kernel(const uin
   };
   fetch(worker, 0);
   int cur = 0;
+  bool stored = false;  // an epilogue's stores were issued after the current tile's loads (a full tile's: only the last
+                        // tile of all, behind which nothing is waited for, may be short)
   for (int tile = worker; tile < ntiles_t; tile += nworkers, cur ^= 1) {
     const uint16_t* mine = buf + cur * (32 * kRow);
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this thread's chunks of the tile have landed
-    __syncthreads();  // the tile is complete; the other buffer was last read before the previous barrier
+    // this thread's chunks of the tile have landed; the two stores of an epilogue behind them may still be on their way
+    // (waiting for those too, as a full barrier does, cost a tile the latency of a store)
+    if (stored) wait_vmem<2>();
+    else wait_vmem<0>();
+    tile_barrier();  // the tile is complete; the other buffer was last read before the previous barrier
     fetch(tile + nworkers, cur ^ 1);
     // The two waves of a SIMD (w and w + 4) take turns on its two pipes: the lower wave runs this tile's matrix
     // instructions first and its SwiGLU epilogue after; the upper wave first runs the epilogue of its PREVIOUS tile
@@ -129,7 +139,9 @@ __global__ __launch_bounds__(64 * kLinWaves) void linear_swiglu_kernel(const uin
     if (wave < kLinWaves / 2) {
       products(mine);
       epilogue(tile);  // (straight-line after the matrix instructions: no run-time branch in between)
+      stored = have;
     } else {
+      stored = have && tile > worker;
       if (tile > worker) epilogue(tile - nworkers);
       products(mine);
     }
@@ -171,11 +183,6 @@ __device__ __forceinline__ float lane_permuted(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
 }
 
-// This wave's LDS writes done, then the barrier, and nothing else: global requests and stores issued before it stay in
-// flight.  (A fence would drain them: the compiler counts loads that land in LDS as LDS writes.  Whoever reads what
-// such a load brings waits for it by itself.)
-__device__ __forceinline__ void tile_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
 template <int KS, int NW, int TPW>
 __global__ __launch_bounds__(64 * NW) void blend_linear_kernel(const uint16_t* __restrict__ o,
                                                               const uint16_t* __restrict__ loc,
@@ -214,30 +221,33 @@ __global__ __launch_bounds__(64 * NW) void blend_linear_kernel(const uint16_t* _
   const int ntiles_t = (T + 31) / 32;
   const float* wg8 = wnorm + ((tid % kCols) & 7) * 8;  // (kThreads % kCols == 0: a thread's octets share their column)
   const float* wl8 = wg8 + 64;
-  typedef __attribute__((address_space(3))) void* lds_ptr_t;
   // requests this thread's octets of a tile into its slots; tokens past the end are not requested (their rows of y
   // hold whatever the slots held: their products are never stored)
   const int col = tid % kCols, row0 = tid / kCols;  // this thread's octets: column col of rows row0 + kRowStep * i
   constexpr int kRowStep = kThreads / kCols;
   const size_t o_col = ((size_t)(col >> 3) * L) * 64 + (col & 7) * 8;  // head col / 8, channels 8 (col % 8) ..
   const size_t o_batch = (size_t)H * L * 64;
+  const uint32_t park0 = __builtin_amdgcn_readfirstlane(lds_offset(park) + wave * (64 * 16));
   auto fetch = [&](int tile) {
 #pragma unroll 1
     for (int i = 0; i < kPer; ++i) {  // (one octet's addresses at a time: the weight tiles leave few registers)
       const int t = tile * 32 + row0 + kRowStep * i;
       if (tile < ntiles_t && t < T) {
         const unsigned b = (unsigned)t / (unsigned)L, l = (unsigned)t - b * (unsigned)L;
-        char* slot = reinterpret_cast<char*>(park + (i * 3) * kThreads + wave * 64);  // (wave-uniform; lanes 16 B apart)
-        __builtin_amdgcn_global_load_lds(o + b * o_batch + (size_t)l * 64 + o_col, (lds_ptr_t)slot, 16, 0, 0);
-        __builtin_amdgcn_global_load_lds(loc + (size_t)t * K + col * 8, (lds_ptr_t)(slot + kThreads * 16), 16, 0, 0);
-        __builtin_amdgcn_global_load_lds(glin + (size_t)t * ldg + col * 8, (lds_ptr_t)(slot + 2 * kThreads * 16), 16, 0, 0);
+        const uint32_t slot = park0 + (i * 3) * (kThreads * 16);  // (wave-uniform; lanes 16 B apart)
+        load_to_lds16(o + b * o_batch + (size_t)l * 64 + o_col, slot);
+        load_to_lds16(loc + (size_t)t * K + col * 8, slot + kThreads * 16);
+        load_to_lds16(glin + (size_t)t * ldg + col * 8, slot + 2 * kThreads * 16);
       }
     }
   };
   const int nworkers = gridDim.x;
   // the blend of this thread's octets of a tile (they wait in its slots), straight into the tile's operand buffer
-  auto blend = [&](uint16_t* mine) {
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the octets are in their slots
+  // (stored: the stores of a tile's result were issued behind the octets' loads and may still be on their way; waited for,
+  // their latency was part of every tile)
+  auto blend = [&](uint16_t* mine, bool stored) {
+    if (stored) wait_vmem<2 * TPW>();
+    else wait_vmem<0>();
 #pragma unroll 1
     for (int i = 0; i < kPer; ++i) {
       const u32x4_t po = park[(i * 3 + 0) * kThreads + tid], pl = park[(i * 3 + 1) * kThreads + tid],
@@ -321,7 +331,7 @@ __global__ __launch_bounds__(64 * NW) void blend_linear_kernel(const uint16_t* _
   // (being refilled now) and tile i's is complete.
   __syncthreads();  // the norm weights are in place
   fetch(blockIdx.x);
-  blend(buf);
+  blend(buf, false);
   fetch(blockIdx.x + nworkers);
   tile_barrier();
   int cur = 0;
@@ -332,12 +342,12 @@ __global__ __launch_bounds__(64 * NW) void blend_linear_kernel(const uint16_t* _
     if ((wave >> 2) != 1) {
       products(mine, tile);
       if (more) {
-        blend(next);
+        blend(next, true);
         fetch(tile + 2 * nworkers);
       }
     } else {
       if (more) {
-        blend(next);
+        blend(next, tile != (int)blockIdx.x);
         fetch(tile + 2 * nworkers);
       }
       products(mine, tile);
