@@ -281,6 +281,27 @@ int vig_dirgate_bwd(const void* gk_lin, const void* d_g, void* d_gk_lin, int B, 
 int vig_dirgate_lowrank_fwd(const void* gk_low, long long low_row_stride, const void* w_up, const void* b_up,
                             void* g_out, int B, int L, int H, int Dk, int rank, float inv_normalizer, float clamp_min,
                             int in_dtype, int out_dtype, void* stream);
+/*
+ * Backward of vig_dirgate_lowrank_fwd for bf16 rows: d_g [2, B, H, L, Dk] (type out_dtype) ->
+ *   d_x [B*L, 2*H*Dk] bf16, the gradient at the up-projection's result (its weight gradient is d_x^T gk_low),
+ *   d_low [B*L, rank] bf16, rows d_low_row_stride elements apart (0 = packed) = d_x w_up.
+ * w_up_t is w_up transposed, [rank, 2*H*Dk].  Dk % 16 == 0, rank 16, in_dtype VIG_BF16.
+ *
+ * Replaces: what autograd derives for classification/models/vig.py:432-441 and the second gk_proj layer in front.
+ */
+int vig_dirgate_lowrank_bwd(const void* gk_low, long long low_row_stride, const void* w_up, const void* w_up_t,
+                            const void* b_up, const void* d_g, void* d_x, void* d_low, long long d_low_row_stride, int B,
+                            int L, int H, int Dk, int rank, float inv_normalizer, float clamp_min, int in_dtype,
+                            int out_dtype, void* stream);
+
+/*
+ * Up to 16 small tensors converted in one launch: dst[j] (type dst_dtype[j]) gets the n[j] elements of src[j] (type
+ * src_dtype[j]); zeros where src[j] is NULL; transposed where transposed_cols[j] > 0 (src is [n/cols, cols], dst
+ * [cols, n/cols]).  What a training step needs of a block's weights after the optimiser has changed them.
+ */
+int vig_cast_many(const void* const* src, void* const* dst, const int* n, const int* transposed_cols, const int* src_dtype,
+                  const int* dst_dtype, int count, void* stream);
+
 
 /*
  * 3x3 depthwise convolution on the token grid, channels-last, zero padding 1.
@@ -292,12 +313,16 @@ int vig_dirgate_lowrank_fwd(const void* gk_low, long long low_row_stride, const 
  */
 int vig_dwconv3x3_fwd(const void* x, const float* weight, const float* bias, void* y,
                       int B, int h, int w, int C, int silu, int io_dtype, void* stream);
+/* The same; with silu, `pre` (may be NULL) also receives the stored result in front of the activation, and the activation
+ * reads that stored value (what a backward needs). */
+int vig_dwconv3x3_fwd_pre(const void* x, const float* weight, const float* bias, void* y, void* pre, int B, int h, int w,
+                          int C, int silu, int io_dtype, void* stream);
+
 
 /*
  * Weight and bias gradients of vig_dwconv3x3_fwd (without its SiLU) from x and dy [B, h*w, C]:
  *   dw_db fp32 [C*9 + C]: dw[c, ky, kx] = sum dy[b, y, x, c] * x[b, y+ky-1, x+kx-1, c], then db[c] = sum dy[b, y, x, c].
- * The input gradient needs no entry point of its own: it is vig_dwconv3x3_fwd on dy with the nine taps of every
- * channel mirrored through the centre.  `workspace` holds vig_dwconv3x3_bwd_weight_workspace(B, C) bytes
+ * `workspace` holds vig_dwconv3x3_bwd_weight_workspace(B, C) bytes
  * (per-workgroup partial sums, added in a fixed order: no atomics).
  *
  * Replaces: the convolution library's depthwise weight-gradient call behind classification/models/vig.py:291-294.
@@ -305,6 +330,12 @@ int vig_dwconv3x3_fwd(const void* x, const float* weight, const float* bias, voi
 size_t vig_dwconv3x3_bwd_weight_workspace(int B, int C);
 int vig_dwconv3x3_bwd_weight(const void* x, const void* dy, float* dw_db, void* workspace, size_t workspace_bytes,
                              int B, int h, int w, int C, int io_dtype, void* stream);
+/* Both gradients in one pass over x and dy: dx (NULL to skip it) and dw_db (NULL to skip it, then no workspace).  With
+ * `pre` (see vig_dwconv3x3_fwd_pre) dy is the gradient behind the SiLU and is taken through it first, rounded to the
+ * storage type. */
+int vig_dwconv3x3_bwd(const void* x, const void* dy, const void* pre, const float* weight, void* dx, float* dw_db,
+                      void* workspace, size_t workspace_bytes, int B, int h, int w, int C, int io_dtype, void* stream);
+
 
 /*
  * Synthetic locality gate of the ViG-B benchmark shape:
@@ -364,6 +395,12 @@ int vig_locality_blend_bwd(const void* o, const void* local, const void* g_lin, 
                            const void* dy, void* d_o, void* d_local, void* d_glin, float* dw, void* workspace,
                            size_t workspace_bytes, int B, int H, int L, int Dv, long long g_row_stride, float eps,
                            int silu_out, int io_dtype, void* stream);
+/* The same with d_glin's rows d_glin_row_stride elements apart (0 = packed). */
+int vig_locality_blend_bwd_strided(const void* o, const void* local, const void* g_lin, const float* w_g, const float* w_l,
+                                   const void* dy, void* d_o, void* d_local, void* d_glin, float* dw, void* workspace,
+                                   size_t workspace_bytes, int B, int H, int L, int Dv, long long g_row_stride,
+                                   long long d_glin_row_stride, float eps, int silu_out, int io_dtype, void* stream);
+
 
 /*
  * Residual-add + RMS norm over the last dimension (rows x C, C % 8 == 0, C <= 4096):
@@ -377,6 +414,12 @@ int vig_locality_blend_bwd(const void* o, const void* local, const void* g_lin, 
  */
 int vig_rmsnorm_fwd(const void* x, const void* residual, const float* weight, void* y, void* residual_out,
                     long long rows, int C, float eps, int round_sum, int io_dtype, void* stream);
+/* The same with a type for each role: residual and sum of sum_dtype, x of x_dtype, y of y_dtype.  One type throughout, or an
+ * fp32 sum with a bf16 y (a bf16 branch meeting the fp32 stream under autocast). */
+int vig_rmsnorm_mixed_fwd(const void* x, const void* residual, const float* weight, void* y, void* residual_out,
+                          long long rows, int C, float eps, int round_sum, int x_dtype, int sum_dtype, int y_dtype,
+                          void* stream);
+
 
 /*
  * LayerNorm over the last dimension (rows x C, C % 8 == 0, C <= 4096), optional SiLU behind it:
@@ -416,6 +459,10 @@ int vig_split_heads_fwd(const void* qkv, void* q, void* k, void* v, int B, int L
  */
 int vig_split_heads_bwd(const void* dq, const void* dk, const void* dv, void* d_qkv, int B, int L, int H, int Dk,
                         int Dv, int io_dtype, void* stream);
+/* The same with d_qkv's rows d_qkv_row_stride elements apart (0 = packed): the columns of a wider matrix. */
+int vig_split_heads_bwd_strided(const void* dq, const void* dk, const void* dv, void* d_qkv, long long d_qkv_row_stride,
+                                int B, int L, int H, int Dk, int Dv, int io_dtype, void* stream);
+
 
 /*
  * SwiGLU product of the MLP:  gate_up [rows, 2*I] = (gate | up)  ->  out [rows, I] = gate * up / (1 + exp(-gate))
@@ -450,6 +497,12 @@ size_t vig_rmsnorm_bwd_workspace(long long rows, int C);
 int vig_rmsnorm_bwd(const void* sum, const float* weight, const void* dy, const void* d_sum, void* ds, float* dweight,
                     void* workspace, size_t workspace_bytes, long long rows, int C, float eps, int io_dtype,
                     void* stream);
+/* The same with a type for each role (see vig_rmsnorm_mixed_fwd); dx (may be NULL) receives ds in y_dtype, for a branch of
+ * that type. */
+int vig_rmsnorm_mixed_bwd(const void* sum, const float* weight, const void* dy, const void* d_sum, void* ds, void* dx,
+                          float* dweight, void* workspace, size_t workspace_bytes, long long rows, int C, float eps,
+                          int sum_dtype, int y_dtype, void* stream);
+
 
 /*
  * gate_proj and the SwiGLU product in one kernel, for a short contraction (K = 384 or 192, the hidden sizes of

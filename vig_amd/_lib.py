@@ -65,6 +65,16 @@ SIGNATURES = {
     "vig_linear_bwd_weight_workspace": (_c_size_t, [_c_longlong, _c_int, _c_int]),
     "vig_linear_bwd_weight": (_c_int, [_c_void_p, _c_longlong, _c_void_p, _c_longlong] + [_c_void_p] * 3 +
                               [_c_size_t, _c_longlong, _c_int, _c_int, _c_void_p]),
+    "vig_dirgate_lowrank_bwd": (_c_int, [_c_void_p, _c_longlong] + [_c_void_p] * 6 + [_c_longlong] + [_c_int] * 5 +
+                                [_c_float, _c_float, _c_int, _c_int, _c_void_p]),
+    "vig_cast_many": (_c_int, [_c_void_p] * 6 + [_c_int, _c_void_p]),
+    "vig_dwconv3x3_fwd_pre": (_c_int, [_c_void_p] * 5 + [_c_int] * 6 + [_c_void_p]),
+    "vig_dwconv3x3_bwd": (_c_int, [_c_void_p] * 7 + [_c_size_t] + [_c_int] * 5 + [_c_void_p]),
+    "vig_locality_blend_bwd_strided": (_c_int, [_c_void_p] * 11 + [_c_size_t] + [_c_int] * 4 +
+                                       [_c_longlong, _c_longlong, _c_float, _c_int, _c_int, _c_void_p]),
+    "vig_split_heads_bwd_strided": (_c_int, [_c_void_p] * 4 + [_c_longlong] + [_c_int] * 6 + [_c_void_p]),
+    "vig_rmsnorm_mixed_fwd": (_c_int, [_c_void_p] * 5 + [_c_longlong, _c_int, _c_float] + [_c_int] * 4 + [_c_void_p]),
+    "vig_rmsnorm_mixed_bwd": (_c_int, [_c_void_p] * 8 + [_c_size_t, _c_longlong, _c_int, _c_float, _c_int, _c_int, _c_void_p]),
     "vig_swiglu_fwd": (_c_int, [_c_void_p, _c_void_p, ctypes.c_longlong, _c_int, _c_int, _c_void_p]),
 }
 

@@ -54,7 +54,7 @@ EXT = os.path.join(LIBDIR, "libvig_torch_ext.so")
 CALLS = os.path.join(LIBDIR, "vig_host.so")
 
 
-def _host_library(src: str, out: str, extra_libs: list[str], verbose: bool) -> str:
+def _host_library(srcs: list[str], out: str, extra_libs: list[str], verbose: bool) -> str:
     """Host code only, compiled with the host compiler against torch's headers and linked to libvig_gla.so next to it."""
     import sysconfig
 
@@ -66,7 +66,7 @@ def _host_library(src: str, out: str, extra_libs: list[str], verbose: bool) -> s
     inc = [f"-I{p}" for p in ce.include_paths()] + ["-I/opt/rocm/include", f"-I{sysconfig.get_paths()['include']}"]
     cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}", "-Wno-deprecated-declarations", *inc,
-           os.path.join(CSRC, src), "-o", out, f"-L{LIBDIR}", "-lvig_gla", f"-L{tlib}", *extra_libs, "-lc10", "-lc10_hip",
+           *(os.path.join(CSRC, s) for s in srcs), "-o", out, f"-L{LIBDIR}", "-lvig_gla", f"-L{tlib}", *extra_libs, "-lc10", "-lc10_hip",
            "-ltorch_cpu", "-ltorch_hip", "-ltorch", "-Wl,-rpath,$ORIGIN", f"-Wl,-rpath,{tlib}"]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
@@ -78,10 +78,11 @@ def _host_library(src: str, out: str, extra_libs: list[str], verbose: bool) -> s
 
 def build_torch_extension(verbose: bool = True) -> str:
     """Builds vig_amd/lib/libvig_torch_ext.so, the PyTorch-ROCm operator library over the C ABI (csrc/torch_ext.cpp), and
-    vig_amd/lib/vig_host.so, the op-level calls as a CPython module (csrc/py_calls.cpp)."""
+    vig_amd/lib/vig_host.so, the op-level calls and the recorded block as a CPython module
+    (csrc/py_calls.cpp, csrc/train_block.cpp)."""
     with ThreadPoolExecutor(max_workers=2) as ex:
-        jobs = [ex.submit(_host_library, "torch_ext.cpp", EXT, [], verbose),
-                ex.submit(_host_library, "py_calls.cpp", CALLS, ["-ltorch_python"], verbose)]
+        jobs = [ex.submit(_host_library, ["torch_ext.cpp"], EXT, [], verbose),
+                ex.submit(_host_library, ["py_calls.cpp", "train_block.cpp"], CALLS, ["-ltorch_python"], verbose)]
         for j in jobs:
             j.result()
     return EXT

@@ -10,11 +10,16 @@ int launch_dirgate(const void* in, void* out, int B, int L, int H, int Dk, float
 int launch_dirgate_bwd(const void* in, const void* d_out, void* d_in, int B, int L, int H, int Dk, float inv_norm,
                        float clamp_min, int in_dtype, int out_dtype, hipStream_t stream);
 int launch_merge_heads(const void* dq, const void* dk, const void* dv, void* dqkv, int B, int L, int H, int Dk, int Dv,
-                       int io_dtype, hipStream_t stream);
+                       long long ld, int io_dtype, hipStream_t stream);
 size_t dwconv3x3_wgrad_workspace(int B, int C);
-int launch_dwconv3x3_wgrad(const void* x, const void* dy, float* dw_db, void* workspace, int B, int h, int w, int C,
-                           int io_dtype, hipStream_t stream);
-int launch_dwconv3x3(const void* x, const float* wt, const float* bias, void* y, int B, int h, int w, int C,
+int launch_dwconv3x3_bwd(const void* x, const void* dy, const void* pre, const float* wt, void* dx, float* dw_db,
+                         void* workspace, int B, int h, int w, int C, int io_dtype, hipStream_t stream);
+int launch_dirgate_lowrank_bwd(const void* low, long long ld, const void* w1, const void* w1t, const void* b1,
+                               const void* d_out, void* dx, void* d_low, long long ldd, int B, int L, int H, int Dk,
+                               float inv_norm, float clamp_min, int out_dtype, hipStream_t stream);
+int launch_cast_many(const void* const* src, void* const* dst, const int* n, const int* cols, const int* src_dtype,
+                     const int* dst_dtype, int count, hipStream_t stream);
+int launch_dwconv3x3(const void* x, const float* wt, const float* bias, void* y, void* pre, int B, int h, int w, int C,
                      int silu, int io_dtype, hipStream_t stream);
 int launch_dirgate_lowrank(const void* low, long long ld, const void* w1, const void* b1, void* out, int B, int L,
                            int H, int Dk, int rank, float inv_norm, float clamp_min, int in_dtype, int out_dtype,
@@ -27,10 +32,11 @@ int launch_locality_blend(const void* o, const void* loc, const void* glin, cons
 size_t locality_blend_bwd_workspace(int B, int L, int Dv);
 int launch_locality_blend_bwd(const void* o, const void* loc, const void* glin, const float* wg, const float* wl,
                               const void* dy, void* d_o, void* d_loc, void* d_glin, float* dw, void* workspace, int B,
-                              int H, int L, int Dv, long long ldg, float eps, int silu_out, int io_dtype,
+                              int H, int L, int Dv, long long ldg, long long ldd, float eps, int silu_out, int io_dtype,
                               hipStream_t stream);
+bool rmsnorm_types_ok(int x_dtype, int sum_dtype, int y_dtype);
 int launch_rmsnorm(const void* x, const void* residual, const float* weight, void* y, void* residual_out, int rows,
-                   int C, float eps, int round_sum, int io_dtype, hipStream_t stream);
+                   int C, float eps, int round_sum, int x_dtype, int sum_dtype, int y_dtype, hipStream_t stream);
 int launch_layernorm(const void* x, const float* weight, const float* bias, void* y, long long rows, int C, float eps,
                      int silu, const float* pre_bias, const void* post_add, int post_rows, int io_dtype,
                      hipStream_t stream);
@@ -40,8 +46,8 @@ int launch_swiglu(const void* in, void* out, long long rows, int I, int io_dtype
 int launch_swiglu_bwd(const void* in, const void* dy, void* din, long long rows, int I, int io_dtype,
                       hipStream_t stream);
 size_t rmsnorm_bwd_workspace(long long rows, int C);
-int launch_rmsnorm_bwd(const void* s, const float* weight, const void* dy, const void* d_sum, void* ds, float* dweight,
-                       void* workspace, long long rows, int C, float eps, int io_dtype, hipStream_t stream);
+int launch_rmsnorm_bwd(const void* s, const float* weight, const void* dy, const void* d_sum, void* ds, void* dx, float* dweight,
+                       void* workspace, long long rows, int C, float eps, int sum_dtype, int y_dtype, hipStream_t stream);
 bool blend_linear_supported(int H, int Dv, int C);
 int launch_blend_linear(const void* o, const void* loc, const void* glin, const float* w_g, const float* w_l,
                         const void* W, void* out, int B, int H, int L, int Dv, int C, long long ldg, float eps,
@@ -390,12 +396,20 @@ int vig_dirgate_bwd(const void* gk_lin, const void* d_g, void* d_gk_lin, int B, 
                                  (hipStream_t)stream);
 }
 
-int vig_split_heads_bwd(const void* dq, const void* dk, const void* dv, void* d_qkv, int B, int L, int H, int Dk,
-                        int Dv, int io_dtype, void* stream) {
+int vig_split_heads_bwd_strided(const void* dq, const void* dk, const void* dv, void* d_qkv, long long d_qkv_row_stride,
+                                int B, int L, int H, int Dk, int Dv, int io_dtype, void* stream) {
   if (!dq || !dk || !dv || !d_qkv || B <= 0 || L <= 0 || H <= 0 || Dk <= 0 || Dv <= 0) return VIG_EINVAL;
   if (!aligned16(dq, dk, dv, d_qkv)) return VIG_EINVAL;
   if (!dtype_ok(io_dtype) || (Dk % 8) != 0 || (Dv % 8) != 0 || B > 65535) return VIG_ENOTSUP;
-  return vig::launch_merge_heads(dq, dk, dv, d_qkv, B, L, H, Dk, Dv, io_dtype, (hipStream_t)stream);
+  const long long packed = (long long)H * (2 * Dk + Dv);
+  const long long ld = d_qkv_row_stride > 0 ? d_qkv_row_stride : packed;
+  if (ld < packed || !strided_rows_ok(d_qkv, ld, io_dtype)) return VIG_EINVAL;
+  return vig::launch_merge_heads(dq, dk, dv, d_qkv, B, L, H, Dk, Dv, ld, io_dtype, (hipStream_t)stream);
+}
+
+int vig_split_heads_bwd(const void* dq, const void* dk, const void* dv, void* d_qkv, int B, int L, int H, int Dk,
+                        int Dv, int io_dtype, void* stream) {
+  return vig_split_heads_bwd_strided(dq, dk, dv, d_qkv, 0, B, L, H, Dk, Dv, io_dtype, stream);
 }
 
 int vig_dirgate_lowrank_fwd(const void* gk_low, long long low_row_stride, const void* w_up, const void* b_up,
@@ -411,12 +425,44 @@ int vig_dirgate_lowrank_fwd(const void* gk_low, long long low_row_stride, const 
                                      in_dtype, out_dtype, (hipStream_t)stream);
 }
 
+int vig_dirgate_lowrank_bwd(const void* gk_low, long long low_row_stride, const void* w_up, const void* w_up_t,
+                            const void* b_up, const void* d_g, void* d_x, void* d_low, long long d_low_row_stride, int B,
+                            int L, int H, int Dk, int rank, float inv_normalizer, float clamp_min, int in_dtype,
+                            int out_dtype, void* stream) {
+  if (!gk_low || !w_up || !w_up_t || !b_up || !d_g || !d_x || !d_low || B <= 0 || L <= 0 || H <= 0 || Dk <= 0) return VIG_EINVAL;
+  if (in_dtype != VIG_BF16 || !dtype_ok(out_dtype) || (Dk % 16) != 0 || rank != 16) return VIG_ENOTSUP;
+  const long long ld = low_row_stride > 0 ? low_row_stride : rank, ldd = d_low_row_stride > 0 ? d_low_row_stride : rank;
+  if (ld < rank || ldd < rank || !strided_rows_ok(gk_low, ld, in_dtype) || !strided_rows_ok(d_low, ldd, in_dtype) ||
+      !aligned16(w_up, w_up_t, b_up, d_g, d_x))
+    return VIG_EINVAL;
+  return vig::launch_dirgate_lowrank_bwd(gk_low, ld, w_up, w_up_t, b_up, d_g, d_x, d_low, ldd, B, L, H, Dk, inv_normalizer,
+                                         clamp_min, out_dtype, (hipStream_t)stream);
+}
+
+int vig_cast_many(const void* const* src, void* const* dst, const int* n, const int* transposed_cols, const int* src_dtype,
+                  const int* dst_dtype, int count, void* stream) {
+  if (!src || !dst || !n || !transposed_cols || !src_dtype || !dst_dtype || count <= 0) return VIG_EINVAL;
+  if (count > vig::kMaxCastJobs) return VIG_ENOTSUP;
+  for (int j = 0; j < count; ++j) {
+    if (!dst[j] || n[j] <= 0 || transposed_cols[j] < 0 || (transposed_cols[j] && n[j] % transposed_cols[j])) return VIG_EINVAL;
+    if (!aligned16(src[j], dst[j]) || src[j] == dst[j]) return VIG_EINVAL;
+    if (!dtype_ok(src_dtype[j]) || !dtype_ok(dst_dtype[j])) return VIG_ENOTSUP;
+  }
+  return vig::launch_cast_many(src, dst, n, transposed_cols, src_dtype, dst_dtype, count, (hipStream_t)stream);
+}
+
+int vig_dwconv3x3_fwd_pre(const void* x, const float* weight, const float* bias, void* y, void* pre, int B, int h, int w,
+                          int C, int silu, int io_dtype, void* stream) {
+  if (!x || !weight || !y || B <= 0 || h <= 0 || w <= 0 || C <= 0 || x == y || (pre && (pre == y || pre == x || !silu)))
+    return VIG_EINVAL;
+  if (!aligned16(x, weight, bias, y, pre)) return VIG_EINVAL;
+  if (!dtype_ok(io_dtype) || (C % 8) != 0) return VIG_ENOTSUP;
+  return vig::launch_dwconv3x3(x, weight, bias, y, pre, B, h, w, C, silu, io_dtype, (hipStream_t)stream);
+}
+
 int vig_dwconv3x3_fwd(const void* x, const float* weight, const float* bias, void* y, int B, int h, int w, int C,
                       int silu, int io_dtype, void* stream) {
-  if (!x || !weight || !y || B <= 0 || h <= 0 || w <= 0 || C <= 0 || x == y) return VIG_EINVAL;
-  if (!aligned16(x, weight, bias, y)) return VIG_EINVAL;
-  if (!dtype_ok(io_dtype) || (C % 8) != 0) return VIG_ENOTSUP;
-  return vig::launch_dwconv3x3(x, weight, bias, y, B, h, w, C, silu, io_dtype, (hipStream_t)stream);
+  return vig_dwconv3x3_fwd_pre(x, weight, bias, y, nullptr, B, h, w, C, silu, io_dtype, stream);
 }
 
 size_t vig_dwconv3x3_bwd_weight_workspace(int B, int C) {
@@ -424,13 +470,20 @@ size_t vig_dwconv3x3_bwd_weight_workspace(int B, int C) {
   return vig::dwconv3x3_wgrad_workspace(B, C);
 }
 
+int vig_dwconv3x3_bwd(const void* x, const void* dy, const void* pre, const float* weight, void* dx, float* dw_db,
+                      void* workspace, size_t workspace_bytes, int B, int h, int w, int C, int io_dtype, void* stream) {
+  if (!x || !dy || (!dx && !dw_db) || (dx && !weight) || B <= 0 || h <= 0 || w <= 0 || C <= 0 || dx == dy || (dx && dx == x))
+    return VIG_EINVAL;
+  if (!aligned16(x, dy, pre, dx, dw_db, workspace)) return VIG_EINVAL;
+  if (!dtype_ok(io_dtype) || (C % 8) != 0) return VIG_ENOTSUP;
+  if (dw_db && (!workspace || workspace_bytes < vig::dwconv3x3_wgrad_workspace(B, C))) return VIG_ENOSPC;
+  return vig::launch_dwconv3x3_bwd(x, dy, pre, weight, dx, dw_db, workspace, B, h, w, C, io_dtype, (hipStream_t)stream);
+}
+
 int vig_dwconv3x3_bwd_weight(const void* x, const void* dy, float* dw_db, void* workspace, size_t workspace_bytes,
                              int B, int h, int w, int C, int io_dtype, void* stream) {
-  if (!x || !dy || !dw_db || B <= 0 || h <= 0 || w <= 0 || C <= 0) return VIG_EINVAL;
-  if (!aligned16(x, dy, dw_db, workspace)) return VIG_EINVAL;
-  if (!dtype_ok(io_dtype) || (C % 8) != 0) return VIG_ENOTSUP;
-  if (!workspace || workspace_bytes < vig::dwconv3x3_wgrad_workspace(B, C)) return VIG_ENOSPC;
-  return vig::launch_dwconv3x3_wgrad(x, dy, dw_db, workspace, B, h, w, C, io_dtype, (hipStream_t)stream);
+  if (!dw_db) return VIG_EINVAL;
+  return vig_dwconv3x3_bwd(x, dy, nullptr, nullptr, nullptr, dw_db, workspace, workspace_bytes, B, h, w, C, io_dtype, stream);
 }
 
 int vig_locality_gate_fwd(const void* o, const float* weight, void* y, int B, int H, int h, int w, int Dv,
@@ -458,29 +511,48 @@ size_t vig_locality_blend_bwd_workspace(int B, int L, int Dv) {
   return vig::locality_blend_bwd_workspace(B, L, Dv);
 }
 
-int vig_locality_blend_bwd(const void* o, const void* local, const void* g_lin, const float* w_g, const float* w_l,
-                           const void* dy, void* d_o, void* d_local, void* d_glin, float* dw, void* workspace,
-                           size_t workspace_bytes, int B, int H, int L, int Dv, long long g_row_stride, float eps,
-                           int silu_out, int io_dtype, void* stream) {
+int vig_locality_blend_bwd_strided(const void* o, const void* local, const void* g_lin, const float* w_g, const float* w_l,
+                                   const void* dy, void* d_o, void* d_local, void* d_glin, float* dw, void* workspace,
+                                   size_t workspace_bytes, int B, int H, int L, int Dv, long long g_row_stride,
+                                   long long d_glin_row_stride, float eps, int silu_out, int io_dtype, void* stream) {
   if (!o || !local || !g_lin || !w_g || !w_l || !dy || !d_o || !d_local || !d_glin || !dw || B <= 0 || H <= 0 ||
       L <= 0)
     return VIG_EINVAL;
   if (!aligned16(o, local, w_g, w_l, dy, d_o, d_local, d_glin, dw, workspace)) return VIG_EINVAL;
   if (!dtype_ok(io_dtype) || !(Dv == 32 || Dv == 64)) return VIG_ENOTSUP;
-  const long long ldg = g_row_stride > 0 ? g_row_stride : (long long)H * Dv;
-  if (ldg < (long long)H * Dv || !strided_rows_ok(g_lin, ldg, io_dtype)) return VIG_EINVAL;
+  const long long row = (long long)H * Dv;
+  const long long ldg = g_row_stride > 0 ? g_row_stride : row, ldd = d_glin_row_stride > 0 ? d_glin_row_stride : row;
+  if (ldg < row || !strided_rows_ok(g_lin, ldg, io_dtype) || ldd < row || !strided_rows_ok(d_glin, ldd, io_dtype))
+    return VIG_EINVAL;
   if (!workspace || workspace_bytes < vig::locality_blend_bwd_workspace(B, L, Dv)) return VIG_ENOSPC;
   return vig::launch_locality_blend_bwd(o, local, g_lin, w_g, w_l, dy, d_o, d_local, d_glin, dw, workspace, B, H, L,
-                                        Dv, ldg, eps, silu_out, io_dtype, (hipStream_t)stream);
+                                        Dv, ldg, ldd, eps, silu_out, io_dtype, (hipStream_t)stream);
+}
+
+int vig_locality_blend_bwd(const void* o, const void* local, const void* g_lin, const float* w_g, const float* w_l,
+                           const void* dy, void* d_o, void* d_local, void* d_glin, float* dw, void* workspace,
+                           size_t workspace_bytes, int B, int H, int L, int Dv, long long g_row_stride, float eps,
+                           int silu_out, int io_dtype, void* stream) {
+  return vig_locality_blend_bwd_strided(o, local, g_lin, w_g, w_l, dy, d_o, d_local, d_glin, dw, workspace, workspace_bytes,
+                                        B, H, L, Dv, g_row_stride, 0, eps, silu_out, io_dtype, stream);
+}
+
+int vig_rmsnorm_mixed_fwd(const void* x, const void* residual, const float* weight, void* y, void* residual_out,
+                          long long rows, int C, float eps, int round_sum, int x_dtype, int sum_dtype, int y_dtype,
+                          void* stream) {
+  if (!x || !weight || !y || rows <= 0 || C <= 0 || rows > 0x7fffffffLL) return VIG_EINVAL;
+  if (!aligned16(x, residual, weight, y, residual_out)) return VIG_EINVAL;
+  if (!dtype_ok(x_dtype) || !dtype_ok(sum_dtype) || !dtype_ok(y_dtype) || (C % 8) != 0 || C > 4096 ||
+      !vig::rmsnorm_types_ok(x_dtype, sum_dtype, y_dtype))
+    return VIG_ENOTSUP;
+  return vig::launch_rmsnorm(x, residual, weight, y, residual_out, (int)rows, C, eps, round_sum, x_dtype, sum_dtype, y_dtype,
+                             (hipStream_t)stream);
 }
 
 int vig_rmsnorm_fwd(const void* x, const void* residual, const float* weight, void* y, void* residual_out,
                     long long rows, int C, float eps, int round_sum, int io_dtype, void* stream) {
-  if (!x || !weight || !y || rows <= 0 || C <= 0 || rows > 0x7fffffffLL) return VIG_EINVAL;
-  if (!aligned16(x, residual, weight, y, residual_out)) return VIG_EINVAL;
-  if (!dtype_ok(io_dtype) || (C % 8) != 0 || C > 4096) return VIG_ENOTSUP;
-  return vig::launch_rmsnorm(x, residual, weight, y, residual_out, (int)rows, C, eps, round_sum, io_dtype,
-                             (hipStream_t)stream);
+  return vig_rmsnorm_mixed_fwd(x, residual, weight, y, residual_out, rows, C, eps, round_sum, io_dtype, io_dtype, io_dtype,
+                               stream);
 }
 
 int vig_layernorm_fwd(const void* x, const float* weight, const float* bias, void* y, long long rows, int C,
@@ -554,15 +626,24 @@ size_t vig_rmsnorm_bwd_workspace(long long rows, int C) {
   return vig::rmsnorm_bwd_workspace(rows, C);
 }
 
+int vig_rmsnorm_mixed_bwd(const void* sum, const float* weight, const void* dy, const void* d_sum, void* ds, void* dx,
+                          float* dweight, void* workspace, size_t workspace_bytes, long long rows, int C, float eps,
+                          int sum_dtype, int y_dtype, void* stream) {
+  if (!sum || !weight || !dy || !ds || rows <= 0 || C <= 0 || rows > 0x7fffffffLL) return VIG_EINVAL;
+  if (!aligned16(sum, weight, dy, d_sum, ds, dx, dweight, workspace)) return VIG_EINVAL;
+  if (!dtype_ok(sum_dtype) || !dtype_ok(y_dtype) || (C % 8) != 0 || C > 1024 ||
+      !vig::rmsnorm_types_ok(sum_dtype, sum_dtype, y_dtype))
+    return VIG_ENOTSUP;
+  if (dweight && (!workspace || workspace_bytes < vig::rmsnorm_bwd_workspace(rows, C))) return VIG_ENOSPC;
+  return vig::launch_rmsnorm_bwd(sum, weight, dy, d_sum, ds, dx, dweight, workspace, rows, C, eps, sum_dtype, y_dtype,
+                                 (hipStream_t)stream);
+}
+
 int vig_rmsnorm_bwd(const void* sum, const float* weight, const void* dy, const void* d_sum, void* ds, float* dweight,
                     void* workspace, size_t workspace_bytes, long long rows, int C, float eps, int io_dtype,
                     void* stream) {
-  if (!sum || !weight || !dy || !ds || rows <= 0 || C <= 0 || rows > 0x7fffffffLL) return VIG_EINVAL;
-  if (!aligned16(sum, weight, dy, d_sum, ds, dweight, workspace)) return VIG_EINVAL;
-  if (!dtype_ok(io_dtype) || (C % 8) != 0 || C > 1024) return VIG_ENOTSUP;
-  if (dweight && (!workspace || workspace_bytes < vig::rmsnorm_bwd_workspace(rows, C))) return VIG_ENOSPC;
-  return vig::launch_rmsnorm_bwd(sum, weight, dy, d_sum, ds, dweight, workspace, rows, C, eps, io_dtype,
-                                 (hipStream_t)stream);
+  return vig_rmsnorm_mixed_bwd(sum, weight, dy, d_sum, ds, nullptr, dweight, workspace, workspace_bytes, rows, C, eps, io_dtype,
+                               io_dtype, stream);
 }
 
 static bool bwd_shape_ok(int Dk, int Dv) {

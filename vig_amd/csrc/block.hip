@@ -66,10 +66,10 @@ __device__ __forceinline__ float wave_sum(float v) {
 // round_sum: s is first rounded to the storage type (the value an explicit add would have stored) and the
 // rounded value is normalised.
 // ---------------------------------------------------------------------------
-template <typename T, int NV>
-__global__ __launch_bounds__(256) void rmsnorm_kernel(const T* __restrict__ x, const T* __restrict__ residual,
-                                                      const float* __restrict__ weight, T* __restrict__ y,
-                                                      T* __restrict__ residual_out, int rows, int C, float eps,
+template <typename TX, typename TS, typename TY, int NV>
+__global__ __launch_bounds__(256) void rmsnorm_kernel(const TX* __restrict__ x, const TS* __restrict__ residual,
+                                                      const float* __restrict__ weight, TY* __restrict__ y,
+                                                      TS* __restrict__ residual_out, int rows, int C, float eps,
                                                       int round_sum) {
   const int lane = threadIdx.x & 63;
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -82,18 +82,18 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const T* __restrict__ x, c
   for (int i = 0; i < NV; ++i) {
     const int v = lane + 64 * i;
     if (v < nvec) {
-      Oct<T>::load(x + base + 8 * v, s[i]);
+      Oct<TX>::load(x + base + 8 * v, s[i]);
       if (residual) {
         float rr[8];
-        Oct<T>::load(residual + base + 8 * v, rr);
+        Oct<TS>::load(residual + base + 8 * v, rr);
 #pragma unroll
         for (int j = 0; j < 8; ++j) s[i][j] += rr[j];
       }
       if (round_sum) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) s[i][j] = Oct<T>::round(s[i][j]);
+        for (int j = 0; j < 8; ++j) s[i][j] = Oct<TS>::round(s[i][j]);
       }
-      if (residual_out) Oct<T>::store(residual_out + base + 8 * v, s[i]);
+      if (residual_out) Oct<TS>::store(residual_out + base + 8 * v, s[i]);
 #pragma unroll
       for (int j = 0; j < 8; ++j) ss = __builtin_fmaf(s[i][j], s[i][j], ss);
     }
@@ -108,19 +108,19 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const T* __restrict__ x, c
       Oct<float>::load(weight + 8 * v, w);
 #pragma unroll
       for (int j = 0; j < 8; ++j) s[i][j] = s[i][j] * rstd * w[j];
-      Oct<T>::store(y + base + 8 * v, s[i]);
+      Oct<TY>::store(y + base + 8 * v, s[i]);
     }
   }
 }
 
-template <typename T>
+template <typename TX, typename TS, typename TY>
 static int launch_rmsnorm_t(const void* x, const void* residual, const float* weight, void* y, void* residual_out,
                             int rows, int C, float eps, int round_sum, hipStream_t stream) {
   const dim3 grid((rows + 3) / 4), block(256);
   const int nvec = C / 8;
-#define VIG_RMS_CASE(NV)                                                                                          \
-  hipLaunchKernelGGL((rmsnorm_kernel<T, NV>), grid, block, 0, stream, (const T*)x, (const T*)residual, weight, \
-                     (T*)y, (T*)residual_out, rows, C, eps, round_sum)
+#define VIG_RMS_CASE(NV)                                                                                             \
+  hipLaunchKernelGGL((rmsnorm_kernel<TX, TS, TY, NV>), grid, block, 0, stream, (const TX*)x, (const TS*)residual, weight, \
+                     (TY*)y, (TS*)residual_out, rows, C, eps, round_sum)
   if (nvec <= 64) VIG_RMS_CASE(1);
   else if (nvec <= 128) VIG_RMS_CASE(2);
   else if (nvec <= 256) VIG_RMS_CASE(4);
@@ -129,11 +129,20 @@ static int launch_rmsnorm_t(const void* x, const void* residual, const float* we
   return hipGetLastError() == hipSuccess ? 0 : -5;
 }
 
+// one type throughout, or an fp32 stream (residual, sum) with a bf16 result and an x of either type: a bf16 branch meeting
+// the fp32 residual under autocast, where separate casts read and wrote [rows, C] two more times
+bool rmsnorm_types_ok(int x_dtype, int sum_dtype, int y_dtype) {
+  return (x_dtype == sum_dtype && y_dtype == sum_dtype) || (sum_dtype == 0 && y_dtype == 1);
+}
+
 int launch_rmsnorm(const void* x, const void* residual, const float* weight, void* y, void* residual_out, int rows,
-                   int C, float eps, int round_sum, int io_dtype, hipStream_t stream) {
-  if (C % 8 != 0 || C > 4096) return -95;
-  return io_dtype == 1 ? launch_rmsnorm_t<uint16_t>(x, residual, weight, y, residual_out, rows, C, eps, round_sum, stream)
-                       : launch_rmsnorm_t<float>(x, residual, weight, y, residual_out, rows, C, eps, round_sum, stream);
+                   int C, float eps, int round_sum, int x_dtype, int sum_dtype, int y_dtype, hipStream_t stream) {
+  if (C % 8 != 0 || C > 4096 || !rmsnorm_types_ok(x_dtype, sum_dtype, y_dtype)) return -95;
+  auto fn = sum_dtype == 1 ? launch_rmsnorm_t<uint16_t, uint16_t, uint16_t>
+            : y_dtype == 0 ? launch_rmsnorm_t<float, float, float>
+            : x_dtype == 1 ? launch_rmsnorm_t<uint16_t, float, uint16_t>
+                           : launch_rmsnorm_t<float, float, uint16_t>;
+  return fn(x, residual, weight, y, residual_out, rows, C, eps, round_sum, stream);
 }
 
 // ---------------------------------------------------------------------------
@@ -309,12 +318,11 @@ int launch_split_heads(const void* qkv, void* q, void* k, void* v, int B, int L,
   return hipGetLastError() == hipSuccess ? 0 : -5;
 }
 
-// the backward of the split: dq, dk, dv (head-major) -> d_qkv [B, L, H*(2*Dk+Dv)] packed rows
+// the backward of the split: dq, dk, dv (head-major) -> d_qkv [B, L, H*(2*Dk+Dv)], rows ld elements apart
 int launch_merge_heads(const void* dq, const void* dk, const void* dv, void* dqkv, int B, int L, int H, int Dk, int Dv,
-                       int io_dtype, hipStream_t stream) {
+                       long long ld, int io_dtype, hipStream_t stream) {
   if (Dk % 8 != 0 || Dv % 8 != 0 || B > 65535) return -95;
   const dim3 grid((L + 31) / 32, B), block(256);
-  const long long ld = (long long)H * (2 * Dk + Dv);
   if (io_dtype == 1)
     hipLaunchKernelGGL((split_heads_kernel<uint16_t, true>), grid, block, 0, stream, (uint16_t*)dqkv,
                        (const uint16_t*)dq, (const uint16_t*)dk, (const uint16_t*)dv, B, L, H, Dk, Dv, ld);
@@ -400,7 +408,8 @@ int launch_swiglu_bwd(const void* in, const void* dy, void* din, long long rows,
 // Backward of the residual-add + RMS norm.  s is the stored sum that was normalised (x, or x + residual as the
 // forward returned it), dy the gradient of y, d_sum (optional) the gradient arriving at the returned sum:
 //   r = rsqrt(mean(s^2) + eps),  g = dy * weight,
-//   ds = r * (g - s * r^2 * mean(g * s)) + d_sum         (the gradient of x and of the residual alike)
+//   ds = r * (g - s * r^2 * mean(g * s)) + d_sum         (the gradient of x and of the residual alike; dx, optional, gets
+//   the same value in the type of a narrower x)
 //   dweight[c] = sum over rows of dy[c] * s[c] * r
 // One wave per row, sixteen waves a workgroup (eight a SIMD: the kernel is a chain of load -> reduce -> store per
 // row, and only occupancy hides it); workgroups walk the rows a grid apart and keep their share of dweight in
@@ -409,11 +418,11 @@ int launch_swiglu_bwd(const void* in, const void* dy, void* din, long long rows,
 // ---------------------------------------------------------------------------
 constexpr int kRmsBwdWaves = 16;
 
-template <typename T, int NV>
-__global__ __launch_bounds__(64 * kRmsBwdWaves) void rmsnorm_bwd_kernel(const T* __restrict__ s_in, const float* __restrict__ weight,
-                                                          const T* __restrict__ dy, const T* __restrict__ d_sum,
-                                                          T* __restrict__ ds, float* __restrict__ partials, int rows,
-                                                          int C, float eps) {
+template <typename TS, typename TY, typename TX, int NV>
+__global__ __launch_bounds__(64 * kRmsBwdWaves) void rmsnorm_bwd_kernel(const TS* __restrict__ s_in, const float* __restrict__ weight,
+                                                          const TY* __restrict__ dy, const TS* __restrict__ d_sum,
+                                                          TS* __restrict__ ds, TX* __restrict__ dx, float* __restrict__ partials,
+                                                          int rows, int C, float eps) {
   extern __shared__ __align__(16) float red[];  // [kRmsBwdWaves][C], only with partials
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int nvec = C >> 3;
@@ -436,8 +445,8 @@ __global__ __launch_bounds__(64 * kRmsBwdWaves) void rmsnorm_bwd_kernel(const T*
 #pragma unroll
       for (int j = 0; j < 8; ++j) s[i][j] = 0.f, g[i][j] = 0.f;
       if (v < nvec) {
-        Oct<T>::load(s_in + base + 8 * v, s[i]);
-        Oct<T>::load(dy + base + 8 * v, g[i]);
+        Oct<TS>::load(s_in + base + 8 * v, s[i]);
+        Oct<TY>::load(dy + base + 8 * v, g[i]);
       }
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
@@ -461,11 +470,12 @@ __global__ __launch_bounds__(64 * kRmsBwdWaves) void rmsnorm_bwd_kernel(const T*
         }
         if (d_sum) {
           float e[8];
-          Oct<T>::load(d_sum + base + 8 * v, e);
+          Oct<TS>::load(d_sum + base + 8 * v, e);
 #pragma unroll
           for (int j = 0; j < 8; ++j) o[j] += e[j];
         }
-        Oct<T>::store(ds + base + 8 * v, o);
+        Oct<TS>::store(ds + base + 8 * v, o);
+        if (dx) Oct<TX>::store(dx + base + 8 * v, o);
       }
     }
   }
@@ -521,16 +531,16 @@ static int rmsnorm_bwd_grid(long long rows) {
 
 size_t rmsnorm_bwd_workspace(long long rows, int C) { return (size_t)rmsnorm_bwd_grid(rows) * C * sizeof(float); }
 
-template <typename T>
-static int launch_rmsnorm_bwd_t(const void* s, const float* weight, const void* dy, const void* d_sum, void* ds,
+template <typename TS, typename TY, typename TX>
+static int launch_rmsnorm_bwd_t(const void* s, const float* weight, const void* dy, const void* d_sum, void* ds, void* dx,
                                 float* dweight, float* partials, int rows, int C, float eps, hipStream_t stream) {
   const int grid = rmsnorm_bwd_grid(rows);
   const size_t lds = dweight ? (size_t)kRmsBwdWaves * C * sizeof(float) : 0;
   float* part = dweight ? partials : nullptr;
   const int nvec = C / 8;
-#define VIG_RMSB_CASE(NV)                                                                                     \
-  hipLaunchKernelGGL((rmsnorm_bwd_kernel<T, NV>), dim3(grid), dim3(64 * kRmsBwdWaves), lds, stream, (const T*)s, \
-                     weight, (const T*)dy, (const T*)d_sum, (T*)ds, part, rows, C, eps)
+#define VIG_RMSB_CASE(NV)                                                                                            \
+  hipLaunchKernelGGL((rmsnorm_bwd_kernel<TS, TY, TX, NV>), dim3(grid), dim3(64 * kRmsBwdWaves), lds, stream, (const TS*)s, \
+                     weight, (const TY*)dy, (const TS*)d_sum, (TS*)ds, (TX*)dx, part, rows, C, eps)
   if (nvec <= 64) VIG_RMSB_CASE(1);
   else VIG_RMSB_CASE(2);
 #undef VIG_RMSB_CASE
@@ -541,13 +551,14 @@ static int launch_rmsnorm_bwd_t(const void* s, const float* weight, const void* 
   return 0;
 }
 
-int launch_rmsnorm_bwd(const void* s, const float* weight, const void* dy, const void* d_sum, void* ds, float* dweight,
-                       void* workspace, long long rows, int C, float eps, int io_dtype, hipStream_t stream) {
+int launch_rmsnorm_bwd(const void* s, const float* weight, const void* dy, const void* d_sum, void* ds, void* dx, float* dweight,
+                       void* workspace, long long rows, int C, float eps, int sum_dtype, int y_dtype, hipStream_t stream) {
   if (C % 8 != 0 || C > 1024 || rows > 0x7fffffffLL - 8192) return -95;  // 16 rows of C floats in 64 KB of LDS
-  return io_dtype == 1 ? launch_rmsnorm_bwd_t<uint16_t>(s, weight, dy, d_sum, ds, dweight, (float*)workspace,
-                                                        (int)rows, C, eps, stream)
-                       : launch_rmsnorm_bwd_t<float>(s, weight, dy, d_sum, ds, dweight, (float*)workspace, (int)rows,
-                                                     C, eps, stream);
+  if (!rmsnorm_types_ok(sum_dtype, sum_dtype, y_dtype)) return -95;
+  auto fn = sum_dtype == 1 ? launch_rmsnorm_bwd_t<uint16_t, uint16_t, uint16_t>
+            : y_dtype == 0 ? launch_rmsnorm_bwd_t<float, float, float>
+                           : launch_rmsnorm_bwd_t<float, uint16_t, uint16_t>;
+  return fn(s, weight, dy, d_sum, ds, dx, dweight, (float*)workspace, (int)rows, C, eps, stream);
 }
 
 // ---------------------------------------------------------------------------
@@ -611,6 +622,57 @@ int launch_pad_channels(const void* src, void* dst, long long rows, int src_c, i
   const long long nvec = rows * (dst_c / 8);
   hipLaunchKernelGGL(pad_channels_kernel, dim3((unsigned)((nvec + 255) / 256)), dim3(256), 0, stream,
                      (const uint16_t*)src, (uint16_t*)dst, nvec, src_c / 8, dst_c / 8);
+  return hipGetLastError() == hipSuccess ? 0 : -5;
+}
+
+// ---------------------------------------------------------------------------
+// Several small tensors converted or transposed in one launch (blockIdx.y = tensor): the weights of a block in the layout and
+// type its kernels read, laid out per training step because the optimiser has just changed them.  A null source writes zeros;
+// cols > 0: the source is [n / cols, cols] and the destination its transpose.
+// ---------------------------------------------------------------------------
+struct CastJobs {
+  const void* src[kMaxCastJobs];
+  void* dst[kMaxCastJobs];
+  int n[kMaxCastJobs], cols[kMaxCastJobs];
+  int src_bf16, dst_bf16;  // one bit a job
+};
+
+__global__ __launch_bounds__(256) void cast_many_kernel(CastJobs jobs) {
+  const int j = blockIdx.y;
+  const int n = jobs.n[j], cols = jobs.cols[j];
+  const bool sb = jobs.src_bf16 >> j & 1, db = jobs.dst_bf16 >> j & 1;
+  auto get = [&](int i) {
+    if (!jobs.src[j]) return 0.f;
+    return sb ? bf16_to_f32(((const uint16_t*)jobs.src[j])[i]) : ((const float*)jobs.src[j])[i];
+  };
+  if (cols == 0 && n % 4 == 0 && jobs.src[j] && !sb && db) {  // fp32 -> bf16, whole quads
+    const f32x4_t* src = (const f32x4_t*)jobs.src[j];
+    u32x2_t* dst = (u32x2_t*)jobs.dst[j];
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < n / 4; i += gridDim.x * 256) {
+      const f32x4_t x = src[i];
+      dst[i] = u32x2_t{pack_bf16x2(x[0], x[1]), pack_bf16x2(x[2], x[3])};
+    }
+    return;
+  }
+  for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
+    const int rows = cols ? n / cols : 0;
+    const float x = get(cols ? i % rows * cols + i / rows : i);
+    if (db) ((uint16_t*)jobs.dst[j])[i] = f32_to_bf16(x);
+    else ((float*)jobs.dst[j])[i] = x;
+  }
+}
+
+int launch_cast_many(const void* const* src, void* const* dst, const int* n, const int* cols, const int* src_dtype,
+                     const int* dst_dtype, int count, hipStream_t stream) {
+  CastJobs jobs{};
+  int largest = 0;
+  for (int j = 0; j < count; ++j) {
+    jobs.src[j] = src[j], jobs.dst[j] = dst[j], jobs.n[j] = n[j], jobs.cols[j] = cols[j];
+    jobs.src_bf16 |= (src_dtype[j] == 1) << j, jobs.dst_bf16 |= (dst_dtype[j] == 1) << j;
+    if (n[j] > largest) largest = n[j];
+  }
+  const int blocks = (largest + 1023) / 1024;
+  hipLaunchKernelGGL(cast_many_kernel, dim3(blocks < 512 ? blocks : 512, count), dim3(256), 0, stream, jobs);
   return hipGetLastError() == hipSuccess ? 0 : -5;
 }
 

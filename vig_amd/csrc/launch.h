@@ -77,6 +77,9 @@ int launch_gla_backward_f32(const void* q, const void* k, const void* v, const v
 // chains the slots of a state pass in place (gla_segment_scan_kernel, no state in or out)
 int launch_gla_segment_scan(float* slots, int nseq, int nseg, int ndir, int ng, hipStream_t stream);
 
+// Most tensors one launch_cast_many takes.
+constexpr int kMaxCastJobs = 16;
+
 // fp32-arithmetic token-recurrent path (any supported dtype combination).
 int launch_gla_recurrent(const GlaArgs& a);
 size_t gla_recurrent_workspace(int B, int H, int L, int Dv, int io_dtype);

@@ -1,0 +1,481 @@
+// The recorded (training) forward of a ViG block as two autograd nodes over the C ABI: the token mixer with the norm in front
+// of it, and the SwiGLU MLP with its own (classification/models/vig.py:530-618; training branch :354-426).  Two, because
+// stochastic depth acts on each branch between them.
+//
+// As separate modules the block was bound by what lay between its products: under autocast the fp32 residual stream was cast
+// and re-cast around every norm, the four projections of the same rows ran as four products forward and their input gradients
+// as four products and three additions, each weight gradient was rounded to bf16 and cast back, and bias gradients were
+// reductions of their own.  Here
+//   - the norms read and write the stream in its type and the branch in the products' type (vig_rmsnorm_mixed_fwd / _bwd);
+//   - q/k/v, gate and low-rank projection are one product over stacked weights (rows padded to a multiple of 128: 35 instead of
+//     62 us at 25088 x 384), their gradients gather into one matrix whose rows the kernels write in place, and one product
+//     returns the input gradient, added to the local branch's in fp32 before it is rounded;
+//   - weight and bias gradients leave vig_linear_bwd_weight as fp32, one launch for the three stacked layers;
+//   - the up-projection of the gates and its input gradient run inside the gate kernels (bf16), and the depthwise
+//     convolution's three gradients are one kernel.
+// ViG-S, B 128 at 224 px under bf16 autocast, forward and backward on one MI355X: 23.9 -> 13.7 ms.
+#include <ATen/autocast_mode.h>
+
+#include "host_calls.h"
+
+namespace vig_host {
+
+namespace {
+
+constexpr int64_t kRank = 16;  // the low-rank width the gate kernels are built for
+
+struct Mix {
+  int64_t B, L, C, h, w, H, Dk, Dv, rows, K, V, n0, n1, n2, nz;  // n0 | n1 | n2: ends of the q/k/v, gate and low-rank columns
+  bool act, out_act, bf16;
+  double norm_eps, eps, inv_norm, clamp;
+  std::vector<int64_t> ints() const { return {B, L, h, w, H, Dk, Dv, act, out_act, bf16}; }
+  std::vector<double> reals() const { return {norm_eps, eps, inv_norm, clamp}; }
+  static Mix from(const std::vector<int64_t>& i, const std::vector<double>& d) {
+    Mix m;
+    m.B = i[0], m.L = i[1], m.h = i[2], m.w = i[3], m.H = i[4], m.Dk = i[5], m.Dv = i[6], m.act = i[7], m.out_act = i[8],
+    m.bf16 = i[9];
+    m.norm_eps = d[0], m.eps = d[1], m.inv_norm = d[2], m.clamp = d[3];
+    m.rows = m.B * m.L, m.K = m.H * m.Dk, m.V = m.H * m.Dv, m.C = m.V;
+    m.n0 = 2 * m.K + m.V, m.n1 = m.n0 + m.V, m.n2 = m.n1 + kRank, m.nz = (m.n2 + 127) / 128 * 128;
+    return m;
+  }
+  at::ScalarType type() const { return bf16 ? at::kBFloat16 : at::kFloat; }
+  int code() const { return bf16 ? VIG_BF16 : VIG_F32; }
+};
+
+at::ScalarType scalar_type(bool bf16) { return bf16 ? at::kBFloat16 : at::kFloat; }
+
+void* at_elem(const Tensor& t, int64_t i) { return static_cast<char*>(t.data_ptr()) + i * t.element_size(); }
+float* fptr(const Tensor& t) { return static_cast<float*>(t.data_ptr()); }
+
+// The weights of a step in one buffer, filled by one launch: pieces of whole 16-byte units, addressed by offset.
+struct Packer {
+  int64_t size = 0;
+  std::vector<const void*> src;
+  std::vector<int64_t> off;
+  std::vector<int> n, cols, sd;
+  int64_t add(const Tensor& t, int64_t count, int64_t transposed_cols = 0, bool align = true) {
+    if (align) size = (size + 63) / 64 * 64;
+    const int64_t at = size;
+    src.push_back(t.defined() ? t.data_ptr() : nullptr);
+    sd.push_back(t.defined() ? dtype_code(t) : VIG_F32);
+    off.push_back(at), n.push_back((int)count), cols.push_back((int)transposed_cols);
+    size += count;
+    return at;
+  }
+  Tensor run(at::ScalarType type, const Tensor& like) const {
+    if (src.empty()) return Tensor();
+    Tensor buf = at::empty({size}, like.options().dtype(type));
+    std::vector<void*> dst;
+    for (auto o : off) dst.push_back(at_elem(buf, o));
+    const std::vector<int> dd(src.size(), dtype_code(buf));
+    check_rc(vig_cast_many(src.data(), dst.data(), n.data(), cols.data(), sd.data(), dd.data(), (int)src.size(), stream_of(like)),
+             "vig_cast_many");
+    return buf;
+  }
+};
+
+Tensor matrix(const Tensor& buf, int64_t off, int64_t rows, int64_t cols) {
+  return buf.as_strided({rows, cols}, {cols, 1}, buf.storage_offset() + off);
+}
+
+// dy^T x in fp32 (and the column sums of dy); rows of both may lie in wider matrices
+Tensor weight_grad(const Tensor& dy, const Tensor& x, Tensor* bias_grad) {
+  const int64_t T = dy.size(0), N = dy.size(1), K = x.size(1);
+  if (dy.scalar_type() == at::kFloat) {
+    if (bias_grad) *bias_grad = dy.sum(0);
+    return at::mm(dy.t(), x);
+  }
+  Tensor dw = at::empty({N, K}, dy.options().dtype(at::kFloat));
+  if (bias_grad) *bias_grad = at::empty({N}, dw.options());
+  const size_t need = vig_linear_bwd_weight_workspace(T, (int)N, (int)K);
+  Tensor ws = bytes_like(need, dy);
+  check_rc(vig_linear_bwd_weight(dy.data_ptr(), dy.stride(0), x.data_ptr(), x.stride(0), fptr(dw),
+                                 bias_grad ? fptr(*bias_grad) : nullptr, ws.data_ptr(), need, T, (int)N, (int)K, stream_of(dy)),
+           "vig_linear_bwd_weight");
+  return dw;
+}
+
+// residual-add + RMS norm: (y, sum); without a residual the sum is x itself
+std::pair<Tensor, Tensor> norm_fwd(const Tensor& x, const Tensor& residual, const float* weight, double eps, at::ScalarType type) {
+  const int64_t C = x.size(-1), rows = x.numel() / C;
+  Tensor y = at::empty(x.sizes(), x.options().dtype(type));
+  const Tensor sum = residual.defined() ? at::empty(x.sizes(), residual.options()) : x;
+  check_rc(vig_rmsnorm_mixed_fwd(x.data_ptr(), residual.defined() ? residual.data_ptr() : nullptr, weight, y.data_ptr(),
+                                 residual.defined() ? sum.data_ptr() : nullptr, rows, (int)C, (float)eps, residual.defined(),
+                                 dtype_code(x), dtype_code(sum), dtype_code(y), stream_of(x)),
+           "vig_rmsnorm_mixed_fwd");
+  return {y, sum};
+}
+
+// its backward: (gradient of the residual, gradient of the branch, gradient of the weight or none)
+struct NormGrads {
+  Tensor residual, branch, weight;
+};
+NormGrads norm_bwd(const Tensor& sum, const float* weight, const Tensor& dy, Tensor d_sum, bool narrow_branch, bool need_weight,
+                   double eps) {
+  const int64_t C = sum.size(-1), rows = sum.numel() / C;
+  if (d_sum.defined() && !plain(d_sum, sum.device())) d_sum = d_sum.clone(at::MemoryFormat::Contiguous);
+  NormGrads g;
+  g.residual = at::empty_like(sum);
+  g.branch = narrow_branch ? at::empty(sum.sizes(), dy.options()) : g.residual;
+  size_t need = 0;
+  Tensor ws;
+  if (need_weight) {
+    g.weight = at::empty({C}, sum.options().dtype(at::kFloat));
+    need = vig_rmsnorm_bwd_workspace(rows, (int)C);
+    ws = bytes_like(need, sum);
+  }
+  check_rc(vig_rmsnorm_mixed_bwd(sum.data_ptr(), weight, dy.data_ptr(), d_sum.defined() ? d_sum.data_ptr() : nullptr,
+                                 g.residual.data_ptr(), narrow_branch ? g.branch.data_ptr() : nullptr,
+                                 need_weight ? fptr(g.weight) : nullptr, need ? ws.data_ptr() : nullptr, need, rows, (int)C,
+                                 (float)eps, dtype_code(sum), dtype_code(dy), stream_of(sum)),
+           "vig_rmsnorm_mixed_bwd");
+  return g;
+}
+
+// a gradient that arrives in the right type, as rows; zeros where none arrived
+Tensor grad_rows(const Tensor& g, int64_t rows, int64_t cols, const Tensor& like, at::ScalarType type) {
+  if (!g.defined()) return at::zeros({rows, cols}, like.options().dtype(type));
+  Tensor r = g.contiguous();
+  if (reinterpret_cast<uintptr_t>(r.data_ptr()) % 16) r = r.clone();
+  return r.view({rows, cols});
+}
+Tensor like_param(const Tensor& grad, const Tensor& param_like, at::IntArrayRef shape) {
+  return grad.defined() ? grad.view(shape).to(param_like.scalar_type()) : grad;
+}
+
+// The kernels take what they are given in the type they are given: casts are explicit here.
+struct NoAutocast {
+  c10::impl::ExcludeDispatchKeyGuard guard{c10::DispatchKeySet({c10::DispatchKey::AutocastCUDA})};
+};
+
+enum MixParam { kNormW, kConvW, kConvB, kQkvW, kGateW, kGateB, kLowW, kUpW, kUpB, kGNorm, kLNorm, kOutW, kMixParams };
+
+struct MixNode : torch::autograd::Function<MixNode> {
+  static variable_list forward(AutogradContext* ctx, const Tensor& branch, const std::optional<Tensor>& residual_arg,
+                               const Tensor& norm_w, const Tensor& conv_w, const std::optional<Tensor>& conv_b,
+                               const Tensor& qkv_w, const Tensor& gate_w, const Tensor& gate_b, const Tensor& low_w,
+                               const Tensor& up_w, const Tensor& up_b, const Tensor& g_norm, const Tensor& l_norm,
+                               const Tensor& out_w, const Mix& m) {
+    const NoAutocast no_autocast;
+    const c10::DeviceGuard guard(branch.device());
+    void* const stream = stream_of(branch);
+    const auto type = m.type();
+    const auto opts = branch.options().dtype(type);
+    const Tensor residual = residual_arg ? *residual_arg : Tensor();
+    const bool same = qkv_w.scalar_type() == type, wide = qkv_w.scalar_type() == at::kFloat;
+    // ---- this step's weights: stacked input projection and its bias, and what the kernels read in another type ----
+    Packer p, f;
+    const int64_t w_off = p.add(qkv_w, m.n0 * m.C);
+    p.add(gate_w, m.V * m.C, 0, false), p.add(low_w, kRank * m.C, 0, false);
+    if (m.nz > m.n2) p.add(Tensor(), (m.nz - m.n2) * m.C, 0, false);
+    const int64_t b_off = p.add(Tensor(), m.n0);
+    p.add(gate_b, m.V, 0, false), p.add(Tensor(), m.nz - m.n1, 0, false);
+    int64_t out_off = 0, up_off = 0, upb_off = 0, upt_off = 0;
+    if (!same) out_off = p.add(out_w, m.C * m.V), up_off = p.add(up_w, 2 * m.K * kRank), upb_off = p.add(up_b, 2 * m.K);
+    if (m.bf16) upt_off = p.add(up_w, 2 * m.K * kRank, kRank);
+    const Tensor packed = p.run(type, branch);
+    Tensor small;  // the kernels' fp32 weights
+    int64_t f_off[5] = {0, 0, 0, 0, 0};
+    if (!wide) {
+      f_off[0] = f.add(norm_w, m.C), f_off[1] = f.add(conv_w, m.C * 9), f_off[2] = f.add(g_norm, m.Dv), f_off[3] = f.add(l_norm, m.Dv);
+      if (conv_b) f_off[4] = f.add(*conv_b, m.C);
+      small = f.run(at::kFloat, branch);
+    }
+    auto f32 = [&](const Tensor& t, int i) { return wide ? fptr(t) : fptr(small) + f_off[i]; };
+    const Tensor w_in = matrix(packed, w_off, m.nz, m.C);
+    const Tensor b_in = packed.as_strided({m.nz}, {1}, b_off);
+    const Tensor w_out = same ? out_w : matrix(packed, out_off, m.C, m.V);
+
+    auto [y, sum] = norm_fwd(branch, residual, f32(norm_w, 0), m.norm_eps, type);
+    Tensor xs = at::empty({m.B, m.L, m.C}, opts), pre;
+    if (m.act) pre = at::empty_like(xs);
+    check_rc(vig_dwconv3x3_fwd_pre(y.data_ptr(), f32(conv_w, 1), conv_b ? f32(*conv_b, 4) : nullptr, xs.data_ptr(),
+                                   m.act ? pre.data_ptr() : nullptr, (int)m.B, (int)m.h, (int)m.w, (int)m.C, m.act, m.code(), stream),
+             "vig_dwconv3x3_fwd_pre");
+    const Tensor z = at::addmm(b_in, xs.view({m.rows, m.C}), w_in.t());
+    Tensor q = at::empty({m.B, m.H, m.L, m.Dk}, opts), k = at::empty_like(q), v = at::empty({m.B, m.H, m.L, m.Dv}, opts);
+    check_rc(vig_split_heads_fwd(z.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), (int)m.B, (int)m.L, (int)m.H, (int)m.Dk,
+                                 (int)m.Dv, m.nz, m.code(), stream),
+             "vig_split_heads_fwd");
+    Tensor gates = at::empty({2 * m.B, m.H, m.L, m.Dk}, opts), gate_lin;
+    if (m.bf16) {
+      check_rc(vig_dirgate_lowrank_fwd(at_elem(z, m.n1), m.nz, same ? up_w.data_ptr() : at_elem(packed, up_off),
+                                       same ? up_b.data_ptr() : at_elem(packed, upb_off), gates.data_ptr(), (int)m.B, (int)m.L,
+                                       (int)m.H, (int)m.Dk, (int)kRank, (float)m.inv_norm, (float)m.clamp, VIG_BF16, VIG_BF16, stream),
+               "vig_dirgate_lowrank_fwd");
+    } else {
+      gate_lin = at::addmm(up_b, z.narrow(1, m.n1, kRank), up_w.t());
+      check_rc(vig_dirgate_fwd(gate_lin.data_ptr(), gates.data_ptr(), (int)m.B, (int)m.L, (int)m.H, (int)m.Dk, (float)m.inv_norm,
+                               (float)m.clamp, VIG_F32, VIG_F32, stream),
+               "vig_dirgate_fwd");
+    }
+    Call c{(int)m.B, (int)m.H, (int)m.L, (int)m.Dk, (int)m.Dv, m.code(), m.code(), (float)std::pow((double)m.Dk, -0.5), 0.5f};
+    Tensor o;
+    check_rc(run_forward(q, k, v, gates, Tensor(), true, kDefault, c, o), "vig_gla_bidir_fwd");
+    Tensor blend = at::empty_like(xs);
+    check_rc(vig_locality_blend_fwd(o.data_ptr(), xs.data_ptr(), at_elem(z, m.n0), f32(g_norm, 2), f32(l_norm, 3), blend.data_ptr(),
+                                    (int)m.B, (int)m.H, (int)m.L, (int)m.Dv, m.nz, (float)m.eps, m.out_act, m.code(), stream),
+             "vig_locality_blend_fwd");
+    const Tensor a = at::mm(blend.view({m.rows, m.V}), w_out.t()).view({m.B, m.L, m.C});
+
+    ctx->set_materialize_grads(false);
+    ctx->save_for_backward({sum, y, xs, pre, z, q, k, v, gates, gate_lin, o, blend, packed, small, norm_w, conv_w, g_norm, l_norm,
+                            out_w, up_w, up_b});
+    ctx->saved_data["ints"] = m.ints();
+    ctx->saved_data["reals"] = m.reals();
+    ctx->saved_data["at"] = std::vector<int64_t>{w_off, out_off, up_off, upb_off, upt_off, f_off[0], f_off[1], f_off[2], f_off[3],
+                                                 branch.scalar_type() != sum.scalar_type(), conv_b.has_value(), residual.defined()};
+    return {a, sum};
+  }
+
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const at::NoGradGuard no_grad;
+    const NoAutocast no_autocast;
+    const auto s = ctx->get_saved_variables();
+    const Tensor &sum = s[0], &y = s[1], &xs = s[2], &pre = s[3], &z = s[4], &q = s[5], &k = s[6], &v = s[7], &gates = s[8],
+                 &gate_lin = s[9], &o = s[10], &blend = s[11], &packed = s[12], &small = s[13], &norm_w = s[14], &conv_w = s[15],
+                 &g_norm = s[16], &l_norm = s[17], &out_w = s[18], &up_w = s[19], &up_b = s[20];
+    const Mix m = Mix::from(ctx->saved_data["ints"].toIntVector(), ctx->saved_data["reals"].toDoubleVector());
+    const auto off = ctx->saved_data["at"].toIntVector();
+    const c10::DeviceGuard guard(sum.device());
+    void* const stream = stream_of(sum);
+    const auto type = m.type();
+    const bool same = out_w.scalar_type() == type, wide = out_w.scalar_type() == at::kFloat;
+    auto f32 = [&](const Tensor& t, int i) { return wide ? fptr(t) : fptr(small) + off[5 + i]; };
+    const Tensor w_in = matrix(packed, off[0], m.n2, m.C);
+    const Tensor w_out = same ? out_w : matrix(packed, off[1], m.C, m.V);
+    // (an argument that was absent has no edge)
+    auto wants = [&](int param) { return ctx->needs_input_grad(param + (off[11] ? 2 : 1) - (param > kConvB && !off[10])); };
+    auto opts = xs.options();
+    variable_list out(2 + kMixParams + 1);
+
+    const Tensor da = grad_rows(grads[0], m.rows, m.C, xs, type);
+    if (wants(kOutW)) out[2 + kOutW] = like_param(weight_grad(da, blend.view({m.rows, m.V}), nullptr), out_w, {m.C, m.V});
+    const Tensor d_blend = at::mm(da, w_out);
+    // gradients of the stacked projection's columns, written in place by the three kernels that produce them
+    Tensor dz = at::empty({m.rows, m.nz}, opts);
+    Tensor d_o = at::empty_like(o), d_xs = at::empty({m.rows, m.C}, opts);
+    Tensor d_norms = at::empty({2, m.Dv}, opts.dtype(at::kFloat));
+    {
+      const size_t need = vig_locality_blend_bwd_workspace((int)m.B, (int)m.L, (int)m.Dv);
+      Tensor ws = bytes_like(need, sum);
+      check_rc(vig_locality_blend_bwd_strided(o.data_ptr(), xs.data_ptr(), at_elem(z, m.n0), f32(g_norm, 2), f32(l_norm, 3),
+                                              d_blend.data_ptr(), d_o.data_ptr(), d_xs.data_ptr(), at_elem(dz, m.n0), fptr(d_norms),
+                                              ws.data_ptr(), need, (int)m.B, (int)m.H, (int)m.L, (int)m.Dv, m.nz, m.nz,
+                                              (float)m.eps, m.out_act, m.code(), stream),
+               "vig_locality_blend_bwd_strided");
+    }
+    if (wants(kGNorm)) out[2 + kGNorm] = like_param(d_norms.select(0, 0), g_norm, {m.Dv});
+    if (wants(kLNorm)) out[2 + kLNorm] = like_param(d_norms.select(0, 1), l_norm, {m.Dv});
+    Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v), dg = at::empty_like(gates);
+    {
+      const size_t need = vig_gla_bidir_bwd_workspace_for((int)m.B, (int)m.H, (int)m.L, (int)m.Dk, (int)m.Dv, m.code(), m.code(), 1);
+      Tensor ws = bytes_like(need, sum);
+      const int64_t half = gates.numel() / 2;
+      check_rc(vig_gla_bidir_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), gates.data_ptr(), at_elem(gates, half), d_o.data_ptr(),
+                                 dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dg.data_ptr(), at_elem(dg, half), ws.data_ptr(), need,
+                                 (int)m.B, (int)m.H, (int)m.L, (int)m.Dk, (int)m.Dv, (float)std::pow((double)m.Dk, -0.5), 0.5f,
+                                 m.code(), m.code(), stream),
+               "vig_gla_bidir_bwd");
+    }
+    check_rc(vig_split_heads_bwd_strided(dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dz.data_ptr(), m.nz, (int)m.B, (int)m.L,
+                                         (int)m.H, (int)m.Dk, (int)m.Dv, m.code(), stream),
+             "vig_split_heads_bwd_strided");
+    Tensor dx = at::empty({m.rows, 2 * m.K}, opts);
+    if (m.bf16) {
+      check_rc(vig_dirgate_lowrank_bwd(at_elem(z, m.n1), m.nz, same ? up_w.data_ptr() : at_elem(packed, off[2]),
+                                       at_elem(packed, off[4]), same ? up_b.data_ptr() : at_elem(packed, off[3]), dg.data_ptr(),
+                                       dx.data_ptr(), at_elem(dz, m.n1), m.nz, (int)m.B, (int)m.L, (int)m.H, (int)m.Dk,
+                                       (int)kRank, (float)m.inv_norm, (float)m.clamp, VIG_BF16, VIG_BF16, stream),
+               "vig_dirgate_lowrank_bwd");
+    } else {
+      check_rc(vig_dirgate_bwd(gate_lin.data_ptr(), dg.data_ptr(), dx.data_ptr(), (int)m.B, (int)m.L, (int)m.H, (int)m.Dk,
+                               (float)m.inv_norm, (float)m.clamp, VIG_F32, VIG_F32, stream),
+               "vig_dirgate_bwd");
+      Tensor d_low = dz.narrow(1, m.n1, kRank);
+      at::mm_out(d_low, dx, up_w);
+    }
+    if (wants(kUpW) || wants(kUpB)) {
+      Tensor db;
+      const Tensor dw = weight_grad(dx, z.narrow(1, m.n1, kRank), &db);
+      out[2 + kUpW] = like_param(dw, up_w, {2 * m.K, kRank});
+      out[2 + kUpB] = like_param(db, up_w, {2 * m.K});
+    }
+    const Tensor dzs = dz.narrow(1, 0, m.n2);
+    if (wants(kQkvW) || wants(kGateW) || wants(kGateB) || wants(kLowW)) {
+      Tensor db;
+      const bool bias = wants(kGateB), bf = m.bf16;
+      const Tensor dw = weight_grad(dzs, xs.view({m.rows, m.C}), bias && bf ? &db : nullptr);
+      out[2 + kQkvW] = like_param(dw.narrow(0, 0, m.n0), out_w, {m.n0, m.C});
+      out[2 + kGateW] = like_param(dw.narrow(0, m.n0, m.V), out_w, {m.V, m.C});
+      out[2 + kLowW] = like_param(dw.narrow(0, m.n1, kRank), out_w, {kRank, m.C});
+      if (bias) out[2 + kGateB] = like_param(bf ? db.narrow(0, m.n0, m.V) : dz.narrow(1, m.n0, m.V).sum(0), out_w, {m.V});
+    }
+    at::addmm_out(d_xs, d_xs, dzs, w_in);
+    const bool conv_grads = wants(kConvW) || (off[10] && wants(kConvB));
+    Tensor d_y = at::empty({m.B, m.L, m.C}, opts), dw_db, ws;
+    size_t need = 0;
+    if (conv_grads) {
+      dw_db = at::empty({m.C * 10}, opts.dtype(at::kFloat));
+      need = vig_dwconv3x3_bwd_weight_workspace((int)m.B, (int)m.C);
+      ws = bytes_like(need, sum);
+    }
+    check_rc(vig_dwconv3x3_bwd(y.data_ptr(), d_xs.data_ptr(), m.act ? pre.data_ptr() : nullptr, f32(conv_w, 1), d_y.data_ptr(),
+                               conv_grads ? fptr(dw_db) : nullptr, need ? ws.data_ptr() : nullptr, need, (int)m.B, (int)m.h,
+                               (int)m.w, (int)m.C, m.code(), stream),
+             "vig_dwconv3x3_bwd");
+    if (wants(kConvW)) out[2 + kConvW] = like_param(dw_db.narrow(0, 0, m.C * 9), conv_w, conv_w.sizes());
+    if (off[10] && wants(kConvB)) out[2 + kConvB] = like_param(dw_db.narrow(0, m.C * 9, m.C), conv_w, {m.C});
+    const auto g = norm_bwd(sum, f32(norm_w, 0), d_y, grads[1], off[9], wants(kNormW), m.norm_eps);
+    out[0] = g.branch;
+    if (off[11]) out[1] = g.residual;
+    out[2 + kNormW] = like_param(g.weight, norm_w, {m.C});
+    return out;
+  }
+};
+
+struct MlpNode : torch::autograd::Function<MlpNode> {
+  static variable_list forward(AutogradContext* ctx, const Tensor& branch, const Tensor& residual, const Tensor& norm_w,
+                               const Tensor& gate_w, const Tensor& down_w, double eps, bool bf16) {
+    const NoAutocast no_autocast;
+    const c10::DeviceGuard guard(branch.device());
+    const auto type = scalar_type(bf16);
+    const int64_t C = branch.size(-1), rows = branch.numel() / C, I = down_w.size(1);
+    const bool same = gate_w.scalar_type() == type, wide = gate_w.scalar_type() == at::kFloat;
+    Packer p, f;
+    int64_t gate_off = 0, down_off = 0;
+    if (!same) gate_off = p.add(gate_w, 2 * I * C), down_off = p.add(down_w, C * I);
+    const Tensor packed = p.run(type, branch);
+    Tensor small;
+    if (!wide) f.add(norm_w, C), small = f.run(at::kFloat, branch);
+    const Tensor wg = same ? gate_w : matrix(packed, gate_off, 2 * I, C), wd = same ? down_w : matrix(packed, down_off, C, I);
+    auto [y, sum] = norm_fwd(branch, residual, wide ? fptr(norm_w) : fptr(small), eps, type);
+    const Tensor z = at::mm(y.view({rows, C}), wg.t());
+    Tensor prod = at::empty({rows, I}, z.options());
+    check_rc(vig_swiglu_fwd(z.data_ptr(), prod.data_ptr(), rows, (int)I, dtype_code(z), stream_of(z)), "vig_swiglu_fwd");
+    const Tensor out = at::mm(prod, wd.t()).view(branch.sizes());
+    ctx->set_materialize_grads(false);
+    ctx->save_for_backward({sum, y, z, prod, packed, small, norm_w, gate_w, down_w});
+    ctx->saved_data["at"] = std::vector<int64_t>{gate_off, down_off, bf16, branch.scalar_type() != sum.scalar_type()};
+    ctx->saved_data["eps"] = eps;
+    return {out, sum};
+  }
+
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const at::NoGradGuard no_grad;
+    const NoAutocast no_autocast;
+    const auto s = ctx->get_saved_variables();
+    const Tensor &sum = s[0], &y = s[1], &z = s[2], &prod = s[3], &packed = s[4], &small = s[5], &norm_w = s[6], &gate_w = s[7],
+                 &down_w = s[8];
+    const auto off = ctx->saved_data["at"].toIntVector();
+    const c10::DeviceGuard guard(sum.device());
+    const auto type = scalar_type(off[2]);
+    const int64_t C = sum.size(-1), rows = sum.numel() / C, I = prod.size(1);
+    const bool same = gate_w.scalar_type() == type, wide = gate_w.scalar_type() == at::kFloat;
+    const Tensor wg = same ? gate_w : matrix(packed, off[0], 2 * I, C), wd = same ? down_w : matrix(packed, off[1], C, I);
+    variable_list out(7);
+    const Tensor d_out = grad_rows(grads[0], rows, C, y, type);
+    if (ctx->needs_input_grad(4)) out[4] = like_param(weight_grad(d_out, prod, nullptr), down_w, {C, I});
+    const Tensor d_prod = at::mm(d_out, wd);
+    Tensor dz = at::empty_like(z);
+    check_rc(vig_swiglu_bwd(z.data_ptr(), d_prod.data_ptr(), dz.data_ptr(), rows, (int)I, dtype_code(z), stream_of(z)),
+             "vig_swiglu_bwd");
+    if (ctx->needs_input_grad(3)) out[3] = like_param(weight_grad(dz, y.view({rows, C}), nullptr), gate_w, {2 * I, C});
+    const Tensor d_y = at::mm(dz, wg);
+    const auto g = norm_bwd(sum, wide ? fptr(norm_w) : fptr(small), d_y, grads[1], off[3], ctx->needs_input_grad(2),
+                            ctx->saved_data["eps"].toDouble());
+    out[0] = g.branch, out[1] = g.residual;
+    out[2] = like_param(g.weight, norm_w, {C});
+    return out;
+  }
+};
+
+// Whether branch and residual are rows the nodes take and the weights share one usable type; sets the products' type.
+bool stream_ok(const Tensor& branch, const Tensor& residual, const Tensor* const* params, int n, bool& bf16) {
+  if (!branch.defined() || !branch.is_cuda() || branch.dim() != 3 || branch.numel() == 0) return false;
+  const auto dev = branch.device();
+  if (!plain(branch, dev) || dtype_code(branch) < 0) return false;
+  if (residual.defined() && (!plain(residual, dev) || residual.sizes() != branch.sizes() || dtype_code(residual) < 0)) return false;
+  const auto sum = residual.defined() ? residual.scalar_type() : branch.scalar_type();
+  const auto param = params[0]->scalar_type();
+  at::ScalarType type = param;
+  if (at::autocast::is_autocast_enabled(at::kCUDA)) {
+    type = at::autocast::get_autocast_dtype(at::kCUDA);
+    if (type != at::kBFloat16) return false;
+  }
+  if ((type != at::kBFloat16 && type != at::kFloat) || (param != type && param != at::kFloat)) return false;
+  bf16 = type == at::kBFloat16;
+  for (int i = 0; i < n; ++i)
+    if (params[i] && (!plain(*params[i], dev) || params[i]->scalar_type() != param)) return false;
+  const int64_t C = branch.size(2), rows = branch.size(0) * branch.size(1);
+  if (C % 8 || C > 1024 || rows > 0x7fffffff - 8192) return false;
+  return (branch.scalar_type() == type && sum == type) || (sum == at::kFloat && bf16);
+}
+
+bool is_shape(const Tensor& t, std::initializer_list<int64_t> shape) { return t.sizes() == at::IntArrayRef(shape); }
+
+}  // namespace
+
+// block_mix(branch, residual or None, norm, conv weight, conv bias or None, qkv, gate weight, gate bias, low-rank, up weight,
+// up bias, global norm, local norm, out, h, w, heads, key width, value width, conv SiLU, output SiLU, norm eps, eps,
+// gate normaliser, clamp or None) -> (mixer output, residual stream), or None for a call the node does not take
+PyObject* block_mix(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK_TYPE(n == 25, "block_mix takes 25 arguments");
+  for (int i = 0; i < 14; ++i)
+    if (!is_tensor(a[i]) && !((i == 1 || i == 4) && a[i] == Py_None)) Py_RETURN_NONE;
+  const Tensor& branch = THPVariable_Unpack(a[0]);
+  const Tensor residual = tensor_arg(a[1]), conv_b = tensor_arg(a[4]);
+  const Tensor* params[kMixParams];
+  for (int i = 0; i < kMixParams; ++i) params[i] = i == kConvB ? (conv_b.defined() ? &conv_b : nullptr) : &THPVariable_Unpack(a[2 + i]);
+  bool bf16;
+  if (!stream_ok(branch, residual, params, kMixParams, bf16)) Py_RETURN_NONE;
+  const int64_t h = PyLong_AsLong(a[14]), w = PyLong_AsLong(a[15]), H = PyLong_AsLong(a[16]), Dk = PyLong_AsLong(a[17]),
+                Dv = PyLong_AsLong(a[18]);
+  const bool act = PyObject_IsTrue(a[19]), out_act = PyObject_IsTrue(a[20]);
+  const double norm_eps = PyFloat_AsDouble(a[21]), eps = PyFloat_AsDouble(a[22]), normalizer = PyFloat_AsDouble(a[23]);
+  const double clamp = a[24] == Py_None ? std::nan("") : PyFloat_AsDouble(a[24]);
+  if (PyErr_Occurred()) return nullptr;
+  const int64_t B = branch.size(0), L = branch.size(1), C = branch.size(2);
+  if (H <= 0 || h <= 0 || w <= 0 || (Dk != 16 && Dk != 32 && Dk != 64) || (Dv != 32 && Dv != 64)) Py_RETURN_NONE;
+  const Mix m = Mix::from({B, L, h, w, H, Dk, Dv, act, out_act, bf16}, {norm_eps, eps, 1.0 / normalizer, clamp});
+  // (a grid row with its halo has to fit the stencil's tile three times)
+  if (h * w != L || C != m.V || B > 65535 || (w + 2) * 64 * (bf16 ? 2 : 4) * 3 > 48 * 1024) Py_RETURN_NONE;
+  if (!is_shape(*params[kNormW], {C}) || params[kConvW]->numel() != C * 9 || (conv_b.defined() && !is_shape(conv_b, {C})) ||
+      !is_shape(*params[kQkvW], {m.n0, C}) || !is_shape(*params[kGateW], {m.V, C}) || !is_shape(*params[kGateB], {m.V}) ||
+      !is_shape(*params[kLowW], {kRank, C}) || !is_shape(*params[kUpW], {2 * m.K, kRank}) || !is_shape(*params[kUpB], {2 * m.K}) ||
+      !is_shape(*params[kGNorm], {Dv}) || !is_shape(*params[kLNorm], {Dv}) || !is_shape(*params[kOutW], {C, m.V}))
+    Py_RETURN_NONE;
+  const auto opt = [](const Tensor& t) { return t.defined() ? std::optional<Tensor>(t) : std::nullopt; };
+  auto r = MixNode::apply(branch, opt(residual), *params[kNormW], *params[kConvW], opt(conv_b), *params[kQkvW], *params[kGateW],
+                          *params[kGateB], *params[kLowW], *params[kUpW], *params[kUpB], *params[kGNorm], *params[kLNorm],
+                          *params[kOutW], m);
+  return Py_BuildValue("(NN)", THPVariable_Wrap(r[0]), THPVariable_Wrap(r[1]));
+  END_HANDLE_TH_ERRORS
+}
+
+// block_mlp(branch, residual, norm, gate and up weight, down weight, eps) -> (MLP output, residual stream), or None
+PyObject* block_mlp(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK_TYPE(n == 6, "block_mlp takes 6 arguments");
+  for (int i = 0; i < 5; ++i)
+    if (!is_tensor(a[i])) Py_RETURN_NONE;
+  const Tensor &branch = THPVariable_Unpack(a[0]), &residual = THPVariable_Unpack(a[1]), &norm_w = THPVariable_Unpack(a[2]),
+               &gate_w = THPVariable_Unpack(a[3]), &down_w = THPVariable_Unpack(a[4]);
+  const Tensor* params[3] = {&norm_w, &gate_w, &down_w};
+  bool bf16;
+  const double eps = PyFloat_AsDouble(a[5]);
+  if (PyErr_Occurred()) return nullptr;
+  if (!stream_ok(branch, residual, params, 3, bf16)) Py_RETURN_NONE;
+  const int64_t C = branch.size(2);
+  if (down_w.dim() != 2 || down_w.size(0) != C) Py_RETURN_NONE;
+  const int64_t I = down_w.size(1);
+  if (I <= 0 || I % 8 || !is_shape(norm_w, {C}) || !is_shape(gate_w, {2 * I, C})) Py_RETURN_NONE;
+  auto r = MlpNode::apply(branch, residual, norm_w, gate_w, down_w, eps, bf16);
+  return Py_BuildValue("(NN)", THPVariable_Wrap(r[0]), THPVariable_Wrap(r[1]));
+  END_HANDLE_TH_ERRORS
+}
+
+}  // namespace vig_host

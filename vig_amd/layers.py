@@ -83,6 +83,12 @@ def _recording(module: nn.Module) -> bool:
     return module.training and torch.is_grad_enabled()
 
 
+def _plain(*modules: nn.Module) -> bool:
+    """True when nothing hangs on calling these modules by themselves: training mode and no hooks."""
+    return all(m.training and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks)
+               for m in modules)
+
+
 class RMSNorm(_CacheMixin, nn.Module):
     """x * rsqrt(mean(x^2) + eps) * weight, arithmetic in fp32 (fla/modules/rmsnorm.py:38-52,491-512).
 
@@ -417,7 +423,40 @@ class GLABlock(nn.Module):
         self.mlp_norm = RMSNorm(hidden_size, eps=eps)
         self.mlp = GLAMLP(hidden_size, intermediate_size=intermediate_size)
 
+    def _recorded(self, branch, residual, patch_resolution, token_position=None, **kwargs):
+        """The block as two autograd nodes (csrc/train_block.cpp), stochastic depth on each branch between them: (branch,
+        residual) in and out as forward_carry has them.  None for what the nodes do not take: submodules of other types,
+        with hooks or partly in evaluation mode, and the shapes and types they refuse; the modules then run one by one."""
+        calls = _ext.calls()
+        at, mlp = self.attn, self.mlp
+        if calls is None or type(at) is not GatedLinearAttention or type(mlp) is not GLAMLP or token_position is not None:
+            return None
+        conv, up = at.in_proj[0], at.gk_proj
+        linears = (at.qkv_proj, at.g_proj, at.o_proj, up[0], up[1], mlp.gate_proj, mlp.down_proj)
+        if not (all(type(m) is nn.Linear for m in linears) and type(conv) is nn.Conv2d
+                and _plain(at, mlp, self.attn_norm, self.mlp_norm, at.g_norm, at.l_norm, at.in_proj, conv, at.in_proj[1], up,
+                           *linears)):
+            return None
+        h, w = patch_resolution
+        mixed = calls.block_mix(branch.contiguous(), residual, self.attn_norm.weight, conv.weight, conv.bias, at.qkv_proj.weight,
+                                at.g_proj.weight, at.g_proj.bias, up[0].weight, up[1].weight, up[1].bias, at.g_norm.weight,
+                                at.l_norm.weight, at.o_proj.weight, h, w, at.num_heads, at.head_qk_dim, at.head_v_dim,
+                                at.use_act_in_conv, at.use_out_act, self.attn_norm.eps, at.layernorm_eps,
+                                at.gate_logit_normalizer, at.clamp_min)
+        if mixed is None:
+            return None
+        branch, residual = self.drop_path(mixed[0]), mixed[1]
+        out = calls.block_mlp(branch, residual, self.mlp_norm.weight, mlp.gate_proj.weight, mlp.down_proj.weight,
+                              self.mlp_norm.eps)
+        if out is None:  # (a drop_path of another kind may return another type)
+            h, residual = self.mlp_norm(branch, residual, True)
+            out = mlp(h), residual
+        return self.drop_path(out[0]), out[1]
+
     def forward(self, hidden_states, **kwargs):
+        out = self._recorded(hidden_states, None, **kwargs) if _recording(self) else None
+        if out is not None:
+            return (out[1] + out[0],)
         residual = hidden_states
         h = self.attn(self.attn_norm(hidden_states), **kwargs)
         h, residual = self.mlp_norm(self.drop_path(h), residual, True)
@@ -426,6 +465,10 @@ class GLABlock(nn.Module):
     def forward_carry(self, branch, residual, **kwargs):
         """Same block, with the closing `residual + mlp(h)` of the previous block folded into this block's first norm:
         takes (branch, residual) with hidden_states = residual + branch and returns the next such pair."""
+        if _recording(self):
+            out = self._recorded(branch, residual, **kwargs)
+            if out is not None:
+                return out
         ext = _ext.load()
         at = self.attn
         if (ext is not None and not _recording(self) and not self.training and branch.is_cuda and branch.is_contiguous()
