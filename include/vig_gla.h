@@ -538,14 +538,45 @@ int vig_locality_blend_linear_fwd(const void* o, const void* local, const void* 
  *   OH = (H + 2*padding - KH) / stride + 1, OW likewise.
  *   w_packed [Cout, Cin*KH, 16] bf16: the kernel rows of the [Cout, Cin, KH, KW] weight, each padded with zeros to
  *   16 columns.
- * Built for the reference's stem: stride 8, padding 1, KW <= 16, Cin*KH = 27 (3 channels x 9 rows), W % 8 == 0,
- * W <= 248, Cout a multiple of 32 from 64 to 256; anything else returns VIG_ENOTSUP (use a library convolution).
+ * Built for the reference's stem: stride 8, padding 1, KW <= 16 (9 where W > 248), Cin*KH = 27 (3 channels x 9 rows),
+ * W % 8 == 0, Cout a multiple of 32 from 64 to 256; anything else returns VIG_ENOTSUP (use a library convolution).
  *
  * Replaces: the first nn.Conv2d of V2PatchEmbed (classification/models/vig.py:651) and the layout change a
  * channels-last convolution library needs in front of it.
  */
 int vig_patch_conv_fwd(const void* x, const void* w_packed, void* y, int B, int Cin, int H, int W, int KH, int KW,
                        int stride, int padding, int Cout, int io_dtype, void* stream);
+
+/*
+ * y [rows, N] = x [rows, K] . weight [N, K]^T (+ bias [N]), bf16, fp32 accumulation, the bias added before the one rounding;
+ * rows of x and y x_row_stride / y_row_stride elements apart.  N % 8 == 0, K % 32 == 0.
+ * vig_linear_preferred: whether this entry point is the better choice for a size (short of large products, where the BLAS
+ * library's kernels win).
+ *
+ * Replaces: the nn.Linear layers of the block and the classifier (classification/models/vig.py:286-312,492-497,826).
+ */
+int vig_linear_preferred(long long rows, int N, int K);
+int vig_linear_fwd(const void* x, long long x_row_stride, const void* weight, const void* bias, void* y, long long y_row_stride,
+                   long long rows, int N, int K, void* stream);
+
+/*
+ * 3x3 convolution, stride 2, padding 1, no bias, bf16 channels-last: x [B, H, W, Cin], weight [Cout, 3, 3, Cin] ->
+ * y [B, (H+1)/2, (W+1)/2, Cout].  Cin % 32 == 0, Cout % 8 == 0.
+ *
+ * Replaces: the second convolution of the v2 patch embedding (classification/models/vig.py:655).
+ */
+int vig_conv3x3s2_fwd(const void* x, const void* weight, void* y, int B, int H, int W, int Cin, int Cout, void* stream);
+
+/*
+ * The closing norm and the mean over tokens in one pass, bf16: out [B, C] = mean over l of the RMS-normalised
+ * (x + residual)[b, l, :], the sum and the normalised value rounded to bf16 as vig_rmsnorm_fwd with round_sum stores them, the mean in fp32.
+ * C % 8 == 0, C <= 1024.
+ *
+ * Replaces: classification/models/vig.py:896-905 (norm_f and the average pool).
+ */
+size_t vig_rmsnorm_pool_workspace(int B, int L, int C);
+int vig_rmsnorm_pool_fwd(const void* x, const void* residual, const float* weight, void* out, void* workspace,
+                         size_t workspace_bytes, int B, int L, int C, float eps, void* stream);
 
 /*
  * Weight and bias gradients of a linear layer over bf16 rows (what autograd derives for the nn.Linear layers of the block):

@@ -1,9 +1,9 @@
-"""The static check of test_isa_hazards.py over the fp32 and weight-gradient kernels."""
+"""The static check of test_isa_hazards.py over the fp32, weight-gradient and linear-layer kernels."""
 import pytest
 
 from .test_isa_hazards import test_no_early_read_of_matrix_results as check
 
 
-@pytest.mark.parametrize("src", ["gla_f32.hip", "gla_backward_f32.hip", "wgrad.hip"])
+@pytest.mark.parametrize("src", ["gla_f32.hip", "gla_backward_f32.hip", "wgrad.hip", "gemm.hip"])
 def test_no_early_read(src):
     check(src)

@@ -1,0 +1,108 @@
+"""The native evaluation forward (plan) and the kernels it adds, at the sizes where they can go wrong: against the module by
+module forward, float64 sums, and after the model has changed under the plan."""
+import pytest
+import torch
+
+import vig_amd
+from vig_amd import _ext, layers, ops
+
+from .util import announce
+
+pytestmark = pytest.mark.gpu
+
+
+def _randn(shape, seed):
+    return torch.randn(shape, generator=torch.Generator().manual_seed(seed)).bfloat16()
+
+
+def _close(got, want64, scale=None):
+    got = got.double().cpu()
+    scale = want64.abs().clamp_min(1.0) if scale is None else scale
+    assert ((got - want64).abs() / scale).max().item() <= 2.0 ** -7
+
+
+# few tiles, tiles past the line, a short contraction over many rows; ragged rows and columns, one stage and many
+@pytest.mark.parametrize("rows,N,K", [(1, 8, 32), (33, 40, 32), (196, 192, 512), (197, 1000, 384), (3200, 200, 224), (1568, 640, 192),
+                                      (33000, 520, 192), (66001, 264, 64)])
+def test_linear(rows, N, K):
+    announce(f"linear rows={rows} N={N} K={K}")
+    x, w, b = _randn((rows, K), 1), _randn((N, K), 2) * K ** -0.5, _randn((N,), 3)
+    assert _ext.calls() is not None
+    assert vig_amd._lib.load().vig_linear_preferred(rows, N, K)
+    for bias in (None, b):
+        got = ops.linear(x.cuda(), w.cuda(), bias.cuda() if bias is not None else None)
+        _close(got, torch.nn.functional.linear(x.double(), w.double(), bias.double() if bias is not None else None))
+
+
+@pytest.mark.parametrize("B,H,W,Cin,Cout", [(1, 1, 1, 32, 8), (2, 7, 9, 96, 192), (1, 28, 28, 384, 768), (9, 27, 28, 64, 200),
+                                            (40, 28, 28, 96, 192), (170, 28, 27, 32, 192)])
+def test_conv3x3s2(B, H, W, Cin, Cout):
+    announce(f"3x3 stride-2 convolution B{B} {H}x{W} {Cin}->{Cout}")
+    x, w = _randn((B, Cin, H, W), 4), _randn((Cout, Cin, 3, 3), 5) * (9 * Cin) ** -0.5
+    got = ops.conv3x3s2(x.cuda().contiguous(memory_format=torch.channels_last), w.cuda().contiguous(memory_format=torch.channels_last))
+    _close(got, torch.nn.functional.conv2d(x.double(), w.double(), None, 2, 1))
+
+
+@pytest.mark.parametrize("B,H,W,Cout", [(2, 24, 256, 96), (1, 40, 264, 64), (1, 17, 1024, 96), (2, 16, 504, 192)])
+def test_patch_conv_wide(B, H, W, Cout):
+    announce(f"patch_conv in pieces B{B} {H}x{W} Cout{Cout}")
+    x, w = _randn((B, 3, H, W), 6), _randn((Cout, 3, 9, 9), 7) * 0.1
+    assert ops.patch_conv_supported(x.cuda(), w.cuda(), 8, 1)
+    got = ops.patch_conv(x.cuda(), ops.pack_patch_conv_weight(w.cuda()), (9, 9), 8, 1)
+    _close(got.permute(0, 3, 1, 2), torch.nn.functional.conv2d(x.double(), w.double(), None, 8, 1))
+
+
+@pytest.mark.parametrize("B,L,C", [(1, 1, 8), (1, 196, 192), (3, 50, 384), (700, 17, 64), (2, 1025, 768)])
+def test_rmsnorm_pool(B, L, C):
+    announce(f"closing norm and mean B{B} L{L} C{C}")
+    x, r, w = _randn((B, L, C), 8), _randn((B, L, C), 9), torch.rand(C, generator=torch.Generator().manual_seed(10)) + 0.5
+    got = ops.rmsnorm_pool(x.cuda(), r.cuda(), w.cuda(), 1e-6)
+    want = ops.rmsnorm(x.cuda(), w.cuda(), 1e-6, residual=r.cuda(), round_sum=True).double().mean(1).cpu()
+    _close(got, want)
+
+
+@pytest.mark.parametrize("kw,side,B", [(dict(embed_dim=192, num_heads=3, use_out_act=True, use_act_in_conv=True), 224, 1),
+                                       (dict(embed_dim=384, num_heads=6), 160, 3),
+                                       (dict(embed_dim=128, num_heads=2, use_bias_in_dwconv=True, num_classes=10), 288, 2)])
+def test_native_forward(kw, side, B, monkeypatch):
+    announce(f"native evaluation forward {kw} side {side} B {B}")
+    torch.manual_seed(0)
+    model = layers.ViG(img_size=side, depth=2, drop_path_rate=0.0, **kw).cuda().bfloat16().eval()
+    x = torch.randn(B, 3, side, side, device="cuda").bfloat16()
+
+    def modules(m, x):
+        with monkeypatch.context() as mp:
+            mp.setattr(layers.ViG, "_planned", lambda self, x: None)
+            with torch.no_grad():
+                return m(x)
+
+    def same(m, x):
+        got, want = m(x), modules(m, x)
+        assert torch.equal(got, want), (got.float() - want.float()).abs().max().item()
+        return got
+
+    first = same(model, x)
+    assert model in layers._PLANS and not first.requires_grad
+    plan = layers._PLANS[model]
+    same(model, x * 0.5)
+    assert layers._PLANS[model] is plan  # (nothing changed: the plan stays)
+    with torch.no_grad():  # written in place, replaced, a setting changed, a whole layer replaced
+        model.blocks[1].mlp.down_proj.weight.mul_(1.5)
+    assert not torch.equal(same(model, x), first)
+    model.blocks[0].attn.o_proj.weight = torch.nn.Parameter(model.blocks[0].attn.o_proj.weight.detach() * 2)
+    same(model, x)
+    model.blocks[0].attn.clamp_min = -0.05
+    same(model, x)
+    model.head = torch.nn.Linear(model.embed_dim, 24).cuda().bfloat16()
+    assert same(model, x).shape == (B, 24)
+    seen = []
+    model.norm.register_forward_hook(lambda *a: seen.append(1))
+    same(model, x)
+    assert len(seen) == 2  # a hook sends the call through the modules
+    model.norm._forward_hooks.clear()
+    big = torch.randn(1, 3, side + 32, side + 32, device="cuda").bfloat16()  # another grid than the position table's
+    same(model, big)
+    model.train()
+    with torch.no_grad():
+        same(model, x)
+    same(model.eval().float(), x.float())

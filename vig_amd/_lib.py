@@ -67,6 +67,11 @@ SIGNATURES = {
                               [_c_size_t, _c_longlong, _c_int, _c_int, _c_void_p]),
     "vig_dirgate_lowrank_bwd": (_c_int, [_c_void_p, _c_longlong] + [_c_void_p] * 6 + [_c_longlong] + [_c_int] * 5 +
                                 [_c_float, _c_float, _c_int, _c_int, _c_void_p]),
+    "vig_linear_preferred": (_c_int, [_c_longlong, _c_int, _c_int]),
+    "vig_linear_fwd": (_c_int, [_c_void_p, _c_longlong] + [_c_void_p] * 3 + [_c_longlong, _c_longlong, _c_int, _c_int, _c_void_p]),
+    "vig_conv3x3s2_fwd": (_c_int, [_c_void_p] * 3 + [_c_int] * 5 + [_c_void_p]),
+    "vig_rmsnorm_pool_workspace": (_c_size_t, [_c_int] * 3),
+    "vig_rmsnorm_pool_fwd": (_c_int, [_c_void_p] * 5 + [_c_size_t] + [_c_int] * 3 + [_c_float, _c_void_p]),
     "vig_cast_many": (_c_int, [_c_void_p] * 6 + [_c_int, _c_void_p]),
     "vig_dwconv3x3_fwd_pre": (_c_int, [_c_void_p] * 5 + [_c_int] * 6 + [_c_void_p]),
     "vig_dwconv3x3_bwd": (_c_int, [_c_void_p] * 7 + [_c_size_t] + [_c_int] * 5 + [_c_void_p]),

@@ -15,7 +15,7 @@ OBJ = os.path.join(CSRC, "build")
 LIBDIR = os.path.join(HERE, "lib")
 LIB = os.path.join(LIBDIR, "libvig_gla.so")
 
-SOURCES = ["api.hip", "gla_recurrent.hip", "gla_mfma.hip", "gla_tiles.hip", "gla_f32.hip", "gates.hip", "block.hip", "gla_backward.hip", "gla_backward_mfma.hip", "gla_backward_f32.hip", "patch_conv.hip", "linear.hip", "wgrad.hip"]
+SOURCES = ["api.hip", "gla_recurrent.hip", "gla_mfma.hip", "gla_tiles.hip", "gla_f32.hip", "gates.hip", "block.hip", "gla_backward.hip", "gla_backward_mfma.hip", "gla_backward_f32.hip", "patch_conv.hip", "linear.hip", "wgrad.hip", "gemm.hip"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 # -packed-fp32-ops is switched off: the compiler must not form packed fp32 VALU ops.
@@ -82,7 +82,7 @@ def build_torch_extension(verbose: bool = True) -> str:
     (csrc/py_calls.cpp, csrc/train_block.cpp)."""
     with ThreadPoolExecutor(max_workers=2) as ex:
         jobs = [ex.submit(_host_library, ["torch_ext.cpp"], EXT, [], verbose),
-                ex.submit(_host_library, ["py_calls.cpp", "train_block.cpp"], CALLS, ["-ltorch_python"], verbose)]
+                ex.submit(_host_library, ["py_calls.cpp", "train_block.cpp", "model_forward.cpp"], CALLS, ["-ltorch_python"], verbose)]
         for j in jobs:
             j.result()
     return EXT

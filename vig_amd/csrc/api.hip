@@ -17,6 +17,13 @@ int launch_dwconv3x3_bwd(const void* x, const void* dy, const void* pre, const f
 int launch_dirgate_lowrank_bwd(const void* low, long long ld, const void* w1, const void* w1t, const void* b1,
                                const void* d_out, void* dx, void* d_low, long long ldd, int B, int L, int H, int Dk,
                                float inv_norm, float clamp_min, int out_dtype, hipStream_t stream);
+bool linear_preferred(long long M, int N, int K);
+int launch_linear(const void* x, long long ldx, const void* w, const void* bias, void* y, long long ldy, long long M, int N, int K,
+                  hipStream_t stream);
+int launch_conv3x3s2(const void* x, const void* w, void* y, int B, int H, int W, int Cin, int Cout, hipStream_t stream);
+size_t rmsnorm_pool_workspace(int B, int L, int C);
+int launch_rmsnorm_pool(const void* x, const void* residual, const float* weight, void* out, void* workspace, int B, int L, int C,
+                        float eps, hipStream_t stream);
 int launch_cast_many(const void* const* src, void* const* dst, const int* n, const int* cols, const int* src_dtype,
                      const int* dst_dtype, int count, hipStream_t stream);
 int launch_dwconv3x3(const void* x, const float* wt, const float* bias, void* y, void* pre, int B, int h, int w, int C,
@@ -437,6 +444,35 @@ int vig_dirgate_lowrank_bwd(const void* gk_low, long long low_row_stride, const 
     return VIG_EINVAL;
   return vig::launch_dirgate_lowrank_bwd(gk_low, ld, w_up, w_up_t, b_up, d_g, d_x, d_low, ldd, B, L, H, Dk, inv_normalizer,
                                          clamp_min, out_dtype, (hipStream_t)stream);
+}
+
+int vig_linear_preferred(long long rows, int N, int K) { return vig::linear_preferred(rows, N, K); }
+
+int vig_linear_fwd(const void* x, long long x_row_stride, const void* weight, const void* bias, void* y, long long y_row_stride,
+                   long long rows, int N, int K, void* stream) {
+  if (!x || !weight || !y || rows <= 0 || N <= 0 || K <= 0 || x_row_stride < K || y_row_stride < N) return VIG_EINVAL;
+  if (N % 8 || K % 32) return VIG_ENOTSUP;
+  if (!strided_rows_ok(x, x_row_stride, VIG_BF16) || !strided_rows_ok(y, y_row_stride, VIG_BF16) || !aligned16(weight, bias))
+    return VIG_EINVAL;
+  return vig::launch_linear(x, x_row_stride, weight, bias, y, y_row_stride, rows, N, K, (hipStream_t)stream);
+}
+
+int vig_conv3x3s2_fwd(const void* x, const void* weight, void* y, int B, int H, int W, int Cin, int Cout, void* stream) {
+  if (!x || !weight || !y || B <= 0 || H <= 0 || W <= 0 || Cin <= 0 || Cout <= 0) return VIG_EINVAL;
+  if (!aligned16(x, weight, y)) return VIG_EINVAL;
+  return vig::launch_conv3x3s2(x, weight, y, B, H, W, Cin, Cout, (hipStream_t)stream);
+}
+
+size_t vig_rmsnorm_pool_workspace(int B, int L, int C) {
+  return B <= 0 || L <= 0 || C <= 0 ? 0 : vig::rmsnorm_pool_workspace(B, L, C);
+}
+
+int vig_rmsnorm_pool_fwd(const void* x, const void* residual, const float* weight, void* out, void* workspace,
+                         size_t workspace_bytes, int B, int L, int C, float eps, void* stream) {
+  if (!x || !residual || !weight || !out || B <= 0 || L <= 0 || C <= 0) return VIG_EINVAL;
+  if (!aligned16(x, residual, weight, out, workspace)) return VIG_EINVAL;
+  if (!workspace || workspace_bytes < vig::rmsnorm_pool_workspace(B, L, C)) return VIG_ENOSPC;
+  return vig::launch_rmsnorm_pool(x, residual, weight, out, workspace, B, L, C, eps, (hipStream_t)stream);
 }
 
 int vig_cast_many(const void* const* src, void* const* dst, const int* n, const int* transposed_cols, const int* src_dtype,

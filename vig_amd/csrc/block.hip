@@ -146,6 +146,100 @@ int launch_rmsnorm(const void* x, const void* residual, const float* weight, voi
 }
 
 // ---------------------------------------------------------------------------
+// The model's closing norm and its mean over the tokens (residual-add + RMS norm as above, the result rounded to bf16 as it
+// would have been stored, then averaged in fp32): the normalised rows are not written.  A workgroup adds up a share of an image's tokens
+// (shares of 16 at least, about 1024 workgroups in all) and a second kernel adds the shares in order.
+// ---------------------------------------------------------------------------
+template <int NV>
+__global__ __launch_bounds__(256) void rmsnorm_pool_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ residual,
+                                                           const float* __restrict__ weight, float* __restrict__ partials,
+                                                           int L, int per, int C, float eps) {
+  extern __shared__ __align__(16) float red[];  // [4][C]
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int nvec = C >> 3;
+  float w[NV][8], sum[NV][8];
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int v = lane + 64 * i;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) sum[i][j] = 0.f, w[i][j] = 0.f;
+    if (v < nvec) Oct<float>::load(weight + 8 * v, w[i]);
+  }
+  const int l1 = min(L, ((int)blockIdx.x + 1) * per);
+  for (int l = blockIdx.x * per + wave; l < l1; l += 4) {
+    const size_t base = ((size_t)blockIdx.y * L + l) * C;
+    float s[NV][8], ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int v = lane + 64 * i;
+      if (v < nvec) {
+        float rr[8];
+        Oct<uint16_t>::load(x + base + 8 * v, s[i]);
+        Oct<uint16_t>::load(residual + base + 8 * v, rr);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          s[i][j] = Oct<uint16_t>::round(s[i][j] + rr[j]);
+          ss = __builtin_fmaf(s[i][j], s[i][j], ss);
+        }
+      }
+    }
+    const float rstd = 1.0f / sqrtf(wave_sum(ss) / (float)C + eps);
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+      if (lane + 64 * i < nvec) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) sum[i][j] += Oct<uint16_t>::round(s[i][j] * rstd * w[i][j]);
+      }
+  }
+#pragma unroll
+  for (int i = 0; i < NV; ++i)
+    if (lane + 64 * i < nvec) Oct<float>::store(red + wave * C + 8 * (lane + 64 * i), sum[i]);
+  __syncthreads();
+  float* out = partials + ((size_t)blockIdx.y * gridDim.x + blockIdx.x) * C;
+  for (int c = threadIdx.x; c < C; c += 256) out[c] = (red[c] + red[C + c]) + (red[2 * C + c] + red[3 * C + c]);
+}
+
+__global__ __launch_bounds__(256) void pool_finish_kernel(const float* __restrict__ partials, uint16_t* __restrict__ out, int shares,
+                                                          int C, float inv_l) {
+  __shared__ float red[4][64];  // 64 channels a workgroup, each wave a quarter of the shares
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int c = blockIdx.x * 64 + lane;
+  const float* p = partials + (size_t)blockIdx.y * shares * C + min(c, C - 1);
+  float acc = 0.f;
+#pragma unroll 8
+  for (int i = wave; i < shares; i += 4) acc += p[(size_t)i * C];
+  red[wave][lane] = acc;
+  __syncthreads();
+  if (wave == 0 && c < C)
+    out[(size_t)blockIdx.y * C + c] = f32_to_bf16(((red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane])) * inv_l);
+}
+
+static int pool_shares(int B, int L) {
+  const int most = (L + 15) / 16, want = 1024 / B;
+  const int shares = want < 1 ? 1 : want;
+  return shares < most ? shares : most;
+}
+size_t rmsnorm_pool_workspace(int B, int L, int C) { return (size_t)B * pool_shares(B, L) * C * sizeof(float); }
+
+int launch_rmsnorm_pool(const void* x, const void* residual, const float* weight, void* out, void* workspace, int B, int L, int C,
+                        float eps, hipStream_t stream) {
+  if (C % 8 != 0 || C > 1024 || B > 65535) return -95;
+  const int want = pool_shares(B, L), per = (L + want - 1) / want, shares = (L + per - 1) / per;
+  const size_t lds = (size_t)4 * C * sizeof(float);
+  float* partials = static_cast<float*>(workspace);
+  if (C <= 512)
+    hipLaunchKernelGGL(rmsnorm_pool_kernel<1>, dim3(shares, B), dim3(256), lds, stream, (const uint16_t*)x, (const uint16_t*)residual,
+                       weight, partials, L, per, C, eps);
+  else
+    hipLaunchKernelGGL(rmsnorm_pool_kernel<2>, dim3(shares, B), dim3(256), lds, stream, (const uint16_t*)x, (const uint16_t*)residual,
+                       weight, partials, L, per, C, eps);
+  if (hipGetLastError() != hipSuccess) return -5;
+  hipLaunchKernelGGL(pool_finish_kernel, dim3((C + 63) / 64, B), dim3(256), 0, stream, partials, (uint16_t*)out, shares, C,
+                     1.0f / (float)L);
+  return hipGetLastError() == hipSuccess ? 0 : -5;
+}
+
+// ---------------------------------------------------------------------------
 // LayerNorm over the last dimension with an optional SiLU behind it (the norms of the patch embedding, applied to
 // channels-last feature maps):  y = (x - mean) * rsqrt(var + eps) * weight + bias, var the biased variance; with
 // silu the normalised value is first rounded to the storage type (the separate activation reads stored values).

@@ -1,0 +1,322 @@
+// y = x . W^T (+ bias) for bf16 rows, fp32 accumulation: the projections of a block, the classifier, and the patch
+// embedding's 3x3 stride-2 convolution (its nine taps are nine row matrices: the contraction runs over (tap, channel) and a
+// row's address depends on the tap).
+#include "common.h"
+#include "launch.h"
+#include "mfma_tiles.h"
+
+namespace vig {
+
+namespace {
+
+struct GemmArgs {
+  const uint16_t *x, *w, *bias;
+  uint16_t* y;
+  long long ldx, ldy;
+  int M, N, K;
+  int gh, gw, oh, ow, cin;  // convolution: input and output grid, input channels
+};
+
+__device__ const u32x4_t kZeroRow = {0u, 0u, 0u, 0u};  // what a tap outside the grid reads
+
+// Matrix row i of a weight tile holds this channel of its 32: accumulator register 4g+m of lane (r, h) is matrix row 8g+4h+m, so
+// the lane ends with channels 16h .. 16h+15 of token r, 32 contiguous bytes.
+__device__ __forceinline__ int channel_of_row(int r) { return 16 * ((r >> 2) & 1) + 4 * (r >> 3) + (r & 3); }
+
+// The row of input pixels behind output row m, and whether tap t of it lies inside the grid.
+struct Pixel {
+  int base, y, x;  // element offset of the image, input coordinates of tap (0, 0)
+};
+__device__ __forceinline__ Pixel pixel_of(const GemmArgs& a, int m) {
+  const int per = a.oh * a.ow, b = m / per, p = m - b * per, oy = p / a.ow;
+  return {b * a.gh * a.gw, 2 * oy - 1, 2 * (p - oy * a.ow) - 1};
+}
+__device__ __forceinline__ const uint16_t* tap_row(const GemmArgs& a, const Pixel& p, int tap) {
+  const int ky = tap / 3, y = p.y + ky, x = p.x + tap - 3 * ky;
+  const bool in = y >= 0 && y < a.gh && x >= 0 && x < a.gw;
+  return in ? a.x + (size_t)(p.base + y * a.gw + x) * a.cin : nullptr;
+}
+
+constexpr int kStageK = 32;  // contraction elements per LDS stage: 64-byte row pieces
+
+// ---------------------------------------------------------------------------
+// Few rows: one workgroup per 32 x 32 tile of y, its waves splitting the contraction.  With a few hundred rows the chip
+// is nearly empty and a product lasts as long as its longest chain of loads and matrix instructions: each wave streams its
+// own stages through its own ring of LDS buffers (no barrier until the tiles are added), three in flight.  The stages go
+// through LDS because a wave's operand fragment is 32 rows of 32 bytes: fetched straight into registers that is 32 separate
+// requests an instruction (M 196, N 768, K 2048: 9.5 us).
+// ---------------------------------------------------------------------------
+constexpr int kFewBufs = 4;
+
+template <int NW, bool TAPS>
+__global__ __launch_bounds__(64 * NW) void gemm_few_kernel(GemmArgs a) {
+  extern __shared__ __align__(16) char smem[];  // [wave][buffer][4 KB: x rows, w rows], then the waves' tiles
+  const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int m0 = blockIdx.y * 32, n0 = blockIdx.x * 32;
+  const int stages = a.K / kStageK, mine = (stages - wave + NW - 1) / NW;  // wave w takes stages w, w + NW, ..
+  const int lrow = lane >> 2, place = lane & 3;
+  const uint16_t *xp[2], *wp[2];
+  Pixel px[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int row = 16 * i + lrow, unit = place ^ ((row >> 1) & 3);
+    const int m = min(m0 + row, a.M - 1), n = min(n0 + row, a.N - 1);
+    if constexpr (TAPS) px[i] = pixel_of(a, m);
+    xp[i] = a.x + (TAPS ? 0 : (size_t)m * a.ldx) + 8 * unit;
+    wp[i] = a.w + (size_t)n * a.K + 8 * unit;
+  }
+  char* const ring = smem + wave * (kFewBufs * 4096);
+  const uint32_t ring0 = lds_offset(smem) + wave * (kFewBufs * 4096);
+  const int tap_stages = TAPS ? a.cin / kStageK : 1;
+  const auto fetch = [&](int at) {
+    const int s = wave + NW * at;
+    const uint32_t buf = ring0 + (at % kFewBufs) * 4096;
+    const int tap = TAPS ? s / tap_stages : 0, c = TAPS ? (s - tap * tap_stages) * kStageK : s * kStageK;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const uint16_t* p = xp[i] + c;
+      if constexpr (TAPS) {
+        const uint16_t* row = tap_row(a, px[i], tap);
+        p = row ? row + (xp[i] - a.x) + c : (const uint16_t*)&kZeroRow;
+      }
+      load_to_lds16(p, buf + 1024 * i);
+      load_to_lds16(wp[i] + s * kStageK, buf + 2048 + 1024 * i);
+    }
+  };
+  f32x16_t acc = {0.f};
+#pragma unroll
+  for (int s = 0; s < kFewBufs - 1; ++s)
+    if (s < mine) fetch(s);
+  for (int s = 0; s < mine; ++s) {
+    const int ahead = min(mine - 1 - s, kFewBufs - 2);
+    if (ahead >= 2) wait_vmem<8>();
+    else if (ahead == 1) wait_vmem<4>();
+    else wait_vmem<0>();
+    const char* buf = ring + (s % kFewBufs) * 4096;
+    bf16x8_t xf[2], wf[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const int off = r * 64 + 16 * ((2 * k + h) ^ ((r >> 1) & 3));
+      xf[k] = *reinterpret_cast<const bf16x8_t*>(buf + off);
+      wf[k] = *reinterpret_cast<const bf16x8_t*>(buf + 2048 + off);
+    }
+    // the buffer read in the step before is refilled: its reads have been waited for by the products that used them
+    if (s + kFewBufs - 1 < mine) fetch(s + kFewBufs - 1);
+#pragma unroll
+    for (int k = 0; k < 2; ++k) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[k], xf[k], acc, 0, 0, 0);
+  }
+  // accumulator register 4g+m of lane (r, h) is channel 8g+4h+m of token r
+  __syncthreads();
+  float(*part)[32][36] = reinterpret_cast<float(*)[32][36]>(smem);
+#pragma unroll
+  for (int g = 0; g < 4; ++g)
+    *reinterpret_cast<f32x4_t*>(&part[wave][r][8 * g + 4 * h]) = f32x4_t{acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]};
+  __syncthreads();
+  for (int i = threadIdx.x; i < 256; i += 64 * NW) {
+    const int row = i >> 3, c = (i & 7) * 4;
+    f32x4_t sum = *reinterpret_cast<const f32x4_t*>(&part[0][row][c]);
+#pragma unroll
+    for (int k = 1; k < NW; ++k) {
+      const f32x4_t v = *reinterpret_cast<const f32x4_t*>(&part[k][row][c]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) sum[j] += v[j];
+    }
+    if (m0 + row < a.M && n0 + c < a.N) {  // N is a multiple of 8
+      if (a.bias) {
+        const u32x2_t b = *reinterpret_cast<const u32x2_t*>(a.bias + n0 + c);
+        sum[0] += bf16lo_to_f32(b[0]), sum[1] += bf16hi_to_f32(b[0]), sum[2] += bf16lo_to_f32(b[1]), sum[3] += bf16hi_to_f32(b[1]);
+      }
+      *reinterpret_cast<u32x2_t*>(a.y + (size_t)(m0 + row) * a.ldy + n0 + c) =
+          u32x2_t{pack_bf16x2(sum[0], sum[1]), pack_bf16x2(sum[2], sum[3])};
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Many rows: tiles of 64 MI x 64 NI by four waves of 32 MI x 32 NI each, operands through kBuffers LDS stages of 32
+// contraction elements (64-byte row pieces, loaded directly to LDS; the 16-byte units of a piece are swapped by the row number so
+// that the eight lanes served together hit different banks).
+// ---------------------------------------------------------------------------
+template <int MI, int NI, int BUFS, bool TAPS>
+__global__ __launch_bounds__(256, (64 * (MI + NI) * 64 * BUFS <= 80 * 1024 ? 2 : 1)) void gemm_many_kernel(GemmArgs a, int tn, int tiles) {
+  constexpr int TM = 64 * MI, TN = 64 * NI, kStage = (TM + TN) * 64;  // bytes
+  extern __shared__ __align__(16) char smem[];
+  const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  // each XCD gets a run of consecutive tiles (all column tiles of a row block before the next one), so that its L2 serves the rows
+  const int run = (tiles + 7) >> 3, at = ((int)blockIdx.x & 7) * run + ((int)blockIdx.x >> 3);
+  if (((int)blockIdx.x >> 3) >= run || at >= tiles) return;
+  const int m0 = at / tn * TM, n0 = (at - at / tn * tn) * TN;
+  const int nstage = a.K / kStageK;
+  const uint32_t lds0 = lds_offset(smem);
+  // a load covers 16 rows of 64 bytes; unit u of row w lies at place u ^ key
+  const int lrow = lane >> 2, place = lane & 3;
+  const uint16_t* xp[MI];
+  Pixel px[MI];
+  const uint16_t* wp[NI];
+#pragma unroll
+  for (int i = 0; i < MI; ++i) {
+    const int row = 16 * (wave * MI + i) + lrow, m = min(m0 + row, a.M - 1);
+    const int unit = place ^ ((row >> 1) & 3);
+    if constexpr (TAPS) px[i] = pixel_of(a, m);
+    xp[i] = a.x + (TAPS ? 0 : (size_t)m * a.ldx) + 8 * unit;
+  }
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int row = 16 * (wave * NI + i) + lrow;  // matrix row: its channel is permuted inside its 32
+    const int n = min(n0 + (row & ~31) + channel_of_row(row & 31), a.N - 1);
+    wp[i] = a.w + (size_t)n * a.K + 8 * (place ^ ((row >> 1) & 3));
+  }
+  const int tap_stages = TAPS ? a.cin / kStageK : 1;
+  const auto fetch = [&](int s) {
+    const uint32_t buf = lds0 + (s % BUFS) * kStage;
+    const int tap = TAPS ? s / tap_stages : 0, c = TAPS ? (s - tap * tap_stages) * kStageK : s * kStageK;
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+      const uint16_t* p = xp[i] + c;
+      if constexpr (TAPS) {
+        const uint16_t* row = tap_row(a, px[i], tap);
+        p = row ? row + (xp[i] - a.x) + c : (const uint16_t*)&kZeroRow;
+      }
+      load_to_lds16(p, buf + (wave * MI + i) * 1024);
+    }
+#pragma unroll
+    for (int i = 0; i < NI; ++i) load_to_lds16(wp[i] + s * kStageK, buf + TM * 64 + (wave * NI + i) * 1024);
+  };
+  const int wm = (wave & 1) * 32 * MI, wn = (wave >> 1) * 32 * NI;
+  int xoff[2], woff[2];
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const int unit = (2 * k + h) ^ ((r >> 1) & 3);
+    xoff[k] = (wm + r) * 64 + 16 * unit;
+    woff[k] = TM * 64 + (wn + r) * 64 + 16 * unit;
+  }
+  f32x16_t acc[MI][NI];
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int j = 0; j < NI; ++j) acc[i][j] = f32x16_t{0.f};
+#pragma unroll
+  for (int s = 0; s < BUFS - 1; ++s)
+    if (s < nstage) fetch(s);
+  for (int s = 0; s < nstage; ++s) {
+    const int ahead = min(nstage - 1 - s, BUFS - 2);
+    if (ahead >= 2) wait_vmem<2 * (MI + NI)>();
+    else if (ahead == 1) wait_vmem<MI + NI>();
+    else wait_vmem<0>();
+    lds_barrier();
+    if (s + BUFS - 1 < nstage) fetch(s + BUFS - 1);
+    const char* buf = smem + (s % BUFS) * kStage;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      bf16x8_t xf[MI], wf[NI];
+#pragma unroll
+      for (int i = 0; i < MI; ++i) xf[i] = *reinterpret_cast<const bf16x8_t*>(buf + xoff[k] + 2048 * i);
+#pragma unroll
+      for (int j = 0; j < NI; ++j) wf[j] = *reinterpret_cast<const bf16x8_t*>(buf + woff[k] + 2048 * j);
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NI; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[j], xf[i], acc[i][j], 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < NI; ++j) {
+    const int c = n0 + wn + 32 * j + 16 * h;
+    float bias[16];
+#pragma unroll
+    for (int e = 0; e < 16; ++e) bias[e] = 0.f;
+    if (a.bias) {
+#pragma unroll
+      for (int p = 0; p < 2; ++p)
+        if (c + 8 * p < a.N) {
+          const u32x4_t b = *reinterpret_cast<const u32x4_t*>(a.bias + c + 8 * p);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) bias[8 * p + 2 * e] = bf16lo_to_f32(b[e]), bias[8 * p + 2 * e + 1] = bf16hi_to_f32(b[e]);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+      const int m = m0 + wm + 32 * i + r;
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        u32x4_t o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = pack_bf16x2(acc[i][j][8 * p + 2 * e] + bias[8 * p + 2 * e], acc[i][j][8 * p + 2 * e + 1] + bias[8 * p + 2 * e + 1]);
+        if (m < a.M && c + 8 * p < a.N) *reinterpret_cast<u32x4_t*>(a.y + (size_t)m * a.ldy + c + 8 * p) = o;
+      }
+    }
+  }
+}
+
+template <int MI, int NI, int BUFS, bool TAPS>
+int launch_many(const GemmArgs& a, hipStream_t stream) {
+  constexpr size_t lds = (size_t)(64 * MI + 64 * NI) * 64 * BUFS;
+  static const bool attr = [] {
+    return hipFuncSetAttribute((const void*)gemm_many_kernel<MI, NI, BUFS, TAPS>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) ==
+           hipSuccess;
+  }();
+  if (!attr) return -5;
+  const int tn = (a.N + 64 * NI - 1) / (64 * NI), tm = (a.M + 64 * MI - 1) / (64 * MI), tiles = tn * tm;
+  hipLaunchKernelGGL((gemm_many_kernel<MI, NI, BUFS, TAPS>), dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(256), lds, stream, a, tn, tiles);
+  return hipGetLastError() == hipSuccess ? 0 : -5;
+}
+
+template <int NW, bool TAPS>
+int launch_few(const GemmArgs& a, hipStream_t stream) {
+  static const bool attr = [] {
+    return hipFuncSetAttribute((const void*)gemm_few_kernel<NW, TAPS>, hipFuncAttributeMaxDynamicSharedMemorySize, NW * kFewBufs * 4096) ==
+           hipSuccess;
+  }();
+  if (!attr) return -5;
+  hipLaunchKernelGGL((gemm_few_kernel<NW, TAPS>), dim3((a.N + 31) / 32, (a.M + 31) / 32), dim3(64 * NW), (size_t)NW * kFewBufs * 4096, stream, a);
+  return hipGetLastError() == hipSuccess ? 0 : -5;
+}
+
+}  // namespace
+
+static long long tiles_of(const GemmArgs& a, int tm, int tn) { return (long long)((a.M + tm - 1) / tm) * ((a.N + tn - 1) / tn); }
+
+// Where these kernels are the better choice (graph-captured runs on one MI355X; library times beside them):
+//   up to 640 tiles of 32 x 32: gemm_few_kernel  (M 196: N 192 K 512 3.1 us against 17.2, N 1280 K 384 3.5 / 5.2,
+//                               N 768 K 2048 4.7 / 6.9; past the line its operand traffic grows with the tile count)
+//   up to 2 GFLOP:              64 x 64 tiles    (M 1568 N 1280 K 384 6.5 / 6.9; M 6272 N 640 K 192 7.1 / 7.3)
+//   K <= 256 with 512 tiles:    256 x 128 tiles  (M 65536 N 640 K 192 35 / 40; M 100352 50 / 60)
+// Beyond that the library's products win (M 50176 N 1280 K 384 67 against 76 us).
+constexpr int kFewTiles = 640;
+static bool short_k_many(const GemmArgs& a) { return a.K <= 256 && tiles_of(a, 256, 128) >= 512; }
+
+bool linear_preferred(long long M, int N, int K) {
+  if (M <= 0 || M > 0x7fffffffLL - 256 || N <= 0 || K <= 0 || N % 8 || K % kStageK) return false;
+  GemmArgs a{};
+  a.M = (int)M, a.N = N, a.K = K;
+  return tiles_of(a, 32, 32) <= kFewTiles || 2.0 * M * N * K <= 2e9 || short_k_many(a);
+}
+
+int launch_linear(const void* x, long long ldx, const void* w, const void* bias, void* y, long long ldy, long long M, int N, int K,
+                  hipStream_t stream) {
+  if (M > 0x7fffffffLL - 256 || N % 8 || K % kStageK) return -95;
+  const GemmArgs a{(const uint16_t*)x, (const uint16_t*)w, (const uint16_t*)bias, (uint16_t*)y, ldx, ldy, (int)M, N, K, 0, 0, 0, 0, 0};
+  if (tiles_of(a, 64, 64) > 0x7fffffffLL - 8) return -95;
+  if (tiles_of(a, 32, 32) <= kFewTiles) return launch_few<4, false>(a, stream);
+  if (short_k_many(a)) return launch_many<4, 2, 3, false>(a, stream);
+  return launch_many<1, 1, 4, false>(a, stream);
+}
+
+// The convolution library took 12 to 138 us where these take 4.3 to 96: B 1, 28 x 28 x 96 -> 192 4.3 / 12.3; B 32, 192 -> 384
+// 26 / 54; B 256 96 / 137.  Long contractions (27 to 108 stages) want eight waves a tile while tiles are fewer than CUs, and
+// 192-column tiles once there is a tile for every CU.
+int launch_conv3x3s2(const void* x, const void* w, void* y, int B, int H, int W, int Cin, int Cout, hipStream_t stream) {
+  const int oh = (H + 1) / 2, ow = (W + 1) / 2;
+  const long long M = (long long)B * oh * ow;
+  if (Cin % kStageK || Cout % 8 || M > 0x7fffffffLL - 256 || (long long)B * H * W > 0x7fffffffLL) return -95;
+  const GemmArgs a{(const uint16_t*)x, (const uint16_t*)w, nullptr, (uint16_t*)y, 0, Cout, (int)M, Cout, 9 * Cin, H, W, oh, ow, Cin};
+  if (tiles_of(a, 64, 64) > 0x7fffffffLL - 8) return -95;
+  if (tiles_of(a, 32, 32) <= 256) return launch_few<8, true>(a, stream);
+  if (tiles_of(a, 32, 32) <= kFewTiles) return launch_few<4, true>(a, stream);
+  if (tiles_of(a, 128, 192) >= 256) return launch_many<2, 3, 4, true>(a, stream);
+  return launch_many<1, 1, 4, true>(a, stream);
+}
+
+}  // namespace vig

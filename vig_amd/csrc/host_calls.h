@@ -91,4 +91,8 @@ inline bool is_tensor(PyObject* o) { return THPVariable_Check(o); }
 PyObject* block_mix(PyObject*, PyObject* const* a, Py_ssize_t n);
 PyObject* block_mlp(PyObject*, PyObject* const* a, Py_ssize_t n);
 
+// the methods of model_forward.cpp
+PyObject* make_plan(PyObject*, PyObject* const* a, Py_ssize_t n);
+PyObject* run_plan(PyObject*, PyObject* const* a, Py_ssize_t n);
+
 }  // namespace vig_host

@@ -2,15 +2,17 @@
 // 3 input channels) as an implicit GEMM on the matrix cores, reading the images in the [B, C, H, W] layout they
 // arrive in and writing channels-last rows [B, OH, OW, Cout] -- what the LayerNorm kernel behind it consumes.
 //
-// One workgroup produces one output row (b, oy): OW <= 32 pixels x Cout channels.  Its input is the slab of
-// Cin * KH image rows (27 for 3 channels x 9 kernel rows); each goes to LDS shifted by one element, so that input
-// column ix sits at element ix + 1 and element 0 is the left padding: pixel ox then finds its 16 kernel columns
+// One workgroup produces up to 32 pixels of one output row (b, oy), all Cout channels.  Its input is the slab of
+// Cin * KH image rows (27 for 3 channels x 9 kernel rows), 256 columns of them; each goes to LDS shifted by one element, so
+// that input column ix of the piece sits at element ix + 1 and element 0 is the column in front (the left padding): pixel ox then finds its 16 kernel columns
 // (9 real ones, the weights of the others are zero) at elements 8*ox .. 8*ox+15, two aligned 16-byte reads.  The
 // contraction runs over (channel, kernel row) steps of 16 kernel columns: one v_mfma_f32_32x32x16_bf16 per step with
 // the weights (matrix rows = output channels) in registers for the life of the workgroup and the pixels as columns.
 // Matrix rows are assigned channels so that a lane ends with 16 consecutive channels of one pixel (32 contiguous
 // bytes).  The one-element shift costs no unaligned access: a lane takes the last element of its left neighbour's
 // 16-byte chunk (a lane shuffle) and funnel-shifts its own chunk behind it.
+// Rows wider than 248 columns are cut into pieces of 256 (a wide row went through a layout copy and the convolution library:
+// 101 us at 8 x 1024 x 1024, 27 us in pieces).
 #include "common.h"
 #include "launch.h"
 
@@ -25,7 +27,7 @@ constexpr int kPcKW = 16;          // kernel columns per contraction step (weigh
 template <int KS, int NW>  // KS = Cin * KH contraction steps, NW = Cout / 32 waves
 __global__ __launch_bounds__(512) void patch_conv_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ wp,
                                                          uint16_t* __restrict__ y, int Cin, int H, int W, int KH, int OH,
-                                                         int OW, int Cout, int nrows) {
+                                                         int OW, int Cout, int pieces, int nitems) {
   extern __shared__ __align__(16) char smem[];
   uint16_t* slab = reinterpret_cast<uint16_t*>(smem);  // [KS][kPcRowElems]
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -45,7 +47,8 @@ __global__ __launch_bounds__(512) void patch_conv_kernel(const uint16_t* __restr
   // image rows of the slab a thread fetches: half-wave (wave, h) takes slab rows 2*p + h, p = wave, wave + nwaves, ..;
   // the chunks of the next output row are in flight while the current one is multiplied
   constexpr int kMaxP = ((KS + 1) / 2 + NW - 1) / NW;  // row pairs per wave
-  auto fetch = [&](int row, u32x4_t (&v)[kMaxP]) {
+  auto fetch = [&](int item, u32x4_t (&v)[kMaxP], uint32_t (&front)[kMaxP]) {
+    const int row = item / pieces, c0 = (item - row * pieces) * 256;
     const int b = row / OH, oy = row - b * OH;
 #pragma unroll
     for (int i = 0; i < kMaxP; ++i) {
@@ -53,28 +56,36 @@ __global__ __launch_bounds__(512) void patch_conv_kernel(const uint16_t* __restr
       const int c = t / KH, ky = t - c * KH;
       const int iy = oy * kPcStride - 1 + ky;
       v[i] = u32x4_t{0u, 0u, 0u, 0u};
-      if (row < nrows && t < KS && iy >= 0 && iy < H && r * 8 < W)
-        v[i] = *reinterpret_cast<const u32x4_t*>(x + (((size_t)b * Cin + c) * H + iy) * (size_t)W + r * 8);
+      front[i] = 0u;
+      if (item < nitems && t < KS && iy >= 0 && iy < H) {
+        const uint16_t* p = x + (((size_t)b * Cin + c) * H + iy) * (size_t)W + c0;
+        if (c0 + r * 8 < W) v[i] = *reinterpret_cast<const u32x4_t*>(p + r * 8);
+        if (c0 > 0 && r == 0) front[i] = *reinterpret_cast<const uint32_t*>(p - 2);
+      }
     }
   };
   u32x4_t v[kMaxP];
-  fetch(blockIdx.x, v);
-  for (int row = blockIdx.x; row < nrows; row += gridDim.x) {
+  uint32_t front[kMaxP];
+  fetch(blockIdx.x, v, front);
+  for (int item = blockIdx.x; item < nitems; item += gridDim.x) {
     // ---- stage the slab: lane r = 16-byte chunk r of its image row, shifted by one element ----
 #pragma unroll
     for (int i = 0; i < kMaxP; ++i) {
       const int t = 2 * (wave + i * nwaves) + h;
-      uint32_t prev = __shfl_up(v[i][3], 1, 32);  // the left neighbour's last pair; chunk 0 has the padding there
-      if (r == 0) prev = 0u;
+      uint32_t prev = __shfl_up(v[i][3], 1, 32);  // the left neighbour's last pair; chunk 0 has the column in front there
+      if (r == 0) prev = front[i];
       u32x4_t o;
       o[0] = __builtin_amdgcn_alignbit(v[i][0], prev, 16);
       o[1] = __builtin_amdgcn_alignbit(v[i][1], v[i][0], 16);
       o[2] = __builtin_amdgcn_alignbit(v[i][2], v[i][1], 16);
       o[3] = __builtin_amdgcn_alignbit(v[i][3], v[i][2], 16);
-      if (t < KS) *reinterpret_cast<u32x4_t*>(slab + t * kPcRowElems + r * 8) = o;
+      if (t < KS) {
+        *reinterpret_cast<u32x4_t*>(slab + t * kPcRowElems + r * 8) = o;
+        if (r == 31) slab[t * kPcRowElems + 256] = (uint16_t)(v[i][3] >> 16);  // the last pixel's ninth column
+      }
     }
     __syncthreads();
-    fetch(row + gridDim.x, v);
+    fetch(item + gridDim.x, v, front);
     // ---- pixels x channels: KS contraction steps ----
     f32x16_t acc;
 #pragma unroll
@@ -91,8 +102,9 @@ __global__ __launch_bounds__(512) void patch_conv_kernel(const uint16_t* __restr
       lo[j] = pack_bf16x2(acc[2 * j], acc[2 * j + 1]);
       hi[j] = pack_bf16x2(acc[8 + 2 * j], acc[8 + 2 * j + 1]);
     }
-    if (r < OW) {
-      uint16_t* dst = y + ((size_t)row * OW + r) * (size_t)Cout + 32 * wave + 16 * h;
+    const int row = item / pieces, ox = (item - row * pieces) * 32 + r;
+    if (ox < OW) {
+      uint16_t* dst = y + ((size_t)row * OW + ox) * (size_t)Cout + 32 * wave + 16 * h;
       *reinterpret_cast<u32x4_t*>(dst) = lo;
       *reinterpret_cast<u32x4_t*>(dst + 8) = hi;
     }
@@ -104,23 +116,24 @@ __global__ __launch_bounds__(512) void patch_conv_kernel(const uint16_t* __restr
 
 bool patch_conv_supported(int Cin, int H, int W, int KH, int KW, int stride, int padding, int Cout) {
   if (stride != kPcStride || padding != 1 || KW < 1 || KW > kPcKW || Cin * KH != 27) return false;
-  if (W % 8 != 0 || W > 248 || H < 1) return false;
+  if (W % 8 != 0 || H < 1 || (W > 248 && KW > 9)) return false;  // (a piece holds nine columns of its last pixel)
   const int OW = (W + 2 - KW) / stride + 1;
-  return OW >= 1 && OW <= 32 && Cout % 32 == 0 && Cout >= 64 && Cout <= 256;  // two to eight waves
+  return OW >= 1 && Cout % 32 == 0 && Cout >= 64 && Cout <= 256;  // two to eight waves
 }
 
 int launch_patch_conv(const void* x, const void* w_packed, void* y, int B, int Cin, int H, int W, int KH, int KW,
                       int Cout, hipStream_t stream) {
   if (!patch_conv_supported(Cin, H, W, KH, KW, kPcStride, 1, Cout)) return -95;
   const int OH = (H + 2 - KH) / kPcStride + 1, OW = (W + 2 - KW) / kPcStride + 1;
-  if (OH < 1 || (long long)B * OH > 0x7fffffffLL - 4096 || Cout / 32 < 2) return -95;
-  const int nrows = B * OH;
-  const int grid = nrows < 512 ? nrows : 512;  // two workgroups a CU; each walks rows grid apart
+  const int pieces = (OW + 31) / 32;
+  if (OH < 1 || (long long)B * OH * pieces > 0x7fffffffLL - 4096 || Cout / 32 < 2) return -95;
+  const int nitems = B * OH * pieces;
+  const int grid = nitems < 512 ? nitems : 512;  // two workgroups a CU; each walks pieces grid apart
   const size_t lds = (size_t)27 * kPcRowElems * sizeof(uint16_t);
 #define VIG_PC_CASE(NW)                                                                                            \
   case NW:                                                                                                         \
     hipLaunchKernelGGL((patch_conv_kernel<27, NW>), dim3(grid), dim3(64 * NW), lds, stream, (const uint16_t*)x, \
-                       (const uint16_t*)w_packed, (uint16_t*)y, Cin, H, W, KH, OH, OW, Cout, nrows);              \
+                       (const uint16_t*)w_packed, (uint16_t*)y, Cin, H, W, KH, OH, OW, Cout, pieces, nitems);              \
     break
   switch (Cout / 32) {
     VIG_PC_CASE(2);

@@ -160,6 +160,8 @@ PyMethodDef kMethods[] = {
     {"gla_gate", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(gla_gate)), METH_FASTCALL, nullptr},
     {"block_mix", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(block_mix)), METH_FASTCALL, nullptr},
     {"block_mlp", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(block_mlp)), METH_FASTCALL, nullptr},
+    {"make_plan", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(make_plan)), METH_FASTCALL, nullptr},
+    {"run_plan", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(run_plan)), METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "vig_host", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};

@@ -69,6 +69,24 @@ Tensor workspace(size_t bytes, const Tensor& like) {
 
 float resolve_scale(double scale, int64_t Dk) { return scale < 0 ? 1.0f / std::sqrt((float)Dk) : (float)scale; }
 
+// x . w^T (+ b): the library's own kernels where they are the better choice for the size, torch's product otherwise
+Tensor product(const Tensor& x, const Tensor& w, const optional<Tensor>& b = c10::nullopt) {
+  const auto dense = [](const Tensor& t) { return t.is_contiguous() && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; };
+  const int64_t N = w.size(0), K = w.size(1);
+  if (!(x.scalar_type() == at::kBFloat16 && w.scalar_type() == at::kBFloat16 && x.is_cuda() && w.device() == x.device() &&
+        x.size(-1) == K && dense(x) && dense(w) && (!b || (b->scalar_type() == at::kBFloat16 && dense(*b))) &&
+        vig_linear_preferred(x.numel() / K, (int)N, (int)K)))
+    return at::linear(x, w, b);
+  const c10::DeviceGuard guard(x.device());
+  auto shape = x.sizes().vec();
+  shape.back() = N;
+  Tensor y = at::empty(shape, x.options());
+  check_rc(vig_linear_fwd(x.data_ptr(), K, w.data_ptr(), b ? b->data_ptr() : nullptr, y.data_ptr(), N, x.numel() / K, (int)N, (int)K,
+                          stream_of(x)),
+           "vig_linear_fwd");
+  return y;
+}
+
 struct GlaDims {
   int B, H, L, Dk, Dv;
 };
@@ -254,7 +272,7 @@ Tensor locality_blend_linear_fwd(const Tensor& o, const Tensor& local, const Ten
   const bool fused = o.scalar_type() == at::kBFloat16 && weight.scalar_type() == at::kBFloat16 && Dv == 64 &&
                      weight.size(1) == H * Dv && C == H * Dv && (C == 384 || C == 192) && weight.is_contiguous() &&
                      reinterpret_cast<uintptr_t>(weight.data_ptr()) % 16 == 0;
-  if (!fused) return at::linear(locality_blend_fwd(o, local, g_lin, w_g, w_l, eps, silu_out), weight);
+  if (!fused) return product(locality_blend_fwd(o, local, g_lin, w_g, w_l, eps, silu_out), weight);
   check_dense(o, o, "o");
   check_dense(local, o, "local");
   const int64_t ldg = token_row_stride(g_lin, o, "g_lin");
@@ -408,7 +426,7 @@ Tensor gla_block_mix(const Tensor& x, int64_t grid_h, int64_t grid_w, const Tens
                      const Tensor& w_gnorm, const Tensor& w_lnorm, double eps, bool out_act, const Tensor& w_o,
                      double out_scale) {
   Tensor xs = dwconv3x3_fwd(x, conv_w, conv_b, grid_h, grid_w, act_in_conv);
-  Tensor z = at::linear(xs, w_in, b_in);
+  Tensor z = product(xs, w_in, b_in);
   const int64_t n0 = H * (2 * Dk + Dv), n1 = n0 + H * Dv, rank = w_up.size(1);
   TORCH_CHECK(z.size(-1) >= n1 + rank, "vig_amd: stacked projection is narrower than qkv | g | gate rows");
   Tensor gates = dirgate_lowrank_fwd(z.narrow(-1, n1, rank), w_up, b_up, H, normalizer, clamp_min);
@@ -459,8 +477,8 @@ std::tuple<Tensor, Tensor> gla_block_carry(const Tensor& branch, const optional<
   if (h.scalar_type() == at::kBFloat16 && w_gate.scalar_type() == at::kBFloat16 && (K == 384 || K == 192) && I % 32 == 0)
     m = linear_swiglu_fwd(h, w_gate);  // no [.., 2*I] intermediate
   else
-    m = swiglu_fwd(at::linear(h, w_gate));
-  return {at::linear(m, w_down), *std::get<1>(n2)};
+    m = swiglu_fwd(product(h, w_gate));
+  return {product(m, w_down), *std::get<1>(n2)};
 }
 
 }  // namespace

@@ -26,6 +26,7 @@ with its flips and concatenations folded into the op).
 from __future__ import annotations
 
 import math
+import weakref
 from typing import Optional
 
 import torch
@@ -49,6 +50,7 @@ def _f32(owner: nn.Module, tag: str, t: Optional[torch.Tensor], shape=None):
     return hit[1]
 
 
+_PLANS = weakref.WeakKeyDictionary()  # model -> plan of its native evaluation forward (ViG._planned)
 _CACHE_ATTRS = ("_f32_cache", "_w32_key", "_w32_cache", "_w1_packed")
 
 
@@ -58,6 +60,7 @@ def invalidate_caches(model: nn.Module) -> None:
     a write through `.data` (p.data.mul_(..), module.weight.data[...] = ..) changes neither the pointer nor the version
     counter they are keyed on, so code that writes that way calls this afterwards.  load_state_dict and train() /
     eval() switches of these modules call it by themselves."""
+    _PLANS.clear()
     for m in model.modules():
         for a in _CACHE_ATTRS:
             m.__dict__.pop(a, None)
@@ -81,6 +84,13 @@ class _CacheMixin:
 def _recording(module: nn.Module) -> bool:
     """True when this call has to leave an autograd graph: training mode with gradients enabled."""
     return module.training and torch.is_grad_enabled()
+
+
+def _linear(module: nn.Linear, x):
+    """module(x) outside of autograd, on the library's product where that is the better choice."""
+    if type(module) is not nn.Linear or module._forward_hooks or module._forward_pre_hooks:
+        return module(x)
+    return ops.linear(x, module.weight, module.bias)
 
 
 def _plain(*modules: nn.Module) -> bool:
@@ -192,7 +202,7 @@ class GatedLinearAttention(_CacheMixin, nn.Module):
         bias add) as in the separate layers.  The stacked copy follows the parameters: it is rebuilt when one of them
         is replaced, moved, cast or written in place."""
         w, b = self._stacked_in()
-        z = F.linear(xs, w, b)
+        z = ops.linear(xs, w, b)
         n0 = self.qkv_proj.weight.shape[0]
         n1 = n0 + self.value_dim
         return z[..., :n0], z[..., n0:n1], z[..., n1:n1 + self.gk_proj[0].weight.shape[0]]
@@ -250,7 +260,7 @@ class GatedLinearAttention(_CacheMixin, nn.Module):
                                              eps=self.layernorm_eps, silu_out=self.use_out_act)
         y = ops.locality_blend(o, xs, g_lin, self.g_norm._w32(), self.l_norm._w32(),
                                eps=self.layernorm_eps, silu_out=self.use_out_act)
-        return self.o_proj(y)
+        return _linear(self.o_proj, y)
 
     def _mix_autograd(self, x, hw, out_scale):
         """_mix with an autograd graph (the reference's training branch, vig.py:354-426,444-463: its flipped copies of
@@ -381,9 +391,12 @@ class GLAMLP(nn.Module):
         if ops.linear_swiglu_supported(x, w):  # ViG-S / ViG-T widths in bf16: no [.., 2*I] intermediate
             ext = _ext.load()
             if ext is not None and x.is_contiguous():
-                return self.down_proj(ext.linear_swiglu_fwd(x, w))
-            return self.down_proj(ops.linear_swiglu(x, w))
-        return self.down_proj(ops.swiglu(self.gate_proj(x)))
+                return self._down(ext.linear_swiglu_fwd(x, w))
+            return self._down(ops.linear_swiglu(x, w))
+        return self._down(ops.swiglu(self.gate_proj(x) if torch.is_grad_enabled() else _linear(self.gate_proj, x)))
+
+    def _down(self, h):
+        return self.down_proj(h) if torch.is_grad_enabled() else _linear(self.down_proj, h)
 
 
 class DropPath(nn.Module):
@@ -574,6 +587,8 @@ class V2PatchEmbed(_CacheMixin, nn.Module):
 
     @staticmethod
     def _conv_nobias(conv, x):
+        if conv.stride == (2, 2) and conv.padding == (1, 1) and conv.dilation == (1, 1) and conv.groups == 1 and not torch.is_grad_enabled():
+            return ops.conv3x3s2(x, conv.weight)
         return F.conv2d(x, conv.weight, None, conv.stride, conv.padding, conv.dilation, conv.groups)
 
 
@@ -624,14 +639,90 @@ class ViG(nn.Module):
         branch, residual = x, None
         for blk in self.blocks:
             branch, residual = blk.forward_carry(branch, residual, patch_resolution=hw, token_position=None)
-        x = self.norm(branch, residual, round_sum=True) if residual is not None else self.norm(branch)
+        if residual is None:
+            x = self.norm(branch)
+        elif (not torch.is_grad_enabled() and type(self.norm) is RMSNorm and branch.is_cuda and self.embed_dim <= 1024
+              and branch.dtype == residual.dtype == torch.bfloat16 and not (self.norm._forward_hooks or self.norm._forward_pre_hooks)):
+            return ops.rmsnorm_pool(branch, residual, self.norm._w32(), self.norm.eps)
+        else:
+            x = self.norm(branch, residual, round_sum=True)
         return x.reshape(B, hw[0] * hw[1], -1).mean(dim=1)
 
     def forward(self, x):
         if _recording(self):
             return self.head(self.forward_features(x))
+        y = self._planned(x)
+        if y is not None:
+            return y
         with torch.no_grad():
-            return self.head(self.forward_features(x))
+            return _linear(self.head, self.forward_features(x))
+
+    def _planned(self, x):
+        """The evaluation forward as one native call (csrc/model_forward.cpp) over a plan of this model, made on first use
+        and remade when the model has changed; None for what the plan does not describe: other dtypes, image sizes with another
+        grid than the position table's, hooks, replaced or subclassed modules, strongly gated layers."""
+        if self.training or type(self) is not ViG or x.dtype is not torch.bfloat16 or not x.is_cuda:
+            return None
+        calls = _ext.calls()
+        if calls is None or _ext.load() is None:
+            return None
+        for _ in range(2):
+            plan = _PLANS.get(self)
+            if plan is None:
+                plan = self._make_plan(calls)
+                if plan is None:
+                    return None
+                _PLANS[self] = plan
+            y = calls.run_plan(plan, x)
+            if y is not False:
+                return y
+            _PLANS.pop(self, None)
+        return None
+
+    def _make_plan(self, calls):
+        pe = self.patch_embed
+        if type(pe) is not V2PatchEmbed or len(self.blocks) == 0 or self.head.weight.dtype is not torch.bfloat16:
+            return None
+        conv1, norm1, act, conv2, norm2 = pe.proj
+        typed = [(conv1, nn.Conv2d), (norm1, LayerNorm2d), (act, nn.SiLU), (conv2, nn.Conv2d), (norm2, LayerNorm2d),
+                 (self.norm, RMSNorm), (self.head, nn.Linear)]
+        for blk in self.blocks:
+            at, mlp = blk.attn, blk.mlp
+            typed += [(blk, GLABlock), (at, GatedLinearAttention), (mlp, GLAMLP), (blk.attn_norm, RMSNorm), (blk.mlp_norm, RMSNorm),
+                      (at.g_norm, RMSNorm), (at.l_norm, RMSNorm), (at.in_proj[0], nn.Conv2d)]
+            typed += [(m, nn.Linear) for m in (at.qkv_proj, at.g_proj, at.o_proj, at.gk_proj[0], at.gk_proj[1], mlp.gate_proj, mlp.down_proj)]
+            if at.strong_gates or at.training or blk.training or at.gk_proj[0].weight.shape[0] != ops.GATE_RANK or at.head_v_dim != 64 or at.head_qk_dim not in (32, 64):
+                return None
+        if not all(type(m) is t for m, t in typed):
+            return None
+        if not (conv1.stride == (8, 8) and conv1.padding == (1, 1) and conv1.dilation == (1, 1) and conv1.groups == 1
+                and conv2.kernel_size == (3, 3) and conv2.stride == (2, 2) and conv2.padding == (1, 1) and conv2.dilation == (1, 1)
+                and conv2.groups == 1 and conv2.in_channels % 32 == 0 and self.embed_dim <= 1024 and self.embed_dim % 32 == 0):
+            return None
+        # besides the module tree and every parameter, what has to stay as it is
+        settings = {GatedLinearAttention: ("strong_gates", "layernorm_eps", "clamp_min", "use_out_act", "use_act_in_conv",
+                                           "gate_logit_normalizer", "num_heads", "training"),
+                    GLABlock: ("training",), RMSNorm: ("eps",), LayerNorm2d: ("eps",), ViG: ("patch_resolution",)}
+        absent = {GLABlock: "forward_carry", GatedLinearAttention: "_mix", ViG: "forward_features"}
+        called = [pe, norm1, act, norm2, self.norm, self.head, torch.nn.modules.module._global_forward_hooks,
+                  torch.nn.modules.module._global_forward_pre_hooks]
+        flag = lambda v: 1 if v else 0  # noqa: E731
+        with torch.no_grad():
+            stem = (pe._packed_w1(), _f32(pe, "b1", conv1.bias), _f32(norm1, "w", norm1.weight), _f32(norm1, "b", norm1.bias), norm1.eps,
+                    conv2.weight.detach().permute(0, 2, 3, 1).contiguous(), _f32(pe, "b2", conv2.bias), _f32(norm2, "w", norm2.weight),
+                    _f32(norm2, "b", norm2.bias), norm2.eps, self.pos_embed.detach().contiguous(), *conv1.kernel_size, *self.patch_resolution)
+            blocks = []
+            for blk in self.blocks:
+                at, mlp = blk.attn, blk.mlp
+                conv, up = at.in_proj[0], at.gk_proj[1]
+                w_in, b_in = at._stacked_in()
+                blocks.append((blk.attn_norm._w32(), blk.attn_norm.eps, _f32(at, "conv_w_flat", conv.weight, (-1,)),
+                               _f32(at, "conv_b", conv.bias), flag(at.use_act_in_conv), w_in, b_in, at.num_heads, at.head_qk_dim,
+                               at.head_v_dim, up.weight.detach(), up.bias.detach(), float(at.gate_logit_normalizer), at.clamp_min,
+                               at.g_norm._w32(), at.l_norm._w32(), at.layernorm_eps, flag(at.use_out_act), at.o_proj.weight.detach(),
+                               blk.mlp_norm._w32(), blk.mlp_norm.eps, mlp.gate_proj.weight.detach(), mlp.down_proj.weight.detach()))
+            tail = (self.norm._w32(), self.norm.eps, self.head.weight.detach(), self.head.bias.detach() if self.head.bias is not None else None)
+        return calls.make_plan(self, settings, absent, called, stem, blocks, tail)
 
 
 def vig_small(**kw):

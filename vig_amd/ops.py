@@ -894,8 +894,8 @@ def patch_conv_supported(x: torch.Tensor, weight: torch.Tensor, stride: int, pad
     """Whether patch_conv takes this convolution (the reference's stem shape in bf16); else use torch's."""
     Cout, Cin, KH, KW = weight.shape
     return (x.dtype == torch.bfloat16 and x.is_cuda and x.dim() == 4 and stride == 8 and padding == 1 and KW <= 16
-            and Cin * KH == 27 and x.shape[1] == Cin and x.shape[3] % 8 == 0 and x.shape[3] <= 248
-            and Cout % 32 == 0 and 64 <= Cout <= 256 and (x.shape[3] + 2 - KW) // 8 + 1 <= 32)
+            and Cin * KH == 27 and x.shape[1] == Cin and x.shape[3] % 8 == 0
+            and (x.shape[3] <= 248 or KW <= 9) and Cout % 32 == 0 and 64 <= Cout <= 256)
 
 
 def patch_conv(x: torch.Tensor, w_packed: torch.Tensor, kernel_hw, stride: int = 8, padding: int = 1) -> torch.Tensor:
@@ -917,6 +917,57 @@ def patch_conv(x: torch.Tensor, w_packed: torch.Tensor, kernel_hw, stride: int =
                                     padding, Cout, _dt(x), _stream_ptr(x))
     _lib.check(rc, "vig_patch_conv_fwd")
     return y
+
+
+def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """x @ weight.T (+ bias): vig_linear_fwd for bf16 rows at the sizes where it is the better choice, torch's product
+    otherwise.  Inference only (no autograd node of its own)."""
+    N, K = weight.shape
+    if (x.dtype == weight.dtype == torch.bfloat16 and x.is_cuda and x.shape[-1] == K and x.is_contiguous()
+            and weight.is_contiguous() and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0
+            and (bias is None or (bias.dtype == x.dtype and bias.is_contiguous() and bias.data_ptr() % 16 == 0))
+            and not torch.is_autocast_enabled()):
+        lib, rows = _lib.load(), x.numel() // K
+        if lib.vig_linear_preferred(rows, N, K):
+            y = torch.empty(*x.shape[:-1], N, dtype=x.dtype, device=x.device)
+            with torch.cuda.device(x.device):
+                rc = lib.vig_linear_fwd(x.data_ptr(), K, weight.data_ptr(), bias.data_ptr() if bias is not None else None,
+                                        y.data_ptr(), N, rows, N, K, _stream_ptr(x))
+            _lib.check(rc, "vig_linear_fwd")
+            return y
+    return torch.nn.functional.linear(x, weight, bias)
+
+
+def conv3x3s2(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """conv2d(x, weight, stride 2, padding 1) without bias on channels-last memory (vig.py:655): vig_conv3x3s2_fwd for bf16
+    maps, torch's convolution otherwise.  x [B, Cin, H, W] -> [B, Cout, (H+1)//2, (W+1)//2], channels-last."""
+    B, Cin, H, W = x.shape
+    Cout = weight.shape[0]
+    xl, wl = x.permute(0, 2, 3, 1), weight.detach().permute(0, 2, 3, 1)
+    if not (x.dtype == weight.dtype == torch.bfloat16 and x.is_cuda and x.numel() and Cin % 32 == 0 and Cout % 8 == 0
+            and weight.shape[1:] == (Cin, 3, 3) and xl.is_contiguous() and wl.is_contiguous()
+            and xl.data_ptr() % 16 == 0 and wl.data_ptr() % 16 == 0 and not torch.is_autocast_enabled()):
+        return torch.nn.functional.conv2d(x, weight, None, 2, 1)
+    y = torch.empty(B, (H + 1) // 2, (W + 1) // 2, Cout, dtype=x.dtype, device=x.device)
+    with torch.cuda.device(x.device):
+        rc = _lib.load().vig_conv3x3s2_fwd(xl.data_ptr(), wl.data_ptr(), y.data_ptr(), B, H, W, Cin, Cout, _stream_ptr(x))
+    _lib.check(rc, "vig_conv3x3s2_fwd")
+    return y.permute(0, 3, 1, 2)
+
+
+def rmsnorm_pool(x: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
+    """mean over tokens of rmsnorm(x + residual) for bf16 [B, L, C] -> [B, C] (vig.py:896-905) in one pass."""
+    x, residual = _dense(x), _dense(residual)
+    B, L, C = x.shape
+    lib = _lib.load()
+    out = torch.empty(B, C, dtype=x.dtype, device=x.device)
+    need = lib.vig_rmsnorm_pool_workspace(B, L, C)
+    ws = torch.empty(need, dtype=torch.uint8, device=x.device)
+    with torch.cuda.device(x.device):
+        rc = lib.vig_rmsnorm_pool_fwd(x.data_ptr(), residual.data_ptr(), weight.data_ptr(), out.data_ptr(), ws.data_ptr(), need,
+                                      B, L, C, float(eps), _stream_ptr(x))
+    _lib.check(rc, "vig_rmsnorm_pool_fwd")
+    return out
 
 
 def linear_swiglu_supported(x: torch.Tensor, weight: torch.Tensor) -> bool:
