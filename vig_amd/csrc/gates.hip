@@ -237,7 +237,7 @@ __global__ __launch_bounds__(256) void dirgate_lowrank_kernel(const TI* __restri
 // Accumulator register 4g+m of lane (r, h) holds matrix row 8g+4h+m of column r; matrix row i is given channel
 // 16*((i>>2)&1) + 4*(i>>3) + (i&3) of the tile, so that lane (r, h) ends up with channels 16h..16h+15 of token r:
 // 32 contiguous bytes of the head-major output.  Tokens are numbered over B*L; a workgroup owns NTG groups of 32 and
-// its four waves take the channel tiles in turn, each weight tile serving all the groups.  Needs Dk % 16 == 0 (a 16-channel run stays inside one head).
+// its four waves take the channel tiles in turn, each weight tile serving all the groups (gridDim.y workgroups share a group's tiles).  Needs Dk % 16 == 0 (a 16-channel run stays inside one head).
 template <typename TO, int NTG>
 __global__ __launch_bounds__(256) void dirgate_lowrank_mfma_kernel(const uint16_t* __restrict__ low, long long ld,
                                                                     const uint16_t* __restrict__ w1,
@@ -273,12 +273,12 @@ __global__ __launch_bounds__(256) void dirgate_lowrank_mfma_kernel(const uint16_
     bhi = *reinterpret_cast<const u32x4_t*>(b1 + c0 + 16 * h + 8);
   };
   u32x4_t wa_next, blo_next, bhi_next;
-  request(wave, wa_next, blo_next, bhi_next);
+  request(wave + 4 * blockIdx.y, wa_next, blo_next, bhi_next);
   const float inv_dk = 1.0f / (float)Dk, inv_h = 1.0f / (float)H;
-  for (int tile = wave; tile < ntiles; tile += 4) {
+  for (int tile = wave + 4 * blockIdx.y; tile < ntiles; tile += 4 * gridDim.y) {
     const int c0 = tile * 32;
     const u32x4_t wa = wa_next, blo = blo_next, bhi = bhi_next;
-    request(tile + 4, wa_next, blo_next, bhi_next);
+    request(tile + 4 * gridDim.y, wa_next, blo_next, bhi_next);
     float bias[16];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -435,7 +435,11 @@ int launch_dirgate_lowrank(const void* low, long long ld, const void* w1, const 
     const int use_clamp = clamp_min == clamp_min;  // NaN disables
     const long long ntok = (long long)B * L;
     constexpr int kGroups = 1;  // token groups of 32 per workgroup (two measured no faster)
-    const dim3 grid((unsigned)((ntok + 32 * kGroups - 1) / (32 * kGroups))), block(256);
+    const unsigned nb = (unsigned)((ntok + 32 * kGroups - 1) / (32 * kGroups));
+    // few tokens: the channel tiles of a token group over up to 1024 workgroups in all (B 1, H 3 4.3 -> 3.3 us; B 4, H 6
+    // 4.2 -> 2.9; B 16 4.6 -> 3.5), a round of four tiles at least for each
+    const int rounds = (2 * H * Dk / 32 + 3) / 4;
+    const dim3 grid(nb, (unsigned)max(1, min(rounds, (int)(1024 / nb)))), block(256);
     if (out_dtype == 1)
       hipLaunchKernelGGL((dirgate_lowrank_mfma_kernel<uint16_t, kGroups>), grid, block, 0, stream, (const uint16_t*)low, ld,
                          (const uint16_t*)w1, (const uint16_t*)b1, (uint16_t*)out, ntok, B, L, H, Dk, inv_norm,
@@ -563,8 +567,14 @@ static int launch_stencil(const void* x, const float* wt, const float* bias, voi
   int band = 48 * 1024 / row_bytes - 2;
   if (band < 1) return -95;
   if (band > h) band = h;
-  const int nband = (h + band - 1) / band;
   const int groups = (cgroup + kStencilGroup - 1) / kStencilGroup;
+  // Few images: shorter bands, until there are kFewBands workgroups.  One image's 3 to 24 workgroups leave the chip empty and a
+  // band lasts as long as its chain of loads and taps: 14 x 14, C 192 B 1 8.1 -> 4.5 us, B 16 8.5 -> 5.6; 32 x 32, C 384 B 1
+  // 10.6 -> 5.0.  (256 workgroups and more: 6.3 at B 16, the halo rows of one-row bands are read three times; 64: 6.6.)
+  constexpr int kFewBands = 128;
+  const int per = (kFewBands + images * groups - 1) / (images * groups);
+  if (per > (h + band - 1) / band) band = max(1, h / per);
+  const int nband = (h + band - 1) / band;
   const size_t lds = (size_t)(band + 2) * row_bytes;
   hipLaunchKernelGGL((stencil3x3_kernel<T, GATE>), dim3(images * groups, nband), dim3(256), lds, stream, (const T*)x, wt,
                      bias, (T*)y, (T*)pre, h, w, stride, groups, wmod, cgroup, band, silu);
