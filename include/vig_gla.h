@@ -516,6 +516,9 @@ int vig_rmsnorm_mixed_bwd(const void* sum, const float* weight, const void* dy, 
  */
 int vig_linear_swiglu_fwd(const void* x, const void* weight, void* y, long long rows, int K, int I, int io_dtype,
                           void* stream);
+/* The same, leaving gate | up as well: gate_up [rows, 2*I], what the backward of the product reads. */
+int vig_linear_swiglu_kept_fwd(const void* x, const void* weight, void* gate_up, void* y, long long rows, int K, int I,
+                               int io_dtype, void* stream);
 
 /*
  * vig_locality_blend_fwd and o_proj in one kernel, for square blocks with 64-channel heads at the widths whose weight

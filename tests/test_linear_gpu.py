@@ -1,0 +1,53 @@
+"""The linear layers with their weights in registers, and SwiGLU of a layer in its three forms, where they can go wrong: against
+float64 sums of the same bf16 values."""
+import pytest
+import torch
+
+import vig_amd
+from vig_amd import _lib, ops
+
+from .util import announce
+
+pytestmark = pytest.mark.gpu
+
+
+def _randn(shape, seed, scale=1.0):
+    return (torch.randn(shape, generator=torch.Generator().manual_seed(seed)) * scale).bfloat16()
+
+
+def _check(got, want64, ulps=1.0):
+    """Within `ulps` bf16 roundings (2^-8 relative) and the fp32 sums' error, 1e-5 of the result's scale."""
+    got = got.double().cpu()
+    assert ((got - want64).abs() <= ulps * 2.0 ** -8 * want64.abs() + 1e-5 * want64.abs().max()).all()
+
+
+# the first size of the rule; ragged token tiles; one, some and all of a workgroup's channel tiles, both contractions
+@pytest.mark.parametrize("rows,N,K", [(16384, 64, 192), (16385, 320, 384), (20011, 704, 192), (16415, 1280, 384)])
+def test_linear_in_registers(rows, N, K):
+    announce(f"linear in registers rows{rows} N{N} K{K}")
+    x, w, b = _randn((rows, K), 1), _randn((N, K), 2, K ** -0.5), _randn((N,), 3)
+    assert vig_amd._lib.load().vig_linear_preferred(rows, N, K)
+    for bias in (None, b):
+        got = ops.linear(x.cuda(), w.cuda(), bias.cuda() if bias is not None else None)
+        _check(got, torch.nn.functional.linear(x.double(), w.double(), bias.double() if bias is not None else None))
+
+
+# both sides of the lines between the forms (256 result tiles, 1024 tokens), ragged tokens, channel tiles of part of a workgroup
+@pytest.mark.parametrize("rows,K,I", [(1, 192, 32), (256, 384, 1024), (257, 384, 1024), (1024, 384, 1056), (1025, 384, 1056),
+                                      (8192, 192, 32), (8193, 192, 32), (9000, 192, 160), (9001, 384, 288)])
+def test_linear_swiglu_forms(rows, K, I):
+    announce(f"linear_swiglu rows{rows} K{K} I{I}")
+    x, w = _randn((rows, K), 4), _randn((2 * I, K), 5, K ** -0.5)
+    xd, wd = x.cuda(), w.cuda()
+    got = ops.linear_swiglu(xd, wd)
+    z, y = (torch.full((rows, n), float("nan"), dtype=torch.bfloat16, device="cuda") for n in (2 * I, I))
+    rc = _lib.load().vig_linear_swiglu_kept_fwd(xd.data_ptr(), wd.data_ptr(), z.data_ptr(), y.data_ptr(), rows, K, I, _lib.VIG_BF16,
+                                                torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    want = x.double() @ w.double().t()
+    _check(z, want)
+    g, u = z.double().cpu().chunk(2, 1)
+    _check(y, torch.nn.functional.silu(g) * u)  # of the values that were kept
+    # a pre-activation that another summation order rounds the other way moves the product by an ulp of each factor
+    g, u = want.chunk(2, 1)
+    _check(got, torch.nn.functional.silu(g) * u, ulps=4.0)

@@ -60,7 +60,7 @@ int launch_blend_linear(const void* o, const void* loc, const void* glin, const 
                         const void* W, void* out, int B, int H, int L, int Dv, int C, long long ldg, float eps,
                         int silu_out, hipStream_t stream);
 bool linear_swiglu_supported(int K, int I);
-int launch_linear_swiglu(const void* A, const void* W, void* out, long long T, int K, int I, hipStream_t stream);
+int launch_linear_swiglu(const void* A, const void* W, void* out, void* kept, long long T, int K, int I, hipStream_t stream);
 bool patch_conv_supported(int Cin, int H, int W, int KH, int KW, int stride, int padding, int Cout);
 int launch_patch_conv(const void* x, const void* w_packed, void* y, int B, int Cin, int H, int W, int KH, int KW,
                       int Cout, hipStream_t stream);
@@ -639,7 +639,17 @@ int vig_linear_swiglu_fwd(const void* x, const void* weight, void* y, long long 
   if (io_dtype != VIG_BF16 || !vig::linear_swiglu_supported(K, I)) return VIG_ENOTSUP;
   if (!strided_rows_ok(x, K, io_dtype) || !strided_rows_ok(weight, K, io_dtype) || !strided_rows_ok(y, I, io_dtype))
     return VIG_EINVAL;
-  return vig::launch_linear_swiglu(x, weight, y, rows, K, I, (hipStream_t)stream);
+  return vig::launch_linear_swiglu(x, weight, y, nullptr, rows, K, I, (hipStream_t)stream);
+}
+
+int vig_linear_swiglu_kept_fwd(const void* x, const void* weight, void* gate_up, void* y, long long rows, int K, int I,
+                               int io_dtype, void* stream) {
+  if (!x || !weight || !gate_up || !y || rows <= 0 || K <= 0 || I <= 0) return VIG_EINVAL;
+  if (io_dtype != VIG_BF16 || !vig::linear_swiglu_supported(K, I)) return VIG_ENOTSUP;
+  if (!strided_rows_ok(x, K, io_dtype) || !strided_rows_ok(weight, K, io_dtype) || !strided_rows_ok(gate_up, 2LL * I, io_dtype) ||
+      !strided_rows_ok(y, I, io_dtype))
+    return VIG_EINVAL;
+  return vig::launch_linear_swiglu(x, weight, y, gate_up, rows, K, I, (hipStream_t)stream);
 }
 
 int vig_swiglu_fwd(const void* gate_up, void* out, long long rows, int I, int io_dtype, void* stream) {

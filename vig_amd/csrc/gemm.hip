@@ -16,6 +16,7 @@ struct GemmArgs {
   int M, N, K;
   int gh, gw, oh, ow, cin;  // convolution: input and output grid, input channels
 };
+enum FewForm { kRows, kTaps, kPair };  // row matrix; convolution; SwiGLU of the products with rows n and N + n of w
 
 __device__ const u32x4_t kZeroRow = {0u, 0u, 0u, 0u};  // what a tap outside the grid reads
 
@@ -48,9 +49,11 @@ constexpr int kStageK = 32;  // contraction elements per LDS stage: 64-byte row 
 // ---------------------------------------------------------------------------
 constexpr int kFewBufs = 4;
 
-template <int NW, bool TAPS>
+template <int NW, FewForm FORM>
 __global__ __launch_bounds__(64 * NW) void gemm_few_kernel(GemmArgs a) {
-  extern __shared__ __align__(16) char smem[];  // [wave][buffer][4 KB: x rows, w rows], then the waves' tiles
+  constexpr bool TAPS = FORM == kTaps;
+  constexpr int kMats = FORM == kPair ? 2 : 1, kLoads = 2 + 2 * kMats, kBuf = 1024 * kLoads;
+  extern __shared__ __align__(16) char smem[];  // [wave][buffer][2 KB each: x rows, w rows, second w rows], then the waves' tiles
   const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int m0 = blockIdx.y * 32, n0 = blockIdx.x * 32;
@@ -66,12 +69,13 @@ __global__ __launch_bounds__(64 * NW) void gemm_few_kernel(GemmArgs a) {
     xp[i] = a.x + (TAPS ? 0 : (size_t)m * a.ldx) + 8 * unit;
     wp[i] = a.w + (size_t)n * a.K + 8 * unit;
   }
-  char* const ring = smem + wave * (kFewBufs * 4096);
-  const uint32_t ring0 = lds_offset(smem) + wave * (kFewBufs * 4096);
+  const size_t second = (size_t)a.N * a.K;
+  char* const ring = smem + wave * (kFewBufs * kBuf);
+  const uint32_t ring0 = lds_offset(smem) + wave * (kFewBufs * kBuf);
   const int tap_stages = TAPS ? a.cin / kStageK : 1;
   const auto fetch = [&](int at) {
     const int s = wave + NW * at;
-    const uint32_t buf = ring0 + (at % kFewBufs) * 4096;
+    const uint32_t buf = ring0 + (at % kFewBufs) * kBuf;
     const int tap = TAPS ? s / tap_stages : 0, c = TAPS ? (s - tap * tap_stages) * kStageK : s * kStageK;
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
@@ -82,53 +86,73 @@ __global__ __launch_bounds__(64 * NW) void gemm_few_kernel(GemmArgs a) {
       }
       load_to_lds16(p, buf + 1024 * i);
       load_to_lds16(wp[i] + s * kStageK, buf + 2048 + 1024 * i);
+      if constexpr (FORM == kPair) load_to_lds16(wp[i] + second + s * kStageK, buf + 4096 + 1024 * i);
     }
   };
-  f32x16_t acc = {0.f};
+  f32x16_t acc[kMats];
+#pragma unroll
+  for (int j = 0; j < kMats; ++j) acc[j] = f32x16_t{0.f};
 #pragma unroll
   for (int s = 0; s < kFewBufs - 1; ++s)
     if (s < mine) fetch(s);
   for (int s = 0; s < mine; ++s) {
     const int ahead = min(mine - 1 - s, kFewBufs - 2);
-    if (ahead >= 2) wait_vmem<8>();
-    else if (ahead == 1) wait_vmem<4>();
+    if (ahead >= 2) wait_vmem<2 * kLoads>();
+    else if (ahead == 1) wait_vmem<kLoads>();
     else wait_vmem<0>();
-    const char* buf = ring + (s % kFewBufs) * 4096;
-    bf16x8_t xf[2], wf[2];
+    const char* buf = ring + (s % kFewBufs) * kBuf;
+    bf16x8_t xf[2], wf[kMats][2];
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
       const int off = r * 64 + 16 * ((2 * k + h) ^ ((r >> 1) & 3));
       xf[k] = *reinterpret_cast<const bf16x8_t*>(buf + off);
-      wf[k] = *reinterpret_cast<const bf16x8_t*>(buf + 2048 + off);
+#pragma unroll
+      for (int j = 0; j < kMats; ++j) wf[j][k] = *reinterpret_cast<const bf16x8_t*>(buf + 2048 * (j + 1) + off);
     }
     // the buffer read in the step before is refilled: its reads have been waited for by the products that used them
     if (s + kFewBufs - 1 < mine) fetch(s + kFewBufs - 1);
 #pragma unroll
-    for (int k = 0; k < 2; ++k) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[k], xf[k], acc, 0, 0, 0);
+    for (int k = 0; k < 2; ++k)
+#pragma unroll
+      for (int j = 0; j < kMats; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[j][k], xf[k], acc[j], 0, 0, 0);
   }
   // accumulator register 4g+m of lane (r, h) is channel 8g+4h+m of token r
   __syncthreads();
-  float(*part)[32][36] = reinterpret_cast<float(*)[32][36]>(smem);
+  float(*part)[kMats][32][36] = reinterpret_cast<float(*)[kMats][32][36]>(smem);
 #pragma unroll
-  for (int g = 0; g < 4; ++g)
-    *reinterpret_cast<f32x4_t*>(&part[wave][r][8 * g + 4 * h]) = f32x4_t{acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]};
+  for (int j = 0; j < kMats; ++j)
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      *reinterpret_cast<f32x4_t*>(&part[wave][j][r][8 * g + 4 * h]) =
+          f32x4_t{acc[j][4 * g], acc[j][4 * g + 1], acc[j][4 * g + 2], acc[j][4 * g + 3]};
   __syncthreads();
   for (int i = threadIdx.x; i < 256; i += 64 * NW) {
     const int row = i >> 3, c = (i & 7) * 4;
-    f32x4_t sum = *reinterpret_cast<const f32x4_t*>(&part[0][row][c]);
+    f32x4_t sum[kMats];
 #pragma unroll
-    for (int k = 1; k < NW; ++k) {
-      const f32x4_t v = *reinterpret_cast<const f32x4_t*>(&part[k][row][c]);
+    for (int m = 0; m < kMats; ++m) {
+      sum[m] = *reinterpret_cast<const f32x4_t*>(&part[0][m][row][c]);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) sum[j] += v[j];
+      for (int k = 1; k < NW; ++k) {
+        const f32x4_t v = *reinterpret_cast<const f32x4_t*>(&part[k][m][row][c]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) sum[m][j] += v[j];
+      }
     }
     if (m0 + row < a.M && n0 + c < a.N) {  // N is a multiple of 8
       if (a.bias) {
         const u32x2_t b = *reinterpret_cast<const u32x2_t*>(a.bias + n0 + c);
-        sum[0] += bf16lo_to_f32(b[0]), sum[1] += bf16hi_to_f32(b[0]), sum[2] += bf16lo_to_f32(b[1]), sum[3] += bf16hi_to_f32(b[1]);
+        sum[0][0] += bf16lo_to_f32(b[0]), sum[0][1] += bf16hi_to_f32(b[0]), sum[0][2] += bf16lo_to_f32(b[1]), sum[0][3] += bf16hi_to_f32(b[1]);
+      }
+      if constexpr (FORM == kPair) {  // on the values the separate layer would have stored
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float g = bf16_to_f32(f32_to_bf16(sum[0][j])), u = bf16_to_f32(f32_to_bf16(sum[1][j]));
+          sum[0][j] = g * u * sigmoidf_(g);
+        }
       }
       *reinterpret_cast<u32x2_t*>(a.y + (size_t)(m0 + row) * a.ldy + n0 + c) =
-          u32x2_t{pack_bf16x2(sum[0], sum[1]), pack_bf16x2(sum[2], sum[3])};
+          u32x2_t{pack_bf16x2(sum[0][0], sum[0][1]), pack_bf16x2(sum[0][2], sum[0][3])};
     }
   }
 }
@@ -263,14 +287,14 @@ int launch_many(const GemmArgs& a, hipStream_t stream) {
   return hipGetLastError() == hipSuccess ? 0 : -5;
 }
 
-template <int NW, bool TAPS>
+template <int NW, FewForm FORM>
 int launch_few(const GemmArgs& a, hipStream_t stream) {
+  constexpr size_t lds = (size_t)NW * kFewBufs * (FORM == kPair ? 6144 : 4096);
   static const bool attr = [] {
-    return hipFuncSetAttribute((const void*)gemm_few_kernel<NW, TAPS>, hipFuncAttributeMaxDynamicSharedMemorySize, NW * kFewBufs * 4096) ==
-           hipSuccess;
+    return hipFuncSetAttribute((const void*)gemm_few_kernel<NW, FORM>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
   }();
   if (!attr) return -5;
-  hipLaunchKernelGGL((gemm_few_kernel<NW, TAPS>), dim3((a.N + 31) / 32, (a.M + 31) / 32), dim3(64 * NW), (size_t)NW * kFewBufs * 4096, stream, a);
+  hipLaunchKernelGGL((gemm_few_kernel<NW, FORM>), dim3((a.N + 31) / 32, (a.M + 31) / 32), dim3(64 * NW), lds, stream, a);
   return hipGetLastError() == hipSuccess ? 0 : -5;
 }
 
@@ -282,16 +306,18 @@ static long long tiles_of(const GemmArgs& a, int tm, int tn) { return (long long
 //   up to 640 tiles of 32 x 32: gemm_few_kernel  (M 196: N 192 K 512 3.1 us against 17.2, N 1280 K 384 3.5 / 5.2,
 //                               N 768 K 2048 4.7 / 6.9; past the line its operand traffic grows with the tile count)
 //   up to 2 GFLOP:              64 x 64 tiles    (M 1568 N 1280 K 384 6.5 / 6.9; M 6272 N 640 K 192 7.1 / 7.3)
-//   K <= 256 with 512 tiles:    256 x 128 tiles  (M 65536 N 640 K 192 35 / 40; M 100352 50 / 60)
-// Beyond that the library's products win (M 50176 N 1280 K 384 67 against 76 us).
+//   K 384 or 192, N % 64 == 0, 16384 rows: weights in registers (linear.hip; its table is beside launch_linear_regs)
+//   K <= 256 with 512 tiles:    256 x 128 tiles  (M 65536 N 520 K 192: other column counts)
+// Beyond that the library's products win (M 50176 N 1280 K 512 and longer contractions).
 constexpr int kFewTiles = 640;
+static bool regs_preferred(long long M, int N, int K) { return M >= 16384 && linear_regs_supported(K, N); }
 static bool short_k_many(const GemmArgs& a) { return a.K <= 256 && tiles_of(a, 256, 128) >= 512; }
 
 bool linear_preferred(long long M, int N, int K) {
   if (M <= 0 || M > 0x7fffffffLL - 256 || N <= 0 || K <= 0 || N % 8 || K % kStageK) return false;
   GemmArgs a{};
   a.M = (int)M, a.N = N, a.K = K;
-  return tiles_of(a, 32, 32) <= kFewTiles || 2.0 * M * N * K <= 2e9 || short_k_many(a);
+  return regs_preferred(M, N, K) || tiles_of(a, 32, 32) <= kFewTiles || 2.0 * M * N * K <= 2e9 || short_k_many(a);
 }
 
 int launch_linear(const void* x, long long ldx, const void* w, const void* bias, void* y, long long ldy, long long M, int N, int K,
@@ -299,9 +325,23 @@ int launch_linear(const void* x, long long ldx, const void* w, const void* bias,
   if (M > 0x7fffffffLL - 256 || N % 8 || K % kStageK) return -95;
   const GemmArgs a{(const uint16_t*)x, (const uint16_t*)w, (const uint16_t*)bias, (uint16_t*)y, ldx, ldy, (int)M, N, K, 0, 0, 0, 0, 0};
   if (tiles_of(a, 64, 64) > 0x7fffffffLL - 8) return -95;
-  if (tiles_of(a, 32, 32) <= kFewTiles) return launch_few<4, false>(a, stream);
+  if (regs_preferred(M, N, K) && ldx == K && ldy == N) return launch_linear_regs(x, w, bias, y, M, N, K, stream);
+  if (tiles_of(a, 32, 32) <= kFewTiles) return launch_few<4, kRows>(a, stream);
   if (short_k_many(a)) return launch_many<4, 2, 3, false>(a, stream);
   return launch_many<1, 1, 4, false>(a, stream);
+}
+
+// SwiGLU of a linear layer with the gate rows first, tiles of 32 x 32 results, while there is at most one for a CU.  Past that
+// the form with its weights in registers (linear.hip) is the better one: 196 rows, K 192, I 512 3.1 us against 4.5; 392 rows
+// 3.1 / 4.0, 588 4.5 / 4.1; K 384, I 1024: 196 rows 3.5 / 5.4, 392 5.3 / 5.3.
+bool few_swiglu(long long T, int K, int I) {
+  if (T <= 0 || T > 0x7fffffffLL - 256 || K <= 0 || K % kStageK || I <= 0 || I % 32) return false;
+  return (T + 31) / 32 * (I / 32) <= 256;
+}
+int launch_few_swiglu(const void* x, const void* w, void* y, long long T, int K, int I, hipStream_t stream) {
+  if (!few_swiglu(T, K, I)) return -95;
+  const GemmArgs a{(const uint16_t*)x, (const uint16_t*)w, nullptr, (uint16_t*)y, K, I, (int)T, I, K, 0, 0, 0, 0, 0};
+  return launch_few<4, kPair>(a, stream);
 }
 
 // The convolution library took 12 to 138 us where these take 4.3 to 96: B 1, 28 x 28 x 96 -> 192 4.3 / 12.3; B 32, 192 -> 384
@@ -313,8 +353,8 @@ int launch_conv3x3s2(const void* x, const void* w, void* y, int B, int H, int W,
   if (Cin % kStageK || Cout % 8 || M > 0x7fffffffLL - 256 || (long long)B * H * W > 0x7fffffffLL) return -95;
   const GemmArgs a{(const uint16_t*)x, (const uint16_t*)w, nullptr, (uint16_t*)y, 0, Cout, (int)M, Cout, 9 * Cin, H, W, oh, ow, Cin};
   if (tiles_of(a, 64, 64) > 0x7fffffffLL - 8) return -95;
-  if (tiles_of(a, 32, 32) <= 256) return launch_few<8, true>(a, stream);
-  if (tiles_of(a, 32, 32) <= kFewTiles) return launch_few<4, true>(a, stream);
+  if (tiles_of(a, 32, 32) <= 256) return launch_few<8, kTaps>(a, stream);
+  if (tiles_of(a, 32, 32) <= kFewTiles) return launch_few<4, kTaps>(a, stream);
   if (tiles_of(a, 128, 192) >= 256) return launch_many<2, 3, 4, true>(a, stream);
   return launch_many<1, 1, 4, true>(a, stream);
 }

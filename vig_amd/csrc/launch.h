@@ -108,4 +108,10 @@ int launch_gla_backward_mfma(const void* q, const void* k, const void* v, const 
                              const void* d_o, void* dq, void* dk, void* dv, void* dgf, void* dgb, int* flags,
                              void* seg_workspace, int B, int H, int L, int Dk, float s, hipStream_t stream);
 
+// bf16 row products (gemm.hip, linear.hip): a layer whose weights stay in registers, and SwiGLU of a layer over few rows
+bool linear_regs_supported(int K, int N);
+int launch_linear_regs(const void* x, const void* w, const void* bias, void* y, long long T, int N, int K, hipStream_t stream);
+bool few_swiglu(long long T, int K, int I);
+int launch_few_swiglu(const void* x, const void* w, void* y, long long T, int K, int I, hipStream_t stream);
+
 }  // namespace vig

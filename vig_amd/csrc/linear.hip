@@ -5,6 +5,8 @@
 // separate layer would have stored (flash-linear-attention/fla/modules/activations.py:109-113 on the two halves of
 // gate_proj's output, classification/models/vig.py:492-495), so the [T, 2*I] intermediate never exists.
 //
+// The same kernel without the SwiGLU makes 64 channels a wave of a plain layer, and for training it keeps both.
+//
 // With K this short a wave's whole slice of W fits in registers: a wave keeps the 32 gate rows and the 32 matching
 // up rows of one channel tile as matrix-instruction A operands for the life of the workgroup, eight waves cover 256
 // channels, and the workgroup streams 32-token tiles of A through LDS, double-buffered: the next tile travels from
@@ -28,35 +30,73 @@ constexpr int kLinWaves = 8;
 // such a load brings waits for it by itself.)
 __device__ __forceinline__ void tile_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-template <int KS>
-__global__ __launch_bounds__(64 * kLinWaves) void linear_swiglu_kernel(const uint16_t* __restrict__ A,
-                                                                       const uint16_t* __restrict__ W,
-                                                                       uint16_t* __restrict__ out, int T, int I,
-                                                                       int nworkers) {
+// Matrix row i of a weight tile holds this channel of its 32: lane (r, h) of the product ends with channels 16h .. 16h+15.
+__device__ __forceinline__ int channel_of_row(int i) { return 16 * ((i >> 2) & 1) + 4 * (i >> 3) + (i & 3); }
+
+// A wave's NT tiles of 32 rows of W (the tile's first row at `first[j]`, K = 16 * KS elements apart) into its registers as
+// matrix operands: w[j][t] = elements 16t + 8h .. of lane (r, h)'s row.  Fetched straight into registers that is 32 bytes of
+// 32 rows an instruction, four times each 128-byte line, and the lines of eight waves do not stay in the 32 KB L1: 14 us
+// of a launch at K 384, 8 at K 192.  So the rows travel in 128-byte pieces through a ring of kRing 4 KB buffers of the wave in
+// LDS (no barrier; unit u of row i lies at place u ^ (i & 7), so that the lanes served together hit different banks).
+// `ring` is free for other use behind the next barrier.
+constexpr int kRing = 2;
+template <int KS, int NT>
+__device__ __forceinline__ void load_weight_tiles(u32x4_t (&w)[NT][KS], const uint16_t* const* first, const char* ring, int lane) {
+  static_assert(KS % 4 == 0, "whole pieces");
+  constexpr int K = 16 * KS, KC = KS / 4, NQ = NT * KC;
+  const int r = lane & 31, h = lane >> 5, row = lane >> 3, unit = (lane & 7) ^ row;
+  const uint32_t ring0 = __builtin_amdgcn_readfirstlane(lds_offset(ring));
+  int off[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) off[i] = channel_of_row(8 * i + row) * K + 8 * unit;
+  const auto fetch = [&](int q) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) load_to_lds16(first[q / KC] + off[i] + 64 * (q % KC), ring0 + (q % kRing) * 4096 + 1024 * i);
+  };
+#pragma unroll
+  for (int q = 0; q < kRing; ++q) fetch(q);
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    if (q + 1 < NQ) wait_vmem<4 * (kRing - 1)>();
+    else wait_vmem<0>();
+    const char* buf = ring + (q % kRing) * 4096 + r * 128;
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+      w[q / KC][4 * (q % KC) + t] = *reinterpret_cast<const u32x4_t*>(buf + 16 * ((2 * t + h) ^ (r & 7)));
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // read before the buffer is filled again
+    if (q + kRing < NQ) fetch(q + kRing);
+  }
+}
+
+// What a wave makes of its two 32-row tiles of W (rows from c0 and from c1):
+//   kSwiglu      c0 = gate, c1 = up channels of one tile: the SwiGLU product
+//   kSwigluKept  the same, and the gate and up values themselves ([T, 2*I], what a backward reads)
+//   kLinear      64 channels of a plain layer, + bias
+enum LinForm { kSwiglu, kSwigluKept, kLinear };
+
+template <int KS, int NW, LinForm FORM>
+__global__ __launch_bounds__(64 * NW, 2) void linear_regs_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ W,
+                                                                 const uint16_t* __restrict__ bias, uint16_t* __restrict__ out,
+                                                                 uint16_t* __restrict__ kept, int T, int N, int nworkers) {
   constexpr int K = 16 * KS;
-  constexpr int kThreads = 64 * kLinWaves;
   constexpr int kCols = K / 8;                 // 16-byte chunks per token row
   constexpr int kRow = K + 8;                  // LDS row stride in elements (conflict-free 16-byte reads)
-  constexpr int kPer = 32 / kLinWaves;         // token rows per wave
-  static_assert(kCols <= 64 && 32 % kLinWaves == 0, "a wave loads whole token rows");
+  constexpr int kPer = 32 / NW;                // token rows per wave
+  constexpr int kStep = FORM == kLinear ? 64 : 32;                             // channels of `out` per wave
+  constexpr int kStores = FORM == kSwiglu ? 2 : FORM == kLinear ? 4 : 6;       // of a whole tile's epilogue
+  static_assert(kCols <= 64 && 32 % NW == 0, "a wave loads whole token rows");
   extern __shared__ __align__(16) char smem[];
-  uint16_t* buf = reinterpret_cast<uint16_t*>(smem);  // [2][32][kRow]
+  // [biases][2][32][kRow]; the weights' ring lies where the second of the two tiles will
+  constexpr size_t kBias = FORM == kLinear ? 64 * NW * sizeof(float) : 0, kTile = 32 * kRow * sizeof(uint16_t);
+  float* const bias_lds = reinterpret_cast<float*>(smem);
+  uint16_t* buf = reinterpret_cast<uint16_t*>(smem + kBias);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int r = lane & 31, h = lane >> 5;
   const int cg = blockIdx.x / nworkers, worker = blockIdx.x - cg * nworkers;
-  const int ct = cg * kLinWaves + wave;  // this wave's channel tile
-  const bool have = 32 * ct < I;
-  // matrix row i holds channel 16*((i>>2)&1) + 4*(i>>3) + (i&3) of the tile: lane (r, h) ends with channels 16h..16h+15
-  const int chan_of_row = 16 * ((r >> 2) & 1) + 4 * (r >> 3) + (r & 3);
-  u32x4_t wg[KS], wu[KS];
-  {
-    const uint16_t* pg = W + (size_t)(have ? 32 * ct + chan_of_row : 0) * K + 8 * h;
-    const uint16_t* pu = pg + (size_t)I * K;
-#pragma unroll
-    for (int t = 0; t < KS; ++t) {
-      wg[t] = *reinterpret_cast<const u32x4_t*>(pg + 16 * t);
-      wu[t] = *reinterpret_cast<const u32x4_t*>(pu + 16 * t);
-    }
+  const int ct = cg * NW + wave;  // this wave's channel tile
+  const bool have = kStep * ct < N;
+  if constexpr (FORM == kLinear) {
+    for (int i = tid; i < 64 * NW; i += 64 * NW) bias_lds[i] = bias && cg * 64 * NW + i < N ? bf16_to_f32(bias[cg * 64 * NW + i]) : 0.f;
   }
   const int ntiles_t = (T + 31) / 32;
   // A tile travels from memory straight into its LDS buffer (no registers): lane i of a wave lands 16 i bytes behind
@@ -70,73 +110,118 @@ __global__ __launch_bounds__(64 * kLinWaves) void linear_swiglu_kernel(const uin
     const uint32_t base = lds0 + which * (32 * kRow * 2);
 #pragma unroll
     for (int i = 0; i < kPer; ++i) {
-      const int row = i * kLinWaves + uwave;
+      const int row = i * NW + uwave;
       if (lane < kCols && tile * 32 + row < T)
         load_to_lds16(A + (size_t)tile * (32 * K) + (size_t)row * K + lane * 8, base + row * (kRow * 2));
     }
   };
+  u32x4_t wt[2][KS];
   f32x16_t g, u;
 #pragma unroll
   for (int j = 0; j < 16; ++j) g[j] = 0.f, u[j] = 0.f;
-  // SwiGLU on the rounded gate and up values of one finished tile, 16 consecutive channels of one token per lane
+  auto store32 = [](uint16_t* dst, const u32x4_t& lo, const u32x4_t& hi) {
+    *reinterpret_cast<u32x4_t*>(dst) = lo;
+    *reinterpret_cast<u32x4_t*>(dst + 8) = hi;
+  };
+  // one finished tile, 16 consecutive channels of one token per lane (SwiGLU on the rounded gate and up values)
   auto epilogue = [&](int etile) {
-    u32x4_t lo, hi;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      float y[2];
-#pragma unroll
-      for (int e = 0; e < 2; ++e) {
-        const float gs = bf16_to_f32(f32_to_bf16(g[2 * j + e])), us = bf16_to_f32(f32_to_bf16(u[2 * j + e]));
-        y[e] = gs * us * sigmoidf_(gs);
-      }
-      const uint32_t pk = pack_bf16x2(y[0], y[1]);
-      if (j < 4) lo[j] = pk;
-      else hi[j - 4] = pk;
-    }
     const int token = etile * 32 + r;
+    u32x4_t lo, hi, glo, ghi, ulo, uhi;
+    if constexpr (FORM != kSwiglu) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        glo[j] = pack_bf16x2(g[2 * j], g[2 * j + 1]), ghi[j] = pack_bf16x2(g[8 + 2 * j], g[8 + 2 * j + 1]);
+        ulo[j] = pack_bf16x2(u[2 * j], u[2 * j + 1]), uhi[j] = pack_bf16x2(u[8 + 2 * j], u[8 + 2 * j + 1]);
+      }
+    }
+    if constexpr (FORM != kLinear) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        float y[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          float gs, us;
+          if constexpr (FORM == kSwigluKept) {
+            const uint32_t gp = j < 4 ? glo[j] : ghi[j - 4], up = j < 4 ? ulo[j] : uhi[j - 4];
+            gs = e ? bf16hi_to_f32(gp) : bf16lo_to_f32(gp), us = e ? bf16hi_to_f32(up) : bf16lo_to_f32(up);
+          } else {
+            gs = bf16_to_f32(f32_to_bf16(g[2 * j + e])), us = bf16_to_f32(f32_to_bf16(u[2 * j + e]));
+          }
+          y[e] = gs * us * sigmoidf_(gs);
+        }
+        const uint32_t pk = pack_bf16x2(y[0], y[1]);
+        if (j < 4) lo[j] = pk;
+        else hi[j - 4] = pk;
+      }
+    }
     if (have && token < T) {
-      uint16_t* dst = out + (size_t)token * I + 32 * ct + 16 * h;
-      *reinterpret_cast<u32x4_t*>(dst) = lo;
-      *reinterpret_cast<u32x4_t*>(dst + 8) = hi;
+      if constexpr (FORM == kLinear) {
+        uint16_t* dst = out + (size_t)token * N + 64 * ct + 16 * h;
+        store32(dst, glo, ghi);
+        store32(dst + 32, ulo, uhi);
+      } else {
+        if constexpr (FORM == kSwigluKept) {
+          uint16_t* dst = kept + (size_t)token * 2 * N + 32 * ct + 16 * h;
+          store32(dst, glo, ghi);
+          store32(dst + N, ulo, uhi);
+        }
+        store32(out + (size_t)token * N + 32 * ct + 16 * h, lo, hi);
+      }
     }
   };
   // this tile's products: operand reads run kAhead k-steps ahead of the matrix instructions that use them
   auto products = [&](const uint16_t* mine) {
+    if constexpr (FORM == kLinear) {
 #pragma unroll
-    for (int j = 0; j < 16; ++j) g[j] = 0.f, u[j] = 0.f;
+      for (int j = 0; j < 4; ++j) {
+        const f32x4_t bg = *reinterpret_cast<const f32x4_t*>(bias_lds + 64 * wave + 16 * h + 4 * j),
+                      bu = *reinterpret_cast<const f32x4_t*>(bias_lds + 64 * wave + 32 + 16 * h + 4 * j);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) g[4 * j + e] = bg[e], u[4 * j + e] = bu[e];
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < 16; ++j) g[j] = 0.f, u[j] = 0.f;
+    }
     const uint16_t* xrow = mine + r * kRow + 8 * h;
-    constexpr int kAhead = 3;
+    constexpr int kAhead = FORM == kSwiglu || KS < 24 ? 3 : 2;  // (as the registers allow)
     u32x4_t x[kAhead];
 #pragma unroll
     for (int t = 0; t < kAhead; ++t) x[t] = *reinterpret_cast<const u32x4_t*>(xrow + 16 * t);
 #pragma unroll
     for (int t = 0; t < KS; ++t) {
       const u32x4_t xt = x[t % kAhead];
-      g = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, wg[t]), __builtin_bit_cast(bf16x8_t, xt),
+      g = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, wt[0][t]), __builtin_bit_cast(bf16x8_t, xt),
                                                   g, 0, 0, 0);
-      u = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, wu[t]), __builtin_bit_cast(bf16x8_t, xt),
+      u = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, wt[1][t]), __builtin_bit_cast(bf16x8_t, xt),
                                                   u, 0, 0, 0);
       if (t + kAhead < KS) x[t % kAhead] = *reinterpret_cast<const u32x4_t*>(xrow + 16 * (t + kAhead));
       __builtin_amdgcn_sched_barrier(0);
     }
   };
   fetch(worker, 0);
+  {
+    const uint16_t* const w0 = W + (size_t)(have ? kStep * (cg * NW + uwave) : 0) * K;
+    const uint16_t* const first[2] = {w0, w0 + (size_t)(FORM == kLinear ? (have ? 32 : 0) : N) * K};
+    load_weight_tiles<KS, 2>(wt, first, smem + kBias + kTile + uwave * (kRing * 4096), lane);
+  }
   int cur = 0;
   bool stored = false;  // an epilogue's stores were issued after the current tile's loads (a full tile's: only the last
                         // tile of all, behind which nothing is waited for, may be short)
   for (int tile = worker; tile < ntiles_t; tile += nworkers, cur ^= 1) {
     const uint16_t* mine = buf + cur * (32 * kRow);
-    // this thread's chunks of the tile have landed; the two stores of an epilogue behind them may still be on their way
+    // this thread's chunks of the tile have landed; the stores of an epilogue behind them may still be on their way
     // (waiting for those too, as a full barrier does, cost a tile the latency of a store)
-    if (stored) wait_vmem<2>();
+    if (stored) wait_vmem<kStores>();
     else wait_vmem<0>();
     tile_barrier();  // the tile is complete; the other buffer was last read before the previous barrier
     fetch(tile + nworkers, cur ^ 1);
-    // The two waves of a SIMD (w and w + 4) take turns on its two pipes: the lower wave runs this tile's matrix
-    // instructions first and its SwiGLU epilogue after; the upper wave first runs the epilogue of its PREVIOUS tile
+    // The two waves of a SIMD (w and w + 4 of eight) take turns on its two pipes: the lower wave runs this tile's matrix
+    // instructions first and its epilogue after; the upper wave first runs the epilogue of its PREVIOUS tile
     // (its accumulators waited in registers) and then this tile's matrix instructions.  So one wave's vector work
-    // runs under the other's matrix work in both halves of a tile's time, with one barrier per tile as before.
-    if (wave < kLinWaves / 2) {
+    // runs under the other's matrix work in both halves of a tile's time, with one barrier per tile as before.  (Four
+    // waves: the second wave of a SIMD is another workgroup's.)
+    if (NW == 4 || wave < NW / 2) {
       products(mine);
       epilogue(tile);  // (straight-line after the matrix instructions: no run-time branch in between)
       stored = have;
@@ -146,23 +231,49 @@ __global__ __launch_bounds__(64 * kLinWaves) void linear_swiglu_kernel(const uin
       products(mine);
     }
   }
-  if (wave >= kLinWaves / 2 && worker < ntiles_t)  // the upper waves' last tile
+  if (NW > 4 && wave >= NW / 2 && worker < ntiles_t)  // the upper waves' last tile
     epilogue(worker + ((ntiles_t - 1 - worker) / nworkers) * nworkers);
 }
 
-template <int KS>
-int launch_linear_swiglu_t(const void* A, const void* W, void* out, long long T, int I, int num_cu, hipStream_t stream) {
-  constexpr int K = 16 * KS;
-  const size_t lds = (size_t)2 * 32 * (K + 8) * sizeof(uint16_t);
-  const int ncg = (I / 32 + kLinWaves - 1) / kLinWaves;
+// allows a kernel its LDS, once per device (concurrent first calls only repeat an idempotent setting)
+bool allow_lds(const void* kernel, size_t bytes, bool (&done)[64]) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return false;
+  if (!done[dev]) done[dev] = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) == hipSuccess;
+  return done[dev];
+}
+
+template <int KS, int NW, LinForm FORM>
+int launch_linear_regs_t(const void* A, const void* W, const void* bias, void* out, void* kept, long long T, int N, int num_cu,
+                         hipStream_t stream) {
+  constexpr int K = 16 * KS, kStep = FORM == kLinear ? 64 : 32;
+  constexpr size_t tile = 32 * (K + 8) * sizeof(uint16_t), ring = (size_t)NW * kRing * 4096;
+  constexpr size_t lds = (FORM == kLinear ? 64 * NW * sizeof(float) : 0) + tile + (tile > ring ? tile : ring);
+  static bool done[64] = {};
+  if (!allow_lds((const void*)linear_regs_kernel<KS, NW, FORM>, lds, done)) return -5;
+  const int ncg = (N / kStep + NW - 1) / NW;
   const long long ntiles_t = (T + 31) / 32;
-  // one workgroup a CU; workers a multiple of 8 so that the column groups of a token tile share an XCD
-  int nworkers = num_cu / ncg / 8 * 8;
+  // eight waves a CU; workers a multiple of 8 so that the column groups of a token tile share an XCD
+  int nworkers = num_cu * 8 / NW / ncg / 8 * 8;
   if (nworkers < 8) nworkers = 8;
   if (nworkers > ntiles_t) nworkers = (int)ntiles_t;
-  hipLaunchKernelGGL((linear_swiglu_kernel<KS>), dim3(ncg * nworkers), dim3(64 * kLinWaves), lds, stream,
-                     (const uint16_t*)A, (const uint16_t*)W, (uint16_t*)out, (int)T, I, nworkers);
+  hipLaunchKernelGGL((linear_regs_kernel<KS, NW, FORM>), dim3(ncg * nworkers), dim3(64 * NW), lds, stream, (const uint16_t*)A,
+                     (const uint16_t*)W, (const uint16_t*)bias, (uint16_t*)out, (uint16_t*)kept, (int)T, N, nworkers);
   return hipGetLastError() == hipSuccess ? 0 : -5;
+}
+
+// compute units of the current device, 0 on an error
+int cu_count() {
+  constexpr int kMaxDevices = 64;
+  static int num_cu_dev[kMaxDevices] = {};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return 0;
+  if (num_cu_dev[dev] == 0) {
+    int n = 0;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
+    num_cu_dev[dev] = n > 0 ? n : 256;
+  }
+  return num_cu_dev[dev];
 }
 
 // ---------------------------------------------------------------------------
@@ -208,16 +319,16 @@ __global__ __launch_bounds__(64 * NW) void blend_linear_kernel(const uint16_t* _
   u32x4_t* park = reinterpret_cast<u32x4_t*>(smem + (size_t)2 * 32 * kRow * sizeof(uint16_t) + 128 * sizeof(float));
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int r = lane & 31, h = lane >> 5;
-  if (tid < 128) wnorm[tid] = tid < 64 ? w_g[tid] : w_l[tid - 64];
-  // matrix row i holds channel 16*((i>>2)&1) + 4*(i>>3) + (i&3) of the tile: lane (r, h) ends with channels 16h..16h+15
-  const int chan_of_row = 16 * ((r >> 2) & 1) + 4 * (r >> 3) + (r & 3);
   u32x4_t wt[TPW][KS];  // channel tiles TPW * wave ..
+  {
+    const int uwave = __builtin_amdgcn_readfirstlane(wave);
+    const uint16_t* first[TPW];
 #pragma unroll
-  for (int j = 0; j < TPW; ++j) {
-    const uint16_t* pw = W + (size_t)(32 * (TPW * wave + j) + chan_of_row) * K + 8 * h;
-#pragma unroll
-    for (int t = 0; t < KS; ++t) wt[j][t] = *reinterpret_cast<const u32x4_t*>(pw + 16 * t);
+    for (int j = 0; j < TPW; ++j) first[j] = W + (size_t)(32 * (TPW * uwave + j)) * K;
+    load_weight_tiles<KS, TPW>(wt, first, smem + uwave * (kRing * 4096), lane);
+    __syncthreads();  // the rings' place becomes the buffers'
   }
+  if (tid < 128) wnorm[tid] = tid < 64 ? w_g[tid] : w_l[tid - 64];
   const int ntiles_t = (T + 31) / 32;
   const float* wg8 = wnorm + ((tid % kCols) & 7) * 8;  // (kThreads % kCols == 0: a thread's octets share their column)
   const float* wl8 = wg8 + 64;
@@ -359,19 +470,14 @@ __global__ __launch_bounds__(64 * NW) void blend_linear_kernel(const uint16_t* _
 template <int KS, int NW, int TPW>
 int launch_blend_linear_t(const void* o, const void* loc, const void* glin, const float* w_g, const float* w_l,
                           const void* W, void* out, long long T, int L, int H, long long ldg, float eps, int silu_out,
-                          int num_cu, int dev, hipStream_t stream) {
+                          int num_cu, hipStream_t stream) {
   constexpr int K = 16 * KS;
-  const size_t lds = (size_t)2 * 32 * (K + 8) * sizeof(uint16_t) + 128 * sizeof(float) +
-                     (size_t)(32 * K / 8) * 3 * sizeof(u32x4_t);
+  constexpr size_t lds = (size_t)2 * 32 * (K + 8) * sizeof(uint16_t) + 128 * sizeof(float) + (size_t)(32 * K / 8) * 3 * sizeof(u32x4_t);
+  static_assert(lds >= (size_t)NW * kRing * 4096, "the weights' rings fit");
   const long long ntiles_t = (T + 31) / 32;
   const int grid = ntiles_t < num_cu ? (int)ntiles_t : num_cu;
-  static bool attr_done[64] = {};
-  if (!attr_done[dev]) {  // (per device; concurrent first calls only repeat an idempotent setting)
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(blend_linear_kernel<KS, NW, TPW>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
-      return -5;
-    attr_done[dev] = true;
-  }
+  static bool done[64] = {};
+  if (!allow_lds((const void*)blend_linear_kernel<KS, NW, TPW>, lds, done)) return -5;
   hipLaunchKernelGGL((blend_linear_kernel<KS, NW, TPW>), dim3(grid), dim3(64 * NW), lds, stream, (const uint16_t*)o,
                      (const uint16_t*)loc, (const uint16_t*)glin, w_g, w_l, (const uint16_t*)W, (uint16_t*)out, (int)T, L,
                      H, ldg, eps, silu_out);
@@ -389,32 +495,44 @@ int launch_blend_linear(const void* o, const void* loc, const void* glin, const 
   if (!blend_linear_supported(H, Dv, C) || B <= 0 || L <= 0 || (long long)B * L > 0x7fffffffLL - 64 || ldg % 8 != 0 ||
       ldg < C)
     return -95;
-  int dev = 0, n = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return -5;
-  if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return -5;
-  const int num_cu = n > 0 ? n : 256;
+  const int num_cu = cu_count();
+  if (!num_cu) return -5;
   const long long T = (long long)B * L;
   // twelve waves with one weight tile each (three per SIMD at 168 registers) at the wider size, six at the narrower
-  return C == 384 ? launch_blend_linear_t<24, 12, 1>(o, loc, glin, w_g, w_l, W, out, T, L, H, ldg, eps, silu_out, num_cu, dev, stream)
-                  : launch_blend_linear_t<12, 6, 1>(o, loc, glin, w_g, w_l, W, out, T, L, H, ldg, eps, silu_out, num_cu, dev, stream);
+  return C == 384 ? launch_blend_linear_t<24, 12, 1>(o, loc, glin, w_g, w_l, W, out, T, L, H, ldg, eps, silu_out, num_cu, stream)
+                  : launch_blend_linear_t<12, 6, 1>(o, loc, glin, w_g, w_l, W, out, T, L, H, ldg, eps, silu_out, num_cu, stream);
 }
 
 bool linear_swiglu_supported(int K, int I) { return (K == 384 || K == 192) && I % 32 == 0 && I >= 32; }
 
-int launch_linear_swiglu(const void* A, const void* W, void* out, long long T, int K, int I, hipStream_t stream) {
+// Waves a workgroup, measured (four / eight, us): the turns of eight waves hide the long SwiGLU epilogue of K 384 with many tokens
+// (25088 tokens 41.6 / 38.9, 50176 72 / 67); with few tokens, or with K 192, two independent workgroups of four
+// fill the chip better (784 tokens 5.7 / 7.5, K 192: 50176 28.6 / 30.3).  Where the values are kept, eight waves spill
+// (25088 tokens 50 / 65; a layer and a SwiGLU pass behind it: 84).
+int launch_linear_swiglu(const void* A, const void* W, void* out, void* kept, long long T, int K, int I, hipStream_t stream) {
+  if (!kept && few_swiglu(T, K, I)) return launch_few_swiglu(A, W, out, T, K, I, stream);
   if (!linear_swiglu_supported(K, I) || T <= 0 || T > 0x7fffffffLL - 64) return -95;
-  constexpr int kMaxDevices = 64;
-  static int num_cu_dev[kMaxDevices] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return -5;
-  if (num_cu_dev[dev] == 0) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return -5;
-    num_cu_dev[dev] = n > 0 ? n : 256;
-  }
-  return K == 384 ? launch_linear_swiglu_t<24>(A, W, out, T, I, num_cu_dev[dev], stream)
-                  : launch_linear_swiglu_t<12>(A, W, out, T, I, num_cu_dev[dev], stream);
+  const int num_cu = cu_count();
+  if (!num_cu) return -5;
+  if (kept)
+    return K == 384 ? launch_linear_regs_t<24, 4, kSwigluKept>(A, W, nullptr, out, kept, T, I, num_cu, stream)
+                    : launch_linear_regs_t<12, 4, kSwigluKept>(A, W, nullptr, out, kept, T, I, num_cu, stream);
+  if (K == 192) return launch_linear_regs_t<12, 4, kSwiglu>(A, W, nullptr, out, nullptr, T, I, num_cu, stream);
+  return T <= 1024 ? launch_linear_regs_t<24, 4, kSwiglu>(A, W, nullptr, out, nullptr, T, I, num_cu, stream)
+                   : launch_linear_regs_t<24, 8, kSwiglu>(A, W, nullptr, out, nullptr, T, I, num_cu, stream);
+}
+
+bool linear_regs_supported(int K, int N) { return (K == 384 || K == 192) && N % 64 == 0 && N >= 64; }
+
+// Against the library's products (us, library / this): K 384: 16384 rows and up; 25088 rows N 1280 33 / 31, N 2048 61 / 45, N 384
+// 26 / 18, N 1024 42 / 26; 50176 rows 66 / 53, 130 / 77, 42 / 25, 58 / 42.  K 192: 32768 rows N 640 26 / 18, 50176 32 / 23,
+// 100352 58 / 40.  With 12544 rows it depends on the tiles (N 1280 19.6 / 21, N 2048 44 / 27).  Bound by its stores.
+int launch_linear_regs(const void* x, const void* w, const void* bias, void* y, long long T, int N, int K, hipStream_t stream) {
+  if (!linear_regs_supported(K, N) || T <= 0 || T > 0x7fffffffLL - 64) return -95;
+  const int num_cu = cu_count();
+  if (!num_cu) return -5;
+  return K == 384 ? launch_linear_regs_t<24, 4, kLinear>(x, w, bias, y, nullptr, T, N, num_cu, stream)
+                  : launch_linear_regs_t<12, 4, kLinear>(x, w, bias, y, nullptr, T, N, num_cu, stream);
 }
 
 }  // namespace vig
-

@@ -96,6 +96,22 @@ Tensor weight_grad(const Tensor& dy, const Tensor& x, Tensor* bias_grad) {
   return dw;
 }
 
+bool aligned(const Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; }
+
+// x w^T (+ bias) for packed rows x [M, K], w [N, K]
+Tensor product(const Tensor& x, const Tensor& w, const Tensor& bias) {
+  const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
+  if (x.scalar_type() == at::kBFloat16 && vig_linear_preferred(M, (int)N, (int)K) && aligned(x) && aligned(w) &&
+      (!bias.defined() || aligned(bias))) {
+    Tensor y = at::empty({M, N}, x.options());
+    check_rc(vig_linear_fwd(x.data_ptr(), K, w.data_ptr(), bias.defined() ? bias.data_ptr() : nullptr, y.data_ptr(), N, M, (int)N, (int)K,
+                            stream_of(x)),
+             "vig_linear_fwd");
+    return y;
+  }
+  return bias.defined() ? at::addmm(bias, x, w.t()) : at::mm(x, w.t());
+}
+
 // residual-add + RMS norm: (y, sum); without a residual the sum is x itself
 std::pair<Tensor, Tensor> norm_fwd(const Tensor& x, const Tensor& residual, const float* weight, double eps, at::ScalarType type) {
   const int64_t C = x.size(-1), rows = x.numel() / C;
@@ -194,7 +210,7 @@ struct MixNode : torch::autograd::Function<MixNode> {
     check_rc(vig_dwconv3x3_fwd_pre(y.data_ptr(), f32(conv_w, 1), conv_b ? f32(*conv_b, 4) : nullptr, xs.data_ptr(),
                                    m.act ? pre.data_ptr() : nullptr, (int)m.B, (int)m.h, (int)m.w, (int)m.C, m.act, m.code(), stream),
              "vig_dwconv3x3_fwd_pre");
-    const Tensor z = at::addmm(b_in, xs.view({m.rows, m.C}), w_in.t());
+    const Tensor z = product(xs.view({m.rows, m.C}), w_in, b_in);
     Tensor q = at::empty({m.B, m.H, m.L, m.Dk}, opts), k = at::empty_like(q), v = at::empty({m.B, m.H, m.L, m.Dv}, opts);
     check_rc(vig_split_heads_fwd(z.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), (int)m.B, (int)m.L, (int)m.H, (int)m.Dk,
                                  (int)m.Dv, m.nz, m.code(), stream),
@@ -218,7 +234,7 @@ struct MixNode : torch::autograd::Function<MixNode> {
     check_rc(vig_locality_blend_fwd(o.data_ptr(), xs.data_ptr(), at_elem(z, m.n0), f32(g_norm, 2), f32(l_norm, 3), blend.data_ptr(),
                                     (int)m.B, (int)m.H, (int)m.L, (int)m.Dv, m.nz, (float)m.eps, m.out_act, m.code(), stream),
              "vig_locality_blend_fwd");
-    const Tensor a = at::mm(blend.view({m.rows, m.V}), w_out.t()).view({m.B, m.L, m.C});
+    const Tensor a = product(blend.view({m.rows, m.V}), w_out, Tensor()).view({m.B, m.L, m.C});
 
     ctx->set_materialize_grads(false);
     ctx->save_for_backward({sum, y, xs, pre, z, q, k, v, gates, gate_lin, o, blend, packed, small, norm_w, conv_w, g_norm, l_norm,
@@ -352,10 +368,17 @@ struct MlpNode : torch::autograd::Function<MlpNode> {
     if (!wide) f.add(norm_w, C), small = f.run(at::kFloat, branch);
     const Tensor wg = same ? gate_w : matrix(packed, gate_off, 2 * I, C), wd = same ? down_w : matrix(packed, down_off, C, I);
     auto [y, sum] = norm_fwd(branch, residual, wide ? fptr(norm_w) : fptr(small), eps, type);
-    const Tensor z = at::mm(y.view({rows, C}), wg.t());
-    Tensor prod = at::empty({rows, I}, z.options());
-    check_rc(vig_swiglu_fwd(z.data_ptr(), prod.data_ptr(), rows, (int)I, dtype_code(z), stream_of(z)), "vig_swiglu_fwd");
-    const Tensor out = at::mm(prod, wd.t()).view(branch.sizes());
+    Tensor z, prod = at::empty({rows, I}, y.options());
+    if (type == at::kBFloat16 && (C == 384 || C == 192) && I % 32 == 0 && aligned(y) && aligned(wg)) {
+      z = at::empty({rows, 2 * I}, y.options());
+      check_rc(vig_linear_swiglu_kept_fwd(y.data_ptr(), wg.data_ptr(), z.data_ptr(), prod.data_ptr(), rows, (int)C, (int)I, VIG_BF16,
+                                          stream_of(z)),
+               "vig_linear_swiglu_kept_fwd");
+    } else {
+      z = product(y.view({rows, C}), wg, Tensor());
+      check_rc(vig_swiglu_fwd(z.data_ptr(), prod.data_ptr(), rows, (int)I, dtype_code(z), stream_of(z)), "vig_swiglu_fwd");
+    }
+    const Tensor out = product(prod, wd, Tensor()).view(branch.sizes());
     ctx->set_materialize_grads(false);
     ctx->save_for_backward({sum, y, z, prod, packed, small, norm_w, gate_w, down_w});
     ctx->saved_data["at"] = std::vector<int64_t>{gate_off, down_off, bf16, branch.scalar_type() != sum.scalar_type()};
