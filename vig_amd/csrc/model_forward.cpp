@@ -154,7 +154,8 @@ Tensor run(const Plan& p, const Tensor& images) {
   if (!whole) q = k.take(T * K2 / 2), kk = k.take(T * K2 / 2), v = k.take(T * C), ws = k.take((int64_t)(gla_ws + 1) / 2);
   int64_t most = k.used;
   k.used = region;
-  const int64_t mid = k.take(T * I), wide = k.take(T * 2 * I);
+  const bool swiglu_kernel = (C == 384 || C == 192) && I % 32 == 0;
+  const int64_t mid = k.take(T * I), wide = swiglu_kernel ? 0 : k.take(T * 2 * I);
   most = std::max(most, k.used);
   k.used = region;
   const int64_t c1 = k.take(n1 * half), c1n = k.take(n1 * half);
@@ -222,7 +223,7 @@ Tensor run(const Plan& p, const Tensor& images) {
     k.norm(branch1, hidden, b.norm2, b.eps2, false, y, next, T);
     residual = next;
     const int64_t width = b.w_down.size(1);
-    if ((C == 384 || C == 192) && width % 32 == 0) {
+    if (swiglu_kernel && width % 32 == 0) {
       check_rc(vig_linear_swiglu_fwd(k.at(y), b.w_gate.data_ptr(), k.at(mid), T, (int)C, (int)width, VIG_BF16, k.stream),
                "vig_linear_swiglu_fwd");
     } else {

@@ -708,20 +708,41 @@ class ViG(nn.Module):
                   torch.nn.modules.module._global_forward_pre_hooks]
         flag = lambda v: 1 if v else 0  # noqa: E731
         with torch.no_grad():
-            stem = (pe._packed_w1(), _f32(pe, "b1", conv1.bias), _f32(norm1, "w", norm1.weight), _f32(norm1, "b", norm1.bias), norm1.eps,
-                    conv2.weight.detach().permute(0, 2, 3, 1).contiguous(), _f32(pe, "b2", conv2.bias), _f32(norm2, "w", norm2.weight),
-                    _f32(norm2, "b", norm2.bias), norm2.eps, self.pos_embed.detach().contiguous(), *conv1.kernel_size, *self.patch_resolution)
-            blocks = []
+            # all small weights in fp32 by one concatenation and one cast, all stacked projections by one concatenation: layer by
+            # layer these are 150 launches, 0.9 ms of a new model's first pass
+            small = [conv1.bias, norm1.weight, norm1.bias, conv2.bias, norm2.weight, norm2.bias, self.norm.weight]
+            rows, biases = [], []
+            zero = self.head.weight.new_zeros(max(m.weight.numel() for m in (self.blocks[0].attn.qkv_proj, self.blocks[0].attn.g_proj)))
             for blk in self.blocks:
+                at, C = blk.attn, self.embed_dim
+                conv, srcs = at.in_proj[0], (at.qkv_proj.weight, at.g_proj.weight, at.gk_proj[0].weight)
+                n = [t.shape[0] for t in srcs]
+                pad = -sum(n) % 128
+                rows += [*srcs, zero[:pad * C].view(pad, C)]
+                biases += [zero[:n[0]], at.g_proj.bias, zero[:n[2] + pad]]
+                small += [blk.attn_norm.weight, conv.weight, conv.bias, at.g_norm.weight, at.l_norm.weight, blk.mlp_norm.weight]
+            dev = zero.device
+            if any(t is not None and (t.device != dev or t.dtype is not torch.bfloat16) for t in small + rows + biases):
+                return None
+            flat = [t.reshape(-1) for t in small if t is not None]
+            parts = iter(torch.cat(flat).float().split([t.numel() for t in flat]))
+            f32 = [next(parts) if t is not None else None for t in small]
+            heights = [sum(t.shape[0] for t in rows[i:i + 4]) for i in range(0, len(rows), 4)]
+            w_in, b_in = torch.cat(rows).split(heights), torch.cat(biases).split(heights)
+            b1, ln1w, ln1b, b2, ln2w, ln2b, norm_w = f32[:7]
+            stem = (pe._packed_w1(), b1, ln1w, ln1b, norm1.eps,
+                    conv2.weight.detach().permute(0, 2, 3, 1), b2, ln2w, ln2b, norm2.eps,
+                    self.pos_embed.detach(), *conv1.kernel_size, *self.patch_resolution)
+            blocks = []
+            for i, blk in enumerate(self.blocks):
                 at, mlp = blk.attn, blk.mlp
-                conv, up = at.in_proj[0], at.gk_proj[1]
-                w_in, b_in = at._stacked_in()
-                blocks.append((blk.attn_norm._w32(), blk.attn_norm.eps, _f32(at, "conv_w_flat", conv.weight, (-1,)),
-                               _f32(at, "conv_b", conv.bias), flag(at.use_act_in_conv), w_in, b_in, at.num_heads, at.head_qk_dim,
-                               at.head_v_dim, up.weight.detach(), up.bias.detach(), float(at.gate_logit_normalizer), at.clamp_min,
-                               at.g_norm._w32(), at.l_norm._w32(), at.layernorm_eps, flag(at.use_out_act), at.o_proj.weight.detach(),
-                               blk.mlp_norm._w32(), blk.mlp_norm.eps, mlp.gate_proj.weight.detach(), mlp.down_proj.weight.detach()))
-            tail = (self.norm._w32(), self.norm.eps, self.head.weight.detach(), self.head.bias.detach() if self.head.bias is not None else None)
+                up = at.gk_proj[1]
+                attn_norm, conv_w, conv_b, g_norm, l_norm, mlp_norm = f32[7 + 6 * i:13 + 6 * i]
+                blocks.append((attn_norm, blk.attn_norm.eps, conv_w, conv_b, flag(at.use_act_in_conv), w_in[i], b_in[i], at.num_heads,
+                               at.head_qk_dim, at.head_v_dim, up.weight.detach(), up.bias.detach(), float(at.gate_logit_normalizer),
+                               at.clamp_min, g_norm, l_norm, at.layernorm_eps, flag(at.use_out_act), at.o_proj.weight.detach(),
+                               mlp_norm, blk.mlp_norm.eps, mlp.gate_proj.weight.detach(), mlp.down_proj.weight.detach()))
+            tail = (norm_w, self.norm.eps, self.head.weight.detach(), self.head.bias.detach() if self.head.bias is not None else None)
         return calls.make_plan(self, settings, absent, called, stem, blocks, tail)
 
 
