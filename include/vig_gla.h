@@ -519,6 +519,18 @@ int vig_linear_swiglu_fwd(const void* x, const void* weight, void* y, long long 
 /* The same, leaving gate | up as well: gate_up [rows, 2*I], what the backward of the product reads. */
 int vig_linear_swiglu_kept_fwd(const void* x, const void* weight, void* gate_up, void* y, long long rows, int K, int I,
                                int io_dtype, void* stream);
+/*
+ * The input gradient of down_proj and the backward of the SwiGLU product in one kernel: d = d_out [rows, K] . w_down [K, I] rounded
+ * to bf16, d_gate_up [rows, 2*I] as vig_swiglu_bwd gives it for (gate_up, d).  K = 384 or 192, I % 32 == 0, bf16.
+ */
+int vig_linear_swiglu_bwd(const void* d_out, const void* w_down, const void* gate_up, void* d_gate_up, long long rows, int K, int I,
+                          int io_dtype, void* stream);
+/*
+ * The input gradient of a linear layer, dx [rows, K] = dy [rows, N] . weight [N, K], bf16, fp32 accumulation; N = 384 or 192,
+ * K % 64 == 0 (else VIG_ENOTSUP).  _preferred: whether it is the better choice next to a BLAS library.
+ */
+int vig_linear_bwd_input_preferred(long long rows, int N, int K);
+int vig_linear_bwd_input(const void* dy, const void* weight, void* dx, long long rows, int N, int K, int io_dtype, void* stream);
 
 /*
  * vig_locality_blend_fwd and o_proj in one kernel, for square blocks with 64-channel heads at the widths whose weight

@@ -51,3 +51,32 @@ def test_linear_swiglu_forms(rows, K, I):
     # a pre-activation that another summation order rounds the other way moves the product by an ulp of each factor
     g, u = want.chunk(2, 1)
     _check(got, torch.nn.functional.silu(g) * u, ulps=4.0)
+
+
+# products with the weight's columns: the first size of the rule and below it, ragged tokens, channel tiles of part of a workgroup
+@pytest.mark.parametrize("rows,N,K", [(1, 192, 64), (33, 384, 704), (16384, 384, 384), (16399, 192, 320)])
+def test_linear_bwd_input(rows, N, K):
+    announce(f"linear input gradient rows{rows} N{N} K{K}")
+    dy, w = _randn((rows, N), 11), _randn((N, K), 12, N ** -0.5)
+    lib, dyd, wd = _lib.load(), dy.cuda(), w.cuda()
+    dx = torch.full((rows, K), float("nan"), dtype=torch.bfloat16, device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+    assert lib.vig_linear_bwd_input(dyd.data_ptr(), wd.data_ptr(), dx.data_ptr(), rows, N, K, _lib.VIG_BF16, stream) == 0
+    _check(dx, dy.double() @ w.double())
+    assert bool(lib.vig_linear_bwd_input_preferred(rows, N, K)) == (rows >= 16384)
+    assert lib.vig_linear_bwd_input(dyd.data_ptr(), wd.data_ptr(), dx.data_ptr(), rows, N, 32, _lib.VIG_BF16, stream) != 0
+
+
+@pytest.mark.parametrize("rows,K,I", [(1, 192, 32), (37, 384, 96), (2049, 192, 160), (9001, 384, 288)])
+def test_linear_swiglu_bwd(rows, K, I):
+    announce(f"linear_swiglu_bwd rows{rows} K{K} I{I}")
+    dy, w, z = _randn((rows, K), 13), _randn((K, I), 14, K ** -0.5), _randn((rows, 2 * I), 15)
+    lib, dyd, wd, zd = _lib.load(), dy.cuda(), w.cuda(), z.cuda()
+    dz = torch.full((rows, 2 * I), float("nan"), dtype=torch.bfloat16, device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+    assert lib.vig_linear_swiglu_bwd(dyd.data_ptr(), wd.data_ptr(), zd.data_ptr(), dz.data_ptr(), rows, K, I, _lib.VIG_BF16, stream) == 0
+    d = dy.double() @ w.double()
+    g, u = z.double().chunk(2, 1)
+    s = torch.sigmoid(g)
+    want = torch.cat((d * u * s * (1 + g * (1 - s)), d * g * s), 1)
+    _check(dz, want, ulps=2.0)  # one rounding of the product's gradient, one of the result

@@ -51,6 +51,9 @@ SIGNATURES = {
     "vig_split_heads_fwd": (_c_int, [_c_void_p] * 4 + [_c_int] * 5 + [_c_longlong, _c_int, _c_void_p]),
     "vig_locality_blend_linear_fwd": (_c_int, [_c_void_p] * 7 + [_c_int] * 5 + [_c_longlong, _c_float, _c_int, _c_int, _c_void_p]),
     "vig_linear_swiglu_kept_fwd": (_c_int, [_c_void_p] * 4 + [_c_longlong, _c_int, _c_int, _c_int, _c_void_p]),
+    "vig_linear_swiglu_bwd": (_c_int, [_c_void_p] * 4 + [_c_longlong, _c_int, _c_int, _c_int, _c_void_p]),
+    "vig_linear_bwd_input_preferred": (_c_int, [_c_longlong, _c_int, _c_int]),
+    "vig_linear_bwd_input": (_c_int, [_c_void_p] * 3 + [_c_longlong, _c_int, _c_int, _c_int, _c_void_p]),
     "vig_linear_swiglu_fwd": (_c_int, [_c_void_p] * 3 + [_c_longlong, _c_int, _c_int, _c_int, _c_void_p]),
     "vig_patch_conv_fwd": (_c_int, [_c_void_p] * 3 + [_c_int] * 10 + [_c_void_p]),
     "vig_locality_blend_bwd_workspace": (_c_size_t, [_c_int] * 3),

@@ -652,6 +652,25 @@ int vig_linear_swiglu_kept_fwd(const void* x, const void* weight, void* gate_up,
   return vig::launch_linear_swiglu(x, weight, y, gate_up, rows, K, I, (hipStream_t)stream);
 }
 
+int vig_linear_swiglu_bwd(const void* d_out, const void* w_down, const void* gate_up, void* d_gate_up, long long rows, int K, int I,
+                          int io_dtype, void* stream) {
+  if (!d_out || !w_down || !gate_up || !d_gate_up || rows <= 0 || K <= 0 || I <= 0) return VIG_EINVAL;
+  if (io_dtype != VIG_BF16 || !vig::linear_swiglu_supported(K, I)) return VIG_ENOTSUP;
+  if (!strided_rows_ok(d_out, K, io_dtype) || !strided_rows_ok(w_down, I, io_dtype) || !strided_rows_ok(gate_up, 2LL * I, io_dtype) ||
+      !strided_rows_ok(d_gate_up, 2LL * I, io_dtype))
+    return VIG_EINVAL;
+  return vig::launch_linear_swiglu_bwd(d_out, w_down, gate_up, d_gate_up, rows, K, I, (hipStream_t)stream);
+}
+
+int vig_linear_bwd_input_preferred(long long rows, int N, int K) { return rows >= 16384 && vig::linear_regs_supported(N, K); }
+
+int vig_linear_bwd_input(const void* dy, const void* weight, void* dx, long long rows, int N, int K, int io_dtype, void* stream) {
+  if (!dy || !weight || !dx || rows <= 0 || N <= 0 || K <= 0) return VIG_EINVAL;
+  if (io_dtype != VIG_BF16 || !vig::linear_regs_supported(N, K)) return VIG_ENOTSUP;
+  if (!strided_rows_ok(dy, N, io_dtype) || !strided_rows_ok(weight, K, io_dtype) || !strided_rows_ok(dx, K, io_dtype)) return VIG_EINVAL;
+  return vig::launch_linear_columns(dy, weight, dx, rows, K, N, (hipStream_t)stream);
+}
+
 int vig_swiglu_fwd(const void* gate_up, void* out, long long rows, int I, int io_dtype, void* stream) {
   if (!gate_up || !out || rows <= 0 || I <= 0) return VIG_EINVAL;
   if (!aligned16(gate_up, out)) return VIG_EINVAL;

@@ -111,6 +111,9 @@ int launch_gla_backward_mfma(const void* q, const void* k, const void* v, const 
 // bf16 row products (gemm.hip, linear.hip): a layer whose weights stay in registers, and SwiGLU of a layer over few rows
 bool linear_regs_supported(int K, int N);
 int launch_linear_regs(const void* x, const void* w, const void* bias, void* y, long long T, int N, int K, hipStream_t stream);
+int launch_linear_columns(const void* x, const void* w, void* y, long long T, int N, int K, hipStream_t stream);
+int launch_linear_swiglu_bwd(const void* d_out, const void* w_down, const void* kept, void* d_kept, long long T, int K, int I,
+                             hipStream_t stream);
 bool few_swiglu(long long T, int K, int I);
 int launch_few_swiglu(const void* x, const void* w, void* y, long long T, int K, int I, hipStream_t stream);
 

@@ -68,11 +68,51 @@ __device__ __forceinline__ void load_weight_tiles(u32x4_t (&w)[NT][KS], const ui
   }
 }
 
+// The same for tiles of 32 columns of a W [K, ldw] (the products of a backward, d_x = d_y . W): pieces of 64 rows of 64 bytes, and
+// ds_read_b64_tr_b16 hands every lane of a group of sixteen four contraction elements of its channel out of a 4 x 16 block.
+typedef short s16x4_t __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s16x4_t* lds_s16x4_t;
+template <int KS, int NT>
+__device__ __forceinline__ void load_weight_columns(u32x4_t (&w)[NT][KS], const uint16_t* const* first, int ldw, char* ring, int lane) {
+  static_assert(KS % 4 == 0, "whole pieces");
+  constexpr int KC = KS / 4, NQ = NT * KC;
+  const int h = lane >> 5, half = (lane >> 4) & 1, block = lane & 3;  // (source lane: row (lane >> 2) & 3 of the block, four columns)
+  const uint32_t ring0 = __builtin_amdgcn_readfirstlane(lds_offset(ring));
+  const int at = ((8 * h + ((lane >> 2) & 3)) * 32 + channel_of_row(16 * half + 4 * block)) * 2;
+  const auto fetch = [&](int q) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      load_to_lds16(first[q / KC] + (size_t)(64 * (q % KC) + 16 * i + (lane >> 2)) * ldw + 8 * (lane & 3),
+                    ring0 + (q % kRing) * 4096 + 1024 * i);
+  };
+#pragma unroll
+  for (int q = 0; q < kRing; ++q) fetch(q);
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    if (q + 1 < NQ) wait_vmem<4 * (kRing - 1)>();
+    else wait_vmem<0>();
+    char* buf = ring + (q % kRing) * 4096 + at;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const s16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t)(buf + 1024 * t));
+      const s16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t)(buf + 1024 * t + 256));
+      const u32x2_t l = __builtin_bit_cast(u32x2_t, lo), u = __builtin_bit_cast(u32x2_t, hi);
+      w[q / KC][4 * (q % KC) + t] = u32x4_t{l[0], l[1], u[0], u[1]};
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (q + kRing < NQ) fetch(q + kRing);
+  }
+}
+
 // What a wave makes of its two 32-row tiles of W (rows from c0 and from c1):
 //   kSwiglu      c0 = gate, c1 = up channels of one tile: the SwiGLU product
 //   kSwigluKept  the same, and the gate and up values themselves ([T, 2*I], what a backward reads)
 //   kLinear      64 channels of a plain layer, + bias
-enum LinForm { kSwiglu, kSwigluKept, kLinear };
+//   kColumns     the same for W [K, N]
+//   kSwigluBwd   one tile of columns of the down projection's W [K, N]: the gradient of the SwiGLU product (rounded to bf16, as
+//                the separate layer would store it) goes through the product's backward with the kept gate and up values:
+//                out = their gradients [T, 2*N]
+enum LinForm { kSwiglu, kSwigluKept, kLinear, kColumns, kSwigluBwd };
 
 template <int KS, int NW, LinForm FORM>
 __global__ __launch_bounds__(64 * NW, 2) void linear_regs_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ W,
@@ -82,8 +122,10 @@ __global__ __launch_bounds__(64 * NW, 2) void linear_regs_kernel(const uint16_t*
   constexpr int kCols = K / 8;                 // 16-byte chunks per token row
   constexpr int kRow = K + 8;                  // LDS row stride in elements (conflict-free 16-byte reads)
   constexpr int kPer = 32 / NW;                // token rows per wave
-  constexpr int kStep = FORM == kLinear ? 64 : 32;                             // channels of `out` per wave
-  constexpr int kStores = FORM == kSwiglu ? 2 : FORM == kLinear ? 4 : 6;       // of a whole tile's epilogue
+  constexpr bool kPlain = FORM == kLinear || FORM == kColumns;
+  constexpr int kStep = kPlain ? 64 : 32;                                       // channels per wave
+  constexpr int kStores = FORM == kSwiglu ? 2 : FORM == kSwigluKept ? 6 : 4;   // of a whole tile's epilogue
+  constexpr int kTiles = FORM == kSwigluBwd ? 1 : 2;
   static_assert(kCols <= 64 && 32 % NW == 0, "a wave loads whole token rows");
   extern __shared__ __align__(16) char smem[];
   // [biases][2][32][kRow]; the weights' ring lies where the second of the two tiles will
@@ -115,10 +157,17 @@ __global__ __launch_bounds__(64 * NW, 2) void linear_regs_kernel(const uint16_t*
         load_to_lds16(A + (size_t)tile * (32 * K) + (size_t)row * K + lane * 8, base + row * (kRow * 2));
     }
   };
-  u32x4_t wt[2][KS];
+  u32x4_t wt[kTiles][KS];
   f32x16_t g, u;
 #pragma unroll
   for (int j = 0; j < 16; ++j) g[j] = 0.f, u[j] = 0.f;
+  // the kept gate and up values behind a tile's gradients, fetched ahead of its products
+  u32x4_t z[4];
+  auto fetch_kept = [&](int tile) {
+    const uint16_t* p = kept + (size_t)min(tile * 32 + r, T - 1) * 2 * N + (have ? 32 * ct : 0) + 16 * h;
+    z[0] = *reinterpret_cast<const u32x4_t*>(p), z[1] = *reinterpret_cast<const u32x4_t*>(p + 8);
+    z[2] = *reinterpret_cast<const u32x4_t*>(p + N), z[3] = *reinterpret_cast<const u32x4_t*>(p + N + 8);
+  };
   auto store32 = [](uint16_t* dst, const u32x4_t& lo, const u32x4_t& hi) {
     *reinterpret_cast<u32x4_t*>(dst) = lo;
     *reinterpret_cast<u32x4_t*>(dst + 8) = hi;
@@ -127,14 +176,30 @@ __global__ __launch_bounds__(64 * NW, 2) void linear_regs_kernel(const uint16_t*
   auto epilogue = [&](int etile) {
     const int token = etile * 32 + r;
     u32x4_t lo, hi, glo, ghi, ulo, uhi;
-    if constexpr (FORM != kSwiglu) {
+    if constexpr (FORM == kSwigluBwd) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const uint32_t zg = z[j >> 2][j & 3], zu = z[2 + (j >> 2)][j & 3];
+        float dg[2], du[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const float d = bf16_to_f32(f32_to_bf16(g[2 * j + e]));
+          const float gv = e ? bf16hi_to_f32(zg) : bf16lo_to_f32(zg), uv = e ? bf16hi_to_f32(zu) : bf16lo_to_f32(zu);
+          const float sg = sigmoidf_(gv);
+          du[e] = d * gv * sg;
+          dg[e] = d * uv * sg * (1.f + gv * (1.f - sg));
+        }
+        (j < 4 ? glo : ghi)[j & 3] = pack_bf16x2(dg[0], dg[1]);
+        (j < 4 ? ulo : uhi)[j & 3] = pack_bf16x2(du[0], du[1]);
+      }
+    } else if constexpr (FORM != kSwiglu) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         glo[j] = pack_bf16x2(g[2 * j], g[2 * j + 1]), ghi[j] = pack_bf16x2(g[8 + 2 * j], g[8 + 2 * j + 1]);
         ulo[j] = pack_bf16x2(u[2 * j], u[2 * j + 1]), uhi[j] = pack_bf16x2(u[8 + 2 * j], u[8 + 2 * j + 1]);
       }
     }
-    if constexpr (FORM != kLinear) {
+    if constexpr (FORM == kSwiglu || FORM == kSwigluKept) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         float y[2];
@@ -155,10 +220,14 @@ __global__ __launch_bounds__(64 * NW, 2) void linear_regs_kernel(const uint16_t*
       }
     }
     if (have && token < T) {
-      if constexpr (FORM == kLinear) {
+      if constexpr (kPlain) {
         uint16_t* dst = out + (size_t)token * N + 64 * ct + 16 * h;
         store32(dst, glo, ghi);
         store32(dst + 32, ulo, uhi);
+      } else if constexpr (FORM == kSwigluBwd) {
+        uint16_t* dst = out + (size_t)token * 2 * N + 32 * ct + 16 * h;
+        store32(dst, glo, ghi);
+        store32(dst + N, ulo, uhi);
       } else {
         if constexpr (FORM == kSwigluKept) {
           uint16_t* dst = kept + (size_t)token * 2 * N + 32 * ct + 16 * h;
@@ -184,7 +253,7 @@ __global__ __launch_bounds__(64 * NW, 2) void linear_regs_kernel(const uint16_t*
       for (int j = 0; j < 16; ++j) g[j] = 0.f, u[j] = 0.f;
     }
     const uint16_t* xrow = mine + r * kRow + 8 * h;
-    constexpr int kAhead = FORM == kSwiglu || KS < 24 ? 3 : 2;  // (as the registers allow)
+    constexpr int kAhead = FORM == kSwiglu || FORM == kSwigluBwd || KS < 24 ? 3 : 2;  // (as the registers allow)
     u32x4_t x[kAhead];
 #pragma unroll
     for (int t = 0; t < kAhead; ++t) x[t] = *reinterpret_cast<const u32x4_t*>(xrow + 16 * t);
@@ -193,17 +262,25 @@ __global__ __launch_bounds__(64 * NW, 2) void linear_regs_kernel(const uint16_t*
       const u32x4_t xt = x[t % kAhead];
       g = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, wt[0][t]), __builtin_bit_cast(bf16x8_t, xt),
                                                   g, 0, 0, 0);
-      u = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, wt[1][t]), __builtin_bit_cast(bf16x8_t, xt),
-                                                  u, 0, 0, 0);
+      if constexpr (kTiles == 2)
+        u = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, wt[kTiles - 1][t]), __builtin_bit_cast(bf16x8_t, xt),
+                                                    u, 0, 0, 0);
       if (t + kAhead < KS) x[t % kAhead] = *reinterpret_cast<const u32x4_t*>(xrow + 16 * (t + kAhead));
       __builtin_amdgcn_sched_barrier(0);
     }
   };
   fetch(worker, 0);
   {
-    const uint16_t* const w0 = W + (size_t)(have ? kStep * (cg * NW + uwave) : 0) * K;
-    const uint16_t* const first[2] = {w0, w0 + (size_t)(FORM == kLinear ? (have ? 32 : 0) : N) * K};
-    load_weight_tiles<KS, 2>(wt, first, smem + kBias + kTile + uwave * (kRing * 4096), lane);
+    char* const ring = smem + kBias + kTile + uwave * (kRing * 4096);
+    const int c0 = have ? kStep * (cg * NW + uwave) : 0;
+    if constexpr (FORM == kColumns || FORM == kSwigluBwd) {
+      const uint16_t* const first[2] = {W + c0, W + c0 + 32};
+      load_weight_columns<KS, kTiles>(wt, first, N, ring, lane);
+    } else {
+      const uint16_t* const w0 = W + (size_t)c0 * K;
+      const uint16_t* const first[2] = {w0, w0 + (size_t)(FORM == kLinear ? 32 : N) * K};
+      load_weight_tiles<KS, 2>(wt, first, ring, lane);
+    }
   }
   int cur = 0;
   bool stored = false;  // an epilogue's stores were issued after the current tile's loads (a full tile's: only the last
@@ -215,6 +292,7 @@ __global__ __launch_bounds__(64 * NW, 2) void linear_regs_kernel(const uint16_t*
     if (stored) wait_vmem<kStores>();
     else wait_vmem<0>();
     tile_barrier();  // the tile is complete; the other buffer was last read before the previous barrier
+    if constexpr (FORM == kSwigluBwd) fetch_kept(tile);
     fetch(tile + nworkers, cur ^ 1);
     // The two waves of a SIMD (w and w + 4 of eight) take turns on its two pipes: the lower wave runs this tile's matrix
     // instructions first and its epilogue after; the upper wave first runs the epilogue of its PREVIOUS tile
@@ -246,7 +324,7 @@ bool allow_lds(const void* kernel, size_t bytes, bool (&done)[64]) {
 template <int KS, int NW, LinForm FORM>
 int launch_linear_regs_t(const void* A, const void* W, const void* bias, void* out, void* kept, long long T, int N, int num_cu,
                          hipStream_t stream) {
-  constexpr int K = 16 * KS, kStep = FORM == kLinear ? 64 : 32;
+  constexpr int K = 16 * KS, kStep = FORM == kLinear || FORM == kColumns ? 64 : 32;
   constexpr size_t tile = 32 * (K + 8) * sizeof(uint16_t), ring = (size_t)NW * kRing * 4096;
   constexpr size_t lds = (FORM == kLinear ? 64 * NW * sizeof(float) : 0) + tile + (tile > ring ? tile : ring);
   static bool done[64] = {};
@@ -533,6 +611,25 @@ int launch_linear_regs(const void* x, const void* w, const void* bias, void* y, 
   if (!num_cu) return -5;
   return K == 384 ? launch_linear_regs_t<24, 4, kLinear>(x, w, bias, y, nullptr, T, N, num_cu, stream)
                   : launch_linear_regs_t<12, 4, kLinear>(x, w, bias, y, nullptr, T, N, num_cu, stream);
+}
+
+// d_x = d_y . W for W [K, N] as it lies (K the layer's width out, N its width in)
+int launch_linear_columns(const void* x, const void* w, void* y, long long T, int N, int K, hipStream_t stream) {
+  if (!linear_regs_supported(K, N) || T <= 0 || T > 0x7fffffffLL - 64) return -95;
+  const int num_cu = cu_count();
+  if (!num_cu) return -5;
+  return K == 384 ? launch_linear_regs_t<24, 4, kColumns>(x, w, nullptr, y, nullptr, T, N, num_cu, stream)
+                  : launch_linear_regs_t<12, 4, kColumns>(x, w, nullptr, y, nullptr, T, N, num_cu, stream);
+}
+
+int launch_linear_swiglu_bwd(const void* d_out, const void* w_down, const void* kept, void* d_kept, long long T, int K, int I,
+                             hipStream_t stream) {
+  if (!linear_swiglu_supported(K, I) || T <= 0 || T > 0x7fffffffLL - 64) return -95;
+  const int num_cu = cu_count();
+  if (!num_cu) return -5;
+  void* const z = const_cast<void*>(kept);  // (read only in this form)
+  return K == 384 ? launch_linear_regs_t<24, 4, kSwigluBwd>(d_out, w_down, nullptr, d_kept, z, T, I, num_cu, stream)
+                  : launch_linear_regs_t<12, 4, kSwigluBwd>(d_out, w_down, nullptr, d_kept, z, T, I, num_cu, stream);
 }
 
 }  // namespace vig

@@ -112,6 +112,18 @@ Tensor product(const Tensor& x, const Tensor& w, const Tensor& bias) {
   return bias.defined() ? at::addmm(bias, x, w.t()) : at::mm(x, w.t());
 }
 
+// dy w for packed rows dy [M, N], w [N, K]
+Tensor input_grad(const Tensor& dy, const Tensor& w) {
+  const int64_t M = dy.size(0), N = w.size(0), K = w.size(1);
+  if (dy.scalar_type() == at::kBFloat16 && vig_linear_bwd_input_preferred(M, (int)N, (int)K) && dy.is_contiguous() && aligned(dy) && aligned(w)) {
+    Tensor dx = at::empty({M, K}, dy.options());
+    check_rc(vig_linear_bwd_input(dy.data_ptr(), w.data_ptr(), dx.data_ptr(), M, (int)N, (int)K, VIG_BF16, stream_of(dy)),
+             "vig_linear_bwd_input");
+    return dx;
+  }
+  return at::mm(dy, w);
+}
+
 // residual-add + RMS norm: (y, sum); without a residual the sum is x itself
 std::pair<Tensor, Tensor> norm_fwd(const Tensor& x, const Tensor& residual, const float* weight, double eps, at::ScalarType type) {
   const int64_t C = x.size(-1), rows = x.numel() / C;
@@ -269,7 +281,7 @@ struct MixNode : torch::autograd::Function<MixNode> {
 
     const Tensor da = grad_rows(grads[0], m.rows, m.C, xs, type);
     if (wants(kOutW)) out[2 + kOutW] = like_param(weight_grad(da, blend.view({m.rows, m.V}), nullptr), out_w, {m.C, m.V});
-    const Tensor d_blend = at::mm(da, w_out);
+    const Tensor d_blend = input_grad(da, w_out);
     // gradients of the stacked projection's columns, written in place by the three kernels that produce them
     Tensor dz = at::empty({m.rows, m.nz}, opts);
     Tensor d_o = at::empty_like(o), d_xs = at::empty({m.rows, m.C}, opts);
@@ -401,10 +413,16 @@ struct MlpNode : torch::autograd::Function<MlpNode> {
     variable_list out(7);
     const Tensor d_out = grad_rows(grads[0], rows, C, y, type);
     if (ctx->needs_input_grad(4)) out[4] = like_param(weight_grad(d_out, prod, nullptr), down_w, {C, I});
-    const Tensor d_prod = at::mm(d_out, wd);
     Tensor dz = at::empty_like(z);
-    check_rc(vig_swiglu_bwd(z.data_ptr(), d_prod.data_ptr(), dz.data_ptr(), rows, (int)I, dtype_code(z), stream_of(z)),
-             "vig_swiglu_bwd");
+    if (type == at::kBFloat16 && d_out.scalar_type() == type && (C == 384 || C == 192) && I % 32 == 0 && d_out.is_contiguous() && aligned(d_out) && aligned(wd)) {
+      check_rc(vig_linear_swiglu_bwd(d_out.data_ptr(), wd.data_ptr(), z.data_ptr(), dz.data_ptr(), rows, (int)C, (int)I, VIG_BF16,
+                                     stream_of(z)),
+               "vig_linear_swiglu_bwd");
+    } else {
+      const Tensor d_prod = input_grad(d_out, wd);
+      check_rc(vig_swiglu_bwd(z.data_ptr(), d_prod.data_ptr(), dz.data_ptr(), rows, (int)I, dtype_code(z), stream_of(z)),
+               "vig_swiglu_bwd");
+    }
     if (ctx->needs_input_grad(3)) out[3] = like_param(weight_grad(dz, y.view({rows, C}), nullptr), gate_w, {2 * I, C});
     const Tensor d_y = at::mm(dz, wg);
     const auto g = norm_bwd(sum, wide ? fptr(norm_w) : fptr(small), d_y, grads[1], off[3], ctx->needs_input_grad(2),
