@@ -63,7 +63,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_few_kernel(GemmArgs a) {
   Pixel px[2];
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
-    const int row = 16 * i + lrow, unit = place ^ ((row >> 1) & 3);
+    const int row = 16 * i + lrow, unit = place ^ ((row >> 2) & 3);
     const int m = min(m0 + row, a.M - 1), n = min(n0 + row, a.N - 1);
     if constexpr (TAPS) px[i] = pixel_of(a, m);
     xp[i] = a.x + (TAPS ? 0 : (size_t)m * a.ldx) + 8 * unit;
@@ -104,7 +104,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_few_kernel(GemmArgs a) {
     bf16x8_t xf[2], wf[kMats][2];
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
-      const int off = r * 64 + 16 * ((2 * k + h) ^ ((r >> 1) & 3));
+      const int off = r * 64 + 16 * ((2 * k + h) ^ ((r >> 2) & 3));
       xf[k] = *reinterpret_cast<const bf16x8_t*>(buf + off);
 #pragma unroll
       for (int j = 0; j < kMats; ++j) wf[j][k] = *reinterpret_cast<const bf16x8_t*>(buf + 2048 * (j + 1) + off);
@@ -159,8 +159,8 @@ __global__ __launch_bounds__(64 * NW) void gemm_few_kernel(GemmArgs a) {
 
 // ---------------------------------------------------------------------------
 // Many rows: tiles of 64 MI x 64 NI by four waves of 32 MI x 32 NI each, operands through kBuffers LDS stages of 32
-// contraction elements (64-byte row pieces, loaded directly to LDS; the 16-byte units of a piece are swapped by the row number so
-// that the eight lanes served together hit different banks).
+// contraction elements (64-byte row pieces, loaded directly to LDS; the 16-byte units of a piece are swapped by a quarter of the row
+// number: the sixteen lanes served together read four rows that start in each bank quarter, and their units differ).
 // ---------------------------------------------------------------------------
 template <int MI, int NI, int BUFS, bool TAPS>
 __global__ __launch_bounds__(256, (64 * (MI + NI) * 64 * BUFS <= 80 * 1024 ? 2 : 1)) void gemm_many_kernel(GemmArgs a, int tn, int tiles) {
@@ -182,7 +182,7 @@ __global__ __launch_bounds__(256, (64 * (MI + NI) * 64 * BUFS <= 80 * 1024 ? 2 :
 #pragma unroll
   for (int i = 0; i < MI; ++i) {
     const int row = 16 * (wave * MI + i) + lrow, m = min(m0 + row, a.M - 1);
-    const int unit = place ^ ((row >> 1) & 3);
+    const int unit = place ^ ((row >> 2) & 3);
     if constexpr (TAPS) px[i] = pixel_of(a, m);
     xp[i] = a.x + (TAPS ? 0 : (size_t)m * a.ldx) + 8 * unit;
   }
@@ -190,7 +190,7 @@ __global__ __launch_bounds__(256, (64 * (MI + NI) * 64 * BUFS <= 80 * 1024 ? 2 :
   for (int i = 0; i < NI; ++i) {
     const int row = 16 * (wave * NI + i) + lrow;  // matrix row: its channel is permuted inside its 32
     const int n = min(n0 + (row & ~31) + channel_of_row(row & 31), a.N - 1);
-    wp[i] = a.w + (size_t)n * a.K + 8 * (place ^ ((row >> 1) & 3));
+    wp[i] = a.w + (size_t)n * a.K + 8 * (place ^ ((row >> 2) & 3));
   }
   const int tap_stages = TAPS ? a.cin / kStageK : 1;
   const auto fetch = [&](int s) {
@@ -212,7 +212,7 @@ __global__ __launch_bounds__(256, (64 * (MI + NI) * 64 * BUFS <= 80 * 1024 ? 2 :
   int xoff[2], woff[2];
 #pragma unroll
   for (int k = 0; k < 2; ++k) {
-    const int unit = (2 * k + h) ^ ((r >> 1) & 3);
+    const int unit = (2 * k + h) ^ ((r >> 2) & 3);
     xoff[k] = (wm + r) * 64 + 16 * unit;
     woff[k] = TM * 64 + (wn + r) * 64 + 16 * unit;
   }

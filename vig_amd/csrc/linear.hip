@@ -114,6 +114,11 @@ __device__ __forceinline__ void load_weight_columns(u32x4_t (&w)[NT][KS], const 
 //                out = their gradients [T, 2*N]
 enum LinForm { kSwiglu, kSwigluKept, kLinear, kColumns, kSwigluBwd };
 
+// Bytes of LDS a wave turns its results in, none where they are stored as they lie.  Turned, an instruction writes whole 64-byte
+// rows: K 192 with the values kept, 50176 x 512, 42 -> 36 us; the SwiGLU backward, 50176 tokens, K 384 113 -> 100, K 192 41 -> 38.
+// The plain layers and the SwiGLU gain nothing at K 192, and at K 384 the addresses spill (50176 x 1280 53 -> 67 us).
+constexpr int turn_bytes(int KS, LinForm f) { return f == kSwigluBwd ? 4096 : f == kSwigluKept && KS == 12 ? 6144 : 0; }
+
 template <int KS, int NW, LinForm FORM>
 __global__ __launch_bounds__(64 * NW, 2) void linear_regs_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ W,
                                                                  const uint16_t* __restrict__ bias, uint16_t* __restrict__ out,
@@ -128,8 +133,9 @@ __global__ __launch_bounds__(64 * NW, 2) void linear_regs_kernel(const uint16_t*
   constexpr int kTiles = FORM == kSwigluBwd ? 1 : 2;
   static_assert(kCols <= 64 && 32 % NW == 0, "a wave loads whole token rows");
   extern __shared__ __align__(16) char smem[];
-  // [biases][2][32][kRow]; the weights' ring lies where the second of the two tiles will
+  // [biases][2][32][kRow][waves' results]; the weights' ring lies where the second of the two tiles will
   constexpr size_t kBias = FORM == kLinear ? 64 * NW * sizeof(float) : 0, kTile = 32 * kRow * sizeof(uint16_t);
+  constexpr int kTurn = turn_bytes(KS, FORM);
   float* const bias_lds = reinterpret_cast<float*>(smem);
   uint16_t* buf = reinterpret_cast<uint16_t*>(smem + kBias);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -171,6 +177,32 @@ __global__ __launch_bounds__(64 * NW, 2) void linear_regs_kernel(const uint16_t*
   auto store32 = [](uint16_t* dst, const u32x4_t& lo, const u32x4_t& hi) {
     *reinterpret_cast<u32x4_t*>(dst) = lo;
     *reinterpret_cast<u32x4_t*>(dst + 8) = hi;
+  };
+  // A lane ends with 16 channels of one token: stored as they lie, an instruction writes 16-byte pieces all over 32 rows.  Where
+  // registers allow, the results are turned in a wave's own piece of LDS first (units swapped by the row, against bank
+  // conflicts), so that four lanes write 64 consecutive bytes.
+  char* const turn = smem + kBias + 2 * kTile + uwave * kTurn;
+  // gate and up values (or their gradients) of a tile to [T, 2*N]
+  auto store_pair = [&](int etile, uint16_t* base, const u32x4_t& glo, const u32x4_t& ghi, const u32x4_t& ulo, const u32x4_t& uhi) {
+    if constexpr (kTurn > 0) {
+      char* const mine = turn + r * 128;
+      *reinterpret_cast<u32x4_t*>(mine + 16 * ((2 * h) ^ ((r >> 1) & 7))) = glo;
+      *reinterpret_cast<u32x4_t*>(mine + 16 * ((2 * h + 1) ^ ((r >> 1) & 7))) = ghi;
+      *reinterpret_cast<u32x4_t*>(mine + 16 * ((4 + 2 * h) ^ ((r >> 1) & 7))) = ulo;
+      *reinterpret_cast<u32x4_t*>(mine + 16 * ((5 + 2 * h) ^ ((r >> 1) & 7))) = uhi;
+      const int unit = lane & 7;
+      uint16_t* const dst = base + (size_t)(etile * 32) * 2 * N + 32 * ct + 8 * (unit & 3) + (unit & 4 ? N : 0);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int row = 8 * i + (lane >> 3);
+        const u32x4_t v = *reinterpret_cast<const u32x4_t*>(turn + row * 128 + 16 * (unit ^ ((row >> 1) & 7)));
+        if (have && etile * 32 + row < T) *reinterpret_cast<u32x4_t*>(dst + (size_t)row * 2 * N) = v;
+      }
+    } else if (have && etile * 32 + r < T) {
+      uint16_t* dst = base + (size_t)(etile * 32 + r) * 2 * N + 32 * ct + 16 * h;
+      store32(dst, glo, ghi);
+      store32(dst + N, ulo, uhi);
+    }
   };
   // one finished tile, 16 consecutive channels of one token per lane (SwiGLU on the rounded gate and up values)
   auto epilogue = [&](int etile) {
@@ -219,21 +251,24 @@ __global__ __launch_bounds__(64 * NW, 2) void linear_regs_kernel(const uint16_t*
         else hi[j - 4] = pk;
       }
     }
-    if (have && token < T) {
+    if constexpr (FORM == kSwigluBwd) store_pair(etile, out, glo, ghi, ulo, uhi);
+    if constexpr (FORM == kSwigluKept) store_pair(etile, kept, glo, ghi, ulo, uhi);
+    if constexpr (FORM == kSwigluKept && kTurn > 0) {
+      char* const mine = turn + 4096 + r * 64;
+      *reinterpret_cast<u32x4_t*>(mine + 16 * ((2 * h) ^ ((r >> 2) & 3))) = lo;
+      *reinterpret_cast<u32x4_t*>(mine + 16 * ((2 * h + 1) ^ ((r >> 2) & 3))) = hi;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int row = 16 * i + (lane >> 2);
+        const u32x4_t v = *reinterpret_cast<const u32x4_t*>(turn + 4096 + row * 64 + 16 * ((lane & 3) ^ ((row >> 2) & 3)));
+        if (have && etile * 32 + row < T) *reinterpret_cast<u32x4_t*>(out + (size_t)(etile * 32 + row) * N + 32 * ct + 8 * (lane & 3)) = v;
+      }
+    } else if (FORM != kSwigluBwd && have && token < T) {
       if constexpr (kPlain) {
         uint16_t* dst = out + (size_t)token * N + 64 * ct + 16 * h;
         store32(dst, glo, ghi);
         store32(dst + 32, ulo, uhi);
-      } else if constexpr (FORM == kSwigluBwd) {
-        uint16_t* dst = out + (size_t)token * 2 * N + 32 * ct + 16 * h;
-        store32(dst, glo, ghi);
-        store32(dst + N, ulo, uhi);
       } else {
-        if constexpr (FORM == kSwigluKept) {
-          uint16_t* dst = kept + (size_t)token * 2 * N + 32 * ct + 16 * h;
-          store32(dst, glo, ghi);
-          store32(dst + N, ulo, uhi);
-        }
         store32(out + (size_t)token * N + 32 * ct + 16 * h, lo, hi);
       }
     }
@@ -326,7 +361,8 @@ int launch_linear_regs_t(const void* A, const void* W, const void* bias, void* o
                          hipStream_t stream) {
   constexpr int K = 16 * KS, kStep = FORM == kLinear || FORM == kColumns ? 64 : 32;
   constexpr size_t tile = 32 * (K + 8) * sizeof(uint16_t), ring = (size_t)NW * kRing * 4096;
-  constexpr size_t lds = (FORM == kLinear ? 64 * NW * sizeof(float) : 0) + tile + (tile > ring ? tile : ring);
+  constexpr size_t two = tile + NW * turn_bytes(KS, FORM);
+  constexpr size_t lds = (FORM == kLinear ? 64 * NW * sizeof(float) : 0) + tile + (two > ring ? two : ring);
   static bool done[64] = {};
   if (!allow_lds((const void*)linear_regs_kernel<KS, NW, FORM>, lds, done)) return -5;
   const int ncg = (N / kStep + NW - 1) / NW;
