@@ -575,6 +575,18 @@ int vig_linear_fwd(const void* x, long long x_row_stride, const void* weight, co
                    long long rows, int N, int K, void* stream);
 
 /*
+ * A linear layer without bias, the residual add and the RMS norm behind it in one kernel, bf16, packed rows:
+ *   sum [rows, N] = residual + x [rows, K] . weight [N, K]^T (the product rounded to bf16, then the sum),  y = rms(sum) * norm_weight
+ * N = 192, K % 64 == 0, else VIG_ENOTSUP.  sum and y are not the inputs.  _preferred: whether it is the better
+ * choice next to a product and vig_rmsnorm_fwd with round_sum, which give the same values.
+ *
+ * Replaces: down_proj, the block's closing add and the next block's attn_norm (classification/models/vig.py:497,598,606).
+ */
+int vig_linear_norm_preferred(long long rows, int N, int K);
+int vig_linear_norm_fwd(const void* x, const void* weight, const void* residual, const float* norm_weight, void* y, void* sum,
+                        long long rows, int N, int K, float eps, void* stream);
+
+/*
  * 3x3 convolution, stride 2, padding 1, no bias, bf16 channels-last: x [B, H, W, Cin], weight [Cout, 3, 3, Cin] ->
  * y [B, (H+1)/2, (W+1)/2, Cout].  Cin % 32 == 0, Cout % 8 == 0.
  *

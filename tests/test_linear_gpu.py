@@ -80,3 +80,22 @@ def test_linear_swiglu_bwd(rows, K, I):
     s = torch.sigmoid(g)
     want = torch.cat((d * u * s * (1 + g * (1 - s)), d * g * s), 1)
     _check(dz, want, ulps=2.0)  # one rounding of the product's gradient, one of the result
+
+
+# whole rows in one workgroup: ragged row tiles, the shortest contractions (stages short of the buffers) and longer ones
+@pytest.mark.parametrize("rows,N,K", [(1, 192, 64), (129, 192, 128), (257, 192, 192), (4097, 192, 512), (16401, 192, 1024)])
+def test_linear_norm(rows, N, K):
+    announce(f"linear, residual add and norm rows{rows} N{N} K{K}")
+    x, w, res = _randn((rows, K), 16), _randn((N, K), 17, K ** -0.5), _randn((rows, N), 18)
+    nw = torch.rand(N, generator=torch.Generator().manual_seed(19)) + 0.5
+    lib, dev = _lib.load(), [t.cuda() for t in (x, w, res, nw)]
+    y, total = (torch.full((rows, N), float("nan"), dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    rc = lib.vig_linear_norm_fwd(*(t.data_ptr() for t in (*dev, y, total)), rows, N, K, 1e-5, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    product = x.double() @ w.double().t()
+    # one rounding of the product, one of the sum
+    err = (total.double().cpu() - (product + res.double())).abs()
+    assert (err <= 2.0 ** -8 * (product.abs() + (product + res.double()).abs()) + 1e-5 * product.abs().max()).all()
+    s = total.double().cpu()
+    _check(y, s / torch.sqrt((s * s).mean(1, keepdim=True) + 1e-5) * nw.double())  # of the sum that was stored
+    assert bool(lib.vig_linear_norm_preferred(rows, N, K)) == (rows >= 16384)

@@ -106,3 +106,19 @@ def test_native_forward(kw, side, B, monkeypatch):
     with torch.no_grad():
         same(model, x)
     same(model.eval().float(), x.float())
+
+
+# enough tokens for the row products with the norm behind them and the layers with their weights in registers
+@pytest.mark.parametrize("kw,side,B", [(dict(embed_dim=384, num_heads=6), 112, 337), (dict(embed_dim=192, num_heads=3, use_out_act=True), 528, 16)])
+def test_native_forward_many_tokens(kw, side, B, monkeypatch):
+    announce(f"native evaluation forward {kw} side {side} B {B}")
+    torch.manual_seed(1)
+    model = layers.ViG(img_size=side, depth=3, drop_path_rate=0.0, **kw).cuda().bfloat16().eval()
+    x = torch.randn(B, 3, side, side, device="cuda").bfloat16()
+    got = model(x).float()
+    assert model in layers._PLANS
+    monkeypatch.setattr(layers.ViG, "_planned", lambda self, x: None)
+    with torch.no_grad():
+        want = model(x).float()
+    # the same roundings; an fp32 sum in another order moves a bf16 value by an ulp here and there, through three blocks
+    assert ((got - want).norm() / want.norm()).item() <= 2.0 ** -8

@@ -71,6 +71,8 @@ SIGNATURES = {
                               [_c_size_t, _c_longlong, _c_int, _c_int, _c_void_p]),
     "vig_dirgate_lowrank_bwd": (_c_int, [_c_void_p, _c_longlong] + [_c_void_p] * 6 + [_c_longlong] + [_c_int] * 5 +
                                 [_c_float, _c_float, _c_int, _c_int, _c_void_p]),
+    "vig_linear_norm_preferred": (_c_int, [_c_longlong, _c_int, _c_int]),
+    "vig_linear_norm_fwd": (_c_int, [_c_void_p] * 6 + [_c_longlong, _c_int, _c_int, _c_float, _c_void_p]),
     "vig_linear_preferred": (_c_int, [_c_longlong, _c_int, _c_int]),
     "vig_linear_fwd": (_c_int, [_c_void_p, _c_longlong] + [_c_void_p] * 3 + [_c_longlong, _c_longlong, _c_int, _c_int, _c_void_p]),
     "vig_conv3x3s2_fwd": (_c_int, [_c_void_p] * 3 + [_c_int] * 5 + [_c_void_p]),

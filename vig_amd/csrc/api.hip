@@ -457,6 +457,17 @@ int vig_linear_fwd(const void* x, long long x_row_stride, const void* weight, co
   return vig::launch_linear(x, x_row_stride, weight, bias, y, y_row_stride, rows, N, K, (hipStream_t)stream);
 }
 
+// (16384 rows 14.3 us against 19.6 of a product and a norm; 8192 13.0 / 13.3, 4096 12.5 / 10.9)
+int vig_linear_norm_preferred(long long rows, int N, int K) { return rows >= 16384 && vig::linear_norm_supported(rows, N, K); }
+
+int vig_linear_norm_fwd(const void* x, const void* weight, const void* residual, const float* norm_weight, void* y, void* sum,
+                        long long rows, int N, int K, float eps, void* stream) {
+  if (!x || !weight || !residual || !norm_weight || !y || !sum || rows <= 0 || N <= 0 || K <= 0) return VIG_EINVAL;
+  if (!vig::linear_norm_supported(rows, N, K)) return VIG_ENOTSUP;
+  if (!aligned16(x, weight, residual, norm_weight, y, sum)) return VIG_EINVAL;
+  return vig::launch_linear_norm(x, weight, residual, norm_weight, y, sum, rows, N, K, eps, (hipStream_t)stream);
+}
+
 int vig_conv3x3s2_fwd(const void* x, const void* weight, void* y, int B, int H, int W, int Cin, int Cout, void* stream) {
   if (!x || !weight || !y || B <= 0 || H <= 0 || W <= 0 || Cin <= 0 || Cout <= 0) return VIG_EINVAL;
   if (!aligned16(x, weight, y)) return VIG_EINVAL;

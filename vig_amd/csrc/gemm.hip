@@ -274,6 +274,139 @@ __global__ __launch_bounds__(256, (64 * (MI + NI) * 64 * BUFS <= 80 * 1024 ? 2 :
   }
 }
 
+// ---------------------------------------------------------------------------
+// A layer of 192 columns followed by the residual add and the RMS norm behind it (a block's down projection and the next
+// block's first norm): y = norm(sum), sum = residual + x . W^T, the product and the sum rounded to bf16 as the separate kernels
+// store them.  A workgroup of eight waves makes 128 whole rows, 32 x 96 a wave, operands through three LDS stages of 64
+// contraction elements (whole 128-byte lines); the finished rows lie in LDS, and a wave adds the residual (fetched before the
+// barrier) and normalises sixteen of them with whole-row loads and stores.  So the product is not written and read again: 32768
+// rows, K 512, 17 us where the library's product and the norm took 27 (100352 rows 55 / 70).  Bound by the LDS reads, four a k-step
+// for three matrix instructions.  (384 columns, K 1024: 63 to 67 us against 72 at 50176 rows, nothing gained in a model.)
+// ---------------------------------------------------------------------------
+struct NormArgs {
+  const uint16_t *x, *w, *residual;
+  const float* norm;
+  uint16_t *y, *sum;
+  int M, K;
+  float eps;
+};
+
+constexpr int kNormStageK = 64;  // 128-byte row pieces
+
+constexpr int kNormCols = 192, kNormRows = 128, kNormBufs = 3, kNormStage = (kNormRows + kNormCols) * 128;
+
+__global__ __launch_bounds__(512, 2) void gemm_norm_kernel(NormArgs a) {
+  constexpr int N = kNormCols, TM = kNormRows, BUFS = kNormBufs, kStage = kNormStage;
+  constexpr int kX = TM / 64, kW = N / 64, kLoads = kX + kW, kPitch = 2 * N + 16;
+  static_assert(TM * kPitch <= BUFS * kStage, "the rows fit");
+  extern __shared__ __align__(16) char smem[];
+  const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int m0 = blockIdx.x * TM, nstage = a.K / kNormStageK;
+  const uint32_t lds0 = lds_offset(smem);
+  // a load covers eight rows; unit u of row w lies at place u ^ (w / 2 mod 8)
+  const int lrow = lane >> 3, place = lane & 7;
+  const uint16_t *xp[kX], *wp[kW];
+#pragma unroll
+  for (int i = 0; i < kX; ++i) {
+    const int row = 8 * (wave * kX + i) + lrow;
+    xp[i] = a.x + (size_t)min(m0 + row, a.M - 1) * a.K + 8 * (place ^ ((row >> 1) & 7));
+  }
+#pragma unroll
+  for (int i = 0; i < kW; ++i) {
+    const int row = 8 * (wave * kW + i) + lrow;
+    wp[i] = a.w + (size_t)((row & ~31) + channel_of_row(row & 31)) * a.K + 8 * (place ^ ((row >> 1) & 7));
+  }
+  const auto fetch = [&](int s) {
+    const uint32_t buf = lds0 + (s % BUFS) * kStage;
+#pragma unroll
+    for (int i = 0; i < kX; ++i) load_to_lds16(xp[i] + s * kNormStageK, buf + (wave * kX + i) * 1024);
+#pragma unroll
+    for (int i = 0; i < kW; ++i) load_to_lds16(wp[i] + s * kNormStageK, buf + TM * 128 + (wave * kW + i) * 1024);
+  };
+  const int wm = (wave & 3) * 32, wn = (wave >> 2) * 96;
+  f32x16_t acc[3];
+#pragma unroll
+  for (int j = 0; j < 3; ++j) acc[j] = f32x16_t{0.f};
+#pragma unroll
+  for (int s = 0; s < BUFS - 1; ++s)
+    if (s < nstage) fetch(s);
+  for (int s = 0; s < nstage; ++s) {
+    const int ahead = min(nstage - 1 - s, BUFS - 2);
+    if (ahead >= 2) wait_vmem<2 * kLoads>();
+    else if (ahead == 1) wait_vmem<kLoads>();
+    else wait_vmem<0>();
+    lds_barrier();
+    if (s + BUFS - 1 < nstage) fetch(s + BUFS - 1);
+    const char* buf = smem + (s % BUFS) * kStage;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const char* at = buf + r * 128 + 16 * ((2 * k + h) ^ ((r >> 1) & 7));
+      const bf16x8_t xf = *reinterpret_cast<const bf16x8_t*>(at + wm * 128);
+      bf16x8_t wf[3];
+#pragma unroll
+      for (int j = 0; j < 3; ++j) wf[j] = *reinterpret_cast<const bf16x8_t*>(at + (TM + wn + 32 * j) * 128);
+#pragma unroll
+      for (int j = 0; j < 3; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[j], xf, acc[j], 0, 0, 0);
+    }
+  }
+  const int oct = lane & 31, first = 16 * wave + h;  // half a wave takes a row
+  const bool has = oct < N / 8;
+  float weight[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) weight[j] = a.norm[8 * (has ? oct : 0) + j];
+  u32x4_t res[8];
+#pragma unroll
+  for (int t = 0; t < 8; ++t)
+    res[t] = *reinterpret_cast<const u32x4_t*>(a.residual + (size_t)min(m0 + first + 2 * t, a.M - 1) * N + 8 * (has ? oct : 0));
+  lds_barrier();  // every wave is past the stages: their place becomes the rows'
+#pragma unroll
+  for (int j = 0; j < 3; ++j)
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      u32x4_t o;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = pack_bf16x2(acc[j][8 * p + 2 * e], acc[j][8 * p + 2 * e + 1]);
+      *reinterpret_cast<u32x4_t*>(smem + (wm + r) * kPitch + 2 * (wn + 32 * j + 16 * h) + 16 * p) = o;
+    }
+  lds_barrier();
+#pragma unroll
+  for (int t = 0; t < 8; ++t) {
+    const int row = first + 2 * t;
+    const u32x4_t v = *reinterpret_cast<const u32x4_t*>(smem + row * kPitch + 16 * (has ? oct : 0));
+    float sum[8], ss = 0.f;
+    u32x4_t o;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      o[j] = pack_bf16x2(bf16lo_to_f32(v[j]) + bf16lo_to_f32(res[t][j]), bf16hi_to_f32(v[j]) + bf16hi_to_f32(res[t][j]));
+      sum[2 * j] = bf16lo_to_f32(o[j]), sum[2 * j + 1] = bf16hi_to_f32(o[j]);
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) ss = __builtin_fmaf(sum[j], sum[j], ss);
+    if (!has) ss = 0.f;
+#pragma unroll
+    for (int off = 16; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
+    const float rstd = 1.0f / sqrtf(ss / (float)N + a.eps);
+    if (has && m0 + row < a.M) {
+      const size_t at = (size_t)(m0 + row) * N + 8 * oct;
+      *reinterpret_cast<u32x4_t*>(a.sum + at) = o;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) o[j] = pack_bf16x2(sum[2 * j] * rstd * weight[2 * j], sum[2 * j + 1] * rstd * weight[2 * j + 1]);
+      *reinterpret_cast<u32x4_t*>(a.y + at) = o;
+    }
+  }
+}
+
+int launch_norm(const NormArgs& a, hipStream_t stream) {
+  constexpr int lds = kNormBufs * kNormStage;
+  static const bool attr = [] {
+    return hipFuncSetAttribute((const void*)gemm_norm_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds) == hipSuccess;
+  }();
+  if (!attr) return -5;
+  hipLaunchKernelGGL(gemm_norm_kernel, dim3((a.M + kNormRows - 1) / kNormRows), dim3(512), lds, stream, a);
+  return hipGetLastError() == hipSuccess ? 0 : -5;
+}
+
 template <int MI, int NI, int BUFS, bool TAPS>
 int launch_many(const GemmArgs& a, hipStream_t stream) {
   constexpr size_t lds = (size_t)(64 * MI + 64 * NI) * 64 * BUFS;
@@ -357,6 +490,16 @@ int launch_conv3x3s2(const void* x, const void* w, void* y, int B, int H, int W,
   if (tiles_of(a, 32, 32) <= kFewTiles) return launch_few<4, kTaps>(a, stream);
   if (tiles_of(a, 128, 192) >= 256) return launch_many<2, 3, 4, true>(a, stream);
   return launch_many<1, 1, 4, true>(a, stream);
+}
+
+bool linear_norm_supported(long long M, int N, int K) {
+  return N == kNormCols && M > 0 && M <= 0x7fffffffLL - 256 && K > 0 && K % kNormStageK == 0;
+}
+int launch_linear_norm(const void* x, const void* w, const void* residual, const float* norm, void* y, void* sum, long long M, int N,
+                       int K, float eps, hipStream_t stream) {
+  if (!linear_norm_supported(M, N, K)) return -95;
+  return launch_norm({(const uint16_t*)x, (const uint16_t*)w, (const uint16_t*)residual, norm, (uint16_t*)y, (uint16_t*)sum, (int)M, K, eps},
+                     stream);
 }
 
 }  // namespace vig

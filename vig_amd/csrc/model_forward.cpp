@@ -180,10 +180,14 @@ Tensor run(const Plan& p, const Tensor& images) {
            "vig_layernorm_fwd");
 
   int64_t residual = -1;
-  for (const auto& b : p.blocks) {
+  bool normed = false;  // the block before left its sum and this block's norm of it
+  for (size_t i = 0; i < p.blocks.size(); ++i) {
+    const Block& b = p.blocks[i];
     const int64_t n0 = (int64_t)b.H * (2 * b.Dk + b.Dv), n1c = n0 + (int64_t)b.H * b.Dv, ld = b.w_in.size(0);
     int64_t hidden = branch0;
-    if (residual < 0) {
+    if (normed) {
+      hidden = residual;
+    } else if (residual < 0) {
       k.norm(branch0, -1, b.norm1, b.eps1, false, y, -1, T);
     } else {  // the explicit add of the reference stores a rounded sum and attn_norm normalises that (vig.py:598,606)
       hidden = residual == res0 ? res1 : res0;
@@ -230,7 +234,17 @@ Tensor run(const Plan& p, const Tensor& images) {
       k.linear(y, b.w_gate, Tensor(), wide, T);
       check_rc(vig_swiglu_fwd(k.at(wide), k.at(mid), T, (int)width, VIG_BF16, k.stream), "vig_swiglu_fwd");
     }
-    k.linear(mid, b.w_down, Tensor(), branch0, T);
+    normed = i + 1 < p.blocks.size() && vig_linear_norm_preferred(T, (int)C, (int)width);
+    if (normed) {
+      const Block& after = p.blocks[i + 1];
+      const int64_t sum = residual == res0 ? res1 : res0;
+      check_rc(vig_linear_norm_fwd(k.at(mid), b.w_down.data_ptr(), k.at(residual), f32(after.norm1), k.at(y), k.at(sum), T, (int)C, (int)width,
+                                   (float)after.eps1, k.stream),
+               "vig_linear_norm_fwd");
+      residual = sum;
+    } else {
+      k.linear(mid, b.w_down, Tensor(), branch0, T);
+    }
   }
   check_rc(vig_rmsnorm_pool_fwd(k.at(branch0), k.at(residual), f32(p.norm), k.at(pooled), k.at(part), pool_ws, (int)B, (int)L, (int)C,
                                 (float)p.norm_eps, k.stream),
