@@ -546,6 +546,10 @@ int vig_locality_blend_linear_fwd(const void* o, const void* local, const void* 
                                   const float* w_g, const float* w_l, const void* weight, void* out,
                                   int B, int H, int L, int Dv, int C, long long g_row_stride, float eps, int silu_out,
                                   int io_dtype, void* stream);
+/* The same, leaving the blended rows as well: blended [B*L, H*Dv], what a backward reads. */
+int vig_locality_blend_linear_kept_fwd(const void* o, const void* local, const void* g_lin, const float* w_g,
+                                       const float* w_l, const void* weight, void* blended, void* out, int B, int H, int L, int Dv,
+                                       int C, long long g_row_stride, float eps, int silu_out, int io_dtype, void* stream);
 
 /*
  * First convolution of the v2 patch embedding, without its bias (vig_layernorm_fwd's pre_bias takes that):

@@ -99,3 +99,24 @@ def test_linear_norm(rows, N, K):
     s = total.double().cpu()
     _check(y, s / torch.sqrt((s * s).mean(1, keepdim=True) + 1e-5) * nw.double())  # of the sum that was stored
     assert bool(lib.vig_linear_norm_preferred(rows, N, K)) == (rows >= 16384)
+
+
+# the mixer's epilogue with the output projection, blended rows kept: one token, ragged tiles, more tiles than workgroups
+@pytest.mark.parametrize("B,L,H", [(1, 1, 3), (3, 37, 6), (1, 65, 3), (90, 197, 6)])
+def test_blend_linear_kept(B, L, H):
+    announce(f"blend_linear with the blended rows kept B{B} L{L} H{H}")
+    C, ld = 64 * H, 64 * H + 64
+    o, loc, w = _randn((B, H, L, 64), 20).cuda(), _randn((B, L, C), 21).cuda(), _randn((C, C), 22, C ** -0.5).cuda()
+    z = _randn((B, L, ld), 23).cuda()
+    g = z[..., :C]
+    wg, wl = (torch.rand(64, generator=torch.Generator().manual_seed(s)).cuda() + 0.5 for s in (24, 25))
+    y, out = (torch.full((B, L, C), float("nan"), dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    rc = _lib.load().vig_locality_blend_linear_kept_fwd(o.data_ptr(), loc.data_ptr(), g.data_ptr(), wg.data_ptr(), wl.data_ptr(), w.data_ptr(),
+                                                        y.data_ptr(), out.data_ptr(), B, H, L, 64, C, ld, 1e-5, 0, _lib.VIG_BF16,
+                                                        torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    assert torch.equal(out, ops.locality_blend_linear(o, loc, g, wg, wl, w, eps=1e-5))
+    od, ld_, gd = o.double().cpu().permute(0, 2, 1, 3), loc.double().cpu().view(B, L, H, 64), torch.sigmoid(g.double().cpu()).view(B, L, H, 64)
+    rms = lambda t, n: t / torch.sqrt((t * t).mean(-1, keepdim=True) + 1e-5) * n.double().cpu()  # noqa: E731
+    want = (rms(od, wg) * gd + rms(ld_, wl) * (1 - gd)).reshape(B, L, C)
+    _check(y, want)

@@ -57,7 +57,7 @@ int launch_rmsnorm_bwd(const void* s, const float* weight, const void* dy, const
                        void* workspace, long long rows, int C, float eps, int sum_dtype, int y_dtype, hipStream_t stream);
 bool blend_linear_supported(int H, int Dv, int C);
 int launch_blend_linear(const void* o, const void* loc, const void* glin, const float* w_g, const float* w_l,
-                        const void* W, void* out, int B, int H, int L, int Dv, int C, long long ldg, float eps,
+                        const void* W, void* out, void* kept, int B, int H, int L, int Dv, int C, long long ldg, float eps,
                         int silu_out, hipStream_t stream);
 bool linear_swiglu_supported(int K, int I);
 int launch_linear_swiglu(const void* A, const void* W, void* out, void* kept, long long T, int K, int I, hipStream_t stream);
@@ -640,7 +640,19 @@ int vig_locality_blend_linear_fwd(const void* o, const void* local, const void* 
   if (io_dtype != VIG_BF16 || !vig::blend_linear_supported(H, Dv, C)) return VIG_ENOTSUP;
   const long long ldg = g_row_stride > 0 ? g_row_stride : (long long)H * Dv;
   if (ldg < (long long)H * Dv || !strided_rows_ok(g_lin, ldg, io_dtype)) return VIG_EINVAL;
-  return vig::launch_blend_linear(o, local, g_lin, w_g, w_l, weight, out, B, H, L, Dv, C, ldg, eps, silu_out,
+  return vig::launch_blend_linear(o, local, g_lin, w_g, w_l, weight, out, nullptr, B, H, L, Dv, C, ldg, eps, silu_out,
+                                  (hipStream_t)stream);
+}
+
+int vig_locality_blend_linear_kept_fwd(const void* o, const void* local, const void* g_lin, const float* w_g,
+                                  const float* w_l, const void* weight, void* blended, void* out, int B, int H, int L, int Dv, int C,
+                                  long long g_row_stride, float eps, int silu_out, int io_dtype, void* stream) {
+  if (!o || !local || !g_lin || !w_g || !w_l || !weight || !blended || !out || B <= 0 || H <= 0 || L <= 0) return VIG_EINVAL;
+  if (!aligned16(o, local, w_g, w_l, weight, blended, out)) return VIG_EINVAL;
+  if (io_dtype != VIG_BF16 || !vig::blend_linear_supported(H, Dv, C)) return VIG_ENOTSUP;
+  const long long ldg = g_row_stride > 0 ? g_row_stride : (long long)H * Dv;
+  if (ldg < (long long)H * Dv || !strided_rows_ok(g_lin, ldg, io_dtype)) return VIG_EINVAL;
+  return vig::launch_blend_linear(o, local, g_lin, w_g, w_l, weight, out, blended, B, H, L, Dv, C, ldg, eps, silu_out,
                                   (hipStream_t)stream);
 }
 

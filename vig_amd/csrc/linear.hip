@@ -408,15 +408,16 @@ __device__ __forceinline__ float lane_permuted(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
 }
 
-template <int KS, int NW, int TPW>
+// kept (KEPT): y as well, which a backward reads.
+template <int KS, int NW, int TPW, bool KEPT>
 __global__ __launch_bounds__(64 * NW) void blend_linear_kernel(const uint16_t* __restrict__ o,
                                                               const uint16_t* __restrict__ loc,
                                                               const uint16_t* __restrict__ glin,
                                                               const float* __restrict__ w_g,
                                                               const float* __restrict__ w_l,
                                                               const uint16_t* __restrict__ W,
-                                                              uint16_t* __restrict__ out, int T, int L, int H,
-                                                              long long ldg, float eps, int silu_out) {
+                                                              uint16_t* __restrict__ out, uint16_t* __restrict__ kept,
+                                                              int T, int L, int H, long long ldg, float eps, int silu_out) {
   constexpr int K = 16 * KS;
   constexpr int C = 32 * TPW * NW;             // TPW 32-channel tiles of W per wave
   constexpr int kThreads = 64 * NW;
@@ -470,7 +471,7 @@ __global__ __launch_bounds__(64 * NW) void blend_linear_kernel(const uint16_t* _
   // the blend of this thread's octets of a tile (they wait in its slots), straight into the tile's operand buffer
   // (stored: the stores of a tile's result were issued behind the octets' loads and may still be on their way; waited for,
   // their latency was part of every tile)
-  auto blend = [&](uint16_t* mine, bool stored) {
+  auto blend = [&](uint16_t* mine, bool stored, int tile) {
     if (stored) wait_vmem<2 * TPW>();
     else wait_vmem<0>();
 #pragma unroll 1
@@ -508,6 +509,10 @@ __global__ __launch_bounds__(64 * NW) void blend_linear_kernel(const uint16_t* _
 #pragma unroll
       for (int j = 0; j < 4; ++j) y[j] = pack_bf16x2(e[2 * j], e[2 * j + 1]);
       *reinterpret_cast<u32x4_t*>(mine + (row0 + kRowStep * i) * kRow + col * 8) = y;
+      if constexpr (KEPT) {  // (older than the loads of the tile after the next: the waits do not count these)
+        const int t = tile * 32 + row0 + kRowStep * i;
+        if (t < T) *reinterpret_cast<u32x4_t*>(kept + (size_t)t * K + col * 8) = y;
+      }
     }
   };
   // this wave's products of a staged tile, and its rows of the result
@@ -556,7 +561,7 @@ __global__ __launch_bounds__(64 * NW) void blend_linear_kernel(const uint16_t* _
   // (being refilled now) and tile i's is complete.
   __syncthreads();  // the norm weights are in place
   fetch(blockIdx.x);
-  blend(buf, false);
+  blend(buf, false, blockIdx.x);
   fetch(blockIdx.x + nworkers);
   tile_barrier();
   int cur = 0;
@@ -567,12 +572,12 @@ __global__ __launch_bounds__(64 * NW) void blend_linear_kernel(const uint16_t* _
     if ((wave >> 2) != 1) {
       products(mine, tile);
       if (more) {
-        blend(next, true);
+        blend(next, true, tile + nworkers);
         fetch(tile + 2 * nworkers);
       }
     } else {
       if (more) {
-        blend(next, tile != (int)blockIdx.x);
+        blend(next, tile != (int)blockIdx.x, tile + nworkers);
         fetch(tile + 2 * nworkers);
       }
       products(mine, tile);
@@ -581,9 +586,9 @@ __global__ __launch_bounds__(64 * NW) void blend_linear_kernel(const uint16_t* _
   }
 }
 
-template <int KS, int NW, int TPW>
+template <int KS, int NW, int TPW, bool KEPT>
 int launch_blend_linear_t(const void* o, const void* loc, const void* glin, const float* w_g, const float* w_l,
-                          const void* W, void* out, long long T, int L, int H, long long ldg, float eps, int silu_out,
+                          const void* W, void* out, void* kept, long long T, int L, int H, long long ldg, float eps, int silu_out,
                           int num_cu, hipStream_t stream) {
   constexpr int K = 16 * KS;
   constexpr size_t lds = (size_t)2 * 32 * (K + 8) * sizeof(uint16_t) + 128 * sizeof(float) + (size_t)(32 * K / 8) * 3 * sizeof(u32x4_t);
@@ -591,9 +596,9 @@ int launch_blend_linear_t(const void* o, const void* loc, const void* glin, cons
   const long long ntiles_t = (T + 31) / 32;
   const int grid = ntiles_t < num_cu ? (int)ntiles_t : num_cu;
   static bool done[64] = {};
-  if (!allow_lds((const void*)blend_linear_kernel<KS, NW, TPW>, lds, done)) return -5;
-  hipLaunchKernelGGL((blend_linear_kernel<KS, NW, TPW>), dim3(grid), dim3(64 * NW), lds, stream, (const uint16_t*)o,
-                     (const uint16_t*)loc, (const uint16_t*)glin, w_g, w_l, (const uint16_t*)W, (uint16_t*)out, (int)T, L,
+  if (!allow_lds((const void*)blend_linear_kernel<KS, NW, TPW, KEPT>, lds, done)) return -5;
+  hipLaunchKernelGGL((blend_linear_kernel<KS, NW, TPW, KEPT>), dim3(grid), dim3(64 * NW), lds, stream, (const uint16_t*)o,
+                     (const uint16_t*)loc, (const uint16_t*)glin, w_g, w_l, (const uint16_t*)W, (uint16_t*)out, (uint16_t*)kept, (int)T, L,
                      H, ldg, eps, silu_out);
   return hipGetLastError() == hipSuccess ? 0 : -5;
 }
@@ -604,7 +609,7 @@ int launch_blend_linear_t(const void* o, const void* loc, const void* glin, cons
 bool blend_linear_supported(int H, int Dv, int C) { return Dv == 64 && C == H * Dv && (C == 384 || C == 192); }
 
 int launch_blend_linear(const void* o, const void* loc, const void* glin, const float* w_g, const float* w_l,
-                        const void* W, void* out, int B, int H, int L, int Dv, int C, long long ldg, float eps,
+                        const void* W, void* out, void* kept, int B, int H, int L, int Dv, int C, long long ldg, float eps,
                         int silu_out, hipStream_t stream) {
   if (!blend_linear_supported(H, Dv, C) || B <= 0 || L <= 0 || (long long)B * L > 0x7fffffffLL - 64 || ldg % 8 != 0 ||
       ldg < C)
@@ -613,8 +618,11 @@ int launch_blend_linear(const void* o, const void* loc, const void* glin, const 
   if (!num_cu) return -5;
   const long long T = (long long)B * L;
   // twelve waves with one weight tile each (three per SIMD at 168 registers) at the wider size, six at the narrower
-  return C == 384 ? launch_blend_linear_t<24, 12, 1>(o, loc, glin, w_g, w_l, W, out, T, L, H, ldg, eps, silu_out, num_cu, stream)
-                  : launch_blend_linear_t<12, 6, 1>(o, loc, glin, w_g, w_l, W, out, T, L, H, ldg, eps, silu_out, num_cu, stream);
+  if (kept)
+    return C == 384 ? launch_blend_linear_t<24, 12, 1, true>(o, loc, glin, w_g, w_l, W, out, kept, T, L, H, ldg, eps, silu_out, num_cu, stream)
+                    : launch_blend_linear_t<12, 6, 1, true>(o, loc, glin, w_g, w_l, W, out, kept, T, L, H, ldg, eps, silu_out, num_cu, stream);
+  return C == 384 ? launch_blend_linear_t<24, 12, 1, false>(o, loc, glin, w_g, w_l, W, out, kept, T, L, H, ldg, eps, silu_out, num_cu, stream)
+                  : launch_blend_linear_t<12, 6, 1, false>(o, loc, glin, w_g, w_l, W, out, kept, T, L, H, ldg, eps, silu_out, num_cu, stream);
 }
 
 bool linear_swiglu_supported(int K, int I) { return (K == 384 || K == 192) && I % 32 == 0 && I >= 32; }

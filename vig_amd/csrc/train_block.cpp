@@ -243,10 +243,19 @@ struct MixNode : torch::autograd::Function<MixNode> {
     Tensor o;
     check_rc(run_forward(q, k, v, gates, Tensor(), true, kDefault, c, o), "vig_gla_bidir_fwd");
     Tensor blend = at::empty_like(xs);
-    check_rc(vig_locality_blend_fwd(o.data_ptr(), xs.data_ptr(), at_elem(z, m.n0), f32(g_norm, 2), f32(l_norm, 3), blend.data_ptr(),
-                                    (int)m.B, (int)m.H, (int)m.L, (int)m.Dv, m.nz, (float)m.eps, m.out_act, m.code(), stream),
-             "vig_locality_blend_fwd");
-    const Tensor a = product(blend.view({m.rows, m.V}), w_out, Tensor()).view({m.B, m.L, m.C});
+    Tensor a;
+    if (m.bf16 && m.Dv == 64 && m.V == m.C && (m.C == 384 || m.C == 192) && aligned(w_out)) {
+      a = at::empty({m.B, m.L, m.C}, opts);
+      check_rc(vig_locality_blend_linear_kept_fwd(o.data_ptr(), xs.data_ptr(), at_elem(z, m.n0), f32(g_norm, 2), f32(l_norm, 3),
+                                                  w_out.data_ptr(), blend.data_ptr(), a.data_ptr(), (int)m.B, (int)m.H, (int)m.L, (int)m.Dv,
+                                                  (int)m.C, m.nz, (float)m.eps, m.out_act, m.code(), stream),
+               "vig_locality_blend_linear_kept_fwd");
+    } else {
+      check_rc(vig_locality_blend_fwd(o.data_ptr(), xs.data_ptr(), at_elem(z, m.n0), f32(g_norm, 2), f32(l_norm, 3), blend.data_ptr(),
+                                      (int)m.B, (int)m.H, (int)m.L, (int)m.Dv, m.nz, (float)m.eps, m.out_act, m.code(), stream),
+               "vig_locality_blend_fwd");
+      a = product(blend.view({m.rows, m.V}), w_out, Tensor()).view({m.B, m.L, m.C});
+    }
 
     ctx->set_materialize_grads(false);
     ctx->save_for_backward({sum, y, xs, pre, z, q, k, v, gates, gate_lin, o, blend, packed, small, norm_w, conv_w, g_norm, l_norm,
