@@ -280,8 +280,9 @@ __global__ __launch_bounds__(256, (64 * (MI + NI) * 64 * BUFS <= 80 * 1024 ? 2 :
 // store them.  A workgroup of eight waves makes 128 whole rows, 32 x 96 a wave, operands through three LDS stages of 64
 // contraction elements (whole 128-byte lines); the finished rows lie in LDS, and a wave adds the residual (fetched before the
 // barrier) and normalises sixteen of them with whole-row loads and stores.  So the product is not written and read again: 32768
-// rows, K 512, 17 us where the library's product and the norm took 27 (100352 rows 55 / 70).  Bound by the LDS reads, four a k-step
-// for three matrix instructions.  (384 columns, K 1024: 63 to 67 us against 72 at 50176 rows, nothing gained in a model.)
+// rows, K 512, 17 us where the library's product and the norm took 27 (100352 rows 55 / 70).  Bound by its waits: half of the
+// waves' time goes to the stages' arrival and barriers (matrix pipe and LDS 14 % busy each).  (384 columns, K 1024: 63 to 67 us
+// against 72 at 50176 rows, nothing gained in a model.)
 // ---------------------------------------------------------------------------
 struct NormArgs {
   const uint16_t *x, *w, *residual;
