@@ -400,10 +400,8 @@ __global__ __launch_bounds__(512, 2) void gemm_norm_kernel(NormArgs a) {
 
 int launch_norm(const NormArgs& a, hipStream_t stream) {
   constexpr int lds = kNormBufs * kNormStage;
-  static const bool attr = [] {
-    return hipFuncSetAttribute((const void*)gemm_norm_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds) == hipSuccess;
-  }();
-  if (!attr) return -5;
+  static bool done[64] = {};
+  if (!allow_lds((const void*)gemm_norm_kernel, lds, done)) return -5;
   hipLaunchKernelGGL(gemm_norm_kernel, dim3((a.M + kNormRows - 1) / kNormRows), dim3(512), lds, stream, a);
   return hipGetLastError() == hipSuccess ? 0 : -5;
 }
@@ -411,11 +409,8 @@ int launch_norm(const NormArgs& a, hipStream_t stream) {
 template <int MI, int NI, int BUFS, bool TAPS>
 int launch_many(const GemmArgs& a, hipStream_t stream) {
   constexpr size_t lds = (size_t)(64 * MI + 64 * NI) * 64 * BUFS;
-  static const bool attr = [] {
-    return hipFuncSetAttribute((const void*)gemm_many_kernel<MI, NI, BUFS, TAPS>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) ==
-           hipSuccess;
-  }();
-  if (!attr) return -5;
+  static bool done[64] = {};
+  if (!allow_lds((const void*)gemm_many_kernel<MI, NI, BUFS, TAPS>, lds, done)) return -5;
   const int tn = (a.N + 64 * NI - 1) / (64 * NI), tm = (a.M + 64 * MI - 1) / (64 * MI), tiles = tn * tm;
   hipLaunchKernelGGL((gemm_many_kernel<MI, NI, BUFS, TAPS>), dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(256), lds, stream, a, tn, tiles);
   return hipGetLastError() == hipSuccess ? 0 : -5;
@@ -424,10 +419,8 @@ int launch_many(const GemmArgs& a, hipStream_t stream) {
 template <int NW, FewForm FORM>
 int launch_few(const GemmArgs& a, hipStream_t stream) {
   constexpr size_t lds = (size_t)NW * kFewBufs * (FORM == kPair ? 6144 : 4096);
-  static const bool attr = [] {
-    return hipFuncSetAttribute((const void*)gemm_few_kernel<NW, FORM>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
-  }();
-  if (!attr) return -5;
+  static bool done[64] = {};
+  if (!allow_lds((const void*)gemm_few_kernel<NW, FORM>, lds, done)) return -5;
   hipLaunchKernelGGL((gemm_few_kernel<NW, FORM>), dim3((a.N + 31) / 32, (a.M + 31) / 32), dim3(64 * NW), lds, stream, a);
   return hipGetLastError() == hipSuccess ? 0 : -5;
 }

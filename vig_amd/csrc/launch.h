@@ -108,6 +108,14 @@ int launch_gla_backward_mfma(const void* q, const void* k, const void* v, const 
                              const void* d_o, void* dq, void* dk, void* dv, void* dgf, void* dgb, int* flags,
                              void* seg_workspace, int B, int H, int L, int Dk, float s, hipStream_t stream);
 
+// allows a kernel its LDS, once per device (concurrent first calls only repeat an idempotent setting)
+inline bool allow_lds(const void* kernel, size_t bytes, bool (&done)[64]) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return false;
+  if (!done[dev]) done[dev] = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) == hipSuccess;
+  return done[dev];
+}
+
 // bf16 row products (gemm.hip, linear.hip): a layer whose weights stay in registers, and SwiGLU of a layer over few rows
 bool linear_regs_supported(int K, int N);
 int launch_linear_regs(const void* x, const void* w, const void* bias, void* y, long long T, int N, int K, hipStream_t stream);

@@ -348,14 +348,6 @@ __global__ __launch_bounds__(64 * NW, 2) void linear_regs_kernel(const uint16_t*
     epilogue(worker + ((ntiles_t - 1 - worker) / nworkers) * nworkers);
 }
 
-// allows a kernel its LDS, once per device (concurrent first calls only repeat an idempotent setting)
-bool allow_lds(const void* kernel, size_t bytes, bool (&done)[64]) {
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return false;
-  if (!done[dev]) done[dev] = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) == hipSuccess;
-  return done[dev];
-}
-
 template <int KS, int NW, LinForm FORM>
 int launch_linear_regs_t(const void* A, const void* W, const void* bias, void* out, void* kept, long long T, int N, int num_cu,
                          hipStream_t stream) {
