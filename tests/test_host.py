@@ -114,3 +114,21 @@ def test_checkpoint_variants_and_cache_invalidation(tmp_path):
     assert torch.equal(norm._w32(), norm.weight.detach().float() / 2)
     layers.invalidate_caches(m)  # ... until the caller says so
     assert torch.equal(norm._w32(), norm.weight.detach().float())
+
+
+def test_weight_copies_follow_weights_that_are_computed_anew():
+    """A weight recomputed on every call (a pruned layer's) may come to lie where the one before it lay."""
+    from vig_amd import layers
+
+    n = 1 << 16
+    owner, norm, at = torch.nn.Module(), layers.RMSNorm(n), layers.GatedLinearAttention(64, 1.0, 0.5, 1)
+    del norm.weight
+    for i in range(6):
+        t = torch.full((n,), float(i), dtype=torch.bfloat16)
+        assert torch.equal(layers._f32(owner, "w", t), t.float())
+        norm.weight = torch.full((n,), float(i), dtype=torch.bfloat16)
+        assert torch.equal(norm._w32(), norm.weight.float())
+        del t, norm.weight
+        at.g_proj._parameters["weight"] = torch.full((64, 64), float(i))
+        assert (at._stacked_in()[0][at.qkv_proj.weight.shape[0]:][:64] == i).all()
+        at.g_proj._parameters["weight"] = None

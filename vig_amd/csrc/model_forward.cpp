@@ -31,7 +31,7 @@ struct Entry {
   Ref dict, key, value;  // value NULL: the key has to be absent
 };
 struct Watched {
-  Tensor t;
+  Tensor t, data;  // data: an alias, so that the storage lives and nothing else can come to lie at ptr
   void* ptr;
   uint32_t version;
   at::ScalarType type;
@@ -293,8 +293,8 @@ bool collect(Plan& p, PyObject* module, PyObject* settings, PyObject* absent, st
     p.entries.push_back({Ref(params), Ref(key), Ref(value)});
     if (value == Py_None) continue;
     const Tensor t = tensor_arg(value);
-    if (!t.defined() || t.scalar_type() != at::kBFloat16) return false;
-    p.watched.push_back({t, t.data_ptr(), (uint32_t)t._version(), t.scalar_type()});
+    if (!t.defined() || t.unsafeGetTensorImpl()->is_python_dispatch() || t.scalar_type() != at::kBFloat16) return false;
+    p.watched.push_back({t, t.detach(), t.data_ptr(), (uint32_t)t._version(), t.scalar_type()});
   }
   for (Py_ssize_t at = 0; PyDict_Next(children, &at, &key, &value);) {
     p.entries.push_back({Ref(children), Ref(key), Ref(value)});

@@ -36,22 +36,32 @@ import torch.nn.functional as F
 from . import _ext, ops
 
 
+def _stamp(*ts):
+    """What tells tensors apart from other ones and from themselves after a write, while their storages live: whoever keeps a
+    stamp keeps the tensors' storages (_hold), or another tensor could come to lie where one of them was."""
+    return tuple((t.data_ptr(), t._version, t.dtype, t.device) for t in ts)
+
+
+def _hold(*ts):
+    return tuple(t.detach() for t in ts)
+
+
 def _f32(owner: nn.Module, tag: str, t: Optional[torch.Tensor], shape=None):
     """fp32 contiguous copy of parameter `t` (the kernels take fp32 weights), kept on `owner` under `tag` and refreshed
     when the parameter is replaced, moved, cast or written in place: no conversion kernel per forward."""
     if t is None:
         return None
-    key = (t.data_ptr(), t._version, t.dtype, t.device)
+    key = _stamp(t)
     cache = owner.__dict__.setdefault("_f32_cache", {})
     hit = cache.get(tag)
     if hit is None or hit[0] != key:
         v = t.detach().float()
-        cache[tag] = hit = (key, (v.reshape(shape) if shape is not None else v).contiguous())
+        cache[tag] = hit = (key, (v.reshape(shape) if shape is not None else v).contiguous(), _hold(t))
     return hit[1]
 
 
 _PLANS = weakref.WeakKeyDictionary()  # model -> plan of its native evaluation forward (ViG._planned)
-_CACHE_ATTRS = ("_f32_cache", "_w32_key", "_w32_cache", "_w1_packed")
+_CACHE_ATTRS = ("_f32_cache", "_w32_key", "_w32_cache", "_w32_from", "_w1_packed")
 
 
 def invalidate_caches(model: nn.Module) -> None:
@@ -114,10 +124,10 @@ class RMSNorm(_CacheMixin, nn.Module):
     def _w32(self):
         """fp32 copy of the weight, refreshed when the parameter changes (the kernels take fp32 weights)."""
         w = self.weight
-        key = (w.data_ptr(), w._version, w.dtype, w.device)
+        key = _stamp(w)
         if getattr(self, "_w32_key", None) != key:
             self._w32_cache = w.detach().float().contiguous()
-            self._w32_key = key
+            self._w32_key, self._w32_from = key, _hold(w)
         return self._w32_cache
 
     def forward(self, x, residual=None, prenorm: bool = False, round_sum: bool = False):
@@ -183,7 +193,7 @@ class GatedLinearAttention(_CacheMixin, nn.Module):
         self.g_norm = RMSNorm(self.head_v_dim, eps=layernorm_eps)
         self.l_norm = RMSNorm(self.head_v_dim, eps=layernorm_eps)
         self.g_proj = nn.Linear(d_model, self.value_dim, bias=True)
-        self._in_cat = None  # (key, weight, bias) of the concatenated input projection, built on first use
+        self._in_cat = None  # (key, weight, bias, sources) of the concatenated input projection, built on first use
         self.reset_parameters()
 
     def reset_parameters(self):
@@ -210,7 +220,7 @@ class GatedLinearAttention(_CacheMixin, nn.Module):
     def _stacked_in(self):
         """(weight, bias) of the stacked input projection: rows qkv | g | low-rank gate, zero-padded to a multiple of 128."""
         srcs = (self.qkv_proj.weight, self.g_proj.weight, self.g_proj.bias, self.gk_proj[0].weight)
-        key = tuple((t.data_ptr(), t._version, t.dtype, t.device) for t in srcs)
+        key = _stamp(*srcs)
         if self._in_cat is None or self._in_cat[0] != key:
             wq, wg, bg, wr = (t.detach() for t in srcs)
             n = wq.shape[0] + wg.shape[0] + wr.shape[0]
@@ -218,7 +228,7 @@ class GatedLinearAttention(_CacheMixin, nn.Module):
             b = wq.new_zeros(w.shape[0])
             w[:n] = torch.cat((wq, wg, wr), 0)
             b[wq.shape[0]:wq.shape[0] + wg.shape[0]] = bg
-            self._in_cat = (key, w, b)
+            self._in_cat = (key, w, b, _hold(*srcs))
         return self._in_cat[1], self._in_cat[2]
 
     def _mix(self, x, hw, out_scale):
@@ -579,10 +589,10 @@ class V2PatchEmbed(_CacheMixin, nn.Module):
     def _packed_w1(self):
         """The first convolution's weight in the kernel's packed form, rebuilt when the parameter changes."""
         w = self.proj[0].weight
-        key = (w.data_ptr(), w._version, w.dtype, w.device)
+        key = _stamp(w)
         hit = self.__dict__.get("_w1_packed")
         if hit is None or hit[0] != key:
-            self.__dict__["_w1_packed"] = hit = (key, ops.pack_patch_conv_weight(w))
+            self.__dict__["_w1_packed"] = hit = (key, ops.pack_patch_conv_weight(w), _hold(w))
         return hit[1]
 
     @staticmethod
