@@ -61,6 +61,75 @@ def test_rmsnorm_pool(B, L, C):
     _close(got, want)
 
 
+def _modules(monkeypatch, m, x):
+    """The same forward through the modules, without a plan."""
+    with monkeypatch.context() as mp:
+        mp.setattr(layers.ViG, "_planned", lambda self, x: None)
+        with torch.no_grad():
+            return m(x)
+
+
+def _tiny(width=192, side=64, **kw):
+    torch.manual_seed(2)
+    kw = dict(img_size=side, depth=2, num_heads=width // 64, embed_dim=width, num_classes=16, drop_path_rate=0.0) | kw
+    return layers.ViG(**kw).cuda().bfloat16().eval(), torch.randn(2, 3, side, side, device="cuda").bfloat16()
+
+
+class _Wrapped(torch.Tensor):
+    """A tensor subclass without data of its own, as quantised weights are."""
+
+    @staticmethod
+    def __new__(cls, t):
+        return torch.Tensor._make_wrapper_subclass(cls, t.shape, dtype=t.dtype, device=t.device)
+
+    def __init__(self, t):
+        self.inner = t
+
+    __torch_function__ = torch._C._disabled_torch_function_impl
+
+    @classmethod
+    def __torch_dispatch__(cls, func, types, args=(), kwargs=None):
+        return func(*torch.utils._pytree.tree_map(lambda a: a.inner if isinstance(a, cls) else a, args), **(kwargs or {}))
+
+
+def test_layers_of_another_shape_or_device(monkeypatch):
+    """Weights the kernels would read or write past their ends, or on the host, never reach them: the calls raise what the
+    modules raise, and widths that differ from block to block have buffers of their own."""
+    announce("layers of another shape or device")
+    x = _randn((196, 192), 1).cuda()
+    w, b = _randn((64, 192), 2), _randn((64,), 3)
+    for bad in ((w, None), (w.cuda(), b), (w.cuda(), b.cuda()[:40])):
+        with pytest.raises(RuntimeError):
+            ops.linear(x, *bad)
+    assert torch.equal(ops.linear(x, w.cuda(), b.cuda()[:1]), torch.nn.functional.linear(x, w.cuda(), b.cuda()[:1]))  # broadcast
+    with pytest.raises(RuntimeError):
+        ops.conv3x3s2(_randn((1, 32, 8, 8), 4).cuda().contiguous(memory_format=torch.channels_last), _randn((8, 32, 3, 3), 5))
+    want = torch.nn.functional.linear(x, w.cuda())
+    assert torch.equal(ops.linear(x, _Wrapped(w.cuda())), want)
+    rows, weight = _randn((1, 4, 64), 6).cuda(), torch.ones(64, device="cuda")
+    for args in ((rows, rows[:, :2], weight), (rows, rows, weight[:32]), (rows, rows, weight.bfloat16())):
+        with pytest.raises(ValueError):
+            ops.rmsnorm_pool(*args, 1e-6)
+    for name, layer in (("down_proj", torch.nn.Linear(512, 200, bias=False)), ("gate_proj", torch.nn.Linear(192, 512, bias=False))):
+        m, x = _tiny()
+        setattr(m.blocks[0].mlp, name, layer.cuda().bfloat16())
+        with pytest.raises(RuntimeError):
+            m(x)
+        assert m not in layers._PLANS
+    m, x = _tiny()
+    m.head.cpu()
+    with pytest.raises(RuntimeError):
+        m(x)
+    m, x = _tiny()
+    want, plain = _modules(monkeypatch, m, x), m.blocks[0].mlp.down_proj.weight
+    m.blocks[0].mlp.down_proj._parameters["weight"] = _Wrapped(plain.detach())  # (the operator's products see it too)
+    err = (m(x).float() - want.float()).norm() / want.float().norm()
+    assert err <= 2.0 ** -8 and m not in layers._PLANS, err
+    m, x = _tiny()
+    m.blocks[1].mlp = layers.GLAMLP(192, intermediate_size=72).cuda().bfloat16()
+    assert torch.equal(m(x), _modules(monkeypatch, m, x)) and m in layers._PLANS
+
+
 @pytest.mark.parametrize("kw,side,B", [(dict(embed_dim=192, num_heads=3, use_out_act=True, use_act_in_conv=True), 224, 1),
                                        (dict(embed_dim=384, num_heads=6), 160, 3),
                                        (dict(embed_dim=128, num_heads=2, use_bias_in_dwconv=True, num_classes=10), 288, 2)])
@@ -70,14 +139,8 @@ def test_native_forward(kw, side, B, monkeypatch):
     model = layers.ViG(img_size=side, depth=2, drop_path_rate=0.0, **kw).cuda().bfloat16().eval()
     x = torch.randn(B, 3, side, side, device="cuda").bfloat16()
 
-    def modules(m, x):
-        with monkeypatch.context() as mp:
-            mp.setattr(layers.ViG, "_planned", lambda self, x: None)
-            with torch.no_grad():
-                return m(x)
-
     def same(m, x):
-        got, want = m(x), modules(m, x)
+        got, want = m(x), _modules(monkeypatch, m, x)
         assert torch.equal(got, want), (got.float() - want.float()).abs().max().item()
         return got
 

@@ -29,8 +29,9 @@ inline int dtype_code(const Tensor& t) {
   const auto s = t.scalar_type();
   return s == at::kBFloat16 ? VIG_BF16 : (s == at::kFloat ? VIG_F32 : -1);
 }
+// (a tensor subclass that dispatches to Python has no data of its own)
 inline bool plain(const Tensor& t, const c10::Device& dev) {
-  return t.defined() && t.layout() == at::kStrided && t.device() == dev && t.is_contiguous() &&
+  return t.defined() && !t.unsafeGetTensorImpl()->is_python_dispatch() && t.layout() == at::kStrided && t.device() == dev && t.is_contiguous() &&
          reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
 }
 

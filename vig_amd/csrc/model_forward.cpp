@@ -137,7 +137,11 @@ Tensor run(const Plan& p, const Tensor& images) {
   const int64_t L = (int64_t)st.gh * st.gw, T = B * L, n1 = B * oh1 * ow1;
   const int64_t classes = p.head_w.size(0);
   int64_t nz = 0, I = 0, K2 = 0;
-  for (const auto& b : p.blocks) nz = std::max(nz, b.w_in.size(0)), I = std::max(I, b.w_down.size(1)), K2 = std::max<int64_t>(K2, 2 * b.H * b.Dk);
+  bool swiglu_kernel = C == 384 || C == 192;  // in every block
+  for (const auto& b : p.blocks) {
+    nz = std::max(nz, b.w_in.size(0)), I = std::max(I, b.w_down.size(1)), K2 = std::max<int64_t>(K2, 2 * b.H * b.Dk);
+    swiglu_kernel = swiglu_kernel && b.w_down.size(1) % 32 == 0;
+  }
   const bool whole = L <= 256;  // q, k, v are read in place from the projection's rows
   size_t gla_ws = 0;
   if (!whole)
@@ -154,7 +158,6 @@ Tensor run(const Plan& p, const Tensor& images) {
   if (!whole) q = k.take(T * K2 / 2), kk = k.take(T * K2 / 2), v = k.take(T * C), ws = k.take((int64_t)(gla_ws + 1) / 2);
   int64_t most = k.used;
   k.used = region;
-  const bool swiglu_kernel = (C == 384 || C == 192) && I % 32 == 0;
   const int64_t mid = k.take(T * I), wide = swiglu_kernel ? 0 : k.take(T * 2 * I);
   most = std::max(most, k.used);
   k.used = region;
@@ -227,7 +230,7 @@ Tensor run(const Plan& p, const Tensor& images) {
     k.norm(branch1, hidden, b.norm2, b.eps2, false, y, next, T);
     residual = next;
     const int64_t width = b.w_down.size(1);
-    if (swiglu_kernel && width % 32 == 0) {
+    if (swiglu_kernel) {
       check_rc(vig_linear_swiglu_fwd(k.at(y), b.w_gate.data_ptr(), k.at(mid), T, (int)C, (int)width, VIG_BF16, k.stream),
                "vig_linear_swiglu_fwd");
     } else {
@@ -353,6 +356,21 @@ PyObject* make_plan(PyObject*, PyObject* const* a, Py_ssize_t n) {
   for (const auto& b : p->blocks) {
     for (const Tensor* x : {&b.w_in, &b.b_in, &b.w_up, &b.b_up, &b.w_o, &b.w_gate, &b.w_down}) ok = ok && usable(*x, dev, at::kBFloat16);
     for (const Tensor* x : {&b.norm1, &b.conv_w, &b.conv_b, &b.gn, &b.ln, &b.norm2}) ok = ok && usable(*x, dev, at::kFloat);
+  }
+  // shapes: the walk lays its buffers out by the stem's width and each block's heads, and the kernels take sizes on trust
+  const auto is = [](const Tensor& t, std::initializer_list<int64_t> shape) { return t.defined() && t.sizes() == at::IntArrayRef(shape); };
+  const auto has = [](const Tensor& t, int64_t n) { return t.defined() && t.numel() == n; };
+  const auto fits = [&](const Tensor& t, int64_t n) { return !t.defined() || t.numel() == n; };
+  const int64_t half = st.w1.size(0), C = st.w2.defined() ? st.w2.size(0) : 0;
+  ok = ok && is(st.w2, {C, 3, 3, half}) && fits(st.b1, half) && has(st.ln1w, half) && has(st.ln1b, half) && fits(st.b2, C) &&
+       has(st.ln2w, C) && has(st.ln2b, C) && is(st.pos, {1, (int64_t)st.gh * st.gw, C}) && has(p->norm, C) && p->head_w.defined() &&
+       p->head_w.dim() == 2 && is(p->head_w, {p->head_w.size(0), C}) && fits(p->head_b, p->head_w.size(0));
+  for (const auto& b : p->blocks) {
+    const int64_t K = (int64_t)b.H * b.Dk, V = (int64_t)b.H * b.Dv, n = 2 * K + 2 * V + 16, nz = (n + 127) / 128 * 128;
+    const int64_t I = b.w_down.defined() && b.w_down.dim() == 2 ? b.w_down.size(1) : 0;
+    ok = ok && V == C && I > 0 && I % 8 == 0 && has(b.norm1, C) && has(b.conv_w, C * 9) && fits(b.conv_b, C) && is(b.w_in, {nz, C}) &&
+         has(b.b_in, nz) && is(b.w_up, {2 * K, 16}) && has(b.b_up, 2 * K) && has(b.gn, b.Dv) && has(b.ln, b.Dv) && is(b.w_o, {C, V}) &&
+         has(b.norm2, C) && is(b.w_gate, {2 * I, C}) && is(b.w_down, {C, I});
   }
   if (!ok) Py_RETURN_NONE;
   return PyCapsule_New(p.release(), kPlanName, [](PyObject* cap) { free_plan(cap); });

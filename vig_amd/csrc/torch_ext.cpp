@@ -71,10 +71,13 @@ float resolve_scale(double scale, int64_t Dk) { return scale < 0 ? 1.0f / std::s
 
 // x . w^T (+ b): the library's own kernels where they are the better choice for the size, torch's product otherwise
 Tensor product(const Tensor& x, const Tensor& w, const optional<Tensor>& b = c10::nullopt) {
-  const auto dense = [](const Tensor& t) { return t.is_contiguous() && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; };
+  const auto dense = [](const Tensor& t) {  // (a tensor subclass that dispatches to Python has no data of its own)
+    return !t.unsafeGetTensorImpl()->is_python_dispatch() && t.is_contiguous() && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+  };
   const int64_t N = w.size(0), K = w.size(1);
   if (!(x.scalar_type() == at::kBFloat16 && w.scalar_type() == at::kBFloat16 && x.is_cuda() && w.device() == x.device() &&
-        x.size(-1) == K && dense(x) && dense(w) && (!b || (b->scalar_type() == at::kBFloat16 && dense(*b))) &&
+        x.size(-1) == K && dense(x) && dense(w) &&
+        (!b || (b->scalar_type() == at::kBFloat16 && b->device() == x.device() && b->numel() == N && dense(*b))) &&
         vig_linear_preferred(x.numel() / K, (int)N, (int)K)))
     return at::linear(x, w, b);
   const c10::DeviceGuard guard(x.device());

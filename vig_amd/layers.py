@@ -709,6 +709,9 @@ class ViG(nn.Module):
                 and conv2.kernel_size == (3, 3) and conv2.stride == (2, 2) and conv2.padding == (1, 1) and conv2.dilation == (1, 1)
                 and conv2.groups == 1 and conv2.in_channels % 32 == 0 and self.embed_dim <= 1024 and self.embed_dim % 32 == 0):
             return None
+        if (conv2.weight.shape != (self.embed_dim, conv2.in_channels, 3, 3)
+                or conv1.weight.shape != (conv2.in_channels, conv1.in_channels, *conv1.kernel_size)):
+            return None
         # besides the module tree and every parameter, what has to stay as it is
         settings = {GatedLinearAttention: ("strong_gates", "layernorm_eps", "clamp_min", "use_out_act", "use_act_in_conv",
                                            "gate_logit_normalizer", "num_heads", "training"),
@@ -726,7 +729,9 @@ class ViG(nn.Module):
             for blk in self.blocks:
                 at, C = blk.attn, self.embed_dim
                 conv, srcs = at.in_proj[0], (at.qkv_proj.weight, at.g_proj.weight, at.gk_proj[0].weight)
-                n = [t.shape[0] for t in srcs]
+                n = [at.num_heads * (2 * at.head_qk_dim + at.head_v_dim), at.num_heads * at.head_v_dim, ops.GATE_RANK]
+                if n[1] != C or any(t.shape != (h, C) for t, h in zip(srcs, n)) or at.g_proj.bias is None:
+                    return None  # (make_plan looks at the other shapes)
                 pad = -sum(n) % 128
                 rows += [*srcs, zero[:pad * C].view(pad, C)]
                 biases += [zero[:n[0]], at.g_proj.bias, zero[:n[2] + pad]]

@@ -919,14 +919,20 @@ def patch_conv(x: torch.Tensor, w_packed: torch.Tensor, kernel_hw, stride: int =
     return y
 
 
+def _owns_data(*ts) -> bool:
+    """Whether these are tensors proper: a subclass may compute its values when it is used, and has no data pointer."""
+    return all(type(t) in (torch.Tensor, torch.nn.Parameter) for t in ts if t is not None)
+
+
 def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """x @ weight.T (+ bias): vig_linear_fwd for bf16 rows at the sizes where it is the better choice, torch's product
     otherwise.  Inference only (no autograd node of its own)."""
     N, K = weight.shape
-    if (x.dtype == weight.dtype == torch.bfloat16 and x.is_cuda and x.shape[-1] == K and x.is_contiguous()
-            and weight.is_contiguous() and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0
-            and (bias is None or (bias.dtype == x.dtype and bias.is_contiguous() and bias.data_ptr() % 16 == 0))
-            and not torch.is_autocast_enabled()):
+    if (x.dtype == weight.dtype == torch.bfloat16 and x.is_cuda and weight.device == x.device and x.shape[-1] == K
+            and x.is_contiguous() and weight.is_contiguous() and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0
+            and (bias is None or (bias.dtype == x.dtype and bias.device == x.device and bias.shape == (N,)
+                                  and bias.is_contiguous() and bias.data_ptr() % 16 == 0))
+            and _owns_data(x, weight, bias) and not torch.is_autocast_enabled()):
         lib, rows = _lib.load(), x.numel() // K
         if lib.vig_linear_preferred(rows, N, K):
             y = torch.empty(*x.shape[:-1], N, dtype=x.dtype, device=x.device)
@@ -944,7 +950,8 @@ def conv3x3s2(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     B, Cin, H, W = x.shape
     Cout = weight.shape[0]
     xl, wl = x.permute(0, 2, 3, 1), weight.detach().permute(0, 2, 3, 1)
-    if not (x.dtype == weight.dtype == torch.bfloat16 and x.is_cuda and x.numel() and Cin % 32 == 0 and Cout % 8 == 0
+    if not (_owns_data(x, weight) and x.dtype == weight.dtype == torch.bfloat16 and x.is_cuda and weight.device == x.device and x.numel()
+            and Cin % 32 == 0 and Cout % 8 == 0
             and weight.shape[1:] == (Cin, 3, 3) and xl.is_contiguous() and wl.is_contiguous()
             and xl.data_ptr() % 16 == 0 and wl.data_ptr() % 16 == 0 and not torch.is_autocast_enabled()):
         return torch.nn.functional.conv2d(x, weight, None, 2, 1)
@@ -957,8 +964,12 @@ def conv3x3s2(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
 
 def rmsnorm_pool(x: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
     """mean over tokens of rmsnorm(x + residual) for bf16 [B, L, C] -> [B, C] (vig.py:896-905) in one pass."""
+    _check_cuda(x, residual, weight)
     x, residual = _dense(x), _dense(residual)
     B, L, C = x.shape
+    if not (x.dtype == residual.dtype == torch.bfloat16 and residual.shape == x.shape and weight.dtype == torch.float32
+            and weight.shape == (C,) and weight.is_contiguous()):
+        raise ValueError("rmsnorm_pool takes bf16 x and residual [B, L, C] and a float32 weight [C]")
     lib = _lib.load()
     out = torch.empty(B, C, dtype=x.dtype, device=x.device)
     need = lib.vig_rmsnorm_pool_workspace(B, L, C)
