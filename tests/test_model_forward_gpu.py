@@ -2,6 +2,7 @@
 module forward, float64 sums, and after the model has changed under the plan."""
 import pytest
 import torch
+from torch.nn.utils import prune
 
 import vig_amd
 from vig_amd import _ext, layers, ops
@@ -128,6 +129,47 @@ def test_layers_of_another_shape_or_device(monkeypatch):
     m, x = _tiny()
     m.blocks[1].mlp = layers.GLAMLP(192, intermediate_size=72).cuda().bfloat16()
     assert torch.equal(m(x), _modules(monkeypatch, m, x)) and m in layers._PLANS
+
+
+@pytest.mark.parametrize("name", ["blocks.1.mlp.down_proj", "blocks.0.attn.qkv_proj", "blocks.0.attn.o_proj", "head",
+                                  "patch_embed.proj.4", "blocks.1.mlp_norm"])
+def test_weights_that_are_not_parameters(name, monkeypatch):
+    """A weight that is computed by a hook or kept as a buffer is read anew on every call: no plan holds it."""
+    announce(f"weights that are not parameters: {name}")
+    m, x = _tiny()
+    layer = m.get_submodule(name)
+    with torch.no_grad():  # (a norm's weights are all alike at first)
+        layer.weight.add_(torch.randn_like(layer.weight) * layer.weight.std().nan_to_num(1.0).clamp_min(0.3))
+    seen = [m(x)]
+    for share in (0.2, 0.5, 0.5):
+        prune.random_unstructured(layer, "weight", share)
+        seen.append(m(x))
+        assert torch.equal(seen[-1], _modules(monkeypatch, m, x)) and not torch.equal(seen[-1], seen[-2])
+    assert m not in layers._PLANS
+    prune.remove(layer, "weight")
+    assert torch.equal(m(x), seen[-1]) and m in layers._PLANS
+    w = layer.weight.detach().clone()
+    del layer.weight
+    layer.register_buffer("weight", w)
+    assert torch.equal(m(x), seen[-1])
+    layer.weight = w * 2
+    assert torch.equal(m(x), _modules(monkeypatch, m, x)) and not torch.equal(m(x), seen[-1])
+
+
+def test_settings_that_change_under_a_plan(monkeypatch):
+    """What the module by module forward reads on every call besides the weights."""
+    announce("settings that change under a plan")
+    m, x = _tiny()
+    first = m(x)
+    m.patch_embed.proj[3].stride = (1, 1)  # four times the tokens
+    assert torch.equal(m(x), _modules(monkeypatch, m, x)) and not torch.equal(m(x), first)
+    m.patch_embed.proj[3].stride = (2, 2)
+    assert torch.equal(m(x), first)
+    seen = []
+    m.blocks[1].mlp.register_forward_hook(lambda *a: seen.append(1))
+    assert torch.equal(m(x), first) and not seen  # (a block with one eps is one operator)
+    m.blocks[1].mlp_norm.eps = 0.5
+    assert torch.equal(m(x), _modules(monkeypatch, m, x)) and len(seen) == 2
 
 
 @pytest.mark.parametrize("kw,side,B", [(dict(embed_dim=192, num_heads=3, use_out_act=True, use_act_in_conv=True), 224, 1),

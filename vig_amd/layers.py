@@ -103,6 +103,13 @@ def _linear(module: nn.Linear, x):
     return ops.linear(x, module.weight, module.bias)
 
 
+def _owns_weights(m: nn.Module, *names) -> bool:
+    """Whether the weights of m are its parameters.  Pruned, weight-normalised, sharded and replicated layers keep their type and
+    make `weight` a plain attribute, which is another tensor whenever it is computed anew; some keep it as a buffer."""
+    names = names or [n for n in ("weight", "bias") if hasattr(m, n)]
+    return all(n in m._parameters and n not in m.__dict__ for n in names)
+
+
 def _plain(*modules: nn.Module) -> bool:
     """True when nothing hangs on calling these modules by themselves: training mode and no hooks."""
     return all(m.training and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks)
@@ -703,7 +710,7 @@ class ViG(nn.Module):
             typed += [(m, nn.Linear) for m in (at.qkv_proj, at.g_proj, at.o_proj, at.gk_proj[0], at.gk_proj[1], mlp.gate_proj, mlp.down_proj)]
             if at.strong_gates or at.training or blk.training or at.gk_proj[0].weight.shape[0] != ops.GATE_RANK or at.head_v_dim != 64 or at.head_qk_dim not in (32, 64):
                 return None
-        if not all(type(m) is t for m, t in typed):
+        if not all(type(m) is t and _owns_weights(m) for m, t in typed) or not _owns_weights(self, "pos_embed"):
             return None
         if not (conv1.stride == (8, 8) and conv1.padding == (1, 1) and conv1.dilation == (1, 1) and conv1.groups == 1
                 and conv2.kernel_size == (3, 3) and conv2.stride == (2, 2) and conv2.padding == (1, 1) and conv2.dilation == (1, 1)
@@ -714,11 +721,17 @@ class ViG(nn.Module):
             return None
         # besides the module tree and every parameter, what has to stay as it is
         settings = {GatedLinearAttention: ("strong_gates", "layernorm_eps", "clamp_min", "use_out_act", "use_act_in_conv",
-                                           "gate_logit_normalizer", "num_heads", "training"),
-                    GLABlock: ("training",), RMSNorm: ("eps",), LayerNorm2d: ("eps",), ViG: ("patch_resolution",)}
+                                           "gate_logit_normalizer", "num_heads", "head_qk_dim", "head_v_dim", "training"),
+                    GLABlock: ("training",), RMSNorm: ("eps",), LayerNorm2d: ("eps",), ViG: ("patch_resolution",),
+                    nn.Conv2d: ("stride", "padding", "dilation", "groups")}
         absent = {GLABlock: "forward_carry", GatedLinearAttention: "_mix", ViG: "forward_features"}
         called = [pe, norm1, act, norm2, self.norm, self.head, torch.nn.modules.module._global_forward_hooks,
                   torch.nn.modules.module._global_forward_pre_hooks]
+        for blk in self.blocks:
+            if blk.attn_norm.eps != blk.mlp_norm.eps:  # such a block runs module by module (GLABlock.forward_carry)
+                called += [blk.attn_norm, blk.attn, blk.mlp_norm, blk.drop_path, blk.mlp, blk.mlp.gate_proj, blk.mlp.down_proj]
+                if type(blk.drop_path) not in (nn.Identity, DropPath):
+                    return None
         flag = lambda v: 1 if v else 0  # noqa: E731
         with torch.no_grad():
             # all small weights in fp32 by one concatenation and one cast, all stacked projections by one concatenation: layer by
