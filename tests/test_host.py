@@ -132,3 +132,35 @@ def test_weight_copies_follow_weights_that_are_computed_anew():
         at.g_proj._parameters["weight"] = torch.full((64, 64), float(i))
         assert (at._stacked_in()[0][at.qkv_proj.weight.shape[0]:][:64] == i).all()
         at.g_proj._parameters["weight"] = None
+
+
+def test_layers_are_called_where_something_hangs_on_the_call():
+    """A product is taken from a layer's weights only where calling the layer comes to no more than that."""
+    from torch.nn.modules import module as g
+    from vig_amd import layers
+
+    x, seen = torch.randn(3, 8), []
+    hook = lambda *a: seen.append(1)  # noqa: E731
+    plain = torch.nn.Linear(8, 4)
+    assert layers._direct(plain) and torch.equal(layers._linear(plain, x), plain(x))
+    for change in ("forward", "compile", "hook", "pre-hook", "global hook", "global pre-hook"):
+        lin, handle = torch.nn.Linear(8, 4), None
+        if change == "forward":
+            lin.forward = lambda x: torch.full((3, 4), 7.0)
+        elif change == "compile":
+            lin._compiled_call_impl = lambda x: torch.full((3, 4), 7.0)
+        elif "global" in change:
+            handle = (g.register_module_forward_hook if change == "global hook" else g.register_module_forward_pre_hook)(hook)
+        else:
+            (lin.register_forward_hook if change == "hook" else lin.register_forward_pre_hook)(hook)
+        try:
+            assert not layers._direct(lin), change
+            y = layers._linear(lin, x)
+        finally:
+            if handle is not None:
+                handle.remove()
+        assert (y == 7.0).all() if change in ("forward", "compile") else len(seen) == 1, change
+        seen.clear()
+    lin = torch.nn.Linear(8, 4)
+    lin.register_full_backward_hook(hook)
+    assert not layers._direct(lin)

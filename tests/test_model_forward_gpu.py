@@ -156,6 +156,30 @@ def test_weights_that_are_not_parameters(name, monkeypatch):
     assert torch.equal(m(x), _modules(monkeypatch, m, x)) and not torch.equal(m(x), seen[-1])
 
 
+@pytest.mark.parametrize("name", ["head", "norm", "patch_embed", "patch_embed.proj.1"])
+def test_forwards_replaced_on_an_instance(name):
+    announce(f"forward replaced on {name}, hooks on all modules")
+    m, x = _tiny()
+    first, layer = m(x), m.get_submodule(name)
+    seen = []
+
+    def forward(*args, **kwargs):
+        seen.append(1)
+        return type(layer).forward(layer, *args, **kwargs)
+
+    layer.forward = forward
+    second = m(x)
+    assert len(seen) == 1 and (second.float() - first.float()).norm() <= 2.0 ** -8 * first.float().norm()
+    del layer.forward
+    assert torch.equal(m(x), first) and len(seen) == 1
+    handle = torch.nn.modules.module.register_module_forward_hook(lambda m, *a: seen.append(m))
+    try:
+        m(x)
+    finally:
+        handle.remove()
+    assert layer in seen[1:]
+
+
 def test_settings_that_change_under_a_plan(monkeypatch):
     """What the module by module forward reads on every call besides the weights."""
     announce("settings that change under a plan")

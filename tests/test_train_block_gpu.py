@@ -2,6 +2,7 @@
 block run module by module in fp32, and against float64 sums."""
 import pytest
 import torch
+from torch.nn.utils import prune
 
 from vig_amd import _lib, layers
 
@@ -74,6 +75,57 @@ def test_recorded_block(B, hw, C, H, Dk, act, bias, clamp, mode, tol):
         for n, w in want.items():
             e = _rel(got[n].detach(), w.detach())
             assert e <= tol * (1 if n in ("y", "total") or mode == "fp32" else 2), (residual, n, e)
+
+
+class _Doubled(layers.RMSNorm):
+    def forward(self, *args, **kwargs):
+        y = super().forward(*args, **kwargs)
+        return (2 * y[0], *y[1:]) if isinstance(y, tuple) else 2 * y
+
+
+@pytest.mark.parametrize("change", ["adapter", "norm", "gate layers", "pruned", "hook on all modules", "mixer"])
+def test_block_runs_module_by_module_where_something_hangs_on_a_call(change):
+    announce(f"recorded block with a changed module: {change}")
+    torch.manual_seed(3)
+    blk = layers.GLABlock(192, 3, 0.5, 1.0, intermediate_size=512).cuda().train()
+    with torch.no_grad():  # (as initialised, the mixer hardly shows in the output)
+        for p in blk.parameters():
+            p.add_(torch.randn_like(p) * p.shape[-1] ** -0.5)
+    at, seen, handle = blk.attn, [], None
+    x = torch.randn(2, 30, 192, device="cuda")
+
+    def run():
+        blk.zero_grad()
+        y, _ = blk.forward_carry(x, None, patch_resolution=(5, 6))
+        y.square().sum().backward()
+        return y, [p.grad.clone() for p in blk.parameters() if p.grad is not None]
+
+    before, _ = run()
+    assert "Mlp" in before.grad_fn.name()
+    if change == "adapter":
+        at.qkv_proj.forward = lambda h, lin=at.qkv_proj: torch.nn.Linear.forward(lin, h) + 0.5 * h.repeat(1, 1, 2)
+    elif change == "norm":
+        norm = _Doubled(192).cuda()
+        norm.load_state_dict(blk.mlp_norm.state_dict())
+        blk.mlp_norm = norm
+    elif change == "gate layers":
+        at.gk_proj.append(torch.nn.Hardtanh(-0.01, 0.01))
+    elif change == "pruned":
+        torch.manual_seed(4)
+        prune.random_unstructured(blk.mlp.down_proj, "weight", 0.5)
+    elif change == "mixer":
+        at._mix_autograd = lambda h, hw, s: 2 * type(at)._mix_autograd(at, h, hw, s)
+    else:
+        handle = torch.nn.modules.module.register_module_forward_hook(lambda *a: seen.append(1))
+    try:
+        got, grads = run()
+        blk._recorded = lambda *a, **k: None
+        want, wanted = run()
+    finally:
+        if handle is not None:
+            handle.remove()
+    assert torch.equal(got, want) and all(torch.equal(a, b) for a, b in zip(grads, wanted, strict=True))
+    assert seen if change == "hook on all modules" else not torch.allclose(got, before, rtol=1e-3, atol=1e-3)
 
 
 @pytest.mark.parametrize("rows,N,K", [(1, 8, 8), (33, 40, 16), (65, 136, 264), (1000, 384, 16), (2500, 1168, 384), (4097, 200, 192)])

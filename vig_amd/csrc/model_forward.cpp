@@ -315,8 +315,8 @@ PyObject* make_plan(PyObject*, PyObject* const* a, Py_ssize_t n) {
   auto p = std::make_unique<Plan>();
   std::vector<PyObject*> seen;
   if (!collect(*p, a[0], a[1], a[2], seen)) Py_RETURN_NONE;
-  const Ref forward(PyUnicode_InternFromString("forward"));
-  Py_DECREF(forward.o);
+  const Ref forward(PyUnicode_InternFromString("forward")), compiled(PyUnicode_InternFromString("_compiled_call_impl"));
+  Py_DECREF(forward.o), Py_DECREF(compiled.o);
   for (Py_ssize_t i = 0; i < PyList_GET_SIZE(a[3]); ++i) {
     PyObject* m = PyList_GET_ITEM(a[3], i);
     if (PyDict_Check(m)) {
@@ -328,7 +328,7 @@ PyObject* make_plan(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const Ref hold(own);
     Py_DECREF(own);
     for (const char* table : {"_forward_hooks", "_forward_pre_hooks"}) p->empty.emplace_back(PyDict_GetItemString(own, table));
-    p->entries.push_back({Ref(own), Ref(forward.o), Ref(nullptr)});
+    for (PyObject* name : {forward.o, compiled.o}) p->entries.push_back({Ref(own), Ref(name), Ref(nullptr)});
   }
   if (!still_valid(*p)) Py_RETURN_NONE;
   a += 1;

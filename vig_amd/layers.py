@@ -96,9 +96,23 @@ def _recording(module: nn.Module) -> bool:
     return module.training and torch.is_grad_enabled()
 
 
+_OVERRIDES = ("forward", "_compiled_call_impl", "_mix", "_mix_autograd")  # what an instance may hold in place of its class's
+
+
+def _direct(*modules: nn.Module) -> bool:
+    """Whether calling these modules comes to their classes' forward and nothing else: no hook of their own or of all modules
+    (adapters and counters hang there), no method replaced on the instance, none compiled.  Every path that takes a
+    module's weights instead of calling it asks this first."""
+    g = torch.nn.modules.module
+    if g._global_forward_hooks or g._global_forward_pre_hooks or g._global_backward_hooks or g._global_backward_pre_hooks:
+        return False
+    return all(not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks)
+               and m.__dict__.keys().isdisjoint(_OVERRIDES) for m in modules)
+
+
 def _linear(module: nn.Linear, x):
     """module(x) outside of autograd, on the library's product where that is the better choice."""
-    if type(module) is not nn.Linear or module._forward_hooks or module._forward_pre_hooks:
+    if type(module) is not nn.Linear or not _direct(module):
         return module(x)
     return ops.linear(x, module.weight, module.bias)
 
@@ -108,12 +122,6 @@ def _owns_weights(m: nn.Module, *names) -> bool:
     make `weight` a plain attribute, which is another tensor whenever it is computed anew; some keep it as a buffer."""
     names = names or [n for n in ("weight", "bias") if hasattr(m, n)]
     return all(n in m._parameters and n not in m.__dict__ for n in names)
-
-
-def _plain(*modules: nn.Module) -> bool:
-    """True when nothing hangs on calling these modules by themselves: training mode and no hooks."""
-    return all(m.training and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks)
-               for m in modules)
 
 
 class RMSNorm(_CacheMixin, nn.Module):
@@ -456,16 +464,18 @@ class GLABlock(nn.Module):
     def _recorded(self, branch, residual, patch_resolution, token_position=None, **kwargs):
         """The block as two autograd nodes (csrc/train_block.cpp), stochastic depth on each branch between them: (branch,
         residual) in and out as forward_carry has them.  None for what the nodes do not take: submodules of other types,
-        with hooks or partly in evaluation mode, and the shapes and types they refuse; the modules then run one by one."""
+        with something hanging on their calls or partly in evaluation mode, and the shapes and types they refuse; the modules
+        then run one by one."""
         calls = _ext.calls()
         at, mlp = self.attn, self.mlp
         if calls is None or type(at) is not GatedLinearAttention or type(mlp) is not GLAMLP or token_position is not None:
             return None
         conv, up = at.in_proj[0], at.gk_proj
         linears = (at.qkv_proj, at.g_proj, at.o_proj, up[0], up[1], mlp.gate_proj, mlp.down_proj)
-        if not (all(type(m) is nn.Linear for m in linears) and type(conv) is nn.Conv2d
-                and _plain(at, mlp, self.attn_norm, self.mlp_norm, at.g_norm, at.l_norm, at.in_proj, conv, at.in_proj[1], up,
-                           *linears)):
+        called = (at, mlp, self.attn_norm, self.mlp_norm, up, *linears)
+        if not (all(type(m) is nn.Linear for m in linears) and type(conv) is nn.Conv2d and type(up) is nn.Sequential and len(up) == 2
+                and type(self.attn_norm) is type(self.mlp_norm) is RMSNorm and _direct(*called)
+                and all(m.training for m in (*called, at.g_norm, at.l_norm, at.in_proj, conv, at.in_proj[1]))):
             return None
         h, w = patch_resolution
         mixed = calls.block_mix(branch.contiguous(), residual, self.attn_norm.weight, conv.weight, conv.bias, at.qkv_proj.weight,
@@ -659,7 +669,7 @@ class ViG(nn.Module):
         if residual is None:
             x = self.norm(branch)
         elif (not torch.is_grad_enabled() and type(self.norm) is RMSNorm and branch.is_cuda and self.embed_dim <= 1024
-              and branch.dtype == residual.dtype == torch.bfloat16 and not (self.norm._forward_hooks or self.norm._forward_pre_hooks)):
+              and branch.dtype == residual.dtype == torch.bfloat16 and _direct(self.norm)):
             return ops.rmsnorm_pool(branch, residual, self.norm._w32(), self.norm.eps)
         else:
             x = self.norm(branch, residual, round_sum=True)
