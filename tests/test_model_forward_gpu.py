@@ -180,6 +180,44 @@ def test_forwards_replaced_on_an_instance(name):
     assert layer in seen[1:]
 
 
+class _Products(torch.utils._python_dispatch.TorchDispatchMode):
+    """Counts the matrix products of the operators that it sees."""
+
+    def __init__(self):
+        super().__init__()
+        self.seen = 0
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        self.seen += "mm" in str(func)
+        return func(*args, **(kwargs or {}))
+
+
+@pytest.mark.filterwarnings("ignore::torch.jit.TracerWarning")
+def test_calls_that_are_observed():
+    """A trace holds the products it needs (or is refused, as the operators that return an optional tensor are); a dispatch
+    mode, which FLOP counters are, sees the products of an evaluation forward and of a training block."""
+    announce("a trace, a dispatch mode")
+    m, x = _tiny()
+    y = m(x)
+    mlp, rows = m.blocks[0].mlp, [_randn((2, 49, 192), s).cuda() for s in (11, 12)]
+    with torch.no_grad():
+        traced = torch.jit.trace(mlp, rows[0], check_trace=False)
+        err = (traced(rows[1]).float() - mlp(rows[1]).float()).norm() / mlp(rows[1]).float().norm()
+        assert err <= 2.0 ** -8, err
+        with pytest.raises(RuntimeError):
+            torch.jit.trace(m, x, check_trace=False)
+    with _Products() as mode:
+        got = m(x)
+    # a block's input and down projection (its other products lie in operators of this package), and the classifier
+    assert mode.seen == 2 * 2 + 1 and (got.float() - y.float()).norm() <= 2.0 ** -8 * y.float().norm()
+    blk = m.blocks[0].float().train()
+    h = torch.randn(2, 16, 192, device="cuda", requires_grad=True)
+    with _Products() as mode:
+        out, total = blk.forward_carry(h, None, patch_resolution=(4, 4))
+        (out.sum() + total.sum()).backward()
+    assert mode.seen == 7 * 3  # seven layers, each with two gradients
+
+
 def test_settings_that_change_under_a_plan(monkeypatch):
     """What the module by module forward reads on every call besides the weights."""
     announce("settings that change under a plan")

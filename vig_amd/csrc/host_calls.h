@@ -2,7 +2,9 @@
 #pragma once
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
+#include <ATen/TracerMode.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
@@ -29,6 +31,10 @@ inline int dtype_code(const Tensor& t) {
   const auto s = t.scalar_type();
   return s == at::kBFloat16 ? VIG_BF16 : (s == at::kFloat ? VIG_F32 : -1);
 }
+// Whether somebody records the operators of this call (a trace, a FLOP counter or another dispatch mode): kernels launched
+// outside of the dispatcher would be missing from the record, a trace would keep their uninitialised outputs.
+inline bool observed() { return at::tracer::impl::is_dispatch_enabled() || c10::impl::dispatch_mode_enabled(); }
+
 // (a tensor subclass that dispatches to Python has no data of its own)
 inline bool plain(const Tensor& t, const c10::Device& dev) {
   return t.defined() && !t.unsafeGetTensorImpl()->is_python_dispatch() && t.layout() == at::kStrided && t.device() == dev && t.is_contiguous() &&

@@ -387,7 +387,7 @@ PyObject* run_plan(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const Tensor images = THPVariable_Unpack(a[1]);
   const Stem& st = p->stem;
   if (images.dim() != 4 || !plain(images, st.w1.device()) || images.scalar_type() != at::kBFloat16 || images.numel() == 0) Py_RETURN_NONE;
-  if (at::autocast::is_autocast_enabled(at::kCUDA)) Py_RETURN_NONE;
+  if (at::autocast::is_autocast_enabled(at::kCUDA) || observed()) Py_RETURN_NONE;
   const int64_t B = images.size(0), S = images.size(2), W = images.size(3), half = st.w1.size(0);
   const int64_t oh1 = (S + 2 - st.KH) / 8 + 1, ow1 = (W + 2 - st.KW) / 8 + 1;
   // the stem's shape, and the grid the position table is for

@@ -7,7 +7,9 @@
 // chunk_fuse.py:554-596 and recurrent_fuse.py:631-676, and the eval branch of GatedLinearAttention.forward
 // (classification/models/vig.py:427-463).
 #include <ATen/ATen.h>
+#include <ATen/TracerMode.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/library.h>
 
@@ -75,7 +77,8 @@ Tensor product(const Tensor& x, const Tensor& w, const optional<Tensor>& b = c10
     return !t.unsafeGetTensorImpl()->is_python_dispatch() && t.is_contiguous() && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
   };
   const int64_t N = w.size(0), K = w.size(1);
-  if (!(x.scalar_type() == at::kBFloat16 && w.scalar_type() == at::kBFloat16 && x.is_cuda() && w.device() == x.device() &&
+  const bool observed = at::tracer::impl::is_dispatch_enabled() || c10::impl::dispatch_mode_enabled();  // (host_calls.h)
+  if (!(!observed && x.scalar_type() == at::kBFloat16 && w.scalar_type() == at::kBFloat16 && x.is_cuda() && w.device() == x.device() &&
         x.size(-1) == K && dense(x) && dense(w) &&
         (!b || (b->scalar_type() == at::kBFloat16 && b->device() == x.device() && b->numel() == N && dense(*b))) &&
         vig_linear_preferred(x.numel() / K, (int)N, (int)K)))

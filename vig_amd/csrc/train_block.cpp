@@ -444,7 +444,7 @@ struct MlpNode : torch::autograd::Function<MlpNode> {
 
 // Whether branch and residual are rows the nodes take and the weights share one usable type; sets the products' type.
 bool stream_ok(const Tensor& branch, const Tensor& residual, const Tensor* const* params, int n, bool& bf16) {
-  if (!branch.defined() || !branch.is_cuda() || branch.dim() != 3 || branch.numel() == 0) return false;
+  if (!branch.defined() || !branch.is_cuda() || branch.dim() != 3 || branch.numel() == 0 || observed()) return false;
   const auto dev = branch.device();
   if (!plain(branch, dev) || dtype_code(branch) < 0) return false;
   if (residual.defined() && (!plain(residual, dev) || residual.sizes() != branch.sizes() || dtype_code(residual) < 0)) return false;

@@ -669,7 +669,7 @@ class ViG(nn.Module):
         if residual is None:
             x = self.norm(branch)
         elif (not torch.is_grad_enabled() and type(self.norm) is RMSNorm and branch.is_cuda and self.embed_dim <= 1024
-              and branch.dtype == residual.dtype == torch.bfloat16 and _direct(self.norm)):
+              and branch.dtype == residual.dtype == torch.bfloat16 and _direct(self.norm) and not ops.observed()):
             return ops.rmsnorm_pool(branch, residual, self.norm._w32(), self.norm.eps)
         else:
             x = self.norm(branch, residual, round_sum=True)

@@ -924,6 +924,12 @@ def _owns_data(*ts) -> bool:
     return all(type(t) in (torch.Tensor, torch.nn.Parameter) for t in ts if t is not None)
 
 
+def observed() -> bool:
+    """Whether somebody records the operators of this call (a trace, a FLOP counter or another dispatch mode): kernels launched
+    outside of the dispatcher would be missing from the record, and a trace would keep their uninitialised outputs."""
+    return torch._C._get_tracing_state() is not None or torch._C._len_torch_dispatch_stack() > 0
+
+
 def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """x @ weight.T (+ bias): vig_linear_fwd for bf16 rows at the sizes where it is the better choice, torch's product
     otherwise.  Inference only (no autograd node of its own)."""
@@ -932,7 +938,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] =
             and x.is_contiguous() and weight.is_contiguous() and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0
             and (bias is None or (bias.dtype == x.dtype and bias.device == x.device and bias.shape == (N,)
                                   and bias.is_contiguous() and bias.data_ptr() % 16 == 0))
-            and _owns_data(x, weight, bias) and not torch.is_autocast_enabled()):
+            and _owns_data(x, weight, bias) and not torch.is_autocast_enabled() and not observed()):
         lib, rows = _lib.load(), x.numel() // K
         if lib.vig_linear_preferred(rows, N, K):
             y = torch.empty(*x.shape[:-1], N, dtype=x.dtype, device=x.device)
@@ -950,8 +956,8 @@ def conv3x3s2(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     B, Cin, H, W = x.shape
     Cout = weight.shape[0]
     xl, wl = x.permute(0, 2, 3, 1), weight.detach().permute(0, 2, 3, 1)
-    if not (_owns_data(x, weight) and x.dtype == weight.dtype == torch.bfloat16 and x.is_cuda and weight.device == x.device and x.numel()
-            and Cin % 32 == 0 and Cout % 8 == 0
+    if not (_owns_data(x, weight) and not observed() and x.dtype == weight.dtype == torch.bfloat16 and x.is_cuda
+            and weight.device == x.device and x.numel() and Cin % 32 == 0 and Cout % 8 == 0
             and weight.shape[1:] == (Cin, 3, 3) and xl.is_contiguous() and wl.is_contiguous()
             and xl.data_ptr() % 16 == 0 and wl.data_ptr() % 16 == 0 and not torch.is_autocast_enabled()):
         return torch.nn.functional.conv2d(x, weight, None, 2, 1)
