@@ -180,6 +180,24 @@ def test_forwards_replaced_on_an_instance(name):
     assert layer in seen[1:]
 
 
+def test_plans_of_other_models_stay(monkeypatch):
+    """train(), eval(), a load and invalidate_caches drop the plan of the model whose modules they touch, and no other."""
+    announce("plans of other models")
+    a, x = _tiny()
+    b, _ = _tiny(128)
+    a(x), b(x)
+    plan = layers._PLANS[a]
+    for touch in (b.eval, b.blocks[0].attn.eval, b.patch_embed.eval, lambda: b.load_state_dict(b.state_dict()),
+                  lambda: layers.invalidate_caches(b.blocks)):
+        assert b in layers._PLANS
+        touch()
+        assert b not in layers._PLANS and layers._PLANS[a] is plan
+        b(x)
+    b.head.weight.data.mul_(2.0), b.blocks[1].mlp_norm.weight.data.mul_(2.0)  # behind the version counter
+    b.eval()
+    assert torch.equal(b(x), _modules(monkeypatch, b, x))
+
+
 class _Products(torch.utils._python_dispatch.TorchDispatchMode):
     """Counts the matrix products of the operators that it sees."""
 

@@ -100,6 +100,7 @@ PyObject* block_mlp(PyObject*, PyObject* const* a, Py_ssize_t n);
 
 // the methods of model_forward.cpp
 PyObject* make_plan(PyObject*, PyObject* const* a, Py_ssize_t n);
+PyObject* plan_describes(PyObject*, PyObject* const* a, Py_ssize_t n);
 PyObject* run_plan(PyObject*, PyObject* const* a, Py_ssize_t n);
 
 }  // namespace vig_host

@@ -51,6 +51,7 @@ struct Plan {
   std::vector<Entry> entries;
   std::vector<Ref> empty;
   std::vector<Watched> watched;
+  std::vector<PyObject*> modules;  // sorted; the model itself, and children that `entries` keep alive
   Stem stem;
   std::vector<Block> blocks;
   Tensor norm, head_w, head_b;
@@ -84,7 +85,10 @@ struct Reader {
     if (!o) throw python_error();
     return o;
   }
-  Tensor tensor() { return tensor_arg(next()); }
+  Tensor tensor() {  // an alias outside of autograd
+    const Tensor t = tensor_arg(next());
+    return t.defined() ? t.detach() : t;
+  }
   double real() {
     PyObject* o = next();
     const double v = o == Py_None ? std::nan("") : PyFloat_AsDouble(o);
@@ -313,8 +317,8 @@ PyObject* make_plan(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   TORCH_CHECK_TYPE(n == 7, "make_plan takes 7 arguments");
   auto p = std::make_unique<Plan>();
-  std::vector<PyObject*> seen;
-  if (!collect(*p, a[0], a[1], a[2], seen)) Py_RETURN_NONE;
+  if (!collect(*p, a[0], a[1], a[2], p->modules)) Py_RETURN_NONE;
+  std::sort(p->modules.begin(), p->modules.end());
   const Ref forward(PyUnicode_InternFromString("forward")), compiled(PyUnicode_InternFromString("_compiled_call_impl"));
   Py_DECREF(forward.o), Py_DECREF(compiled.o);
   for (Py_ssize_t i = 0; i < PyList_GET_SIZE(a[3]); ++i) {
@@ -374,6 +378,18 @@ PyObject* make_plan(PyObject*, PyObject* const* a, Py_ssize_t n) {
   }
   if (!ok) Py_RETURN_NONE;
   return PyCapsule_New(p.release(), kPlanName, [](PyObject* cap) { free_plan(cap); });
+  END_HANDLE_TH_ERRORS
+}
+
+// plan_describes(plan, modules [list]) -> whether one of them is the plan's model or part of it
+PyObject* plan_describes(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK_TYPE(n == 2 && PyList_Check(a[1]), "plan_describes takes a plan and a list");
+  const auto* p = static_cast<const Plan*>(PyCapsule_GetPointer(a[0], kPlanName));
+  if (!p) return nullptr;
+  for (Py_ssize_t i = 0; i < PyList_GET_SIZE(a[1]); ++i)
+    if (std::binary_search(p->modules.begin(), p->modules.end(), PyList_GET_ITEM(a[1], i))) Py_RETURN_TRUE;
+  Py_RETURN_FALSE;
   END_HANDLE_TH_ERRORS
 }
 

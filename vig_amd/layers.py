@@ -70,8 +70,11 @@ def invalidate_caches(model: nn.Module) -> None:
     a write through `.data` (p.data.mul_(..), module.weight.data[...] = ..) changes neither the pointer nor the version
     counter they are keyed on, so code that writes that way calls this afterwards.  load_state_dict and train() /
     eval() switches of these modules call it by themselves."""
-    _PLANS.clear()
-    for m in model.modules():
+    modules = list(model.modules())
+    for owner, plan in list(_PLANS.items()) if len(_PLANS) else ():  # (a plan goes when any module that it describes is named here, and stays otherwise)
+        if owner is model or _ext.calls().plan_describes(plan, modules):
+            _PLANS.pop(owner, None)
+    for m in modules:
         for a in _CACHE_ATTRS:
             m.__dict__.pop(a, None)
         if "_in_cat" in m.__dict__:
@@ -117,11 +120,19 @@ def _linear(module: nn.Linear, x):
     return ops.linear(x, module.weight, module.bias)
 
 
-def _owns_weights(m: nn.Module, *names) -> bool:
-    """Whether the weights of m are its parameters.  Pruned, weight-normalised, sharded and replicated layers keep their type and
-    make `weight` a plain attribute, which is another tensor whenever it is computed anew; some keep it as a buffer."""
-    names = names or [n for n in ("weight", "bias") if hasattr(m, n)]
-    return all(n in m._parameters and n not in m.__dict__ for n in names)
+class _NoPlan(Exception):
+    """A model that no plan describes (ViG._planned)."""
+
+
+def _own(m: nn.Module, kind):
+    """(weight, bias) of m as its parameters, for a module of exactly this kind.  Pruned, weight-normalised, sharded and replicated
+    layers keep their type and make `weight` a plain attribute, which is another tensor whenever it is computed anew; some
+    keep it as a buffer.  (The dictionaries are read directly: nn.Module's attribute lookup takes 0.4 us, a plan needs 700.)"""
+    d = m.__dict__
+    p = d["_parameters"]
+    if type(m) is not kind or p.get("weight") is None or "weight" in d or "bias" in d or "bias" in d["_buffers"]:
+        raise _NoPlan
+    return p["weight"], p.get("bias")
 
 
 class RMSNorm(_CacheMixin, nn.Module):
@@ -707,80 +718,90 @@ class ViG(nn.Module):
         return None
 
     def _make_plan(self, calls):
-        pe = self.patch_embed
-        if type(pe) is not V2PatchEmbed or len(self.blocks) == 0 or self.head.weight.dtype is not torch.bfloat16:
+        try:
+            return self._describe(calls)
+        except _NoPlan:
             return None
+
+    def _describe(self, calls):
+        kids = self.__dict__["_modules"]
+        pe, C = kids["patch_embed"], self.embed_dim
+        if type(pe) is not V2PatchEmbed or len(kids["blocks"]) == 0 or "pos_embed" not in self._parameters:
+            raise _NoPlan
         conv1, norm1, act, conv2, norm2 = pe.proj
-        typed = [(conv1, nn.Conv2d), (norm1, LayerNorm2d), (act, nn.SiLU), (conv2, nn.Conv2d), (norm2, LayerNorm2d),
-                 (self.norm, RMSNorm), (self.head, nn.Linear)]
-        for blk in self.blocks:
-            at, mlp = blk.attn, blk.mlp
-            typed += [(blk, GLABlock), (at, GatedLinearAttention), (mlp, GLAMLP), (blk.attn_norm, RMSNorm), (blk.mlp_norm, RMSNorm),
-                      (at.g_norm, RMSNorm), (at.l_norm, RMSNorm), (at.in_proj[0], nn.Conv2d)]
-            typed += [(m, nn.Linear) for m in (at.qkv_proj, at.g_proj, at.o_proj, at.gk_proj[0], at.gk_proj[1], mlp.gate_proj, mlp.down_proj)]
-            if at.strong_gates or at.training or blk.training or at.gk_proj[0].weight.shape[0] != ops.GATE_RANK or at.head_v_dim != 64 or at.head_qk_dim not in (32, 64):
-                return None
-        if not all(type(m) is t and _owns_weights(m) for m, t in typed) or not _owns_weights(self, "pos_embed"):
-            return None
-        if not (conv1.stride == (8, 8) and conv1.padding == (1, 1) and conv1.dilation == (1, 1) and conv1.groups == 1
+        w1, b1 = _own(conv1, nn.Conv2d)
+        ln1w, ln1b = _own(norm1, LayerNorm2d)
+        w2, b2 = _own(conv2, nn.Conv2d)
+        ln2w, ln2b = _own(norm2, LayerNorm2d)
+        norm_w, _ = _own(kids["norm"], RMSNorm)
+        head_w, head_b = _own(kids["head"], nn.Linear)
+        if type(act) is not nn.SiLU or head_w.dtype is not torch.bfloat16 or not (
+                conv1.stride == (8, 8) and conv1.padding == (1, 1) and conv1.dilation == (1, 1) and conv1.groups == 1
                 and conv2.kernel_size == (3, 3) and conv2.stride == (2, 2) and conv2.padding == (1, 1) and conv2.dilation == (1, 1)
-                and conv2.groups == 1 and conv2.in_channels % 32 == 0 and self.embed_dim <= 1024 and self.embed_dim % 32 == 0):
-            return None
-        if (conv2.weight.shape != (self.embed_dim, conv2.in_channels, 3, 3)
-                or conv1.weight.shape != (conv2.in_channels, conv1.in_channels, *conv1.kernel_size)):
-            return None
+                and conv2.groups == 1 and conv2.in_channels % 32 == 0 and C <= 1024 and C % 32 == 0
+                and w2.shape == (C, conv2.in_channels, 3, 3)
+                and w1.shape == (conv2.in_channels, conv1.in_channels, *conv1.kernel_size)):
+            raise _NoPlan
         # besides the module tree and every parameter, what has to stay as it is
         settings = {GatedLinearAttention: ("strong_gates", "layernorm_eps", "clamp_min", "use_out_act", "use_act_in_conv",
                                            "gate_logit_normalizer", "num_heads", "head_qk_dim", "head_v_dim", "training"),
                     GLABlock: ("training",), RMSNorm: ("eps",), LayerNorm2d: ("eps",), ViG: ("patch_resolution",),
                     nn.Conv2d: ("stride", "padding", "dilation", "groups")}
         absent = {GLABlock: "forward_carry", GatedLinearAttention: "_mix", ViG: "forward_features"}
-        called = [pe, norm1, act, norm2, self.norm, self.head, torch.nn.modules.module._global_forward_hooks,
+        called = [pe, norm1, act, norm2, kids["norm"], kids["head"], torch.nn.modules.module._global_forward_hooks,
                   torch.nn.modules.module._global_forward_pre_hooks]
-        for blk in self.blocks:
-            if blk.attn_norm.eps != blk.mlp_norm.eps:  # such a block runs module by module (GLABlock.forward_carry)
-                called += [blk.attn_norm, blk.attn, blk.mlp_norm, blk.drop_path, blk.mlp, blk.mlp.gate_proj, blk.mlp.down_proj]
-                if type(blk.drop_path) not in (nn.Identity, DropPath):
-                    return None
         flag = lambda v: 1 if v else 0  # noqa: E731
         with torch.no_grad():
             # all small weights in fp32 by one concatenation and one cast, all stacked projections by one concatenation: layer by
             # layer these are 150 launches, 0.9 ms of a new model's first pass
-            small = [conv1.bias, norm1.weight, norm1.bias, conv2.bias, norm2.weight, norm2.bias, self.norm.weight]
-            rows, biases = [], []
-            zero = self.head.weight.new_zeros(max(m.weight.numel() for m in (self.blocks[0].attn.qkv_proj, self.blocks[0].attn.g_proj)))
-            for blk in self.blocks:
-                at, C = blk.attn, self.embed_dim
-                conv, srcs = at.in_proj[0], (at.qkv_proj.weight, at.g_proj.weight, at.gk_proj[0].weight)
+            small = [b1, ln1w, ln1b, b2, ln2w, ln2b, norm_w]
+            rows, biases, parts = [], [], []
+            zero = None
+            for blk in kids["blocks"]:
+                own = blk.__dict__["_modules"]
+                at, mlp, norm, norm2_ = own["attn"], own["mlp"], own["attn_norm"], own["mlp_norm"]
+                if (type(blk) is not GLABlock or type(at) is not GatedLinearAttention or type(mlp) is not GLAMLP or at.strong_gates
+                        or at.training or blk.training or at.head_v_dim != 64 or at.head_qk_dim not in (32, 64)):
+                    raise _NoPlan
+                if norm.eps != norm2_.eps:  # such a block runs module by module (GLABlock.forward_carry)
+                    if type(own["drop_path"]) not in (nn.Identity, DropPath):
+                        raise _NoPlan
+                    called += [norm, at, norm2_, own["drop_path"], mlp, mlp.gate_proj, mlp.down_proj]
+                layer, mlp_layer = at.__dict__["_modules"], mlp.__dict__["_modules"]
+                low, up = list(layer["gk_proj"].__dict__["_modules"].values())[:2]
+                w_qkv, w_low = _own(layer["qkv_proj"], nn.Linear)[0], _own(low, nn.Linear)[0]
+                w_g, b_g = _own(layer["g_proj"], nn.Linear)
                 n = [at.num_heads * (2 * at.head_qk_dim + at.head_v_dim), at.num_heads * at.head_v_dim, ops.GATE_RANK]
-                if n[1] != C or any(t.shape != (h, C) for t, h in zip(srcs, n)) or at.g_proj.bias is None:
-                    return None  # (make_plan looks at the other shapes)
+                if n[1] != C or b_g is None or w_qkv.shape != (n[0], C) or w_g.shape != (n[1], C) or w_low.shape != (n[2], C):
+                    raise _NoPlan  # (calls.make_plan looks at the other shapes)
                 pad = -sum(n) % 128
-                rows += [*srcs, zero[:pad * C].view(pad, C)]
-                biases += [zero[:n[0]], at.g_proj.bias, zero[:n[2] + pad]]
-                small += [blk.attn_norm.weight, conv.weight, conv.bias, at.g_norm.weight, at.l_norm.weight, blk.mlp_norm.weight]
-            dev = zero.device
+                if zero is None or zero.numel() < max(n[0], pad * C):
+                    zero = head_w.new_zeros(max(n[0], 128 * C))
+                rows += [w_qkv, w_g, w_low, zero[:pad * C].view(pad, C)]
+                biases += [zero[:n[0]], b_g, zero[:n[2] + pad]]
+                conv_w, conv_b = _own(next(iter(layer["in_proj"].__dict__["_modules"].values())), nn.Conv2d)
+                small += [_own(norm, RMSNorm)[0], conv_w, conv_b, _own(layer["g_norm"], RMSNorm)[0], _own(layer["l_norm"], RMSNorm)[0],
+                          _own(norm2_, RMSNorm)[0]]
+                parts.append((at, norm, norm2_, *_own(up, nn.Linear), _own(layer["o_proj"], nn.Linear)[0],
+                              _own(mlp_layer["gate_proj"], nn.Linear)[0], _own(mlp_layer["down_proj"], nn.Linear)[0]))
+            dev = head_w.device
             if any(t is not None and (t.device != dev or t.dtype is not torch.bfloat16) for t in small + rows + biases):
-                return None
+                raise _NoPlan
             flat = [t.reshape(-1) for t in small if t is not None]
-            parts = iter(torch.cat(flat).float().split([t.numel() for t in flat]))
-            f32 = [next(parts) if t is not None else None for t in small]
+            pieces = iter(torch.cat(flat).float().split([t.numel() for t in flat]))
+            f32 = [next(pieces) if t is not None else None for t in small]
             heights = [sum(t.shape[0] for t in rows[i:i + 4]) for i in range(0, len(rows), 4)]
             w_in, b_in = torch.cat(rows).split(heights), torch.cat(biases).split(heights)
             b1, ln1w, ln1b, b2, ln2w, ln2b, norm_w = f32[:7]
-            stem = (pe._packed_w1(), b1, ln1w, ln1b, norm1.eps,
-                    conv2.weight.detach().permute(0, 2, 3, 1), b2, ln2w, ln2b, norm2.eps,
+            stem = (pe._packed_w1(), b1, ln1w, ln1b, norm1.eps, w2.detach().permute(0, 2, 3, 1), b2, ln2w, ln2b, norm2.eps,
                     self.pos_embed.detach(), *conv1.kernel_size, *self.patch_resolution)
             blocks = []
-            for i, blk in enumerate(self.blocks):
-                at, mlp = blk.attn, blk.mlp
-                up = at.gk_proj[1]
+            for i, (at, norm, norm2_, w_up, b_up, w_o, w_gate, w_down) in enumerate(parts):
                 attn_norm, conv_w, conv_b, g_norm, l_norm, mlp_norm = f32[7 + 6 * i:13 + 6 * i]
-                blocks.append((attn_norm, blk.attn_norm.eps, conv_w, conv_b, flag(at.use_act_in_conv), w_in[i], b_in[i], at.num_heads,
-                               at.head_qk_dim, at.head_v_dim, up.weight.detach(), up.bias.detach(), float(at.gate_logit_normalizer),
-                               at.clamp_min, g_norm, l_norm, at.layernorm_eps, flag(at.use_out_act), at.o_proj.weight.detach(),
-                               mlp_norm, blk.mlp_norm.eps, mlp.gate_proj.weight.detach(), mlp.down_proj.weight.detach()))
-            tail = (norm_w, self.norm.eps, self.head.weight.detach(), self.head.bias.detach() if self.head.bias is not None else None)
+                blocks.append((attn_norm, norm.eps, conv_w, conv_b, flag(at.use_act_in_conv), w_in[i], b_in[i], at.num_heads,
+                               at.head_qk_dim, at.head_v_dim, w_up, b_up, float(at.gate_logit_normalizer), at.clamp_min, g_norm, l_norm,
+                               at.layernorm_eps, flag(at.use_out_act), w_o, mlp_norm, norm2_.eps, w_gate, w_down))
+            tail = (norm_w, kids["norm"].eps, head_w, head_b)
         return calls.make_plan(self, settings, absent, called, stem, blocks, tail)
 
 
