@@ -29,8 +29,44 @@ def test_forward(B, H, L, Dk, gate_scale):
         assert mine <= max(2 * serial, 3e-7)
 
 
+# what leaves the range of the common form, in one direction or both, and how: a whole tile's gates, one channel's, single tokens
+# (on both sides of every level's split), and what the form for any gates does not take either: gates that grow, no numbers
+@pytest.mark.parametrize("kind", ["one tile", "one channel", "tokens", "infinite", "reverse only", "growing", "growing a little"])
+@pytest.mark.parametrize("L,Dk", [(31, 64), (64, 32), (197, 64), (224, 32), (450, 64)])
+def test_forward_beyond_the_range(L, Dk, kind):
+    announce(f"fp32 forward, gates beyond the range: {kind}, L={L} Dk={Dk}")
+    q, k, v, gf, gb = make_gla_inputs(1, 3, L, Dk, 64, seed=300 + L, dtype=torch.float32)
+    if kind == "one tile":
+        gf[0, 1, L // 2:L // 2 + 20] -= 3.0
+    elif kind == "one channel":
+        gf[0, :, :, 5] -= 2.0
+        gb[0, :, :, Dk - 1] -= 5.0
+    elif kind == "tokens":
+        for t in (0, 1, 3, 7, 15, 16, 30):
+            gf[0, :, t::32] -= 9.0
+            gb[0, :, (31 - t)::32] -= 9.0
+    elif kind == "infinite":
+        gf[0, :, 3::5, 1::3] = -float("inf")
+        gb[0, :, 2::9] = -float("inf")
+    elif kind == "reverse only":
+        gb[0, 0] -= 1.5
+    else:
+        gf[0, 1] -= 1.5
+        gf[0, 1, 4:9, 3] = 0.5 if kind == "growing a little" else 2.0
+    for args in ((q, k, v, gf, gb), (q, k, v, gf, None)):
+        want = oracle_bidir(*args)
+        x = [a.cuda() if a is not None else None for a in args]
+        err = lambda o: np.linalg.norm(f64(o) - want) / np.linalg.norm(want)
+        mine, serial = err(vig_amd.gla_bidir_forward(*x)), err(vig_amd.gla_bidir_forward(*x, exact=True))
+        print(f"  relative error {mine:.2e}, token-recurrent {serial:.2e}", flush=True)
+        assert mine <= max(2 * serial, 3e-7)
+    gf[0, 2, 1, 2] = float("nan")
+    got = f64(vig_amd.gla_bidir_forward(q.cuda(), k.cuda(), v.cuda(), gf.cuda()))
+    assert np.isnan(got[0, 2, 1]).all() and np.isfinite(got[0, 0, :]).all()
+
+
 def test_forward_magnitudes_and_infinite_gates():
-    """Inputs beyond the tile form's magnitude bound, and gates of -inf, take the serial form."""
+    """Inputs beyond the tile form's magnitude bound take the serial form, gates of -inf the form for any gates."""
     announce("fp32 forward, large magnitudes and gates of -inf")
     q, k, v, gf, gb = make_gla_inputs(1, 2, 300, 64, 64, seed=5, dtype=torch.float32)
     q[0, 0, 3] *= 1e14

@@ -14,8 +14,11 @@
 //
 // Decays per tile as in gla_tiles.hip, in log2 units: G = inclusive cumulative gate in the direction's walk order, T the
 // tile's total, q^ = q 2^G for the walk, k^ = k 2^(T-G) published, q' = q 2^(G-T) against k^ for the wave's own tile (one
-// set of key pieces serves both).  Only q' grows, so the form holds while |G| <= 40 in every channel of every tile (a mean gate of -0.87 per token) and the inputs stay
-// below 1e12; a workgroup that meets anything else takes the serial form for its tokens (serial_segment).
+// set of key pieces serves both).  Only q' grows, so the form holds while |G| <= 40 in every channel of every tile (a mean
+// gate of -0.87 per token) and the inputs stay below 1e12.  A workgroup that meets stronger gates does its tokens again with
+// operands for any gates (prepare32_any); inputs beyond the bound, gates that grow and gates that are no numbers take the
+// serial form (serial_segment).  All sequences strongly gated: B 32, H 6, L 197, D 64 81 us (mildly gated 38; the
+// token-recurrent kernel 182, the serial form, one wave of a workgroup, 1069); 768 sequences 233 us (112 / 221 / 3214).
 #include "f32_tiles.h"
 
 namespace vig {
@@ -96,6 +99,75 @@ __device__ __forceinline__ bool prepare32(const f32x8_t (&q)[NG], const f32x8_t 
     P[c] = keep ? P[c] + Ps[c] : 0.f;
   }
   return wide;
+}
+
+// x where every bit of m is set, y where none is (one instruction; a choice by condition became branches here)
+__device__ __forceinline__ float pick(uint32_t m, float x, float y) {
+  return __uint_as_float((__float_as_uint(x) & m) | (__float_as_uint(y) & ~m));
+}
+
+// The same for any gates that do not grow (sums down to -inf): no factor is ever above one.  A pair of tokens (query i, key j)
+// differs first in some bit m of its numbers; the start of the upper half of their common 2m tokens lies between them, and
+// the decay splits there: the query's gates summed over its own m tokens up to it (inc), the key's over the rest of its m
+// tokens (exc), both plain sums of gates.  A token is a query or a key of a level, never both, so one operand holds both,
+// and a level is one product of it with itself of which the level's pairs are taken.  Five levels and the pair i = j (which
+// decays nothing) take the place of the one product above; the vector instructions of a level bound it: 700 of them beside
+// 24 matrix instructions at Dk = 64.
+template <int NG, bool FWD>
+__device__ __forceinline__ void prepare32_any(const f32x8_t (&q)[NG], const f32x8_t (&k)[NG], f32x8_t (&inc)[NG], float* dtab,
+                                              char* kreg, int lane, f32x8_t (&qh)[NG], f32x16_t& P) {
+  constexpr int HC = 8 * NG;
+  const int r = lane & 31, h = lane >> 5;
+  f32x8_t exc[NG];
+  float dot = 0.f;
+#pragma unroll
+  for (int c = 0; c < NG; ++c) {
+    inc[c] *= kLog2e;
+    exc[c] = f32x8_t{0.f};
+#pragma unroll
+    for (int e = 0; e < 8; ++e) dot = __builtin_fmaf(q[c][e], k[c][e], dot);
+  }
+  dot += __shfl_xor(dot, 32, 64);
+#pragma unroll
+  for (int c = 0; c < 16; ++c) P[c] = 8 * (c >> 2) + (c & 3) + 4 * h == r ? dot : 0.f;
+#pragma unroll 1
+  for (int m = 1; m < 32; m *= 2) {
+    const uint32_t query = ((r & m) != 0) == FWD ? ~0u : 0u;
+    // the lane that holds the whole sum of the other m tokens
+    const int other = 4 * (32 * h + (FWD ? (r ^ m) | (m - 1) : (r ^ m) & ~(m - 1)));
+    f32x16_t Pm = {0.f}, Ps = {0.f};
+#pragma unroll
+    for (int c = 0; c < NG; ++c) {
+      f32x8_t x;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        x[e] = pick(query, q[c][e], k[c][e]) * exp2_fast(pick(query, inc[c][e], exc[c][e]));
+        const float t = __uint_as_float(__builtin_amdgcn_ds_bpermute(other, __float_as_uint(inc[c][e])));
+        inc[c][e] += pick(query, t, 0.f);
+        exc[c][e] += pick(query, 0.f, t);
+      }
+      const P3 p = split8(x);
+      mfma6(p, p, Pm, Ps);
+    }
+#pragma unroll
+    for (int c = 0; c < 16; ++c) {
+      const int key = 8 * (c >> 2) + (c & 3) + 4 * h;
+      const bool mine = ((r ^ key) & -m) == m && (FWD ? r > key : key > r);
+      P[c] = mine ? Pm[c] + Ps[c] : P[c];
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < NG; ++c) {
+    f32x8_t kh;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float d = exp2_fast(inc[c][e]);
+      kh[e] = k[c][e] * exp2_fast(exc[c][e]);
+      qh[c][e] = q[c][e] * d;
+      if (r == (FWD ? 31 : 0)) dtab[HC * h + 8 * c + e] = d;
+    }
+    if (kreg) store_p3(kreg, c, lane, split8(kh));
+  }
 }
 
 // O^T += V^T P
@@ -205,6 +277,165 @@ __device__ __noinline__ void serial_segment(const float* q, const float* k, cons
   for (int t = 0; t < n; ++t) o[(size_t)t * 64 + lane] = oscale * obuf[t * 64 + lane];
 }
 
+// Where a workgroup's tokens and this wave's tile lie.
+template <int NG>
+struct F32Place {
+  const float *q, *k, *v, *gf, *gb, *slots;  // the segment's first token; states that enter it, or null
+  float* o;
+  int n, NT, ti;  // tokens left from the segment's start on, tiles, this wave's tile
+  rsrc_t rq, rk, rv, rgf, rgb, ro;  // its tile's rows
+};
+template <int NG, bool BIDIR>
+__device__ __forceinline__ F32Place<NG> f32_place(const float* q, const float* k, const float* v, const float* gf, const float* gb,
+                                                  float* o, const F32Geo& geo) {
+  constexpr int DK = 16 * NG;
+  F32Place<NG> p;
+  const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  // waves w and w + 4 share a SIMD: tiles NT-1-w and w together see NT + 3 - w - (NT-1-w) ... the same number of tiles
+  // in both directions
+  p.NT = geo.NT, p.ti = w < 4 ? p.NT - 1 - w : w - 4;
+  const int first = 32 * (int)blockIdx.y * p.NT;
+  const size_t at = (size_t)blockIdx.x * geo.L + first;
+  p.n = geo.L - first;
+  p.q = q + at * DK, p.k = k + at * DK, p.v = v + at * 64, p.gf = gf + at * DK, p.gb = (BIDIR ? gb : gf) + at * DK, p.o = o + at * 64;
+  p.slots = geo.states ? geo.states + ((size_t)blockIdx.x * geo.nseg + blockIdx.y) * 2 * kGlaStateFloats : nullptr;
+  const int nvalid = __builtin_amdgcn_readfirstlane(max(0, min(32, p.n - 32 * p.ti)));
+  const int tile = 32 * p.ti;
+  p.rq = chunk_rsrc(p.q + tile * DK, nvalid, 4 * DK), p.rk = chunk_rsrc(p.k + tile * DK, nvalid, 4 * DK);
+  p.rv = chunk_rsrc(p.v + tile * 64, nvalid, 256), p.ro = chunk_rsrc(p.o + tile * 64, nvalid, 256);
+  p.rgf = chunk_rsrc(p.gf + tile * DK, nvalid, 4 * DK), p.rgb = chunk_rsrc(p.gb + tile * DK, nvalid, 4 * DK);
+  return p;
+}
+
+enum F32Range { kInRange = 0, kGatesBeyond = 1, kValuesBeyond = 2 };
+
+// The walk of both directions; ANY: with prepare32_any, over the values' pieces that the pass before left in LDS.  Returns
+// (workgroup-uniform) what is beyond the form's range, before anything is stored.
+template <int NG, bool BIDIR, bool ANY>
+__device__ __forceinline__ int f32_pass(const F32Place<NG>& p, char* lds, float oscale) {
+  const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
+  const int NT = p.NT, ti = p.ti;
+  const F32Lds<NG> lay(NT);
+  char* vreg = lds + lay.v + ti * F32Lds<NG>::VB;
+  float* sc = reinterpret_cast<float*>(lds + lay.sc) + 64 * ti;
+  float* dall = reinterpret_cast<float*>(lds + lay.d);
+  int* flags = reinterpret_cast<int*>(lds + lay.flag);
+  const auto beyond = [&](int why) { return __builtin_amdgcn_ballot_w64(lane < NT && (flags[lane < NT ? lane : 0] & why)) != 0; };
+
+  f32x8_t xq[NG], xk[NG], xg[NG], qh[NG];
+  f32x16_t P, O[2] = {f32x16_t{0.f}, f32x16_t{0.f}};
+  char* kreg = ti < NT - 1 ? lds + ti * F32Lds<NG>::KB : nullptr;
+  if (ANY) {
+    lds_barrier();  // everyone has read the flags
+    float grows = 0.f, sum = 0.f;
+#pragma unroll
+    for (int dir = 0; dir < (BIDIR ? 2 : 1); ++dir) {
+      load_rows_f32<NG>(dir ? p.rgb : p.rgf, r, h, xg);
+#pragma unroll
+      for (int c = 0; c < NG; ++c)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) grows = fmaxf(grows, xg[c][e]), sum += xg[c][e];
+    }
+    // (a gate that grows: 32 tokens of the largest stay in the range; sums of -inf are fine, of no number are not)
+    const bool refused = __builtin_amdgcn_ballot_w64(!(grows * (32 * kLog2e) <= kRange32) || sum != sum) != 0;
+    if (lane == 0) flags[ti] = refused ? kGatesBeyond : kInRange;
+    lds_barrier();
+    if (beyond(kGatesBeyond)) return kGatesBeyond;
+    load_rows_f32<NG>(p.rgf, r, h, xg);
+    load_rows_f32<NG>(p.rq, r, h, xq);
+    load_rows_f32<NG>(p.rk, r, h, xk);
+    prepare32_any<NG, true>(xq, xk, xg, dall + 64 * ti, kreg, lane, qh, P);
+    apply_values32(P, vreg, lane, O);
+    lds_barrier();
+  } else {
+    float mag = 0.f;
+    {
+      f32x8_t xv[2][2];
+      load_pairs_f32(p.rv, r, h, xv);
+      load_rows_f32<NG>(p.rgf, r, h, xg);
+      load_rows_f32<NG>(p.rq, r, h, xq);
+      load_rows_f32<NG>(p.rk, r, h, xk);
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int pv = 0; pv < 2; ++pv) {
+          store_p3(vreg, 2 * t + pv, lane, split8(xv[pv][t]));
+          mag += sum_abs(xv[pv][t]);  // (a sum: NaN and inf stay visible)
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < NG; ++c) mag += sum_abs(xq[c]) + sum_abs(xk[c]);
+    const bool large = __builtin_amdgcn_ballot_w64(!(mag < kMagnitude32)) != 0;
+    const bool wide = prepare32<NG, true>(xq, xk, xg, sc, dall + 64 * ti, kreg, lane, qh, P);
+    wave_lds_sync();
+    apply_values32(P, vreg, lane, O);
+    if (lane == 0) flags[ti] = large ? kValuesBeyond : wide ? kGatesBeyond : kInRange;
+    lds_barrier();
+    if (beyond(kGatesBeyond | kValuesBeyond)) return beyond(kValuesBeyond) ? kValuesBeyond : kGatesBeyond;
+  }
+  walk32<NG, true>(lds, lay, ti, NT, lane, qh, O);
+  if (p.slots) apply_state32<NG, true>(p.slots, dall, ti > 0, lane, qh, O);
+  if (BIDIR) {
+    int r2 = r;
+    asm volatile("" : "+v"(r2));  // (fetched again: carried across the walk, q and k would take 64 registers)
+    load_rows_f32<NG>(p.rgb, r2, h, xg);
+    load_rows_f32<NG>(p.rq, r2, h, xq);
+    load_rows_f32<NG>(p.rk, r2, h, xk);
+    lds_barrier();  // the forward keys and decays have been read
+    kreg = ti > 0 ? lds + (ti - 1) * F32Lds<NG>::KB : nullptr;
+    if (ANY) {
+      prepare32_any<NG, false>(xq, xk, xg, dall + 64 * ti, kreg, lane, qh, P);
+      apply_values32(P, vreg, lane, O);
+      lds_barrier();
+    } else {
+      const bool wide = prepare32<NG, false>(xq, xk, xg, sc, dall + 64 * ti, kreg, lane, qh, P);
+      apply_values32(P, vreg, lane, O);
+      if (lane == 0) flags[ti] = wide ? kGatesBeyond : kInRange;
+      lds_barrier();
+      if (beyond(kGatesBeyond)) return kGatesBeyond;
+    }
+    walk32<NG, false>(lds, lay, ti, NT, lane, qh, O);
+    if (p.slots) apply_state32<NG, false>(p.slots + kGlaStateFloats, dall + 64 * (NT - 1), ti < NT - 1, lane, qh, O);
+  }
+  // lane (r, h) holds channels [32h, 32h + 32) of token r: register 4g + m of O[pv] is channel 32h + 8g + 2m + pv
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    u32x4_t x;
+#pragma unroll
+    for (int m = 0; m < 4; ++m) x[m] = __float_as_uint(O[m & 1][2 * i + (m >> 1)] * oscale);
+    __builtin_amdgcn_raw_buffer_store_b128(x, p.ro, (unsigned)r * 256u + 128u * h + 16u * i, 0, 0);
+  }
+  return kInRange;
+}
+
+// The kernel's argument block as the hardware lays it out (every argument at its natural alignment).
+struct F32KernArgs {
+  const float *q, *k, *v, *gf, *gb;
+  float* o;
+  F32Geo geo;
+  float oscale;
+};
+static_assert(offsetof(F32KernArgs, geo) == 6 * sizeof(void*) && offsetof(F32KernArgs, oscale) == 48 + sizeof(F32Geo) && alignof(F32Geo) == 8,
+              "F32KernArgs has to mirror the parameter list of gla_f32_kernel");
+
+// What is beyond the range, as a function of its own: its registers stay out of the common path's allocation.  (Arguments of a
+// called function come in vector registers, and a descriptor built from one puts a loop around every load: the function
+// reads the kernel's own through the argument block.)
+template <int NG, bool BIDIR>
+__device__ __noinline__ void f32_beyond(const F32KernArgs* ka_in, int why) {
+#if defined(__HIP_DEVICE_COMPILE__)  // (the host pass has no constant address space to copy the geometry from)
+  extern __shared__ __align__(16) char lds[];
+  const uint64_t kp = reinterpret_cast<uint64_t>(ka_in);
+  typedef const F32KernArgs __attribute__((address_space(4))) * KernArgPtr;
+  const KernArgPtr ka = (KernArgPtr)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(kp >> 32)) << 32) |
+                                     (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)kp));
+  const F32Geo geo = ka->geo;
+  const auto p = f32_place<NG, BIDIR>(ka->q, ka->k, ka->v, ka->gf, ka->gb, ka->o, geo);
+  if (__builtin_amdgcn_readfirstlane(why) == kGatesBeyond && f32_pass<NG, BIDIR, true>(p, lds, ka->oscale) == kInRange) return;
+  serial_segment<NG, BIDIR>(p.q, p.k, p.v, p.gf, p.gb, p.o, p.slots, min(32 * p.NT, p.n), p.NT * 8192, ka->oscale);
+#endif
+}
+
 }  // namespace
 
 template <int NG, bool BIDIR>
@@ -213,87 +444,8 @@ __global__ __launch_bounds__(512, 2) void gla_f32_kernel(const float* __restrict
                                                          const float* __restrict__ gb, float* __restrict__ o, F32Geo geo,
                                                          float oscale) {
   extern __shared__ __align__(16) char lds[];
-  constexpr int DK = 16 * NG;
-  const int NT = geo.NT, lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
-  const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  // waves w and w + 4 share a SIMD: tiles NT-1-w and w together see NT + 3 - w - (NT-1-w) ... the same number of tiles
-  // in both directions
-  const int ti = w < 4 ? NT - 1 - w : w - 4;
-  const F32Lds<NG> lay(NT);
-  const int first = 32 * (int)blockIdx.y * NT, tok = first + 32 * ti;
-  const int nvalid = __builtin_amdgcn_readfirstlane(max(0, min(32, geo.L - tok)));
-  const size_t seq0 = (size_t)blockIdx.x * geo.L, off = seq0 + tok;
-  const rsrc_t rq = chunk_rsrc(q + off * DK, nvalid, 4 * DK), rk = chunk_rsrc(k + off * DK, nvalid, 4 * DK);
-  const rsrc_t rv = chunk_rsrc(v + off * 64, nvalid, 256), ro = chunk_rsrc(o + off * 64, nvalid, 256);
-  const float* slots = geo.states ? geo.states + ((size_t)blockIdx.x * geo.nseg + blockIdx.y) * 2 * kGlaStateFloats : nullptr;
-  char* vreg = lds + lay.v + ti * F32Lds<NG>::VB;
-  float* sc = reinterpret_cast<float*>(lds + lay.sc) + 64 * ti;
-  float* dall = reinterpret_cast<float*>(lds + lay.d);
-  int* flags = reinterpret_cast<int*>(lds + lay.flag);
-
-  f32x8_t xq[NG], xk[NG], xg[NG], qh[NG];
-  f32x16_t P, O[2] = {f32x16_t{0.f}, f32x16_t{0.f}};
-  float mag = 0.f;
-  {
-    f32x8_t xv[2][2];
-    load_pairs_f32(rv, r, h, xv);
-    load_rows_f32<NG>(chunk_rsrc(gf + off * DK, nvalid, 4 * DK), r, h, xg);
-    load_rows_f32<NG>(rq, r, h, xq);
-    load_rows_f32<NG>(rk, r, h, xk);
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int pv = 0; pv < 2; ++pv) {
-        store_p3(vreg, 2 * t + pv, lane, split8(xv[pv][t]));
-        mag += sum_abs(xv[pv][t]);  // (a sum: NaN and inf stay visible)
-      }
-  }
-#pragma unroll
-  for (int c = 0; c < NG; ++c) mag += sum_abs(xq[c]) + sum_abs(xk[c]);
-  bool wide = __builtin_amdgcn_ballot_w64(!(mag < kMagnitude32)) != 0;
-  wide |= prepare32<NG, true>(xq, xk, xg, sc, dall + 64 * ti, ti < NT - 1 ? lds + ti * F32Lds<NG>::KB : nullptr, lane, qh, P);
-  wave_lds_sync();
-  apply_values32(P, vreg, lane, O);
-  if (lane == 0) flags[ti] = wide;
-  lds_barrier();
-  const auto refused = [&] { return __builtin_amdgcn_ballot_w64(lane < NT && flags[lane < NT ? lane : 0] != 0) != 0; };
-  const auto serial = [&] {
-    serial_segment<NG, BIDIR>(q + (seq0 + first) * DK, k + (seq0 + first) * DK, v + (seq0 + first) * 64,
-                              gf + (seq0 + first) * DK, BIDIR ? gb + (seq0 + first) * DK : nullptr, o + (seq0 + first) * 64,
-                              slots, min(32 * NT, geo.L - first), NT * 8192, oscale);
-  };
-  if (refused()) {
-    serial();
-    return;
-  }
-  walk32<NG, true>(lds, lay, ti, NT, lane, qh, O);
-  if (slots) apply_state32<NG, true>(slots, dall, ti > 0, lane, qh, O);
-  if (BIDIR) {
-    int r2 = r;
-    asm volatile("" : "+v"(r2));  // (fetched again: carried across the walk, q and k would take 64 registers)
-    load_rows_f32<NG>(chunk_rsrc(gb + off * DK, nvalid, 4 * DK), r2, h, xg);
-    load_rows_f32<NG>(rq, r2, h, xq);
-    load_rows_f32<NG>(rk, r2, h, xk);
-    lds_barrier();  // the forward keys and decays have been read
-    wide = prepare32<NG, false>(xq, xk, xg, sc, dall + 64 * ti, ti > 0 ? lds + (ti - 1) * F32Lds<NG>::KB : nullptr, lane, qh, P);
-    apply_values32(P, vreg, lane, O);
-    if (lane == 0) flags[ti] = wide;
-    lds_barrier();
-    if (refused()) {
-      serial();
-      return;
-    }
-    walk32<NG, false>(lds, lay, ti, NT, lane, qh, O);
-    if (slots) apply_state32<NG, false>(slots + kGlaStateFloats, dall + 64 * (NT - 1), ti < NT - 1, lane, qh, O);
-  }
-  // lane (r, h) holds channels [32h, 32h + 32) of token r: register 4g + m of O[pv] is channel 32h + 8g + 2m + pv
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    u32x4_t x;
-#pragma unroll
-    for (int m = 0; m < 4; ++m) x[m] = __float_as_uint(O[m & 1][2 * i + (m >> 1)] * oscale);
-    __builtin_amdgcn_raw_buffer_store_b128(x, ro, (unsigned)r * 256u + 128u * h + 16u * i, 0, 0);
-  }
+  const int why = f32_pass<NG, BIDIR, false>(f32_place<NG, BIDIR>(q, k, v, gf, gb, o, geo), lds, oscale);
+  if (why != kInRange) f32_beyond<NG, BIDIR>((const F32KernArgs*)__builtin_amdgcn_kernarg_segment_ptr(), why);
 }
 
 // State pass of a long sequence: what every segment adds to the state of each direction, U = sum_t 2^(gates walked after
@@ -409,7 +561,7 @@ __global__ __launch_bounds__(256, 2) void gla_f32_state_kernel(const float* __re
   }
 }
 
-// Measured at B 32, H 6, L 197, D 64 (58 MB): 36.5 us per call, token-recurrent kernel 181 us.
+// Measured at B 32, H 6, L 197, D 64 (58 MB): 38 us per call, token-recurrent kernel 181 us.
 constexpr int kF32MaxLds = 160 * 1024;
 
 bool gla_f32_supported(const GlaArgs& a) {

@@ -71,7 +71,7 @@ def invalidate_caches(model: nn.Module) -> None:
     counter they are keyed on, so code that writes that way calls this afterwards.  load_state_dict and train() /
     eval() switches of these modules call it by themselves."""
     modules = list(model.modules())
-    for owner, plan in list(_PLANS.items()) if len(_PLANS) else ():  # (a plan goes when any module that it describes is named here, and stays otherwise)
+    for owner, plan in list(_PLANS.items()) if len(_PLANS) else ():  # (a plan goes when a module that it describes is touched)
         if owner is model or _ext.calls().plan_describes(plan, modules):
             _PLANS.pop(owner, None)
     for m in modules:
