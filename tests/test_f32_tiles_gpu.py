@@ -79,7 +79,8 @@ def test_forward_magnitudes_and_infinite_gates():
 
 @pytest.mark.parametrize("gate_scale", [1 / 16, 1.0])  # in range; beyond it (flagged for the recurrent kernel)
 @pytest.mark.parametrize("B,H,L,Dk", [(1, 1, 2, 64), (2, 2, 33, 32), (2, 3, 196, 32), (1, 2, 224, 64), (1, 2, 225, 64),
-                                      (1, 2, 256, 32), (1, 2, 449, 64), (1, 1, 700, 32)])
+                                      (1, 2, 256, 32), (1, 2, 449, 64), (1, 1, 700, 32),
+                                      (1, 769, 5, 64), (1, 768, 16, 64), (2, 1, 17, 64)])
 def test_backward(B, H, L, Dk, gate_scale):
     announce(f"fp32 backward on the matrix cores B{B} H{H} L={L} Dk={Dk} gates x {gate_scale}")
     t = make_gla_inputs(B, H, L, Dk, 64, seed=950 + L, dtype=torch.float32, gate_scale=gate_scale)

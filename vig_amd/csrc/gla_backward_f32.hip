@@ -647,8 +647,12 @@ __global__ __launch_bounds__(512, 2) void gla_backward_f32_kernel(
 constexpr int kBwdF32MaxLds = 160 * 1024;
 
 // Segments of up to seven tiles, as in the forward (eight would not fit beside 64 key channels).  A causal call of 225 to
-// 256 tokens has no room for two segments' states in the workspace its size promises: the recurrent kernel keeps it.
+// 256 tokens has no room for two segments' states in the workspace its size promises: the recurrent kernel keeps it.  It also
+// keeps sequences of one of its token blocks at 64 key channels while they fill the chip no more than three times over (tile
+// form / recurrent kernel, us: 6 sequences of 8 tokens 37.9 / 27.0, of 16 38.9 / 32.0, of 17 38.9 / 54.3; 768 of 16
+// 57.4 / 50.4, of 17 58.4 / 83.7; 1536 of 8 67 / 77, of 16 77 / 99; one direction alike; 32 channels 23 / 26 at least).
 bool gla_backward_f32_supported(int B, int H, int L, int Dk, int Dv, int io_dtype, int gate_dtype, bool bidir) {
+  if (Dk == 64 && L <= 16 && (long long)B * H <= 768) return false;
   return io_dtype == 0 && gate_dtype == 0 && (Dk == 64 || Dk == 32) && Dv == 64 && gla_f32_segments(L) <= 65535 &&
          (gla_f32_segments(L) == 1 || (long long)B * H * 4 <= 65535) && (bidir || L <= 224 || L > 256);
 }
