@@ -21,8 +21,9 @@ def _check(got, want64, ulps=1.0):
     assert ((got - want64).abs() <= ulps * 2.0 ** -8 * want64.abs() + 1e-5 * want64.abs().max()).all()
 
 
-# the first size of the rule; ragged token tiles; one, some and all of a workgroup's channel tiles, both contractions
-@pytest.mark.parametrize("rows,N,K", [(16384, 64, 192), (16385, 320, 384), (20011, 704, 192), (16415, 1280, 384)])
+# the first sizes of the rule; ragged token tiles; one, some and all of a workgroup's channel tiles, both contractions
+@pytest.mark.parametrize("rows,N,K", [(16384, 64, 192), (16385, 320, 384), (20011, 704, 192), (16415, 1280, 384),
+                                      (8192, 512, 192), (8209, 768, 192), (10752, 1536, 384), (10783, 2112, 384)])
 def test_linear_in_registers(rows, N, K):
     announce(f"linear in registers rows{rows} N{N} K{K}")
     x, w, b = _randn((rows, K), 1), _randn((N, K), 2, K ** -0.5), _randn((N,), 3)

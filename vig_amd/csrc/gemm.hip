@@ -433,11 +433,21 @@ static long long tiles_of(const GemmArgs& a, int tm, int tn) { return (long long
 //   up to 640 tiles of 32 x 32: gemm_few_kernel  (M 196: N 192 K 512 3.1 us against 17.2, N 1280 K 384 3.5 / 5.2,
 //                               N 768 K 2048 4.7 / 6.9; past the line its operand traffic grows with the tile count)
 //   up to 2 GFLOP:              64 x 64 tiles    (M 1568 N 1280 K 384 6.5 / 6.9; M 6272 N 640 K 192 7.1 / 7.3)
-//   K 384 or 192, N % 64 == 0, 16384 rows: weights in registers (linear.hip; its table is beside launch_linear_regs)
+//   K 384 or 192, N % 64 == 0, 16384 rows and fewer for some N (regs_rows): weights in registers (linear.hip)
 //   K <= 256 with 512 tiles:    256 x 128 tiles  (M 65536 N 520 K 192: other column counts)
 // Beyond that the library's products win (M 50176 N 1280 K 512 and longer contractions).
 constexpr int kFewTiles = 640;
-static bool regs_preferred(long long M, int N, int K) { return M >= 16384 && linear_regs_supported(K, N); }
+// Rows from which the form with its weights in registers is the better one; the table for 16384 rows and up is beside
+// launch_linear_regs.  Below, the library's time goes up and down with its choice of tiles, by up to two between neighbouring
+// sizes (us, library / registers): K 192, N 640: 8192 rows 10.9 / 8.3, 9408 9.2 / 9.3, 14112 18.2 / 11.5; N 704 15.5 / 9.2 at 9408;
+// N 512 and 768 2 % apart at worst; N 1024 13.5 / 14.1 at 12544.  K 384, N 2048: 8192 rows 19.3 / 20.5, 9216 29 / 23, 12544 43 / 28;
+// N 1536: 10192 18.9 / 20.0, 10976 38 / 22, 14112 34 / 25; but N 1280: 12544 19.0 / 21.1, N 384 10.9 / 12.0.  The lines
+// lie where no measured size loses more than 2 %.
+static long long regs_rows(int N, int K) {
+  if (K == 192) return N >= 512 && N <= 768 ? 8192 : 16384;
+  return N >= 1536 ? 10752 : 16384;
+}
+static bool regs_preferred(long long M, int N, int K) { return linear_regs_supported(K, N) && M >= regs_rows(N, K); }
 static bool short_k_many(const GemmArgs& a) { return a.K <= 256 && tiles_of(a, 256, 128) >= 512; }
 
 bool linear_preferred(long long M, int N, int K) {

@@ -640,7 +640,7 @@ bool linear_regs_supported(int K, int N) { return (K == 384 || K == 192) && N % 
 
 // Against the library's products (us, library / this): K 384: 16384 rows and up; 25088 rows N 1280 33 / 31, N 2048 61 / 45, N 384
 // 26 / 18, N 1024 42 / 26; 50176 rows 66 / 53, 130 / 77, 42 / 25, 58 / 42.  K 192: 32768 rows N 640 26 / 18, 50176 32 / 23,
-// 100352 58 / 40.  With 12544 rows it depends on the tiles (N 1280 19.6 / 21, N 2048 44 / 27).  Bound by its stores.
+// 100352 58 / 40.  Fewer rows: regs_rows (gemm.hip).  Bound by its stores.
 int launch_linear_regs(const void* x, const void* w, const void* bias, void* y, long long T, int N, int K, hipStream_t stream) {
   if (!linear_regs_supported(K, N) || T <= 0 || T > 0x7fffffffLL - 64) return -95;
   const int num_cu = cu_count();
