@@ -13,7 +13,7 @@
 //   - weight and bias gradients leave vig_linear_bwd_weight as fp32, one launch for the three stacked layers;
 //   - the up-projection of the gates and its input gradient run inside the gate kernels (bf16), and the depthwise
 //     convolution's three gradients are one kernel.
-// ViG-S, B 128 at 224 px under bf16 autocast, forward and backward on one MI355X: 23.9 -> 13.7 ms.
+// ViG-S, B 128 at 224 px under bf16 autocast, forward and backward on one MI355X: 23.7 -> 12.1 ms.
 #include <ATen/autocast_mode.h>
 
 #include "host_calls.h"
@@ -244,6 +244,8 @@ struct MixNode : torch::autograd::Function<MixNode> {
     check_rc(run_forward(q, k, v, gates, Tensor(), true, kDefault, c, o), "vig_gla_bidir_fwd");
     Tensor blend = at::empty_like(xs);
     Tensor a;
+    // At any number of tokens (us, fused / blend and product): C 192: 49 4.8 / 10.7, 1568 5.3 / 12.4, 25088 16 / 29; C 384: 49 7.7 / 11.2,
+    // 1568 8.8 / 16.4, 25088 26 / 37; a single token 7.0 / 4.8.
     if (m.bf16 && m.Dv == 64 && m.V == m.C && (m.C == 384 || m.C == 192) && aligned(w_out)) {
       a = at::empty({m.B, m.L, m.C}, opts);
       check_rc(vig_locality_blend_linear_kept_fwd(o.data_ptr(), xs.data_ptr(), at_elem(z, m.n0), f32(g_norm, 2), f32(l_norm, 3),
@@ -390,6 +392,8 @@ struct MlpNode : torch::autograd::Function<MlpNode> {
     const Tensor wg = same ? gate_w : matrix(packed, gate_off, 2 * I, C), wd = same ? down_w : matrix(packed, down_off, C, I);
     auto [y, sum] = norm_fwd(branch, residual, wide ? fptr(norm_w) : fptr(small), eps, type);
     Tensor z, prod = at::empty({rows, I}, y.options());
+    // At any number of tokens (us, fused / product and SwiGLU pass): C 192: 1 4.0 / 4.1, 196 4.4 / 4.6, 1568 5.2 / 7.4, 25088 27 / 36; C 384:
+    // 49 5.3 / 4.8 (and a launch more), 196 5.6 / 5.7, 1568 10.6 / 12.7, 12544 37 / 66, 25088 66 / 71.
     if (type == at::kBFloat16 && (C == 384 || C == 192) && I % 32 == 0 && aligned(y) && aligned(wg)) {
       z = at::empty({rows, 2 * I}, y.options());
       check_rc(vig_linear_swiglu_kept_fwd(y.data_ptr(), wg.data_ptr(), z.data_ptr(), prod.data_ptr(), rows, (int)C, (int)I, VIG_BF16,
@@ -423,6 +427,8 @@ struct MlpNode : torch::autograd::Function<MlpNode> {
     const Tensor d_out = grad_rows(grads[0], rows, C, y, type);
     if (ctx->needs_input_grad(4)) out[4] = like_param(weight_grad(d_out, prod, nullptr), down_w, {C, I});
     Tensor dz = at::empty_like(z);
+    // At any number of tokens (us, fused / input gradient and SwiGLU pass): C 192: 1 3.5 / 6.6, 1568 5.0 / 9.2, 25088 28 / 41; C 384: 1 3.9 / 5.8,
+    // 1568 8.5 / 13.7, 25088 53 / 72.
     if (type == at::kBFloat16 && d_out.scalar_type() == type && (C == 384 || C == 192) && I % 32 == 0 && d_out.is_contiguous() && aligned(d_out) && aligned(wd)) {
       check_rc(vig_linear_swiglu_bwd(d_out.data_ptr(), wd.data_ptr(), z.data_ptr(), dz.data_ptr(), rows, (int)C, (int)I, VIG_BF16,
                                      stream_of(z)),
