@@ -198,6 +198,29 @@ def test_plans_of_other_models_stay(monkeypatch):
     assert torch.equal(b(x), _modules(monkeypatch, b, x))
 
 
+@pytest.mark.parametrize("change", ["features", "no bias", "odd stem", "two gate layers more"])
+def test_models_of_another_tree(change, monkeypatch):
+    """What no plan describes runs through the modules: a classifier taken off, layers added, another stem."""
+    announce(f"a model of another tree: {change}")
+    m, x = _tiny()
+    m(x)
+    if change == "features":
+        m.head = torch.nn.Identity()
+    elif change == "no bias":
+        m.head = torch.nn.Linear(192, 16, bias=False).cuda().bfloat16()
+    elif change == "odd stem":
+        m.patch_embed.proj[0] = torch.nn.Conv2d(3, 96, (9, 12), 8, 1).cuda().bfloat16()
+        x = torch.randn(1, 3, 256, 256, device="cuda").bfloat16()
+        m.patch_resolution = (16, 16)
+        m.pos_embed = torch.nn.Parameter(torch.randn(1, 256, 192, device="cuda").bfloat16())
+    else:
+        for _ in range(2):
+            m.blocks[0].attn.gk_proj.append(torch.nn.Identity())
+    got = m(x)
+    assert torch.equal(got, _modules(monkeypatch, m, x))
+    assert got.shape[1] == (192 if change == "features" else 16)
+
+
 class _Products(torch.utils._python_dispatch.TorchDispatchMode):
     """Counts the matrix products of the operators that it sees."""
 
