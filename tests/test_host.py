@@ -110,6 +110,9 @@ def test_checkpoint_variants_and_cache_invalidation(tmp_path):
     m.train()
     assert "_w32_cache" not in norm.__dict__
     norm._w32()
+    m.to(torch.float64).to(torch.bfloat16)  # (a move)
+    assert "_w32_cache" not in norm.__dict__
+    norm._w32()
     norm.weight.data.mul_(2.0)  # behind the version counter: the stale copy would survive ...
     assert torch.equal(norm._w32(), norm.weight.detach().float() / 2)
     layers.invalidate_caches(m)  # ... until the caller says so

@@ -198,6 +198,23 @@ def test_plans_of_other_models_stay(monkeypatch):
     assert torch.equal(b(x), _modules(monkeypatch, b, x))
 
 
+def test_models_that_are_moved_give_back_what_they_held():
+    announce("a moved model's memory")
+    import gc
+
+    m, x = _tiny()
+    y = m(x)
+    gc.collect()
+    held = [t.untyped_storage().nbytes() for t in m.parameters()]
+    before = torch.cuda.memory_allocated()
+    m.cpu()
+    gc.collect()
+    freed = before - torch.cuda.memory_allocated()
+    assert m not in layers._PLANS and freed >= sum(held)
+    m.cuda()
+    assert torch.equal(m(x), y)
+
+
 @pytest.mark.parametrize("change", ["features", "no bias", "odd stem", "two gate layers more"])
 def test_models_of_another_tree(change, monkeypatch):
     """What no plan describes runs through the modules: a classifier taken off, layers added, another stem."""

@@ -69,7 +69,7 @@ def invalidate_caches(model: nn.Module) -> None:
     refreshed by themselves when a parameter is replaced, moved, cast or written through torch's in-place operations;
     a write through `.data` (p.data.mul_(..), module.weight.data[...] = ..) changes neither the pointer nor the version
     counter they are keyed on, so code that writes that way calls this afterwards.  load_state_dict and train() /
-    eval() switches of these modules call it by themselves."""
+    eval() switches and moves of these modules call it by themselves."""
     modules = list(model.modules())
     for owner, plan in list(_PLANS.items()) if len(_PLANS) else ():  # (a plan goes when a module that it describes is touched)
         if owner is model or _ext.calls().plan_describes(plan, modules):
@@ -82,12 +82,17 @@ def invalidate_caches(model: nn.Module) -> None:
 
 
 class _CacheMixin:
-    """For the modules that keep derived weight copies: the copies do not outlive a state-dict load or a switch
-    between training and evaluation (the usual places where weights change behind the version counter)."""
+    """For the modules that keep derived weight copies: the copies do not outlive a state-dict load, a switch between
+    training and evaluation (the usual places where weights change behind the version counter) or a move to another device
+    or type (they hold the storages they were made from)."""
 
     def train(self, mode: bool = True):
         invalidate_caches(self)
         return super().train(mode)
+
+    def _apply(self, *args, **kwargs):
+        invalidate_caches(self)
+        return super()._apply(*args, **kwargs)
 
     def _load_from_state_dict(self, *args, **kwargs):
         invalidate_caches(self)
@@ -720,7 +725,7 @@ class ViG(nn.Module):
     def _make_plan(self, calls):
         try:
             return self._describe(calls)
-        except _NoPlan:
+        except (_NoPlan, LookupError, AttributeError, TypeError, ValueError):  # (another tree than a ViG's: its modules know better)
             return None
 
     def _describe(self, calls):
