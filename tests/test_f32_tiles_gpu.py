@@ -97,3 +97,23 @@ def test_backward(B, H, L, Dk, gate_scale):
             err = lambda y: np.linalg.norm(f64(y) - w) / np.linalg.norm(w)
             assert err(a) <= max(2 * err(b), 4e-7), (name, err(a), err(b))
 
+
+# some sequences flagged for the recurrent kernel, whose two directions then run side by side, among others that are not
+@pytest.mark.parametrize("B,H,L,Dk", [(2, 3, 17, 32), (3, 7, 197, 64), (1, 5, 450, 32)])
+def test_backward_of_some_sequences_beyond_the_range(B, H, L, Dk):
+    announce(f"fp32 backward, every third sequence beyond the range, B{B} H{H} L={L} Dk={Dk}")
+    t = make_gla_inputs(B, H, L, Dk, 64, seed=970 + L, dtype=torch.float32)
+    for g in t[3:]:
+        g.view(B * H, L, Dk)[::3] -= 2.5
+    d_o = torch.randn(t[2].shape, generator=torch.Generator().manual_seed(5))
+    want = O.bidir_gla_backward(*(f64(a) for a in t), f64(d_o), out_scale=0.5)
+    x = [a.cuda() for a in (*t, d_o)]
+    mine = vig_amd.gla_bidir_backward(*x, out_scale=0.5)
+    serial = vig_amd.gla_bidir_backward(*x, out_scale=0.5, exact=True)
+    for name, a, b, w in zip(("dq", "dk", "dv", "dg_fwd", "dg_bwd"), mine, serial, want):
+        flat = w.reshape(B * H, -1)
+        err = lambda y: np.linalg.norm(f64(y).reshape(B * H, -1) - flat, axis=1) / np.linalg.norm(flat, axis=1)
+        assert (err(a) <= np.maximum(2 * err(b), 4e-7)).all(), (name, err(a), err(b))
+        assert torch.equal(a.view(B * H, L, -1)[::3], b.view(B * H, L, -1)[::3]), name  # (the same sums, whichever direction ends first)
+    for _ in range(5):
+        assert all(torch.equal(a, b) for a, b in zip(mine, vig_amd.gla_bidir_backward(*x, out_scale=0.5)))

@@ -29,17 +29,26 @@ struct GlaBwdArgs {
   float scale, out_scale;
   int io_dtype, gate_dtype;
   hipStream_t stream;
-  const int* only_flagged;  // null: every slab; else one int per (batch, head): slabs with 0 are skipped
+  int* only_flagged;  // null: every slab; else one int per (batch, head): slabs with 0 are skipped
+  bool split;         // the two directions in workgroups of their own (fp32 tensors, flagged slabs)
 };
+
+// Stores and loads of what the two workgroups of a split slab hand each other: through to memory, past the L2 of their own chiplet
+// (plain ones with fences around them write all of it back at each: 768 slabs of 196 tokens 1025 us instead of 716).
+__device__ __forceinline__ void store_shared(float* p, float x, bool shared) {
+  if (shared) __hip_atomic_store(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  else *p = x;
+}
+__device__ __forceinline__ float load_shared(const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
 template <typename TIO, typename TG, int DK, int DV, int TB>
 __global__ __launch_bounds__(256) void gla_backward_kernel(
     const TIO* __restrict__ q, const TIO* __restrict__ k, const TIO* __restrict__ v, const TG* __restrict__ gf,
     const TG* __restrict__ gb, const TIO* __restrict__ d_o, TIO* dq, TIO* dk, TIO* dv, TG* dgf, TG* dgb,
-    float* ws_dq, float* ws_acc_k, float* ws_acc_v, int L, float scale, float out_scale,
-    const int* __restrict__ only_flagged) {
+    float* ws_dq, float* ws_acc_k, float* ws_acc_v, int L, float scale, float out_scale, int* only_flagged, int split) {
   // second pass behind the matrix-core kernel: only the slabs it left out (uniform per workgroup, before any barrier)
   if (only_flagged && only_flagged[blockIdx.x] == 0) return;
+  constexpr bool kSplit = sizeof(TIO) == 4;
   constexpr int DKG = DK / 4;  // rows per wave, layout A
   constexpr int DVG = DV / 4;  // columns per wave, layout B
   __shared__ __align__(16) float sq[TB][DK];   // scale * q
@@ -88,7 +97,7 @@ __global__ __launch_bounds__(256) void gla_backward_kernel(
     }
   };
 
-  for (int dir = 0; dir < ndir; ++dir) {
+  for (int dir = split ? (int)blockIdx.y : 0; dir < (split ? (int)blockIdx.y + 1 : ndir); ++dir) {
     const TG* g = dir ? gb : gf;
     TG* dg = dir ? dgb : dgf;
     const bool rev = dir == 1;              // the direction walks tokens L-1 .. 0
@@ -123,7 +132,8 @@ __global__ __launch_bounds__(256) void gla_backward_kernel(
         for (int idx = tid; idx < TB * DK; idx += 256) {
           const int t = idx / DK, d = idx % DK;
           const int tok = t0 + t;
-          if (tok < L) my_dq[(size_t)tok * DK + d] = scale * ((pk[0][t][d] + pk[1][t][d]) + (pk[2][t][d] + pk[3][t][d]));
+          if (tok < L)
+            store_shared(my_dq + (size_t)tok * DK + d, scale * ((pk[0][t][d] + pk[1][t][d]) + (pk[2][t][d] + pk[3][t][d])), split);
         }
         __syncthreads();
       }
@@ -179,8 +189,12 @@ __global__ __launch_bounds__(256) void gla_backward_kernel(
             float s = (pv[0][t][c] + pv[1][t][c]) + (pv[2][t][c] + pv[3][t][c]);
             const size_t off = vo_base + (size_t)tok * DV + c;
             if (ndir == 2 && !last_dir) {
-              ws_acc_v[off] = s;
+              store_shared(ws_acc_v + off, s, split);
             } else {
+              if (split) {
+                if constexpr (kSplit) store_shared(dv + off, s, true);
+                continue;
+              }
               if (ndir == 2) s += ws_acc_v[off];
               Elem<TIO>::store(dv + off, s);
             }
@@ -199,8 +213,12 @@ __global__ __launch_bounds__(256) void gla_backward_kernel(
             // 384 sequences of 32 key channels 493 -> 426 us, 768 of 64 745 -> 678)
             pk[0][t][d] = Elem<TIO>::load(q + off) * sq_ - sk[t][d] * s;
             if (ndir == 2 && !last_dir) {
-              ws_acc_k[off] = s;
+              store_shared(ws_acc_k + off, s, split);
             } else {
+              if (split) {
+                if constexpr (kSplit) store_shared(dk + off, s, true);
+                continue;
+              }
               if (ndir == 2) {
                 s += ws_acc_k[off];
                 sq_ += ws_dq[bh * (size_t)L * DK + (size_t)tok * DK + d];  // the first direction's dq
@@ -227,6 +245,23 @@ __global__ __launch_bounds__(256) void gla_backward_kernel(
       }
     }
   }
+  if constexpr (kSplit) {
+    if (!split) return;
+    // whichever direction ends second adds the two up (the slab's flag, 1 so far, counts)
+    __shared__ int ended;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's stores have arrived
+    __syncthreads();
+    if (tid == 0) ended = atomicAdd(only_flagged + bh, 1);
+    __syncthreads();
+    if (ended != 2) return;
+    const float* dq0 = ws_dq + bh * (size_t)L * DK;
+    const float* dq1 = dq0 + gridDim.x * (size_t)L * DK;
+    for (size_t i = tid; i < (size_t)L * DK; i += 256) {
+      dk[qk_base + i] = load_shared(dk + qk_base + i) + load_shared(ws_acc_k + qk_base + i);
+      dq[qk_base + i] = load_shared(dq1 + i) + load_shared(dq0 + i);
+    }
+    for (size_t i = tid; i < (size_t)L * DV; i += 256) dv[vo_base + i] = load_shared(dv + vo_base + i) + load_shared(ws_acc_v + vo_base + i);
+  }
 }
 
 template <typename TIO, typename TG, int DK, int DV>
@@ -239,10 +274,10 @@ static int launch_bwd_t(const GlaBwdArgs& a) {
   float* ws_acc_k = ws + (size_t)ndir * n_qk;
   float* ws_acc_v = ws_acc_k + n_qk;
   (void)n_v;
-  hipLaunchKernelGGL((gla_backward_kernel<TIO, TG, DK, DV, TB>), dim3(a.B * a.H), dim3(256), 0, a.stream,
+  hipLaunchKernelGGL((gla_backward_kernel<TIO, TG, DK, DV, TB>), dim3(a.B * a.H, a.split ? 2 : 1), dim3(256), 0, a.stream,
                      (const TIO*)a.q, (const TIO*)a.k, (const TIO*)a.v, (const TG*)a.g_fwd, (const TG*)a.g_bwd,
                      (const TIO*)a.d_o, (TIO*)a.dq, (TIO*)a.dk, (TIO*)a.dv, (TG*)a.dg_fwd, (TG*)a.dg_bwd, ws_dq,
-                     ws_acc_k, ws_acc_v, a.L, a.scale, a.out_scale, a.only_flagged);
+                     ws_acc_k, ws_acc_v, a.L, a.scale, a.out_scale, a.only_flagged, (int)a.split);
   return hipGetLastError() == hipSuccess ? 0 : -5;
 }
 
@@ -280,7 +315,7 @@ int launch_gla_backward(const void* q, const void* k, const void* v, const void*
                         int B, int H, int L, int Dk, int Dv, float scale, float out_scale, int io_dtype,
                         int gate_dtype, bool exact, hipStream_t stream) {
   GlaBwdArgs a{q, k, v, g_fwd, g_bwd, d_o, dq, dk, dv, dg_fwd, dg_bwd, workspace, B, H, L, Dk, Dv,
-               scale, out_scale, io_dtype, gate_dtype, stream, nullptr};
+               scale, out_scale, io_dtype, gate_dtype, stream, nullptr, false};
   if (!exact && gla_backward_mfma_supported(B, H, L, Dk, Dv, io_dtype, gate_dtype, g_bwd != nullptr)) {
     int* flags = reinterpret_cast<int*>((float*)workspace + recurrent_floats(B, H, L, Dk, Dv, g_bwd != nullptr));
     void* seg_ws = (char*)workspace + flags_end(B, H, L, Dk, Dv, g_bwd != nullptr);
@@ -302,6 +337,10 @@ int launch_gla_backward(const void* q, const void* k, const void* v, const void*
                                            Dk, scale * out_scale, stream);
     if (rc != 0) return rc;
     a.only_flagged = flags;
+    // A flagged sequence takes as long as a launch full of them, behind everybody else's tile form: its directions side by side
+    // halve that (192 sequences of 197 tokens, D 64, one in seven flagged: 587 -> 389 us, none 145; 24 of 1025, Dk 32: 2260 ->
+    // 1105; 768 of 196, D 64: one in seven 944 -> 743, all 727 -> 716)
+    a.split = g_bwd != nullptr;
   }
   if (io_dtype == 0) return gate_dtype == 0 ? launch_bwd_d<float, float>(a) : launch_bwd_d<float, uint16_t>(a);
   return gate_dtype == 0 ? launch_bwd_d<uint16_t, float>(a) : launch_bwd_d<uint16_t, uint16_t>(a);
