@@ -17,7 +17,7 @@
 // set of key pieces serves both).  Only q' grows, so the form holds while |G| <= 40 in every channel of every tile (a mean
 // gate of -0.87 per token) and the inputs stay below 1e12.  A workgroup that meets stronger gates does its tokens again with
 // operands for any gates (prepare32_any); inputs beyond the bound, gates that grow and gates that are no numbers take the
-// serial form (serial_segment).  All sequences strongly gated: B 32, H 6, L 197, D 64 81 us (mildly gated 38; the
+// serial form (serial_segment).  All sequences strongly gated: B 32, H 6, L 197, D 64 81 us (mildly gated 37; the
 // token-recurrent kernel 182, the serial form, one wave of a workgroup, 1069); 768 sequences 233 us (112 / 221 / 3214).
 #include "f32_tiles.h"
 
@@ -197,6 +197,9 @@ __device__ __forceinline__ void walk32(char* lds, const F32Lds<NG>& lay, int ti,
   for (int s = 1; s <= n; ++s) {
     const int j = FWD ? ti - s : ti + s;
     if (s > 1) decay_q<NG>(reinterpret_cast<const float*>(lds + lay.d) + 64 * (FWD ? j + 1 : j - 1), lane >> 5, qh);
+    // matrix and vector instructions in turns: left to itself the compiler put the cutting of a tile's operands into one run in
+    // front of its products (B 64, H 6, L 196, Dk 32 51.7 -> 48.9 us, one image 23.2 -> 21.7)
+    __builtin_amdgcn_iglp_opt(0);
     char* kreg = lds + (FWD ? j : j - 1) * F32Lds<NG>::KB;
     f32x16_t P = {0.f}, Ps = {0.f};
 #pragma unroll
@@ -366,6 +369,7 @@ __device__ __forceinline__ int f32_pass(const F32Place<NG>& p, char* lds, float 
 #pragma unroll
     for (int c = 0; c < NG; ++c) mag += sum_abs(xq[c]) + sum_abs(xk[c]);
     const bool large = __builtin_amdgcn_ballot_w64(!(mag < kMagnitude32)) != 0;
+    __builtin_amdgcn_sched_barrier(0);  // (the values' registers are free before the operands' are needed: 35.5 -> 34.8 us)
     const bool wide = prepare32<NG, true>(xq, xk, xg, sc, dall + 64 * ti, kreg, lane, qh, P);
     wave_lds_sync();
     apply_values32(P, vreg, lane, O);
@@ -561,7 +565,7 @@ __global__ __launch_bounds__(256, 2) void gla_f32_state_kernel(const float* __re
   }
 }
 
-// Measured at B 32, H 6, L 197, D 64 (58 MB): 38 us per call, token-recurrent kernel 181 us.
+// Measured at B 32, H 6, L 197, D 64 (58 MB): 37 us per call (34.7 in a captured run), token-recurrent kernel 181 us.
 constexpr int kF32MaxLds = 160 * 1024;
 
 bool gla_f32_supported(const GlaArgs& a) {

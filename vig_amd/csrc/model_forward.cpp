@@ -276,7 +276,7 @@ bool usable(const Tensor& t, const c10::Device& dev, at::ScalarType type) {
 }  // namespace
 
 // Adds what has to stay as it is of a module and its children: their places in the tree, every parameter, and the entries of the
-// module's own dictionary that `settings` (type -> names) lists; false where a name of `absent` (type -> name) is there.
+// module's own dictionary that `settings` (type or module -> names) lists; false where a name of `absent` (type -> name) is there.
 bool collect(Plan& p, PyObject* module, PyObject* settings, PyObject* absent, std::vector<PyObject*>& seen) {
   if (std::find(seen.begin(), seen.end(), module) != seen.end()) return true;
   seen.push_back(module);
@@ -287,7 +287,9 @@ bool collect(Plan& p, PyObject* module, PyObject* settings, PyObject* absent, st
   PyObject *children = PyDict_GetItemString(own, "_modules"), *params = PyDict_GetItemString(own, "_parameters");
   if (!children || !params || !PyDict_Check(children) || !PyDict_Check(params)) return false;
   PyObject *key, *value, *type = reinterpret_cast<PyObject*>(Py_TYPE(module));
-  if (PyObject* names = PyDict_GetItemWithError(settings, type))
+  PyObject* names = PyDict_GetItemWithError(settings, type);
+  if (!names) names = PyDict_GetItemWithError(settings, module);
+  if (names)
     for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(names); ++i) {
       PyObject* v = PyDict_GetItemWithError(own, PyTuple_GET_ITEM(names, i));
       p.entries.push_back({Ref(own), Ref(PyTuple_GET_ITEM(names, i)), Ref(v)});

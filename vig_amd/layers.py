@@ -751,7 +751,7 @@ class ViG(nn.Module):
         settings = {GatedLinearAttention: ("strong_gates", "layernorm_eps", "clamp_min", "use_out_act", "use_act_in_conv",
                                            "gate_logit_normalizer", "num_heads", "head_qk_dim", "head_v_dim", "training"),
                     GLABlock: ("training",), RMSNorm: ("eps",), LayerNorm2d: ("eps",), ViG: ("patch_resolution",),
-                    nn.Conv2d: ("stride", "padding", "dilation", "groups")}
+                    **dict.fromkeys((conv1, conv2), ("stride", "padding", "dilation", "groups"))}
         absent = {GLABlock: "forward_carry", GatedLinearAttention: "_mix", ViG: "forward_features"}
         called = [pe, norm1, act, norm2, kids["norm"], kids["head"], torch.nn.modules.module._global_forward_hooks,
                   torch.nn.modules.module._global_forward_pre_hooks]
