@@ -31,7 +31,8 @@ struct Entry {
   Ref dict, key, value;  // value NULL: the key has to be absent
 };
 struct Watched {
-  Tensor t, data;  // data: an alias, so that the storage lives and nothing else can come to lie at ptr
+  Tensor t;
+  c10::Storage storage;  // kept, so that nothing else can come to lie at ptr
   void* ptr;
   uint32_t version;
   at::ScalarType type;
@@ -85,10 +86,7 @@ struct Reader {
     if (!o) throw python_error();
     return o;
   }
-  Tensor tensor() {  // an alias outside of autograd
-    const Tensor t = tensor_arg(next());
-    return t.defined() ? t.detach() : t;
-  }
+  Tensor tensor() { return tensor_arg(next()); }
   double real() {
     PyObject* o = next();
     const double v = o == Py_None ? std::nan("") : PyFloat_AsDouble(o);
@@ -303,7 +301,7 @@ bool collect(Plan& p, PyObject* module, PyObject* settings, PyObject* absent, st
     if (value == Py_None) continue;
     const Tensor t = tensor_arg(value);
     if (!t.defined() || t.unsafeGetTensorImpl()->is_python_dispatch() || t.scalar_type() != at::kBFloat16) return false;
-    p.watched.push_back({t, t.detach(), t.data_ptr(), (uint32_t)t._version(), t.scalar_type()});
+    p.watched.push_back({t, t.storage(), t.data_ptr(), (uint32_t)t._version(), t.scalar_type()});
   }
   for (Py_ssize_t at = 0; PyDict_Next(children, &at, &key, &value);) {
     p.entries.push_back({Ref(children), Ref(key), Ref(value)});

@@ -70,15 +70,19 @@ def invalidate_caches(model: nn.Module) -> None:
     a write through `.data` (p.data.mul_(..), module.weight.data[...] = ..) changes neither the pointer nor the version
     counter they are keyed on, so code that writes that way calls this afterwards.  load_state_dict and train() /
     eval() switches and moves of these modules call it by themselves."""
-    modules = list(model.modules())
+    _forget(list(model.modules()))
+
+
+def _forget(modules: list) -> None:
     for owner, plan in list(_PLANS.items()) if len(_PLANS) else ():  # (a plan goes when a module that it describes is touched)
-        if owner is model or _ext.calls().plan_describes(plan, modules):
+        if _ext.calls().plan_describes(plan, modules):
             _PLANS.pop(owner, None)
     for m in modules:
+        d = m.__dict__
         for a in _CACHE_ATTRS:
-            m.__dict__.pop(a, None)
-        if "_in_cat" in m.__dict__:
-            m.__dict__["_in_cat"] = None
+            d.pop(a, None)
+        if "_in_cat" in d:
+            d["_in_cat"] = None
 
 
 class _CacheMixin:
@@ -86,16 +90,17 @@ class _CacheMixin:
     training and evaluation (the usual places where weights change behind the version counter) or a move to another device
     or type (they hold the storages they were made from)."""
 
+    # (each of the three comes by every submodule by itself)
     def train(self, mode: bool = True):
-        invalidate_caches(self)
+        _forget([self])
         return super().train(mode)
 
     def _apply(self, *args, **kwargs):
-        invalidate_caches(self)
+        _forget([self])
         return super()._apply(*args, **kwargs)
 
     def _load_from_state_dict(self, *args, **kwargs):
-        invalidate_caches(self)
+        _forget([self])
         return super()._load_from_state_dict(*args, **kwargs)
 
 
@@ -792,7 +797,7 @@ class ViG(nn.Module):
             dev = head_w.device
             if any(t is not None and (t.device != dev or t.dtype is not torch.bfloat16) for t in small + rows + biases):
                 raise _NoPlan
-            flat = [t.reshape(-1) for t in small if t is not None]
+            flat = [t if t.dim() == 1 else t.reshape(-1) for t in small if t is not None]
             pieces = iter(torch.cat(flat).float().split([t.numel() for t in flat]))
             f32 = [next(pieces) if t is not None else None for t in small]
             heights = [sum(t.shape[0] for t in rows[i:i + 4]) for i in range(0, len(rows), 4)]
