@@ -77,8 +77,9 @@ const char* vig_gla_strerror(int code);
  * HierViG's head shape (bf16, Dk = 16, Dv = 32, both directions) takes the same
  * paths from L = 128 on, zero-padded to Dk 32 / Dv 64 in the workspace
  * (classification/models/vig_h.py:377-385 with EXPAND_K 0.5, EXPAND_V 1.0).
- * Other combinations run on the
- * fp32-arithmetic kernel, which has no such limit.
+ * fp32 tensors and gates with Dk in {32, 64}, Dv = 64: matrix-core kernels too, every operand in three bf16 pieces
+ * (fp32 precision), any gates and magnitudes; sequences longer than 224 tokens as segments linked by states in the
+ * workspace.  Other combinations run on the fp32-arithmetic token-recurrent kernel, which has no limit either.
  */
 int vig_gla_bidir_fwd(const void* q, const void* k, const void* v,
                       const void* g_fwd, const void* g_bwd, void* o,
@@ -208,8 +209,10 @@ int vig_gla_bidir_fwd_exact(const void* q, const void* k, const void* v,
  * g_bwd == NULL) -> matrix-core kernel (bf16 operands, fp32 accumulation; gradients within ~1e-2 of their largest
  * magnitude): one quadratic form per (batch, head) for L <= 256; a longer sequence as segments of <= 256 tokens linked
  * by their states (two state passes of the forward kernel, a segment scan, then one quadratic form per segment;
- * B*H*directions <= 65535).  A sequence with a segment whose gate total exceeds ~83 in some channel, and every other
- * case -> fp32-arithmetic token-recurrent kernel.
+ * B*H*directions <= 65535).  fp32 tensors and gates with the same head widths -> matrix-core kernel on operands in
+ * three bf16 pieces (fp32 precision).  A sequence with a segment whose gate total exceeds ~83 in some channel (fp32: a
+ * 32-token tile with a total beyond ~28, or values beyond 1e12), and every other case -> fp32-arithmetic token-recurrent
+ * kernel.
  *
  * Replaces: FusedChunkGLAFunction.backward (flash-linear-attention/fla/ops/gla/chunk_fuse.py:413-518; gate
  * gradient :505-518) under the flip-concat glue of classification/models/vig.py:407-426, for both directions in

@@ -521,7 +521,6 @@ __global__ __launch_bounds__(256, 2) void gla_f32_state_kernel(const float* __re
       // registers 4u .. 4u + 3 are tokens 8u + 4h + (0 .. 3)
 #pragma unroll
       for (int x = 0; x < 4; ++x) {
-        const int u = dir == 0 ? 3 - x : x;
         const float mine = dir == 0 ? tot[3 - x] : tot[x], theirs = dir == 0 ? other[3 - x] : other[x];
         // the half whose four tokens come first against the walk order: the upper one forward, the lower one reverse
         const bool late = (h == 1) != (dir == 0);
@@ -541,7 +540,6 @@ __global__ __launch_bounds__(256, 2) void gla_f32_state_kernel(const float* __re
             xk[p][i] *= exp2_fast(ex);
           }
         }
-        (void)u;
       }
 #pragma unroll
       for (int t = 0; t < 2; ++t) mfma6(split8(octet(xk[p], t)), pvv[t], acc[p], accs[p]);

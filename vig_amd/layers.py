@@ -1,9 +1,9 @@
 """Block- and model-level host side: the reference's module interfaces over the HIP ops.
 
 `GatedLinearAttention` keeps the constructor arguments, forward signature and parameter names of
-classification/models/vig.py:241-464, so a reference state_dict loads unchanged.  The three GEMMs
-(qkv_proj, gk_proj, g_proj, o_proj) stay in torch (hipBLASLt); everything between them runs in this
-package's kernels:
+classification/models/vig.py:241-464, so a reference state_dict loads unchanged.  The projections
+(qkv_proj, gk_proj, g_proj, o_proj) run on this package's row products where those are the better choice for
+the size and in torch (hipBLASLt) otherwise; everything between them runs in this package's kernels:
     3x3 depthwise conv on the token grid   -> vig_dwconv3x3_fwd      (vig.py:291-294,428-430)
     direction-wise gate preparation        -> vig_dirgate_fwd        (vig.py:432-441)
     bidirectional GLA                      -> vig_gla_bidir_fwd      (vig.py:442-443)
@@ -11,17 +11,17 @@ package's kernels:
     split + three head rearranges          -> vig_split_heads_fwd    (vig.py:401-409)
     residual add + RMSNorm (prenorm)       -> vig_rmsnorm_fwd        (rmsnorm.py:69-125; vig.py:598,602-606,896)
     SwiGLU product                         -> vig_swiglu_fwd         (activations.py:109-113; vig.py:492-495)
-The surrounding ViG shell (patch embedding, MLP GEMMs, head) is plain torch and follows
-vig.py:469-497,530-618,625-672,705-912 for the options the shipped configs use.  There is no CPU path: every
-library op raises on tensors that are not on the GPU.
+The surrounding ViG shell (patch embedding, MLP, head) follows vig.py:469-497,530-618,625-672,705-912 for the options
+the shipped configs use.  There is no CPU path: every library op raises on tensors that are not on the GPU.
 
 Two ways through every module.  In eval mode, or whenever gradients are not being recorded, the forward runs on the
 library's fused inference kernels and leaves no autograd graph.  In training mode with gradients enabled
-(`model.train()` outside `torch.no_grad()`) the block records one: the GEMMs and the patch embedding are torch's
-differentiable operations, and everything between them -- depthwise conv, head split, gate preparation, the
-bidirectional GLA, the norm/blend epilogue, the residual RMS norms and the SwiGLU product -- runs on the library's
-kernels in both directions through the autograd nodes of `ops` (the reference's training branch, vig.py:354-426,
-with its flips and concatenations folded into the op).
+(`model.train()` outside `torch.no_grad()`) the block records one, as two native nodes (csrc/train_block.cpp); where
+something hangs on a submodule's call it runs module by module: the GEMMs are torch's differentiable operations, and
+everything between them -- depthwise conv, head split, gate preparation, the bidirectional GLA, the norm/blend
+epilogue, the residual RMS norms and the SwiGLU product -- runs on the library's kernels in both directions through
+the autograd nodes of `ops` (the reference's training branch, vig.py:354-426, with its flips and concatenations
+folded into the op).  The patch embedding is torch's in training.
 """
 from __future__ import annotations
 
