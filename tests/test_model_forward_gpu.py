@@ -238,6 +238,40 @@ def test_models_of_another_tree(change, monkeypatch):
     assert got.shape[1] == (192 if change == "features" else 16)
 
 
+def test_plans_of_several_threads(monkeypatch):
+    """Models served by threads, some shared, with eval() before some of the requests."""
+    announce("plans of several threads")
+    import sys
+    import threading
+
+    models, x = [_tiny(128)[0] for _ in range(6)], _tiny(128)[1]
+    want = [_modules(monkeypatch, m, x) for m in models]
+    errors, interval = [], sys.getswitchinterval()
+
+    def serve(i):
+        try:
+            for k in range(200):
+                at = (i + k) % 6 if i < 2 else i
+                if k % 3 == 0:
+                    models[at].eval()
+                y = models[at](x)
+                if k % 40 == 0 and not torch.equal(y, want[at]):
+                    errors.append(f"thread {i}, request {k}: another result")
+        except Exception as e:
+            errors.append(f"thread {i}: {e!r}")
+
+    sys.setswitchinterval(1e-6)
+    try:
+        threads = [threading.Thread(target=serve, args=(i,)) for i in range(4)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+    finally:
+        sys.setswitchinterval(interval)
+    assert not errors, errors
+
+
 class _Products(torch.utils._python_dispatch.TorchDispatchMode):
     """Counts the matrix products of the operators that it sees."""
 

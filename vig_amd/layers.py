@@ -26,6 +26,7 @@ folded into the op).  The patch embedding is torch's in training.
 from __future__ import annotations
 
 import math
+import threading
 import weakref
 from typing import Optional
 
@@ -61,6 +62,7 @@ def _f32(owner: nn.Module, tag: str, t: Optional[torch.Tensor], shape=None):
 
 
 _PLANS = weakref.WeakKeyDictionary()  # model -> plan of its native evaluation forward (ViG._planned)
+_PLANS_LOCK = threading.RLock()  # (held where the dictionary grows, shrinks or is gone through; a model may be served by several threads)
 _CACHE_ATTRS = ("_f32_cache", "_w32_key", "_w32_cache", "_w32_from", "_w1_packed")
 
 
@@ -74,9 +76,11 @@ def invalidate_caches(model: nn.Module) -> None:
 
 
 def _forget(modules: list) -> None:
-    for owner, plan in list(_PLANS.items()) if len(_PLANS) else ():  # (a plan goes when a module that it describes is touched)
-        if _ext.calls().plan_describes(plan, modules):
-            _PLANS.pop(owner, None)
+    if len(_PLANS):
+        with _PLANS_LOCK:
+            for owner, plan in list(_PLANS.items()):  # (a plan goes when a module that it describes is touched)
+                if _ext.calls().plan_describes(plan, modules):
+                    _PLANS.pop(owner, None)
     for m in modules:
         d = m.__dict__
         for a in _CACHE_ATTRS:
@@ -720,11 +724,13 @@ class ViG(nn.Module):
                 plan = self._make_plan(calls)
                 if plan is None:
                     return None
-                _PLANS[self] = plan
+                with _PLANS_LOCK:
+                    _PLANS[self] = plan
             y = calls.run_plan(plan, x)
             if y is not False:
                 return y
-            _PLANS.pop(self, None)
+            with _PLANS_LOCK:
+                _PLANS.pop(self, None)
         return None
 
     def _make_plan(self, calls):

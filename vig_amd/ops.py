@@ -935,10 +935,10 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] =
     otherwise.  Inference only (no autograd node of its own)."""
     N, K = weight.shape
     if (x.dtype == weight.dtype == torch.bfloat16 and x.is_cuda and weight.device == x.device and x.shape[-1] == K
+            and _owns_data(x, weight, bias) and not torch.is_autocast_enabled() and not observed()
             and x.is_contiguous() and weight.is_contiguous() and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0
             and (bias is None or (bias.dtype == x.dtype and bias.device == x.device and bias.shape == (N,)
-                                  and bias.is_contiguous() and bias.data_ptr() % 16 == 0))
-            and _owns_data(x, weight, bias) and not torch.is_autocast_enabled() and not observed()):
+                                  and bias.is_contiguous() and bias.data_ptr() % 16 == 0))):
         lib, rows = _lib.load(), x.numel() // K
         if lib.vig_linear_preferred(rows, N, K):
             y = torch.empty(*x.shape[:-1], N, dtype=x.dtype, device=x.device)
@@ -956,8 +956,8 @@ def conv3x3s2(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     B, Cin, H, W = x.shape
     Cout = weight.shape[0]
     xl, wl = x.permute(0, 2, 3, 1), weight.detach().permute(0, 2, 3, 1)
-    if not (_owns_data(x, weight) and not observed() and x.dtype == weight.dtype == torch.bfloat16 and x.is_cuda
-            and weight.device == x.device and x.numel() and Cin % 32 == 0 and Cout % 8 == 0
+    if not (x.dtype == weight.dtype == torch.bfloat16 and x.is_cuda and weight.device == x.device and x.numel()
+            and _owns_data(x, weight) and not observed() and Cin % 32 == 0 and Cout % 8 == 0
             and weight.shape[1:] == (Cin, 3, 3) and xl.is_contiguous() and wl.is_contiguous()
             and xl.data_ptr() % 16 == 0 and wl.data_ptr() % 16 == 0 and not torch.is_autocast_enabled()):
         return torch.nn.functional.conv2d(x, weight, None, 2, 1)
