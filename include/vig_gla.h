@@ -61,13 +61,13 @@ const char* vig_gla_strerror(int code);
  * Numeric range of the matrix-core paths (bf16 tensors and gates, Dk in {32, 64},
  * Dv = 64).  q, k and v may hold any finite bf16 values; the kernels check
  * magnitudes and gate totals themselves and switch arithmetic where needed:
- *   L <= 256 (one workgroup per sequence, one wave per 32-token tile): fp16
+ *   L <= 512 at Dk 32, 416 at Dk 64 (one workgroup per sequence, one wave per 32-token tile): fp16
  *   operands while every tile's gate total stays within about 7 (natural log
  *   units) per channel and rows of q / k / v have sums of squares below 2^15 /
  *   2^10 / 10^8; a sequence outside that is redone by the same workgroup with
  *   power-of-two input scales and split-bf16 diagonal tiles, good for gates down
  *   to about -5 per token (beyond: exponents are clamped, far tokens count as 0).
- *   L > 256 (segments of <= 224 tokens, seven tiles each, chained through states
+ *   longer (from 257 on for vig_gla_bidir_fwd_wide; segments of <= 224 tokens, seven tiles each, chained through states
  *   in the workspace: a state pass, a scan, then the kernel above once more per
  *   segment with the entering states; refused with VIG_ENOTSUP when
  *   B*H*directions > 65535): the same per-tile behaviour for the outputs, and for
@@ -108,11 +108,26 @@ int vig_gla_bidir_fwd_strided(const void* q, const void* k, const void* v,
                               float scale, float out_scale,
                               int io_dtype, int gate_dtype, void* stream);
 
+/* Longest sequence that one workgroup takes whole, tensors in LDS (0: no such kernel for this Dk). */
+int vig_gla_slab_tokens(int Dk);
+
+/*
+ * The one-launch kernel behind vig_gla_bidir_fwd, _strided and vig_gla_bidir_locgate_fwd at every length it takes
+ * (L <= vig_gla_slab_tokens(Dk); those two stop at 256): strides as for _strided, each NULL for a plain tensor; with
+ * gate_weight [H*Dv, 3, 3] f32 (NULL: none) the locality gate of vig_gla_bidir_locgate_fwd on a grid_h x grid_w token grid
+ * (both directions, plain tensors, grid_w <= 126, a grid whose padded rows fit LDS).  VIG_ENOTSUP for anything else.  No workspace.
+ */
+int vig_gla_slab_fwd(const void* q, const void* k, const void* v, const void* g_fwd, const void* g_bwd,
+                     const float* gate_weight, void* o, int B, int H, int L, int Dk, int Dv,
+                     const long long* q_strides, const long long* k_strides, const long long* v_strides,
+                     int grid_h, int grid_w, float scale, float out_scale, int io_dtype, int gate_dtype, void* stream);
+
 /* Workspace that is enough for every gate dtype and for one or two directions (the largest over the kernels the
  * call may dispatch to for this shape and io_dtype). */
 size_t vig_gla_bidir_fwd_workspace(int B, int H, int L, int Dk, int Dv, int io_dtype);
 /* Workspace of exactly the kernel vig_gla_bidir_fwd / _wide dispatch to for these arguments (bidirectional: g_bwd
- * given): 0 for bf16 tensors and gates with Dk in {32, 64}, Dv = 64, L <= 256. */
+ * given): 0 for bf16 tensors and gates with Dk in {32, 64}, Dv = 64, L <= 256 (between 257 tokens and the one-launch
+ * kernel's limit only _wide uses it, but both ask for it). */
 size_t vig_gla_bidir_fwd_workspace_for(int B, int H, int L, int Dk, int Dv, int io_dtype, int gate_dtype,
                                        int bidirectional);
 

@@ -240,6 +240,25 @@ int vig_gla_bidir_fwd_strided(const void* q, const void* k, const void* v, const
   return vig::launch_gla_mfma(a);
 }
 
+// The one-launch kernel at every length it takes, with q, k, v in place and the locality gate as options; no workspace.
+int vig_gla_slab_tokens(int Dk) { return Dk == 64 || Dk == 32 ? vig::gla_slab_tokens(Dk) : 0; }
+
+int vig_gla_slab_fwd(const void* q, const void* k, const void* v, const void* g_fwd, const void* g_bwd, const float* gate_weight,
+                     void* o, int B, int H, int L, int Dk, int Dv, const long long* q_strides, const long long* k_strides,
+                     const long long* v_strides, int grid_h, int grid_w, float scale, float out_scale, int io_dtype,
+                     int gate_dtype, void* stream) {
+  vig::GlaArgs a;
+  const int rc = fill_args(a, q, k, v, g_fwd, g_bwd, o, nullptr, 0, B, H, L, Dk, Dv, scale, out_scale, io_dtype, gate_dtype, stream);
+  if (rc != VIG_OK) return rc;
+  a.q_strides = q_strides, a.k_strides = k_strides, a.v_strides = v_strides;
+  if (gate_weight) {
+    if (!g_bwd || grid_h <= 0 || grid_w <= 0 || (long long)grid_h * grid_w != L || !aligned16(gate_weight)) return VIG_EINVAL;
+    if (grid_w > 126) return VIG_ENOTSUP;  // (grids that vig_locality_gate_fwd takes: one op, whichever way it runs)
+    a.gate_w = gate_weight, a.gate_rows = grid_h, a.gate_cols = grid_w;
+  }
+  return vig::gla_tiles_supported(a) ? vig::launch_gla_tiles(a) : VIG_ENOTSUP;
+}
+
 // The causal op with a state carried in and / or out.
 static size_t causal_state_workspace(int B, int H, int L, int Dk, int Dv, int io_dtype, int gate_dtype) {
   if (io_dtype == VIG_BF16 && gate_dtype == VIG_BF16 && (Dk == 64 || Dk == 32) && Dv == 64)

@@ -1,6 +1,6 @@
 // Bidirectional GLA forward on MFMA tiles (gfx950), Dk in {32, 64}, Dv = 64, bf16 in and out: one workgroup per
-// (batch, head) slab of up to 256 tokens, one wave per 32-token query tile, both directions in the same wave.  A longer
-// sequence is cut into segments of at most seven tiles, each handled like a slab plus the products with the states
+// (batch, head) slab of up to 512 tokens (Dk 64: 416), one wave per 32-token query tile, both directions in the same wave.
+// A longer sequence is cut into segments of at most seven tiles, each handled like a slab plus the products with the states
 // that enter it from either side (apply_state; the states come from a state pass and a scan, gla_mfma.hip).
 //
 // Wave i owns the queries of tile i.  Along the forward direction they see the keys of tiles j <= i, along the
@@ -769,7 +769,7 @@ __device__ __noinline__ void tile_pass_general(const TileKernArgs* ka_in) {
 }  // namespace
 
 template <int NG, bool BIDIR, bool PITCHED, bool GATE, bool CHAIN = false>
-__global__ __launch_bounds__(512, 4) void gla_tile_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
+__global__ __launch_bounds__(1024, 4) void gla_tile_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
                                                           const uint16_t* __restrict__ v,
                                                           const uint16_t* __restrict__ gf,
                                                           const uint16_t* __restrict__ gb, uint16_t* __restrict__ o,
@@ -803,15 +803,23 @@ __global__ __launch_bounds__(512, 2) void gla_tile_wide_kernel(const uint16_t* _
 
 constexpr int kTileMaxLds = 160 * 1024;
 
+// Whole sequences up to 13 tiles (Dk 64: 158 KB of LDS) or 16 (Dk 32: sixteen waves of 128 registers, all that a CU holds) go
+// through one workgroup: k, v and the gates are read once instead of twice, no states pass through memory, one launch instead
+// of three.  us, one workgroup / segments linked by states: Dk 32: 3 sequences of 257 10.4 / 19.6, 480 of 300 29 / 75, 312 of 512
+// 38 / 81; Dk 64: 3 of 257 13.7 / 22.7, 6 of 400 18.8 / 24.0, 480 of 300 40 / 96, 360 of 416 49 / 76.
+// The general form's own kernel has twice the registers per wave and takes eight.
+int gla_slab_tokens(int Dk) { return Dk == 64 ? 416 : 512; }
+
 bool gla_tiles_supported(const GlaArgs& a) {
-  if (!(a.io_dtype == 1 && a.gate_dtype == 1 && (a.Dk == 64 || a.Dk == 32) && a.Dv == 64 && a.L <= 256 &&
-        !a.init_state && !a.final_state && !a.state_pass))
+  if (!(a.io_dtype == 1 && a.gate_dtype == 1 && (a.Dk == 64 || a.Dk == 32) && a.Dv == 64 &&
+        a.L <= (a.wide_gates ? 256 : gla_slab_tokens(a.Dk)) && !a.init_state && !a.final_state && !a.state_pass))
     return false;
   if (a.gate_w) {  // fused locality gate: both directions, plain tensors, the padded grid has to fit in LDS
     if (!a.g_bwd || a.q_strides || a.k_strides || a.v_strides || a.gate_cols <= 0 || a.gate_rows <= 0 ||
         (long long)a.gate_cols * a.gate_rows != a.L)
       return false;
-    if (TileLds<4>((a.L + 31) / 32, gate_stage_bytes(a.gate_cols, a.gate_rows)).total > kTileMaxLds) return false;
+    const int NT = (a.L + 31) / 32, stage = gate_stage_bytes(a.gate_cols, a.gate_rows);
+    if ((a.Dk == 64 ? TileLds<4>(NT, stage).total : TileLds<2>(NT, stage).total) > kTileMaxLds) return false;
   }
   return true;
 }

@@ -89,6 +89,7 @@ bool gla_mfma_supported(const GlaArgs& a);
 int launch_gla_mfma(const GlaArgs& a);
 // bf16 tile-pair path for whole-sequence slabs (L <= 256): one wave per 32-token tile, both directions per wave.
 bool gla_tiles_supported(const GlaArgs& a);
+int gla_slab_tokens(int Dk);  // longest sequence that one workgroup takes whole
 int launch_gla_tiles(const GlaArgs& a);
 // the same kernel as the output pass of a long sequence (L > 256): one workgroup per (sequence, segment), the states
 // entering the segments (scanned slots, kGlaStateFloats floats per (sequence, segment, direction)) and their maxima

@@ -144,7 +144,8 @@ Tensor run(const Plan& p, const Tensor& images) {
     nz = std::max(nz, b.w_in.size(0)), I = std::max(I, b.w_down.size(1)), K2 = std::max<int64_t>(K2, 2 * b.H * b.Dk);
     swiglu_kernel = swiglu_kernel && b.w_down.size(1) % 32 == 0;
   }
-  const bool whole = L <= 256;  // q, k, v are read in place from the projection's rows
+  bool whole = true;  // q, k, v are read in place from the projection's rows
+  for (const auto& b : p.blocks) whole = whole && L <= vig_gla_slab_tokens(b.Dk);
   size_t gla_ws = 0;
   if (!whole)
     for (const auto& b : p.blocks)
@@ -208,9 +209,9 @@ Tensor run(const Plan& p, const Tensor& images) {
     const int64_t gb = gates + T * b.H * b.Dk;
     if (whole) {
       const long long sqk[3] = {(long long)(L * ld), b.Dk, ld}, sv[3] = {(long long)(L * ld), b.Dv, ld};
-      check_rc(vig_gla_bidir_fwd_strided(k.at(z), k.at(z + b.H * b.Dk), k.at(z + 2 * b.H * b.Dk), k.at(gates), k.at(gb), k.at(o), (int)B,
-                                         b.H, (int)L, b.Dk, b.Dv, sqk, sqk, sv, scale, 0.25f, VIG_BF16, VIG_BF16, k.stream),
-               "vig_gla_bidir_fwd_strided");
+      check_rc(vig_gla_slab_fwd(k.at(z), k.at(z + b.H * b.Dk), k.at(z + 2 * b.H * b.Dk), k.at(gates), k.at(gb), nullptr, k.at(o), (int)B,
+                                b.H, (int)L, b.Dk, b.Dv, sqk, sqk, sv, 0, 0, scale, 0.25f, VIG_BF16, VIG_BF16, k.stream),
+               "vig_gla_slab_fwd");
     } else {
       check_rc(vig_split_heads_fwd(k.at(z), k.at(q), k.at(kk), k.at(v), (int)B, (int)L, b.H, b.Dk, b.Dv, ld, VIG_BF16, k.stream),
                "vig_split_heads_fwd");

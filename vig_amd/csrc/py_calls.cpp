@@ -143,6 +143,9 @@ PyObject* gla_gate(PyObject*, PyObject* const* a, Py_ssize_t n) {
                                                     y.data_ptr(), c.B, c.H, c.L, c.Dk, c.Dv, (int)h, (int)w, c.scale,
                                                     c.out_scale, c.io, c.gd, stream_of(q))
                         : VIG_ENOTSUP;
+  if (rc == VIG_ENOTSUP && gb.defined() && c.L > 256)
+    rc = vig_gla_slab_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), gf.data_ptr(), gb.data_ptr(), wt, y.data_ptr(), c.B, c.H, c.L,
+                          c.Dk, c.Dv, nullptr, nullptr, nullptr, (int)h, (int)w, c.scale, c.out_scale, c.io, c.gd, stream_of(q));
   if (rc == VIG_ENOTSUP) {
     Tensor o;
     rc = run_forward(q, k, v, gf, gb, false, kDefault, c, o);
