@@ -1,0 +1,45 @@
+"""The matrix-core backward's workgroups of two, four and eight tiles at the edges of their ranges, and with more slabs than
+workgroups (each walks several)."""
+import pytest
+import torch
+
+import vig_amd
+from oracle import gla_oracle as O
+from vig_amd.synthetic import make_gla_inputs
+
+from .test_backward_gpu import _check_mfma, _do
+from .util import announce, f64
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("both", [True, False])
+@pytest.mark.parametrize("B,H,L,Dk", [(2, 2, 63, 32), (2, 2, 65, 64), (1, 3, 65, 32), (1, 2, 127, 64), (1, 3, 128, 32), (1, 2, 129, 64),
+                                      (1, 2, 129, 32)])
+def test_lengths(B, H, L, Dk, both):
+    announce(f"backward slabs B{B} H{H} L{L} Dk{Dk} both={both}")
+    q, k, v, gf, gb = make_gla_inputs(B, H, L, Dk, 64, seed=40 + L, dtype=torch.bfloat16)
+    do = _do(v.shape, 3, torch.bfloat16)
+    if both:
+        want = O.bidir_gla_backward(f64(q), f64(k), f64(v), f64(gf), f64(gb), f64(do), out_scale=0.5)
+    else:
+        want = O.gla_recurrent_backward(f64(q), f64(k), f64(v), f64(gf), f64(do))
+    got = vig_amd.gla_bidir_backward(q.cuda(), k.cuda(), v.cuda(), gf.cuda(), gb.cuda() if both else None, do.cuda(),
+                                     out_scale=0.5 if both else 1.0)
+    _check_mfma(got if both else got[:4], want, q)
+
+
+@pytest.mark.parametrize("B,H,L,Dk", [(360, 3, 57, 32), (180, 6, 40, 64), (90, 6, 100, 64)])
+def test_more_slabs_than_workgroups(B, H, L, Dk):
+    """Every ninth slab beyond the quadratic form's range: those from the recurrent kernel bit for bit, the rest within the bound."""
+    announce(f"backward slabs, {B * H} of {L} tokens, Dk{Dk}")
+    q, k, v, gf, gb = (t.cuda() for t in make_gla_inputs(B, H, L, Dk, 64, seed=5, dtype=torch.bfloat16))
+    strong = (torch.arange(B * H, device="cuda") % 9 == 4).reshape(B, H)
+    gf = torch.where(strong[:, :, None, None], torch.full_like(gf, -4.0), gf)
+    do = _do(v.shape, 4, torch.bfloat16).cuda()
+    exact = vig_amd.gla_bidir_backward(q, k, v, gf, gb, do, out_scale=0.5, exact=True)
+    got = vig_amd.gla_bidir_backward(q, k, v, gf, gb, do, out_scale=0.5)
+    for g, e in zip(got, exact):
+        assert torch.equal(g[strong], e[strong])
+    keep = ~strong
+    _check_mfma([g[keep] for g in got], [f64(e[keep]) for e in exact], q[keep].cpu())

@@ -11,7 +11,7 @@
 // s = scale * out_scale.  This is the natural-order form of flash-linear-attention/fla/ops/gla/chunk_fuse.py:413-518
 // with one chunk per sequence; the flip-concat glue of classification/models/vig.py:407-426 never materialises.
 //
-// One persistent workgroup of 8 waves per CU walks slabs; wave w owns the 32-token tile w.  Per direction the
+// One persistent workgroup of 8 waves per CU (two of 4, four of 2 for short slabs) walks slabs; wave w owns the 32-token tile w.  Per direction the
 // workgroup stages q~, k~ (and once v, do) as bf16 rows in LDS; then wave w accumulates dq of its tile over the key
 // tiles the direction keeps, and dk, dv of its tile over the query tiles: score tiles P, A come out of the matrix
 // cores in the register layout that feeds the next product directly (mfma_tiles.h), operands with tokens in the
@@ -34,16 +34,17 @@ namespace vig {
 
 namespace {
 
-constexpr int kBwdTiles = 8;                                // 32-token tiles per slab
-constexpr int kBwdMatBytes = kBwdTiles * 32 * kKtStride * 2;  // one staged 256 x 64 bf16 matrix, 144-byte rows
-constexpr int kBwdLdsQ = 0;
-constexpr int kBwdLdsK = kBwdMatBytes;
-constexpr int kBwdLdsV = 2 * kBwdMatBytes;
-constexpr int kBwdLdsDo = 3 * kBwdMatBytes;
-constexpr int kBwdLdsTot = 4 * kBwdMatBytes;           // [8][64] f32: gate totals of the tiles
-constexpr int kBwdLdsOff = kBwdLdsTot + 8 * 64 * 4;    // [8][64] f32: per wave, (prefix - anchor) of its tile
-constexpr int kBwdLdsDgTot = kBwdLdsOff + 8 * 64 * 4;  // [8][64] f32: totals of q dq - k dk of the tiles
-constexpr int kBwdLdsTotal = kBwdLdsDgTot + 8 * 64 * 4;
+constexpr int kBwdTiles = 8;  // most 32-token tiles per slab
+// LDS of a workgroup of TW tiles, one wave each
+template <int TW>
+struct BwdLds {
+  static constexpr int mat = TW * 32 * kKtStride * 2;  // one staged (32 TW) x 64 bf16 matrix, 144-byte rows
+  static constexpr int q = 0, k = mat, v = 2 * mat, d_o = 3 * mat;
+  static constexpr int tot = 4 * mat;               // [TW][64] f32: gate totals of the tiles
+  static constexpr int off = tot + TW * 64 * 4;     // [TW][64] f32: per wave, (prefix - anchor) of its tile
+  static constexpr int dgtot = off + TW * 64 * 4;   // [TW][64] f32: totals of q dq - k dk of the tiles
+  static constexpr int total = dgtot + TW * 64 * 4;
+};
 constexpr float kBwdHalfRange = 60.0f;
 
 
@@ -144,11 +145,11 @@ __device__ __forceinline__ void issue_bwd_row_loads(const BwdNext& n, int w, int
 
 // Tile-local cumulative gates of the direction whose gate dwords have arrived: G^T = g^T T, lane = token, registers =
 // channels HC*h + 8g + 2m + p; the tile total (at the tile's last token in walking order) goes to `tot`.
-template <bool FWD, int NG>
+template <bool FWD, int NG, int TW>
 __device__ __forceinline__ void bwd_cumulate_gates(const BwdLoads<NG>& ld, int w, int lane, char* lds, f32x16_t (&G)[2]) {
   constexpr int HC = 8 * NG;
   const int r = lane & 31, h = lane >> 5;
-  float* tot = reinterpret_cast<float*>(lds + kBwdLdsTot);
+  float* tot = reinterpret_cast<float*>(lds + BwdLds<TW>::tot);
   u32x4_t gfrag[2][2];
   finish_tfrags<2>(ld.gD, gfrag);  // (rows that carry no channel, NG = 2, hold zeros)
   const u32x4_t tri0 = tri_frag<FWD>(0, 0, r, h), tri1 = tri_frag<FWD>(1, 0, r, h);
@@ -178,7 +179,7 @@ __device__ __forceinline__ void bwd_cumulate_gates(const BwdLoads<NG>& ld, int w
 //   dq^_i += S_in' do_i,   dk^_j += R_out' v_j,   dv_j += R_out'^T k~_j
 // (the e^{G_i - a}, e^{a - G_j} factors applied to dq^, dk^ at the end turn e^a into e^{G_i}, e^{T - G_j}), and the
 // running sum of the gate gradient starts from the total of q dq - k dk over the segments walked later.
-template <bool FWD, bool FIRST, bool LAST, int NG, bool SEG>
+template <bool FWD, bool FIRST, bool LAST, int NG, bool SEG, int TW>
 __device__ __forceinline__ bool bwd_direction(const BwdSlab& sl, int L, int ntiles, int w, int lane, char* lds,
                                               float s, f32x16_t (&dv)[2], u32x4_t (&keepq)[NG], u32x4_t (&keepk)[NG],
                                               BwdLoads<NG>& ld, const BwdNext& nxt, f32x16_t (&G)[2]) {
@@ -190,13 +191,13 @@ __device__ __forceinline__ bool bwd_direction(const BwdSlab& sl, int L, int ntil
   constexpr int HC = 8 * NG;    // channels per lane half
   asm volatile("" : "+v"(lane));  // per-lane constants are rebuilt per direction instead of living across the slab loop
   const int r = lane & 31, h = lane >> 5;
-  uint16_t* Q = reinterpret_cast<uint16_t*>(lds + kBwdLdsQ);
-  uint16_t* K = reinterpret_cast<uint16_t*>(lds + kBwdLdsK);
-  uint16_t* V = reinterpret_cast<uint16_t*>(lds + kBwdLdsV);
-  uint16_t* DO = reinterpret_cast<uint16_t*>(lds + kBwdLdsDo);
-  float* tot = reinterpret_cast<float*>(lds + kBwdLdsTot);
-  float* offs = reinterpret_cast<float*>(lds + kBwdLdsOff) + w * 64;
-  float* dgtot = reinterpret_cast<float*>(lds + kBwdLdsDgTot);
+  uint16_t* Q = reinterpret_cast<uint16_t*>(lds + BwdLds<TW>::q);
+  uint16_t* K = reinterpret_cast<uint16_t*>(lds + BwdLds<TW>::k);
+  uint16_t* V = reinterpret_cast<uint16_t*>(lds + BwdLds<TW>::v);
+  uint16_t* DO = reinterpret_cast<uint16_t*>(lds + BwdLds<TW>::d_o);
+  float* tot = reinterpret_cast<float*>(lds + BwdLds<TW>::tot);
+  float* offs = reinterpret_cast<float*>(lds + BwdLds<TW>::off) + w * 64;
+  float* dgtot = reinterpret_cast<float*>(lds + BwdLds<TW>::dgtot);
   const int rows = __builtin_amdgcn_readfirstlane(min(max(L - 32 * w, 0), 32));  // valid tokens of this wave's tile
   const size_t tk = (size_t)32 * w * DK, tv = (size_t)32 * w * 64;
 
@@ -217,7 +218,7 @@ __device__ __forceinline__ bool bwd_direction(const BwdSlab& sl, int L, int ntil
   {
     float pre = 0.f, all = 0.f;
 #pragma unroll
-    for (int t = 0; t < kBwdTiles; ++t) {
+    for (int t = 0; t < TW; ++t) {
       const float x = lane < DK ? tot[t * 64 + lane] : 0.f;
       all += x;
       pre += (FWD ? (t < w) : (t > w)) ? x : 0.f;
@@ -483,13 +484,13 @@ __device__ __forceinline__ bool bwd_direction(const BwdSlab& sl, int L, int ntil
     // the next direction's rows travel while this one finishes; its cumulative gates and tile totals are prepared
     // here, so that one barrier serves both exchanges
     issue_bwd_row_loads<LAST, NG>(nxt, w, r, h, ld);
-    bwd_cumulate_gates<LAST, NG>(ld, w, lane, lds, G);
+    bwd_cumulate_gates<LAST, NG, TW>(ld, w, lane, lds, G);
     lds_barrier();  // (4) tile totals of X and of the next gates visible; nobody reads q~, k~, v, do of this direction
     {
       const int cl = lane < DK ? lane : 0;
       float run = 0.f;
 #pragma unroll
-      for (int t = 0; t < kBwdTiles; ++t) {
+      for (int t = 0; t < TW; ++t) {
         const float y = dgtot[t * 64 + cl];
         run += (FWD ? (t >= w) : (t < w)) ? y : 0.f;
       }
@@ -533,8 +534,8 @@ struct BwdSegments {
   int nseg, seg_len;
 };
 
-template <int NG, bool BIDIR, bool SEG>
-__global__ __launch_bounds__(512) void gla_backward_mfma_kernel(
+template <int NG, bool BIDIR, bool SEG, int TW>
+__global__ __launch_bounds__(64 * TW, 2) void gla_backward_mfma_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
     const uint16_t* __restrict__ gf, const uint16_t* __restrict__ gb, const uint16_t* __restrict__ d_o,
     uint16_t* __restrict__ dq, uint16_t* __restrict__ dk, uint16_t* __restrict__ dv, uint16_t* __restrict__ dgf,
@@ -571,7 +572,7 @@ __global__ __launch_bounds__(512) void gla_backward_mfma_kernel(
     const BwdNext first{s0, s0.gf, s0.L};
     issue_bwd_gate_loads<NG>(first, w, r, h, ld);
     issue_bwd_row_loads<true, NG>(first, w, r, h, ld);
-    bwd_cumulate_gates<true, NG>(ld, w, lane, lds, G);
+    bwd_cumulate_gates<true, NG, TW>(ld, w, lane, lds, G);
     lds_barrier();
   }
   for (int slab = blockIdx.x; slab < nslabs; slab += gridDim.x) {
@@ -584,13 +585,13 @@ __global__ __launch_bounds__(512) void gla_backward_mfma_kernel(
     u32x4_t keepq[NG], keepk[NG];
     bool ok;
     if constexpr (BIDIR) {
-      ok = bwd_direction<true, true, false, NG, SEG>(sl, sl.L, ntiles, w, lane, lds, s, dvacc, keepq, keepk, ld, second, G);
+      ok = bwd_direction<true, true, false, NG, SEG, TW>(sl, sl.L, ntiles, w, lane, lds, s, dvacc, keepq, keepk, ld, second, G);
       if (ok) {
-        ok = bwd_direction<false, false, true, NG, SEG>(sl, sl.L, ntiles, w, lane, lds, s, dvacc, keepq, keepk, ld,
+        ok = bwd_direction<false, false, true, NG, SEG, TW>(sl, sl.L, ntiles, w, lane, lds, s, dvacc, keepq, keepk, ld,
                                                         next_first, G);
       }
     } else {  // the causal op: the forward direction alone, first and last at once
-      ok = bwd_direction<true, true, true, NG, SEG>(sl, sl.L, ntiles, w, lane, lds, s, dvacc, keepq, keepk, ld,
+      ok = bwd_direction<true, true, true, NG, SEG, TW>(sl, sl.L, ntiles, w, lane, lds, s, dvacc, keepq, keepk, ld,
                                                     next_first, G);
     }
     // a direction that left early has neither issued the loads of the slab that follows nor prepared its gates
@@ -598,7 +599,7 @@ __global__ __launch_bounds__(512) void gla_backward_mfma_kernel(
       lds_barrier();  // a wave that has left must not touch the gate totals the others still read
       issue_bwd_gate_loads<NG>(next_first, w, r, h, ld);
       issue_bwd_row_loads<true, NG>(next_first, w, r, h, ld);
-      bwd_cumulate_gates<true, NG>(ld, w, lane, lds, G);
+      bwd_cumulate_gates<true, NG, TW>(ld, w, lane, lds, G);
       lds_barrier();
     }
     if (SEG) {  // one flag per sequence, cleared by the segment scan: any segment out of range gives the sequence away
@@ -760,6 +761,38 @@ size_t gla_backward_mfma_workspace(int B, int H, int L, int Dk, int Dv) {
   return n * ((2 * (size_t)kGlaStateFloats + kBwdStateElems + 128) * sizeof(float) + 3 * (size_t)kBwdStateElems * 2);
 }
 
+struct BwdLaunch {
+  const void *q, *k, *v, *gf, *gb, *d_o;
+  void *dq, *dk, *dv, *dgf, *dgb;
+  int* flags;
+  int nslabs, L;
+  float s;
+  BwdSegments sg;
+  int num_cu;
+  hipStream_t stream;
+};
+template <int NG, bool BIDIR, bool SEG, int TW>
+static int launch_bwd_t(const BwdLaunch& l) {
+  static bool done[64] = {};
+  auto* kernel = gla_backward_mfma_kernel<NG, BIDIR, SEG, TW>;
+  if (!allow_lds(reinterpret_cast<const void*>(kernel), BwdLds<TW>::total, done)) return -5;
+  const int most = l.num_cu * (kBwdTiles / TW);
+  hipLaunchKernelGGL(kernel, dim3(l.nslabs < most ? l.nslabs : most), dim3(64 * TW), BwdLds<TW>::total, l.stream,
+                     (const uint16_t*)l.q, (const uint16_t*)l.k, (const uint16_t*)l.v, (const uint16_t*)l.gf, (const uint16_t*)l.gb,
+                     (const uint16_t*)l.d_o, (uint16_t*)l.dq, (uint16_t*)l.dk, (uint16_t*)l.dv, (uint16_t*)l.dgf, (uint16_t*)l.dgb,
+                     l.flags, l.nslabs, l.L, l.s, l.sg);
+  return hipGetLastError() == hipSuccess ? 0 : -5;
+}
+// Slabs of up to 64 and up to 128 tokens get workgroups of two and four waves, four and two of them to a CU: in one of eight, the
+// waves without a tile idle and nothing runs beside the loads.  us, eight waves / as many as the slab has tiles: Dk 64: 2010 slabs of
+// 57 tokens 119 / 62, 1200 of 128 113 / 83, 3 of 49 20 / 16; Dk 32: 91 / 37, 82 / 51, 16 / 13.
+template <int NG, bool BIDIR>
+static int launch_bwd(const BwdLaunch& l, bool seg, int tokens) {
+  if (seg) return tokens <= 128 ? launch_bwd_t<NG, BIDIR, true, 4>(l) : launch_bwd_t<NG, BIDIR, true, 8>(l);
+  if (tokens <= 64) return launch_bwd_t<NG, BIDIR, false, 2>(l);
+  return tokens <= 128 ? launch_bwd_t<NG, BIDIR, false, 4>(l) : launch_bwd_t<NG, BIDIR, false, 8>(l);
+}
+
 // flags: one int per (batch, head) sequence, written by every launch: 1 = not computed here (gates out of range)
 int launch_gla_backward_mfma(const void* q, const void* k, const void* v, const void* gf, const void* gb,
                              const void* d_o, void* dq, void* dk, void* dv, void* dgf, void* dgb, int* flags,
@@ -770,16 +803,6 @@ int launch_gla_backward_mfma(const void* q, const void* k, const void* v, const 
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return -5;
   if (!attr_done_dev[dev]) {
-    const void* kernels[8] = {reinterpret_cast<const void*>(gla_backward_mfma_kernel<4, true, false>),
-                              reinterpret_cast<const void*>(gla_backward_mfma_kernel<2, true, false>),
-                              reinterpret_cast<const void*>(gla_backward_mfma_kernel<4, false, false>),
-                              reinterpret_cast<const void*>(gla_backward_mfma_kernel<2, false, false>),
-                              reinterpret_cast<const void*>(gla_backward_mfma_kernel<4, true, true>),
-                              reinterpret_cast<const void*>(gla_backward_mfma_kernel<2, true, true>),
-                              reinterpret_cast<const void*>(gla_backward_mfma_kernel<4, false, true>),
-                              reinterpret_cast<const void*>(gla_backward_mfma_kernel<2, false, true>)};
-    for (const void* kf : kernels)
-      if (hipFuncSetAttribute(kf, hipFuncAttributeMaxDynamicSharedMemorySize, kBwdLdsTotal) != hipSuccess) return -5;
     int n = 0;
     if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return -5;
     num_cu_dev[dev] = n > 0 ? n : 256;
@@ -817,27 +840,10 @@ int launch_gla_backward_mfma(const void* q, const void* k, const void* v, const 
     sg = BwdSegments{sp, rp, rpt, carry, gla_segments(L), gla_segment_len(L)};
     nslabs = B * H * sg.nseg;
   }
-  const int grid = nslabs < num_cu_dev[dev] ? nslabs : num_cu_dev[dev];
-#define VIG_BWD_LAUNCH(NG, BIDIR, SEG)                                                                          \
-  hipLaunchKernelGGL((gla_backward_mfma_kernel<NG, BIDIR, SEG>), dim3(grid), dim3(512), kBwdLdsTotal, stream,    \
-                     (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, (const uint16_t*)gf,            \
-                     (const uint16_t*)gb, (const uint16_t*)d_o, (uint16_t*)dq, (uint16_t*)dk, (uint16_t*)dv,     \
-                     (uint16_t*)dgf, (uint16_t*)dgb, flags, nslabs, L, s, sg)
-#define VIG_BWD_LAUNCH_SEG(NG, BIDIR) \
-  do {                                \
-    if (seg) VIG_BWD_LAUNCH(NG, BIDIR, true); \
-    else VIG_BWD_LAUNCH(NG, BIDIR, false);    \
-  } while (0)
-  if (gb) {
-    if (Dk == 64) VIG_BWD_LAUNCH_SEG(4, true);
-    else VIG_BWD_LAUNCH_SEG(2, true);
-  } else {
-    if (Dk == 64) VIG_BWD_LAUNCH_SEG(4, false);
-    else VIG_BWD_LAUNCH_SEG(2, false);
-  }
-#undef VIG_BWD_LAUNCH_SEG
-#undef VIG_BWD_LAUNCH
-  return hipGetLastError() == hipSuccess ? 0 : -5;
+  const BwdLaunch l{q, k, v, gf, gb, d_o, dq, dk, dv, dgf, dgb, flags, nslabs, L, s, sg, num_cu_dev[dev], stream};
+  const int tokens = seg ? sg.seg_len : L;
+  if (gb) return Dk == 64 ? launch_bwd<4, true>(l, seg, tokens) : launch_bwd<2, true>(l, seg, tokens);
+  return Dk == 64 ? launch_bwd<4, false>(l, seg, tokens) : launch_bwd<2, false>(l, seg, tokens);
 }
 
 }  // namespace vig
