@@ -120,18 +120,6 @@ __device__ __forceinline__ uint32_t keep_bits(int r, int h) {
   const uint32_t K = FWD ? (2u << r) - 1u : 0xFFFFFFFFu << r;
   return K >> (4 * h);
 }
-// 0xFFFF for each of the two token slots of dword X of k-step T (tokens jmap(T, h, 2X) and the next one) that is kept
-template <int T, int X>
-__device__ __forceinline__ uint32_t keep_mask(uint32_t kh) {
-  constexpr unsigned j0 = 16 * T + 8 * (X >> 1) + 2 * (X & 1);
-  const uint32_t lo = (uint32_t)__builtin_amdgcn_sbfe((int)kh, j0, 1), hi = (uint32_t)__builtin_amdgcn_sbfe((int)kh, j0 + 1, 1);
-  return __builtin_amdgcn_perm(hi, lo, 0x07060100u);
-}
-template <int T>
-__device__ __forceinline__ u32x4_t keep_masks(uint32_t kh) {
-  return u32x4_t{keep_mask<T, 0>(kh), keep_mask<T, 1>(kh), keep_mask<T, 2>(kh), keep_mask<T, 3>(kh)};
-}
-
 // tile-local cumulative gates of one direction: G[p][4g+m] = channel 8*NG*h + 8g + 2m + p of token r
 template <bool FWD>
 __device__ __forceinline__ void cumulative_gates(const uint32_t (&gD)[2][8], int r, int h, f32x16_t (&G)[2]) {
@@ -337,6 +325,12 @@ __device__ __forceinline__ void walk_tiles(char* lds, const TileLds<NG>& lay, in
   }
 }
 
+// power of two that brings a direction's states to at most 2^14, from the maxima that the scan left
+__device__ __forceinline__ int state_shift(float top) {
+  const int ex = (int)((__float_as_uint(wave_max(top)) >> 23) & 0xffu) - 127;  // (inf / nan: 128, the result is not finite anyway)
+  return __builtin_amdgcn_readfirstlane(max(ex - 13, -30));
+}
+
 // Long sequences: what the state entering the segment (from the left for the forward direction, from the right for
 // the reverse one) adds to this wave's tile,  O^T[pv] += S_in^T q^,  q^ anchored at the segment's edge.  The slot holds
 // S_in in the matrix cores' register order: unit (pk, pv, g), lane, m is S_in[k channel 32h + 8g + 2m + pk][v column of
@@ -344,7 +338,7 @@ __device__ __forceinline__ void walk_tiles(char* lds, const TileLds<NG>& lay, in
 // directly while the scan saw nothing above 2^14, scaled by a power of two otherwise (`shift`, wave-uniform), the
 // product then passing through an accumulator of its own.  extra: power of two the result still needs (general form).
 template <int NG, bool FWD>
-__device__ __forceinline__ void apply_state(const float* slot, const float* top16, const char* dtab_edge, bool cross,
+__device__ __forceinline__ void apply_state(const float* slot, int shift, const char* dtab_edge, bool cross,
                                             int lane, int extra, u32x4_t (&qh)[NG], f32x16_t (&O)[2]) {
   if (cross) {  // q^ over the segment's edge tile (tile 0 forward, the last one reverse)
 #pragma unroll
@@ -354,10 +348,6 @@ __device__ __forceinline__ void apply_state(const float* slot, const float* top1
       for (int m = 0; m < 4; ++m) qh[g][m] = mul_f16x2(qh[g][m], d[m]);
     }
   }
-  float top = lane < kGlaScanMaxima ? top16[lane] : 0.f;
-  top = wave_max(top);
-  const int ex = (int)((__float_as_uint(top) >> 23) & 0xffu) - 127;  // (inf / nan: 128, the result is not finite anyway)
-  const int shift = __builtin_amdgcn_readfirstlane(max(ex - 13, -30));
   // (directly down to a top of 2^-4: smaller entries keep their weight relative to it in fp16's subnormal range)
   if (shift <= 0 && shift >= -17 && extra == 0) {
     // (two k-steps' worth of the state in flight at a time: sixteen registers)
@@ -385,18 +375,16 @@ __device__ __forceinline__ void apply_state(const float* slot, const float* top1
 #pragma unroll
   for (int pv = 0; pv < 2; ++pv) {
     f32x16_t acc = {0.f};
-    f32x4_t a[NG], b[NG];
+#pragma unroll 1
+    for (int g = 0; g < NG; ++g) {  // (rare: few registers rather than many loads in flight)
+      const f32x4_t a = *reinterpret_cast<const f32x4_t*>(slot + (((0 * 2 + pv) * 4 + g) * 64 + lane) * 4);
+      const f32x4_t b = *reinterpret_cast<const f32x4_t*>(slot + (((1 * 2 + pv) * 4 + g) * 64 + lane) * 4);
+      u32x4_t f, q = qh[0];
 #pragma unroll
-    for (int g = 0; g < NG; ++g) {
-      a[g] = *reinterpret_cast<const f32x4_t*>(slot + (((0 * 2 + pv) * 4 + g) * 64 + lane) * 4);
-      b[g] = *reinterpret_cast<const f32x4_t*>(slot + (((1 * 2 + pv) * 4 + g) * 64 + lane) * 4);
-    }
+      for (int j = 1; j < NG; ++j) q = g == j ? qh[j] : q;
 #pragma unroll
-    for (int g = 0; g < NG; ++g) {
-      u32x4_t f;
-#pragma unroll
-      for (int m = 0; m < 4; ++m) f[m] = pack_f16x2(a[g][m] * pre, b[g][m] * pre);
-      acc = mfma_f16(f, qh[g], acc);
+      for (int m = 0; m < 4; ++m) f[m] = pack_f16x2(a[m] * pre, b[m] * pre);
+      acc = mfma_f16(f, q, acc);
     }
 #pragma unroll
     for (int i = 0; i < 16; ++i) O[pv][i] = __builtin_fmaf(acc[i], post, O[pv][i]);
@@ -514,10 +502,28 @@ __device__ __forceinline__ void locality_gate_epilogue(f32x16_t O0, f32x16_t O1,
     }
 }
 
-// Everything one wave does for its slab.  The fp16 form (GENERAL false) returns true, for every wave of the workgroup
-// alike and before anything is stored, when some tile of the slab is outside its range.
+// The kernel's argument block as the hardware lays it out (every argument at its natural alignment).
+struct TileKernArgs {
+  const uint16_t *q, *k, *v, *gf, *gb;
+  uint16_t* o;
+  TileGeo geo;
+  float oscale;
+  const float* gate_w;
+};
+
+static_assert(offsetof(TileKernArgs, geo) == 6 * sizeof(void*) && offsetof(TileKernArgs, oscale) == 48 + sizeof(TileGeo) &&
+                  offsetof(TileKernArgs, gate_w) == 48 + sizeof(TileGeo) + 8 && alignof(TileGeo) == 8,
+              "TileKernArgs has to mirror the parameter list of gla_tile_kernel");
+
+template <int NG, bool BIDIR, bool PITCHED, bool GATE, bool CHAIN>
+__device__ void tile_pass_general(const TileKernArgs* ka_in);
+
+// Everything one wave does for its slab.  When some tile of the slab is outside the fp16 form's range (GENERAL false), every wave
+// of the workgroup, before anything is stored, runs the general form (ka: the kernel's argument block) and ends there: a call
+// that came back would keep the accumulators alive across it, and the compiler then kept sixteen of them in per-lane memory
+// throughout, walks included (long sequences at Dk 32, 144 of 784 tokens: this kernel 38.7 -> 23.5 us).
 template <int NG, bool BIDIR, bool PITCHED, bool GENERAL, bool GATE, bool CHAIN>
-__device__ __forceinline__ bool tile_pass(const TileCtx& cx) {
+__device__ __forceinline__ void tile_pass(const TileCtx& cx, const TileKernArgs* ka) {
   const int lane = cx.lane, r = lane & 31, h = lane >> 5;
   const int ti = cx.ti, NT = cx.NT;
   const TileLds<NG> lay(NT, GATE ? gate_stage_bytes(cx.gw, cx.gh) : 0);
@@ -542,6 +548,8 @@ __device__ __forceinline__ bool tile_pass(const TileCtx& cx) {
     issue_raw_tile<NG>(cx.k, 0, r, h, rawk);
   }
   if (BIDIR) issue_tdwords<0, 2, NG>(cx.gb, r, h, gDb);
+  float top_f = 0.f, top_b = 0.f;
+  if (CHAIN && lane < kGlaScanMaxima) top_f = cx.state_top[lane], top_b = BIDIR ? cx.state_top[kGlaScanMaxima + lane] : 0.f;
   // ---- magnitudes (Gram matrices of the raw rows); values: bf16 pairs -> fp16 pairs, published ----
   int eq = 0, ek = 0, ev = 0;
   bool veto = false;
@@ -649,11 +657,15 @@ __device__ __forceinline__ bool tile_pass(const TileCtx& cx) {
       for (int pv = 0; pv < 2; ++pv) vf[t][pv] = *reinterpret_cast<const u32x4_t*>(unit_ptr(vregion, 2 * t + pv, lane));
     apply_values16(p16, vf, O);
   }
+  const int shift_f = CHAIN ? state_shift(top_f) : 0, shift_b = CHAIN && BIDIR ? state_shift(top_b) : 0;
   if (!GENERAL && lane == 0) guard[4 * ti] = veto ? 1.0f : 0.0f;
   lds_barrier();  // every tile's k^, V and decays are visible
   if (!GENERAL) {
     const float mine = lane < NT ? guard[4 * lane] : 0.0f;
-    if (__builtin_amdgcn_ballot_w64(mine != 0.0f) != 0) return true;
+    if (__builtin_amdgcn_ballot_w64(mine != 0.0f) != 0) {
+      tile_pass_general<NG, BIDIR, PITCHED, GATE, CHAIN>(ka);
+      __builtin_amdgcn_endpgm();
+    }
   }
   // (from here on a wave holds what the others wait for, its slot on the CU included: ahead of the waves of the other
   // workgroup that are still preparing operands; measured 3 % on the Dk = 32 layer shape, nothing at Dk = 64)
@@ -664,18 +676,18 @@ __device__ __forceinline__ bool tile_pass(const TileCtx& cx) {
   walk_tiles<NG, true>(lds, lay, ti, NT, lane_w, qhf, O);
   // (general form: the state's term joins accumulators that carry 2^-(eq + ek + ev); q^ carries 2^-eq itself)
   if (CHAIN)
-    apply_state<NG, true>(cx.state_in, cx.state_top, lds + lay.d + 16 * NG * (lane_w >> 5), ti > 0, lane_w,
+    apply_state<NG, true>(cx.state_in, shift_f, lds + lay.d + 16 * NG * (lane_w >> 5), ti > 0, lane_w,
                           GENERAL ? -(ek + ev) : 0, qhf, O);
   if (BIDIR) walk_tiles<NG, false>(lds, lay, ti, NT, lane_w, qhb, O);
   if (CHAIN && BIDIR)
-    apply_state<NG, false>(cx.state_in + kGlaStateFloats, cx.state_top + kGlaScanMaxima,
+    apply_state<NG, false>(cx.state_in + kGlaStateFloats, shift_b,
                            lds + lay.d + (NT + NT - 1) * 128 + 16 * NG * (lane_w >> 5), ti < NT - 1, lane_w,
                            GENERAL ? -(ek + ev) : 0, qhb, O);
   float os = cx.oscale;
   if (GENERAL) os *= __builtin_amdgcn_exp2f((float)(eq + ek + ev));
   if (GATE) {
     locality_gate_epilogue(O[0], O[1], os, lds, cx.gate_w, cx.o, cx.gw, cx.gh, ti, NT, lane_w);
-    return false;
+    return;
   }
   // ---- store: lane (r, h) holds channels [32h, 32h + 32) of token r; rows beyond the sequence are dropped ----
 #pragma unroll
@@ -685,7 +697,6 @@ __device__ __forceinline__ bool tile_pass(const TileCtx& cx) {
     for (int m = 0; m < 4; ++m) x[m] = pack_bf16x2(O[0][4 * gq + m] * os, O[1][4 * gq + m] * os);
     __builtin_amdgcn_raw_buffer_store_b128(x, cx.o, (unsigned)(lane_w & 31) * 128u + 64u * (lane_w >> 5) + 16u * gq, 0, 0);
   }
-  return false;
 }
 
 template <int NG, bool BIDIR, bool PITCHED, bool GATE, bool CHAIN>
@@ -730,19 +741,6 @@ __device__ __forceinline__ TileCtx make_tile_ctx(const uint16_t* q, const uint16
   return cx;
 }
 
-// The kernel's argument block as the hardware lays it out (every argument at its natural alignment).
-struct TileKernArgs {
-  const uint16_t *q, *k, *v, *gf, *gb;
-  uint16_t* o;
-  TileGeo geo;
-  float oscale;
-  const float* gate_w;
-};
-
-static_assert(offsetof(TileKernArgs, geo) == 6 * sizeof(void*) && offsetof(TileKernArgs, oscale) == 48 + sizeof(TileGeo) &&
-                  offsetof(TileKernArgs, gate_w) == 48 + sizeof(TileGeo) + 8 && alignof(TileGeo) == 8,
-              "TileKernArgs has to mirror the parameter list of gla_tile_kernel");
-
 // The general form as a function of its own: its register needs stay out of the fp16 form's allocation.  It reads
 // the kernel's arguments from the argument block itself (ka: the kernel's own kernarg segment pointer; the builtin
 // yields null inside a called function): handed over as parameters, the geometry would need a copy in per-lane
@@ -762,7 +760,7 @@ __device__ __noinline__ void tile_pass_general(const TileKernArgs* ka_in) {
   const TileGeo geo = ka->geo;
   const TileCtx cx = make_tile_ctx<NG, BIDIR, PITCHED, GATE, CHAIN>(ka->q, ka->k, ka->v, ka->gf, ka->gb, ka->o, geo,
                                                                      ka->oscale, ka->gate_w, lds);
-  tile_pass<NG, BIDIR, PITCHED, true, GATE, CHAIN>(cx);
+  tile_pass<NG, BIDIR, PITCHED, true, GATE, CHAIN>(cx, nullptr);
 #endif
 }
 
@@ -776,13 +774,9 @@ __global__ __launch_bounds__(1024, 4) void gla_tile_kernel(const uint16_t* __res
                                                           TileGeo geo, float oscale,
                                                           const float* __restrict__ gate_w) {
   extern __shared__ __align__(16) char lds[];
-  bool redo = true;
-  if (!geo.wide) {
-    const TileCtx cx = make_tile_ctx<NG, BIDIR, PITCHED, GATE, CHAIN>(q, k, v, gf, gb, o, geo, oscale, gate_w, lds);
-    redo = tile_pass<NG, BIDIR, PITCHED, false, GATE, CHAIN>(cx);
-  }
-  if (redo)
-    tile_pass_general<NG, BIDIR, PITCHED, GATE, CHAIN>((const TileKernArgs*)__builtin_amdgcn_kernarg_segment_ptr());
+  const TileKernArgs* ka = (const TileKernArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+  const TileCtx cx = make_tile_ctx<NG, BIDIR, PITCHED, GATE, CHAIN>(q, k, v, gf, gb, o, geo, oscale, gate_w, lds);
+  tile_pass<NG, BIDIR, PITCHED, false, GATE, CHAIN>(cx, ka);
 }
 
 // The general form alone, for launches whose caller knows the gates to be strong: with 256 registers per wave (one
@@ -798,7 +792,7 @@ __global__ __launch_bounds__(512, 2) void gla_tile_wide_kernel(const uint16_t* _
                                                                const float* __restrict__ gate_w) {
   extern __shared__ __align__(16) char lds[];
   const TileCtx cx = make_tile_ctx<NG, BIDIR, PITCHED, GATE, CHAIN>(q, k, v, gf, gb, o, geo, oscale, gate_w, lds);
-  tile_pass<NG, BIDIR, PITCHED, true, GATE, CHAIN>(cx);
+  tile_pass<NG, BIDIR, PITCHED, true, GATE, CHAIN>(cx, nullptr);
 }
 
 constexpr int kTileMaxLds = 160 * 1024;

@@ -155,6 +155,19 @@ __device__ __forceinline__ u32x4_t tri_frag(int t, int it, int r, int h) {
   return f;
 }
 
+// 0xFFFF for each of the two token slots of dword X of k-step T (tokens jmap(T, h, 2X) and the next one) that a bit
+// mask of tokens, shifted right by 4h, keeps
+template <int T, int X>
+__device__ __forceinline__ uint32_t keep_mask(uint32_t kh) {
+  constexpr unsigned j0 = 16 * T + 8 * (X >> 1) + 2 * (X & 1);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_sbfe((int)kh, j0, 1), hi = (uint32_t)__builtin_amdgcn_sbfe((int)kh, j0 + 1, 1);
+  return __builtin_amdgcn_perm(hi, lo, 0x07060100u);
+}
+template <int T>
+__device__ __forceinline__ u32x4_t keep_masks(uint32_t kh) {
+  return u32x4_t{keep_mask<T, 0>(kh), keep_mask<T, 1>(kh), keep_mask<T, 2>(kh), keep_mask<T, 3>(kh)};
+}
+
 template <int NG, int STRIDE = kKtStride>
 __device__ __forceinline__ void store_kt(uint16_t* kt, int row, int h, const u32x4_t (&kh)[NG]) {
 #pragma unroll
