@@ -74,6 +74,8 @@ size_t gla_backward_f32_states(int B, int H, int L);
 int launch_gla_backward_f32(const void* q, const void* k, const void* v, const void* gf, const void* gb, const void* d_o,
                             void* dq, void* dk, void* dv, void* dgf, void* dgb, int* flags, float* states, int B, int H, int L,
                             int Dk, float s, hipStream_t stream);
+// bf16: contributions and decays of every segment of seg_len tokens, and with q and d_o the gradient states (gla_states.hip)
+int launch_gla_states(const GlaArgs& a, int seg_len, int nseg, float* slots, const void* q, const void* d_o, float* grad_slots);
 // chains the slots of a state pass in place (gla_segment_scan_kernel, no state in or out)
 int launch_gla_segment_scan(float* slots, int nseq, int nseg, int ndir, int ng, hipStream_t stream);
 
