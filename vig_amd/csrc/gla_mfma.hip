@@ -943,76 +943,81 @@ __global__ __launch_bounds__(512) void gla_mfma_kernel(const uint16_t* __restric
 
 // Chains the segments of every sequence: in place, the workspace slot of segment s (its own contribution U_s and
 // decay D_s) is replaced by the state entering it,  S_in(s') = D_s * S_in(s) + U_s  with s' the next segment in the
-// direction's walk order.  One thread per state element; all accesses are coalesced (unit order is kept).  The
-// contributions and decays of kBatch segments are fetched together, so that the serial part is arithmetic only; a batch
-// fetches whether or not the sequence has that many segments, so the launch picks the smallest of 2, 4, 8 and 24 that holds
-// them (24: a 4096-token sequence in one round).  144 sequences of 784 tokens, Dk 32, whole op: 24 always 75.2 us, chosen 63.8.
+// direction's walk order.  A thread holds the four consecutive elements of one lane and unit (NG blocks of four units per
+// sequence and direction: quads beyond Dk/16 carry no channel).  The contributions and decays of kBatch segments are fetched
+// together, so that the serial part is arithmetic only; a batch fetches whether or not the sequence has that many segments,
+// so the launch picks the smallest of 2, 4, 8 and 12 that holds them, or 12 at a time.
 // The causal op may start from a caller's state and hand the last one back (init / final: fp32 [nseq, Dk, Dv] row-major,
-// null: zero / not wanted; one direction only): the thread of state element e is also the one that knows its row
+// null: zero / not wanted; one direction only): the thread of a state element is also the one that knows its row
 // (k channel) and column (v channel).
-// maxima (null: not wanted): [nseq][2 directions][kGlaScanMaxima], the largest |state entering a segment| each block saw.
+// maxima (null: not wanted): [nseq][2 directions][kGlaScanMaxima], the largest |state entering a segment| each wave saw.
+// Whole op, us, against one thread per element (half the blocks without channels at Dk 32, two loads of 4 bytes a segment): Dk 32:
+// 144 sequences of 784 tokens 48.2 -> 44.3, 147 of 534 35.1 -> 31.0, 45 of 1679 32.4 -> 31.2; Dk 64: 147 of 534 49.5 -> 47.0.
 template <int kBatch>
 __global__ __launch_bounds__(256) void gla_segment_scan_kernel(float* state_ws, int nseq, int nseg, int ndir, int ng,
                                                                const float* __restrict__ init, float* __restrict__ final,
                                                                float* __restrict__ maxima) {
-  static_assert(64 * 64 / 256 == kGlaScanMaxima, "one partial maximum per block of the scan");
-  __shared__ float wave_top[4];
-  const int e = blockIdx.x * 256 + threadIdx.x;  // element in unit order: ((u*64 + lane)*4 + m)
+  static_assert(4 * 4 == kGlaScanMaxima, "one partial maximum per wave of up to four blocks");
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, h = lane >> 5;
   const int seq = blockIdx.y / ndir, dir = blockIdx.y % ndir;
   if (seq >= nseq) return;
-  const int m = e & 3, lane = (e >> 2) & 63, u = e >> 8;
-  const int pk = u >> 3, cq = u & 3, h = lane >> 5;
-  if (cq >= ng) {  // register quads beyond Dk/16 carry no channel (a whole block at a time: u is block-uniform)
-    if (maxima && threadIdx.x == 0) maxima[((size_t)seq * 2 + dir) * kGlaScanMaxima + blockIdx.x] = 0.f;
-    return;
-  }
-  const int ch = 8 * ng * h + 8 * cq + 2 * m + pk;
-  float S = 0.f, top = 0.f;
+  const int cq = blockIdx.x, pk = wave >> 1, pv = wave & 1, u = wave * 4 + cq;  // unit (pk, pv, cq)
+  const int e = (u * 64 + lane) * 4, ch = 8 * ng * h + 8 * cq;  // element m: channel ch + 2 m + pk
+  f32x4_t S = {0.f, 0.f, 0.f, 0.f};
+  float top = 0.f;
   // column of the state held by (lane, unit): the v channel the accumulator column r of output tile pv belongs to
-  const int vch = 2 * cpair<4>(lane & 31) + ((u >> 2) & 1);
-  const size_t rc = ((size_t)seq * (16 * ng) + ch) * 64 + vch;
-  if (init) S = init[rc];
+  const int vch = 2 * cpair<4>(lane & 31) + pv;
+  const size_t rc = ((size_t)seq * (16 * ng) + ch + pk) * 64 + vch;
+  if (init)
+#pragma unroll
+    for (int m = 0; m < 4; ++m) S[m] = init[rc + 128 * m];
   for (int i0 = 0; i0 < nseg; i0 += kBatch) {
-    float us[kBatch], ds[kBatch];
+    f32x4_t us[kBatch], ds[kBatch];
 #pragma unroll
     for (int j = 0; j < kBatch; ++j) {
       const int i = min(i0 + j, nseg - 1);
       const int seg = dir == 0 ? i : nseg - 1 - i;
       const float* slot = state_ws + (((size_t)seq * nseg + seg) * 2 + dir) * kStateFloats;
-      us[j] = slot[e];
-      ds[j] = slot[64 * 64 + ch];
+      us[j] = *reinterpret_cast<const f32x4_t*>(slot + e);
+      const f32x4_t d0 = *reinterpret_cast<const f32x4_t*>(slot + 64 * 64 + ch), d1 = *reinterpret_cast<const f32x4_t*>(slot + 64 * 64 + ch + 4);
+      ds[j] = pk ? f32x4_t{d0[1], d0[3], d1[1], d1[3]} : f32x4_t{d0[0], d0[2], d1[0], d1[2]};
     }
 #pragma unroll
     for (int j = 0; j < kBatch; ++j) {
       const int i = i0 + j;
       if (i < nseg) {
         const int seg = dir == 0 ? i : nseg - 1 - i;
-        state_ws[(((size_t)seq * nseg + seg) * 2 + dir) * kStateFloats + e] = S;
-        top = fmaxf(top, fabsf(S));
-        S = __builtin_fmaf(ds[j], S, us[j]);
+        *reinterpret_cast<f32x4_t*>(state_ws + (((size_t)seq * nseg + seg) * 2 + dir) * kStateFloats + e) = S;
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+          top = fmaxf(top, fabsf(S[m]));
+          S[m] = __builtin_fmaf(ds[j][m], S[m], us[j][m]);
+        }
       }
     }
   }
-  if (final) final[rc] = S;
-  if (maxima) {  // (uniform: every thread of the block is still here)
+  if (final)
+#pragma unroll
+    for (int m = 0; m < 4; ++m) final[rc + 128 * m] = S[m];
+  if (maxima) {
 #pragma unroll
     for (int s = 32; s >= 1; s >>= 1) top = fmaxf(top, __shfl_xor(top, s, 64));
-    if ((threadIdx.x & 63) == 0) wave_top[threadIdx.x >> 6] = top;
-    __syncthreads();
-    if (threadIdx.x == 0)
-      maxima[((size_t)seq * 2 + dir) * kGlaScanMaxima + blockIdx.x] =
-          fmaxf(fmaxf(wave_top[0], wave_top[1]), fmaxf(wave_top[2], wave_top[3]));
+    float* mine = maxima + ((size_t)seq * 2 + dir) * kGlaScanMaxima + 4 * cq + wave;
+    if (lane == 0) {
+      *mine = top;
+      if (ng == 2) mine[8] = 0.f;
+    }
   }
 }
 
 static void launch_scan(float* slots, int nseq, int nseg, int ndir, int ng, const float* init, float* final, float* maxima,
                         hipStream_t stream) {
-  const dim3 grid(64 * 64 / 256, nseq * ndir), block(256);
+  const dim3 grid(ng, nseq * ndir), block(256);
 #define VIG_SCAN(N) hipLaunchKernelGGL(gla_segment_scan_kernel<N>, grid, block, 0, stream, slots, nseq, nseg, ndir, ng, init, final, maxima)
   if (nseg <= 2) VIG_SCAN(2);
   else if (nseg <= 4) VIG_SCAN(4);
   else if (nseg <= 8) VIG_SCAN(8);
-  else VIG_SCAN(24);
+  else VIG_SCAN(12);
 #undef VIG_SCAN
 }
 
