@@ -43,3 +43,18 @@ def test_more_slabs_than_workgroups(B, H, L, Dk):
         assert torch.equal(g[strong], e[strong])
     keep = ~strong
     _check_mfma([g[keep] for g in got], [f64(e[keep]) for e in exact], q[keep].cpu())
+
+
+@pytest.mark.parametrize("B,H,L,Dk,both", [(1, 2, 6200, 32, True), (1, 1, 12400, 64, True), (1, 1, 6200, 32, False), (2, 3, 513, 32, True),
+                                           (1, 3, 385, 32, True), (1, 2, 640, 32, False), (1, 2, 385, 64, True)])
+def test_segments(B, H, L, Dk, both):
+    """Long sequences at the edges of their segmentations: more segments than one chunk of the scan holds, last segments of one
+    token and of whole tiles."""
+    announce(f"backward segments B{B} H{H} L{L} Dk{Dk} both={both}")
+    q, k, v, gf, gb = (t.cuda() for t in make_gla_inputs(B, H, L, Dk, 64, seed=90, dtype=torch.bfloat16))
+    do = _do(v.shape, 6, torch.bfloat16).cuda()
+    gb, out = (gb, 0.5) if both else (None, 1.0)
+    want = vig_amd.gla_bidir_backward(q, k, v, gf, gb, do, out_scale=out, exact=True)
+    got = vig_amd.gla_bidir_backward(q, k, v, gf, gb, do, out_scale=out)
+    n = 5 if both else 4
+    _check_mfma(got[:n], [f64(t) for t in want[:n]], q.cpu())

@@ -319,8 +319,9 @@ int launch_gla_backward(const void* q, const void* k, const void* v, const void*
   if (!exact && gla_backward_mfma_supported(B, H, L, Dk, Dv, io_dtype, gate_dtype, g_bwd != nullptr)) {
     int* flags = reinterpret_cast<int*>((float*)workspace + recurrent_floats(B, H, L, Dk, Dv, g_bwd != nullptr));
     void* seg_ws = (char*)workspace + flags_end(B, H, L, Dk, Dv, g_bwd != nullptr);
-    const int rc = launch_gla_backward_mfma(q, k, v, g_fwd, g_bwd, d_o, dq, dk, dv, dg_fwd, dg_bwd, flags, seg_ws, B,
-                                            H, L, Dk, scale * out_scale, stream);
+    const int rc = launch_gla_backward_mfma(q, k, v, g_fwd, g_bwd, d_o, dq, dk, dv, dg_fwd, dg_bwd, flags, workspace,
+                                            recurrent_floats(B, H, L, Dk, Dv, g_bwd != nullptr) * sizeof(float), seg_ws,
+                                            gla_backward_mfma_workspace(B, H, L, Dk, Dv), B, H, L, Dk, scale * out_scale, stream);
     if (rc != 0) return rc;
     a.only_flagged = flags;  // slabs with gates beyond the matrix-core kernel's range
   }

@@ -1,5 +1,5 @@
 // Backward of the bidirectional GLA op on MFMA tiles (gfx950): bf16 tensors and gates, Dk in {32, 64}, Dv = 64.
-// L <= 256 is one slab per (batch, head); a longer sequence is cut into the forward's segments (<= 256 tokens), each
+// L <= 256 is one slab per (batch, head); a longer sequence is cut into segments (<= 256 tokens), each
 // handled like a slab plus three products with the states that link it to the other segments (see SEG below).
 //
 // Per direction the whole (batch, head) slab is one quadratic form (no chunk states): with G the inclusive
@@ -110,7 +110,6 @@ struct BwdSlab {
   const float* carry;             // [2 directions][2 partial sums][64]: q dq - k dk summed over the segments walked later
   int L;                          // tokens of this slab / segment
 };
-constexpr int kBwdStateElems = 64 * 64;
 
 // What a wave loads for one direction of one slab (its own 32-token tile), issued one phase ahead.
 template <int NG>
@@ -289,7 +288,7 @@ __device__ __forceinline__ bool bwd_direction(const BwdSlab& sl, int L, int ntil
       T = Tn;
     }
     if (SEG) {  // the state entering the segment: rows = the k channels of this lane's accumulator rows, over v
-      const uint16_t* sp = sl.sp + (FWD ? 0 : kBwdStateElems);
+      const uint16_t* sp = sl.sp + (FWD ? 0 : DK * 64);
       const bool row_ok = row_has_channel<NG>(r);
       const int row0 = row_ok ? 2 * cpair<NG>(r) : 0;
 #pragma unroll
@@ -391,16 +390,16 @@ __device__ __forceinline__ bool bwd_direction(const BwdSlab& sl, int L, int ntil
       }
     }
     if (SEG) {  // the gradient of the state leaving the segment, against this tile's k~ rows (dv) and v rows (dk)
-      const uint16_t* rpt = sl.rpt + (FWD ? 0 : kBwdStateElems);
+      const uint16_t* rpt = sl.rpt + (FWD ? 0 : DK * 64);
       const int vrow = 2 * cpair<4>(r);
 #pragma unroll
       for (int p = 0; p < 2; ++p)
 #pragma unroll
         for (int ks = 0; ks < NG; ++ks) {
-          const u32x4_t a = *reinterpret_cast<const u32x4_t*>(rpt + (vrow + p) * 64 + 16 * ks + 8 * h);
+          const u32x4_t a = *reinterpret_cast<const u32x4_t*>(rpt + (vrow + p) * DK + 16 * ks + 8 * h);
           dv[p] = mfma(a, row_frag(K, 32 * w + r, ks, h), dv[p]);
         }
-      const uint16_t* rp = sl.rp + (FWD ? 0 : kBwdStateElems);
+      const uint16_t* rp = sl.rp + (FWD ? 0 : DK * 64);
       const bool row_ok = row_has_channel<NG>(r);
       const int row0 = row_ok ? 2 * cpair<NG>(r) : 0;
 #pragma unroll
@@ -553,9 +552,9 @@ __global__ __launch_bounds__(64 * TW, 2) void gla_backward_mfma_kernel(
       const int seq = i / sg.nseg, seg = i - seq * sg.nseg;
       t0 = (size_t)seq * L + (size_t)seg * sg.seg_len;
       len = min(sg.seg_len, L - seg * sg.seg_len);
-      sl.sp = sg.sp + (size_t)i * 2 * kBwdStateElems;
-      sl.rp = sg.rp + (size_t)i * 2 * kBwdStateElems;
-      sl.rpt = sg.rpt + (size_t)i * 2 * kBwdStateElems;
+      sl.sp = sg.sp + (size_t)i * 2 * (16 * NG * 64);
+      sl.rp = sg.rp + (size_t)i * 2 * (16 * NG * 64);
+      sl.rpt = sg.rpt + (size_t)i * 2 * (16 * NG * 64);
       sl.carry = sg.carry + (size_t)i * 256;
     }
     const size_t bk = t0 * (16 * NG), bv = t0 * 64;
@@ -613,135 +612,109 @@ __global__ __launch_bounds__(64 * TW, 2) void gla_backward_mfma_kernel(
 // Links the segments of every (sequence, direction) for the backward.  Per segment s (walked in the direction's order)
 // it reads the forward's state pass (contribution U_s, decay D_s) and the gradient state pass (Q_s = sum over the
 // segment's tokens of (q e^{G})^T do, unscaled), and leaves
-//   sp   = sqrt(D_s) S_in(s),     S_in(s') = D_s S_in(s) + U_s   for the segment s' walked next,
+//   sp   = sqrt(D_s) S_in(s),     S_in(s') = S_out(s) = D_s S_in(s) + U_s   for the segment s' walked next,
 //   rp   = sqrt(D_s) R_out(s),    R_out(s) = Q_{s'} + D_{s'} R_out(s'),  zero for the segment walked last,
 //   rpt  = rp transposed,
-//   carry(s) = sum over the segments walked after s of rowsum_v(S_in Q - R_out U): what q dq - k dk adds up to there
-// (bf16 matrices in plain row-major order; carry in the first of two slots per channel, the second zero).
-// A thread holds the four state elements (k channels c, c+1) x (v columns x, x+1) of the passes' register order
-// (units pk = 0, 1 and pv = 0, 1 of one register quad cq, lane, register m), so that its bf16 results leave as
-// 4-byte words: whole 128-byte rows of sp and rp per 32 lanes, 16-byte pieces of rpt per four threads.  `term` holds
-// S_in Q between the two sweeps.  Both sweeps fetch eight segments at a time: the serial part is arithmetic only.
-__global__ __launch_bounds__(256) void gla_backward_segment_scan_kernel(
+//   carry(s) = rowsum_v(S_out(s) R_out(s)): what q dq - k dk adds up to over the segments walked after s, since a segment's
+//              part, rowsum_v(S_in Q - R_out U), is the difference of two such products and R_out is zero behind the last
+// (bf16 matrices in plain row-major order; carry as two partial sums per channel, over 16 accumulator lanes each).
+// One wave per (sequence, direction, register quad cq, 16 lanes of the passes' register order).  The walks are serial and short,
+// so everything is fetched into LDS in one round trip and the loops stay small: unrolled over segments in registers this
+// kernel took 1 us a segment, its code being read once and cold.  A thread holds the four state elements (k channels c, c+1) x
+// (v columns x, x+1), so that its bf16 results leave as 4-byte words.  Chunks of kScanChunk segments; with more than one,
+// S_out waits in `term` between the walks.
+constexpr int kScanChunk = 48;
+constexpr int kScanSegFloats = 256 + 256 + 128 + 8;  // U or S_out, Q, products, decays
+__global__ __launch_bounds__(64) void gla_backward_segment_scan_kernel(
     const float* __restrict__ ws_fwd, const float* __restrict__ ws_grad, float* __restrict__ term, uint16_t* __restrict__ sp,
-    uint16_t* __restrict__ rp, uint16_t* __restrict__ rpt, float* __restrict__ carry, int* __restrict__ flags, int nseq,
-    int nseg, int ndir, int ng) {
-  constexpr int kBatch = 8;
-  __shared__ float red[kBatch][2][256];
-  const int tid = threadIdx.x;
-  const int cq = blockIdx.x;  // register quad: 4 blocks per (sequence, direction)
-  const int seq = blockIdx.y / ndir, dir = blockIdx.y % ndir;
-  if (cq == 0 && tid == 0 && dir == 0) flags[seq] = 0;
-  if (cq >= ng) return;  // register quads beyond Dk/16 carry no channel (whole blocks)
-  const int m = tid & 3, lane = tid >> 2, h = lane >> 5;
-  const int ch0 = 8 * ng * h + 8 * cq + 2 * m;  // k channels ch0 (pk = 0), ch0 + 1 (pk = 1)
-  const int v0 = 2 * cpair<4>(lane & 31);         // v columns v0 (pv = 0), v0 + 1 (pv = 1)
-  // element (pk, pv) of this thread in register order: unit u = (pk*2 + pv)*4 + cq
-  int e[2][2];
-#pragma unroll
-  for (int pk = 0; pk < 2; ++pk)
-#pragma unroll
-    for (int pv = 0; pv < 2; ++pv) e[pk][pv] = ((((pk * 2 + pv) * 4 + cq) * 64 + lane) << 2) + m;
-  auto slot = [&](int seg, int d) { return (((size_t)seq * nseg + seg) * 2 + d); };
-  // the gradient state pass ran with the directions' roles exchanged (see launch_gla_backward_mfma)
-  const int gdir = 1 - dir;
-  float S[2][2] = {{0.f, 0.f}, {0.f, 0.f}};
-  for (int i0 = 0; i0 < nseg; i0 += kBatch) {
-    float U[kBatch][2][2], Q[kBatch][2][2], D[kBatch][2];
-#pragma unroll
-    for (int j = 0; j < kBatch; ++j) {
-      const int i = min(i0 + j, nseg - 1);
-      const int seg = dir == 0 ? i : nseg - 1 - i;
-      const float* f = ws_fwd + slot(seg, dir) * kGlaStateFloats;
-      const float* g = ws_grad + slot(seg, gdir) * kGlaStateFloats;
+    uint16_t* __restrict__ rp, uint16_t* __restrict__ rpt, float* __restrict__ carry, int* __restrict__ flags, int nseq, int nseg,
+    int ndir, int ng, int grad_swapped) {
+  extern __shared__ __align__(16) float sh[];
+  const int t = threadIdx.x, cq = blockIdx.y >> 2, quarter = blockIdx.y & 3;
+  const int seq = blockIdx.x / ndir, dir = blockIdx.x % ndir, gdir = grad_swapped ? 1 - dir : dir;
+  if (seq >= nseq) return;
+  const int chunk = min(nseg, kScanChunk), nchunks = (nseg + chunk - 1) / chunk;
+  float *F = sh, *Q = F + chunk * 256, *P = Q + chunk * 256, *D = P + chunk * 128;
+  const size_t state_elems = 16 * ng * 64;
+  if (blockIdx.y == 0 && t == 0 && dir == 0) flags[seq] = 0;
+  const int m = t & 3, lane = 16 * quarter + (t >> 2), h = lane >> 5;
+  const int cbase = 8 * ng * h + 8 * cq, ch0 = cbase + 2 * m;  // k channels ch0 (pk = 0), ch0 + 1 (pk = 1)
+  const int v0 = 2 * cpair<4>(lane & 31);                        // v columns v0 (pv = 0), v0 + 1 (pv = 1)
+  auto slot = [&](int i, int d) { return (((size_t)seq * nseg + (dir == 0 ? i : nseg - 1 - i)) * 2 + d); };  // i-th segment walked
+  // lane t fetches 16 bytes (four channels) of unit (pk, pv) = t >> 4: element (pk, pv) of thread t lies at 64 (2 pk + pv) + t
+  const int fetched = ((((t >> 4) * 4 + cq) * 64) + 16 * quarter + (t & 15)) * 4;
+  auto fetch = [&](const float* from, int d, int i0, int n, float* to) {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // (what lay there has been read and written)
+    for (int i = 0; i < n; ++i) load_to_lds16(from + slot(i0 + i, d) * kGlaStateFloats + fetched, lds_offset(to + i * 256));
+  };
+  auto fetch_decays = [&](int i0, int n) {
+    for (int i = t >> 3; i < n; i += 8) D[8 * i + (t & 7)] = ws_fwd[slot(i0 + i, dir) * kGlaStateFloats + 64 * 64 + cbase + (t & 7)];
+  };
+  auto kept = [&](int i) { return term + ((slot(i, dir) * ng * 4 + blockIdx.y) * 64 + t) * 4; };
+  float S[4] = {0.f, 0.f, 0.f, 0.f};
+  for (int c = 0; c < nchunks; ++c) {
+    const int i0 = c * chunk, n = min(chunk, nseg - i0);
+    fetch(ws_fwd, dir, i0, n, F);
+    if (nchunks == 1) fetch(ws_grad, gdir, i0, n, Q);
+    fetch_decays(i0, n);
+    wait_vmem<0>();
+    wave_lds_sync();
+    for (int i = 0; i < n; ++i) {
+      uint16_t* out = sp + slot(i0 + i, dir) * state_elems + ch0 * 64 + v0;
 #pragma unroll
       for (int pk = 0; pk < 2; ++pk) {
-        D[j][pk] = f[64 * 64 + ch0 + pk];
+        const float d = D[8 * i + 2 * m + pk], rd = __builtin_amdgcn_sqrtf(d);
+        *reinterpret_cast<uint32_t*>(out + 64 * pk) = pack_bf16x2(rd * S[2 * pk], rd * S[2 * pk + 1]);
 #pragma unroll
-        for (int pv = 0; pv < 2; ++pv) U[j][pk][pv] = f[e[pk][pv]], Q[j][pk][pv] = g[e[pk][pv]];
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < kBatch; ++j) {
-      const int i = i0 + j;
-      if (i < nseg) {
-        const int seg = dir == 0 ? i : nseg - 1 - i;
-        uint16_t* spm = sp + slot(seg, dir) * kBwdStateElems;
-        float* tm = term + slot(seg, dir) * kBwdStateElems;
-#pragma unroll
-        for (int pk = 0; pk < 2; ++pk) {
-          const float rd = __builtin_sqrtf(D[j][pk]);
-          *reinterpret_cast<uint32_t*>(spm + (ch0 + pk) * 64 + v0) = pack_bf16x2(rd * S[pk][0], rd * S[pk][1]);
-#pragma unroll
-          for (int pv = 0; pv < 2; ++pv) {
-            tm[e[pk][pv]] = S[pk][pv] * Q[j][pk][pv];
-            S[pk][pv] = __builtin_fmaf(D[j][pk], S[pk][pv], U[j][pk][pv]);
-          }
+        for (int pv = 0; pv < 2; ++pv) {
+          const int x = 2 * pk + pv;
+          S[x] = __builtin_fmaf(d, S[x], F[256 * i + 64 * x + t]);
+          F[256 * i + 64 * x + t] = S[x];
         }
       }
+      if (nchunks > 1) *reinterpret_cast<f32x4_t*>(kept(i0 + i)) = f32x4_t{S[0], S[1], S[2], S[3]};
     }
   }
-  float R[2][2] = {{0.f, 0.f}, {0.f, 0.f}}, later[2] = {0.f, 0.f};
-  for (int i0 = nseg - 1; i0 >= 0; i0 -= kBatch) {  // segments i0, i0 - 1, ... in this batch
-    float U[kBatch][2][2], Q[kBatch][2][2], T1[kBatch][2][2], D[kBatch][2];
+  float R[4] = {0.f, 0.f, 0.f, 0.f};
+  for (int c = nchunks - 1; c >= 0; --c) {
+    const int i0 = c * chunk, n = min(chunk, nseg - i0);
+    if (nchunks > 1) {
+      wave_lds_sync();  // (the chunk before has been read)
+      fetch(ws_grad, gdir, i0, n, Q);
+      fetch_decays(i0, n);
+      for (int i = 0; i < n; ++i) {
+        const f32x4_t x = *reinterpret_cast<const f32x4_t*>(kept(i0 + i));
 #pragma unroll
-    for (int j = 0; j < kBatch; ++j) {
-      const int i = max(i0 - j, 0);
-      const int seg = dir == 0 ? i : nseg - 1 - i;
-      const float* f = ws_fwd + slot(seg, dir) * kGlaStateFloats;
-      const float* g = ws_grad + slot(seg, gdir) * kGlaStateFloats;
-      const float* tm = term + slot(seg, dir) * kBwdStateElems;
-#pragma unroll
-      for (int pk = 0; pk < 2; ++pk) {
-        D[j][pk] = f[64 * 64 + ch0 + pk];
-#pragma unroll
-        for (int pv = 0; pv < 2; ++pv)
-          U[j][pk][pv] = f[e[pk][pv]], Q[j][pk][pv] = g[e[pk][pv]], T1[j][pk][pv] = tm[e[pk][pv]];
+        for (int j = 0; j < 4; ++j) F[256 * i + 64 * j + t] = x[j];
       }
+      wait_vmem<0>();
+      wave_lds_sync();
     }
+    for (int i = n - 1; i >= 0; --i) {
+      const size_t at = slot(i0 + i, dir) * state_elems;
+      float x[4], q[4];
 #pragma unroll
-    for (int j = 0; j < kBatch; ++j) {
-      const int i = i0 - j;
-      red[j][0][tid] = later[0];
-      red[j][1][tid] = later[1];
-      if (i >= 0) {
-        const int seg = dir == 0 ? i : nseg - 1 - i;
-        uint16_t* rpm = rp + slot(seg, dir) * kBwdStateElems;
-        uint16_t* rtm = rpt + slot(seg, dir) * kBwdStateElems;
-        float x[2][2];
+      for (int j = 0; j < 4; ++j) x[j] = F[256 * i + 64 * j + t], q[j] = Q[256 * i + 64 * j + t];
+      const float d[2] = {D[8 * i + 2 * m], D[8 * i + 2 * m + 1]};
+      const float rd[2] = {__builtin_amdgcn_sqrtf(d[0]), __builtin_amdgcn_sqrtf(d[1])};
+      P[128 * i + t] = x[0] * R[0] + x[1] * R[1];
+      P[128 * i + 64 + t] = x[2] * R[2] + x[3] * R[3];
 #pragma unroll
-        for (int pk = 0; pk < 2; ++pk) {
-          const float rd = __builtin_sqrtf(D[j][pk]);
-          x[pk][0] = rd * R[pk][0], x[pk][1] = rd * R[pk][1];
-          *reinterpret_cast<uint32_t*>(rpm + (ch0 + pk) * 64 + v0) = pack_bf16x2(x[pk][0], x[pk][1]);
-        }
-#pragma unroll
-        for (int pv = 0; pv < 2; ++pv)
-          *reinterpret_cast<uint32_t*>(rtm + (v0 + pv) * 64 + ch0) = pack_bf16x2(x[0][pv], x[1][pv]);
-#pragma unroll
-        for (int pk = 0; pk < 2; ++pk)
-#pragma unroll
-          for (int pv = 0; pv < 2; ++pv) {
-            later[pk] += T1[j][pk][pv] - R[pk][pv] * U[j][pk][pv];
-            R[pk][pv] = __builtin_fmaf(D[j][pk], R[pk][pv], Q[j][pk][pv]);
-          }
+      for (int p = 0; p < 2; ++p) {
+        *reinterpret_cast<uint32_t*>(rp + at + (ch0 + p) * 64 + v0) = pack_bf16x2(rd[p] * R[2 * p], rd[p] * R[2 * p + 1]);
+        *reinterpret_cast<uint32_t*>(rpt + at + (v0 + p) * 16 * ng + ch0) = pack_bf16x2(rd[0] * R[p], rd[1] * R[2 + p]);
       }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) R[j] = __builtin_fmaf(d[j >> 1], R[j], q[j]);
     }
-    // the block holds 16 channels (lane half h, register m, pk) x all 64 v columns: summed in a fixed order
-    __syncthreads();
-    if (tid < 16 * kBatch) {
-      const int j = tid >> 4, hh = (tid >> 3) & 1, mm = (tid >> 1) & 3, pk = tid & 1;
-      const int i = i0 - j;
-      if (i >= 0) {
-        const int seg = dir == 0 ? i : nseg - 1 - i;
-        float acc = 0.f;
-        for (int x = 0; x < 32; ++x) acc += red[j][pk][(32 * hh + x) * 4 + mm];
-        const int ch = 8 * ng * hh + 8 * cq + 2 * mm + pk;
-        carry[slot(seg, dir) * 128 + ch] = acc;
-        carry[slot(seg, dir) * 128 + 64 + ch] = 0.f;
-      }
+    wave_lds_sync();
+    for (int j = t; j < 8 * n; j += 64) {  // (segment, channel 2 mm + pk): the 16 lanes' products, in a fixed order
+      const int i = j >> 3, mm = (j >> 1) & 3, pk = j & 1;
+      float acc = 0.f;
+#pragma unroll
+      for (int l = 0; l < 16; ++l) acc += P[128 * i + 64 * pk + 4 * l + mm];
+      carry[slot(i0 + i, dir) * 128 + 64 * (quarter & 1) + cbase + (j & 7)] = acc;
     }
-    __syncthreads();
   }
 }
 
@@ -754,11 +727,10 @@ bool gla_backward_mfma_supported(int B, int H, int L, int Dk, int Dv, int io_dty
 
 // Long sequences: two state passes (kGlaStateFloats floats per sequence, segment and direction each), the S_in Q terms
 // and the carries (fp32), then the three bf16 matrices the segments read.
-static size_t seg_slots(int B, int H, int L) { return (size_t)B * H * gla_segments(L) * 2; }
+static size_t seg_slots(int B, int H, int nseg) { return (size_t)B * H * nseg * 2; }
 size_t gla_backward_mfma_workspace(int B, int H, int L, int Dk, int Dv) {
   if (L <= 32 * kBwdTiles || !(Dk == 64 || Dk == 32) || Dv != 64) return 0;
-  const size_t n = seg_slots(B, H, L);
-  return n * ((2 * (size_t)kGlaStateFloats + kBwdStateElems + 128) * sizeof(float) + 3 * (size_t)kBwdStateElems * 2);
+  return seg_slots(B, H, gla_segments(L)) * ((2 * (size_t)kGlaStateFloats + 64 * 64 + 128) * sizeof(float) + 3 * (size_t)64 * 64 * 2);
 }
 
 struct BwdLaunch {
@@ -793,10 +765,42 @@ static int launch_bwd(const BwdLaunch& l, bool seg, int tokens) {
   return tokens <= 128 ? launch_bwd_t<NG, BIDIR, false, 4>(l) : launch_bwd_t<NG, BIDIR, false, 8>(l);
 }
 
+// Where the segments of a call keep what links them: n slots, one per (sequence, segment, direction).
+struct BwdRoom {
+  float *fwd, *grad, *term, *carry;
+  uint16_t *sp, *rp, *rpt;
+  // pieces go to `scratch` (the recurrent kernel's, which runs when everything here has been read) while they fit there, else to `ws`
+  bool lay_out(size_t n, int Dk, void* scratch, size_t scratch_bytes, void* ws, size_t ws_bytes) {
+    bool ok = true;
+    const auto take = [&](size_t bytes) -> char* {
+      char* p;
+      if (bytes <= scratch_bytes) p = (char*)scratch, scratch = p + bytes, scratch_bytes -= bytes;
+      else if (bytes <= ws_bytes) p = (char*)ws, ws = p + bytes, ws_bytes -= bytes;
+      else p = nullptr, ok = false;
+      return p;
+    };
+    const size_t state = (size_t)Dk * 64;
+    fwd = (float*)take(2 * n * kGlaStateFloats * sizeof(float));
+    grad = fwd + (ok ? n * kGlaStateFloats : 0);
+    term = (float*)take(n * state * sizeof(float));
+    sp = (uint16_t*)take(n * state * 2);
+    rp = (uint16_t*)take(n * state * 2);
+    rpt = (uint16_t*)take(n * state * 2);
+    carry = (float*)take(n * 128 * sizeof(float));
+    return ok;
+  }
+};
+// Segments of 128 tokens, two workgroups of four waves to a CU, or of up to 256, one of eight.  The short ones take less than half
+// the time each and overlap, but double what the states cost.  us of the whole backward, long / short, at the number of long ones:
+// Dk 32: 6 39 / 31, 48 44.5 / 36, 240 56.4 / 55.8, 360 92 / 76, 576 137 / 117, 384 of 256 99.8 / 101.7: always short;
+// Dk 64: 6 46 / 41, 48 57 / 47 and 65 / 60, 192 71 / 76, 240 81 / 92, 576 194 / 219: short up to half a round.
+static bool short_segments(int B, int H, int L, int Dk) { return Dk == 32 || (long long)B * H * gla_segments(L) <= 128; }
+
 // flags: one int per (batch, head) sequence, written by every launch: 1 = not computed here (gates out of range)
 int launch_gla_backward_mfma(const void* q, const void* k, const void* v, const void* gf, const void* gb,
                              const void* d_o, void* dq, void* dk, void* dv, void* dgf, void* dgb, int* flags,
-                             void* seg_workspace, int B, int H, int L, int Dk, float s, hipStream_t stream) {
+                             void* scratch, size_t scratch_bytes, void* seg_workspace, size_t seg_bytes, int B, int H, int L,
+                             int Dk, float s, hipStream_t stream) {
   constexpr int kMaxDevices = 64;
   static bool attr_done_dev[kMaxDevices] = {};
   static int num_cu_dev[kMaxDevices] = {};
@@ -813,31 +817,42 @@ int launch_gla_backward_mfma(const void* q, const void* k, const void* v, const 
   int nslabs = B * H;
   if (seg) {
     if (!seg_workspace || !seg_grid_ok(B, H, gb != nullptr)) return -22;
-    const size_t n = seg_slots(B, H, L);
-    float* ws_fwd = (float*)seg_workspace;
-    float* ws_grad = ws_fwd + n * kGlaStateFloats;
-    float* term = ws_grad + n * kGlaStateFloats;
-    float* carry = term + n * kBwdStateElems;
-    uint16_t* sp = (uint16_t*)(carry + n * 128);
-    uint16_t* rp = sp + n * kBwdStateElems;
-    uint16_t* rpt = rp + n * kBwdStateElems;
-    // One launch for both state passes.  The forward's: contributions k~^T v and decays of every segment, both
-    // directions.  The gradient states: the same pass on (q for k, do for v) with each token's own gate included in
-    // its weight.  A state pass anchors a token at the END of its walk (the weight of token j is the decay from j to
-    // the last token walked); the gradient state needs the decay from the FIRST token walked to i, i.e. the walk of
-    // the other direction over the same gates: the forward gates go to the reverse waves and the reverse gates to the
-    // forward waves, and slot d of that pass belongs to direction 1 - d.  (The causal op runs both directions on its
-    // one gate tensor and uses the forward slot of the first pass and the reverse slot of the second.)
+    const int ndir = gb ? 2 : 1, ng = Dk / 16;
+    BwdRoom r;
+    if (!(short_segments(B, H, L, Dk) && r.lay_out(seg_slots(B, H, (L + 127) / 128), Dk, scratch, scratch_bytes, seg_workspace, seg_bytes))) {
+      r = BwdRoom();
+      if (!r.lay_out(seg_slots(B, H, gla_segments(L)), Dk, nullptr, 0, seg_workspace, seg_bytes)) return -28;
+      sg.nseg = gla_segments(L), sg.seg_len = gla_segment_len(L);
+    } else {
+      sg.nseg = (L + 127) / 128, sg.seg_len = 128;
+    }
+    // One launch for both state passes: contributions k~^T v and decays of every segment, both directions, and the gradient
+    // states, the same sums over (q, do) with each token's own gate included in its weight.
     GlaArgs a{};
-    a.q = q, a.k = k, a.v = v, a.g_fwd = gf, a.g_bwd = gb ? gb : gf, a.o = const_cast<void*>(d_o), a.workspace = ws_fwd;
+    a.q = q, a.k = k, a.v = v, a.g_fwd = gf, a.g_bwd = gb, a.o = const_cast<void*>(d_o), a.workspace = r.fwd;
     a.B = B, a.H = H, a.L = L, a.Dk = Dk, a.Dv = 64, a.scale = 1.f, a.out_scale = 1.f, a.io_dtype = 1, a.gate_dtype = 1;
-    a.stream = stream, a.state_pass = 2;
-    const int rc = launch_gla_mfma(a);
+    a.stream = stream;
+    int rc;
+    if (Dk == 32) {
+      rc = launch_gla_states(a, sg.seg_len, sg.nseg, r.fwd, q, d_o, r.grad);
+    } else {
+      // The chunked kernel's state pass anchors a token at the END of its walk (the weight of token j is the decay from j to
+      // the last token walked); the gradient state needs the decay from the FIRST token walked to i, i.e. the walk of
+      // the other direction over the same gates: the forward gates go to the reverse waves and the reverse gates to the
+      // forward waves, and slot d of that pass belongs to direction 1 - d.  (The causal op runs both directions on its
+      // one gate tensor and uses the forward slot of the first pass and the reverse slot of the second.)
+      if (!gb) a.g_bwd = gf;
+      a.state_pass = 1, a.state_segments = sg.nseg, a.state_seg_len = sg.seg_len;
+      rc = launch_gla_mfma(a);
+    }
     if (rc != 0) return rc;
-    const int ndir = gb ? 2 : 1;
-    hipLaunchKernelGGL(gla_backward_segment_scan_kernel, dim3(4, B * H * ndir), dim3(256), 0, stream, ws_fwd,
-                       ws_grad, term, sp, rp, rpt, carry, flags, B * H, gla_segments(L), ndir, Dk / 16);
-    sg = BwdSegments{sp, rp, rpt, carry, gla_segments(L), gla_segment_len(L)};
+    static bool done[64] = {};
+    if (!allow_lds(reinterpret_cast<const void*>(gla_backward_segment_scan_kernel), kScanChunk * kScanSegFloats * sizeof(float), done)) return -5;
+    const int held = sg.nseg < kScanChunk ? sg.nseg : kScanChunk;
+    hipLaunchKernelGGL(gla_backward_segment_scan_kernel, dim3((B * H * ndir + 7) / 8 * 8, 4 * ng), dim3(64),
+                       held * kScanSegFloats * sizeof(float), stream, r.fwd, r.grad, r.term, r.sp, r.rp, r.rpt, r.carry, flags, B * H,
+                       sg.nseg, ndir, ng, (int)(Dk == 64));
+    sg.sp = r.sp, sg.rp = r.rp, sg.rpt = r.rpt, sg.carry = r.carry;
     nslabs = B * H * sg.nseg;
   }
   const BwdLaunch l{q, k, v, gf, gb, d_o, dq, dk, dv, dgf, dgb, flags, nslabs, L, s, sg, num_cu_dev[dev], stream};

@@ -1075,14 +1075,17 @@ static int launch_gla_mfma_t(const GlaArgs& a, int num_cu, int dev) {
   static bool attr_done_dev[kMaxDevices] = {};
   bool& attr_done = attr_done_dev[dev];
   if (!attr_done) {
-    const void* kernels[6] = {reinterpret_cast<const void*>(gla_mfma_kernel<kModeSlab, NG>),
+    const void* kernels[5] = {reinterpret_cast<const void*>(gla_mfma_kernel<kModeSlab, NG>),
                               reinterpret_cast<const void*>(gla_mfma_kernel<kModeSlabPitched, NG>),
                               reinterpret_cast<const void*>(gla_mfma_kernel<kModeState, NG>),
                               reinterpret_cast<const void*>(gla_mfma_kernel<kModeChain, NG>),
-                              reinterpret_cast<const void*>(gla_mfma_kernel<kModeSlab, NG, true>),
-                              reinterpret_cast<const void*>(gla_mfma_kernel<kModeStateDual, NG>)};
+                              reinterpret_cast<const void*>(gla_mfma_kernel<kModeSlab, NG, true>)};
     for (const void* kf : kernels)
       if (hipFuncSetAttribute(kf, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsTotal) != hipSuccess) return -5;
+    if constexpr (NG == 4)
+      if (hipFuncSetAttribute(reinterpret_cast<const void*>(gla_mfma_kernel<kModeStateDual, NG>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, kLdsTotal) != hipSuccess)
+        return -5;
     attr_done = true;
   }
   // long sequences whose output pass the tile-pair kernel can do are cut its way
@@ -1092,6 +1095,10 @@ static int launch_gla_mfma_t(const GlaArgs& a, int num_cu, int dev) {
   }();
   const bool tile_chain = !chunked_only && !a.state_pass && gla_tiles_chain_supported(a);
   Geometry geo = make_geometry(a.B * a.H, a.L, tile_chain);
+  if (a.state_segments > 0) {
+    geo.nseg = a.state_segments, geo.seg_len = a.state_seg_len;
+    geo.cw = (geo.seg_len + 3) / 4, geo.nitems = a.B * a.H * geo.nseg;
+  }
   geo.wide_gates = a.wide_gates;
   geo.H = a.H;
   geo.sq = make_strides(a.q_strides, a.H, a.L, a.Dk);
@@ -1116,18 +1123,18 @@ static int launch_gla_mfma_t(const GlaArgs& a, int num_cu, int dev) {
   const float oscale = a.scale * a.out_scale;
   const float* no_gate = nullptr;
   if (a.state_pass) {
-    // one state pass alone: contributions and decays of every (sequence, segment, direction), no scan, no outputs
-    if (a.state_pass == 2) {
-      // plain set on (k, v, gates) and gradient-state set on (q for k, o for v, gates exchanged) in one launch
+    // both state passes of the backward alone, no scan, no outputs: the plain set on (k, v, gates) and the gradient-state set on
+    // (q for k, o for v, gates exchanged) in one launch (Dk 32 has gla_states.hip)
+    if constexpr (NG == 4) {
       if (!gb) return -22;
       geo.dual_first = geo.nitems;
       geo.nitems *= 2;
       grid = geo.nitems < num_cu ? geo.nitems : num_cu;
       hipLaunchKernelGGL((gla_mfma_kernel<kModeStateDual, NG>), dim3(grid), dim3(512), kLdsTotal, a.stream, q, k, v,
                          gf, gb, o, geo, oscale, (float*)a.workspace, no_gate);
-    } else
-      hipLaunchKernelGGL((gla_mfma_kernel<kModeState, NG>), dim3(grid), dim3(512), kLdsTotal, a.stream, q, k, v, gf, gb,
-                         o, geo, oscale, (float*)a.workspace, no_gate);
+    } else {
+      return -95;
+    }
   } else if (a.gate_w) {
     // fused locality gate: whole-sequence slabs, both directions, the padded token grid must fit the staging cells
     if (geo.nseg != 1 || !gb || a.gate_cols <= 0 || a.gate_rows <= 0 || a.gate_cols * a.gate_rows != a.L ||

@@ -28,11 +28,12 @@ struct GlaArgs {
   // causal op only (g_bwd null): fp32 [B, H, Dk, Dv] state before the first token / after the last one; null: zero / not wanted
   const float* init_state = nullptr;
   float* final_state = nullptr;
-  // bf16 MFMA path, any L: run state passes alone into `workspace`, per (sequence, segment, direction)
-  // kGlaStateFloats floats, no scan, no outputs.  1: the forward's pass on (k, v, gates).  2 (both directions only):
-  // that pass and, behind its slots, the gradient-state pass of the backward on (q for k, `o` read as the output
-  // gradient for v, the two directions' gates exchanged, cumulative gates exclusive of each token's own gate).
+  // bf16 MFMA path, Dk 64, both directions, any L: run the backward's state passes alone into `workspace`, per (sequence,
+  // segment, direction) kGlaStateFloats floats, no scan, no outputs: the forward's pass on (k, v, gates) and, behind its slots,
+  // the gradient-state pass on (q for k, `o` read as the output gradient for v, the two directions' gates exchanged,
+  // cumulative gates exclusive of each token's own gate).
   int state_pass = 0;
+  int state_segments = 0, state_seg_len = 0;  // the segmentation (at most 256 tokens each)
   // bf16 MFMA path: q, k, v that are not plain [B, H, L, D] tensors: element strides (batch, head, token) with the
   // channels of a (token, head) contiguous, e.g. column blocks of a projection output [B, L, H*(2*Dk + Dv)] read in
   // place.  Null (or token stride 0): plain layout.  Strides are multiples of 8 elements.
@@ -104,12 +105,13 @@ size_t gla_mfma_state_workspace(int B, int H, int L, int Dk, int Dv);  // causal
 
 // bf16 matrix-core backward (quadratic form per slab, or per <= 256-token segment of a longer sequence with the
 // segments chained through states); flags[b*H + h] = 1 marks sequences it left to the recurrent kernel.
-// seg_workspace: gla_backward_mfma_workspace() bytes, used for L > 256 only.
+// seg_workspace: gla_backward_mfma_workspace() bytes (seg_bytes), used for L > 256 only, and with it `scratch`, if there is room.
 bool gla_backward_mfma_supported(int B, int H, int L, int Dk, int Dv, int io_dtype, int gate_dtype, bool bidir);
 size_t gla_backward_mfma_workspace(int B, int H, int L, int Dk, int Dv);
 int launch_gla_backward_mfma(const void* q, const void* k, const void* v, const void* gf, const void* gb,
                              const void* d_o, void* dq, void* dk, void* dv, void* dgf, void* dgb, int* flags,
-                             void* seg_workspace, int B, int H, int L, int Dk, float s, hipStream_t stream);
+                             void* scratch, size_t scratch_bytes, void* seg_workspace, size_t seg_bytes, int B, int H, int L,
+                             int Dk, float s, hipStream_t stream);
 
 // allows a kernel its LDS, once per device (concurrent first calls only repeat an idempotent setting)
 inline bool allow_lds(const void* kernel, size_t bytes, bool (&done)[64]) {
