@@ -208,7 +208,7 @@ static int gla_bidir_fwd(const void* q, const void* k, const void* v, const void
   }
   // fp32 on the matrix cores; a caller that brought no room for a long sequence's states gets the recurrent kernel
   if (vig::gla_f32_supported(a)) {
-    const size_t n = vig::gla_f32_workspace(B, H, L, Dk, Dv);
+    const size_t n = vig::gla_f32_least_workspace(B, H, L, Dk, Dv);
     if (n == 0 || (workspace && workspace_bytes >= n)) return vig::launch_gla_f32(a);
   }
   const size_t need = g_bwd ? vig::gla_recurrent_workspace(B, H, L, Dv, io_dtype) : 0;

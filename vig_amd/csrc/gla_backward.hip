@@ -326,16 +326,14 @@ int launch_gla_backward(const void* q, const void* k, const void* v, const void*
     a.only_flagged = flags;  // slabs with gates beyond the matrix-core kernel's range
   }
   if (!exact && gla_backward_f32_supported(B, H, L, Dk, Dv, io_dtype, gate_dtype, g_bwd != nullptr)) {
-    // the states of a long sequence lie in the segment workspace (two 16.6 KB slots per set and 224 tokens; 149 KB are there
-    // per 256), of 225 to 256 tokens in the recurrent kernel's scratch, which runs after everything has read them
-    int* flags = reinterpret_cast<int*>((float*)workspace + recurrent_floats(B, H, L, Dk, Dv, g_bwd != nullptr));
-    const bool behind = L > 256;
-    const size_t room = behind ? gla_backward_mfma_workspace(B, H, L, Dk, Dv)
-                               : recurrent_floats(B, H, L, Dk, Dv, g_bwd != nullptr) * sizeof(float);
-    if (gla_backward_f32_states(B, H, L) > room) return -28;
-    float* states = behind ? (float*)((char*)workspace + flags_end(B, H, L, Dk, Dv, g_bwd != nullptr)) : (float*)workspace;
-    const int rc = launch_gla_backward_f32(q, k, v, g_fwd, g_bwd, d_o, dq, dk, dv, dg_fwd, dg_bwd, flags, states, B, H, L,
-                                           Dk, scale * out_scale, stream);
+    // the states of a long sequence lie in the recurrent kernel's scratch, which runs after everything has read them, and in the
+    // segment workspace (of 225 to 256 tokens: none)
+    const size_t scratch = recurrent_floats(B, H, L, Dk, Dv, g_bwd != nullptr) * sizeof(float);
+    const size_t behind = gla_backward_mfma_workspace(B, H, L, Dk, Dv);
+    int* flags = reinterpret_cast<int*>((char*)workspace + scratch);
+    const int rc = launch_gla_backward_f32(q, k, v, g_fwd, g_bwd, d_o, dq, dk, dv, dg_fwd, dg_bwd, flags, workspace, scratch,
+                                           (char*)workspace + flags_end(B, H, L, Dk, Dv, g_bwd != nullptr), behind, B, H, L, Dk,
+                                           scale * out_scale, stream);
     if (rc != 0) return rc;
     a.only_flagged = flags;
     // A flagged sequence takes as long as a launch full of them, behind everybody else's tile form: its directions side by side

@@ -29,8 +29,7 @@ constexpr float kMagnitude32 = 1e12f;
 struct BwdF32Geo {
   int L, NT, nseg;
   float s;              // scale * out_scale
-  const float* states;  // scanned slots of the forward states, then those of the gradient states; null: whole sequences
-  size_t grad_states;   // floats between the two sets
+  const float *states, *grad_states;  // scanned slots of the forward states and of the gradient states; null: whole sequences
 };
 
 // byte offsets: per tile the operand over key channels (k^ or q^) and the one over value channels (v or d'), decays,
@@ -425,7 +424,7 @@ __global__ __launch_bounds__(512, 2) void gla_backward_f32_kernel(
   int* flags = reinterpret_cast<int*>(lds + lay.flag);
   const size_t item = (size_t)blockIdx.x * geo.nseg + blockIdx.y;
   const float* st = geo.states ? geo.states + item * 2 * kGlaStateFloats : nullptr;
-  const float* dst = geo.states ? st + geo.grad_states : nullptr;
+  const float* dst = geo.states ? geo.grad_states + item * 2 * kGlaStateFloats : nullptr;
 
   // Rows come from memory again for every loop that needs them (they would not fit in registers), asked for in front of
   // the barrier before their staging (168 -> 163 us against loads where they are used; asked for a whole loop ahead they
@@ -656,15 +655,10 @@ bool gla_backward_f32_supported(int B, int H, int L, int Dk, int Dv, int io_dtyp
   return io_dtype == 0 && gate_dtype == 0 && (Dk == 64 || Dk == 32) && Dv == 64 && gla_f32_segments(L) <= 65535 &&
          (gla_f32_segments(L) == 1 || (long long)B * H * 4 <= 65535) && (bidir || L <= 224 || L > 256);
 }
-// the two sets of states of a long sequence
-size_t gla_backward_f32_states(int B, int H, int L) {
-  return gla_f32_segments(L) == 1 ? 0 : (size_t)B * H * gla_f32_segments(L) * 4 * kGlaStateFloats * sizeof(float);
-}
-
 template <int NG, bool BIDIR>
 static int launch_bwd_f32_t(const float* q, const float* k, const float* v, const float* gf, const float* gb, const float* d_o,
-                            float* dq, float* dk, float* dv, float* dgf, float* dgb, int* flags, float* states, int B, int H,
-                            int L, float s, int dev, hipStream_t stream) {
+                            float* dq, float* dk, float* dv, float* dgf, float* dgb, int* flags, void* room0, size_t bytes0,
+                            void* room1, size_t bytes1, int B, int H, int L, float s, int dev, hipStream_t stream) {
   static bool attr_done[64] = {};
   if (!attr_done[dev]) {
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(gla_backward_f32_kernel<NG, BIDIR>),
@@ -674,17 +668,29 @@ static int launch_bwd_f32_t(const float* q, const float* k, const float* v, cons
   }
   BwdF32Geo geo{};
   geo.L = L;
-  geo.nseg = gla_f32_segments(L);
-  geo.NT = gla_f32_segment_tiles(L);
+  const int tiles = (L + 31) / 32;
+  float *states = nullptr, *grads = nullptr;
+  // the segments that fill the chip, or the next longer ones whose states have room
+  const int most = gla_f32_segment_tiles(L);
+  for (int NT = gla_f32_fine_tiles((long long)B * H, L); NT <= most; ++NT) {
+    geo.NT = NT, geo.nseg = (tiles + NT - 1) / NT;
+    const size_t set = geo.nseg == 1 ? 0 : (size_t)B * H * geo.nseg * 2 * kGlaStateFloats;
+    const size_t n = set * sizeof(float);
+    if (2 * n <= bytes0) states = (float*)room0, grads = states + set;
+    else if (2 * n <= bytes1) states = (float*)room1, grads = states + set;
+    else if (n <= bytes0 && n <= bytes1) states = (float*)room0, grads = (float*)room1;
+    else continue;
+    break;
+  }
+  if (!states) return -28;
   geo.s = s;
   const BwdF32Lds<NG> lay(geo.NT);
   if (lay.total > kBwdF32MaxLds || geo.NT > 7) return -95;
   if (geo.nseg > 1) {
-    geo.states = states;
-    geo.grad_states = (size_t)B * H * geo.nseg * 2 * kGlaStateFloats;
-    int rc = launch_gla_f32_states(NG, k, v, q, d_o, gf, gb, states, flags, B * H, L, geo.NT, geo.nseg, stream);
+    geo.states = states, geo.grad_states = grads;
+    int rc = launch_gla_f32_states(NG, k, v, q, d_o, gf, gb, states, grads, flags, B * H, L, geo.NT, geo.nseg, stream);
     if (rc) return rc;
-    rc = launch_gla_segment_scan(states, 2 * B * H, geo.nseg, 2, NG, stream);
+    rc = launch_gla_segment_scan(states, grads, B * H, geo.nseg, 2, NG, stream);
     if (rc) return rc;
   }
   hipLaunchKernelGGL((gla_backward_f32_kernel<NG, BIDIR>), dim3(B * H, geo.nseg), dim3(64 * geo.NT), lay.total, stream, q, k, v,
@@ -693,13 +699,13 @@ static int launch_bwd_f32_t(const float* q, const float* k, const float* v, cons
 }
 
 int launch_gla_backward_f32(const void* q, const void* k, const void* v, const void* gf, const void* gb, const void* d_o,
-                            void* dq, void* dk, void* dv, void* dgf, void* dgb, int* flags, float* states, int B, int H, int L,
-                            int Dk, float s, hipStream_t stream) {
+                            void* dq, void* dk, void* dv, void* dgf, void* dgb, int* flags, void* room0, size_t bytes0,
+                            void* room1, size_t bytes1, int B, int H, int L, int Dk, float s, hipStream_t stream) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return -5;
 #define VIG_BWD_F32(NG, BI)                                                                                                   \
   launch_bwd_f32_t<NG, BI>((const float*)q, (const float*)k, (const float*)v, (const float*)gf, (const float*)gb,             \
-                           (const float*)d_o, (float*)dq, (float*)dk, (float*)dv, (float*)dgf, (float*)dgb, flags, states, B, \
+                           (const float*)d_o, (float*)dq, (float*)dk, (float*)dv, (float*)dgf, (float*)dgb, flags, room0, bytes0, room1, bytes1, B, \
                            H, L, s, dev, stream)
   if (Dk == 64) return gb ? VIG_BWD_F32(4, true) : VIG_BWD_F32(4, false);
   return gb ? VIG_BWD_F32(2, true) : VIG_BWD_F32(2, false);

@@ -463,7 +463,8 @@ template <int NG>
 __global__ __launch_bounds__(256, 2) void gla_f32_state_kernel(const float* __restrict__ k0, const float* __restrict__ v0,
                                                                const float* __restrict__ q1, const float* __restrict__ do1,
                                                                const float* __restrict__ gf, const float* __restrict__ gb,
-                                                               float* __restrict__ ws, int* __restrict__ flags, int L, int NT,
+                                                               float* __restrict__ ws, float* __restrict__ grad_ws,
+                                                               int* __restrict__ flags, int L, int NT,
                                                                int nseg) {
   constexpr int DK = 16 * NG, NP = NG / 2;
   const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
@@ -545,8 +546,7 @@ __global__ __launch_bounds__(256, 2) void gla_f32_state_kernel(const float* __re
       for (int t = 0; t < 2; ++t) mfma6(split8(octet(xk[p], t)), pvv[t], acc[p], accs[p]);
     }
   }
-  const size_t set = grad ? (size_t)gridDim.x * nseg : 0;
-  float* slot = ws + ((set + (size_t)blockIdx.x * nseg + blockIdx.y) * 2 + dir) * kGlaStateFloats;
+  float* slot = (grad ? grad_ws : ws) + (((size_t)blockIdx.x * nseg + blockIdx.y) * 2 + dir) * kGlaStateFloats;
 #pragma unroll
   for (int p = 0; p < NP; ++p) acc[p] += accs[p];
 #pragma unroll
@@ -571,9 +571,16 @@ bool gla_f32_supported(const GlaArgs& a) {
          !a.state_pass && !a.gate_w && !a.q_strides && !a.k_strides && !a.v_strides && gla_f32_segments(a.L) <= 65535 &&
          (gla_f32_segments(a.L) == 1 || (long long)a.B * a.H * 2 <= 65535);
 }
+static size_t f32_states(long long nseq, int L, int NT) {
+  return (size_t)nseq * (((L + 31) / 32 + NT - 1) / NT) * 2 * kGlaStateFloats * sizeof(float);
+}
+// (a call with room for segments of seven tiles only gets those)
+size_t gla_f32_least_workspace(int B, int H, int L, int Dk, int Dv) {
+  return gla_f32_workspace(B, H, L, Dk, Dv) == 0 ? 0 : f32_states((long long)B * H, L, gla_f32_segment_tiles(L));
+}
 size_t gla_f32_workspace(int B, int H, int L, int Dk, int Dv) {
   if ((Dk != 64 && Dk != 32) || Dv != 64 || gla_f32_segments(L) == 1) return 0;
-  return (size_t)B * H * gla_f32_segments(L) * 2 * kGlaStateFloats * sizeof(float);
+  return f32_states((long long)B * H, L, gla_f32_fine_tiles((long long)B * H, L));
 }
 
 template <int NG, bool BIDIR>
@@ -590,8 +597,8 @@ static int launch_f32_t(const GlaArgs& a, const F32Geo& geo, int dev) {
   if (geo.states) {
     hipLaunchKernelGGL((gla_f32_state_kernel<NG>), dim3(a.B * a.H, geo.nseg), dim3(BIDIR ? 256 : 128), 0, a.stream,
                        (const float*)a.k, (const float*)a.v, nullptr, nullptr, (const float*)a.g_fwd, (const float*)a.g_bwd,
-                       (float*)a.workspace, (int*)nullptr, a.L, geo.NT, geo.nseg);
-    const int rc = launch_gla_segment_scan((float*)a.workspace, a.B * a.H, geo.nseg, BIDIR ? 2 : 1, NG, a.stream);
+                       (float*)a.workspace, (float*)nullptr, (int*)nullptr, a.L, geo.NT, geo.nseg);
+    const int rc = launch_gla_segment_scan((float*)a.workspace, nullptr, a.B * a.H, geo.nseg, BIDIR ? 2 : 1, NG, a.stream);
     if (rc) return rc;
   }
   hipLaunchKernelGGL((gla_f32_kernel<NG, BIDIR>), dim3(a.B * a.H, geo.nseg), dim3(64 * geo.NT), lay.total, a.stream,
@@ -601,14 +608,14 @@ static int launch_f32_t(const GlaArgs& a, const F32Geo& geo, int dev) {
 }
 
 int launch_gla_f32_states(int NG, const float* k, const float* v, const float* q, const float* d_o, const float* gf,
-                          const float* gb, float* slots, int* flags, int nseq, int L, int NT, int nseg, hipStream_t stream) {
+                          const float* gb, float* slots, float* grad_slots, int* flags, int nseq, int L, int NT, int nseg, hipStream_t stream) {
   // (a causal call has no reverse gates: its second direction's slots are computed with the forward ones and not read)
   const float* g2 = gb ? gb : gf;
   if (NG == 4)
-    hipLaunchKernelGGL((gla_f32_state_kernel<4>), dim3(nseq, nseg, 2), dim3(256), 0, stream, k, v, q, d_o, gf, g2, slots, flags, L, NT,
+    hipLaunchKernelGGL((gla_f32_state_kernel<4>), dim3(nseq, nseg, 2), dim3(256), 0, stream, k, v, q, d_o, gf, g2, slots, grad_slots, flags, L, NT,
                        nseg);
   else
-    hipLaunchKernelGGL((gla_f32_state_kernel<2>), dim3(nseq, nseg, 2), dim3(256), 0, stream, k, v, q, d_o, gf, g2, slots, flags, L, NT,
+    hipLaunchKernelGGL((gla_f32_state_kernel<2>), dim3(nseq, nseg, 2), dim3(256), 0, stream, k, v, q, d_o, gf, g2, slots, grad_slots, flags, L, NT,
                        nseg);
   return hipGetLastError() == hipSuccess ? 0 : -5;
 }
@@ -618,8 +625,10 @@ int launch_gla_f32(const GlaArgs& a) {
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return -5;
   F32Geo geo{};
   geo.L = a.L;
-  geo.nseg = gla_f32_segments(a.L);
-  geo.NT = gla_f32_segment_tiles(a.L);
+  const long long nseq = (long long)a.B * a.H;
+  geo.NT = gla_f32_fine_tiles(nseq, a.L);
+  if (f32_states(nseq, a.L, geo.NT) > a.workspace_bytes) geo.NT = gla_f32_segment_tiles(a.L);
+  geo.nseg = ((a.L + 31) / 32 + geo.NT - 1) / geo.NT;
   geo.states = geo.nseg > 1 ? (const float*)a.workspace : nullptr;
   if (a.Dk == 64) return a.g_bwd ? launch_f32_t<4, true>(a, geo, dev) : launch_f32_t<4, false>(a, geo, dev);
   return a.g_bwd ? launch_f32_t<2, true>(a, geo, dev) : launch_f32_t<2, false>(a, geo, dev);

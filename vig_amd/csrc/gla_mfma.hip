@@ -950,17 +950,19 @@ __global__ __launch_bounds__(512) void gla_mfma_kernel(const uint16_t* __restric
 // The causal op may start from a caller's state and hand the last one back (init / final: fp32 [nseq, Dk, Dv] row-major,
 // null: zero / not wanted; one direction only): the thread of a state element is also the one that knows its row
 // (k channel) and column (v channel).
+// more (null: none): a second set of slots, chained by the blocks of grid.z = 1.
 // maxima (null: not wanted): [nseq][2 directions][kGlaScanMaxima], the largest |state entering a segment| each wave saw.
 // Whole op, us, against one thread per element (half the blocks without channels at Dk 32, two loads of 4 bytes a segment): Dk 32:
 // 144 sequences of 784 tokens 48.2 -> 44.3, 147 of 534 35.1 -> 31.0, 45 of 1679 32.4 -> 31.2; Dk 64: 147 of 534 49.5 -> 47.0.
 template <int kBatch>
-__global__ __launch_bounds__(256) void gla_segment_scan_kernel(float* state_ws, int nseq, int nseg, int ndir, int ng,
+__global__ __launch_bounds__(256) void gla_segment_scan_kernel(float* state_ws, float* more, int nseq, int nseg, int ndir, int ng,
                                                                const float* __restrict__ init, float* __restrict__ final,
                                                                float* __restrict__ maxima) {
   static_assert(4 * 4 == kGlaScanMaxima, "one partial maximum per wave of up to four blocks");
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, h = lane >> 5;
   const int seq = blockIdx.y / ndir, dir = blockIdx.y % ndir;
   if (seq >= nseq) return;
+  if (blockIdx.z != 0) state_ws = more;
   const int cq = blockIdx.x, pk = wave >> 1, pv = wave & 1, u = wave * 4 + cq;  // unit (pk, pv, cq)
   const int e = (u * 64 + lane) * 4, ch = 8 * ng * h + 8 * cq;  // element m: channel ch + 2 m + pk
   f32x4_t S = {0.f, 0.f, 0.f, 0.f};
@@ -1010,10 +1012,10 @@ __global__ __launch_bounds__(256) void gla_segment_scan_kernel(float* state_ws, 
   }
 }
 
-static void launch_scan(float* slots, int nseq, int nseg, int ndir, int ng, const float* init, float* final, float* maxima,
+static void launch_scan(float* slots, float* more, int nseq, int nseg, int ndir, int ng, const float* init, float* final, float* maxima,
                         hipStream_t stream) {
-  const dim3 grid(ng, nseq * ndir), block(256);
-#define VIG_SCAN(N) hipLaunchKernelGGL(gla_segment_scan_kernel<N>, grid, block, 0, stream, slots, nseq, nseg, ndir, ng, init, final, maxima)
+  const dim3 grid(ng, nseq * ndir, more ? 2 : 1), block(256);
+#define VIG_SCAN(N) hipLaunchKernelGGL(gla_segment_scan_kernel<N>, grid, block, 0, stream, slots, more, nseq, nseg, ndir, ng, init, final, maxima)
   if (nseg <= 2) VIG_SCAN(2);
   else if (nseg <= 4) VIG_SCAN(4);
   else if (nseg <= 8) VIG_SCAN(8);
@@ -1021,8 +1023,8 @@ static void launch_scan(float* slots, int nseq, int nseg, int ndir, int ng, cons
 #undef VIG_SCAN
 }
 
-int launch_gla_segment_scan(float* slots, int nseq, int nseg, int ndir, int ng, hipStream_t stream) {
-  launch_scan(slots, nseq, nseg, ndir, ng, nullptr, nullptr, nullptr, stream);
+int launch_gla_segment_scan(float* slots, float* more, int nseq, int nseg, int ndir, int ng, hipStream_t stream) {
+  launch_scan(slots, more, nseq, nseg, ndir, ng, nullptr, nullptr, nullptr, stream);
   return hipGetLastError() == hipSuccess ? 0 : -5;
 }
 
@@ -1165,7 +1167,7 @@ static int launch_gla_mfma_t(const GlaArgs& a, int num_cu, int dev) {
                          geo, oscale, ws, no_gate);
     }
     float* maxima = tile_chain ? ws + (size_t)geo.nitems * 2 * kStateFloats : nullptr;
-    launch_scan(ws, a.B * a.H, geo.nseg, gb ? 2 : 1, NG, a.init_state, a.final_state, maxima, a.stream);
+    launch_scan(ws, nullptr, a.B * a.H, geo.nseg, gb ? 2 : 1, NG, a.init_state, a.final_state, maxima, a.stream);
     if (tile_chain) {
       if (hipGetLastError() != hipSuccess) return -5;
       return launch_gla_tiles_chain(a, ws, maxima);

@@ -58,27 +58,37 @@ inline int gla_tile_segment_tiles(int L) { return ((L + gla_tile_segments(L) - 1
 constexpr int kGlaScanMaxima = 16;
 
 // fp32 tensors and gates on the matrix cores (operands in three bf16 pieces): segments of up to seven 32-token tiles, as
-// the tile-pair kernel cuts them.
+// the tile-pair kernel cuts them, or, where those leave compute units idle (256 of them), of as few tiles as one workgroup a
+// unit allows: a workgroup's time grows faster than its tiles.  us, segments of seven
+// tiles / these: forward Dk 32 12 sequences of 1031 44.8 / 28.0, 36 of 1024 46.6 / 39.2, Dk 64 66 / 38.5 and 72 / 61.6; backward
+// Dk 32 105 / 64 and 124 / 102, Dk 64 196 / 114 and 220 / 185.  (One tile more a segment than fits 256 units: 36 of 1024, Dk 64,
+// backward 276.)  Whole sequences of seven tiles stay whole: 120 of 196, Dk 64, backward 141 / 153.
 inline int gla_f32_segments(int L) { return gla_tile_segments(L); }
 inline int gla_f32_segment_tiles(int L) { return gla_tile_segment_tiles(L); }
+inline int gla_f32_fine_tiles(long long nseq, int L) {
+  const int tiles = (L + 31) / 32;
+  for (int NT = 2; tiles > 7 && NT < 7; ++NT)
+    if (nseq * ((tiles + NT - 1) / NT) <= 256) return NT;
+  return gla_f32_segment_tiles(L);
+}
 bool gla_f32_supported(const GlaArgs& a);
 size_t gla_f32_workspace(int B, int H, int L, int Dk, int Dv);
+size_t gla_f32_least_workspace(int B, int H, int L, int Dk, int Dv);
 int launch_gla_f32(const GlaArgs& a);
-// both sets of segment contributions of an fp32 backward: the states (k, v) and, behind them, the gradient states (q, d_o)
+// both sets of segment contributions of an fp32 backward: the states (k, v) and the gradient states (q, d_o)
 // (flags, one int per sequence, are cleared on the way)
 int launch_gla_f32_states(int NG, const float* k, const float* v, const float* q, const float* d_o, const float* gf,
-                          const float* gb, float* slots, int* flags, int nseq, int L, int NT, int nseg, hipStream_t stream);
-// fp32 backward on the matrix cores; one flag per sequence marks what it left to the recurrent kernel; states:
-// gla_backward_f32_states() bytes
+                          const float* gb, float* slots, float* grad_slots, int* flags, int nseq, int L, int NT, int nseg, hipStream_t stream);
+// fp32 backward on the matrix cores; one flag per sequence marks what it left to the recurrent kernel; the two sets of states go
+// to two pieces of memory, either of which may be empty
 bool gla_backward_f32_supported(int B, int H, int L, int Dk, int Dv, int io_dtype, int gate_dtype, bool bidir);
-size_t gla_backward_f32_states(int B, int H, int L);
 int launch_gla_backward_f32(const void* q, const void* k, const void* v, const void* gf, const void* gb, const void* d_o,
-                            void* dq, void* dk, void* dv, void* dgf, void* dgb, int* flags, float* states, int B, int H, int L,
-                            int Dk, float s, hipStream_t stream);
+                            void* dq, void* dk, void* dv, void* dgf, void* dgb, int* flags, void* room0, size_t bytes0,
+                            void* room1, size_t bytes1, int B, int H, int L, int Dk, float s, hipStream_t stream);
 // bf16: contributions and decays of every segment of seg_len tokens, and with q and d_o the gradient states (gla_states.hip)
 int launch_gla_states(const GlaArgs& a, int seg_len, int nseg, float* slots, const void* q, const void* d_o, float* grad_slots);
-// chains the slots of a state pass in place (gla_segment_scan_kernel, no state in or out)
-int launch_gla_segment_scan(float* slots, int nseq, int nseg, int ndir, int ng, hipStream_t stream);
+// chains the slots of a state pass in place (gla_segment_scan_kernel, no state in or out), and those of another if there is one
+int launch_gla_segment_scan(float* slots, float* more, int nseq, int nseg, int ndir, int ng, hipStream_t stream);
 
 // Most tensors one launch_cast_many takes.
 constexpr int kMaxCastJobs = 16;
