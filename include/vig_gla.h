@@ -617,6 +617,23 @@ int vig_linear_norm_fwd(const void* x, const void* weight, const void* residual,
 int vig_conv3x3s2_fwd(const void* x, const void* weight, void* y, int B, int H, int W, int Cin, int Cout, void* stream);
 
 /*
+ * fp32 product on the matrix cores, operands in three bf16 pieces (fp32 precision):
+ *   out[m, n] = sum_k A(m, k) B(n, k) + bias[n] + add[m, n]     (bias, add: NULL for none)
+ * A(m, k) = a[m*lda + k], or a[k*lda + m] with a_across; B(n, k) = b[n*ldb + k], or b[k*ldb + n] with b_across (not a_across
+ * alone).  With a_across also a_sums[m] = sum_k A(m, k) unless NULL.  A layer, its input gradient and its weight gradient are
+ * (x, w), (dy, w across) and (dy across, x across).  a, b and the workspace start on 16-byte boundaries; where the
+ * contraction is contiguous, K is a multiple of 8 and the row distance one of 4.  Operands beyond 1 GiB and other
+ * shapes: VIG_ENOTSUP.  The workspace (vig_matmul_f32_workspace bytes) holds partial tiles of long contractions over
+ * few tiles; they are added in a fixed order.
+ *
+ * Replaces: the fp32 linear layers and their gradients of classification/models/vig.py:295-330,486-497 (cuBLAS).
+ */
+size_t vig_matmul_f32_workspace(long long M, int N, long long K);
+int vig_matmul_f32(const float* a, long long lda, int a_across, const float* b, long long ldb, int b_across,
+                   const float* bias, const float* add, long long ldadd, float* out, long long ldo, float* a_sums,
+                   long long M, int N, long long K, void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * The closing norm and the mean over tokens in one pass, bf16: out [B, C] = mean over l of the RMS-normalised
  * (x + residual)[b, l, :], the sum and the normalised value rounded to bf16 as vig_rmsnorm_fwd with round_sum stores them, the mean in fp32.
  * C % 8 == 0, C <= 1024.

@@ -76,6 +76,11 @@ bool linear_wgrad_supported(long long T, int N, int K);
 size_t linear_wgrad_workspace(long long T, int N, int K);
 int launch_linear_wgrad(const void* dy, long long ldy, const void* x, long long ldx, long long T, int N, int K, float* dw,
                         float* db, void* workspace, hipStream_t stream);
+size_t matmul_f32_workspace(long long M, int N, long long K);
+bool matmul_f32_supported(long long lda, bool ta, long long ldb, bool tb, long long M, int N, long long K);
+int launch_matmul_f32(const float* a, long long lda, bool ta, const float* b, long long ldb, bool tb, const float* bias, const float* add,
+                      long long ldadd, float* out, long long ldo, float* a_sums, long long M, int N, long long K, void* workspace,
+                      hipStream_t stream);
 }  // namespace vig
 
 static bool dtype_ok(int d) { return d == VIG_F32 || d == VIG_BF16; }
@@ -491,6 +496,22 @@ int vig_conv3x3s2_fwd(const void* x, const void* weight, void* y, int B, int H, 
   if (!x || !weight || !y || B <= 0 || H <= 0 || W <= 0 || Cin <= 0 || Cout <= 0) return VIG_EINVAL;
   if (!aligned16(x, weight, y)) return VIG_EINVAL;
   return vig::launch_conv3x3s2(x, weight, y, B, H, W, Cin, Cout, (hipStream_t)stream);
+}
+
+size_t vig_matmul_f32_workspace(long long M, int N, long long K) {
+  return M <= 0 || N <= 0 || K <= 0 ? 0 : vig::matmul_f32_workspace(M, N, K);
+}
+
+int vig_matmul_f32(const float* a, long long lda, int a_across, const float* b, long long ldb, int b_across, const float* bias,
+                   const float* add, long long ldadd, float* out, long long ldo, float* a_sums, long long M, int N, long long K,
+                   void* workspace, size_t workspace_bytes, void* stream) {
+  if (!a || !b || !out || M <= 0 || N <= 0 || K <= 0 || !aligned16(a, b, workspace)) return VIG_EINVAL;
+  const bool ta = a_across != 0, tb = b_across != 0;
+  if (lda < (ta ? M : K) || ldb < (tb ? N : K) || ldo < N || (add && ldadd < N) || (a_sums && !ta)) return VIG_EINVAL;
+  if (!vig::matmul_f32_supported(lda, ta, ldb, tb, M, N, K)) return VIG_ENOTSUP;
+  const size_t need = vig::matmul_f32_workspace(M, N, K);
+  if (need > workspace_bytes || (need && !workspace)) return VIG_ENOSPC;
+  return vig::launch_matmul_f32(a, lda, ta, b, ldb, tb, bias, add, ldadd, out, ldo, a_sums, M, N, K, workspace, (hipStream_t)stream);
 }
 
 size_t vig_rmsnorm_pool_workspace(int B, int L, int C) {

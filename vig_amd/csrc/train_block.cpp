@@ -79,12 +79,42 @@ Tensor matrix(const Tensor& buf, int64_t off, int64_t rows, int64_t cols) {
   return buf.as_strided({rows, cols}, {cols, 1}, buf.storage_offset() + off);
 }
 
+bool aligned(const Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; }
+
+// out = A B^T (+ bias) (+ add) of fp32 rows, A [M, K] or its transpose lying as rows, B [N, K] or its transpose, on the matrix cores;
+// false where the library's product is to be taken.
+// Where the line lies: a call costs 4 us of host time here and 22 us there, and products of up to about 5e9 multiply-adds take as long or
+// less here as well (us, here / library; layer, input gradient, weight gradient with column sums): 400 x 2048 x 384 10 / 10, 18 / 17, 18 / 22;
+// 1960 x 768 x 768 28 / 26, 30 / 30, 34 / 42; 8100 x 192 x 512 21 / 17, 24 / 30, 29 / 71; 8100 x 768 x 768 87 / 80, 85 / 90, 106 / 117; beyond,
+// 8100 x 2048 x 384 117 / 103, 106 / 110, 146 / 121.  Training passes (ms, line here / library alone): 32 images of 224 px, ViG-T
+// 7.9 / 10.1; 30, ViG-S 13.3 / 15.0 (line at 2.5e9: 14.2; at 9e9: 13.5).
+bool matmul_f32(const Tensor& a, bool a_across, const Tensor& b, bool b_across, const float* bias, const Tensor& add, Tensor& out,
+                float* a_sums = nullptr) {
+  const int64_t M = a.size(a_across), K = a.size(!a_across), N = b.size(b_across);
+  if ((double)M * N * K > 5e9 || !aligned(a) || !aligned(b) || a.stride(1) != 1 || b.stride(1) != 1) return false;
+  const auto ld = [](const Tensor& t) { return t.size(0) == 1 ? t.size(1) : t.stride(0); };  // (a single row's stride says nothing)
+  const size_t need = vig_matmul_f32_workspace(M, (int)N, K);
+  const Tensor ws = need ? bytes_like(need, a) : Tensor();
+  const int rc = vig_matmul_f32(fptr(a), ld(a), a_across, fptr(b), ld(b), b_across, bias, add.defined() ? fptr(add) : nullptr,
+                                add.defined() ? ld(add) : 0, fptr(out), ld(out), a_sums, M, (int)N, K,
+                                need ? ws.data_ptr() : nullptr, need, stream_of(a));
+  if (rc == VIG_ENOTSUP) return false;
+  check_rc(rc, "vig_matmul_f32");
+  return true;
+}
+
 // dy^T x in fp32 (and the column sums of dy); rows of both may lie in wider matrices
 Tensor weight_grad(const Tensor& dy, const Tensor& x, Tensor* bias_grad) {
   const int64_t T = dy.size(0), N = dy.size(1), K = x.size(1);
   if (dy.scalar_type() == at::kFloat) {
-    if (bias_grad) *bias_grad = dy.sum(0);
-    return at::mm(dy.t(), x);
+    Tensor dw = at::empty({N, K}, dy.options()), db;
+    if (bias_grad) db = at::empty({N}, dy.options());
+    if (!matmul_f32(dy, true, x, true, nullptr, Tensor(), dw, bias_grad ? fptr(db) : nullptr)) {
+      if (bias_grad) db = dy.sum(0);
+      at::mm_out(dw, dy.t(), x);
+    }
+    if (bias_grad) *bias_grad = db;
+    return dw;
   }
   Tensor dw = at::empty({N, K}, dy.options().dtype(at::kFloat));
   if (bias_grad) *bias_grad = at::empty({N}, dw.options());
@@ -96,9 +126,7 @@ Tensor weight_grad(const Tensor& dy, const Tensor& x, Tensor* bias_grad) {
   return dw;
 }
 
-bool aligned(const Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; }
-
-// x w^T (+ bias) for packed rows x [M, K], w [N, K]
+// x w^T (+ bias) for rows x [M, K] (packed ones in bf16), packed w [N, K]
 Tensor product(const Tensor& x, const Tensor& w, const Tensor& bias) {
   const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
   if (x.scalar_type() == at::kBFloat16 && vig_linear_preferred(M, (int)N, (int)K) && aligned(x) && aligned(w) &&
@@ -108,6 +136,10 @@ Tensor product(const Tensor& x, const Tensor& w, const Tensor& bias) {
                             stream_of(x)),
              "vig_linear_fwd");
     return y;
+  }
+  if (x.scalar_type() == at::kFloat) {
+    Tensor y = at::empty({M, N}, x.options());
+    if (matmul_f32(x, false, w, false, bias.defined() ? fptr(bias) : nullptr, Tensor(), y)) return y;
   }
   return bias.defined() ? at::addmm(bias, x, w.t()) : at::mm(x, w.t());
 }
@@ -120,6 +152,10 @@ Tensor input_grad(const Tensor& dy, const Tensor& w) {
     check_rc(vig_linear_bwd_input(dy.data_ptr(), w.data_ptr(), dx.data_ptr(), M, (int)N, (int)K, VIG_BF16, stream_of(dy)),
              "vig_linear_bwd_input");
     return dx;
+  }
+  if (dy.scalar_type() == at::kFloat) {
+    Tensor dx = at::empty({M, K}, dy.options());
+    if (matmul_f32(dy, false, w, true, nullptr, Tensor(), dx)) return dx;
   }
   return at::mm(dy, w);
 }
@@ -234,7 +270,7 @@ struct MixNode : torch::autograd::Function<MixNode> {
                                        (int)m.H, (int)m.Dk, (int)kRank, (float)m.inv_norm, (float)m.clamp, VIG_BF16, VIG_BF16, stream),
                "vig_dirgate_lowrank_fwd");
     } else {
-      gate_lin = at::addmm(up_b, z.narrow(1, m.n1, kRank), up_w.t());
+      gate_lin = product(z.narrow(1, m.n1, kRank), up_w, up_b);
       check_rc(vig_dirgate_fwd(gate_lin.data_ptr(), gates.data_ptr(), (int)m.B, (int)m.L, (int)m.H, (int)m.Dk, (float)m.inv_norm,
                                (float)m.clamp, VIG_F32, VIG_F32, stream),
                "vig_dirgate_fwd");
@@ -334,7 +370,7 @@ struct MixNode : torch::autograd::Function<MixNode> {
                                (float)m.inv_norm, (float)m.clamp, VIG_F32, VIG_F32, stream),
                "vig_dirgate_bwd");
       Tensor d_low = dz.narrow(1, m.n1, kRank);
-      at::mm_out(d_low, dx, up_w);
+      if (!matmul_f32(dx, false, up_w, true, nullptr, Tensor(), d_low)) at::mm_out(d_low, dx, up_w);
     }
     if (wants(kUpW) || wants(kUpB)) {
       Tensor db;
@@ -345,14 +381,14 @@ struct MixNode : torch::autograd::Function<MixNode> {
     const Tensor dzs = dz.narrow(1, 0, m.n2);
     if (wants(kQkvW) || wants(kGateW) || wants(kGateB) || wants(kLowW)) {
       Tensor db;
-      const bool bias = wants(kGateB), bf = m.bf16;
-      const Tensor dw = weight_grad(dzs, xs.view({m.rows, m.C}), bias && bf ? &db : nullptr);
+      const bool bias = wants(kGateB);
+      const Tensor dw = weight_grad(dzs, xs.view({m.rows, m.C}), bias ? &db : nullptr);
       out[2 + kQkvW] = like_param(dw.narrow(0, 0, m.n0), out_w, {m.n0, m.C});
       out[2 + kGateW] = like_param(dw.narrow(0, m.n0, m.V), out_w, {m.V, m.C});
       out[2 + kLowW] = like_param(dw.narrow(0, m.n1, kRank), out_w, {kRank, m.C});
-      if (bias) out[2 + kGateB] = like_param(bf ? db.narrow(0, m.n0, m.V) : dz.narrow(1, m.n0, m.V).sum(0), out_w, {m.V});
+      if (bias) out[2 + kGateB] = like_param(db.narrow(0, m.n0, m.V), out_w, {m.V});
     }
-    at::addmm_out(d_xs, d_xs, dzs, w_in);
+    if (m.bf16 || !matmul_f32(dzs, false, w_in, true, nullptr, d_xs, d_xs)) at::addmm_out(d_xs, d_xs, dzs, w_in);
     const bool conv_grads = wants(kConvW) || (off[10] && wants(kConvB));
     Tensor d_y = at::empty({m.B, m.L, m.C}, opts), dw_db, ws;
     size_t need = 0;
@@ -439,7 +475,7 @@ struct MlpNode : torch::autograd::Function<MlpNode> {
                "vig_swiglu_bwd");
     }
     if (ctx->needs_input_grad(3)) out[3] = like_param(weight_grad(dz, y.view({rows, C}), nullptr), gate_w, {2 * I, C});
-    const Tensor d_y = at::mm(dz, wg);
+    const Tensor d_y = type == at::kFloat ? input_grad(dz, wg) : at::mm(dz, wg);
     const auto g = norm_bwd(sum, wide ? fptr(norm_w) : fptr(small), d_y, grads[1], off[3], ctx->needs_input_grad(2),
                             ctx->saved_data["eps"].toDouble());
     out[0] = g.branch, out[1] = g.residual;
