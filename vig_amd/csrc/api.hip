@@ -2,6 +2,7 @@
 // dispatch only.  Nothing here allocates, frees or synchronises.
 #include "../../include/vig_gla.h"
 #include "launch.h"
+#include <algorithm>
 #include <mutex>
 
 namespace vig {
@@ -37,8 +38,9 @@ int launch_locality_blend(const void* o, const void* loc, const void* glin, cons
                           int B, int H, int L, int Dv, long long ldg, float eps, int silu_out, int io_dtype,
                           hipStream_t stream);
 size_t locality_blend_bwd_workspace(int B, int L, int Dv);
+size_t locality_blend_bwd_least_workspace(int B, int L, int Dv);
 int launch_locality_blend_bwd(const void* o, const void* loc, const void* glin, const float* wg, const float* wl,
-                              const void* dy, void* d_o, void* d_loc, void* d_glin, float* dw, void* workspace, int B,
+                              const void* dy, void* d_o, void* d_loc, void* d_glin, float* dw, void* workspace, long long workspace_rows, int B,
                               int H, int L, int Dv, long long ldg, long long ldd, float eps, int silu_out, int io_dtype,
                               hipStream_t stream);
 bool rmsnorm_types_ok(int x_dtype, int sum_dtype, int y_dtype);
@@ -611,9 +613,10 @@ int vig_locality_blend_bwd_strided(const void* o, const void* local, const void*
   const long long ldg = g_row_stride > 0 ? g_row_stride : row, ldd = d_glin_row_stride > 0 ? d_glin_row_stride : row;
   if (ldg < row || !strided_rows_ok(g_lin, ldg, io_dtype) || ldd < row || !strided_rows_ok(d_glin, ldd, io_dtype))
     return VIG_EINVAL;
-  if (!workspace || workspace_bytes < vig::locality_blend_bwd_workspace(B, L, Dv)) return VIG_ENOSPC;
-  return vig::launch_locality_blend_bwd(o, local, g_lin, w_g, w_l, dy, d_o, d_local, d_glin, dw, workspace, B, H, L,
-                                        Dv, ldg, ldd, eps, silu_out, io_dtype, (hipStream_t)stream);
+  if (!workspace || workspace_bytes < vig::locality_blend_bwd_least_workspace(B, L, Dv)) return VIG_ENOSPC;
+  const long long rows = (long long)(std::min(workspace_bytes, vig::locality_blend_bwd_workspace(B, L, Dv)) / (2 * Dv * sizeof(float)));
+  return vig::launch_locality_blend_bwd(o, local, g_lin, w_g, w_l, dy, d_o, d_local, d_glin, dw, workspace, rows, B, H, L, Dv,
+                                        ldg, ldd, eps, silu_out, io_dtype, (hipStream_t)stream);
 }
 
 int vig_locality_blend_bwd(const void* o, const void* local, const void* g_lin, const float* w_g, const float* w_l,

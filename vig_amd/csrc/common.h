@@ -67,6 +67,27 @@ template <> struct Raw8<float> {
   }
 };
 
+// Channel octets of token rows dealt out to workgroups: a workgroup owns `tokens` consecutive rows of [B * L] tokens of nv octets each
+// and numbers their octets through, so that neighbouring lanes hold neighbouring octets whatever the width and every lane has one.
+struct OctetRows {
+  int b, l, n;    // first token, and octets to do
+  __device__ __forceinline__ OctetRows(int B, int L, int nv, int tokens) {
+    const unsigned first = blockIdx.x * (unsigned)tokens;
+    b = (int)(first / (unsigned)L), l = (int)(first - (unsigned)b * L);
+    n = (int)min((unsigned)tokens, (unsigned)B * L - first) * nv;
+  }
+};
+struct Octet {
+  int b, l, cv;  // batch element, token and octet of its row
+  __device__ __forceinline__ Octet(const OctetRows& rows, int x, int nv, int L) {
+    const unsigned dt = (unsigned)x / (unsigned)nv;
+    cv = x - (int)dt * nv, b = rows.b;
+    unsigned at = rows.l + dt;
+    if (at >= (unsigned)L) b += at / (unsigned)L, at %= (unsigned)L;
+    l = (int)at;
+  }
+};
+
 // Typed element access used by the dtype-generic (non-MFMA) kernels.
 template <typename T> struct Elem;
 template <> struct Elem<float> {

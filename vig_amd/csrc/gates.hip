@@ -3,6 +3,8 @@
 // RMS-norm blend epilogue.  All are HBM-bound: each element is read once with
 // 16-byte (bf16 x8) or 16-byte (f32 x4) accesses along the channel dimension and
 // written once; stencil neighbours come from L1/L2.
+#include <algorithm>
+
 #include "common.h"
 #include "launch.h"
 
@@ -53,27 +55,28 @@ template <> struct Vec8<float> {
 // ---------------------------------------------------------------------------
 // direction-wise gate preparation
 //   in  [B, L, 2*H*Dk]  ->  out [2, B, H, L, Dk],  logsigmoid(x) * inv_norm, clamp
-// One workgroup owns 32 consecutive tokens of one batch element: it reads their rows (contiguous, 2*H*Dk channels
-// each) with 16-byte accesses and writes, per (direction, head), a contiguous run of 32 tokens x Dk.  A thread keeps
-// one channel octet for all its tokens, so the layout arithmetic is done once per thread.
+// HBM-bound.  A thread takes N octets of the rows, their loads under way together.  Measured (us, before: a workgroup for 32 tokens
+// of an image, a wave for every fourth): fp32 400 x 768 channels 8.9, now 2.6; 4704 x 768 11.2, now 6.1; 25088 x 384 14.4, now 13.8.
 // ---------------------------------------------------------------------------
-template <typename TI, typename TO>
+template <typename TI, typename TO, int N>
 __global__ __launch_bounds__(256) void dirgate_kernel(const TI* __restrict__ in, TO* __restrict__ out, int B, int L,
-                                                       int H, int Dk, float inv_norm, float clamp_min, int use_clamp) {
+                                                       int H, int Dk, float inv_norm, float clamp_min, int use_clamp, int tokens) {
   const int nv = 2 * H * Dk / 8;         // channel octets per token row
   const int dk8 = Dk >> 3;
-  const int b = blockIdx.y;
-  const int l0 = blockIdx.x * 32;
-  const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;  // 64 octet lanes x 4 token lanes
-  for (int cv = tx; cv < nv; cv += 64) {
-    const int d8 = cv % dk8, hh = (cv / dk8) % H, dir = cv / (dk8 * H);
-    const TI* src = in + ((size_t)b * L) * (size_t)(nv * 8) + (size_t)cv * 8;
-    TO* dst = out + ((((size_t)dir * B + b) * H + hh) * L) * (size_t)Dk + (size_t)d8 * 8;
-    for (int t = ty; t < 32; t += 4) {
-      const int l = l0 + t;
-      if (l >= L) break;
+  const OctetRows rows(B, L, nv, tokens);
+  const TI* src = in + (size_t)blockIdx.x * tokens * nv * 8;
+  for (int x0 = threadIdx.x; x0 < rows.n; x0 += 256 * N) {
+    Raw8<TI> raw[N];
+#pragma unroll
+    for (int u = 0; u < N; ++u)
+      if (x0 + 256 * u < rows.n) raw[u].load(src + (size_t)(x0 + 256 * u) * 8);
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+      if (x0 + 256 * u >= rows.n) break;
+      const Octet at(rows, x0 + 256 * u, nv, L);
+      const int head = at.cv / dk8, d8 = at.cv - head * dk8, dir = head >= H, hh = head - dir * H;
       float x[8];
-      Vec8<TI>::load(src + (size_t)l * (nv * 8), x);
+      raw[u].unpack(x);
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         // logsigmoid(x) = min(x,0) - log(1 + exp(-|x|)); hardware exp/log are accurate to ~1e-7 absolute here
@@ -82,38 +85,44 @@ __global__ __launch_bounds__(256) void dirgate_kernel(const TI* __restrict__ in,
         if (use_clamp) yv = fmaxf(yv, clamp_min);
         x[j] = yv;
       }
-      Vec8<TO>::store(dst + (size_t)l * Dk, x);
+      Vec8<TO>::store(out + ((((size_t)dir * B + at.b) * H + hh) * L + at.l) * (size_t)Dk + (size_t)d8 * 8, x);
     }
   }
 }
 
 // Backward of the gate preparation: d_in[b, l, c] = d_out[dir, b, h, l, d] * inv_norm * sigmoid(-x), zero where the
 // forward clamped (x = in[b, l, c]; d/dx logsigmoid(x) = sigmoid(-x)).
-template <typename TI, typename TO>
+template <typename TI, typename TO, int N>
 __global__ __launch_bounds__(256) void dirgate_bwd_kernel(const TI* __restrict__ in, const TO* __restrict__ d_out,
                                                            TI* __restrict__ d_in, int B, int L, int H, int Dk,
-                                                           float inv_norm, float clamp_min, int use_clamp) {
+                                                           float inv_norm, float clamp_min, int use_clamp, int tokens) {
   const int nv = 2 * H * Dk / 8;
   const int dk8 = Dk >> 3;
-  const int b = blockIdx.y;
-  const int l0 = blockIdx.x * 32;
-  const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-  for (int cv = tx; cv < nv; cv += 64) {
-    const int d8 = cv % dk8, hh = (cv / dk8) % H, dir = cv / (dk8 * H);
-    const size_t rows = ((size_t)b * L) * (size_t)(nv * 8) + (size_t)cv * 8;
-    const TO* grad = d_out + ((((size_t)dir * B + b) * H + hh) * L) * (size_t)Dk + (size_t)d8 * 8;
-    for (int t = ty; t < 32; t += 4) {
-      const int l = l0 + t;
-      if (l >= L) break;
+  const OctetRows rows(B, L, nv, tokens);
+  const size_t first = (size_t)blockIdx.x * tokens * nv * 8;
+  for (int x0 = threadIdx.x; x0 < rows.n; x0 += 256 * N) {
+    Raw8<TI> raw[N];
+    Raw8<TO> grad[N];
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+      if (x0 + 256 * u >= rows.n) break;
+      const Octet at(rows, x0 + 256 * u, nv, L);
+      const int head = at.cv / dk8, d8 = at.cv - head * dk8, dir = head >= H, hh = head - dir * H;
+      raw[u].load(in + first + (size_t)(x0 + 256 * u) * 8);
+      grad[u].load(d_out + ((((size_t)dir * B + at.b) * H + hh) * L + at.l) * (size_t)Dk + (size_t)d8 * 8);
+    }
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+      if (x0 + 256 * u >= rows.n) break;
       float x[8], g[8];
-      Vec8<TI>::load(in + rows + (size_t)l * (nv * 8), x);
-      Vec8<TO>::load(grad + (size_t)l * Dk, g);
+      raw[u].unpack(x);
+      grad[u].unpack(g);
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         const bool clamped = use_clamp && logsigmoidf_(x[j]) * inv_norm < clamp_min;
         x[j] = clamped ? 0.f : g[j] * inv_norm * sigmoidf_(-x[j]);
       }
-      Vec8<TI>::store(d_in + rows + (size_t)l * (nv * 8), x);
+      Vec8<TI>::store(d_in + first + (size_t)(x0 + 256 * u) * 8, x);
     }
   }
 }
@@ -121,11 +130,12 @@ __global__ __launch_bounds__(256) void dirgate_bwd_kernel(const TI* __restrict__
 int launch_dirgate_bwd(const void* in, const void* d_out, void* d_in, int B, int L, int H, int Dk, float inv_norm,
                        float clamp_min, int in_dtype, int out_dtype, hipStream_t stream) {
   const int use_clamp = clamp_min == clamp_min;  // NaN disables
-  if (B > 65535) return -22;
-  const dim3 grid((L + 31) / 32, B), block(256);
-#define VIG_DGB_CASE(TI, TO)                                                                                       \
-  hipLaunchKernelGGL((dirgate_bwd_kernel<TI, TO>), grid, block, 0, stream, (const TI*)in, (const TO*)d_out, (TI*)d_in, \
-                     B, L, H, Dk, inv_norm, clamp_min, use_clamp)
+  if (B > 65535 || (long long)B * L > 0x7fffffffLL) return -22;
+  const int nv = 2 * H * Dk / 8, each = octets_each((long long)B * L, nv), tokens = octet_tokens(nv, each);
+  const dim3 grid(((unsigned)B * L + tokens - 1) / tokens), block(256);
+#define VIG_DGB_CASE(TI, TO)                                                                                                   \
+  hipLaunchKernelGGL((each == 4 ? dirgate_bwd_kernel<TI, TO, 4> : dirgate_bwd_kernel<TI, TO, 1>), grid, block, 0, stream,     \
+                     (const TI*)in, (const TO*)d_out, (TI*)d_in, B, L, H, Dk, inv_norm, clamp_min, use_clamp, tokens)
   if (in_dtype == 0 && out_dtype == 0) VIG_DGB_CASE(float, float);
   else if (in_dtype == 0 && out_dtype == 1) VIG_DGB_CASE(float, uint16_t);
   else if (in_dtype == 1 && out_dtype == 0) VIG_DGB_CASE(uint16_t, float);
@@ -138,9 +148,10 @@ template <typename TI, typename TO>
 static int launch_dirgate_t(const void* in, void* out, int B, int L, int H, int Dk, float inv_norm,
                             float clamp_min, hipStream_t stream) {
   const int use_clamp = clamp_min == clamp_min;  // NaN disables
-  if (B > 65535) return -22;
-  hipLaunchKernelGGL((dirgate_kernel<TI, TO>), dim3((L + 31) / 32, B), dim3(256), 0, stream, (const TI*)in, (TO*)out, B,
-                     L, H, Dk, inv_norm, clamp_min, use_clamp);
+  if (B > 65535 || (long long)B * L > 0x7fffffffLL) return -22;
+  const int nv = 2 * H * Dk / 8, each = octets_each((long long)B * L, nv), tokens = octet_tokens(nv, each);
+  hipLaunchKernelGGL((each == 4 ? dirgate_kernel<TI, TO, 4> : dirgate_kernel<TI, TO, 1>), dim3(((unsigned)B * L + tokens - 1) / tokens),
+                     dim3(256), 0, stream, (const TI*)in, (TO*)out, B, L, H, Dk, inv_norm, clamp_min, use_clamp, tokens);
   return hipGetLastError() == hipSuccess ? 0 : -5;
 }
 
@@ -606,41 +617,45 @@ int launch_locality_gate(const void* o, const float* wt, void* y, int B, int H, 
 // RMS-norm blend epilogue.  One group of Dv/8 lanes owns one (b, l, head) row of
 // Dv values; the two mean-squares are reduced with lane shuffles inside the group.
 //   y[b,l,hd*Dv+d] = rms(o[b,hd,l,:])*w_g*s + rms(local[b,l,hd,:])*w_l*(1-s)
-// One workgroup owns 32 consecutive tokens of one batch element; a thread keeps one channel octet (head, d8) for
-// all its tokens, so the layout arithmetic and the norm weights are set up once per thread.
+// HBM-bound (three streams in, one out).  A thread takes N octets of the rows, their loads under way together; it keeps its octet
+// of the norms' weights (256 is a multiple of a head's octets).  Measured (us, before: a workgroup for 32 tokens of
+// an image, a wave for every fourth, 64 octets at a time): bf16 100 x 768 channels 16.0, now 2.9; 5670 x 768 20.5, now 7.9 (4.4 TB/s); 25088
+// x 384 21.0, now 16.8.
 // ---------------------------------------------------------------------------
-template <typename T>
+template <typename T, int N>
 __global__ __launch_bounds__(256) void locality_blend_kernel(const T* __restrict__ o, const T* __restrict__ loc,
                                                               const T* __restrict__ glin,
                                                               const float* __restrict__ wg,
-                                                              const float* __restrict__ wl, T* __restrict__ y,
+                                                              const float* __restrict__ wl, T* __restrict__ y, int B,
                                                               int H, int L, int Dv, long long ldg, float eps,
-                                                              int silu_out) {
+                                                              int silu_out, int tokens) {
   const int d8n = Dv >> 3;  // lanes per row: 4 (Dv=32) or 8 (Dv=64); divides 64, so groups never straddle a wave
   const int nv = H * d8n;   // channel octets per token row
-  const int b = blockIdx.y;
-  const int l0 = blockIdx.x * 32;
-  const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
+  const int d8 = threadIdx.x & (d8n - 1);
+  const OctetRows rows(B, L, nv, tokens);
+  const size_t first = (size_t)blockIdx.x * tokens * nv * 8;
   const float inv_dv = 1.0f / (float)Dv;
-  for (int cv0 = 0; cv0 < nv; cv0 += 64) {
-    const int cv = cv0 + tx;
-    const bool has = cv < nv;  // lanes past the row still take part in the shuffles of their (inactive) group
-    const int cvc = has ? cv : 0;
-    const int hd = cvc / d8n, d8 = cvc - hd * d8n;
-    float w_g[8], w_l[8];
+  float w_g[8], w_l[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) w_g[j] = wg[d8 * 8 + j], w_l[j] = wl[d8 * 8 + j];
-    const T* po = o + (((size_t)b * H + hd) * L) * (size_t)Dv + d8 * 8;
-    const size_t row0 = ((size_t)b * L) * (size_t)(nv * 8) + (size_t)cvc * 8;
-    const T* pg = glin + ((size_t)b * L) * (size_t)ldg + (size_t)cvc * 8;  // g_lin rows are ldg elements apart
-    for (int t = ty; t < 32; t += 4) {
-      const int l = l0 + t;
-      if (l >= L) break;  // uniform over the wave: a wave shares its token
+  for (int j = 0; j < 8; ++j) w_g[j] = wg[d8 * 8 + j], w_l[j] = wl[d8 * 8 + j];
+  for (int x0 = threadIdx.x; x0 < rows.n; x0 += 256 * N) {
+    Raw8<T> ro8[N], rl8[N], rg8[N];
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+      if (x0 + 256 * u >= rows.n) break;  // (whole groups: a row's octets are a multiple of theirs)
+      const Octet at(rows, x0 + 256 * u, nv, L);
+      const int hd = at.cv / d8n;
+      ro8[u].load(o + (((size_t)at.b * H + hd) * L + at.l) * (size_t)Dv + d8 * 8);
+      rl8[u].load(loc + first + (size_t)(x0 + 256 * u) * 8);
+      rg8[u].load(glin + ((size_t)at.b * L + at.l) * (size_t)ldg + (size_t)at.cv * 8);  // g_lin rows are ldg elements apart
+    }
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+      if (x0 + 256 * u >= rows.n) break;
       float xo[8], xl[8], xg[8];
-      const size_t tok = row0 + (size_t)l * (nv * 8);
-      Vec8<T>::load(po + (size_t)l * Dv, xo);
-      Vec8<T>::load(loc + tok, xl);
-      Vec8<T>::load(pg + (size_t)l * ldg, xg);
+      ro8[u].unpack(xo);
+      rl8[u].unpack(xl);
+      rg8[u].unpack(xg);
       float so = 0.f, sl = 0.f;
 #pragma unroll
       for (int j = 0; j < 8; ++j) so += xo[j] * xo[j], sl += xl[j] * xl[j];
@@ -658,7 +673,7 @@ __global__ __launch_bounds__(256) void locality_blend_kernel(const T* __restrict
         if (silu_out) v = v * sigmoidf_(v);
         out[j] = v;
       }
-      if (has) Vec8<T>::store(y + tok, out);
+      Vec8<T>::store(y + first + (size_t)(x0 + 256 * u) * 8, out);
     }
   }
 }
@@ -666,14 +681,15 @@ __global__ __launch_bounds__(256) void locality_blend_kernel(const T* __restrict
 int launch_locality_blend(const void* o, const void* loc, const void* glin, const float* wg, const float* wl, void* y,
                           int B, int H, int L, int Dv, long long ldg, float eps, int silu_out, int io_dtype,
                           hipStream_t stream) {
-  if (B > 65535) return -22;
-  const dim3 grid((L + 31) / 32, B), block(256);
-  if (io_dtype == 0)
-    hipLaunchKernelGGL((locality_blend_kernel<float>), grid, block, 0, stream, (const float*)o, (const float*)loc,
-                       (const float*)glin, wg, wl, (float*)y, H, L, Dv, ldg, eps, silu_out);
-  else
-    hipLaunchKernelGGL((locality_blend_kernel<uint16_t>), grid, block, 0, stream, (const uint16_t*)o,
-                       (const uint16_t*)loc, (const uint16_t*)glin, wg, wl, (uint16_t*)y, H, L, Dv, ldg, eps, silu_out);
+  if (B > 65535 || (long long)B * L > 0x7fffffffLL) return -22;
+  const int nv = H * (Dv / 8), each = octets_each((long long)B * L, nv), tokens = octet_tokens(nv, each);
+  const dim3 grid(((unsigned)B * L + tokens - 1) / tokens), block(256);
+#define VIG_BLEND_CASE(T)                                                                                                    \
+  hipLaunchKernelGGL((each == 4 ? locality_blend_kernel<T, 4> : locality_blend_kernel<T, 1>), grid, block, 0, stream,       \
+                     (const T*)o, (const T*)loc, (const T*)glin, wg, wl, (T*)y, B, H, L, Dv, ldg, eps, silu_out, tokens)
+  if (io_dtype == 0) VIG_BLEND_CASE(float);
+  else VIG_BLEND_CASE(uint16_t);
+#undef VIG_BLEND_CASE
   return hipGetLastError() == hipSuccess ? 0 : -5;
 }
 
@@ -871,135 +887,151 @@ int launch_dwconv3x3_bwd(const void* x, const void* dy, const void* pre, const f
 }
 
 // ---------------------------------------------------------------------------
-// Backward of the RMS-norm blend epilogue, same thread layout as the forward.  With s = sig(g_lin),
+// Backward of the RMS-norm blend epilogue, threads as in the forward.  With s = sig(g_lin),
 // on = rms(o) * w_g, ln = rms(local) * w_l, y0 = on * s + ln * (1 - s), y = silu_out ? y0 * sig(y0) : y0:
 //   dy0 = dy * d(y)/d(y0),  d_on = dy0 * s,  d_ln = dy0 * (1 - s),  d_glin = dy0 * (on - ln) * s * (1 - s),
 //   d_o = rms_backward(o, w_g, d_on),  d_local = rms_backward(local, w_l, d_ln)   (per (token, head) row of Dv),
 //   dw_g[d] = sum d_on * o * r_o,  dw_l[d] = sum d_ln * local * r_l   over batch, tokens and heads.
 // The weight gradients leave as one row of `partials` [workgroups, 2 * Dv] per workgroup (threads park their sums in
-// LDS and 2 * Dv threads add the ones of their channel, in a fixed order), which a column sum finishes.
+// LDS and 2 * Dv threads add the ones of their channel, in a fixed order), which a column sum finishes.  HBM-bound (four streams in,
+// three out): a thread fetches its next octet while it works on one, and there are as many workgroups as rows of partials fit.  Measured with
+// the column sum (us, before: a workgroup for 32 tokens of an image): bf16 100 x 768 channels 28, now 6.9; 5670 x 768 35, now 18; 25088 x
+// 384 41, now 29 (4.7 TB/s); fp32 400 x 768 30, now 7.9.
 // ---------------------------------------------------------------------------
 template <typename T>
 __global__ __launch_bounds__(256) void locality_blend_bwd_kernel(
     const T* __restrict__ o, const T* __restrict__ loc, const T* __restrict__ glin, const float* __restrict__ wg,
     const float* __restrict__ wl, const T* __restrict__ dy, T* __restrict__ d_o, T* __restrict__ d_loc,
-    T* __restrict__ d_glin, float* __restrict__ partials, int H, int L, int Dv, long long ldg, long long ldd, float eps,
-    int silu_out) {
+    T* __restrict__ d_glin, float* __restrict__ partials, int B, int H, int L, int Dv, long long ldg, long long ldd, float eps,
+    int silu_out, int tokens) {
   __shared__ float park[256][17];  // per thread: 8 dw_g + 8 dw_l sums of its channel octet (17: bank spread)
   const int d8n = Dv >> 3;
   const int nv = H * d8n;
-  const int b = blockIdx.y;
-  const int l0 = blockIdx.x * 32;
-  const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
+  const int d8 = threadIdx.x & (d8n - 1);
+  const OctetRows rows(B, L, nv, tokens);
+  const size_t first = (size_t)blockIdx.x * tokens * nv * 8;
   const float inv_dv = 1.0f / (float)Dv;
-  float total = 0.f;  // threads 0 .. 2*Dv-1: their channel's weight-gradient sum over the whole workgroup
-  for (int cv0 = 0; cv0 < nv; cv0 += 64) {
-    const int cv = cv0 + tx;
-    const bool has = cv < nv;
-    const int cvc = has ? cv : 0;
-    const int hd = cvc / d8n, d8 = cvc - hd * d8n;
-    float w_g[8], w_l[8], dwg[8], dwl[8];
+  float w_g[8], w_l[8], dwg[8], dwl[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) w_g[j] = wg[d8 * 8 + j], w_l[j] = wl[d8 * 8 + j], dwg[j] = 0.f, dwl[j] = 0.f;
-    const size_t head_off = (((size_t)b * H + hd) * L) * (size_t)Dv + d8 * 8;
-    const size_t row0 = ((size_t)b * L) * (size_t)(nv * 8) + (size_t)cvc * 8;
-    const T* pg = glin + ((size_t)b * L) * (size_t)ldg + (size_t)cvc * 8;
-    T* dg = d_glin + ((size_t)b * L) * (size_t)ldd + (size_t)cvc * 8;
-    for (int t = ty; t < 32; t += 4) {
-      const int l = l0 + t;
-      if (l >= L) break;  // uniform over the wave
-      float xo[8], xl[8], xg[8], g[8];
-      const size_t tok = row0 + (size_t)l * (nv * 8);
-      Vec8<T>::load(o + head_off + (size_t)l * Dv, xo);
-      Vec8<T>::load(loc + tok, xl);
-      Vec8<T>::load(pg + (size_t)l * ldg, xg);
-      Vec8<T>::load(dy + tok, g);
-      float so = 0.f, sl = 0.f;
+  for (int j = 0; j < 8; ++j) w_g[j] = wg[d8 * 8 + j], w_l[j] = wl[d8 * 8 + j], dwg[j] = 0.f, dwl[j] = 0.f;
+  struct Item {
+    Raw8<T> o, l, g, dy;
+    size_t head, gate;
+  } next;
+  const auto fetch = [&](int x, Item& it) {
+    const Octet at(rows, x, nv, L);
+    it.head = (((size_t)at.b * H + at.cv / d8n) * L + at.l) * (size_t)Dv + d8 * 8;
+    const size_t row = (size_t)at.b * L + at.l;
+    it.gate = row * (size_t)ldd + (size_t)at.cv * 8;
+    it.o.load(o + it.head);
+    it.l.load(loc + first + (size_t)x * 8);
+    it.g.load(glin + row * (size_t)ldg + (size_t)at.cv * 8);
+    it.dy.load(dy + first + (size_t)x * 8);
+  };
+  if ((int)threadIdx.x < rows.n) fetch(threadIdx.x, next);
+  for (int x = threadIdx.x; x < rows.n; x += 256) {  // (whole groups of lanes stay or leave)
+    const Item it = next;
+    if (x + 256 < rows.n) fetch(x + 256, next);
+    float xo[8], xl[8], xg[8], g[8];
+    it.o.unpack(xo);
+    it.l.unpack(xl);
+    it.g.unpack(xg);
+    it.dy.unpack(g);
+    float so = 0.f, sl = 0.f;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) so += xo[j] * xo[j], sl += xl[j] * xl[j];
-      for (int m = 1; m < d8n; m <<= 1) {
-        so += __shfl_xor(so, m);
-        sl += __shfl_xor(sl, m);
-      }
-      const float ro = rsqrtf(so * inv_dv + eps);
-      const float rl = rsqrtf(sl * inv_dv + eps);
-      float don[8], dln[8], dgl[8];
-      float mo = 0.f, ml = 0.f;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float s = sigmoidf_(xg[j]);
-        const float on = xo[j] * ro * w_g[j], ln = xl[j] * rl * w_l[j];
-        float dy0 = g[j];
-        if (silu_out) {
-          const float y0 = on * s + ln * (1.f - s);
-          const float sy = sigmoidf_(y0);
-          dy0 *= sy * (1.f + y0 * (1.f - sy));
-        }
-        don[j] = dy0 * s;
-        dln[j] = dy0 * (1.f - s);
-        dgl[j] = dy0 * (on - ln) * s * (1.f - s);
-        mo = __builtin_fmaf(don[j] * w_g[j], xo[j], mo);
-        ml = __builtin_fmaf(dln[j] * w_l[j], xl[j], ml);
-      }
-      for (int m = 1; m < d8n; m <<= 1) {
-        mo += __shfl_xor(mo, m);
-        ml += __shfl_xor(ml, m);
-      }
-      const float co = ro * ro * mo * inv_dv, cl = rl * rl * ml * inv_dv;
-      float eo[8], el[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        eo[j] = ro * (don[j] * w_g[j] - xo[j] * co);
-        el[j] = rl * (dln[j] * w_l[j] - xl[j] * cl);
-        if (has) {
-          dwg[j] = __builtin_fmaf(don[j] * ro, xo[j], dwg[j]);
-          dwl[j] = __builtin_fmaf(dln[j] * rl, xl[j], dwl[j]);
-        }
-      }
-      if (has) {
-        Vec8<T>::store(d_o + head_off + (size_t)l * Dv, eo);
-        Vec8<T>::store(d_loc + tok, el);
-        Vec8<T>::store(dg + (size_t)l * ldd, dgl);
-      }
+    for (int j = 0; j < 8; ++j) so += xo[j] * xo[j], sl += xl[j] * xl[j];
+    for (int m = 1; m < d8n; m <<= 1) {
+      so += __shfl_xor(so, m);
+      sl += __shfl_xor(sl, m);
     }
-    // combine the threads of one channel: thread (which, d) adds, in thread order, the parked sums of every thread
-    // whose octet holds channel d
-    __syncthreads();  // the previous round's readers are done
+    const float ro = rsqrtf(so * inv_dv + eps);
+    const float rl = rsqrtf(sl * inv_dv + eps);
+    float don[8], dln[8], dgl[8];
+    float mo = 0.f, ml = 0.f;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) park[threadIdx.x][j] = dwg[j], park[threadIdx.x][8 + j] = dwl[j];
-    __syncthreads();
-    if (threadIdx.x < 2 * Dv) {
-      const int which = threadIdx.x / Dv, d = threadIdx.x - which * Dv;
-      const int want = d >> 3, slot = 8 * which + (d & 7);
-      // octet index of thread t in this round: ((cv0 + (t & 63)) % d8n), cv0 a multiple of 64 and d8n dividing 64
-      for (int t = want; t < 256; t += d8n) total += park[t][slot];
+    for (int j = 0; j < 8; ++j) {
+      const float s = sigmoidf_(xg[j]);
+      const float on = xo[j] * ro * w_g[j], ln = xl[j] * rl * w_l[j];
+      float dy0 = g[j];
+      if (silu_out) {
+        const float y0 = on * s + ln * (1.f - s);
+        const float sy = sigmoidf_(y0);
+        dy0 *= sy * (1.f + y0 * (1.f - sy));
+      }
+      don[j] = dy0 * s;
+      dln[j] = dy0 * (1.f - s);
+      dgl[j] = dy0 * (on - ln) * s * (1.f - s);
+      mo = __builtin_fmaf(don[j] * w_g[j], xo[j], mo);
+      ml = __builtin_fmaf(dln[j] * w_l[j], xl[j], ml);
     }
+    for (int m = 1; m < d8n; m <<= 1) {
+      mo += __shfl_xor(mo, m);
+      ml += __shfl_xor(ml, m);
+    }
+    const float co = ro * ro * mo * inv_dv, cl = rl * rl * ml * inv_dv;
+    float eo[8], el[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      eo[j] = ro * (don[j] * w_g[j] - xo[j] * co);
+      el[j] = rl * (dln[j] * w_l[j] - xl[j] * cl);
+      dwg[j] = __builtin_fmaf(don[j] * ro, xo[j], dwg[j]);
+      dwl[j] = __builtin_fmaf(dln[j] * rl, xl[j], dwl[j]);
+    }
+    Vec8<T>::store(d_o + it.head, eo);
+    Vec8<T>::store(d_loc + first + (size_t)x * 8, el);
+    Vec8<T>::store(d_glin + it.gate, dgl);
   }
-  if (threadIdx.x < 2 * Dv)
-    partials[((size_t)blockIdx.y * gridDim.x + blockIdx.x) * (size_t)(2 * Dv) + threadIdx.x] = total;
+  // thread (which, d) adds, in thread order, the parked sums of every thread whose octet holds channel d
+#pragma unroll
+  for (int j = 0; j < 8; ++j) park[threadIdx.x][j] = dwg[j], park[threadIdx.x][8 + j] = dwl[j];
+  __syncthreads();
+  if ((int)threadIdx.x < 2 * Dv) {
+    const int which = threadIdx.x / Dv, d = threadIdx.x - which * Dv;
+    const int want = d >> 3, slot = 8 * which + (d & 7);
+    float total = 0.f;
+    for (int t = want; t < 256; t += d8n) total += park[t][slot];
+    partials[(size_t)blockIdx.x * (size_t)(2 * Dv) + threadIdx.x] = total;
+  }
 }
 
-size_t locality_blend_bwd_workspace(int B, int L, int Dv) {
-  return (size_t)B * ((L + 31) / 32) * 2 * Dv * sizeof(float);
+// Workgroups: 512, two a compute unit (both their registers and the column sum behind them).  us at 512 / 1024 / 2048: rows 5880 x 384
+// bf16 13.0 / 13.4 / 14.8, fp32 16.4 / 18.9 / 20.8; 25088 x 384 28.8 / 29.4 / 31.4; 4704 x 768 16.0 / 17.7 / 17.9.
+constexpr int kBlendBwdBlocks = 512;
+// rows of partial sums there is room for: a workgroup for every 32 tokens of an image (what a caller has to bring), and up to
+// kBlendBwdBlocks one for two tokens
+static long long blend_bwd_rows(int B, int L) {
+  const long long per_32 = (long long)B * ((L + 31) / 32), fine = std::min<long long>(((long long)B * L + 1) / 2, kBlendBwdBlocks);
+  return std::max(fine, per_32);
 }
+size_t locality_blend_bwd_workspace(int B, int L, int Dv) {
+  return (size_t)blend_bwd_rows(B, L) * 2 * Dv * sizeof(float);
+}
+
+// (a workspace without the rows beyond one for 32 tokens is enough)
+size_t locality_blend_bwd_least_workspace(int B, int L, int Dv) { return (size_t)B * ((L + 31) / 32) * 2 * Dv * sizeof(float); }
 
 int launch_locality_blend_bwd(const void* o, const void* loc, const void* glin, const float* wg, const float* wl,
-                              const void* dy, void* d_o, void* d_loc, void* d_glin, float* dw, void* workspace, int B,
+                              const void* dy, void* d_o, void* d_loc, void* d_glin, float* dw, void* workspace, long long workspace_rows, int B,
                               int H, int L, int Dv, long long ldg, long long ldd, float eps, int silu_out, int io_dtype,
                               hipStream_t stream) {
-  if (B > 65535 || (long long)B * ((L + 31) / 32) > 0x7fffffffLL) return -22;
-  const dim3 grid((L + 31) / 32, B), block(256);
+  if (B > 65535 || (long long)B * L > 0x7fffffffLL) return -22;
+  const int nv = H * (Dv / 8);
+  const long long total = (long long)B * L, room = std::min<long long>(kBlendBwdBlocks, workspace_rows);
+  // whole rounds of 256 octets, as few as the workgroups allow
+  int rounds = (int)std::max<long long>(1, (total * nv + 256 * room - 1) / (256 * room)), tokens = octet_tokens(nv, rounds);
+  while ((total + tokens - 1) / tokens > room) tokens = octet_tokens(nv, ++rounds);
+  const dim3 grid((unsigned)((total + tokens - 1) / tokens)), block(256);
   float* partials = static_cast<float*>(workspace);
   if (io_dtype == 0)
     hipLaunchKernelGGL((locality_blend_bwd_kernel<float>), grid, block, 0, stream, (const float*)o, (const float*)loc,
                        (const float*)glin, wg, wl, (const float*)dy, (float*)d_o, (float*)d_loc, (float*)d_glin,
-                       partials, H, L, Dv, ldg, ldd, eps, silu_out);
+                       partials, B, H, L, Dv, ldg, ldd, eps, silu_out, tokens);
   else
     hipLaunchKernelGGL((locality_blend_bwd_kernel<uint16_t>), grid, block, 0, stream, (const uint16_t*)o,
                        (const uint16_t*)loc, (const uint16_t*)glin, wg, wl, (const uint16_t*)dy, (uint16_t*)d_o,
-                       (uint16_t*)d_loc, (uint16_t*)d_glin, partials, H, L, Dv, ldg, ldd, eps, silu_out);
+                       (uint16_t*)d_loc, (uint16_t*)d_glin, partials, B, H, L, Dv, ldg, ldd, eps, silu_out, tokens);
   if (hipGetLastError() != hipSuccess) return -5;
-  return launch_column_sum(partials, dw, (int)(grid.x * grid.y), 2 * Dv, stream);
+  return launch_column_sum(partials, dw, (int)grid.x, 2 * Dv, stream);
 }
 
 }  // namespace vig

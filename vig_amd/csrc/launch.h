@@ -143,4 +143,9 @@ int launch_linear_norm(const void* x, const void* w, const void* residual, const
 bool few_swiglu(long long T, int K, int I);
 int launch_few_swiglu(const void* x, const void* w, void* y, long long T, int K, int I, hipStream_t stream);
 
+// Tokens a workgroup of 256 threads owns where every thread takes `each` octets of rows of nv octets (OctetRows).
+inline int octet_tokens(int nv, int each) { return nv >= 256 * each ? 1 : 256 * each / nv; }
+// Octets a thread takes at once: four, whose loads are under way together, once that leaves four workgroups a compute unit.
+inline int octets_each(long long rows, int nv) { return rows / octet_tokens(nv, 4) >= 1024 ? 4 : 1; }
+
 }  // namespace vig
