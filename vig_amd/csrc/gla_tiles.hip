@@ -61,6 +61,10 @@ struct TileGeo {
   int nseg;
   const float* states;
   const float* maxima;
+  // gates made here from rank-16 rows (row `low_ld` elements apart) and their second layer [2 * heads * 32, 16]
+  const uint16_t *low, *up_w, *up_b;
+  long long low_ld;
+  float inv_norm, clamp;
 };
 
 // byte offsets of the workgroup's LDS areas
@@ -99,6 +103,19 @@ struct TileCtx {
   float oscale;
   const float* state_in;  // long sequences: this segment's slots (forward, then reverse direction)
   const float* state_top;  // ... and the sequence's maxima (kGlaScanMaxima floats per direction)
+  // gates from rank-16 rows: the tile's rows, the two directions' weights and biases of the slab's head
+  rsrc_t low;
+  unsigned low_pitch;
+  const uint16_t *up_w[2], *up_b[2];
+  int nvalid;  // tokens of the tile
+  float inv_norm, clamp;
+};
+
+// What a wave fetches to make its tile's gates: its tokens' rank-16 rows and, per direction, the weights and the bias of a lane's
+// channel (lane row r < 16: the even channel of pair cpair(r), else the odd one of pair cpair(r - 16)).
+struct LowRank {
+  u32x4_t x, w[2];
+  uint32_t b[2];
 };
 
 __device__ __forceinline__ float wave_max(float x) {
@@ -137,6 +154,37 @@ __device__ __forceinline__ void cumulative_gates(const uint32_t (&gD)[2][8], int
   }
 }
 
+// The same from rank-16 rows (32 key channels): x = low . w^T + b rounded to bf16, gate = logsigmoid(x) * inv_norm, clamped and
+// rounded to bf16, as vig_dirgate_lowrank_fwd stores it.  One matrix instruction makes the tile's 32 x 32 gates with a channel
+// per lane row and the tokens in the registers, which is the left operand of the cumulative product as it stands; with even
+// and odd channels in the two halves of the rows that product is one too: C[8p + c] = G[p][c].  Same bits as in two launches; the
+// gates' trip through memory (half as many bytes again as q, k and v) and a launch are gone.  Whole forward, two launches / this: ViG-T, one
+// image of 224 px 462 / 442 us, ViG-S, 256 images 4432 / 4299.
+template <bool FWD>
+__device__ __forceinline__ void cumulative_lowrank(const LowRank& low, float inv_norm, float clamp, int nvalid, int r, int h,
+                                                   f32x16_t& C) {
+  constexpr int dir = FWD ? 0 : 1;
+  const float bias = __uint_as_float(low.b[dir] << 16);
+  f32x16_t acc = {0.f};
+  acc = mfma(low.x, low.w[dir], acc);
+  u32x4_t gate[2];
+#pragma unroll
+  for (int i = 0; i < 16; i += 2) {
+    const uint32_t x = pack_bf16x2(acc[i] + bias, acc[i + 1] + bias);
+    // (no clamp: clamp is NaN and fmaxf returns the other operand)
+    gate[i >> 3][(i & 7) >> 1] = pack_bf16x2(fmaxf(logsigmoidf_(bf16lo_to_f32(x)) * inv_norm, clamp),
+                                             fmaxf(logsigmoidf_(bf16hi_to_f32(x)) * inv_norm, clamp));
+  }
+  if (nvalid < 32) {  // (tokens past the end: no gate)
+    const uint32_t kept = nvalid > 0 ? (0xFFFFFFFFu >> (32 - nvalid)) >> (4 * h) : 0u;
+    gate[0] &= keep_masks<0>(kept), gate[1] &= keep_masks<1>(kept);
+  }
+  const uint32_t kh = keep_bits<FWD>(r, h);
+  C = f32x16_t{0.f};
+  C = mfma(gate[0], keep_masks<0>(kh) & 0x3F803F80u, C);
+  C = mfma(gate[1], keep_masks<1>(kh) & 0x3F803F80u, C);
+}
+
 // the tile totals (G at the last token walked) travel from the one lane pair that holds them to a lane per channel:
 // sc[32h + 16p + 4g + m] = total of channel 8*NG*h + 8g + 2m + p
 template <bool FWD>
@@ -157,6 +205,23 @@ __device__ __forceinline__ void park_totals(f32x16_t (&G)[2], float* sc, int r, 
   wave_lds_sync();
 }
 
+// ... of gates in one accumulator (cumulative_lowrank); the places of channels there are not get zeros
+template <bool FWD>
+__device__ __forceinline__ void park_totals(f32x16_t& C, float* sc, int r, int h) {
+  asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 3" : "+v"(C));  // (as above)
+  if (r == (FWD ? 31 : 0)) {
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+#pragma unroll
+      for (int g = 0; g < 2; ++g) {
+        const f32x4_t x = {C[8 * p + 4 * g], C[8 * p + 4 * g + 1], C[8 * p + 4 * g + 2], C[8 * p + 4 * g + 3]};
+        *reinterpret_cast<f32x4_t*>(sc + 32 * h + 16 * p + 4 * g) = x;
+        *reinterpret_cast<f32x4_t*>(sc + 32 * h + 16 * p + 8 + 4 * g) = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      }
+  }
+  wave_lds_sync();
+}
+
 // Operands of one direction for this wave's tile, the publication of what other tiles need from it, and the diagonal
 // score tile (masked to the pairs the direction sees and rounded to fp16 pairs: the B operand of the value product).
 //   qh: q^ = q exp(G)      (B operand of every score product of this wave; kept)
@@ -166,14 +231,21 @@ __device__ __forceinline__ void park_totals(f32x16_t (&G)[2], float* sc, int r, 
 // channel's tile total is outside the form's range.
 // General form: inputs carry the power-of-two scales 2^-eq, 2^-ek; the diagonal tile uses the half-anchored pair
 // q~ = q exp(G - T/2), k~ = k exp(T/2 - G) as bf16 hi + lo, three MFMA terms per k-step.
-template <int NG, bool FWD, bool GENERAL>
-__device__ __forceinline__ bool prepare_direction(const uint32_t (&gD)[2][8], const u32x4_t (&rawq)[NG],
+template <int NG, bool FWD, bool GENERAL, bool LOW>
+__device__ __forceinline__ bool prepare_direction(const uint32_t (&gD)[2][8], const LowRank& low, float inv_norm, float clamp,
+                                                  int nvalid, const u32x4_t (&rawq)[NG],
                                                   const u32x4_t (&rawk)[NG], float* sc, _Float16* dtab, char* kreg,
                                                   int lane, int eq, int ek, u32x4_t (&qh)[NG], u32x4_t (&p16)[2]) {
   constexpr int HC = 8 * NG;
   f32x16_t G[2];
-  cumulative_gates<FWD>(gD, lane & 31, lane >> 5, G);
-  park_totals<FWD>(G, sc, lane & 31, lane >> 5);
+  if constexpr (LOW) {
+    cumulative_lowrank<FWD>(low, inv_norm, clamp, nvalid, lane & 31, lane >> 5, G[0]);
+    park_totals<FWD>(G[0], sc, lane & 31, lane >> 5);
+  } else {
+    cumulative_gates<FWD>(gD, lane & 31, lane >> 5, G);
+    park_totals<FWD>(G, sc, lane & 31, lane >> 5);
+  }
+  const auto gates = [&](int p, int c) { return LOW ? G[0][8 * p + c] : G[p][c]; };
   float tl = sc[lane] * kLog2e;
   bool wide = false;
   if (!GENERAL) wide = __builtin_amdgcn_ballot_w64(!(fabsf(tl) <= kTileRange)) != 0;
@@ -206,7 +278,7 @@ __device__ __forceinline__ bool prepare_direction(const uint32_t (&gD)[2][8], co
 #pragma unroll
       for (int m = 0; m < 4; ++m) {
         const int c = 4 * g + m;
-        const float x0 = G[0][c] * kLog2e, x1 = G[1][c] * kLog2e;
+        const float x0 = gates(0, c) * kLog2e, x1 = gates(1, c) * kLog2e;
         const uint32_t a16 = pack_f16x2(exp2_fast(x0), exp2_fast(x1));
         const uint32_t b16 = pack_f16x2(exp2_fast(-x0), exp2_fast(-x1));
         qh[g][m] = mul_f16x2(rawq[g][m], a16);
@@ -224,7 +296,7 @@ __device__ __forceinline__ bool prepare_direction(const uint32_t (&gD)[2][8], co
 #pragma unroll
         for (int p = 0; p < 2; ++p) {
           const float tl_c = p ? d1[m] : d0[m];
-          const float x = fmaxf(G[p][c] * kLog2e, kExpFloor);
+          const float x = fmaxf(gates(p, c) * kLog2e, kExpFloor);
           const float an = 0.5f * tl_c;
           qhat[p] = qv[p] * exp2_fast(x + fq);
           khat[p] = kv[p] * exp2_fast(tl_c - x + fk);
@@ -515,14 +587,14 @@ static_assert(offsetof(TileKernArgs, geo) == 6 * sizeof(void*) && offsetof(TileK
                   offsetof(TileKernArgs, gate_w) == 48 + sizeof(TileGeo) + 8 && alignof(TileGeo) == 8,
               "TileKernArgs has to mirror the parameter list of gla_tile_kernel");
 
-template <int NG, bool BIDIR, bool PITCHED, bool GATE, bool CHAIN>
+template <int NG, bool BIDIR, bool PITCHED, bool GATE, bool CHAIN, bool LOW>
 __device__ void tile_pass_general(const TileKernArgs* ka_in);
 
 // Everything one wave does for its slab.  When some tile of the slab is outside the fp16 form's range (GENERAL false), every wave
 // of the workgroup, before anything is stored, runs the general form (ka: the kernel's argument block) and ends there: a call
 // that came back would keep the accumulators alive across it, and the compiler then kept sixteen of them in per-lane memory
 // throughout, walks included (long sequences at Dk 32, 144 of 784 tokens: this kernel 38.7 -> 23.5 us).
-template <int NG, bool BIDIR, bool PITCHED, bool GENERAL, bool GATE, bool CHAIN>
+template <int NG, bool BIDIR, bool PITCHED, bool GENERAL, bool GATE, bool CHAIN, bool LOW>
 __device__ __forceinline__ void tile_pass(const TileCtx& cx, const TileKernArgs* ka) {
   const int lane = cx.lane, r = lane & 31, h = lane >> 5;
   const int ti = cx.ti, NT = cx.NT;
@@ -539,7 +611,18 @@ __device__ __forceinline__ void tile_pass(const TileCtx& cx, const TileKernArgs*
   u32x4_t rawq[NG], rawk[NG];
   if (PITCHED) issue_tdwords_pitched<0, 2, 4>(cx.v, r, h, cx.v_pitch, vD);
   else issue_tdwords<0, 2, 4>(cx.v, r, h, vD);
-  issue_tdwords<0, 2, NG>(cx.gf, r, h, gDf);
+  LowRank low;
+  if (LOW) {
+    const int c = 2 * cpair<2>(r & 15) + (r >> 4);
+    low.x = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(cx.low, (unsigned)r * cx.low_pitch + 16u * h, 0, 0));
+#pragma unroll
+    for (int d = 0; d < 2; ++d) {
+      low.w[d] = *reinterpret_cast<const u32x4_t*>(cx.up_w[d] + 16 * c + 8 * h);
+      low.b[d] = cx.up_b[d][c];
+    }
+  } else {
+    issue_tdwords<0, 2, NG>(cx.gf, r, h, gDf);
+  }
   if (PITCHED) {
     issue_raw_tile_pitched<NG>(cx.q, 0, r, h, cx.q_pitch, rawq);
     issue_raw_tile_pitched<NG>(cx.k, 0, r, h, cx.k_pitch, rawk);
@@ -547,7 +630,7 @@ __device__ __forceinline__ void tile_pass(const TileCtx& cx, const TileKernArgs*
     issue_raw_tile<NG>(cx.q, 0, r, h, rawq);
     issue_raw_tile<NG>(cx.k, 0, r, h, rawk);
   }
-  if (BIDIR) issue_tdwords<0, 2, NG>(cx.gb, r, h, gDb);
+  if (BIDIR && !LOW) issue_tdwords<0, 2, NG>(cx.gb, r, h, gDb);
   float top_f = 0.f, top_b = 0.f;
   if (CHAIN && lane < kGlaScanMaxima) top_f = cx.state_top[lane], top_b = BIDIR ? cx.state_top[kGlaScanMaxima + lane] : 0.f;
   // ---- magnitudes (Gram matrices of the raw rows); values: bf16 pairs -> fp16 pairs, published ----
@@ -618,7 +701,7 @@ __device__ __forceinline__ void tile_pass(const TileCtx& cx, const TileKernArgs*
   u32x4_t p16[2];
   {
     char* kreg = ti < NT - 1 ? lds + lay.kf + ti * TileLds<NG>::KB : nullptr;
-    if (prepare_direction<NG, true, GENERAL>(gDf, rawq, rawk, sc, dtab_f, kreg, lane, eq, ek, qhf, p16)) veto = true;
+    if (prepare_direction<NG, true, GENERAL, LOW>(gDf, low, cx.inv_norm, cx.clamp, cx.nvalid, rawq, rawk, sc, dtab_f, kreg, lane, eq, ek, qhf, p16)) veto = true;
   }
   VIG_PHASE();
   if (BIDIR) {
@@ -638,7 +721,7 @@ __device__ __forceinline__ void tile_pass(const TileCtx& cx, const TileKernArgs*
     // (lane-derived constants of this direction are built here, not carried from the top of the kernel)
     int lane_b = lane;
     asm volatile("" : "+v"(lane_b));
-    if (prepare_direction<NG, false, GENERAL>(gDb, rawq, rawk, sc, dtab_b, kreg, lane_b, eq, ek, qhb, pb)) veto = true;
+    if (prepare_direction<NG, false, GENERAL, LOW>(gDb, low, cx.inv_norm, cx.clamp, cx.nvalid, rawq, rawk, sc, dtab_b, kreg, lane_b, eq, ek, qhb, pb)) veto = true;
     // (the two directions meet on the pairs j = i only: one more fp16 rounding there)
 #pragma unroll
     for (int t = 0; t < 2; ++t)
@@ -663,7 +746,7 @@ __device__ __forceinline__ void tile_pass(const TileCtx& cx, const TileKernArgs*
   if (!GENERAL) {
     const float mine = lane < NT ? guard[4 * lane] : 0.0f;
     if (__builtin_amdgcn_ballot_w64(mine != 0.0f) != 0) {
-      tile_pass_general<NG, BIDIR, PITCHED, GATE, CHAIN>(ka);
+      tile_pass_general<NG, BIDIR, PITCHED, GATE, CHAIN, LOW>(ka);
       __builtin_amdgcn_endpgm();
     }
   }
@@ -699,7 +782,7 @@ __device__ __forceinline__ void tile_pass(const TileCtx& cx, const TileKernArgs*
   }
 }
 
-template <int NG, bool BIDIR, bool PITCHED, bool GATE, bool CHAIN>
+template <int NG, bool BIDIR, bool PITCHED, bool GATE, bool CHAIN, bool LOW>
 __device__ __forceinline__ TileCtx make_tile_ctx(const uint16_t* q, const uint16_t* k, const uint16_t* v,
                                                  const uint16_t* gf, const uint16_t* gb, uint16_t* o,
                                                  const TileGeo& geo, float oscale, const float* gate_w, char* lds) {
@@ -735,8 +818,21 @@ __device__ __forceinline__ TileCtx make_tile_ctx(const uint16_t* q, const uint16
     cx.k = chunk_rsrc(k + off * DK, nvalid, 2 * DK);
     cx.v = chunk_rsrc(v + off * 64, nvalid, 128);
   }
-  cx.gf = chunk_rsrc(gf + off * DK, nvalid, 2 * DK);
-  cx.gb = chunk_rsrc(BIDIR ? gb + off * DK : gf, BIDIR ? nvalid : 0, 2 * DK);
+  if (LOW) {
+    static_assert(!LOW || (NG == 2 && BIDIR && PITCHED && !GATE && !CHAIN), "gates from rank-16 rows: whole slabs of 32 key channels");
+    const int b = seq / geo.H, hd = seq - b * geo.H;
+    cx.low_pitch = 2u * (unsigned)geo.low_ld;
+    cx.low = chunk_rsrc(geo.low + ((long long)b * geo.L + tok) * geo.low_ld, nvalid, cx.low_pitch);
+    cx.nvalid = nvalid, cx.inv_norm = geo.inv_norm, cx.clamp = geo.clamp;
+#pragma unroll
+    for (int d = 0; d < 2; ++d) {
+      const int c = (d * geo.H + hd) * DK;
+      cx.up_w[d] = geo.up_w + 16 * c, cx.up_b[d] = geo.up_b + c;
+    }
+  } else {
+    cx.gf = chunk_rsrc(gf + off * DK, nvalid, 2 * DK);
+    cx.gb = chunk_rsrc(BIDIR ? gb + off * DK : gf, BIDIR ? nvalid : 0, 2 * DK);
+  }
   cx.o = chunk_rsrc(o + off * 64, nvalid, 128);
   return cx;
 }
@@ -745,7 +841,7 @@ __device__ __forceinline__ TileCtx make_tile_ctx(const uint16_t* q, const uint16
 // the kernel's arguments from the argument block itself (ka: the kernel's own kernarg segment pointer; the builtin
 // yields null inside a called function): handed over as parameters, the geometry would need a copy in per-lane
 // memory, and the compiler writes that copy at the top of the kernel, for every wave, redo or not.
-template <int NG, bool BIDIR, bool PITCHED, bool GATE, bool CHAIN>
+template <int NG, bool BIDIR, bool PITCHED, bool GATE, bool CHAIN, bool LOW>
 __device__ __noinline__ void tile_pass_general(const TileKernArgs* ka_in) {
 #if defined(__HIP_DEVICE_COMPILE__)  // (the host pass has no constant address space to copy the geometry from)
   // (a called function gets its arguments in vector registers: back to scalars, or every argument read through the
@@ -758,15 +854,15 @@ __device__ __noinline__ void tile_pass_general(const TileKernArgs* ka_in) {
   const KernArgPtr ka = (KernArgPtr)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(kp >> 32)) << 32) |
                                      (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)kp));
   const TileGeo geo = ka->geo;
-  const TileCtx cx = make_tile_ctx<NG, BIDIR, PITCHED, GATE, CHAIN>(ka->q, ka->k, ka->v, ka->gf, ka->gb, ka->o, geo,
+  const TileCtx cx = make_tile_ctx<NG, BIDIR, PITCHED, GATE, CHAIN, LOW>(ka->q, ka->k, ka->v, ka->gf, ka->gb, ka->o, geo,
                                                                      ka->oscale, ka->gate_w, lds);
-  tile_pass<NG, BIDIR, PITCHED, true, GATE, CHAIN>(cx, nullptr);
+  tile_pass<NG, BIDIR, PITCHED, true, GATE, CHAIN, LOW>(cx, nullptr);
 #endif
 }
 
 }  // namespace
 
-template <int NG, bool BIDIR, bool PITCHED, bool GATE, bool CHAIN = false>
+template <int NG, bool BIDIR, bool PITCHED, bool GATE, bool CHAIN = false, bool LOW = false>
 __global__ __launch_bounds__(1024, 4) void gla_tile_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
                                                           const uint16_t* __restrict__ v,
                                                           const uint16_t* __restrict__ gf,
@@ -775,14 +871,14 @@ __global__ __launch_bounds__(1024, 4) void gla_tile_kernel(const uint16_t* __res
                                                           const float* __restrict__ gate_w) {
   extern __shared__ __align__(16) char lds[];
   const TileKernArgs* ka = (const TileKernArgs*)__builtin_amdgcn_kernarg_segment_ptr();
-  const TileCtx cx = make_tile_ctx<NG, BIDIR, PITCHED, GATE, CHAIN>(q, k, v, gf, gb, o, geo, oscale, gate_w, lds);
-  tile_pass<NG, BIDIR, PITCHED, false, GATE, CHAIN>(cx, ka);
+  const TileCtx cx = make_tile_ctx<NG, BIDIR, PITCHED, GATE, CHAIN, LOW>(q, k, v, gf, gb, o, geo, oscale, gate_w, lds);
+  tile_pass<NG, BIDIR, PITCHED, false, GATE, CHAIN, LOW>(cx, ka);
 }
 
 // The general form alone, for launches whose caller knows the gates to be strong: with 256 registers per wave (one
 // workgroup per CU) it keeps its unpacked operands in registers, which the function above, bound to the fp16 form's
 // 128, has to send through per-lane memory.
-template <int NG, bool BIDIR, bool PITCHED, bool GATE, bool CHAIN = false>
+template <int NG, bool BIDIR, bool PITCHED, bool GATE, bool CHAIN = false, bool LOW = false>
 __global__ __launch_bounds__(512, 2) void gla_tile_wide_kernel(const uint16_t* __restrict__ q,
                                                                const uint16_t* __restrict__ k,
                                                                const uint16_t* __restrict__ v,
@@ -791,8 +887,8 @@ __global__ __launch_bounds__(512, 2) void gla_tile_wide_kernel(const uint16_t* _
                                                                TileGeo geo, float oscale,
                                                                const float* __restrict__ gate_w) {
   extern __shared__ __align__(16) char lds[];
-  const TileCtx cx = make_tile_ctx<NG, BIDIR, PITCHED, GATE, CHAIN>(q, k, v, gf, gb, o, geo, oscale, gate_w, lds);
-  tile_pass<NG, BIDIR, PITCHED, true, GATE, CHAIN>(cx, nullptr);
+  const TileCtx cx = make_tile_ctx<NG, BIDIR, PITCHED, GATE, CHAIN, LOW>(q, k, v, gf, gb, o, geo, oscale, gate_w, lds);
+  tile_pass<NG, BIDIR, PITCHED, true, GATE, CHAIN, LOW>(cx, nullptr);
 }
 
 constexpr int kTileMaxLds = 160 * 1024;
@@ -808,6 +904,7 @@ bool gla_tiles_supported(const GlaArgs& a) {
   if (!(a.io_dtype == 1 && a.gate_dtype == 1 && (a.Dk == 64 || a.Dk == 32) && a.Dv == 64 &&
         a.L <= (a.wide_gates ? 256 : gla_slab_tokens(a.Dk)) && !a.init_state && !a.final_state && !a.state_pass))
     return false;
+  if (a.low) return a.Dk == 32 && a.q_strides && a.k_strides && a.v_strides && !a.gate_w && !a.wide_gates && a.low_ld <= (1 << 20);
   if (a.gate_w) {  // fused locality gate: both directions, plain tensors, the padded grid has to fit in LDS
     if (!a.g_bwd || a.q_strides || a.k_strides || a.v_strides || a.gate_cols <= 0 || a.gate_rows <= 0 ||
         (long long)a.gate_cols * a.gate_rows != a.L)
@@ -818,29 +915,26 @@ bool gla_tiles_supported(const GlaArgs& a) {
   return true;
 }
 
-template <int NG, bool BIDIR, bool PITCHED, bool GATE, bool CHAIN = false>
+template <int NG, bool BIDIR, bool PITCHED, bool GATE, bool CHAIN = false, bool LOW = false>
 static int launch_tiles_t(const GlaArgs& a, const TileGeo& geo, int dev) {
   constexpr int kMaxDevices = 64;
   static bool attr_done_dev[kMaxDevices] = {};
-  const void* kf = reinterpret_cast<const void*>(gla_tile_kernel<NG, BIDIR, PITCHED, GATE, CHAIN>);
-  const void* kw = reinterpret_cast<const void*>(gla_tile_wide_kernel<NG, BIDIR, PITCHED, GATE, CHAIN>);
+  const void* kf = reinterpret_cast<const void*>(gla_tile_kernel<NG, BIDIR, PITCHED, GATE, CHAIN, LOW>);
+  const void* kw = nullptr;
+  if constexpr (!LOW) kw = reinterpret_cast<const void*>(gla_tile_wide_kernel<NG, BIDIR, PITCHED, GATE, CHAIN, LOW>);
   if (!attr_done_dev[dev]) {
     if (hipFuncSetAttribute(kf, hipFuncAttributeMaxDynamicSharedMemorySize, kTileMaxLds) != hipSuccess) return -5;
-    if (hipFuncSetAttribute(kw, hipFuncAttributeMaxDynamicSharedMemorySize, kTileMaxLds) != hipSuccess) return -5;
+    if (kw && hipFuncSetAttribute(kw, hipFuncAttributeMaxDynamicSharedMemorySize, kTileMaxLds) != hipSuccess) return -5;
     attr_done_dev[dev] = true;
   }
   const TileLds<NG> lay(geo.NT, GATE ? gate_stage_bytes(geo.gw, geo.gh) : 0);
   if (lay.total > kTileMaxLds) return -95;
-  if (geo.wide)
-    hipLaunchKernelGGL((gla_tile_wide_kernel<NG, BIDIR, PITCHED, GATE, CHAIN>), dim3(a.B * a.H, CHAIN ? geo.nseg : 1),
-                       dim3(64 * geo.NT), lay.total, a.stream,
-                       (const uint16_t*)a.q, (const uint16_t*)a.k, (const uint16_t*)a.v, (const uint16_t*)a.g_fwd,
-                       (const uint16_t*)a.g_bwd, (uint16_t*)a.o, geo, a.scale * a.out_scale, a.gate_w);
-  else
-    hipLaunchKernelGGL((gla_tile_kernel<NG, BIDIR, PITCHED, GATE, CHAIN>), dim3(a.B * a.H, CHAIN ? geo.nseg : 1),
-                       dim3(64 * geo.NT), lay.total, a.stream,
-                       (const uint16_t*)a.q, (const uint16_t*)a.k, (const uint16_t*)a.v, (const uint16_t*)a.g_fwd,
-                       (const uint16_t*)a.g_bwd, (uint16_t*)a.o, geo, a.scale * a.out_scale, a.gate_w);
+  auto kernel = gla_tile_kernel<NG, BIDIR, PITCHED, GATE, CHAIN, LOW>;
+  if constexpr (!LOW)
+    if (geo.wide) kernel = gla_tile_wide_kernel<NG, BIDIR, PITCHED, GATE, CHAIN, LOW>;
+  hipLaunchKernelGGL(kernel, dim3(a.B * a.H, CHAIN ? geo.nseg : 1), dim3(64 * geo.NT), lay.total, a.stream, (const uint16_t*)a.q,
+                     (const uint16_t*)a.k, (const uint16_t*)a.v, (const uint16_t*)a.g_fwd, (const uint16_t*)a.g_bwd, (uint16_t*)a.o, geo,
+                     a.scale * a.out_scale, a.gate_w);
   return hipGetLastError() == hipSuccess ? 0 : -5;
 }
 
@@ -875,6 +969,11 @@ int launch_gla_tiles(const GlaArgs& a) {
     return a.Dk == 64 ? launch_tiles_t<4, true, false, true>(a, geo, dev) : launch_tiles_t<2, true, false, true>(a, geo, dev);
   }
   geo.heads = 1;
+  if (a.low) {
+    geo.low = (const uint16_t*)a.low, geo.up_w = (const uint16_t*)a.up_w, geo.up_b = (const uint16_t*)a.up_b;
+    geo.low_ld = a.low_ld, geo.inv_norm = a.inv_norm, geo.clamp = a.clamp;
+    return launch_tiles_t<2, true, true, false, false, true>(a, geo, dev);
+  }
   if (a.Dk == 64) {
     if (pitched)
       return bidir ? launch_tiles_t<4, true, true, false>(a, geo, dev) : launch_tiles_t<4, false, true, false>(a, geo, dev);

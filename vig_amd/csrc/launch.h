@@ -40,6 +40,11 @@ struct GlaArgs {
   const long long* q_strides = nullptr;
   const long long* k_strides = nullptr;
   const long long* v_strides = nullptr;
+  // one-launch kernel, Dk 32, both directions, strided q, k, v: gates made from rank-16 rows [B, L, 16] (low_ld elements apart) and
+  // their second layer up_w [2 * H * Dk, 16], up_b, all bf16 (g_fwd, g_bwd are not read)
+  const void *low = nullptr, *up_w = nullptr, *up_b = nullptr;
+  long long low_ld = 0;
+  float inv_norm = 0.f, clamp = 0.f;  // (clamp NaN: none)
 };
 
 // Per (sequence, segment, direction) slot of a state pass: the 64 x 64 state contribution in the matrix cores' register

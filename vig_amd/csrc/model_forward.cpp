@@ -202,16 +202,25 @@ Tensor run(const Plan& p, const Tensor& images) {
     check_rc(vig_dwconv3x3_fwd(k.at(y), f32(b.conv_w), f32(b.conv_b), k.at(xs), (int)B, st.gh, st.gw, (int)C, b.act, VIG_BF16, k.stream),
              "vig_dwconv3x3_fwd");
     k.linear(xs, b.w_in, b.b_in, z, T);
-    check_rc(vig_dirgate_lowrank_fwd(k.at(z + n1c), ld, b.w_up.data_ptr(), b.b_up.data_ptr(), k.at(gates), (int)B, (int)L, b.H, b.Dk,
-                                     (int)b.w_up.size(1), (float)b.inv_norm, (float)b.clamp, VIG_BF16, VIG_BF16, k.stream),
-             "vig_dirgate_lowrank_fwd");
+    const bool fused = whole && b.Dk == 32 && b.w_up.size(1) == 16;
+    if (!fused)
+      check_rc(vig_dirgate_lowrank_fwd(k.at(z + n1c), ld, b.w_up.data_ptr(), b.b_up.data_ptr(), k.at(gates), (int)B, (int)L, b.H, b.Dk,
+                                       (int)b.w_up.size(1), (float)b.inv_norm, (float)b.clamp, VIG_BF16, VIG_BF16, k.stream),
+               "vig_dirgate_lowrank_fwd");
     const float scale = 1.0f / std::sqrt((float)b.Dk);
     const int64_t gb = gates + T * b.H * b.Dk;
     if (whole) {
       const long long sqk[3] = {(long long)(L * ld), b.Dk, ld}, sv[3] = {(long long)(L * ld), b.Dv, ld};
-      check_rc(vig_gla_slab_fwd(k.at(z), k.at(z + b.H * b.Dk), k.at(z + 2 * b.H * b.Dk), k.at(gates), k.at(gb), nullptr, k.at(o), (int)B,
-                                b.H, (int)L, b.Dk, b.Dv, sqk, sqk, sv, 0, 0, scale, 0.25f, VIG_BF16, VIG_BF16, k.stream),
-               "vig_gla_slab_fwd");
+      if (fused) {
+        check_rc(vig_gla_slab_lowrank_fwd(k.at(z), k.at(z + b.H * b.Dk), k.at(z + 2 * b.H * b.Dk), k.at(z + n1c), ld, b.w_up.data_ptr(),
+                                          b.b_up.data_ptr(), k.at(o), (int)B, b.H, (int)L, b.Dk, b.Dv, sqk, sqk, sv, (float)b.inv_norm,
+                                          (float)b.clamp, scale, 0.25f, VIG_BF16, k.stream),
+                 "vig_gla_slab_lowrank_fwd");
+      } else {
+        check_rc(vig_gla_slab_fwd(k.at(z), k.at(z + b.H * b.Dk), k.at(z + 2 * b.H * b.Dk), k.at(gates), k.at(gb), nullptr, k.at(o), (int)B,
+                                  b.H, (int)L, b.Dk, b.Dv, sqk, sqk, sv, 0, 0, scale, 0.25f, VIG_BF16, VIG_BF16, k.stream),
+                 "vig_gla_slab_fwd");
+      }
     } else {
       check_rc(vig_split_heads_fwd(k.at(z), k.at(q), k.at(kk), k.at(v), (int)B, (int)L, b.H, b.Dk, b.Dv, ld, VIG_BF16, k.stream),
                "vig_split_heads_fwd");

@@ -435,25 +435,39 @@ Tensor gla_block_mix(const Tensor& x, int64_t grid_h, int64_t grid_w, const Tens
   Tensor z = product(xs, w_in, b_in);
   const int64_t n0 = H * (2 * Dk + Dv), n1 = n0 + H * Dv, rank = w_up.size(1);
   TORCH_CHECK(z.size(-1) >= n1 + rank, "vig_amd: stacked projection is narrower than qkv | g | gate rows");
-  Tensor gates = dirgate_lowrank_fwd(z.narrow(-1, n1, rank), w_up, b_up, H, normalizer, clamp_min);
   Tensor o;
   const int64_t B = z.size(0), L = z.size(1), ld = z.size(-1);
-  if (z.scalar_type() == at::kBFloat16 && gates.scalar_type() == at::kBFloat16 && L <= vig_gla_slab_tokens((int)Dk) && Dv == 64 && ld % 8 == 0 && z.is_contiguous() && reinterpret_cast<uintptr_t>(z.data_ptr()) % 16 == 0) {
-    // the matrix-core slab kernel reads q, k, v in place from the projection's rows: no head-major copies
+  const auto in_place = [&](const Tensor& t) {
+    return t.device() == z.device() && t.scalar_type() == at::kBFloat16 && t.is_contiguous() && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+  };
+  const bool slab = in_place(z) && L <= vig_gla_slab_tokens((int)Dk) && Dv == 64 && ld % 8 == 0;
+  // the matrix-core slab kernel reads q, k, v in place from the projection's rows: no head-major copies
+  const long long sqk[3] = {(long long)(L * ld), (long long)Dk, (long long)ld}, sv[3] = {(long long)(L * ld), (long long)Dv, (long long)ld};
+  const auto* base = static_cast<const at::BFloat16*>(z.data_ptr());
+  const float scale = resolve_scale(-1.0, (int)Dk);
+  if (slab && Dk == 32 && rank == 16 && w_up.dim() == 2 && w_up.size(0) == 2 * H * Dk && b_up.numel() == 2 * H * Dk && in_place(w_up) &&
+      in_place(b_up)) {
     const c10::DeviceGuard guard(z.device());
     o = at::empty({B, H, L, Dv}, z.options());
-    const long long sqk[3] = {(long long)(L * ld), (long long)Dk, (long long)ld};
-    const long long sv[3] = {(long long)(L * ld), (long long)Dv, (long long)ld};
-    const auto* base = static_cast<const at::BFloat16*>(z.data_ptr());
-    Tensor gf = gates.select(0, 0), gb = gates.select(0, 1);
-    check_rc(vig_gla_slab_fwd(base, base + H * Dk, base + 2 * H * Dk, gf.data_ptr(), gb.data_ptr(), nullptr, o.data_ptr(), (int)B,
-                              (int)H, (int)L, (int)Dk, (int)Dv, sqk, sqk, sv, 0, 0, resolve_scale(-1.0, (int)Dk),
-                              (float)out_scale, VIG_BF16, VIG_BF16, stream_of(z)),
-             "vig_gla_slab_fwd");
+    check_rc(vig_gla_slab_lowrank_fwd(base, base + H * Dk, base + 2 * H * Dk, base + n1, ld, w_up.data_ptr(), b_up.data_ptr(), o.data_ptr(),
+                                      (int)B, (int)H, (int)L, (int)Dk, (int)Dv, sqk, sqk, sv, (float)(1.0 / normalizer),
+                                      clamp_arg(clamp_min), scale, (float)out_scale, VIG_BF16, stream_of(z)),
+             "vig_gla_slab_lowrank_fwd");
   } else {
-    auto qkv = split_heads_fwd(z.narrow(-1, 0, n0), H, Dk, Dv);
-    o = gla_bidir_fwd(std::get<0>(qkv), std::get<1>(qkv), std::get<2>(qkv), gates.select(0, 0), gates.select(0, 1), -1.0,
-                      out_scale, 0);
+    Tensor gates = dirgate_lowrank_fwd(z.narrow(-1, n1, rank), w_up, b_up, H, normalizer, clamp_min);
+    if (slab && gates.scalar_type() == at::kBFloat16) {
+      const c10::DeviceGuard guard(z.device());
+      o = at::empty({B, H, L, Dv}, z.options());
+      Tensor gf = gates.select(0, 0), gb = gates.select(0, 1);
+      check_rc(vig_gla_slab_fwd(base, base + H * Dk, base + 2 * H * Dk, gf.data_ptr(), gb.data_ptr(), nullptr, o.data_ptr(), (int)B,
+                                (int)H, (int)L, (int)Dk, (int)Dv, sqk, sqk, sv, 0, 0, scale, (float)out_scale, VIG_BF16, VIG_BF16,
+                                stream_of(z)),
+               "vig_gla_slab_fwd");
+    } else {
+      auto qkv = split_heads_fwd(z.narrow(-1, 0, n0), H, Dk, Dv);
+      o = gla_bidir_fwd(std::get<0>(qkv), std::get<1>(qkv), std::get<2>(qkv), gates.select(0, 0), gates.select(0, 1), -1.0,
+                        out_scale, 0);
+    }
   }
   return locality_blend_linear_fwd(o, xs, z.narrow(-1, n0, H * Dv), w_gnorm, w_lnorm, w_o, eps, out_act);
 }
