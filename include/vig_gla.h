@@ -123,16 +123,19 @@ int vig_gla_slab_fwd(const void* q, const void* k, const void* v, const void* g_
                      int grid_h, int grid_w, float scale, float out_scale, int io_dtype, int gate_dtype, void* stream);
 
 /*
- * vig_gla_slab_fwd with the gates made on the way, as vig_dirgate_lowrank_fwd makes them (same roundings), instead of read:
- * low [B, L, 16] (rows low_row_stride elements apart), up_w [2*H*Dk, 16], up_b [2*H*Dk], clamp_min NaN for none; all bf16.
- * Dk 32, Dv 64, both directions, L <= vig_gla_slab_tokens(32), all three strides given; VIG_ENOTSUP for anything else.
+ * The bidirectional op with q, k, v read in place and the gates made on the way, as vig_dirgate_lowrank_fwd makes them (same
+ * roundings), instead of read: low [B, L, 16] (rows low_row_stride elements apart), up_w [2*H*Dk, 16], up_b [2*H*Dk], clamp_min NaN
+ * for none; all bf16.  Dk 32, Dv 64, all three strides given (as for _strided); VIG_ENOTSUP for anything else.  Any length; past
+ * vig_gla_slab_tokens(32) tokens the workspace (vig_gla_lowrank_fwd_workspace bytes) holds the states that link the segments.
  *
- * Replaces: classification/models/vig.py:410-435 in one launch (gate up-projection, log-sigmoid, direction split, the op).
+ * Replaces: classification/models/vig.py:401-435 (head split, gate up-projection, log-sigmoid, direction split, the op).
  */
-int vig_gla_slab_lowrank_fwd(const void* q, const void* k, const void* v, const void* low, long long low_row_stride,
-                             const void* up_w, const void* up_b, void* o, int B, int H, int L, int Dk, int Dv,
-                             const long long* q_strides, const long long* k_strides, const long long* v_strides,
-                             float inv_norm, float clamp_min, float scale, float out_scale, int io_dtype, void* stream);
+size_t vig_gla_lowrank_fwd_workspace(int B, int H, int L, int Dk, int Dv);
+int vig_gla_lowrank_fwd(const void* q, const void* k, const void* v, const void* low, long long low_row_stride,
+                        const void* up_w, const void* up_b, void* o, void* workspace, size_t workspace_bytes,
+                        int B, int H, int L, int Dk, int Dv,
+                        const long long* q_strides, const long long* k_strides, const long long* v_strides,
+                        float inv_norm, float clamp_min, float scale, float out_scale, int io_dtype, void* stream);
 
 /* Workspace that is enough for every gate dtype and for one or two directions (the largest over the kernels the
  * call may dispatch to for this shape and io_dtype). */

@@ -30,7 +30,8 @@ SIGNATURES = {
     "vig_gla_bidir_fwd_wide": (_c_int, _GLA_SIG),
     "vig_gla_bidir_fwd_strided": (_c_int, [_c_void_p] * 6 + [_c_int] * 5 + [_c_void_p] * 3 + [_c_float, _c_float, _c_int, _c_int, _c_void_p]),
     "vig_gla_slab_tokens": (_c_int, [_c_int]),
-    "vig_gla_slab_lowrank_fwd": (_c_int, [_c_void_p] * 4 + [_c_longlong] + [_c_void_p] * 3 + [_c_int] * 5 + [_c_void_p] * 3 + [_c_float] * 4 + [_c_int, _c_void_p]),
+    "vig_gla_lowrank_fwd_workspace": (_c_size_t, [_c_int] * 5),
+    "vig_gla_lowrank_fwd": (_c_int, [_c_void_p] * 4 + [_c_longlong] + [_c_void_p] * 4 + [_c_size_t] + [_c_int] * 5 + [_c_void_p] * 3 + [_c_float] * 4 + [_c_int, _c_void_p]),
     "vig_gla_slab_fwd": (_c_int, [_c_void_p] * 7 + [_c_int] * 5 + [_c_void_p] * 3 + [_c_int] * 2 + [_c_float, _c_float, _c_int, _c_int, _c_void_p]),
     "vig_gla_bidir_fwd_workspace": (_c_size_t, [_c_int] * 6),
     "vig_gla_bidir_fwd_noalloc": (_c_int, [_c_void_p] * 6 + [_c_int] * 5 + [_c_float, _c_float, _c_int, _c_int, _c_void_p]),

@@ -266,18 +266,22 @@ int vig_gla_slab_fwd(const void* q, const void* k, const void* v, const void* g_
   return vig::gla_tiles_supported(a) ? vig::launch_gla_tiles(a) : VIG_ENOTSUP;
 }
 
-// The same with the gates made on the way from their rank-16 rows.
-int vig_gla_slab_lowrank_fwd(const void* q, const void* k, const void* v, const void* low, long long low_row_stride, const void* up_w,
-                             const void* up_b, void* o, int B, int H, int L, int Dk, int Dv, const long long* q_strides,
-                             const long long* k_strides, const long long* v_strides, float inv_norm, float clamp_min, float scale,
-                             float out_scale, int io_dtype, void* stream) {
+// The op with the gates made on the way from their rank-16 rows, q, k, v in place.
+size_t vig_gla_lowrank_fwd_workspace(int B, int H, int L, int Dk, int Dv) {
+  return B <= 0 || H <= 0 || L <= 0 || Dk != 32 || Dv != 64 || L <= vig::gla_slab_tokens(Dk) ? 0 : vig::gla_mfma_workspace(B, H, L, Dk, Dv);
+}
+
+int vig_gla_lowrank_fwd(const void* q, const void* k, const void* v, const void* low, long long low_row_stride, const void* up_w,
+                        const void* up_b, void* o, void* workspace, size_t workspace_bytes, int B, int H, int L, int Dk, int Dv,
+                        const long long* q_strides, const long long* k_strides, const long long* v_strides, float inv_norm,
+                        float clamp_min, float scale, float out_scale, int io_dtype, void* stream) {
   vig::GlaArgs a;
-  const int rc = fill_args(a, q, k, v, low, low, o, nullptr, 0, B, H, L, Dk, Dv, scale, out_scale, io_dtype, io_dtype, stream);
+  const int rc = fill_args(a, q, k, v, low, low, o, workspace, workspace_bytes, B, H, L, Dk, Dv, scale, out_scale, io_dtype, io_dtype, stream);
   if (rc != VIG_OK) return rc;
   if (!up_w || !up_b || !aligned16(up_w) || low_row_stride < 16 || !strided_rows_ok(low, low_row_stride, io_dtype)) return VIG_EINVAL;
   a.q_strides = q_strides, a.k_strides = k_strides, a.v_strides = v_strides;
   a.low = low, a.up_w = up_w, a.up_b = up_b, a.low_ld = low_row_stride, a.inv_norm = inv_norm, a.clamp = clamp_min;
-  return vig::gla_tiles_supported(a) ? vig::launch_gla_tiles(a) : VIG_ENOTSUP;
+  return vig::launch_gla_lowrank(a);
 }
 
 // The causal op with a state carried in and / or out.

@@ -1178,6 +1178,21 @@ static int launch_gla_mfma_t(const GlaArgs& a, int num_cu, int dev) {
   return hipGetLastError() == hipSuccess ? 0 : -5;
 }
 
+// a sequence of any length with its gates made on the way (GlaArgs::low)
+int launch_gla_lowrank(const GlaArgs& a) {
+  if (gla_tiles_supported(a)) return launch_gla_tiles(a);
+  if (!gla_tiles_chain_supported(a)) return -95;
+  if (!a.workspace || a.workspace_bytes < gla_mfma_workspace(a.B, a.H, a.L, a.Dk, a.Dv)) return -28;
+  const Geometry geo = make_geometry(a.B * a.H, a.L, true);
+  float* ws = (float*)a.workspace;
+  const int rc = launch_gla_states(a, geo.seg_len, geo.nseg, ws, nullptr, nullptr, nullptr);
+  if (rc) return rc;
+  float* maxima = ws + (size_t)geo.nitems * 2 * kStateFloats;
+  launch_scan(ws, nullptr, a.B * a.H, geo.nseg, 2, 2, nullptr, nullptr, maxima, a.stream);
+  if (hipGetLastError() != hipSuccess) return -5;
+  return launch_gla_tiles_chain(a, ws, maxima);
+}
+
 int launch_gla_mfma(const GlaArgs& a) {
   // whole-sequence slabs go to the tile-pair kernel (VIG_GLA_CHUNKED_SLABS=1 keeps them here: comparisons only)
   static const bool chunked_slabs = [] {

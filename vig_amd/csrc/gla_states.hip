@@ -26,6 +26,11 @@ struct StateArgs {
   const uint16_t *q, *d_o;          // gradient set (blockIdx.z = 1), or null
   float *slots, *grad_slots;        // [sequence][segment][2] slots of kGlaStateFloats
   int L, seg_len, nseg;
+  // k, v inside wider rows: strides (batch, head, token) in elements; gates made from rank-16 rows (low_ld elements apart), see gla_tiles.hip
+  long long sk[3], sv[3], low_ld;
+  const uint16_t *low, *up_w, *up_b;
+  float inv_norm, clamp;
+  int H;
 };
 
 constexpr int kStateTiles = 16;  // most tiles of a segment
@@ -61,9 +66,18 @@ __device__ __forceinline__ void add_tile(const u32x4_t (&kf)[2][2], const u32x4_
     }
 }
 
+// LOW (Dk 32): one matrix instruction per channel parity makes a tile's gates of both directions from its rank-16 rows, where the lanes
+// would have read them.
+__device__ __forceinline__ void lowrank_gates(u32x4_t x, u32x4_t w, float bias, float inv_norm, float clamp, int rows, int h,
+                                              u32x4_t (&gate)[2]) {
+  f32x16_t acc = {0.f};
+  acc = mfma(x, w, acc);
+  lowrank_to_gates(acc, bias, inv_norm, clamp, rows, h, gate);
+}
+
 }  // namespace
 
-template <int NG>
+template <int NG, bool LOW = false>
 __global__ __launch_bounds__(512, 2) void gla_states_kernel(StateArgs a) {
   extern __shared__ __align__(16) char lds[];
   constexpr int DK = 16 * NG;
@@ -71,7 +85,7 @@ __global__ __launch_bounds__(512, 2) void gla_states_kernel(StateArgs a) {
   constexpr int NDIR = kJoint ? 1 : 2;
   const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), waves = (int)blockDim.x >> 6;
   const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
-  const bool grad = blockIdx.z != 0, bidir = a.gb != nullptr;
+  const bool grad = !LOW && blockIdx.z != 0, bidir = LOW || a.gb != nullptr;
   const int seq = blockIdx.x, seg = blockIdx.y;
   float* tot = reinterpret_cast<float*>(lds);  // [direction][tile][p][lane row]
   char* red = lds + 2 * kStateTiles * 64 * 4;
@@ -80,6 +94,18 @@ __global__ __launch_bounds__(512, 2) void gla_states_kernel(StateArgs a) {
   const int rho = kJoint ? r & 15 : r;
   const unsigned ch2 = cpair<NG>(rho);
   uint32_t gD[NDIR][2][2][8], kD[2][2][8], vD[2][2][8];
+  static_assert(!LOW || kJoint, "gates from rank-16 rows: 32 key channels");
+  const int batch = LOW ? seq / a.H : 0, head = LOW ? seq - batch * a.H : 0;
+  u32x4_t lowx[2], loww[2];
+  uint32_t lowb[2];
+  if (LOW) {
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      const int c = ((r >> 4) * a.H + head) * DK + 2 * (int)ch2 + p;
+      loww[p] = *reinterpret_cast<const u32x4_t*>(a.up_w + 16 * (size_t)c + 8 * h);
+      lowb[p] = a.up_b[c];
+    }
+  }
   const unsigned base = (4u * h) * (2u * DK) + 4u * ch2;
   size_t at[2];
   int rows[2];
@@ -87,7 +113,13 @@ __global__ __launch_bounds__(512, 2) void gla_states_kernel(StateArgs a) {
   for (int i = 0; i < 2; ++i) {  // (all gates first: the totals are out, and the first tile's products at work, while the rest arrives)
     const int tok = seg * a.seg_len + 32 * (2 * w + i);
     rows[i] = __builtin_amdgcn_readfirstlane(max(0, min(32, min(a.L, (seg + 1) * a.seg_len) - tok)));
-    at[i] = (size_t)seq * a.L + (rows[i] > 0 ? tok : 0);
+    at[i] = LOW ? (size_t)(rows[i] > 0 ? tok : 0) : (size_t)seq * a.L + (rows[i] > 0 ? tok : 0);
+    if constexpr (LOW) {
+      const unsigned pitch = 2u * (unsigned)a.low_ld;
+      const rsrc_t rl = chunk_rsrc(a.low + ((long long)batch * a.L + (long long)at[i]) * a.low_ld, rows[i], pitch);
+      lowx[i] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rl, (unsigned)r * pitch + 16u * h, 0, 0));
+      continue;
+    }
     const rsrc_t rf = chunk_rsrc(a.gf + at[i] * DK, rows[i], 2 * DK);
     const rsrc_t rb = chunk_rsrc((bidir ? a.gb : a.gf) + at[i] * DK, bidir ? rows[i] : 0, 2 * DK);
 #pragma unroll
@@ -107,6 +139,18 @@ __global__ __launch_bounds__(512, 2) void gla_states_kernel(StateArgs a) {
   }
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
+    if constexpr (LOW) {
+      const unsigned pk = 2u * (unsigned)a.sk[2], pv = 2u * (unsigned)a.sv[2];
+      const rsrc_t rk = chunk_rsrc(a.k + batch * a.sk[0] + head * a.sk[1] + (long long)at[i] * a.sk[2], rows[i], pk);
+      const rsrc_t rv = chunk_rsrc(a.v + batch * a.sv[0] + head * a.sv[1] + (long long)at[i] * a.sv[2], rows[i], pv);
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          kD[i][t][e] = __builtin_amdgcn_raw_buffer_load_b32(rk, (4u * h) * pk + 4u * ch2, (unsigned)jmap(t, 0, e) * pk, 0);
+      issue_tdwords_pitched<0, 2, 4>(rv, r, h, pv, vD[i]);
+      continue;
+    }
     const rsrc_t rk = chunk_rsrc((grad ? a.q : a.k) + at[i] * DK, rows[i], 2 * DK);
     const rsrc_t rv = chunk_rsrc((grad ? a.d_o : a.v) + at[i] * 64, rows[i], 128);
 #pragma unroll
@@ -124,9 +168,14 @@ __global__ __launch_bounds__(512, 2) void gla_states_kernel(StateArgs a) {
   for (int d = 0; d < NDIR; ++d)
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-      finish_tfrags<2>(gD[d][i], gfrag[d][i]);
+      if constexpr (!LOW) finish_tfrags<2>(gD[d][i], gfrag[d][i]);
 #pragma unroll
       for (int p = 0; p < 2; ++p) {
+        if constexpr (LOW) {
+          u32x4_t gate[2];
+          lowrank_gates(lowx[i], loww[p], __uint_as_float(lowb[p] << 16), a.inv_norm, a.clamp, rows[i], h, gate);
+          gfrag[d][i][0][p] = gate[0], gfrag[d][i][1][p] = gate[1];
+        }
         f32x16_t T = {0.f};
         T = mfma(ones, gfrag[d][i][0][p], T);
         T = mfma(ones, gfrag[d][i][1][p], T);
@@ -227,11 +276,20 @@ __global__ __launch_bounds__(512, 2) void gla_states_kernel(StateArgs a) {
 int launch_gla_states(const GlaArgs& a, int seg_len, int nseg, float* slots, const void* q, const void* d_o, float* grad_slots) {
   const int NT = (seg_len + 31) / 32;
   if (NT < 1 || NT > kStateTiles || nseg > 65535) return -22;
-  const StateArgs s{(const uint16_t*)a.k, (const uint16_t*)a.v, (const uint16_t*)a.g_fwd, (const uint16_t*)a.g_bwd,
-                    (const uint16_t*)q, (const uint16_t*)d_o, slots, grad_slots, a.L, seg_len, nseg};
+  StateArgs s{(const uint16_t*)a.k, (const uint16_t*)a.v, (const uint16_t*)a.g_fwd, (const uint16_t*)a.g_bwd,
+              (const uint16_t*)q, (const uint16_t*)d_o, slots, grad_slots, a.L, seg_len, nseg};
   const int waves = (NT + 1) / 2;
   const dim3 grid(a.B * a.H, nseg, q ? 2 : 1), block(64 * waves);
-  static bool done[2][64] = {};
+  static bool done[3][64] = {};
+  if (a.low) {
+    if (a.Dk != 32 || q || !a.k_strides || !a.v_strides) return -22;
+    for (int j = 0; j < 3; ++j) s.sk[j] = a.k_strides[j], s.sv[j] = a.v_strides[j];
+    s.low = (const uint16_t*)a.low, s.up_w = (const uint16_t*)a.up_w, s.up_b = (const uint16_t*)a.up_b;
+    s.low_ld = a.low_ld, s.inv_norm = a.inv_norm, s.clamp = a.clamp, s.H = a.H;
+    if (!allow_lds(reinterpret_cast<const void*>(gla_states_kernel<2, true>), state_lds(kStateTiles / 2), done[2])) return -5;
+    hipLaunchKernelGGL((gla_states_kernel<2, true>), grid, block, state_lds(waves), a.stream, s);
+    return hipGetLastError() == hipSuccess ? 0 : -5;
+  }
   const void* kernel = a.Dk == 64 ? reinterpret_cast<const void*>(gla_states_kernel<4>) : reinterpret_cast<const void*>(gla_states_kernel<2>);
   if (!allow_lds(kernel, state_lds(kStateTiles / 2), done[a.Dk == 64])) return -5;
   if (a.Dk == 64) hipLaunchKernelGGL(gla_states_kernel<4>, grid, block, state_lds(waves), a.stream, s);

@@ -168,17 +168,7 @@ __device__ __forceinline__ void cumulative_lowrank(const LowRank& low, float inv
   f32x16_t acc = {0.f};
   acc = mfma(low.x, low.w[dir], acc);
   u32x4_t gate[2];
-#pragma unroll
-  for (int i = 0; i < 16; i += 2) {
-    const uint32_t x = pack_bf16x2(acc[i] + bias, acc[i + 1] + bias);
-    // (no clamp: clamp is NaN and fmaxf returns the other operand)
-    gate[i >> 3][(i & 7) >> 1] = pack_bf16x2(fmaxf(logsigmoidf_(bf16lo_to_f32(x)) * inv_norm, clamp),
-                                             fmaxf(logsigmoidf_(bf16hi_to_f32(x)) * inv_norm, clamp));
-  }
-  if (nvalid < 32) {  // (tokens past the end: no gate)
-    const uint32_t kept = nvalid > 0 ? (0xFFFFFFFFu >> (32 - nvalid)) >> (4 * h) : 0u;
-    gate[0] &= keep_masks<0>(kept), gate[1] &= keep_masks<1>(kept);
-  }
+  lowrank_to_gates(acc, bias, inv_norm, clamp, nvalid, h, gate);
   const uint32_t kh = keep_bits<FWD>(r, h);
   C = f32x16_t{0.f};
   C = mfma(gate[0], keep_masks<0>(kh) & 0x3F803F80u, C);
@@ -819,7 +809,7 @@ __device__ __forceinline__ TileCtx make_tile_ctx(const uint16_t* q, const uint16
     cx.v = chunk_rsrc(v + off * 64, nvalid, 128);
   }
   if (LOW) {
-    static_assert(!LOW || (NG == 2 && BIDIR && PITCHED && !GATE && !CHAIN), "gates from rank-16 rows: whole slabs of 32 key channels");
+    static_assert(!LOW || (NG == 2 && BIDIR && PITCHED && !GATE), "gates from rank-16 rows: 32 key channels, both directions");
     const int b = seq / geo.H, hd = seq - b * geo.H;
     cx.low_pitch = 2u * (unsigned)geo.low_ld;
     cx.low = chunk_rsrc(geo.low + ((long long)b * geo.L + tok) * geo.low_ld, nvalid, cx.low_pitch);
@@ -900,11 +890,16 @@ constexpr int kTileMaxLds = 160 * 1024;
 // The general form's own kernel has twice the registers per wave and takes eight.
 int gla_slab_tokens(int Dk) { return Dk == 64 ? 416 : 512; }
 
+static bool lowrank_ok(const GlaArgs& a) {
+  return a.io_dtype == 1 && a.Dk == 32 && a.Dv == 64 && a.g_bwd && a.q_strides && a.k_strides && a.v_strides && !a.gate_w && !a.wide_gates &&
+         a.low_ld <= (1 << 20);
+}
+
 bool gla_tiles_supported(const GlaArgs& a) {
   if (!(a.io_dtype == 1 && a.gate_dtype == 1 && (a.Dk == 64 || a.Dk == 32) && a.Dv == 64 &&
         a.L <= (a.wide_gates ? 256 : gla_slab_tokens(a.Dk)) && !a.init_state && !a.final_state && !a.state_pass))
     return false;
-  if (a.low) return a.Dk == 32 && a.q_strides && a.k_strides && a.v_strides && !a.gate_w && !a.wide_gates && a.low_ld <= (1 << 20);
+  if (a.low) return lowrank_ok(a);
   if (a.gate_w) {  // fused locality gate: both directions, plain tensors, the padded grid has to fit in LDS
     if (!a.g_bwd || a.q_strides || a.k_strides || a.v_strides || a.gate_cols <= 0 || a.gate_rows <= 0 ||
         (long long)a.gate_cols * a.gate_rows != a.L)
@@ -938,6 +933,29 @@ static int launch_tiles_t(const GlaArgs& a, const TileGeo& geo, int dev) {
   return hipGetLastError() == hipSuccess ? 0 : -5;
 }
 
+// the caller's strides, plain ones where there are none: rows 16-byte aligned, pitches within the descriptors' 32-bit extents
+static int fill_strides(const GlaArgs& a, TileGeo& geo) {
+  const long long* given[3] = {a.q_strides, a.k_strides, a.v_strides};
+  long long* dst[3] = {geo.sq, geo.sk, geo.sv};
+  const int D[3] = {a.Dk, a.Dk, a.Dv};
+  for (int i = 0; i < 3; ++i) {
+    if (given[i] && given[i][2] != 0) {
+      // rows 16-byte aligned, pitches within the descriptors' 32-bit extents
+      for (int j = 0; j < 3; ++j)
+        if (given[i][j] <= 0 || given[i][j] % 8 != 0) return -22;
+      if (given[i][2] > (1 << 20)) return -22;
+      dst[i][0] = given[i][0], dst[i][1] = given[i][1], dst[i][2] = given[i][2];
+    } else {
+      dst[i][0] = (long long)a.H * a.L * D[i], dst[i][1] = (long long)a.L * D[i], dst[i][2] = D[i];
+    }
+  }
+  return 0;
+}
+static void fill_lowrank(const GlaArgs& a, TileGeo& geo) {
+  geo.low = (const uint16_t*)a.low, geo.up_w = (const uint16_t*)a.up_w, geo.up_b = (const uint16_t*)a.up_b;
+  geo.low_ld = a.low_ld, geo.inv_norm = a.inv_norm, geo.clamp = a.clamp;
+}
+
 int launch_gla_tiles(const GlaArgs& a) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return -5;
@@ -947,22 +965,8 @@ int launch_gla_tiles(const GlaArgs& a) {
   geo.H = a.H;
   geo.wide = a.wide_gates;
   const bool pitched = a.q_strides || a.k_strides || a.v_strides;
-  if (pitched) {
-    const long long* given[3] = {a.q_strides, a.k_strides, a.v_strides};
-    long long* dst[3] = {geo.sq, geo.sk, geo.sv};
-    const int D[3] = {a.Dk, a.Dk, a.Dv};
-    for (int i = 0; i < 3; ++i) {
-      if (given[i] && given[i][2] != 0) {
-        // rows 16-byte aligned, pitches within the descriptors' 32-bit extents
-        for (int j = 0; j < 3; ++j)
-          if (given[i][j] <= 0 || given[i][j] % 8 != 0) return -22;
-        if (given[i][2] > (1 << 20)) return -22;
-        dst[i][0] = given[i][0], dst[i][1] = given[i][1], dst[i][2] = given[i][2];
-      } else {
-        dst[i][0] = (long long)a.H * a.L * D[i], dst[i][1] = (long long)a.L * D[i], dst[i][2] = D[i];
-      }
-    }
-  }
+  if (pitched)
+    if (const int rc = fill_strides(a, geo)) return rc;
   const bool bidir = a.g_bwd != nullptr;
   if (a.gate_w) {
     geo.gw = a.gate_cols, geo.gh = a.gate_rows, geo.heads = a.H;
@@ -970,8 +974,7 @@ int launch_gla_tiles(const GlaArgs& a) {
   }
   geo.heads = 1;
   if (a.low) {
-    geo.low = (const uint16_t*)a.low, geo.up_w = (const uint16_t*)a.up_w, geo.up_b = (const uint16_t*)a.up_b;
-    geo.low_ld = a.low_ld, geo.inv_norm = a.inv_norm, geo.clamp = a.clamp;
+    fill_lowrank(a, geo);
     return launch_tiles_t<2, true, true, false, false, true>(a, geo, dev);
   }
   if (a.Dk == 64) {
@@ -986,7 +989,7 @@ int launch_gla_tiles(const GlaArgs& a) {
 
 bool gla_tiles_chain_supported(const GlaArgs& a) {
   return a.io_dtype == 1 && a.gate_dtype == 1 && (a.Dk == 64 || a.Dk == 32) && a.Dv == 64 && a.L > 256 && !a.init_state &&
-         !a.final_state && !a.state_pass && !a.gate_w && !a.q_strides && !a.k_strides && !a.v_strides &&
+         !a.final_state && !a.state_pass && !a.gate_w && (a.low ? lowrank_ok(a) : !a.q_strides && !a.k_strides && !a.v_strides) &&
          gla_tile_segments(a.L) <= 65535;
 }
 
@@ -1003,6 +1006,11 @@ int launch_gla_tiles_chain(const GlaArgs& a, const float* states, const float* m
   geo.nseg = gla_tile_segments(a.L);
   geo.states = states;
   geo.maxima = maxima;
+  if (a.low) {
+    if (const int rc = fill_strides(a, geo)) return rc;
+    fill_lowrank(a, geo);
+    return launch_tiles_t<2, true, true, false, true, true>(a, geo, dev);
+  }
   const bool bidir = a.g_bwd != nullptr;
   if (a.Dk == 64)
     return bidir ? launch_tiles_t<4, true, false, false, true>(a, geo, dev) : launch_tiles_t<4, false, false, false, true>(a, geo, dev);

@@ -40,7 +40,7 @@ struct GlaArgs {
   const long long* q_strides = nullptr;
   const long long* k_strides = nullptr;
   const long long* v_strides = nullptr;
-  // one-launch kernel, Dk 32, both directions, strided q, k, v: gates made from rank-16 rows [B, L, 16] (low_ld elements apart) and
+  // tile-pair and state kernels, Dk 32, both directions, strided q, k, v: gates made from rank-16 rows [B, L, 16] (low_ld elements apart) and
   // their second layer up_w [2 * H * Dk, 16], up_b, all bf16 (g_fwd, g_bwd are not read)
   const void *low = nullptr, *up_w = nullptr, *up_b = nullptr;
   long long low_ld = 0;
@@ -105,6 +105,7 @@ size_t gla_recurrent_workspace(int B, int H, int L, int Dv, int io_dtype);
 // bf16 MFMA chunked path (bf16 io and gates).
 bool gla_mfma_supported(const GlaArgs& a);
 int launch_gla_mfma(const GlaArgs& a);
+int launch_gla_lowrank(const GlaArgs& a);
 // bf16 tile-pair path for whole-sequence slabs (L <= 256): one wave per 32-token tile, both directions per wave.
 bool gla_tiles_supported(const GlaArgs& a);
 int gla_slab_tokens(int Dk);  // longest sequence that one workgroup takes whole

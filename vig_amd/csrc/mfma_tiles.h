@@ -168,6 +168,24 @@ __device__ __forceinline__ u32x4_t keep_masks(uint32_t kh) {
   return u32x4_t{keep_mask<T, 0>(kh), keep_mask<T, 1>(kh), keep_mask<T, 2>(kh), keep_mask<T, 3>(kh)};
 }
 
+// Gates of a 32-token tile from the second layer's product (a lane: one channel, accumulator register 8t + e the token of slot e of
+// k-step t): x = product + bias rounded to bf16, logsigmoid(x) * inv_norm, clamped (clamp NaN: not), rounded to bf16; tokens from
+// `rows` on get no gate.
+__device__ __forceinline__ void lowrank_to_gates(const f32x16_t& acc, float bias, float inv_norm, float clamp, int rows, int h,
+                                                 u32x4_t (&gate)[2]) {
+#pragma unroll
+  for (int i = 0; i < 16; i += 2) {
+    const uint32_t x = pack_bf16x2(acc[i] + bias, acc[i + 1] + bias);
+    // (fmaxf returns the other operand of a NaN)
+    gate[i >> 3][(i & 7) >> 1] = pack_bf16x2(fmaxf(logsigmoidf_(bf16lo_to_f32(x)) * inv_norm, clamp),
+                                             fmaxf(logsigmoidf_(bf16hi_to_f32(x)) * inv_norm, clamp));
+  }
+  if (rows < 32) {
+    const uint32_t kept = rows > 0 ? (0xFFFFFFFFu >> (32 - rows)) >> (4 * h) : 0u;
+    gate[0] &= keep_masks<0>(kept), gate[1] &= keep_masks<1>(kept);
+  }
+}
+
 template <int NG, int STRIDE = kKtStride>
 __device__ __forceinline__ void store_kt(uint16_t* kt, int row, int h, const u32x4_t (&kh)[NG]) {
 #pragma unroll

@@ -144,21 +144,27 @@ Tensor run(const Plan& p, const Tensor& images) {
     nz = std::max(nz, b.w_in.size(0)), I = std::max(I, b.w_down.size(1)), K2 = std::max<int64_t>(K2, 2 * b.H * b.Dk);
     swiglu_kernel = swiglu_kernel && b.w_down.size(1) % 32 == 0;
   }
-  bool whole = true;  // q, k, v are read in place from the projection's rows
-  for (const auto& b : p.blocks) whole = whole && L <= vig_gla_slab_tokens(b.Dk);
+  // q, k, v are read in place from the projection's rows, with the gates made in the same kernels or by one of their own, or split into heads
+  const auto lowrank = [&](const Block& b) { return b.Dk == 32 && b.Dv == 64 && b.w_up.size(1) == 16; };
+  const auto whole = [&](const Block& b) { return L <= vig_gla_slab_tokens(b.Dk); };
+  bool all_lowrank = true, all_in_place = true;
   size_t gla_ws = 0;
-  if (!whole)
-    for (const auto& b : p.blocks)
-      gla_ws = std::max(gla_ws, vig_gla_bidir_fwd_workspace_for((int)B, b.H, (int)L, b.Dk, b.Dv, VIG_BF16, VIG_BF16, 1));
+  for (const auto& b : p.blocks) {
+    all_lowrank = all_lowrank && lowrank(b), all_in_place = all_in_place && (lowrank(b) || whole(b));
+    const size_t need = lowrank(b) ? vig_gla_lowrank_fwd_workspace((int)B, b.H, (int)L, b.Dk, b.Dv)
+                        : whole(b) ? 0
+                                   : vig_gla_bidir_fwd_workspace_for((int)B, b.H, (int)L, b.Dk, b.Dv, VIG_BF16, VIG_BF16, 1);
+    gla_ws = std::max(gla_ws, need);
+  }
   Walk k;
   k.stream = stream_of(images);
   // branch and residual alternate between two places each; the mixer's and the MLP's intermediates share one region
   const int64_t branch0 = k.take(T * C), branch1 = k.take(T * C), res0 = k.take(T * C), res1 = k.take(T * C), y = k.take(T * C),
                 xs = k.take(T * C), o = k.take(T * C);
   const int64_t region = k.used;
-  const int64_t z = k.take(T * nz), gates = k.take(T * K2);
-  int64_t q = 0, kk = 0, v = 0, ws = 0;
-  if (!whole) q = k.take(T * K2 / 2), kk = k.take(T * K2 / 2), v = k.take(T * C), ws = k.take((int64_t)(gla_ws + 1) / 2);
+  const int64_t z = k.take(T * nz), gates = all_lowrank ? 0 : k.take(T * K2), ws = k.take((int64_t)(gla_ws + 1) / 2);
+  int64_t q = 0, kk = 0, v = 0;
+  if (!all_in_place) q = k.take(T * K2 / 2), kk = k.take(T * K2 / 2), v = k.take(T * C);
   int64_t most = k.used;
   k.used = region;
   const int64_t mid = k.take(T * I), wide = swiglu_kernel ? 0 : k.take(T * 2 * I);
@@ -202,31 +208,29 @@ Tensor run(const Plan& p, const Tensor& images) {
     check_rc(vig_dwconv3x3_fwd(k.at(y), f32(b.conv_w), f32(b.conv_b), k.at(xs), (int)B, st.gh, st.gw, (int)C, b.act, VIG_BF16, k.stream),
              "vig_dwconv3x3_fwd");
     k.linear(xs, b.w_in, b.b_in, z, T);
-    const bool fused = whole && b.Dk == 32 && b.w_up.size(1) == 16;
-    if (!fused)
+    const float scale = 1.0f / std::sqrt((float)b.Dk);
+    const long long sqk[3] = {(long long)(L * ld), b.Dk, ld}, sv[3] = {(long long)(L * ld), b.Dv, ld};
+    if (lowrank(b)) {
+      check_rc(vig_gla_lowrank_fwd(k.at(z), k.at(z + b.H * b.Dk), k.at(z + 2 * b.H * b.Dk), k.at(z + n1c), ld, b.w_up.data_ptr(),
+                                   b.b_up.data_ptr(), k.at(o), gla_ws ? k.at(ws) : nullptr, gla_ws, (int)B, b.H, (int)L, b.Dk, b.Dv, sqk,
+                                   sqk, sv, (float)b.inv_norm, (float)b.clamp, scale, 0.25f, VIG_BF16, k.stream),
+               "vig_gla_lowrank_fwd");
+    } else {
       check_rc(vig_dirgate_lowrank_fwd(k.at(z + n1c), ld, b.w_up.data_ptr(), b.b_up.data_ptr(), k.at(gates), (int)B, (int)L, b.H, b.Dk,
                                        (int)b.w_up.size(1), (float)b.inv_norm, (float)b.clamp, VIG_BF16, VIG_BF16, k.stream),
                "vig_dirgate_lowrank_fwd");
-    const float scale = 1.0f / std::sqrt((float)b.Dk);
-    const int64_t gb = gates + T * b.H * b.Dk;
-    if (whole) {
-      const long long sqk[3] = {(long long)(L * ld), b.Dk, ld}, sv[3] = {(long long)(L * ld), b.Dv, ld};
-      if (fused) {
-        check_rc(vig_gla_slab_lowrank_fwd(k.at(z), k.at(z + b.H * b.Dk), k.at(z + 2 * b.H * b.Dk), k.at(z + n1c), ld, b.w_up.data_ptr(),
-                                          b.b_up.data_ptr(), k.at(o), (int)B, b.H, (int)L, b.Dk, b.Dv, sqk, sqk, sv, (float)b.inv_norm,
-                                          (float)b.clamp, scale, 0.25f, VIG_BF16, k.stream),
-                 "vig_gla_slab_lowrank_fwd");
-      } else {
+      const int64_t gb = gates + T * b.H * b.Dk;
+      if (whole(b)) {
         check_rc(vig_gla_slab_fwd(k.at(z), k.at(z + b.H * b.Dk), k.at(z + 2 * b.H * b.Dk), k.at(gates), k.at(gb), nullptr, k.at(o), (int)B,
                                   b.H, (int)L, b.Dk, b.Dv, sqk, sqk, sv, 0, 0, scale, 0.25f, VIG_BF16, VIG_BF16, k.stream),
                  "vig_gla_slab_fwd");
+      } else {
+        check_rc(vig_split_heads_fwd(k.at(z), k.at(q), k.at(kk), k.at(v), (int)B, (int)L, b.H, b.Dk, b.Dv, ld, VIG_BF16, k.stream),
+                 "vig_split_heads_fwd");
+        check_rc(vig_gla_bidir_fwd(k.at(q), k.at(kk), k.at(v), k.at(gates), k.at(gb), k.at(o), k.at(ws), gla_ws, (int)B, b.H, (int)L, b.Dk,
+                                   b.Dv, scale, 0.25f, VIG_BF16, VIG_BF16, k.stream),
+                 "vig_gla_bidir_fwd");
       }
-    } else {
-      check_rc(vig_split_heads_fwd(k.at(z), k.at(q), k.at(kk), k.at(v), (int)B, (int)L, b.H, b.Dk, b.Dv, ld, VIG_BF16, k.stream),
-               "vig_split_heads_fwd");
-      check_rc(vig_gla_bidir_fwd(k.at(q), k.at(kk), k.at(v), k.at(gates), k.at(gb), k.at(o), k.at(ws), gla_ws, (int)B, b.H, (int)L, b.Dk,
-                                 b.Dv, scale, 0.25f, VIG_BF16, VIG_BF16, k.stream),
-               "vig_gla_bidir_fwd");
     }
     if (b.Dv == 64 && (C == 384 || C == 192)) {
       check_rc(vig_locality_blend_linear_fwd(k.at(o), k.at(xs), k.at(z + n0), f32(b.gn), f32(b.ln), b.w_o.data_ptr(), k.at(branch1), (int)B,

@@ -440,19 +440,21 @@ Tensor gla_block_mix(const Tensor& x, int64_t grid_h, int64_t grid_w, const Tens
   const auto in_place = [&](const Tensor& t) {
     return t.device() == z.device() && t.scalar_type() == at::kBFloat16 && t.is_contiguous() && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
   };
-  const bool slab = in_place(z) && L <= vig_gla_slab_tokens((int)Dk) && Dv == 64 && ld % 8 == 0;
-  // the matrix-core slab kernel reads q, k, v in place from the projection's rows: no head-major copies
+  const bool rows = in_place(z) && Dv == 64 && ld % 8 == 0, slab = rows && L <= vig_gla_slab_tokens((int)Dk);
+  // the matrix-core kernels read q, k, v in place from the projection's rows: no head-major copies
   const long long sqk[3] = {(long long)(L * ld), (long long)Dk, (long long)ld}, sv[3] = {(long long)(L * ld), (long long)Dv, (long long)ld};
   const auto* base = static_cast<const at::BFloat16*>(z.data_ptr());
   const float scale = resolve_scale(-1.0, (int)Dk);
-  if (slab && Dk == 32 && rank == 16 && w_up.dim() == 2 && w_up.size(0) == 2 * H * Dk && b_up.numel() == 2 * H * Dk && in_place(w_up) &&
+  if (rows && Dk == 32 && rank == 16 && w_up.dim() == 2 && w_up.size(0) == 2 * H * Dk && b_up.numel() == 2 * H * Dk && in_place(w_up) &&
       in_place(b_up)) {
     const c10::DeviceGuard guard(z.device());
     o = at::empty({B, H, L, Dv}, z.options());
-    check_rc(vig_gla_slab_lowrank_fwd(base, base + H * Dk, base + 2 * H * Dk, base + n1, ld, w_up.data_ptr(), b_up.data_ptr(), o.data_ptr(),
-                                      (int)B, (int)H, (int)L, (int)Dk, (int)Dv, sqk, sqk, sv, (float)(1.0 / normalizer),
-                                      clamp_arg(clamp_min), scale, (float)out_scale, VIG_BF16, stream_of(z)),
-             "vig_gla_slab_lowrank_fwd");
+    const size_t need = vig_gla_lowrank_fwd_workspace((int)B, (int)H, (int)L, (int)Dk, (int)Dv);
+    Tensor ws = need ? at::empty({(int64_t)need}, z.options().dtype(at::kByte)) : Tensor();
+    check_rc(vig_gla_lowrank_fwd(base, base + H * Dk, base + 2 * H * Dk, base + n1, ld, w_up.data_ptr(), b_up.data_ptr(), o.data_ptr(),
+                                 need ? ws.data_ptr() : nullptr, need, (int)B, (int)H, (int)L, (int)Dk, (int)Dv, sqk, sqk, sv,
+                                 (float)(1.0 / normalizer), clamp_arg(clamp_min), scale, (float)out_scale, VIG_BF16, stream_of(z)),
+             "vig_gla_lowrank_fwd");
   } else {
     Tensor gates = dirgate_lowrank_fwd(z.narrow(-1, n1, rank), w_up, b_up, H, normalizer, clamp_min);
     if (slab && gates.scalar_type() == at::kBFloat16) {
