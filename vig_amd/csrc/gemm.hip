@@ -432,11 +432,16 @@ static long long tiles_of(const GemmArgs& a, int tm, int tn) { return (long long
 // Where these kernels are the better choice (graph-captured runs on one MI355X; library times beside them):
 //   up to 640 tiles of 32 x 32: gemm_few_kernel  (M 196: N 192 K 512 3.1 us against 17.2, N 1280 K 384 3.5 / 5.2,
 //                               N 768 K 2048 4.7 / 6.9; past the line its operand traffic grows with the tile count)
-//   up to 2 GFLOP:              64 x 64 tiles    (M 1568 N 1280 K 384 6.5 / 6.9; M 6272 N 640 K 192 7.1 / 7.3)
+//   up to 9 GFLOP:              64 x 64 tiles    (M 1568 N 1280 K 384 6.1 / 6.9; M 2500 N 384 K 1024 8.0 / 8.0)
+//                               or, past 512 of them, 128 x 128 tiles  (M 3136 N 1280 K 384 8.3 / 9.1, with 64 x 64 tiles 10.3; M 9216 17.6 /
+//                               21.8, 22.9; M 4000 N 768 K 768 11.1 / 10.1, 13.3; M 1000 N 4096 K 768 13.4 / 11.2, 19.7)
+//                               (between 2 and 9 GFLOP a few us slower than the library on some sizes, at worst 18 %; but the library's
+//                               front end takes 22 us of host time a call, this one 4, and models of such products wait for the host, whole forward:
+//                               ViG-B, 2 images of 288 px, 37 products: 1.81 -> 1.06 ms; 8 of 208 px 1.84 -> 1.19; 4 of 320 px 2.05 -> 1.36; ViG-S, 16 of 224 px 0.95 -> 0.85)
 //   K 384 or 192, N % 64 == 0, 16384 rows and fewer for some N (regs_rows): weights in registers (linear.hip)
 //   K <= 256 with 512 tiles:    256 x 128 tiles  (M 65536 N 520 K 192: other column counts)
 // Beyond that the library's products win (M 50176 N 1280 K 512 and longer contractions).
-constexpr int kFewTiles = 640;
+constexpr int kFewTiles = 640, kSmallTiles = 512;
 // Rows from which the form with its weights in registers is the better one; the table for 16384 rows and up is beside
 // launch_linear_regs.  Below, the library's time goes up and down with its choice of tiles, by up to two between neighbouring
 // sizes (us, library / registers): K 192, N 640: 8192 rows 10.9 / 8.3, 9408 9.2 / 9.3, 14112 18.2 / 11.5; N 704 15.5 / 9.2 at 9408;
@@ -454,7 +459,7 @@ bool linear_preferred(long long M, int N, int K) {
   if (M <= 0 || M > 0x7fffffffLL - 256 || N <= 0 || K <= 0 || N % 8 || K % kStageK) return false;
   GemmArgs a{};
   a.M = (int)M, a.N = N, a.K = K;
-  return regs_preferred(M, N, K) || tiles_of(a, 32, 32) <= kFewTiles || 2.0 * M * N * K <= 2e9 || short_k_many(a);
+  return regs_preferred(M, N, K) || tiles_of(a, 32, 32) <= kFewTiles || 2.0 * M * N * K <= 9e9 || short_k_many(a);
 }
 
 int launch_linear(const void* x, long long ldx, const void* w, const void* bias, void* y, long long ldy, long long M, int N, int K,
@@ -465,6 +470,7 @@ int launch_linear(const void* x, long long ldx, const void* w, const void* bias,
   if (regs_preferred(M, N, K) && ldx == K && ldy == N) return launch_linear_regs(x, w, bias, y, M, N, K, stream);
   if (tiles_of(a, 32, 32) <= kFewTiles) return launch_few<4, kRows>(a, stream);
   if (short_k_many(a)) return launch_many<4, 2, 3, false>(a, stream);
+  if (tiles_of(a, 64, 64) > kSmallTiles) return launch_many<2, 2, 3, false>(a, stream);
   return launch_many<1, 1, 4, false>(a, stream);
 }
 
