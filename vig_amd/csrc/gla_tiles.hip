@@ -387,6 +387,48 @@ __device__ __forceinline__ void walk_tiles(char* lds, const TileLds<NG>& lay, in
   }
 }
 
+// The same at 32 key channels with a tile's keys fetched while the tile before is at work (whole sequences only: 64 channels have no
+// registers left for it, 768 sequences of 196 36 -> 44 us, and a segment's walk is too short, 48 of 1802 32.1 -> 32.9).  us: 3 sequences of 196
+// 8.36 -> 8.11, 240 10.94 -> 10.81, 768 25.1 -> 24.7, 720 of 150 18.8 -> 18.5.
+template <int NG, bool FWD>
+__device__ __forceinline__ void walk_tiles_ahead(char* lds, const TileLds<NG>& lay, int ti, int NT, int lane,
+                                                 u32x4_t (&qh)[NG], f32x16_t (&O)[2]) {
+  const int h = lane >> 5;
+  constexpr int HC = 8 * NG;
+  const int kbase = FWD ? lay.kf : lay.kb - TileLds<NG>::KB;  // reverse regions start at tile 1
+  const char* dbase = lds + lay.d + (FWD ? 0 : NT * 128) + 2 * HC * h;
+  const int n = FWD ? ti : NT - 1 - ti;
+  if (n == 0) return;
+  const auto load_k = [&](int j, u32x4_t (&kf)[NG]) {
+    char* kreg = lds + kbase + j * TileLds<NG>::KB;
+#pragma unroll
+    for (int g = 0; g < NG; ++g) kf[g] = *reinterpret_cast<const u32x4_t*>(unit_ptr(kreg, g, lane));
+  };
+  u32x4_t kf[NG];
+  load_k(FWD ? ti - 1 : ti + 1, kf);
+#pragma unroll 1
+  for (int s = 1; s <= n; ++s) {
+    const int j = FWD ? ti - s : ti + s;
+    char* vreg = lds + lay.v + j * TileLds<NG>::VB;
+    u32x4_t vf[2][2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int pv = 0; pv < 2; ++pv) vf[t][pv] = *reinterpret_cast<const u32x4_t*>(unit_ptr(vreg, 2 * t + pv, lane));
+    u32x4_t d[NG];
+    const char* dp = dbase + j * 128;
+#pragma unroll
+    for (int g = 0; g < NG; ++g) d[g] = *reinterpret_cast<const u32x4_t*>(dp + 16 * g);
+    const f32x16_t P = score_tile16<NG>(kf, qh);
+    load_k(FWD ? max(j - 1, 0) : min(j + 1, NT - 1), kf);
+#pragma unroll
+    for (int g = 0; g < NG; ++g)
+#pragma unroll
+      for (int m = 0; m < 4; ++m) qh[g][m] = mul_f16x2(qh[g][m], s < n ? d[g][m] : 0x3C003C00u);
+    apply_values(P, vf, O);
+  }
+}
+
 // power of two that brings a direction's states to at most 2^14, from the maxima that the scan left
 __device__ __forceinline__ int state_shift(float top) {
   const int ex = (int)((__float_as_uint(wave_max(top)) >> 23) & 0xffu) - 127;  // (inf / nan: 128, the result is not finite anyway)
@@ -746,12 +788,15 @@ __device__ __forceinline__ void tile_pass(const TileCtx& cx, const TileKernArgs*
   // ---- the other tiles, outwards ----
   int lane_w = lane;
   asm volatile("" : "+v"(lane_w));
-  walk_tiles<NG, true>(lds, lay, ti, NT, lane_w, qhf, O);
+  constexpr bool kAhead = NG == 2 && !CHAIN;
+  if constexpr (kAhead) walk_tiles_ahead<NG, true>(lds, lay, ti, NT, lane_w, qhf, O);
+  else walk_tiles<NG, true>(lds, lay, ti, NT, lane_w, qhf, O);
   // (general form: the state's term joins accumulators that carry 2^-(eq + ek + ev); q^ carries 2^-eq itself)
   if (CHAIN)
     apply_state<NG, true>(cx.state_in, shift_f, lds + lay.d + 16 * NG * (lane_w >> 5), ti > 0, lane_w,
                           GENERAL ? -(ek + ev) : 0, qhf, O);
-  if (BIDIR) walk_tiles<NG, false>(lds, lay, ti, NT, lane_w, qhb, O);
+  if constexpr (BIDIR && kAhead) walk_tiles_ahead<NG, false>(lds, lay, ti, NT, lane_w, qhb, O);
+  else if constexpr (BIDIR) walk_tiles<NG, false>(lds, lay, ti, NT, lane_w, qhb, O);
   if (CHAIN && BIDIR)
     apply_state<NG, false>(cx.state_in + kGlaStateFloats, shift_b,
                            lds + lay.d + (NT + NT - 1) * 128 + 16 * NG * (lane_w >> 5), ti < NT - 1, lane_w,
