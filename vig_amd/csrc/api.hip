@@ -13,8 +13,9 @@ int launch_dirgate_bwd(const void* in, const void* d_out, void* d_in, int B, int
 int launch_merge_heads(const void* dq, const void* dk, const void* dv, void* dqkv, int B, int L, int H, int Dk, int Dv,
                        long long ld, int io_dtype, hipStream_t stream);
 size_t dwconv3x3_wgrad_workspace(int B, int C);
+size_t dwconv3x3_wgrad_least_workspace(int B, int C);
 int launch_dwconv3x3_bwd(const void* x, const void* dy, const void* pre, const float* wt, void* dx, float* dw_db,
-                         void* workspace, int B, int h, int w, int C, int io_dtype, hipStream_t stream);
+                         void* workspace, size_t workspace_bytes, int B, int h, int w, int C, int io_dtype, hipStream_t stream);
 int launch_dirgate_lowrank_bwd(const void* low, long long ld, const void* w1, const void* w1t, const void* b1,
                                const void* d_out, void* dx, void* d_low, long long ldd, int B, int L, int H, int Dk,
                                float inv_norm, float clamp_min, int out_dtype, hipStream_t stream);
@@ -583,8 +584,8 @@ int vig_dwconv3x3_bwd(const void* x, const void* dy, const void* pre, const floa
     return VIG_EINVAL;
   if (!aligned16(x, dy, pre, dx, dw_db, workspace)) return VIG_EINVAL;
   if (!dtype_ok(io_dtype) || (C % 8) != 0) return VIG_ENOTSUP;
-  if (dw_db && (!workspace || workspace_bytes < vig::dwconv3x3_wgrad_workspace(B, C))) return VIG_ENOSPC;
-  return vig::launch_dwconv3x3_bwd(x, dy, pre, weight, dx, dw_db, workspace, B, h, w, C, io_dtype, (hipStream_t)stream);
+  if (dw_db && (!workspace || workspace_bytes < vig::dwconv3x3_wgrad_least_workspace(B, C))) return VIG_ENOSPC;
+  return vig::launch_dwconv3x3_bwd(x, dy, pre, weight, dx, dw_db, workspace, workspace_bytes, B, h, w, C, io_dtype, (hipStream_t)stream);
 }
 
 int vig_dwconv3x3_bwd_weight(const void* x, const void* dy, float* dw_db, void* workspace, size_t workspace_bytes,

@@ -704,10 +704,11 @@ int launch_locality_blend(const void* o, const void* loc, const void* glin, cons
 // [workgroups, 10 * C] (columns c*9 + tap, then 9*C + c for the bias), which a column sum finishes.
 // With `pre` (the stored convolution result in front of a SiLU) dy is the gradient behind the activation and is taken through
 // it while the tile is staged, rounded to the storage type.
-// Measured at B 128, 14 x 14, C 384 bf16: 28 us, where the mirrored forward stencil took 14 and a weight-gradient kernel that
-// fetched the nine neighbours of every row from cache 68.
+// Measured with the column sum (us, bf16; before: bands as tall as LDS allows and at most four workgroups an image and channel group, its weights
+// as 36 loads of a float): 128 images of 14 x 14, C 384 27.5, now 23.8; 256 46, now 40; 24 of 28 x 28 26, now 22.5; 8 of 64 x 64, C 192 101, now 32;
+// 2 of 61 x 61 54, now 13; 1 of 14 x 14 16, now 8.5.  (Two or four positions' rows of x under way instead of one: 24.1, 30 at 128 images.)
 // ---------------------------------------------------------------------------
-constexpr int kWgradSplit = 4;  // workgroups per image and channel group, at most
+constexpr int kWgradSplit = 4, kWgradMostSplit = 32, kWgradFill = 512;  // workgroups per image and channel group, at most
 constexpr int kBwdWaves = 4;
 
 template <typename T> struct Vec4;
@@ -741,9 +742,16 @@ __global__ __launch_bounds__(64 * kBwdWaves) void dwconv3x3_bwd_kernel(
   const bool quad_ok = ch < C;
   f32x4_t wk[9], dw[10];
 #pragma unroll
-  for (int t = 0; t < 9; ++t)
+  for (int i = 0; i < 9; ++i) {  // 36 consecutive floats
+    f32x4_t x = {0.f, 0.f, 0.f, 0.f};
+    const float* w4 = wt + (size_t)ch * 9 + 4 * i;
+    if (quad_ok && dx) {
+      if ((reinterpret_cast<uintptr_t>(wt) & 15) == 0) x = *reinterpret_cast<const f32x4_t*>(w4);
+      else x = f32x4_t{w4[0], w4[1], w4[2], w4[3]};  // (a caller's weights may start anywhere)
+    }
 #pragma unroll
-    for (int j = 0; j < 4; ++j) wk[t][j] = quad_ok && dx ? wt[(size_t)(ch + j) * 9 + t] : 0.f;
+    for (int e = 0; e < 4; ++e) wk[(4 * i + e) % 9][(4 * i + e) / 9] = x[e];
+  }
 #pragma unroll
   for (int t = 0; t < 10; ++t) dw[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   for (int band = blockIdx.y; band < nbands; band += gridDim.y) {
@@ -854,18 +862,31 @@ __global__ __launch_bounds__(64 * kBwdWaves) void dwconv3x3_bwd_kernel(
 
 int launch_column_sum(const float* partials, float* out, int n, int C, hipStream_t stream);
 
-size_t dwconv3x3_wgrad_workspace(int B, int C) { return (size_t)B * kWgradSplit * C * 10 * sizeof(float); }
+// Workgroups an image's channel group may be split over: four, or as many as bring a thousand workgroups.
+static int wgrad_split(int B, int C) {
+  const long long have = (long long)B * ((C + kStencilGroup - 1) / kStencilGroup);
+  return (int)std::min<long long>(kWgradMostSplit, std::max<long long>(kWgradSplit, (kWgradFill + have - 1) / have));
+}
+size_t dwconv3x3_wgrad_workspace(int B, int C) { return (size_t)B * wgrad_split(B, C) * C * 10 * sizeof(float); }
+// (a workspace for four is enough)
+size_t dwconv3x3_wgrad_least_workspace(int B, int C) { return (size_t)B * kWgradSplit * C * 10 * sizeof(float); }
 
 template <typename T, bool SILU>
 static int launch_dwconv3x3_bwd_t(const void* x, const void* dy, const void* pre, const float* wt, void* dx, float* dw_db,
-                                  float* partials, int B, int h, int w, int C, hipStream_t stream) {
+                                  float* partials, int most_split, int B, int h, int w, int C, hipStream_t stream) {
   constexpr int kCells = 48 * 1024 / (kStencilGroup * (int)sizeof(T));  // three workgroups' tiles fit a CU's LDS
   const int band_cols = w < kCells / 6 - 2 ? w : kCells / 6 - 2;        // four rows at least
   const int rows = kCells / (band_cols + 2) - 2;
-  const int band_rows = rows < h ? rows : h;
-  const int row_bands = (h + band_rows - 1) / band_rows, col_bands = (w + band_cols - 1) / band_cols;
-  const int nbands = row_bands * col_bands, groups = (C + kStencilGroup - 1) / kStencilGroup;
-  const int split = nbands < kWgradSplit ? nbands : kWgradSplit;
+  const int col_bands = (w + band_cols - 1) / band_cols, groups = (C + kStencilGroup - 1) / kStencilGroup;
+  int band_rows = rows < h ? rows : h;
+  // Few images: shorter bands, a workgroup each, until there are two a compute unit (us at 256 / 512 / 768 / 1024: 16 images of 14 x 14,
+  // C 384 11.5 / 11.2 / 12.4 / 12.5; 20 of 20 x 20 15.8 / 15.2 / 17.6 / 17.7; 9 of 47 x 47 30.5 / 23.3 / 23.9 / 27.5; 8 of 64 x 64, C 192
+  // 33 / 32 / 24 / 24: a workgroup's weights, lane exchanges and partial sums cost about as much as two rows of a grid)
+  const long long have = (long long)B * groups * col_bands;
+  while (band_rows > 2 && have * ((h + band_rows - 1) / band_rows) < kWgradFill && (h + band_rows - 2) / (band_rows - 1) * col_bands <= most_split)
+    --band_rows;
+  const int nbands = (h + band_rows - 1) / band_rows * col_bands;
+  const int split = nbands < most_split ? nbands : most_split;
   size_t lds = (size_t)(band_rows + 2) * (band_cols + 2) * kStencilGroup * sizeof(T);
   const size_t sums = (size_t)kBwdWaves * 16 * 10 * sizeof(f32x4_t);
   if (lds < sums) lds = sums;
@@ -877,13 +898,15 @@ static int launch_dwconv3x3_bwd_t(const void* x, const void* dy, const void* pre
 }
 
 int launch_dwconv3x3_bwd(const void* x, const void* dy, const void* pre, const float* wt, void* dx, float* dw_db,
-                         void* workspace, int B, int h, int w, int C, int io_dtype, hipStream_t stream) {
+                         void* workspace, size_t workspace_bytes, int B, int h, int w, int C, int io_dtype, hipStream_t stream) {
   if (B > 65535 || C % 8 != 0 || (long long)h * w > 0x7fffffffLL - 64 || (long long)C * 10 > 0x7fffffffLL ||
       (long long)B * ((C + 63) / 64) > 0x7fffffffLL)
     return -22;
   auto fn = io_dtype == 0 ? (pre ? launch_dwconv3x3_bwd_t<float, true> : launch_dwconv3x3_bwd_t<float, false>)
                           : (pre ? launch_dwconv3x3_bwd_t<uint16_t, true> : launch_dwconv3x3_bwd_t<uint16_t, false>);
-  return fn(x, dy, pre, wt, dx, dw_db, static_cast<float*>(workspace), B, h, w, C, stream);
+  // (without weight gradients nobody's partial sums need room)
+  const int most = dw_db ? (int)std::min<size_t>(wgrad_split(B, C), workspace_bytes / ((size_t)B * C * 10 * sizeof(float))) : wgrad_split(B, C);
+  return fn(x, dy, pre, wt, dx, dw_db, static_cast<float*>(workspace), most, B, h, w, C, stream);
 }
 
 // ---------------------------------------------------------------------------
