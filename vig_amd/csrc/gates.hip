@@ -331,11 +331,15 @@ __global__ __launch_bounds__(256) void dirgate_lowrank_mfma_kernel(const uint16_
 // is formed as in the forward, dx = d_out * inv_norm * sigmoid(-x) (zero where the forward clamped) is rounded to bf16 and
 // goes to memory (the weight gradient reads it), and the same registers are the operand of the second product
 // d_low = dx . w1: a lane's sixteen channels are two runs of eight, which is what one step's operand takes, and the transposed
-// weights (w1t [16][2*H*Dk]) are addressed to match.  A workgroup owns 32 tokens; its four waves take the channel tiles in
+// weights (w1t [16][2*H*Dk]) are addressed to match.  A workgroup owns 32 tokens; its waves take the channel tiles in
 // turn and add their d_low through LDS.  Bound by reading d_out and writing dx once: the separate layer's two products and
 // the elementwise pass moved the [B*L, 2*H*Dk] matrix five times.
+// us at 4 / 6 / 8 / 12 waves (a wave per channel tile at most): rows 784, 768 channels 12.5 / 10.7 / 9.1 / 8.4; 4704, 768 13.4 / 11.5 / 10.0 / 9.6;
+// 25088, 384 17.1 / 18.1 / 15.7 / 19.3; 11760, 768 18.7 / 18.9 / 16.0 / 17.5.
+constexpr int kGateBwdWaves = 8;
+
 template <typename TO>
-__global__ __launch_bounds__(256) void dirgate_lowrank_bwd_kernel(const uint16_t* __restrict__ low, long long ld,
+__global__ __launch_bounds__(64 * kGateBwdWaves) void dirgate_lowrank_bwd_kernel(const uint16_t* __restrict__ low, long long ld,
                                                                   const uint16_t* __restrict__ w1,
                                                                   const uint16_t* __restrict__ w1t,
                                                                   const uint16_t* __restrict__ b1,
@@ -344,8 +348,8 @@ __global__ __launch_bounds__(256) void dirgate_lowrank_bwd_kernel(const uint16_t
                                                                   long long ntok, int B, int L, int H, int Dk,
                                                                   float inv_norm, float clamp_min) {
   constexpr int R = kGateRank;
-  __shared__ f32x4_t part[4][2][64];  // [wave][rank octet][lane]
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  __shared__ f32x4_t part[kGateBwdWaves][2][64];  // [wave][rank octet][lane]
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
   const int r = lane & 31, h = lane >> 5;
   const unsigned tok = blockIdx.x * 32u + r;
   const bool tok_ok = tok < (unsigned)ntok;
@@ -359,7 +363,7 @@ __global__ __launch_bounds__(256) void dirgate_lowrank_bwd_kernel(const uint16_t
   f32x16_t dl;
 #pragma unroll
   for (int j = 0; j < 16; ++j) dl[j] = 0.f;
-  for (int tile = wave; tile < ntiles; tile += 4) {
+  for (int tile = wave; tile < ntiles; tile += waves) {
     const int c = tile * 32 + 16 * h;  // first of this lane's 16 channels
     const int cd = c / Dk, d = c - cd * Dk, dir = cd / H, hh = cd - dir * H;
     const TO* src = d_out + (size_t)dir * dir_stride + (size_t)hh * L * Dk + d + row_off;
@@ -401,13 +405,11 @@ __global__ __launch_bounds__(256) void dirgate_lowrank_bwd_kernel(const uint16_t
 #pragma unroll
   for (int g = 0; g < 2; ++g) part[wave][g][lane] = f32x4_t{dl[4 * g], dl[4 * g + 1], dl[4 * g + 2], dl[4 * g + 3]};
   __syncthreads();
-  if (wave < 2 && tok_ok) {
-    f32x4_t sum = part[0][wave][lane];
-#pragma unroll
-    for (int k = 1; k < 4; ++k)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) sum[j] += part[k][wave][lane][j];
-    *reinterpret_cast<u32x2_t*>(d_low + (size_t)tok * (size_t)ldd + 8 * wave + 4 * h) =
+  for (int g = wave; g < 2; g += waves) {  // (a single wave where there is a single tile)
+    if (!tok_ok) break;
+    f32x4_t sum = part[0][g][lane];
+    for (int k = 1; k < waves; ++k) sum += part[k][g][lane];
+    *reinterpret_cast<u32x2_t*>(d_low + (size_t)tok * (size_t)ldd + 8 * g + 4 * h) =
         u32x2_t{pack_bf16x2(sum[0], sum[1]), pack_bf16x2(sum[2], sum[3])};
   }
 }
@@ -417,7 +419,7 @@ int launch_dirgate_lowrank_bwd(const void* low, long long ld, const void* w1, co
                                float inv_norm, float clamp_min, int out_dtype, hipStream_t stream) {
   const long long ntok = (long long)B * L;
   if (Dk % 16 != 0 || ntok >= 0x7fffffffLL - 64 || 2LL * H * Dk > (1 << 20)) return -95;
-  const dim3 grid((unsigned)((ntok + 31) / 32)), block(256);
+  const dim3 grid((unsigned)((ntok + 31) / 32)), block(64 * std::min(kGateBwdWaves, 2 * H * Dk / 32));
 #define VIG_DLB_CASE(TO)                                                                                             \
   hipLaunchKernelGGL((dirgate_lowrank_bwd_kernel<TO>), grid, block, 0, stream, (const uint16_t*)low, ld,             \
                      (const uint16_t*)w1, (const uint16_t*)w1t, (const uint16_t*)b1, (const TO*)d_out, (uint16_t*)dx, \
