@@ -73,8 +73,8 @@ int launch_pad_channels_multi(const void* const* src, void* const* dst, const in
 int launch_gla_backward(const void* q, const void* k, const void* v, const void* g_fwd, const void* g_bwd,
                         const void* d_o, void* dq, void* dk, void* dv, void* dg_fwd, void* dg_bwd, void* workspace,
                         int B, int H, int L, int Dk, int Dv, float scale, float out_scale, int io_dtype,
-                        int gate_dtype, bool exact, hipStream_t stream);
-size_t gla_backward_workspace(int B, int H, int L, int Dk, int Dv, int bidir);
+                        int gate_dtype, bool exact, size_t beyond, hipStream_t stream);
+size_t gla_backward_workspace(int B, int H, int L, int Dk, int Dv, int bidir);  // (launch_gla_backward's; `beyond`: bytes behind it)
 bool linear_wgrad_supported(long long T, int N, int K);
 size_t linear_wgrad_workspace(long long T, int N, int K);
 int launch_linear_wgrad(const void* dy, long long ldy, const void* x, long long ldx, long long T, int N, int K, float* dw,
@@ -819,7 +819,8 @@ size_t vig_gla_bidir_bwd_workspace_for(int B, int H, int L, int Dk, int Dv, int 
                                        int bidirectional) {
   if (B <= 0 || H <= 0 || L <= 0 || !bwd_shape_ok(Dk, Dv) || !dtype_ok(io_dtype) || !dtype_ok(gate_dtype)) return 0;
   if (padded_shape(L, Dk, Dv, io_dtype, gate_dtype, bidirectional != 0)) return padded_bwd_workspace(B, H, L);
-  return vig::gla_backward_workspace(B, H, L, Dk, Dv, bidirectional);
+  const size_t beyond = io_dtype == VIG_F32 && gate_dtype == VIG_F32 && bidirectional ? vig::gla_backward_f32_extra(B, H, L, Dk, Dv) : 0;
+  return vig::gla_backward_workspace(B, H, L, Dk, Dv, bidirectional) + beyond;
 }
 
 static int gla_bidir_bwd(const void* q, const void* k, const void* v, const void* g_fwd, const void* g_bwd,
@@ -850,7 +851,7 @@ static int gla_bidir_bwd(const void* q, const void* k, const void* v, const void
     }
     const int e = vig::launch_gla_backward(qp, kp, vp, gfp, gbp, dop, dqp, dkp, dvp, dgfp, dgbp,
                                            (char*)workspace + padded_bwd_tensors(B, H, L), B, H, L, 32, 64, scale,
-                                           out_scale, io_dtype, gate_dtype, false, st);
+                                           out_scale, io_dtype, gate_dtype, false, 0, st);
     if (e) return e;
     const void* srcs[5] = {dqp, dkp, dgfp, dgbp, dvp};
     void* dsts[5] = {dq, dk, dg_fwd, dg_bwd, dv};
@@ -860,7 +861,7 @@ static int gla_bidir_bwd(const void* q, const void* k, const void* v, const void
   const size_t need = vig::gla_backward_workspace(B, H, L, Dk, Dv, g_bwd != nullptr);
   if (!workspace || workspace_bytes < need) return VIG_ENOSPC;
   return vig::launch_gla_backward(q, k, v, g_fwd, g_bwd, d_o, dq, dk, dv, dg_fwd, dg_bwd, workspace, B, H, L, Dk, Dv,
-                                  scale, out_scale, io_dtype, gate_dtype, exact, (hipStream_t)stream);
+                                  scale, out_scale, io_dtype, gate_dtype, exact, workspace_bytes - need, (hipStream_t)stream);
 }
 
 int vig_gla_bidir_bwd(const void* q, const void* k, const void* v, const void* g_fwd, const void* g_bwd,

@@ -313,7 +313,7 @@ size_t gla_backward_workspace(int B, int H, int L, int Dk, int Dv, int bidir) {
 int launch_gla_backward(const void* q, const void* k, const void* v, const void* g_fwd, const void* g_bwd,
                         const void* d_o, void* dq, void* dk, void* dv, void* dg_fwd, void* dg_bwd, void* workspace,
                         int B, int H, int L, int Dk, int Dv, float scale, float out_scale, int io_dtype,
-                        int gate_dtype, bool exact, hipStream_t stream) {
+                        int gate_dtype, bool exact, size_t beyond, hipStream_t stream) {
   GlaBwdArgs a{q, k, v, g_fwd, g_bwd, d_o, dq, dk, dv, dg_fwd, dg_bwd, workspace, B, H, L, Dk, Dv,
                scale, out_scale, io_dtype, gate_dtype, stream, nullptr, false};
   if (!exact && gla_backward_mfma_supported(B, H, L, Dk, Dv, io_dtype, gate_dtype, g_bwd != nullptr)) {
@@ -332,7 +332,8 @@ int launch_gla_backward(const void* q, const void* k, const void* v, const void*
     const size_t behind = gla_backward_mfma_workspace(B, H, L, Dk, Dv);
     int* flags = reinterpret_cast<int*>((char*)workspace + scratch);
     const int rc = launch_gla_backward_f32(q, k, v, g_fwd, g_bwd, d_o, dq, dk, dv, dg_fwd, dg_bwd, flags, workspace, scratch,
-                                           (char*)workspace + flags_end(B, H, L, Dk, Dv, g_bwd != nullptr), behind, B, H, L, Dk,
+                                           (char*)workspace + flags_end(B, H, L, Dk, Dv, g_bwd != nullptr), behind,
+                                           (char*)workspace + flags_end(B, H, L, Dk, Dv, g_bwd != nullptr) + behind, behind ? beyond : 0, B, H, L, Dk,
                                            scale * out_scale, stream);
     if (rc != 0) return rc;
     a.only_flagged = flags;

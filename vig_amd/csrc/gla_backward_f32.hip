@@ -17,6 +17,7 @@
 // cutting of the score tiles; measured figures at launch_gla_backward_f32.  The token-recurrent kernel (gla_backward.hip)
 // serves the sequences that leave the tile form's range: they are flagged.
 #include "f32_tiles.h"
+#include <algorithm>
 #include <type_traits>
 
 namespace vig {
@@ -30,6 +31,10 @@ struct BwdF32Geo {
   int L, NT, nseg;
   float s;              // scale * out_scale
   const float *states, *grad_states;  // scanned slots of the forward states and of the gradient states; null: whole sequences
+  // An item is a sequence's segment, numbered (segment, sequence); from `whole` on an item's directions go to two workgroups, the
+  // reverse one leaving its dq, dk, dv in `half`: per item 32 NT rows of dq, then of dk, then of dv.
+  int nseq, whole;
+  float* half;
 };
 
 // byte offsets: per tile the operand over key channels (k^ or q^) and the one over value channels (v or d'), decays,
@@ -396,25 +401,25 @@ __device__ __forceinline__ void carry_sums(const float* S, const float* dS, floa
     }
 }
 
-}  // namespace
-
-template <int NG, bool BIDIR>
-__global__ __launch_bounds__(512, 2) void gla_backward_f32_kernel(
-    const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v, const float* __restrict__ gf,
-    const float* __restrict__ gb, const float* __restrict__ d_o, float* dq, float* dk, float* dv_out, float* dgf, float* dgb,
-    int* flags_out, BwdF32Geo geo) {
-  extern __shared__ __align__(16) char lds[];
+// DIRS: the directions this workgroup does, 1 forward, 2 reverse (of a bidirectional call it checks the ranges of both)
+template <int NG, bool BIDIR, int DIRS>
+__device__ __forceinline__ void backward_item(const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
+                                              const float* __restrict__ gf, const float* __restrict__ gb, const float* __restrict__ d_o,
+                                              float* dq, float* dk, float* dv_out, float* dgf, float* dgb, int* flags_out,
+                                              const BwdF32Geo geo, int seq, int seg, float* half, char* lds) {
   constexpr int DK = 16 * NG, NP = NG / 2;
   const int NT = geo.NT, lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
   const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int ti = w < 4 ? NT - 1 - w : w - 4;  // (the two waves of a SIMD meet NT + 1 tiles together, see gla_f32.hip)
   const BwdF32Lds<NG> lay(NT);
-  const int tok = 32 * ((int)blockIdx.y * NT + ti);
+  constexpr bool fwd_on = (DIRS & 1) != 0, rev_on = (DIRS & 2) != 0;
+  const int tok = 32 * (seg * NT + ti);
   const int nvalid = __builtin_amdgcn_readfirstlane(max(0, min(32, geo.L - tok)));
-  const size_t off = (size_t)blockIdx.x * geo.L + tok;
+  const size_t off = (size_t)seq * geo.L + tok;
   const rsrc_t rq = chunk_rsrc(q + off * DK, nvalid, 4 * DK), rk = chunk_rsrc(k + off * DK, nvalid, 4 * DK);
   const rsrc_t rv = chunk_rsrc(v + off * 64, nvalid, 256), rdo = chunk_rsrc(d_o + off * 64, nvalid, 256);
-  const rsrc_t rdq = chunk_rsrc(dq + off * DK, nvalid, 4 * DK), rdk = chunk_rsrc(dk + off * DK, nvalid, 4 * DK);
+  const rsrc_t rdq = chunk_rsrc(fwd_on ? dq + off * DK : half + 32 * ti * DK, nvalid, 4 * DK);
+  const rsrc_t rdk = chunk_rsrc(fwd_on ? dk + off * DK : half + 32 * (NT + ti) * DK, nvalid, 4 * DK);
   char* ktile = lds + ti * BwdF32Lds<NG>::KB;
   char* vtile = lds + lay.v + ti * BwdF32Lds<NG>::VB;
   float* sc = reinterpret_cast<float*>(lds + lay.sc) + 64 * ti;
@@ -422,7 +427,7 @@ __global__ __launch_bounds__(512, 2) void gla_backward_f32_kernel(
   float* tot = reinterpret_cast<float*>(lds + lay.tot);
   float* carry = reinterpret_cast<float*>(lds + lay.carry);
   int* flags = reinterpret_cast<int*>(lds + lay.flag);
-  const size_t item = (size_t)blockIdx.x * geo.nseg + blockIdx.y;
+  const size_t item = (size_t)seq * geo.nseg + seg;
   const float* st = geo.states ? geo.states + item * 2 * kGlaStateFloats : nullptr;
   const float* dst = geo.states ? geo.grad_states + item * 2 * kGlaStateFloats : nullptr;
 
@@ -453,18 +458,19 @@ __global__ __launch_bounds__(512, 2) void gla_backward_f32_kernel(
   const rsrc_t rgf = chunk_rsrc(gf + off * DK, nvalid, 4 * DK), rgb = chunk_rsrc(BIDIR ? gb + off * DK : gf, BIDIR ? nvalid : 0, 4 * DK);
 
   // ---- ranges; carries of the gate gradients into the segment ----
-  if (BIDIR) load_rows_f32<NG>(rgb, r, h, rest);
-  load_rows_f32<NG>(rgf, r, h, x);
+  // (the direction that comes first last: its factors stay)
+  if (BIDIR) load_rows_f32<NG>(fwd_on ? rgb : rgf, r, h, rest);
+  load_rows_f32<NG>(fwd_on ? rgf : rgb, r, h, x);
   load_rows_f32<NG>(rq, r, h, xq);
   load_rows_f32<NG>(rk, r, h, xk);
   load_rows_f32<4>(rv, r, h, nv);
   load_rows_f32<4>(rdo, r, h, no);
   float mag = 0.f;
   bool wide = false;
-  if (BIDIR) wide = gate_factors<NG, false>(sc, dtab, lane, rest);
+  if (BIDIR) wide = fwd_on ? gate_factors<NG, false>(sc, dtab, lane, rest) : gate_factors<NG, true>(sc, dtab, lane, rest);
 #pragma unroll
   for (int c = 0; c < NG; ++c) rest[c] = x[c];
-  wide |= gate_factors<NG, true>(sc, dtab, lane, rest);
+  wide |= fwd_on ? gate_factors<NG, true>(sc, dtab, lane, rest) : gate_factors<NG, false>(sc, dtab, lane, rest);
 #pragma unroll
   for (int c = 0; c < NG; ++c) mag += sum_abs(xq[c]) + sum_abs(xk[c]);
 #pragma unroll
@@ -473,62 +479,32 @@ __global__ __launch_bounds__(512, 2) void gla_backward_f32_kernel(
   if (lane == 0) flags[ti] = wide;
   for (int d = w; d < 2; d += NT) {
     // forward: what lies to the right (the next segment's incoming state against the gradient state from there)
-    const bool inner = st && (d == 0 ? (int)blockIdx.y + 1 < geo.nseg : blockIdx.y > 0) && (d == 0 || BIDIR);
+    const bool inner = st && (d == 0 ? seg + 1 < geo.nseg : seg > 0) && (d == 0 || BIDIR);
     if (inner)
       carry_sums<NG>(d == 0 ? st + 2 * kGlaStateFloats : st - kGlaStateFloats, d == 0 ? dst + kGlaStateFloats : dst, geo.s,
                      carry + 64 * d, lane);
     else
       carry[64 * d + lane] = 0.f;
   }
-  // ---- forward direction, queries ----
-  decayed_keys();
-  stage_key_columns<NG>(ktile, lane, x);
-  stage_values(vtile, lane, nv, 1.0f);
-  set_own(geo.s);
+  if (fwd_on) {  // ---- forward direction, queries ----
+    decayed_keys();
+    stage_key_columns<NG>(ktile, lane, x);
+    stage_values(vtile, lane, nv, 1.0f);
+    set_own(geo.s);
+  } else {  // ---- reverse direction, keys (as below, behind the forward one) ----
+    decayed_queries();
+    stage_key_columns<NG>(ktile, lane, x);
+    stage_values(vtile, lane, no, geo.s);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) own[c] = split8(nv[c]);
+  }
   lds_barrier();
   const bool refused = __builtin_amdgcn_ballot_w64(lane < NT && flags[lane < NT ? lane : 0] != 0) != 0;
-  if (threadIdx.x == 0 && (refused || geo.nseg == 1)) flags_out[blockIdx.x] = refused;
+  if (threadIdx.x == 0 && (refused || geo.nseg == 1)) flags_out[seq] = refused;  // (both halves of an item: the same)
   if (refused) return;
 
-  f32x16_t acc[NP];
-  query_loop<NG, true>(lay, lds, ti, NT, lane, own, st, acc);
-  load_columns(rdo, r, h, nv);
-  refetch(true, true);
-  {
-    f32x8_t g[NG];
-    unpack_acc<NG>(acc, g);
-#pragma unroll
-    for (int c = 0; c < NG; ++c) g[c] *= exp2_octet(-rest[c]);
-    store_rows<NG>(rdq, r, h, g);  // parked (the same lanes add the reverse direction's)
-#pragma unroll
-    for (int c = 0; c < NG; ++c) g[c] *= xq[c];
-    store_rows<NG>(chunk_rsrc(dgf + off * DK, nvalid, 4 * DK), r, h, g);
-  }
-  // ---- forward direction, keys ----
-  f32x16_t dv[2] = {f32x16_t{0.f}, f32x16_t{0.f}};
-  lds_barrier();
-  decayed_queries();
-  stage_key_rows<NG>(ktile, lane, x);
-  stage_values(vtile, lane, nv, geo.s);
-  decayed_keys();
-  lds_barrier();
-  value_loop<NG, true>(lay, lds, ti, NT, lane, x, dst ? dst + kGlaStateFloats : nullptr, geo.s, dv);
-  load_rows_f32<4>(rdo, r, h, nv);
-  load_rows_f32<4>(rv, r, h, no);
-  refetch(true, false);
-  lds_barrier();
-  decayed_queries();
-  stage_key_columns<NG>(ktile, lane, x);
-  stage_values(vtile, lane, nv, geo.s);
-  set_own(1.0f);
-  lds_barrier();
-  const rsrc_t rdgf = chunk_rsrc(dgf + off * DK, nvalid, 4 * DK);
+  f32x16_t acc[NP], dv[2] = {f32x16_t{0.f}, f32x16_t{0.f}};
   f32x8_t z[NG];
-  key_loop<NG, true>(lay, lds, ti, NT, lane, own, dst ? dst + kGlaStateFloats : nullptr, geo.s, acc);
-  load_rows_f32<NG>(rdgf, r, h, z);
-  if (BIDIR) load_rows_f32<NG>(rgb, r, h, x);
-  refetch(BIDIR, true);
-
   // a direction's gate gradient: q dq - k dk summed over the tokens behind (forward) or before (reverse)
   const auto gate_gradient = [&](auto fwd, const f32x8_t (&g)[NG], rsrc_t rdg, const float* dc) {
     constexpr bool FWD = decltype(fwd)::value;
@@ -555,30 +531,71 @@ __global__ __launch_bounds__(512, 2) void gla_backward_f32_kernel(
     for (int c = 0; c < NG; ++c) z[c] += lds_f32x8(sc + 8 * NG * h + 8 * c);
     store_rows<NG>(rdg, r, h, z);
   };
-  {
-    f32x8_t g[NG];
-    unpack_acc<NG>(acc, g);
+  if (fwd_on) {
+    query_loop<NG, true>(lay, lds, ti, NT, lane, own, st, acc);
+    load_columns(rdo, r, h, nv);
+    refetch(true, true);
+    {
+      f32x8_t g[NG];
+      unpack_acc<NG>(acc, g);
 #pragma unroll
-    for (int c = 0; c < NG; ++c) {
-      g[c] *= exp2_octet(rest[c]);
-      z[c] -= xk[c] * g[c];
+      for (int c = 0; c < NG; ++c) g[c] *= exp2_octet(-rest[c]);
+      store_rows<NG>(rdq, r, h, g);  // parked (the same lanes add the reverse direction's)
+#pragma unroll
+      for (int c = 0; c < NG; ++c) g[c] *= xq[c];
+      store_rows<NG>(chunk_rsrc(dgf + off * DK, nvalid, 4 * DK), r, h, g);
     }
-    store_rows<NG>(rdk, r, h, g);
-    gate_gradient(std::true_type{}, z, rdgf, carry);
-  }
-  if (BIDIR) {
-    const rsrc_t rdgb = chunk_rsrc(dgb + off * DK, nvalid, 4 * DK);
-    lds_barrier();  // (the totals have been read)
-    // ---- reverse direction, keys (d' rows stay) ----
-#pragma unroll
-    for (int c = 0; c < NG; ++c) rest[c] = x[c];
-    gate_factors<NG, false>(sc, dtab, lane, rest);
+    // ---- forward direction, keys ----
+    lds_barrier();
+    decayed_queries();
+    stage_key_rows<NG>(ktile, lane, x);
+    stage_values(vtile, lane, nv, geo.s);
+    decayed_keys();
+    lds_barrier();
+    value_loop<NG, true>(lay, lds, ti, NT, lane, x, dst ? dst + kGlaStateFloats : nullptr, geo.s, dv);
+    load_rows_f32<4>(rdo, r, h, nv);
+    load_rows_f32<4>(rv, r, h, no);
+    refetch(true, false);
+    lds_barrier();
     decayed_queries();
     stage_key_columns<NG>(ktile, lane, x);
+    stage_values(vtile, lane, nv, geo.s);
+    set_own(1.0f);
     lds_barrier();
+    const rsrc_t rdgf = chunk_rsrc(dgf + off * DK, nvalid, 4 * DK);
+    key_loop<NG, true>(lay, lds, ti, NT, lane, own, dst ? dst + kGlaStateFloats : nullptr, geo.s, acc);
+    load_rows_f32<NG>(rdgf, r, h, z);
+    if (rev_on) load_rows_f32<NG>(rgb, r, h, x);
+    refetch(BIDIR, true);
+    {
+      f32x8_t g[NG];
+      unpack_acc<NG>(acc, g);
+#pragma unroll
+      for (int c = 0; c < NG; ++c) {
+        g[c] *= exp2_octet(rest[c]);
+        z[c] -= xk[c] * g[c];
+      }
+      store_rows<NG>(rdk, r, h, g);
+      gate_gradient(std::true_type{}, z, rdgf, carry);
+    }
+  }
+  if (rev_on) {
+    const rsrc_t rdgb = chunk_rsrc(dgb + off * DK, nvalid, 4 * DK);
+    if (fwd_on) {
+      lds_barrier();  // (the totals have been read)
+      // ---- reverse direction, keys (d' rows stay) ----
+#pragma unroll
+      for (int c = 0; c < NG; ++c) rest[c] = x[c];
+      gate_factors<NG, false>(sc, dtab, lane, rest);
+      decayed_queries();
+      stage_key_columns<NG>(ktile, lane, x);
+      lds_barrier();
+    }
     key_loop<NG, false>(lay, lds, ti, NT, lane, own, dst, geo.s, acc);
     load_columns(rdo, r, h, nv);
-    load_rows_f32<NG>(rdk, r, h, z);
+#pragma unroll
+    for (int c = 0; c < NG; ++c) z[c] = f32x8_t{0.f};
+    if (fwd_on) load_rows_f32<NG>(rdk, r, h, z);
     refetch(true, true);
     {
       f32x8_t kdk[NG];
@@ -604,7 +621,7 @@ __global__ __launch_bounds__(512, 2) void gla_backward_f32_kernel(
     refetch(false, true);
   }
   {
-    const rsrc_t rdv = chunk_rsrc(dv_out + off * 64, nvalid, 256);
+    const rsrc_t rdv = chunk_rsrc(fwd_on ? dv_out + off * 64 : half + (size_t)64 * NT * DK + 32 * ti * 64, nvalid, 256);
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       u32x4_t o;
@@ -613,7 +630,7 @@ __global__ __launch_bounds__(512, 2) void gla_backward_f32_kernel(
       __builtin_amdgcn_raw_buffer_store_b128(o, rdv, (unsigned)r * 256u + 128u * h + 16u * i, 0, 0);
     }
   }
-  if (BIDIR) {
+  if (rev_on) {
     const rsrc_t rdgb = chunk_rsrc(dgb + off * DK, nvalid, 4 * DK);
     lds_barrier();
     // ---- reverse direction, queries ----
@@ -624,7 +641,9 @@ __global__ __launch_bounds__(512, 2) void gla_backward_f32_kernel(
     lds_barrier();
     f32x8_t zq[NG];
     query_loop<NG, false>(lay, lds, ti, NT, lane, own, st ? st + kGlaStateFloats : nullptr, acc);
-    load_rows_f32<NG>(rdq, r, h, zq);
+#pragma unroll
+    for (int c = 0; c < NG; ++c) zq[c] = f32x8_t{0.f};
+    if (fwd_on) load_rows_f32<NG>(rdq, r, h, zq);
     load_rows_f32<NG>(rdgb, r, h, z);
     refetch(true, false);
     f32x8_t g[NG];
@@ -640,7 +659,44 @@ __global__ __launch_bounds__(512, 2) void gla_backward_f32_kernel(
   }
 }
 
-// Measured at B 64, H 6, L 196, Dk 32 (384 workgroups, one to a CU): 163 us, token-recurrent kernel 485 us.  Half of a wave's
+}  // namespace
+
+template <int NG, bool BIDIR, bool HALVES>
+__global__ __launch_bounds__(512, 2) void gla_backward_f32_kernel(
+    const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v, const float* __restrict__ gf,
+    const float* __restrict__ gb, const float* __restrict__ d_o, float* dq, float* dk, float* dv, float* dgf, float* dgb,
+    int* flags, BwdF32Geo geo) {
+  extern __shared__ __align__(16) char lds[];
+  if constexpr (!HALVES) {  // (a kernel of its own: the three bodies in one cost the whole items 2 % at 64 channels)
+    backward_item<NG, BIDIR, BIDIR ? 3 : 1>(q, k, v, gf, gb, d_o, dq, dk, dv, dgf, dgb, flags, geo, blockIdx.x, blockIdx.y, nullptr, lds);
+  } else {
+    const int which = (int)blockIdx.x - geo.whole, work = which < 0 ? blockIdx.x : geo.whole + (which >> 1);
+    const int seg = work / geo.nseq, seq = work - seg * geo.nseq;
+    float* half = geo.half + (size_t)max(which >> 1, 0) * (32 * geo.NT) * (32 * NG + 64);
+    if (which < 0) backward_item<NG, true, 3>(q, k, v, gf, gb, d_o, dq, dk, dv, dgf, dgb, flags, geo, seq, seg, half, lds);
+    else if ((which & 1) == 0) backward_item<NG, true, 1>(q, k, v, gf, gb, d_o, dq, dk, dv, dgf, dgb, flags, geo, seq, seg, half, lds);
+    else backward_item<NG, true, 2>(q, k, v, gf, gb, d_o, dq, dk, dv, dgf, dgb, flags, geo, seq, seg, half, lds);
+  }
+}
+
+// What the reverse workgroups of items in two halves left is added to the forward ones' (a workgroup: a quarter of an item).
+template <int DK>
+__global__ __launch_bounds__(256) void gla_backward_f32_add_kernel(float* __restrict__ dq, float* __restrict__ dk, float* __restrict__ dv,
+                                                                   BwdF32Geo geo) {
+  const int work = geo.whole + blockIdx.x, seg = work / geo.nseq, seq = work - seg * geo.nseq, rows = 32 * geo.NT;
+  const int first = seg * rows, valid = min(rows, geo.L - first);
+  const float* half = geo.half + (size_t)blockIdx.x * rows * (2 * DK + 64);
+  const size_t at = (size_t)seq * geo.L + first;
+  const auto add = [&](float* to, const float* from, int width) {
+    for (int i = (blockIdx.y * 256 + threadIdx.x) * 4; i < valid * width; i += 4096)
+      *reinterpret_cast<f32x4_t*>(to + i) += *reinterpret_cast<const f32x4_t*>(from + i);
+  };
+  add(dq + at * DK, half, DK);
+  add(dk + at * DK, half + rows * DK, DK);
+  add(dv + at * 64, half + 2 * rows * DK, 64);
+}
+
+// Measured at B 64, H 6, L 196, Dk 32 (384 sequences, one to a CU; the last 128 in two halves): 133 us, whole 150, token-recurrent kernel 485 us.  Half of a wave's
 // time is waiting: at the fifteen barriers, and for rows read with a lane per row (67 clocks of the CU's load path per
 // 16-byte load instruction).
 constexpr int kBwdF32MaxLds = 160 * 1024;
@@ -655,17 +711,33 @@ bool gla_backward_f32_supported(int B, int H, int L, int Dk, int Dv, int io_dtyp
   return io_dtype == 0 && gate_dtype == 0 && (Dk == 64 || Dk == 32) && Dv == 64 && gla_f32_segments(L) <= 65535 &&
          (gla_f32_segments(L) == 1 || (long long)B * H * 4 <= 65535) && (bidir || L <= 224 || L > 256);
 }
+// Items whose directions go to two workgroups: what is left over of full rounds of the chip, where that fills no more than half of
+// one.  A half takes 55 to 60 % of the whole (it loads and checks the same), and adding up takes 3 us.  us, whole / halves: Dk 32: 18
+// sequences of 64 32 / 22.5, of 185 63.5 / 43.0, 120 of 196 74 / 55, 384 (256 and 128) 150 / 133; Dk 64: 18 of 64 56 / 34.5, 60 of 196 136
+// / 88, 384 292 / 251.
+template <int NG>
+static int f32_halves(int n, int NT) {
+  const int slots = 256 * std::max(1, std::min(kBwdF32MaxLds / BwdF32Lds<NG>(NT).total, 8 / NT)), rest = n % slots;
+  return 2 * rest <= slots ? rest : 0;
+}
+template <int NG>
+static size_t half_floats(int NT) { return (size_t)32 * NT * (32 * NG + 64); }
+
+// what the halves of a long sequence's items want beside the states (those of whole sequences lie in the recurrent kernel's scratch)
+size_t gla_backward_f32_extra(int B, int H, int L, int Dk, int Dv) {
+  if ((Dk != 64 && Dk != 32) || Dv != 64 || L <= 256 || (long long)B * H * 4 > 65535) return 0;
+  const int NT = gla_f32_fine_tiles((long long)B * H, L), n = B * H * (((L + 31) / 32 + NT - 1) / NT);
+  return Dk == 64 ? f32_halves<4>(n, NT) * half_floats<4>(NT) * sizeof(float) : f32_halves<2>(n, NT) * half_floats<2>(NT) * sizeof(float);
+}
+
 template <int NG, bool BIDIR>
 static int launch_bwd_f32_t(const float* q, const float* k, const float* v, const float* gf, const float* gb, const float* d_o,
                             float* dq, float* dk, float* dv, float* dgf, float* dgb, int* flags, void* room0, size_t bytes0,
-                            void* room1, size_t bytes1, int B, int H, int L, float s, int dev, hipStream_t stream) {
-  static bool attr_done[64] = {};
-  if (!attr_done[dev]) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(gla_backward_f32_kernel<NG, BIDIR>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, kBwdF32MaxLds) != hipSuccess)
-      return -5;
-    attr_done[dev] = true;
-  }
+                            void* room1, size_t bytes1, void* room2, size_t bytes2, int B, int H, int L, float s, hipStream_t stream) {
+  static bool done[64] = {}, done_halves[64] = {};
+  if (!allow_lds(reinterpret_cast<const void*>(gla_backward_f32_kernel<NG, BIDIR, false>), kBwdF32MaxLds, done)) return -5;
+  if constexpr (BIDIR)
+    if (!allow_lds(reinterpret_cast<const void*>(gla_backward_f32_kernel<NG, true, true>), kBwdF32MaxLds, done_halves)) return -5;
   BwdF32Geo geo{};
   geo.L = L;
   const int tiles = (L + 31) / 32;
@@ -693,20 +765,38 @@ static int launch_bwd_f32_t(const float* q, const float* k, const float* v, cons
     rc = launch_gla_segment_scan(states, grads, B * H, geo.nseg, 2, NG, stream);
     if (rc) return rc;
   }
-  hipLaunchKernelGGL((gla_backward_f32_kernel<NG, BIDIR>), dim3(B * H, geo.nseg), dim3(64 * geo.NT), lay.total, stream, q, k, v,
-                     gf, gb, d_o, dq, dk, dv, dgf, dgb, flags, geo);
+  const int n = B * H * geo.nseg;
+  geo.nseq = B * H, geo.whole = n;
+  if (BIDIR) {
+    const int rest = f32_halves<NG>(n, geo.NT);
+    const size_t need = (size_t)rest * half_floats<NG>(geo.NT) * sizeof(float);
+    const size_t used = geo.nseg == 1 ? 0 : (size_t)n * 2 * kGlaStateFloats * sizeof(float);  // of a room, by a set of states
+    const size_t used0 = states == room0 && geo.nseg > 1 ? (grads == room1 ? used : 2 * used) : 0;
+    const size_t used1 = geo.nseg > 1 ? (states == room1 ? 2 * used : grads == room1 ? used : 0) : 0;
+    if (rest > 0) {
+      if (used0 + need <= bytes0) geo.half = (float*)((char*)room0 + used0), geo.whole = n - rest;
+      else if (used1 + need <= bytes1) geo.half = (float*)((char*)room1 + used1), geo.whole = n - rest;
+      else if (need <= bytes2) geo.half = (float*)room2, geo.whole = n - rest;
+    }
+  }
+  auto kernel = gla_backward_f32_kernel<NG, BIDIR, false>;
+  dim3 grid(B * H, geo.nseg);
+  if constexpr (BIDIR)
+    if (geo.whole < n) kernel = gla_backward_f32_kernel<NG, true, true>, grid = dim3(2 * n - geo.whole);
+  hipLaunchKernelGGL(kernel, grid, dim3(64 * geo.NT), lay.total, stream, q, k, v, gf, gb, d_o, dq, dk, dv, dgf, dgb, flags,
+                     geo);
+  if (geo.whole < n) hipLaunchKernelGGL((gla_backward_f32_add_kernel<16 * NG>), dim3(n - geo.whole, 4), dim3(256), 0, stream, dq, dk, dv, geo);
   return hipGetLastError() == hipSuccess ? 0 : -5;
 }
 
 int launch_gla_backward_f32(const void* q, const void* k, const void* v, const void* gf, const void* gb, const void* d_o,
                             void* dq, void* dk, void* dv, void* dgf, void* dgb, int* flags, void* room0, size_t bytes0,
-                            void* room1, size_t bytes1, int B, int H, int L, int Dk, float s, hipStream_t stream) {
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return -5;
+                            void* room1, size_t bytes1, void* room2, size_t bytes2, int B, int H, int L, int Dk, float s,
+                            hipStream_t stream) {
 #define VIG_BWD_F32(NG, BI)                                                                                                   \
   launch_bwd_f32_t<NG, BI>((const float*)q, (const float*)k, (const float*)v, (const float*)gf, (const float*)gb,             \
-                           (const float*)d_o, (float*)dq, (float*)dk, (float*)dv, (float*)dgf, (float*)dgb, flags, room0, bytes0, room1, bytes1, B, \
-                           H, L, s, dev, stream)
+                           (const float*)d_o, (float*)dq, (float*)dk, (float*)dv, (float*)dgf, (float*)dgb, flags, room0, bytes0, room1, bytes1, \
+                           room2, bytes2, B, H, L, s, stream)
   if (Dk == 64) return gb ? VIG_BWD_F32(4, true) : VIG_BWD_F32(4, false);
   return gb ? VIG_BWD_F32(2, true) : VIG_BWD_F32(2, false);
 #undef VIG_BWD_F32

@@ -85,11 +85,12 @@ int launch_gla_f32(const GlaArgs& a);
 int launch_gla_f32_states(int NG, const float* k, const float* v, const float* q, const float* d_o, const float* gf,
                           const float* gb, float* slots, float* grad_slots, int* flags, int nseq, int L, int NT, int nseg, hipStream_t stream);
 // fp32 backward on the matrix cores; one flag per sequence marks what it left to the recurrent kernel; the two sets of states go
-// to two pieces of memory, either of which may be empty
+// to two pieces of memory, either of which may be empty; a third one takes what else there may be room for
+size_t gla_backward_f32_extra(int B, int H, int L, int Dk, int Dv);  // memory beyond gla_backward_workspace that speeds it up
 bool gla_backward_f32_supported(int B, int H, int L, int Dk, int Dv, int io_dtype, int gate_dtype, bool bidir);
 int launch_gla_backward_f32(const void* q, const void* k, const void* v, const void* gf, const void* gb, const void* d_o,
                             void* dq, void* dk, void* dv, void* dgf, void* dgb, int* flags, void* room0, size_t bytes0,
-                            void* room1, size_t bytes1, int B, int H, int L, int Dk, float s, hipStream_t stream);
+                            void* room1, size_t bytes1, void* room2, size_t bytes2, int B, int H, int L, int Dk, float s, hipStream_t stream);
 // bf16: contributions and decays of every segment of seg_len tokens, and with q and d_o the gradient states (gla_states.hip)
 int launch_gla_states(const GlaArgs& a, int seg_len, int nseg, float* slots, const void* q, const void* d_o, float* grad_slots);
 // chains the slots of a state pass in place (gla_segment_scan_kernel, no state in or out), and those of another if there is one
