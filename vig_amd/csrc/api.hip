@@ -148,7 +148,7 @@ static size_t padded_workspace(int B, int H, int L) {
 static size_t fwd_workspace_exact(int B, int H, int L, int Dk, int Dv, int io_dtype, int gate_dtype, bool bidir) {
   if (io_dtype == VIG_BF16 && gate_dtype == VIG_BF16 && (Dk == 64 || Dk == 32) && Dv == 64)
     return vig::gla_mfma_workspace(B, H, L, Dk, Dv);
-  if (io_dtype == VIG_F32 && gate_dtype == VIG_F32) return vig::gla_f32_workspace(B, H, L, Dk, Dv);
+  if (io_dtype == VIG_F32 && gate_dtype == VIG_F32) return vig::gla_f32_workspace(B, H, L, Dk, Dv, bidir);
   if (padded_shape(L, Dk, Dv, io_dtype, gate_dtype, bidir)) return padded_workspace(B, H, L);
   return bidir ? vig::gla_recurrent_workspace(B, H, L, Dv, io_dtype) : 0;
 }
@@ -171,7 +171,7 @@ size_t vig_gla_bidir_fwd_workspace(int B, int H, int L, int Dk, int Dv, int io_d
     const size_t m = vig::gla_mfma_workspace(B, H, L, Dk, Dv);
     if (m > need) need = m;
   } else {
-    const size_t m = vig::gla_f32_workspace(B, H, L, Dk, Dv);
+    const size_t m = vig::gla_f32_workspace(B, H, L, Dk, Dv, true);
     if (m > need) need = m;
   }
   return need;

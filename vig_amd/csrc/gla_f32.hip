@@ -19,6 +19,8 @@
 // operands for any gates (prepare32_any); inputs beyond the bound, gates that grow and gates that are no numbers take the
 // serial form (serial_segment).  All sequences strongly gated: B 32, H 6, L 197, D 64 81 us (mildly gated 37; the
 // token-recurrent kernel 182, the serial form, one wave of a workgroup, 1069); 768 sequences 233 us (112 / 221 / 3214).
+#include <algorithm>
+
 #include "f32_tiles.h"
 
 namespace vig {
@@ -31,6 +33,10 @@ constexpr float kMagnitude32 = 1e12f;
 struct F32Geo {
   int L, NT, nseg;      // tokens per sequence, tiles per segment, segments per sequence
   const float* states;  // long sequences: scanned slots; null: whole sequences
+  // from sequence `whole` on a (whole) sequence's directions go to two workgroups, the reverse one leaving its outputs in `half`: 32 NT
+  // rows a sequence
+  int whole;
+  float* half;
 };
 
 template <int NG>
@@ -265,7 +271,7 @@ __device__ __forceinline__ void serial_direction(const float* q, const float* k,
   }
 }
 
-template <int NG, bool BIDIR>
+template <int NG, int DIRS>  // 1 forward, 2 reverse
 __device__ __noinline__ void serial_segment(const float* q, const float* k, const float* v, const float* gf, const float* gb,
                                             float* o, const float* slots, int n, int stage_at, float oscale) {
   extern __shared__ __align__(16) char lds[];
@@ -274,9 +280,9 @@ __device__ __noinline__ void serial_segment(const float* q, const float* k, cons
   const int lane = threadIdx.x & 63;
   lds_barrier();  // everyone is done with the tiles
   if (threadIdx.x >= 64) return;
-  serial_direction<NG, true>(q, k, v, gf, n, slots, stage, obuf, false, lane);
-  if (BIDIR)
-    serial_direction<NG, false>(q, k, v, gb, n, slots ? slots + kGlaStateFloats : nullptr, stage, obuf, true, lane);
+  if (DIRS & 1) serial_direction<NG, true>(q, k, v, gf, n, slots, stage, obuf, false, lane);
+  if (DIRS & 2)
+    serial_direction<NG, false>(q, k, v, gb, n, slots ? slots + kGlaStateFloats : nullptr, stage, obuf, DIRS == 3, lane);
   for (int t = 0; t < n; ++t) o[(size_t)t * 64 + lane] = oscale * obuf[t * 64 + lane];
 }
 
@@ -288,7 +294,7 @@ struct F32Place {
   int n, NT, ti;  // tokens left from the segment's start on, tiles, this wave's tile
   rsrc_t rq, rk, rv, rgf, rgb, ro;  // its tile's rows
 };
-template <int NG, bool BIDIR>
+template <int NG, int DIRS, bool HALVES>
 __device__ __forceinline__ F32Place<NG> f32_place(const float* q, const float* k, const float* v, const float* gf, const float* gb,
                                                   float* o, const F32Geo& geo) {
   constexpr int DK = 16 * NG;
@@ -297,11 +303,15 @@ __device__ __forceinline__ F32Place<NG> f32_place(const float* q, const float* k
   // waves w and w + 4 share a SIMD: tiles NT-1-w and w together see NT + 3 - w - (NT-1-w) ... the same number of tiles
   // in both directions
   p.NT = geo.NT, p.ti = w < 4 ? p.NT - 1 - w : w - 4;
-  const int first = 32 * (int)blockIdx.y * p.NT;
-  const size_t at = (size_t)blockIdx.x * geo.L + first;
+  int seq = blockIdx.x, seg = blockIdx.y;
+  const int which = (int)blockIdx.x - geo.whole;
+  if (HALVES) seg = 0, seq = which < 0 ? blockIdx.x : geo.whole + (which >> 1);
+  const int first = 32 * seg * p.NT;
+  const size_t at = (size_t)seq * geo.L + first;
   p.n = geo.L - first;
-  p.q = q + at * DK, p.k = k + at * DK, p.v = v + at * 64, p.gf = gf + at * DK, p.gb = (BIDIR ? gb : gf) + at * DK, p.o = o + at * 64;
-  p.slots = geo.states ? geo.states + ((size_t)blockIdx.x * geo.nseg + blockIdx.y) * 2 * kGlaStateFloats : nullptr;
+  p.q = q + at * DK, p.k = k + at * DK, p.v = v + at * 64, p.gf = gf + at * DK, p.gb = (DIRS & 2 ? gb : gf) + at * DK;
+  p.o = DIRS == 2 ? geo.half + (size_t)(which >> 1) * (32 * p.NT) * 64 : o + at * 64;
+  p.slots = geo.states ? geo.states + ((size_t)seq * geo.nseg + seg) * 2 * kGlaStateFloats : nullptr;
   const int nvalid = __builtin_amdgcn_readfirstlane(max(0, min(32, p.n - 32 * p.ti)));
   const int tile = 32 * p.ti;
   p.rq = chunk_rsrc(p.q + tile * DK, nvalid, 4 * DK), p.rk = chunk_rsrc(p.k + tile * DK, nvalid, 4 * DK);
@@ -314,8 +324,9 @@ enum F32Range { kInRange = 0, kGatesBeyond = 1, kValuesBeyond = 2 };
 
 // The walk of both directions; ANY: with prepare32_any, over the values' pieces that the pass before left in LDS.  Returns
 // (workgroup-uniform) what is beyond the form's range, before anything is stored.
-template <int NG, bool BIDIR, bool ANY>
+template <int NG, int DIRS, bool ANY>
 __device__ __forceinline__ int f32_pass(const F32Place<NG>& p, char* lds, float oscale) {
+  constexpr bool F1 = DIRS != 2;  // the first direction, or the only one
   const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
   const int NT = p.NT, ti = p.ti;
   const F32Lds<NG> lay(NT);
@@ -327,12 +338,13 @@ __device__ __forceinline__ int f32_pass(const F32Place<NG>& p, char* lds, float 
 
   f32x8_t xq[NG], xk[NG], xg[NG], qh[NG];
   f32x16_t P, O[2] = {f32x16_t{0.f}, f32x16_t{0.f}};
-  char* kreg = ti < NT - 1 ? lds + ti * F32Lds<NG>::KB : nullptr;
+  char* kreg = F1 ? (ti < NT - 1 ? lds + ti * F32Lds<NG>::KB : nullptr) : (ti > 0 ? lds + (ti - 1) * F32Lds<NG>::KB : nullptr);
   if (ANY) {
     lds_barrier();  // everyone has read the flags
     float grows = 0.f, sum = 0.f;
 #pragma unroll
-    for (int dir = 0; dir < (BIDIR ? 2 : 1); ++dir) {
+    for (int dir = 0; dir < 2; ++dir) {
+      if (!(DIRS & (1 << dir))) continue;
       load_rows_f32<NG>(dir ? p.rgb : p.rgf, r, h, xg);
 #pragma unroll
       for (int c = 0; c < NG; ++c)
@@ -344,10 +356,10 @@ __device__ __forceinline__ int f32_pass(const F32Place<NG>& p, char* lds, float 
     if (lane == 0) flags[ti] = refused ? kGatesBeyond : kInRange;
     lds_barrier();
     if (beyond(kGatesBeyond)) return kGatesBeyond;
-    load_rows_f32<NG>(p.rgf, r, h, xg);
+    load_rows_f32<NG>(F1 ? p.rgf : p.rgb, r, h, xg);
     load_rows_f32<NG>(p.rq, r, h, xq);
     load_rows_f32<NG>(p.rk, r, h, xk);
-    prepare32_any<NG, true>(xq, xk, xg, dall + 64 * ti, kreg, lane, qh, P);
+    prepare32_any<NG, F1>(xq, xk, xg, dall + 64 * ti, kreg, lane, qh, P);
     apply_values32(P, vreg, lane, O);
     lds_barrier();
   } else {
@@ -355,7 +367,7 @@ __device__ __forceinline__ int f32_pass(const F32Place<NG>& p, char* lds, float 
     {
       f32x8_t xv[2][2];
       load_pairs_f32(p.rv, r, h, xv);
-      load_rows_f32<NG>(p.rgf, r, h, xg);
+      load_rows_f32<NG>(F1 ? p.rgf : p.rgb, r, h, xg);
       load_rows_f32<NG>(p.rq, r, h, xq);
       load_rows_f32<NG>(p.rk, r, h, xk);
 #pragma unroll
@@ -370,16 +382,17 @@ __device__ __forceinline__ int f32_pass(const F32Place<NG>& p, char* lds, float 
     for (int c = 0; c < NG; ++c) mag += sum_abs(xq[c]) + sum_abs(xk[c]);
     const bool large = __builtin_amdgcn_ballot_w64(!(mag < kMagnitude32)) != 0;
     __builtin_amdgcn_sched_barrier(0);  // (the values' registers are free before the operands' are needed: 35.5 -> 34.8 us)
-    const bool wide = prepare32<NG, true>(xq, xk, xg, sc, dall + 64 * ti, kreg, lane, qh, P);
+    const bool wide = prepare32<NG, F1>(xq, xk, xg, sc, dall + 64 * ti, kreg, lane, qh, P);
     wave_lds_sync();
     apply_values32(P, vreg, lane, O);
     if (lane == 0) flags[ti] = large ? kValuesBeyond : wide ? kGatesBeyond : kInRange;
     lds_barrier();
     if (beyond(kGatesBeyond | kValuesBeyond)) return beyond(kValuesBeyond) ? kValuesBeyond : kGatesBeyond;
   }
-  walk32<NG, true>(lds, lay, ti, NT, lane, qh, O);
-  if (p.slots) apply_state32<NG, true>(p.slots, dall, ti > 0, lane, qh, O);
-  if (BIDIR) {
+  walk32<NG, F1>(lds, lay, ti, NT, lane, qh, O);
+  if (p.slots)
+    apply_state32<NG, F1>(p.slots + (F1 ? 0 : kGlaStateFloats), dall + (F1 ? 0 : 64 * (NT - 1)), F1 ? ti > 0 : ti < NT - 1, lane, qh, O);
+  if (DIRS == 3) {
     int r2 = r;
     asm volatile("" : "+v"(r2));  // (fetched again: carried across the walk, q and k would take 64 registers)
     load_rows_f32<NG>(p.rgb, r2, h, xg);
@@ -425,7 +438,7 @@ static_assert(offsetof(F32KernArgs, geo) == 6 * sizeof(void*) && offsetof(F32Ker
 // What is beyond the range, as a function of its own: its registers stay out of the common path's allocation.  (Arguments of a
 // called function come in vector registers, and a descriptor built from one puts a loop around every load: the function
 // reads the kernel's own through the argument block.)
-template <int NG, bool BIDIR>
+template <int NG, int DIRS, bool HALVES>
 __device__ __noinline__ void f32_beyond(const F32KernArgs* ka_in, int why) {
 #if defined(__HIP_DEVICE_COMPILE__)  // (the host pass has no constant address space to copy the geometry from)
   extern __shared__ __align__(16) char lds[];
@@ -434,22 +447,45 @@ __device__ __noinline__ void f32_beyond(const F32KernArgs* ka_in, int why) {
   const KernArgPtr ka = (KernArgPtr)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(kp >> 32)) << 32) |
                                      (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)kp));
   const F32Geo geo = ka->geo;
-  const auto p = f32_place<NG, BIDIR>(ka->q, ka->k, ka->v, ka->gf, ka->gb, ka->o, geo);
-  if (__builtin_amdgcn_readfirstlane(why) == kGatesBeyond && f32_pass<NG, BIDIR, true>(p, lds, ka->oscale) == kInRange) return;
-  serial_segment<NG, BIDIR>(p.q, p.k, p.v, p.gf, p.gb, p.o, p.slots, min(32 * p.NT, p.n), p.NT * 8192, ka->oscale);
+  const auto p = f32_place<NG, DIRS, HALVES>(ka->q, ka->k, ka->v, ka->gf, ka->gb, ka->o, geo);
+  if (__builtin_amdgcn_readfirstlane(why) == kGatesBeyond && f32_pass<NG, DIRS, true>(p, lds, ka->oscale) == kInRange) return;
+  serial_segment<NG, DIRS>(p.q, p.k, p.v, p.gf, p.gb, p.o, p.slots, min(32 * p.NT, p.n), p.NT * 8192, ka->oscale);
 #endif
 }
 
 }  // namespace
 
-template <int NG, bool BIDIR>
+template <int NG, int DIRS, bool HALVES>
 __global__ __launch_bounds__(512, 2) void gla_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
                                                          const float* __restrict__ v, const float* __restrict__ gf,
                                                          const float* __restrict__ gb, float* __restrict__ o, F32Geo geo,
                                                          float oscale) {
   extern __shared__ __align__(16) char lds[];
-  const int why = f32_pass<NG, BIDIR, false>(f32_place<NG, BIDIR>(q, k, v, gf, gb, o, geo), lds, oscale);
-  if (why != kInRange) f32_beyond<NG, BIDIR>((const F32KernArgs*)__builtin_amdgcn_kernarg_segment_ptr(), why);
+  const F32KernArgs* ka = (const F32KernArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+  if constexpr (!HALVES) {
+    const int why = f32_pass<NG, DIRS, false>(f32_place<NG, DIRS, false>(q, k, v, gf, gb, o, geo), lds, oscale);
+    if (why != kInRange) f32_beyond<NG, DIRS, false>(ka, why);
+  } else {
+    const int which = (int)blockIdx.x - geo.whole;
+    if (which < 0) {
+      const int why = f32_pass<NG, 3, false>(f32_place<NG, 3, true>(q, k, v, gf, gb, o, geo), lds, oscale);
+      if (why != kInRange) f32_beyond<NG, 3, true>(ka, why);
+    } else if ((which & 1) == 0) {
+      const int why = f32_pass<NG, 1, false>(f32_place<NG, 1, true>(q, k, v, gf, gb, o, geo), lds, oscale);
+      if (why != kInRange) f32_beyond<NG, 1, true>(ka, why);
+    } else {
+      const int why = f32_pass<NG, 2, false>(f32_place<NG, 2, true>(q, k, v, gf, gb, o, geo), lds, oscale);
+      if (why != kInRange) f32_beyond<NG, 2, true>(ka, why);
+    }
+  }
+}
+
+// What the reverse workgroups of sequences in two halves left is added to the forward ones' (a workgroup: a quarter of a sequence).
+__global__ __launch_bounds__(256) void gla_f32_add_kernel(float* __restrict__ o, F32Geo geo) {
+  const float* half = geo.half + (size_t)blockIdx.x * (32 * geo.NT) * 64;
+  float* to = o + (size_t)(geo.whole + blockIdx.x) * geo.L * 64;
+  for (int i = (blockIdx.y * 256 + threadIdx.x) * 4; i < geo.L * 64; i += 4096)
+    *reinterpret_cast<f32x4_t*>(to + i) += *reinterpret_cast<const f32x4_t*>(half + i);
 }
 
 // State pass of a long sequence: what every segment adds to the state of each direction, U = sum_t 2^(gates walked after
@@ -574,24 +610,36 @@ bool gla_f32_supported(const GlaArgs& a) {
 static size_t f32_states(long long nseq, int L, int NT) {
   return (size_t)nseq * (((L + 31) / 32 + NT - 1) / NT) * 2 * kGlaStateFloats * sizeof(float);
 }
-// (a call with room for segments of seven tiles only gets those)
-size_t gla_f32_least_workspace(int B, int H, int L, int Dk, int Dv) {
-  return gla_f32_workspace(B, H, L, Dk, Dv) == 0 ? 0 : f32_states((long long)B * H, L, gla_f32_segment_tiles(L));
+// Whole sequences whose directions go to two workgroups: what is left over of full rounds of the chip, where that fills no more than
+// half of one, from five tiles on.  us, whole / halves: Dk 32: 18 sequences of 185 tokens 21.0 / 16.2, 120 of 196 23.9 / 22.1, 384 50.3 /
+// 48.0; Dk 64: 18 of 185 30.0 / 21.9, 60 of 196 33.4 / 26.6, 384 71.7 / 65.5.  Below, the second launch and its memory cost what the
+// halves gain (Dk 32, 18 of 64 10.4 / 9.7; 108 of 85 called one by one 11.9 / 12.4), and so they do for segments (12 of 1031 28.0 / 30.4).
+template <int NG>
+static int f32_fwd_halves(int n, int NT) {
+  const int slots = 256 * std::max(1, std::min(kF32MaxLds / F32Lds<NG>(NT).total, 8 / NT)), rest = n % slots;
+  return NT >= 5 && 2 * rest <= slots ? rest : 0;
 }
-size_t gla_f32_workspace(int B, int H, int L, int Dk, int Dv) {
-  if ((Dk != 64 && Dk != 32) || Dv != 64 || gla_f32_segments(L) == 1) return 0;
-  return f32_states((long long)B * H, L, gla_f32_fine_tiles((long long)B * H, L));
+static size_t f32_half_bytes(int Dk, long long n, int NT) {
+  if (n > 0x3fffffff) return 0;
+  return (size_t)(Dk == 64 ? f32_fwd_halves<4>((int)n, NT) : f32_fwd_halves<2>((int)n, NT)) * 32 * NT * 64 * sizeof(float);
+}
+// (a call with room for segments of seven tiles only gets those; the halves' room is the last to go)
+size_t gla_f32_least_workspace(int B, int H, int L, int Dk, int Dv) {
+  return (Dk != 64 && Dk != 32) || Dv != 64 || gla_f32_segments(L) == 1 ? 0 : f32_states((long long)B * H, L, gla_f32_segment_tiles(L));
+}
+size_t gla_f32_workspace(int B, int H, int L, int Dk, int Dv, bool bidir) {
+  if ((Dk != 64 && Dk != 32) || Dv != 64 || (long long)B * H > 65535) return gla_f32_least_workspace(B, H, L, Dk, Dv);
+  const int NT = gla_f32_fine_tiles((long long)B * H, L), nseg = ((L + 31) / 32 + NT - 1) / NT;
+  return nseg > 1 ? f32_states((long long)B * H, L, NT) : bidir ? f32_half_bytes(Dk, (long long)B * H, NT) : 0;
 }
 
 template <int NG, bool BIDIR>
-static int launch_f32_t(const GlaArgs& a, const F32Geo& geo, int dev) {
-  static bool attr_done[64] = {};
-  if (!attr_done[dev]) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(gla_f32_kernel<NG, BIDIR>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                            kF32MaxLds) != hipSuccess)
-      return -5;
-    attr_done[dev] = true;
-  }
+static int launch_f32_t(const GlaArgs& a, F32Geo geo) {
+  constexpr int DIRS = BIDIR ? 3 : 1;
+  static bool done[64] = {}, done_halves[64] = {};
+  if (!allow_lds(reinterpret_cast<const void*>(gla_f32_kernel<NG, DIRS, false>), kF32MaxLds, done)) return -5;
+  if constexpr (BIDIR)
+    if (!allow_lds(reinterpret_cast<const void*>(gla_f32_kernel<NG, 3, true>), kF32MaxLds, done_halves)) return -5;
   const F32Lds<NG> lay(geo.NT);
   if (lay.total > kF32MaxLds || geo.NT * 8192 + 12 * 16 * NG * 4 > lay.total) return -95;
   if (geo.states) {
@@ -601,9 +649,22 @@ static int launch_f32_t(const GlaArgs& a, const F32Geo& geo, int dev) {
     const int rc = launch_gla_segment_scan((float*)a.workspace, nullptr, a.B * a.H, geo.nseg, BIDIR ? 2 : 1, NG, a.stream);
     if (rc) return rc;
   }
-  hipLaunchKernelGGL((gla_f32_kernel<NG, BIDIR>), dim3(a.B * a.H, geo.nseg), dim3(64 * geo.NT), lay.total, a.stream,
-                     (const float*)a.q, (const float*)a.k, (const float*)a.v, (const float*)a.g_fwd, (const float*)a.g_bwd,
-                     (float*)a.o, geo, a.scale * a.out_scale);
+  auto kernel = gla_f32_kernel<NG, DIRS, false>;
+  dim3 grid(a.B * a.H, geo.nseg);
+  int halves = 0;
+  if constexpr (BIDIR) {
+    const long long n = (long long)a.B * a.H;
+    const size_t need = geo.nseg == 1 ? f32_half_bytes(16 * NG, n, geo.NT) : 0;
+    if (need > 0 && a.workspace && need <= a.workspace_bytes) {
+      kernel = gla_f32_kernel<NG, 3, true>;
+      halves = f32_fwd_halves<NG>((int)n, geo.NT);
+      geo.whole = (int)n - halves, geo.half = (float*)a.workspace;
+      grid = dim3((unsigned)(n + halves));
+    }
+  }
+  hipLaunchKernelGGL(kernel, grid, dim3(64 * geo.NT), lay.total, a.stream, (const float*)a.q, (const float*)a.k, (const float*)a.v,
+                     (const float*)a.g_fwd, (const float*)a.g_bwd, (float*)a.o, geo, a.scale * a.out_scale);
+  if (halves) hipLaunchKernelGGL(gla_f32_add_kernel, dim3(halves, 4), dim3(256), 0, a.stream, (float*)a.o, geo);
   return hipGetLastError() == hipSuccess ? 0 : -5;
 }
 
@@ -621,17 +682,15 @@ int launch_gla_f32_states(int NG, const float* k, const float* v, const float* q
 }
 
 int launch_gla_f32(const GlaArgs& a) {
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return -5;
   F32Geo geo{};
   geo.L = a.L;
   const long long nseq = (long long)a.B * a.H;
   geo.NT = gla_f32_fine_tiles(nseq, a.L);
-  if (f32_states(nseq, a.L, geo.NT) > a.workspace_bytes) geo.NT = gla_f32_segment_tiles(a.L);
+  if (geo.NT * 32 < a.L && f32_states(nseq, a.L, geo.NT) > a.workspace_bytes) geo.NT = gla_f32_segment_tiles(a.L);
   geo.nseg = ((a.L + 31) / 32 + geo.NT - 1) / geo.NT;
   geo.states = geo.nseg > 1 ? (const float*)a.workspace : nullptr;
-  if (a.Dk == 64) return a.g_bwd ? launch_f32_t<4, true>(a, geo, dev) : launch_f32_t<4, false>(a, geo, dev);
-  return a.g_bwd ? launch_f32_t<2, true>(a, geo, dev) : launch_f32_t<2, false>(a, geo, dev);
+  if (a.Dk == 64) return a.g_bwd ? launch_f32_t<4, true>(a, geo) : launch_f32_t<4, false>(a, geo);
+  return a.g_bwd ? launch_f32_t<2, true>(a, geo) : launch_f32_t<2, false>(a, geo);
 }
 
 }  // namespace vig

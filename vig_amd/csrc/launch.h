@@ -77,7 +77,7 @@ inline int gla_f32_fine_tiles(long long nseq, int L) {
   return gla_f32_segment_tiles(L);
 }
 bool gla_f32_supported(const GlaArgs& a);
-size_t gla_f32_workspace(int B, int H, int L, int Dk, int Dv);
+size_t gla_f32_workspace(int B, int H, int L, int Dk, int Dv, bool bidir);
 size_t gla_f32_least_workspace(int B, int H, int L, int Dk, int Dv);
 int launch_gla_f32(const GlaArgs& a);
 // both sets of segment contributions of an fp32 backward: the states (k, v) and the gradient states (q, d_o)
