@@ -171,7 +171,8 @@ size_t vig_gla_bidir_fwd_workspace(int B, int H, int L, int Dk, int Dv, int io_d
     const size_t m = vig::gla_mfma_workspace(B, H, L, Dk, Dv);
     if (m > need) need = m;
   } else {
-    const size_t m = vig::gla_f32_workspace(B, H, L, Dk, Dv, true);
+    // (without the room for the directions' halves of leftover whole sequences, a quicker form that no call needs)
+    const size_t m = vig::gla_f32_workspace(B, H, L, Dk, Dv, false);
     if (m > need) need = m;
   }
   return need;
