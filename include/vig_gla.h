@@ -612,6 +612,18 @@ int vig_linear_fwd(const void* x, long long x_row_stride, const void* weight, co
                    long long rows, int N, int K, void* stream);
 
 /*
+ * Residual add, RMS norm and the SwiGLU layer behind it in one kernel, bf16, packed rows:
+ *   sum [rows, K] = x + residual (stored rounded; the norm is of the sum in fp32),  y [rows, I] = SwiGLU of rms(sum) * norm_weight . weight^T,
+ * weight [2*I, K] with the gate rows first: what vig_rmsnorm_fwd (round_sum 0) and vig_linear_swiglu_fwd give one after the other.
+ * K = 192 or 384, I % 32 == 0 and few rows (vig_norm_swiglu_preferred), else VIG_ENOTSUP.  sum is neither x nor residual.
+ *
+ * Replaces: classification/models/vig.py:486-496,604-606 (prenorm add, mlp_norm, gate_proj, up_proj and their product).
+ */
+int vig_norm_swiglu_preferred(long long rows, int K, int I);
+int vig_norm_swiglu_fwd(const void* x, const void* residual, const float* norm_weight, const void* weight, void* sum, void* y,
+                        long long rows, int K, int I, float eps, void* stream);
+
+/*
  * A linear layer without bias, the residual add and the RMS norm behind it in one kernel, bf16, packed rows:
  *   sum [rows, N] = residual + x [rows, K] . weight [N, K]^T (the product rounded to bf16, then the sum),  y = rms(sum) * norm_weight
  * N = 192, K % 64 == 0, else VIG_ENOTSUP.  sum and y are not the inputs.  _preferred: whether it is the better

@@ -1,0 +1,48 @@
+"""Residual add, RMS norm and SwiGLU layer of few rows in one kernel against the two kernels it stands for: one row, ragged row tiles, one
+and many column tiles, both widths."""
+import pytest
+import torch
+
+from vig_amd import _lib
+
+from .util import announce
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("rows,K,I", [(1, 192, 32), (49, 192, 512), (196, 192, 512), (33, 384, 1024), (196, 384, 1024), (256, 384, 1024), (2048, 192, 128)])
+def test_against_two_kernels(rows, K, I):
+    announce(f"norm and SwiGLU rows{rows} K{K} I{I}")
+    gen = torch.Generator().manual_seed(rows)
+    x, res = (torch.randn(rows, K, generator=gen).bfloat16().cuda() for _ in range(2))
+    w = (torch.randn(2 * I, K, generator=gen) * K ** -0.5).bfloat16().cuda()
+    nw = (torch.rand(K, generator=gen) + 0.5).cuda()
+    lib, st = _lib.load(), torch.cuda.current_stream().cuda_stream
+    assert lib.vig_norm_swiglu_preferred(rows, K, I)
+    total, y = torch.full_like(x, float("nan")), torch.full((rows, I), float("nan"), dtype=x.dtype, device="cuda")
+    assert lib.vig_norm_swiglu_fwd(*(t.data_ptr() for t in (x, res, nw, w, total, y)), rows, K, I, 1e-5, st) == _lib.VIG_OK
+    normed, sum2, want = torch.empty_like(x), torch.empty_like(x), torch.empty_like(y)
+    assert lib.vig_rmsnorm_fwd(x.data_ptr(), res.data_ptr(), nw.data_ptr(), normed.data_ptr(), sum2.data_ptr(), rows, K, 1e-5, 0, 1, st) == _lib.VIG_OK
+    assert lib.vig_linear_swiglu_fwd(normed.data_ptr(), w.data_ptr(), want.data_ptr(), rows, K, I, 1, st) == _lib.VIG_OK
+    assert torch.equal(total, sum2)
+    # a norm that differs in its last fp32 bit moves a value by an ulp of bf16 now and then, a pre-activation and the output likewise
+    s = x.double() + res.double()
+    n = s * torch.rsqrt(s.pow(2).mean(-1, keepdim=True) + 1e-5) * nw.double()
+    g, u = (n @ w.double().t()).chunk(2, 1)
+    exact = torch.nn.functional.silu(g) * u
+    spread = (n.abs() @ w.double().abs().t()).chunk(2, 1)
+    # inputs rounded to bf16 once (errors add up as the root of the terms: 8 sigma of 2^-9 relative), factors and product once each
+    bound = 8 * 2.0 ** -9 * K ** -0.5 * (spread[0] * u.abs() + spread[1] * g.abs()) + 2.0 ** -6 * exact.abs() + 2.0 ** -7 * (g.abs() + u.abs()) * 2.0 ** -2
+    assert ((y.double() - exact).abs() <= bound).all()
+    assert (y.double() - want.double()).abs().max() <= 2.0 ** -6 * want.double().abs().max() and (y != want).float().mean() < 0.02
+
+
+def test_refused():
+    t = torch.zeros(4096, 384, dtype=torch.bfloat16, device="cuda")
+    f, lib, st = torch.ones(384, device="cuda"), _lib.load(), torch.cuda.current_stream().cuda_stream
+    call = lambda x, s, rows, K, I: lib.vig_norm_swiglu_fwd(x, t.data_ptr(), f.data_ptr(), t.data_ptr(), s, t.data_ptr(), rows, K, I, 1e-5, st)  # noqa: E731
+    other = torch.zeros_like(t)
+    assert call(other.data_ptr(), other.data_ptr(), 32, 384, 32) == _lib.VIG_EINVAL  # the sum over its input
+    out = torch.zeros_like(t)
+    assert call(other.data_ptr(), out.data_ptr(), 4096, 384, 1024) == _lib.VIG_ENOTSUP  # many rows
+    assert call(other.data_ptr(), out.data_ptr(), 32, 256, 32) == _lib.VIG_ENOTSUP  # another width

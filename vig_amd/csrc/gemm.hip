@@ -158,6 +158,122 @@ __global__ __launch_bounds__(64 * NW) void gemm_few_kernel(GemmArgs a) {
 }
 
 // ---------------------------------------------------------------------------
+// Few rows: residual add, RMS norm and the SwiGLU layer behind it in one kernel, K = 64 NV.  A workgroup's 32 rows are whole rows of the
+// contraction, so it makes their sums and norms itself (eight lanes a row; every column tile again, out of the L2, the first one
+// stores the sums) while its weights arrive; a launch costs more than that.  us, norm and layer / this, rows x K -> I:
+// 1 x 192 -> 512 4.4 / 3.4, 196 x 192 -> 512 5.1 / 3.6, 392 x 192 -> 512 5.1 / 3.8, 1 x 384 -> 1024 4.8 / 4.6, 256 x 384 -> 1024
+// 5.6 / 5.3; other widths, and more rows than 256 workgroups take, keep the two.
+// ---------------------------------------------------------------------------
+struct NormPairArgs {
+  const uint16_t *x, *residual, *w;  // rows [M, K], [M, K]; weights [2 N, K], gate rows first
+  const float* norm;
+  uint16_t *sum, *y;  // [M, K], [M, N]
+  int M, N;
+  float eps;
+};
+template <int NV>
+__global__ __launch_bounds__(256) void gemm_norm_pair_kernel(NormPairArgs a) {
+  constexpr int K = 64 * NV, NW = 4, kStages = K / kStageK, kMine = (kStages + NW - 1) / NW, kX = 2048 * kStages;
+  __shared__ __align__(16) char smem[kX + NW * kMine * 4096 > 36864 ? kX + NW * kMine * 4096 : 36864];
+  const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int m0 = blockIdx.y * 32, n0 = blockIdx.x * 32;
+  // ---- the weights of this wave's stages (wave, wave + 4, ..), all of them under way at once ----
+  const uint32_t w0 = lds_offset(smem) + kX + wave * (kMine * 4096);
+#pragma unroll
+  for (int at = 0; at < kMine; ++at) {
+    const int s = wave + NW * at;
+    if (s < kStages) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int row = 16 * i + (lane >> 2), unit = (lane & 3) ^ ((row >> 2) & 3);
+        const uint16_t* wp = a.w + (size_t)min(n0 + row, a.N - 1) * K + 8 * unit + s * kStageK;
+        load_to_lds16(wp, w0 + at * 4096 + 1024 * i);
+        load_to_lds16(wp + (size_t)a.N * K, w0 + at * 4096 + 2048 + 1024 * i);
+      }
+    }
+  }
+  // ---- sums and norms of 8 rows a wave ----
+  {
+    const int row = 8 * wave + (lane >> 3), sub = lane & 7, m = min(m0 + row, a.M - 1);
+    const size_t base = (size_t)m * K;
+    Raw8<uint16_t> x[NV], res[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) x[i].load(a.x + base + 8 * (sub + 8 * i)), res[i].load(a.residual + base + 8 * (sub + 8 * i));
+    float s[NV][8], ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      float b[8];
+      x[i].unpack(s[i]);
+      res[i].unpack(b);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) s[i][j] += b[j], ss = __builtin_fmaf(s[i][j], s[i][j], ss);
+    }
+#pragma unroll
+    for (int d = 1; d < 8; d <<= 1) ss += __shfl_xor(ss, d);
+    const float rstd = 1.0f / sqrtf(ss / (float)K + a.eps);
+    const bool keep = blockIdx.x == 0 && m0 + row < a.M;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int o = sub + 8 * i;
+      const f32x4_t wa = *reinterpret_cast<const f32x4_t*>(a.norm + 8 * o), wb = *reinterpret_cast<const f32x4_t*>(a.norm + 8 * o + 4);
+      u32x4_t y, sum;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float p = j < 2 ? wa[2 * j] : wb[2 * j - 4], q = j < 2 ? wa[2 * j + 1] : wb[2 * j - 3];
+        y[j] = pack_bf16x2(s[i][2 * j] * rstd * p, s[i][2 * j + 1] * rstd * q);
+        sum[j] = pack_bf16x2(s[i][2 * j], s[i][2 * j + 1]);
+      }
+      *reinterpret_cast<u32x4_t*>(smem + (o >> 2) * 2048 + row * 64 + 16 * ((o & 3) ^ ((row >> 2) & 3))) = y;
+      if (keep) *reinterpret_cast<u32x4_t*>(a.sum + base + 8 * o) = sum;
+    }
+  }
+  wait_vmem<0>();
+  __syncthreads();
+  f32x16_t acc[2] = {f32x16_t{0.f}, f32x16_t{0.f}};
+#pragma unroll
+  for (int at = 0; at < kMine; ++at) {
+    const int s = wave + NW * at;
+    if (s < kStages) {
+      const char* wbuf = smem + kX + wave * (kMine * 4096) + at * 4096;
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const int off = r * 64 + 16 * ((2 * k + h) ^ ((r >> 2) & 3));
+        const bf16x8_t xf = *reinterpret_cast<const bf16x8_t*>(smem + s * 2048 + off);
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const bf16x8_t*>(wbuf + 2048 * j + off), xf, acc[j], 0, 0, 0);
+      }
+    }
+  }
+  // accumulator register 4g+m of lane (r, h) is channel 8g+4h+m of token r
+  __syncthreads();
+  float(*part)[2][32][36] = reinterpret_cast<float(*)[2][32][36]>(smem);
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      *reinterpret_cast<f32x4_t*>(&part[wave][j][r][8 * g + 4 * h]) = f32x4_t{acc[j][4 * g], acc[j][4 * g + 1], acc[j][4 * g + 2], acc[j][4 * g + 3]};
+  __syncthreads();
+  const int row = threadIdx.x >> 3, c = (threadIdx.x & 7) * 4;
+  f32x4_t sum[2];
+#pragma unroll
+  for (int m = 0; m < 2; ++m) {
+    sum[m] = *reinterpret_cast<const f32x4_t*>(&part[0][m][row][c]);
+#pragma unroll
+    for (int k = 1; k < NW; ++k) sum[m] += *reinterpret_cast<const f32x4_t*>(&part[k][m][row][c]);
+  }
+  if (m0 + row < a.M && n0 + c < a.N) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {  // on the values the separate layer would have stored
+      const float g = bf16_to_f32(f32_to_bf16(sum[0][j])), u = bf16_to_f32(f32_to_bf16(sum[1][j]));
+      sum[0][j] = g * u * sigmoidf_(g);
+    }
+    *reinterpret_cast<u32x2_t*>(a.y + (size_t)(m0 + row) * a.N + n0 + c) = u32x2_t{pack_bf16x2(sum[0][0], sum[0][1]), pack_bf16x2(sum[0][2], sum[0][3])};
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Many rows: tiles of 64 MI x 64 NI by four waves of 32 MI x 32 NI each, operands through kBuffers LDS stages of 32
 // contraction elements (64-byte row pieces, loaded directly to LDS; the 16-byte units of a piece are swapped by a quarter of the row
 // number: the sixteen lanes served together read four rows that start in each bank quarter, and their units differ).
@@ -485,6 +601,18 @@ int launch_few_swiglu(const void* x, const void* w, void* y, long long T, int K,
   if (!few_swiglu(T, K, I)) return -95;
   const GemmArgs a{(const uint16_t*)x, (const uint16_t*)w, nullptr, (uint16_t*)y, K, I, (int)T, I, K, 0, 0, 0, 0, 0};
   return launch_few<4, kPair>(a, stream);
+}
+
+// The same with the residual add and the RMS norm in front.
+bool norm_swiglu_supported(long long T, int K, int I) { return (K == 192 || K == 384) && few_swiglu(T, K, I); }
+int launch_norm_swiglu(const void* x, const void* residual, const float* norm, const void* w, void* sum, void* y, long long T, int K, int I,
+                       float eps, hipStream_t stream) {
+  if (!norm_swiglu_supported(T, K, I)) return -95;
+  const NormPairArgs a{(const uint16_t*)x, (const uint16_t*)residual, (const uint16_t*)w, norm, (uint16_t*)sum, (uint16_t*)y, (int)T, I, eps};
+  const dim3 grid(I / 32, (unsigned)((T + 31) / 32));
+  if (K == 192) hipLaunchKernelGGL(gemm_norm_pair_kernel<3>, grid, dim3(256), 0, stream, a);
+  else hipLaunchKernelGGL(gemm_norm_pair_kernel<6>, grid, dim3(256), 0, stream, a);
+  return hipGetLastError() == hipSuccess ? 0 : -5;
 }
 
 // The convolution library took 12 to 138 us where these take 4.3 to 96: B 1, 28 x 28 x 96 -> 192 4.3 / 12.3; B 32, 192 -> 384

@@ -144,6 +144,9 @@ int launch_linear_regs(const void* x, const void* w, const void* bias, void* y, 
 int launch_linear_columns(const void* x, const void* w, void* y, long long T, int N, int K, hipStream_t stream);
 int launch_linear_swiglu_bwd(const void* d_out, const void* w_down, const void* kept, void* d_kept, long long T, int K, int I,
                              hipStream_t stream);
+bool norm_swiglu_supported(long long T, int K, int I);
+int launch_norm_swiglu(const void* x, const void* residual, const float* norm, const void* w, void* sum, void* y, long long T, int K, int I,
+                       float eps, hipStream_t stream);
 bool linear_norm_supported(long long M, int N, int K);
 int launch_linear_norm(const void* x, const void* w, const void* residual, const float* norm, void* y, void* sum, long long M, int N,
                        int K, float eps, hipStream_t stream);

@@ -243,10 +243,15 @@ Tensor run(const Plan& p, const Tensor& images) {
       k.linear(y, b.w_o, Tensor(), branch1, T);
     }
     const int64_t next = hidden == res0 ? res1 : res0;
-    k.norm(branch1, hidden, b.norm2, b.eps2, false, y, next, T);
     residual = next;
     const int64_t width = b.w_down.size(1);
-    if (swiglu_kernel) {
+    const bool with_norm = swiglu_kernel && vig_norm_swiglu_preferred(T, (int)C, (int)width);
+    if (!with_norm) k.norm(branch1, hidden, b.norm2, b.eps2, false, y, next, T);
+    if (with_norm) {
+      check_rc(vig_norm_swiglu_fwd(k.at(branch1), k.at(hidden), f32(b.norm2), b.w_gate.data_ptr(), k.at(next), k.at(mid), T, (int)C, (int)width,
+                                   (float)b.eps2, k.stream),
+               "vig_norm_swiglu_fwd");
+    } else if (swiglu_kernel) {
       check_rc(vig_linear_swiglu_fwd(k.at(y), b.w_gate.data_ptr(), k.at(mid), T, (int)C, (int)width, VIG_BF16, k.stream),
                "vig_linear_swiglu_fwd");
     } else {
