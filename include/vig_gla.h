@@ -612,6 +612,18 @@ int vig_linear_fwd(const void* x, long long x_row_stride, const void* weight, co
                    long long rows, int N, int K, void* stream);
 
 /*
+ * Residual add, RMS norm and the depthwise 3x3 convolution behind it in one kernel, bf16, few grid rows:
+ *   sum [B, h*w, C] = x + residual (rounded; residual NULL: x),  y = conv3x3(rms(sum) * norm_weight) (+ bias, SiLU): what
+ * vig_rmsnorm_fwd (round_sum 1) and vig_dwconv3x3_fwd give one after the other.  weight [C, 9], bias [C] or NULL; sum may be NULL.
+ * C = 192 or 384 and few rows (vig_norm_dwconv3x3_preferred), else VIG_ENOTSUP.  No output may be an input.
+ *
+ * Replaces: classification/models/vig.py:291-294,364-366,598-606 (attn_norm, local convolution).
+ */
+int vig_norm_dwconv3x3_preferred(int B, int h, int w, int C);
+int vig_norm_dwconv3x3_fwd(const void* x, const void* residual, const float* norm_weight, const float* weight, const float* bias,
+                           void* sum, void* y, int B, int h, int w, int C, float eps, int silu, void* stream);
+
+/*
  * Residual add, RMS norm and the SwiGLU layer behind it in one kernel, bf16, packed rows:
  *   sum [rows, K] = x + residual (stored rounded; the norm is of the sum in fp32),  y [rows, I] = SwiGLU of rms(sum) * norm_weight . weight^T,
  * weight [2*I, K] with the gate rows first: what vig_rmsnorm_fwd (round_sum 0) and vig_linear_swiglu_fwd give one after the other.

@@ -585,6 +585,20 @@ int vig_dwconv3x3_fwd(const void* x, const float* weight, const float* bias, voi
   return vig_dwconv3x3_fwd_pre(x, weight, bias, y, nullptr, B, h, w, C, silu, io_dtype, stream);
 }
 
+int vig_norm_dwconv3x3_preferred(int B, int h, int w, int C) {
+  return B > 0 && h > 0 && w > 0 && vig::norm_dwconv3x3_supported(B, h, w, C);
+}
+
+int vig_norm_dwconv3x3_fwd(const void* x, const void* residual, const float* norm_weight, const float* weight, const float* bias,
+                           void* sum, void* y, int B, int h, int w, int C, float eps, int silu, void* stream) {
+  if (!x || !norm_weight || !weight || !y || B <= 0 || h <= 0 || w <= 0 || C <= 0) return VIG_EINVAL;
+  // (a workgroup reads its neighbours' rows: nothing may be written over an input)
+  if (y == x || y == residual || y == sum || (sum && (sum == x || sum == residual))) return VIG_EINVAL;
+  if (!aligned16(x, residual, norm_weight, weight, sum, y) || !aligned16(bias)) return VIG_EINVAL;
+  if (!vig::norm_dwconv3x3_supported(B, h, w, C)) return VIG_ENOTSUP;
+  return vig::launch_norm_dwconv3x3(x, residual, norm_weight, weight, bias, sum, y, B, h, w, C, eps, silu, (hipStream_t)stream);
+}
+
 size_t vig_dwconv3x3_bwd_weight_workspace(int B, int C) {
   if (B <= 0 || C <= 0) return 0;
   return vig::dwconv3x3_wgrad_workspace(B, C);

@@ -616,6 +616,127 @@ int launch_locality_gate(const void* o, const float* wt, void* y, int B, int H, 
 }
 
 // ---------------------------------------------------------------------------
+// Few grid rows: residual add, RMS norm and the depthwise 3x3 convolution behind it in one kernel, bf16, C = 24 LANES channels.  A
+// workgroup makes up to 14 cells of a grid row: the sums and norms of these and of the cells around them (LANES lanes a token; a row's norm is
+// made three times, out of the L2), the norms staged rounded in LDS between zeros, then the taps.  Latency bounds it: two launches
+// with a chain of loads each became one, every load of a workgroup under way at once, the taps' weights by way of LDS (fetched by the
+// octets of 72 that a thread needs, as above, they cost 1.8 us at C 192 and 3 at 384).  us, the two kernels / this: C 192 1 x 14 x 14 6.5
+// / 4.3, 2 x 48 x 48 9.7 / 5.8, 48 x 14 x 14 13.7 / 7.9; C 384 1 x 14 x 14 6.5 / 4.9, 32 x 14 x 14 13.8 / 9.2.
+// ---------------------------------------------------------------------------
+constexpr int kNormStencilCols = 14;  // with the two beside them in three rows: 48 tokens
+
+struct NormStencilArgs {
+  const uint16_t *x, *residual;  // [B, h*w, C]; no residual: null
+  const float *norm, *wt, *bias; // [C], [C, 9], [C] or null
+  uint16_t *sum, *y;             // [B, h*w, C]; sum may be null
+  int h, w, cols, silu;
+  float eps;
+};
+template <int LANES>  // all the tokens at a time; then four columns of channel pairs
+__global__ __launch_bounds__(48 * LANES) void norm_stencil_kernel(NormStencilArgs a) {
+  constexpr int NV = 3, C = 8 * NV * LANES, kThreads = 48 * LANES, kPairs = C / 2, kCols = kThreads / kPairs;
+  extern __shared__ __align__(16) char smem[];
+  uint16_t* tile = reinterpret_cast<uint16_t*>(smem);  // [3 * (columns + 2)][C]
+  const int img = blockIdx.x / a.h, row = blockIdx.x - img * a.h;
+  const int c0 = blockIdx.y * a.cols, cols = min(a.cols, a.w - c0), pw = cols + 2;
+  const size_t image = (size_t)img * a.h * a.w * C;
+  float* wts = reinterpret_cast<float*>(smem + 6 * (kNormStencilCols + 2) * C);  // [C][9]
+  const int pair = threadIdx.x % kPairs, col = threadIdx.x / kPairs;
+  constexpr int kWLoads = (C * 9 / 4 + kThreads - 1) / kThreads;
+  f32x4_t wraw[kWLoads];
+#pragma unroll
+  for (int i = 0; i < kWLoads; ++i) {
+    const int at = (int)threadIdx.x + i * kThreads;
+    if (at < C * 9 / 4) wraw[i] = *reinterpret_cast<const f32x4_t*>(a.wt + 4 * at);
+  }
+  const float b0 = a.bias ? a.bias[2 * pair] : 0.f, b1 = a.bias ? a.bias[2 * pair + 1] : 0.f;
+  const int sub = threadIdx.x % LANES;
+  const int t = threadIdx.x / LANES;
+  if (t < 3 * pw) {  // padded cell (pr, pc) is grid cell (row - 1 + pr, c0 + pc - 1)
+    const int pr = t / pw, r = row - 1 + pr, pc = t - pr * pw, c = c0 + pc - 1;
+    const bool in = r >= 0 && r < a.h && c >= 0 && c < a.w;
+    const size_t at = in ? image + (size_t)(r * a.w + c) * C : 0;
+    Raw8<uint16_t> x[NV], res[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      x[i].zero(), res[i].zero();
+      if (in) x[i].load(a.x + at + 8 * (sub + LANES * i));
+      if (in && a.residual) res[i].load(a.residual + at + 8 * (sub + LANES * i));
+    }
+    float s[NV][8], ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      float b[8];
+      x[i].unpack(s[i]);
+      res[i].unpack(b);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {  // the rounded sum
+        res[i].a[j] = pack_bf16x2(s[i][2 * j] + b[2 * j], s[i][2 * j + 1] + b[2 * j + 1]);
+      }
+      res[i].unpack(s[i]);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) ss = __builtin_fmaf(s[i][j], s[i][j], ss);
+    }
+#pragma unroll
+    for (int d = 1; d < LANES; d <<= 1) ss += __shfl_xor(ss, d);
+    const float rstd = 1.0f / sqrtf(ss / (float)C + a.eps);
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int o = 8 * (sub + LANES * i);
+      const f32x4_t wa = *reinterpret_cast<const f32x4_t*>(a.norm + o), wb = *reinterpret_cast<const f32x4_t*>(a.norm + o + 4);
+      u32x4_t n;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float p = j < 2 ? wa[2 * j] : wb[2 * j - 4], q = j < 2 ? wa[2 * j + 1] : wb[2 * j - 3];
+        n[j] = in ? pack_bf16x2(s[i][2 * j] * rstd * p, s[i][2 * j + 1] * rstd * q) : 0u;
+      }
+      *reinterpret_cast<u32x4_t*>(tile + t * C + o) = n;
+      if (in && pr == 1 && pc >= 1 && pc <= cols && a.sum) res[i].store(a.sum + at + o);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < kWLoads; ++i) {
+    const int at = (int)threadIdx.x + i * kThreads;
+    if (at < C * 9 / 4) *reinterpret_cast<f32x4_t*>(wts + 4 * at) = wraw[i];
+  }
+  __syncthreads();
+  float wreg[18];
+#pragma unroll
+  for (int i = 0; i < 9; ++i) wreg[2 * i] = wts[pair * 18 + 2 * i], wreg[2 * i + 1] = wts[pair * 18 + 2 * i + 1];
+  for (int c = col; c < cols; c += kCols) {
+    const uint16_t* p = tile + c * C + pair * 2;  // padded cell of tap (-1, -1)
+    float lo = b0, hi = b1;
+#pragma unroll
+    for (int di = 0; di < 3; ++di)
+#pragma unroll
+      for (int dj = 0; dj < 3; ++dj) {
+        const uint32_t v = *reinterpret_cast<const uint32_t*>(p + (di * pw + dj) * C);
+        lo = __builtin_fmaf(bf16lo_to_f32(v), wreg[di * 3 + dj], lo), hi = __builtin_fmaf(bf16hi_to_f32(v), wreg[9 + di * 3 + dj], hi);
+      }
+    if (a.silu) lo = lo * sigmoidf_(lo), hi = hi * sigmoidf_(hi);
+    *reinterpret_cast<uint32_t*>(a.y + image + (size_t)(row * a.w + c0 + c) * C + pair * 2) = pack_bf16x2(lo, hi);
+  }
+}
+
+bool norm_dwconv3x3_supported(int B, int h, int w, int C) {
+  const int parts = (w - 1) / kNormStencilCols + 1;
+  // Up to 1024 workgroups of 384 channels.  Past that the cells around a workgroup's, read and normed three times, cost what the launch
+  // saves: C 192 128 x 14 x 14 21.3 / 18.4 us, 256 x 14 x 14 30.8 / 30.4; C 384 64 x 14 x 14 19.5 / 17.8, 96 x 14 x 14 25.1 / 24.6, 128 x 14 x 14 27.8 / 30.0.
+  return (C == 192 || C == 384) && parts <= 65535 && (long long)B * h * w <= 0x7fffffff && (long long)B * h * parts <= 1024 * 384 / C;
+}
+int launch_norm_dwconv3x3(const void* x, const void* residual, const float* norm, const float* wt, const float* bias, void* sum, void* y,
+                          int B, int h, int w, int C, float eps, int silu, hipStream_t stream) {
+  if (!norm_dwconv3x3_supported(B, h, w, C)) return -95;
+  const int parts = (w - 1) / kNormStencilCols + 1, cols = (w + parts - 1) / parts;
+  const NormStencilArgs a{(const uint16_t*)x, (const uint16_t*)residual, norm, wt, bias, (uint16_t*)sum, (uint16_t*)y, h, w, cols, silu, eps};
+  const size_t lds = (6 * (kNormStencilCols + 2) + 36) * (size_t)C;
+  const dim3 grid(B * h, (w + cols - 1) / cols);
+  if (C == 192) hipLaunchKernelGGL(norm_stencil_kernel<8>, grid, dim3(2 * C), lds, stream, a);
+  else hipLaunchKernelGGL(norm_stencil_kernel<16>, grid, dim3(2 * C), lds, stream, a);
+  return hipGetLastError() == hipSuccess ? 0 : -5;
+}
+
+// ---------------------------------------------------------------------------
 // RMS-norm blend epilogue.  One group of Dv/8 lanes owns one (b, l, head) row of
 // Dv values; the two mean-squares are reduced with lane shuffles inside the group.
 //   y[b,l,hd*Dv+d] = rms(o[b,hd,l,:])*w_g*s + rms(local[b,l,hd,:])*w_l*(1-s)

@@ -144,6 +144,9 @@ int launch_linear_regs(const void* x, const void* w, const void* bias, void* y, 
 int launch_linear_columns(const void* x, const void* w, void* y, long long T, int N, int K, hipStream_t stream);
 int launch_linear_swiglu_bwd(const void* d_out, const void* w_down, const void* kept, void* d_kept, long long T, int K, int I,
                              hipStream_t stream);
+bool norm_dwconv3x3_supported(int B, int h, int w, int C);
+int launch_norm_dwconv3x3(const void* x, const void* residual, const float* norm, const float* wt, const float* bias, void* sum, void* y,
+                          int B, int h, int w, int C, float eps, int silu, hipStream_t stream);
 bool norm_swiglu_supported(long long T, int K, int I);
 int launch_norm_swiglu(const void* x, const void* residual, const float* norm, const void* w, void* sum, void* y, long long T, int K, int I,
                        float eps, hipStream_t stream);

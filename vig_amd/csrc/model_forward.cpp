@@ -197,16 +197,19 @@ Tensor run(const Plan& p, const Tensor& images) {
     const Block& b = p.blocks[i];
     const int64_t n0 = (int64_t)b.H * (2 * b.Dk + b.Dv), n1c = n0 + (int64_t)b.H * b.Dv, ld = b.w_in.size(0);
     int64_t hidden = branch0;
-    if (normed) {
-      hidden = residual;
-    } else if (residual < 0) {
-      k.norm(branch0, -1, b.norm1, b.eps1, false, y, -1, T);
-    } else {  // the explicit add of the reference stores a rounded sum and attn_norm normalises that (vig.py:598,606)
-      hidden = residual == res0 ? res1 : res0;
-      k.norm(branch0, residual, b.norm1, b.eps1, true, y, hidden, T);
+    // the explicit add of the reference stores a rounded sum and attn_norm normalises that (vig.py:598,606)
+    const bool sums = !normed && residual >= 0;
+    if (normed) hidden = residual;
+    else if (sums) hidden = residual == res0 ? res1 : res0;
+    if (!normed && vig_norm_dwconv3x3_preferred((int)B, st.gh, st.gw, (int)C)) {
+      check_rc(vig_norm_dwconv3x3_fwd(k.at(branch0), sums ? k.at(residual) : nullptr, f32(b.norm1), f32(b.conv_w), f32(b.conv_b),
+                                      sums ? k.at(hidden) : nullptr, k.at(xs), (int)B, st.gh, st.gw, (int)C, (float)b.eps1, b.act, k.stream),
+               "vig_norm_dwconv3x3_fwd");
+    } else {
+      if (!normed) k.norm(branch0, sums ? residual : -1, b.norm1, b.eps1, sums, y, sums ? hidden : -1, T);
+      check_rc(vig_dwconv3x3_fwd(k.at(y), f32(b.conv_w), f32(b.conv_b), k.at(xs), (int)B, st.gh, st.gw, (int)C, b.act, VIG_BF16, k.stream),
+               "vig_dwconv3x3_fwd");
     }
-    check_rc(vig_dwconv3x3_fwd(k.at(y), f32(b.conv_w), f32(b.conv_b), k.at(xs), (int)B, st.gh, st.gw, (int)C, b.act, VIG_BF16, k.stream),
-             "vig_dwconv3x3_fwd");
     k.linear(xs, b.w_in, b.b_in, z, T);
     const float scale = 1.0f / std::sqrt((float)b.Dk);
     const long long sqk[3] = {(long long)(L * ld), b.Dk, ld}, sv[3] = {(long long)(L * ld), b.Dv, ld};
