@@ -612,10 +612,10 @@ int vig_linear_fwd(const void* x, long long x_row_stride, const void* weight, co
                    long long rows, int N, int K, void* stream);
 
 /*
- * Residual add, RMS norm and the depthwise 3x3 convolution behind it in one kernel, bf16, few grid rows:
+ * Residual add, RMS norm and the depthwise 3x3 convolution behind it in one kernel, bf16:
  *   sum [B, h*w, C] = x + residual (rounded; residual NULL: x),  y = conv3x3(rms(sum) * norm_weight) (+ bias, SiLU): what
  * vig_rmsnorm_fwd (round_sum 1) and vig_dwconv3x3_fwd give one after the other.  weight [C, 9], bias [C] or NULL; sum may be NULL.
- * C = 192 or 384 and few rows (vig_norm_dwconv3x3_preferred), else VIG_ENOTSUP.  No output may be an input.
+ * C = 192 or 384 and sizes where it is quicker than those (vig_norm_dwconv3x3_preferred), else VIG_ENOTSUP.  No output may be an input.
  *
  * Replaces: classification/models/vig.py:291-294,364-366,598-606 (attn_norm, local convolution).
  */

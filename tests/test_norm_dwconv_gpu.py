@@ -1,5 +1,6 @@
-"""Residual add, RMS norm and depthwise convolution of few grid rows in one kernel against the two kernels it stands for: single cells, rows
-narrower and wider than a workgroup's cells, a last part of one column, images next to each other, both widths, with and without the options."""
+"""Residual add, RMS norm and depthwise convolution in one kernel against the two kernels it stands for: single cells, rows
+narrower and wider than a workgroup's cells, images next to each other, both widths, with and without the options; walks of a few
+rows with a short last band, and of all rows."""
 import pytest
 import torch
 
@@ -11,7 +12,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("B,h,w,C,full", [(1, 1, 1, 192, True), (1, 14, 14, 192, True), (2, 14, 14, 384, False), (3, 5, 15, 384, True),
-                                          (1, 3, 17, 192, False), (1, 4, 29, 384, True), (1, 2, 64, 192, True)])
+                                          (1, 3, 17, 192, False), (1, 4, 29, 384, True), (1, 2, 64, 192, True),
+                                          (100, 13, 14, 384, True), (64, 13, 27, 192, False), (250, 14, 14, 384, True)])
 def test_against_two_kernels(B, h, w, C, full):
     announce(f"norm and convolution {B}x{h}x{w}x{C} options {full}")
     gen = torch.Generator().manual_seed(h * w)
@@ -27,11 +29,11 @@ def test_against_two_kernels(B, h, w, C, full):
     assert lib.vig_rmsnorm_fwd(p(x), p(res), p(nw), p(normed), sum2.data_ptr() if full else None, B * h * w, C, 1e-5, int(full), 1, st) == _lib.VIG_OK
     assert lib.vig_dwconv3x3_fwd(p(normed), p(wt), p(bias), p(want), B, h, w, C, int(full), 1, st) == _lib.VIG_OK
     assert not full or torch.equal(total, sum2)
-    # a norm whose last fp32 bit differs moves a normed value by an ulp of bf16 now and then: 2^-8 of it, so of the taps' sum of
-    # magnitudes (SiLU's slope is below 1.1), and the result is rounded once more
+    # a norm whose last fp32 bit differs moves a normed value by an ulp of bf16 now and then: 2^-7 of it at most, so of the taps' sum of
+    # magnitudes (SiLU's slope is below 1.1); the two results are rounded by half an ulp each
     grid = normed.float().abs().view(B, h, w, C).permute(0, 3, 1, 2)
     taps = torch.nn.functional.conv2d(grid, wt.abs().view(C, 1, 3, 3), padding=1, groups=C).permute(0, 2, 3, 1).reshape(B, h * w, C)
-    assert ((y.float() - want.float()).abs() <= 1.1 * 2.0 ** -8 * taps + 2.0 ** -8 * want.float().abs()).all()
+    assert ((y.float() - want.float()).abs() <= 1.1 * 2.0 ** -7 * taps + 2.0 ** -7 * want.float().abs()).all()
     assert (y != want).float().mean() < 0.02
 
 

@@ -616,12 +616,13 @@ int launch_locality_gate(const void* o, const float* wt, void* y, int B, int H, 
 }
 
 // ---------------------------------------------------------------------------
-// Few grid rows: residual add, RMS norm and the depthwise 3x3 convolution behind it in one kernel, bf16, C = 24 LANES channels.  A
-// workgroup makes up to 14 cells of a grid row: the sums and norms of these and of the cells around them (LANES lanes a token; a row's norm is
-// made three times, out of the L2), the norms staged rounded in LDS between zeros, then the taps.  Latency bounds it: two launches
-// with a chain of loads each became one, every load of a workgroup under way at once, the taps' weights by way of LDS (fetched by the
-// octets of 72 that a thread needs, as above, they cost 1.8 us at C 192 and 3 at 384).  us, the two kernels / this: C 192 1 x 14 x 14 6.5
-// / 4.3, 2 x 48 x 48 9.7 / 5.8, 48 x 14 x 14 13.7 / 7.9; C 384 1 x 14 x 14 6.5 / 4.9, 32 x 14 x 14 13.8 / 9.2.
+// Residual add, RMS norm and the depthwise 3x3 convolution behind it in one kernel, bf16, C = 24 LANES channels.  A workgroup makes
+// up to 14 columns of the grid, of one row or of a band that it walks three rows at a time (WALK): the sums and norms of these cells
+// and of those around them (LANES lanes a token), staged rounded in LDS between zeros, three rows or the five that three rows of taps
+// reach; then the taps.  One row is bound by latency (two launches with a chain of loads each became one; the taps' weights come by
+// way of LDS: fetched by the octets of 72 that a thread needs, as above, they cost 1.8 us at C 192 and 3 at 384), the walk by the
+// vector pipe: 115 registers leave C 384 one workgroup a CU (80 registers for two spill 35: 46 -> 61 us), its next rows are fetched
+// during the taps.  C 384, 256 x 14 x 14: 37.6 us = 4.1 TB/s of the two inputs and two outputs; the two kernels 46.4.
 // ---------------------------------------------------------------------------
 constexpr int kNormStencilCols = 14;  // with the two beside them in three rows: 48 tokens
 
@@ -629,18 +630,19 @@ struct NormStencilArgs {
   const uint16_t *x, *residual;  // [B, h*w, C]; no residual: null
   const float *norm, *wt, *bias; // [C], [C, 9], [C] or null
   uint16_t *sum, *y;             // [B, h*w, C]; sum may be null
-  int h, w, cols, silu;
+  int h, w, rows, cols, silu;  // rows and columns of a workgroup
   float eps;
 };
-template <int LANES>  // all the tokens at a time; then four columns of channel pairs
+template <int LANES, bool WALK>  // three rows of tokens at a time; then four columns of channel pairs
 __global__ __launch_bounds__(48 * LANES) void norm_stencil_kernel(NormStencilArgs a) {
-  constexpr int NV = 3, C = 8 * NV * LANES, kThreads = 48 * LANES, kPairs = C / 2, kCols = kThreads / kPairs;
+  constexpr int NV = 3, C = 8 * NV * LANES, kThreads = 48 * LANES, kPairs = C / 2, kCols = kThreads / kPairs, kRing = WALK ? 5 : 3;
   extern __shared__ __align__(16) char smem[];
-  uint16_t* tile = reinterpret_cast<uint16_t*>(smem);  // [3 * (columns + 2)][C]
-  const int img = blockIdx.x / a.h, row = blockIdx.x - img * a.h;
+  uint16_t* tile = reinterpret_cast<uint16_t*>(smem);  // [kRing rows][columns + 2][C]
+  const int bands = (a.h + a.rows - 1) / a.rows, img = blockIdx.x / bands, row0 = (blockIdx.x - img * bands) * a.rows;
+  const int rows = WALK ? min(a.rows, a.h - row0) : 1, steps = WALK ? (rows + 4) / 3 : 1;
   const int c0 = blockIdx.y * a.cols, cols = min(a.cols, a.w - c0), pw = cols + 2;
   const size_t image = (size_t)img * a.h * a.w * C;
-  float* wts = reinterpret_cast<float*>(smem + 6 * (kNormStencilCols + 2) * C);  // [C][9]
+  float* wts = reinterpret_cast<float*>(smem + 2 * kRing * (kNormStencilCols + 2) * C);  // [C][9]
   const int pair = threadIdx.x % kPairs, col = threadIdx.x / kPairs;
   constexpr int kWLoads = (C * 9 / 4 + kThreads - 1) / kThreads;
   f32x4_t wraw[kWLoads];
@@ -650,89 +652,140 @@ __global__ __launch_bounds__(48 * LANES) void norm_stencil_kernel(NormStencilArg
     if (at < C * 9 / 4) wraw[i] = *reinterpret_cast<const f32x4_t*>(a.wt + 4 * at);
   }
   const float b0 = a.bias ? a.bias[2 * pair] : 0.f, b1 = a.bias ? a.bias[2 * pair + 1] : 0.f;
-  const int sub = threadIdx.x % LANES;
-  const int t = threadIdx.x / LANES;
-  if (t < 3 * pw) {  // padded cell (pr, pc) is grid cell (row - 1 + pr, c0 + pc - 1)
-    const int pr = t / pw, r = row - 1 + pr, pc = t - pr * pw, c = c0 + pc - 1;
-    const bool in = r >= 0 && r < a.h && c >= 0 && c < a.w;
-    const size_t at = in ? image + (size_t)(r * a.w + c) * C : 0;
-    Raw8<uint16_t> x[NV], res[NV];
+  // padded cell (p, pc) of the band is grid cell (row0 - 1 + p, c0 + pc - 1); step k brings rows 3k .. 3k + 2
+  const int sub = threadIdx.x % LANES, t = threadIdx.x / LANES, pr = t / pw, pc = t - pr * pw, c = c0 + pc - 1;
+  const bool own = t < 3 * pw;
+  Raw8<uint16_t> x[NV], res[NV];
+  const auto inside = [&](int p) { return own && p <= rows + 1 && row0 - 1 + p >= 0 && row0 - 1 + p < a.h && c >= 0 && c < a.w; };
+  const auto fetch = [&](int p) {
+    const bool in = inside(p);
+    const size_t at = in ? image + (size_t)((row0 - 1 + p) * a.w + c) * C : 0;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
       x[i].zero(), res[i].zero();
       if (in) x[i].load(a.x + at + 8 * (sub + LANES * i));
       if (in && a.residual) res[i].load(a.residual + at + 8 * (sub + LANES * i));
     }
-    float s[NV][8], ss = 0.f;
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      float b[8];
-      x[i].unpack(s[i]);
-      res[i].unpack(b);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {  // the rounded sum
-        res[i].a[j] = pack_bf16x2(s[i][2 * j] + b[2 * j], s[i][2 * j + 1] + b[2 * j + 1]);
-      }
-      res[i].unpack(s[i]);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) ss = __builtin_fmaf(s[i][j], s[i][j], ss);
-    }
-#pragma unroll
-    for (int d = 1; d < LANES; d <<= 1) ss += __shfl_xor(ss, d);
-    const float rstd = 1.0f / sqrtf(ss / (float)C + a.eps);
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int o = 8 * (sub + LANES * i);
-      const f32x4_t wa = *reinterpret_cast<const f32x4_t*>(a.norm + o), wb = *reinterpret_cast<const f32x4_t*>(a.norm + o + 4);
-      u32x4_t n;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float p = j < 2 ? wa[2 * j] : wb[2 * j - 4], q = j < 2 ? wa[2 * j + 1] : wb[2 * j - 3];
-        n[j] = in ? pack_bf16x2(s[i][2 * j] * rstd * p, s[i][2 * j + 1] * rstd * q) : 0u;
-      }
-      *reinterpret_cast<u32x4_t*>(tile + t * C + o) = n;
-      if (in && pr == 1 && pc >= 1 && pc <= cols && a.sum) res[i].store(a.sum + at + o);
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < kWLoads; ++i) {
-    const int at = (int)threadIdx.x + i * kThreads;
-    if (at < C * 9 / 4) *reinterpret_cast<f32x4_t*>(wts + 4 * at) = wraw[i];
-  }
-  __syncthreads();
+  };
+  fetch(pr);
   float wreg[18];
+  for (int k = 0; k < steps; ++k) {
+    if (own) {
+      const int p = 3 * k + pr;
+      const bool in = inside(p);
+      float s[NV][8], ss = 0.f;
 #pragma unroll
-  for (int i = 0; i < 9; ++i) wreg[2 * i] = wts[pair * 18 + 2 * i], wreg[2 * i + 1] = wts[pair * 18 + 2 * i + 1];
-  for (int c = col; c < cols; c += kCols) {
-    const uint16_t* p = tile + c * C + pair * 2;  // padded cell of tap (-1, -1)
-    float lo = b0, hi = b1;
+      for (int i = 0; i < NV; ++i) {
+        float b[8];
+        x[i].unpack(s[i]);
+        res[i].unpack(b);
 #pragma unroll
-    for (int di = 0; di < 3; ++di)
+        for (int j = 0; j < 4; ++j) res[i].a[j] = pack_bf16x2(s[i][2 * j] + b[2 * j], s[i][2 * j + 1] + b[2 * j + 1]);  // the rounded sum
+        if (a.sum && in && p >= 1 && p <= rows && pc >= 1 && pc <= cols)
+          res[i].store(a.sum + image + (size_t)((row0 - 1 + p) * a.w + c) * C + 8 * (sub + LANES * i));
+        res[i].unpack(s[i]);
 #pragma unroll
-      for (int dj = 0; dj < 3; ++dj) {
-        const uint32_t v = *reinterpret_cast<const uint32_t*>(p + (di * pw + dj) * C);
-        lo = __builtin_fmaf(bf16lo_to_f32(v), wreg[di * 3 + dj], lo), hi = __builtin_fmaf(bf16hi_to_f32(v), wreg[9 + di * 3 + dj], hi);
+        for (int j = 0; j < 8; ++j) ss = __builtin_fmaf(s[i][j], s[i][j], ss);
       }
-    if (a.silu) lo = lo * sigmoidf_(lo), hi = hi * sigmoidf_(hi);
-    *reinterpret_cast<uint32_t*>(a.y + image + (size_t)(row * a.w + c0 + c) * C + pair * 2) = pack_bf16x2(lo, hi);
+#pragma unroll
+      for (int d = 1; d < LANES; d <<= 1) ss += __shfl_xor(ss, d);
+      const float rstd = 1.0f / sqrtf(ss / (float)C + a.eps);
+      uint16_t* const cell = tile + ((p % kRing) * pw + pc) * C;
+#pragma unroll
+      for (int i = 0; i < NV; ++i) {
+        const int o = 8 * (sub + LANES * i);
+        const f32x4_t wa = *reinterpret_cast<const f32x4_t*>(a.norm + o), wb = *reinterpret_cast<const f32x4_t*>(a.norm + o + 4);
+        u32x4_t n;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float f = j < 2 ? wa[2 * j] : wb[2 * j - 4], g = j < 2 ? wa[2 * j + 1] : wb[2 * j - 3];
+          n[j] = in ? pack_bf16x2(s[i][2 * j] * rstd * f, s[i][2 * j + 1] * rstd * g) : 0u;
+        }
+        *reinterpret_cast<u32x4_t*>(cell + o) = n;
+      }
+    }
+    if (k == 0) {
+#pragma unroll
+      for (int i = 0; i < kWLoads; ++i) {
+        const int at = (int)threadIdx.x + i * kThreads;
+        if (at < C * 9 / 4) *reinterpret_cast<f32x4_t*>(wts + 4 * at) = wraw[i];
+      }
+    }
+    if (WALK && k + 1 < steps) fetch(3 * k + 3 + pr);
+    __syncthreads();
+    if (k == 0) {
+#pragma unroll
+      for (int i = 0; i < 9; ++i) wreg[2 * i] = wts[pair * 18 + 2 * i], wreg[2 * i + 1] = wts[pair * 18 + 2 * i + 1];
+    }
+    // rows 3k - 2 .. 3k of the band, of the five (one of the three) rows in LDS
+    constexpr int kOut = WALK ? 3 : 1;
+    const int first = WALK ? 3 * k - 2 : 0;
+    const uint16_t* taps[kOut + 2];
+#pragma unroll
+    for (int i = 0; i < kOut + 2; ++i) taps[i] = tile + ((first + kRing + i) % kRing) * pw * C + pair * 2;
+    for (int cc = col; cc < cols; cc += kCols) {
+      float lo[kOut], hi[kOut];
+#pragma unroll
+      for (int i = 0; i < kOut; ++i) lo[i] = b0, hi[i] = b1;
+#pragma unroll
+      for (int i = 0; i < kOut + 2; ++i)
+#pragma unroll
+        for (int dj = 0; dj < 3; ++dj) {
+          const uint32_t v = *reinterpret_cast<const uint32_t*>(taps[i] + (cc + dj) * C);
+#pragma unroll
+          for (int o = 0; o < kOut; ++o) {
+            if (i - o < 0 || i - o > 2) continue;
+            lo[o] = __builtin_fmaf(bf16lo_to_f32(v), wreg[(i - o) * 3 + dj], lo[o]);
+            hi[o] = __builtin_fmaf(bf16hi_to_f32(v), wreg[9 + (i - o) * 3 + dj], hi[o]);
+          }
+        }
+#pragma unroll
+      for (int o = 0; o < kOut; ++o) {
+        if (WALK && (first + o < 0 || first + o >= rows)) continue;
+        if (a.silu) lo[o] = lo[o] * sigmoidf_(lo[o]), hi[o] = hi[o] * sigmoidf_(hi[o]);
+        *reinterpret_cast<uint32_t*>(a.y + image + (size_t)((row0 + first + o) * a.w + c0 + cc) * C + pair * 2) = pack_bf16x2(lo[o], hi[o]);
+      }
+    }
+    if (WALK && k + 1 < steps) __syncthreads();
   }
 }
 
-bool norm_dwconv3x3_supported(int B, int h, int w, int C) {
-  const int parts = (w - 1) / kNormStencilCols + 1;
-  // Up to 1024 workgroups of 384 channels.  Past that the cells around a workgroup's, read and normed three times, cost what the launch
-  // saves: C 192 128 x 14 x 14 21.3 / 18.4 us, 256 x 14 x 14 30.8 / 30.4; C 384 64 x 14 x 14 19.5 / 17.8, 96 x 14 x 14 25.1 / 24.6, 128 x 14 x 14 27.8 / 30.0.
-  return (C == 192 || C == 384) && parts <= 65535 && (long long)B * h * w <= 0x7fffffff && (long long)B * h * parts <= 1024 * 384 / C;
+// Rows of the grid for a workgroup, 0: the two kernels are quicker.  One row costs 3 us and 0.015 for each workgroup of 384 channels (the
+// rows around are read and normed three times), a walk 5 us for every step of a round (two workgroups to a CU, one at C 384) and for
+// the round's start, the two kernels 10.5 us and 0.77 for 1000 cells of 384 channels.  us, the two kernels / one row / 4 / 7 / 14 rows:
+//   C 192 64 x 14 x 14 15.2 / 8.9 / 10.5 / 13.6 / 23.7, 128 images 21.9 / 17.1 / 14.5 / 14.9 / 25.0, 256 31.5 / 28.6 / 32.4 / 21.6 / 27.5,
+//   512 52.4 / 51.0 / 53.5 / 45.6 / 38.6; C 384 32 x 14 x 14 14.1 / 9.0 / 12.4 / 17.1 / 30.5, 64 images 19.9 / 17.1 / 14.0 / 17.5 / 30.1,
+//   128 28.5 / 29.0 / 26.9 / 20.9 / 32.0, 256 46.4 / 51.5 / 50.1 / 39.3 / 37.6, 512 91 / 97 / 100 / 82 / 79.
+// Rounds that are half empty leave it to the two kernels.
+static int norm_stencil_rows(int B, int h, int w, int C) {
+  if ((C != 192 && C != 384) || h > 1024 || w > 1024 || (long long)B * h * w > 0x7fffffff) return 0;
+  const long long columns = (long long)B * ((w - 1) / kNormStencilCols + 1), slots = C == 192 ? 512 : 256;
+  const double two = 0.95 * (10.5 + 2e-6 * C * B * h * w);
+  double least = 3 + 4e-5 * C * columns * h;
+  int best = 1;
+  for (int rows = 4; rows < h + 3; rows += 3) {
+    const double us = 5.0 * ((columns * ((h + rows - 1) / rows) + slots - 1) / slots * ((std::min(rows, h) + 4) / 3 + 1));
+    if (us < least) best = rows, least = us;
+  }
+  return least <= two ? best : 0;
 }
+bool norm_dwconv3x3_supported(int B, int h, int w, int C) { return norm_stencil_rows(B, h, w, C) > 0; }
 int launch_norm_dwconv3x3(const void* x, const void* residual, const float* norm, const float* wt, const float* bias, void* sum, void* y,
                           int B, int h, int w, int C, float eps, int silu, hipStream_t stream) {
-  if (!norm_dwconv3x3_supported(B, h, w, C)) return -95;
+  const int rows = norm_stencil_rows(B, h, w, C);
+  if (rows == 0) return -95;
   const int parts = (w - 1) / kNormStencilCols + 1, cols = (w + parts - 1) / parts;
-  const NormStencilArgs a{(const uint16_t*)x, (const uint16_t*)residual, norm, wt, bias, (uint16_t*)sum, (uint16_t*)y, h, w, cols, silu, eps};
-  const size_t lds = (6 * (kNormStencilCols + 2) + 36) * (size_t)C;
-  const dim3 grid(B * h, (w + cols - 1) / cols);
-  if (C == 192) hipLaunchKernelGGL(norm_stencil_kernel<8>, grid, dim3(2 * C), lds, stream, a);
-  else hipLaunchKernelGGL(norm_stencil_kernel<16>, grid, dim3(2 * C), lds, stream, a);
+  const NormStencilArgs a{(const uint16_t*)x, (const uint16_t*)residual, norm, wt, bias, (uint16_t*)sum, (uint16_t*)y, h, w, rows, cols, silu, eps};
+  const bool walk = rows > 1;
+  const size_t lds = (2 * (walk ? 5 : 3) * (kNormStencilCols + 2) + 36) * (size_t)C;
+  const dim3 grid(B * ((h + rows - 1) / rows), (w + cols - 1) / cols);
+  auto kernel = C == 192 ? (walk ? norm_stencil_kernel<8, true> : norm_stencil_kernel<8, false>)
+                         : (walk ? norm_stencil_kernel<16, true> : norm_stencil_kernel<16, false>);
+  if (walk && C == 384) {
+    static bool done[64] = {};
+    if (!allow_lds(reinterpret_cast<const void*>(kernel), lds, done)) return -5;
+  }
+  hipLaunchKernelGGL(kernel, grid, dim3(2 * C), lds, stream, a);
   return hipGetLastError() == hipSuccess ? 0 : -5;
 }
 
