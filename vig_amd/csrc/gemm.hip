@@ -274,6 +274,114 @@ __global__ __launch_bounds__(256) void gemm_norm_pair_kernel(NormPairArgs a) {
 }
 
 // ---------------------------------------------------------------------------
+// Few rows: the mixer's epilogue (both head norms, the sigmoid blend, as in blend_linear_kernel) and o_proj in one kernel, K = N = 64 NV.
+// One workgroup per 32 x 32 tile of the result: for a few hundred tokens the kernel that makes whole rows fills a handful of CUs, each
+// with all the weights to fetch; here a CU has a sixth or a twelfth of them, and the blend is made once a column tile.
+// ---------------------------------------------------------------------------
+struct BlendFewArgs {
+  const uint16_t *o, *loc, *glin;  // [B, H, L, 64]; [M, K]; rows of pitch ldg
+  const float *wg, *wl;            // 64 each
+  const uint16_t* w;               // [K, K]
+  uint16_t* y;                     // [M, K]
+  long long ldg;
+  int M, L, silu_out;
+  float eps;
+};
+template <int NV>
+__global__ __launch_bounds__(256) void gemm_blend_kernel(BlendFewArgs a) {
+  constexpr int K = 64 * NV, NW = 4, kStages = K / kStageK, kMine = (kStages + NW - 1) / NW, kX = 2048 * kStages;
+  constexpr int kLds = kX + NW * kMine * 2048, kPart = NW * 32 * 36 * 4;
+  __shared__ __align__(16) char smem[kLds > kPart ? kLds : kPart];
+  const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int m0 = blockIdx.y * 32, n0 = blockIdx.x * 32;
+  // ---- the weights of this wave's stages (wave, wave + 4, ..), all of them under way at once ----
+  const uint32_t w0 = lds_offset(smem) + kX + wave * (kMine * 2048);
+#pragma unroll
+  for (int at = 0; at < kMine; ++at) {
+    const int s = wave + NW * at;
+    if (s < kStages) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int row = 16 * i + (lane >> 2), unit = (lane & 3) ^ ((row >> 2) & 3);
+        load_to_lds16(a.w + (size_t)(n0 + row) * K + 8 * unit + s * kStageK, w0 + at * 2048 + 1024 * i);
+      }
+    }
+  }
+  // ---- the blend of 8 rows a wave: a head is eight lanes' ----
+  {
+    const int row = 8 * wave + (lane >> 3), sub = lane & 7, m = min(m0 + row, a.M - 1);
+    const unsigned b = (unsigned)m / (unsigned)a.L, l = (unsigned)m - b * (unsigned)a.L;
+    const uint16_t* const o = a.o + ((size_t)b * NV * a.L + l) * 64 + 8 * sub;
+    Raw8<uint16_t> ro8[NV], rl8[NV], rg8[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      ro8[i].load(o + (size_t)i * a.L * 64);
+      rl8[i].load(a.loc + (size_t)m * K + 64 * i + 8 * sub);
+      rg8[i].load(a.glin + (size_t)m * a.ldg + 64 * i + 8 * sub);
+    }
+    float wg[8], wl[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) wg[j] = a.wg[8 * sub + j], wl[j] = a.wl[8 * sub + j];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      float fo[8], fl[8], fg[8], e[8], so = 0.f, sl = 0.f;
+      ro8[i].unpack(fo);
+      rl8[i].unpack(fl);
+      rg8[i].unpack(fg);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) so += fo[j] * fo[j], sl += fl[j] * fl[j];
+#pragma unroll
+      for (int d = 1; d < 8; d <<= 1) so += __shfl_xor(so, d), sl += __shfl_xor(sl, d);
+      const float ro = rsqrtf(so * (1.0f / 64.0f) + a.eps), rl = rsqrtf(sl * (1.0f / 64.0f) + a.eps);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float sg = sigmoidf_(fg[j]);
+        e[j] = fo[j] * ro * wg[j] * sg + fl[j] * rl * wl[j] * (1.f - sg);
+      }
+      if (a.silu_out) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) e[j] = e[j] * sigmoidf_(e[j]);
+      }
+      u32x4_t y;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) y[j] = pack_bf16x2(e[2 * j], e[2 * j + 1]);
+      const int oct = sub + 8 * i;
+      *reinterpret_cast<u32x4_t*>(smem + (oct >> 2) * 2048 + row * 64 + 16 * ((oct & 3) ^ ((row >> 2) & 3))) = y;
+    }
+  }
+  wait_vmem<0>();
+  __syncthreads();
+  f32x16_t acc = f32x16_t{0.f};
+#pragma unroll
+  for (int at = 0; at < kMine; ++at) {
+    const int s = wave + NW * at;
+    if (s < kStages) {
+      const char* wbuf = smem + kX + wave * (kMine * 2048) + at * 2048;
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const int off = r * 64 + 16 * ((2 * k + h) ^ ((r >> 2) & 3));
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const bf16x8_t*>(wbuf + off),
+                                                      *reinterpret_cast<const bf16x8_t*>(smem + s * 2048 + off), acc, 0, 0, 0);
+      }
+    }
+  }
+  // accumulator register 4g+m of lane (r, h) is channel 8g+4h+m of token r
+  __syncthreads();
+  float(*part)[32][36] = reinterpret_cast<float(*)[32][36]>(smem);
+#pragma unroll
+  for (int g = 0; g < 4; ++g)
+    *reinterpret_cast<f32x4_t*>(&part[wave][r][8 * g + 4 * h]) = f32x4_t{acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]};
+  __syncthreads();
+  const int row = threadIdx.x >> 3, c = (threadIdx.x & 7) * 4;
+  f32x4_t sum = *reinterpret_cast<const f32x4_t*>(&part[0][row][c]);
+#pragma unroll
+  for (int k = 1; k < NW; ++k) sum += *reinterpret_cast<const f32x4_t*>(&part[k][row][c]);
+  if (m0 + row < a.M)
+    *reinterpret_cast<u32x2_t*>(a.y + (size_t)(m0 + row) * K + n0 + c) = u32x2_t{pack_bf16x2(sum[0], sum[1]), pack_bf16x2(sum[2], sum[3])};
+}
+
+// ---------------------------------------------------------------------------
 // Many rows: tiles of 64 MI x 64 NI by four waves of 32 MI x 32 NI each, operands through kBuffers LDS stages of 32
 // contraction elements (64-byte row pieces, loaded directly to LDS; the 16-byte units of a piece are swapped by a quarter of the row
 // number: the sixteen lanes served together read four rows that start in each bank quarter, and their units differ).
@@ -612,6 +720,20 @@ int launch_norm_swiglu(const void* x, const void* residual, const float* norm, c
   const dim3 grid(I / 32, (unsigned)((T + 31) / 32));
   if (K == 192) hipLaunchKernelGGL(gemm_norm_pair_kernel<3>, grid, dim3(256), 0, stream, a);
   else hipLaunchKernelGGL(gemm_norm_pair_kernel<6>, grid, dim3(256), 0, stream, a);
+  return hipGetLastError() == hipSuccess ? 0 : -5;
+}
+
+// The mixer's epilogue and o_proj of few rows (checked by launch_blend_linear), while there is a tile for a CU.  us, whole rows a
+// workgroup / this: C 192 196 rows 4.65 / 3.47, 1176 4.72 / 3.66, 1568 (294 tiles) 4.73 / 4.40, 2548 4.79 / 4.72; C 384 196 rows
+// 7.40 / 5.17, 392 7.44 / 5.29, 784 (300 tiles) 7.48 / 7.09, 1176 7.54 / 7.41.
+bool few_blend_linear(long long T, int C) { return (C == 192 || C == 384) && (T + 31) / 32 * (C / 32) <= 256; }
+int launch_few_blend_linear(const void* o, const void* loc, const void* glin, const float* w_g, const float* w_l, const void* W, void* out,
+                            long long T, int L, int C, long long ldg, float eps, int silu_out, hipStream_t stream) {
+  const BlendFewArgs a{(const uint16_t*)o, (const uint16_t*)loc, (const uint16_t*)glin, w_g, w_l, (const uint16_t*)W, (uint16_t*)out,
+                       ldg, (int)T, L, silu_out, eps};
+  const dim3 grid(C / 32, (unsigned)((T + 31) / 32));
+  if (C == 192) hipLaunchKernelGGL(gemm_blend_kernel<3>, grid, dim3(256), 0, stream, a);
+  else hipLaunchKernelGGL(gemm_blend_kernel<6>, grid, dim3(256), 0, stream, a);
   return hipGetLastError() == hipSuccess ? 0 : -5;
 }
 

@@ -606,9 +606,10 @@ int launch_blend_linear(const void* o, const void* loc, const void* glin, const 
   if (!blend_linear_supported(H, Dv, C) || B <= 0 || L <= 0 || (long long)B * L > 0x7fffffffLL - 64 || ldg % 8 != 0 ||
       ldg < C)
     return -95;
+  const long long T = (long long)B * L;
+  if (!kept && few_blend_linear(T, C)) return launch_few_blend_linear(o, loc, glin, w_g, w_l, W, out, T, L, C, ldg, eps, silu_out, stream);
   const int num_cu = cu_count();
   if (!num_cu) return -5;
-  const long long T = (long long)B * L;
   // twelve waves with one weight tile each (three per SIMD at 168 registers) at the wider size, six at the narrower
   if (kept)
     return C == 384 ? launch_blend_linear_t<24, 12, 1, true>(o, loc, glin, w_g, w_l, W, out, kept, T, L, H, ldg, eps, silu_out, num_cu, stream)
