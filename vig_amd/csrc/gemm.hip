@@ -158,11 +158,11 @@ __global__ __launch_bounds__(64 * NW) void gemm_few_kernel(GemmArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// Few rows: residual add, RMS norm and the SwiGLU layer behind it in one kernel, K = 64 NV.  A workgroup's 32 rows are whole rows of the
-// contraction, so it makes their sums and norms itself (eight lanes a row; every column tile again, out of the L2, the first one
+// Few rows: residual add, RMS norm and the SwiGLU layer behind it in one kernel, K = 48 NW.  A workgroup's 32 rows are whole rows of the
+// contraction, so it makes their sums and norms itself (2 NW lanes a row; every column tile again, out of the L2, the first one
 // stores the sums) while its weights arrive; a launch costs more than that.  us, norm and layer / this, rows x K -> I:
-// 1 x 192 -> 512 4.4 / 3.4, 196 x 192 -> 512 5.1 / 3.6, 392 x 192 -> 512 5.1 / 3.8, 1 x 384 -> 1024 4.8 / 4.6, 256 x 384 -> 1024
-// 5.6 / 5.3; other widths, and more rows than 256 workgroups take, keep the two.
+// 1 x 192 -> 512 4.5 / 3.2, 196 x 192 -> 512 5.0 / 3.4, 392 x 192 -> 512 5.1 / 3.6, 1 x 384 -> 1024 4.7 / 3.7, 256 x 384 -> 1024
+// 5.7 / 4.4 (four waves 5.3: six octets of a row to a lane); other widths, and more rows than 256 workgroups take, keep the two.
 // ---------------------------------------------------------------------------
 struct NormPairArgs {
   const uint16_t *x, *residual, *w;  // rows [M, K], [M, K]; weights [2 N, K], gate rows first
@@ -171,35 +171,37 @@ struct NormPairArgs {
   int M, N;
   float eps;
 };
-template <int NV>
-__global__ __launch_bounds__(256) void gemm_norm_pair_kernel(NormPairArgs a) {
-  constexpr int K = 64 * NV, NW = 4, kStages = K / kStageK, kMine = (kStages + NW - 1) / NW, kX = 2048 * kStages;
-  __shared__ __align__(16) char smem[kX + NW * kMine * 4096 > 36864 ? kX + NW * kMine * 4096 : 36864];
+template <int NW>
+__global__ __launch_bounds__(64 * NW) void gemm_norm_pair_kernel(NormPairArgs a) {
+  constexpr int K = 48 * NW, NV = 3, kLanes = 2 * NW, kStages = K / kStageK, kX = 2048 * kStages;
+  constexpr int kMats = NW == 4 ? 2 : 1, kMine = (kStages + 3) / 4, kMat = kMats * 2048;  // eight waves: four for the gate rows, four for the others
+  __shared__ __align__(16) char smem[kX + NW * kMine * kMat > 36864 ? kX + NW * kMine * kMat : 36864];
   const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int m0 = blockIdx.y * 32, n0 = blockIdx.x * 32;
-  // ---- the weights of this wave's stages (wave, wave + 4, ..), all of them under way at once ----
-  const uint32_t w0 = lds_offset(smem) + kX + wave * (kMine * 4096);
+  const int part0 = wave & 3, mat0 = wave >> 2;
+  // ---- the weights of this wave's stages (part0, part0 + 4, ..), all of them under way at once ----
+  const uint32_t w0 = lds_offset(smem) + kX + wave * (kMine * kMat);
 #pragma unroll
   for (int at = 0; at < kMine; ++at) {
-    const int s = wave + NW * at;
+    const int s = part0 + 4 * at;
     if (s < kStages) {
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
         const int row = 16 * i + (lane >> 2), unit = (lane & 3) ^ ((row >> 2) & 3);
-        const uint16_t* wp = a.w + (size_t)min(n0 + row, a.N - 1) * K + 8 * unit + s * kStageK;
-        load_to_lds16(wp, w0 + at * 4096 + 1024 * i);
-        load_to_lds16(wp + (size_t)a.N * K, w0 + at * 4096 + 2048 + 1024 * i);
+        const uint16_t* wp = a.w + (size_t)(min(n0 + row, a.N - 1) + mat0 * a.N) * K + 8 * unit + s * kStageK;
+        load_to_lds16(wp, w0 + at * kMat + 1024 * i);
+        if constexpr (kMats == 2) load_to_lds16(wp + (size_t)a.N * K, w0 + at * kMat + 2048 + 1024 * i);
       }
     }
   }
-  // ---- sums and norms of 8 rows a wave ----
+  // ---- sums and norms, 8 or 4 rows a wave ----
   {
-    const int row = 8 * wave + (lane >> 3), sub = lane & 7, m = min(m0 + row, a.M - 1);
+    const int row = threadIdx.x / kLanes, sub = threadIdx.x % kLanes, m = min(m0 + row, a.M - 1);
     const size_t base = (size_t)m * K;
     Raw8<uint16_t> x[NV], res[NV];
 #pragma unroll
-    for (int i = 0; i < NV; ++i) x[i].load(a.x + base + 8 * (sub + 8 * i)), res[i].load(a.residual + base + 8 * (sub + 8 * i));
+    for (int i = 0; i < NV; ++i) x[i].load(a.x + base + 8 * (sub + kLanes * i)), res[i].load(a.residual + base + 8 * (sub + kLanes * i));
     float s[NV][8], ss = 0.f;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
@@ -210,12 +212,12 @@ __global__ __launch_bounds__(256) void gemm_norm_pair_kernel(NormPairArgs a) {
       for (int j = 0; j < 8; ++j) s[i][j] += b[j], ss = __builtin_fmaf(s[i][j], s[i][j], ss);
     }
 #pragma unroll
-    for (int d = 1; d < 8; d <<= 1) ss += __shfl_xor(ss, d);
+    for (int d = 1; d < kLanes; d <<= 1) ss += __shfl_xor(ss, d);
     const float rstd = 1.0f / sqrtf(ss / (float)K + a.eps);
     const bool keep = blockIdx.x == 0 && m0 + row < a.M;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
-      const int o = sub + 8 * i;
+      const int o = sub + kLanes * i;
       const f32x4_t wa = *reinterpret_cast<const f32x4_t*>(a.norm + 8 * o), wb = *reinterpret_cast<const f32x4_t*>(a.norm + 8 * o + 4);
       u32x4_t y, sum;
 #pragma unroll
@@ -230,18 +232,20 @@ __global__ __launch_bounds__(256) void gemm_norm_pair_kernel(NormPairArgs a) {
   }
   wait_vmem<0>();
   __syncthreads();
-  f32x16_t acc[2] = {f32x16_t{0.f}, f32x16_t{0.f}};
+  f32x16_t acc[kMats];
+#pragma unroll
+  for (int j = 0; j < kMats; ++j) acc[j] = f32x16_t{0.f};
 #pragma unroll
   for (int at = 0; at < kMine; ++at) {
-    const int s = wave + NW * at;
+    const int s = part0 + 4 * at;
     if (s < kStages) {
-      const char* wbuf = smem + kX + wave * (kMine * 4096) + at * 4096;
+      const char* wbuf = smem + kX + wave * (kMine * kMat) + at * kMat;
 #pragma unroll
       for (int k = 0; k < 2; ++k) {
         const int off = r * 64 + 16 * ((2 * k + h) ^ ((r >> 2) & 3));
         const bf16x8_t xf = *reinterpret_cast<const bf16x8_t*>(smem + s * 2048 + off);
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < kMats; ++j)
           acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const bf16x8_t*>(wbuf + 2048 * j + off), xf, acc[j], 0, 0, 0);
       }
     }
@@ -250,18 +254,19 @@ __global__ __launch_bounds__(256) void gemm_norm_pair_kernel(NormPairArgs a) {
   __syncthreads();
   float(*part)[2][32][36] = reinterpret_cast<float(*)[2][32][36]>(smem);
 #pragma unroll
-  for (int j = 0; j < 2; ++j)
+  for (int j = 0; j < kMats; ++j)
 #pragma unroll
     for (int g = 0; g < 4; ++g)
-      *reinterpret_cast<f32x4_t*>(&part[wave][j][r][8 * g + 4 * h]) = f32x4_t{acc[j][4 * g], acc[j][4 * g + 1], acc[j][4 * g + 2], acc[j][4 * g + 3]};
+      *reinterpret_cast<f32x4_t*>(&part[part0][mat0 + j][r][8 * g + 4 * h]) = f32x4_t{acc[j][4 * g], acc[j][4 * g + 1], acc[j][4 * g + 2], acc[j][4 * g + 3]};
   __syncthreads();
+  if (threadIdx.x >= 256) return;
   const int row = threadIdx.x >> 3, c = (threadIdx.x & 7) * 4;
   f32x4_t sum[2];
 #pragma unroll
   for (int m = 0; m < 2; ++m) {
     sum[m] = *reinterpret_cast<const f32x4_t*>(&part[0][m][row][c]);
 #pragma unroll
-    for (int k = 1; k < NW; ++k) sum[m] += *reinterpret_cast<const f32x4_t*>(&part[k][m][row][c]);
+    for (int k = 1; k < 4; ++k) sum[m] += *reinterpret_cast<const f32x4_t*>(&part[k][m][row][c]);
   }
   if (m0 + row < a.M && n0 + c < a.N) {
 #pragma unroll
@@ -274,7 +279,7 @@ __global__ __launch_bounds__(256) void gemm_norm_pair_kernel(NormPairArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// Few rows: the mixer's epilogue (both head norms, the sigmoid blend, as in blend_linear_kernel) and o_proj in one kernel, K = N = 64 NV.
+// Few rows: the mixer's epilogue (both head norms, the sigmoid blend, as in blend_linear_kernel) and o_proj in one kernel, K = N = 48 NW.
 // One workgroup per 32 x 32 tile of the result: for a few hundred tokens the kernel that makes whole rows fills a handful of CUs, each
 // with all the weights to fetch; here a CU has a sixth or a twelfth of them, and the blend is made once a column tile.
 // ---------------------------------------------------------------------------
@@ -287,9 +292,9 @@ struct BlendFewArgs {
   int M, L, silu_out;
   float eps;
 };
-template <int NV>
-__global__ __launch_bounds__(256) void gemm_blend_kernel(BlendFewArgs a) {
-  constexpr int K = 64 * NV, NW = 4, kStages = K / kStageK, kMine = (kStages + NW - 1) / NW, kX = 2048 * kStages;
+template <int NW>
+__global__ __launch_bounds__(64 * NW) void gemm_blend_kernel(BlendFewArgs a) {
+  constexpr int K = 48 * NW, NV = 3, H = K / 64, kLanes = 2 * NW, kStages = K / kStageK, kMine = (kStages + NW - 1) / NW, kX = 2048 * kStages;
   constexpr int kLds = kX + NW * kMine * 2048, kPart = NW * 32 * 36 * 4;
   __shared__ __align__(16) char smem[kLds > kPart ? kLds : kPart];
   const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
@@ -308,17 +313,18 @@ __global__ __launch_bounds__(256) void gemm_blend_kernel(BlendFewArgs a) {
       }
     }
   }
-  // ---- the blend of 8 rows a wave: a head is eight lanes' ----
+  // ---- the blend, 8 or 4 rows a wave: a head is eight lanes' ----
   {
-    const int row = 8 * wave + (lane >> 3), sub = lane & 7, m = min(m0 + row, a.M - 1);
+    const int row = threadIdx.x / kLanes, oct0 = threadIdx.x % kLanes, sub = lane & 7, m = min(m0 + row, a.M - 1);
     const unsigned b = (unsigned)m / (unsigned)a.L, l = (unsigned)m - b * (unsigned)a.L;
-    const uint16_t* const o = a.o + ((size_t)b * NV * a.L + l) * 64 + 8 * sub;
+    const uint16_t* const o = a.o + ((size_t)b * H * a.L + l) * 64 + 8 * sub;
     Raw8<uint16_t> ro8[NV], rl8[NV], rg8[NV];
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
-      ro8[i].load(o + (size_t)i * a.L * 64);
-      rl8[i].load(a.loc + (size_t)m * K + 64 * i + 8 * sub);
-      rg8[i].load(a.glin + (size_t)m * a.ldg + 64 * i + 8 * sub);
+      const int oct = oct0 + kLanes * i;
+      ro8[i].load(o + (size_t)(oct >> 3) * a.L * 64);
+      rl8[i].load(a.loc + (size_t)m * K + 8 * oct);
+      rg8[i].load(a.glin + (size_t)m * a.ldg + 8 * oct);
     }
     float wg[8], wl[8];
 #pragma unroll
@@ -346,7 +352,7 @@ __global__ __launch_bounds__(256) void gemm_blend_kernel(BlendFewArgs a) {
       u32x4_t y;
 #pragma unroll
       for (int j = 0; j < 4; ++j) y[j] = pack_bf16x2(e[2 * j], e[2 * j + 1]);
-      const int oct = sub + 8 * i;
+      const int oct = oct0 + kLanes * i;
       *reinterpret_cast<u32x4_t*>(smem + (oct >> 2) * 2048 + row * 64 + 16 * ((oct & 3) ^ ((row >> 2) & 3))) = y;
     }
   }
@@ -373,6 +379,7 @@ __global__ __launch_bounds__(256) void gemm_blend_kernel(BlendFewArgs a) {
   for (int g = 0; g < 4; ++g)
     *reinterpret_cast<f32x4_t*>(&part[wave][r][8 * g + 4 * h]) = f32x4_t{acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]};
   __syncthreads();
+  if (threadIdx.x >= 256) return;
   const int row = threadIdx.x >> 3, c = (threadIdx.x & 7) * 4;
   f32x4_t sum = *reinterpret_cast<const f32x4_t*>(&part[0][row][c]);
 #pragma unroll
@@ -718,22 +725,22 @@ int launch_norm_swiglu(const void* x, const void* residual, const float* norm, c
   if (!norm_swiglu_supported(T, K, I)) return -95;
   const NormPairArgs a{(const uint16_t*)x, (const uint16_t*)residual, (const uint16_t*)w, norm, (uint16_t*)sum, (uint16_t*)y, (int)T, I, eps};
   const dim3 grid(I / 32, (unsigned)((T + 31) / 32));
-  if (K == 192) hipLaunchKernelGGL(gemm_norm_pair_kernel<3>, grid, dim3(256), 0, stream, a);
-  else hipLaunchKernelGGL(gemm_norm_pair_kernel<6>, grid, dim3(256), 0, stream, a);
+  if (K == 192) hipLaunchKernelGGL(gemm_norm_pair_kernel<4>, grid, dim3(256), 0, stream, a);
+  else hipLaunchKernelGGL(gemm_norm_pair_kernel<8>, grid, dim3(512), 0, stream, a);
   return hipGetLastError() == hipSuccess ? 0 : -5;
 }
 
 // The mixer's epilogue and o_proj of few rows (checked by launch_blend_linear), while there is a tile for a CU.  us, whole rows a
 // workgroup / this: C 192 196 rows 4.65 / 3.47, 1176 4.72 / 3.66, 1568 (294 tiles) 4.73 / 4.40, 2548 4.79 / 4.72; C 384 196 rows
-// 7.40 / 5.17, 392 7.44 / 5.29, 784 (300 tiles) 7.48 / 7.09, 1176 7.54 / 7.41.
+// 7.44 / 4.73 (four waves 5.17), 588 7.51 / 4.92, 784 (300 tiles, four waves) 7.48 / 7.09, 1176 7.54 / 7.41.
 bool few_blend_linear(long long T, int C) { return (C == 192 || C == 384) && (T + 31) / 32 * (C / 32) <= 256; }
 int launch_few_blend_linear(const void* o, const void* loc, const void* glin, const float* w_g, const float* w_l, const void* W, void* out,
                             long long T, int L, int C, long long ldg, float eps, int silu_out, hipStream_t stream) {
   const BlendFewArgs a{(const uint16_t*)o, (const uint16_t*)loc, (const uint16_t*)glin, w_g, w_l, (const uint16_t*)W, (uint16_t*)out,
                        ldg, (int)T, L, silu_out, eps};
   const dim3 grid(C / 32, (unsigned)((T + 31) / 32));
-  if (C == 192) hipLaunchKernelGGL(gemm_blend_kernel<3>, grid, dim3(256), 0, stream, a);
-  else hipLaunchKernelGGL(gemm_blend_kernel<6>, grid, dim3(256), 0, stream, a);
+  if (C == 192) hipLaunchKernelGGL(gemm_blend_kernel<4>, grid, dim3(256), 0, stream, a);
+  else hipLaunchKernelGGL(gemm_blend_kernel<8>, grid, dim3(512), 0, stream, a);
   return hipGetLastError() == hipSuccess ? 0 : -5;
 }
 
