@@ -29,12 +29,7 @@ def test_against_two_kernels(B, h, w, C, full):
     assert lib.vig_rmsnorm_fwd(p(x), p(res), p(nw), p(normed), sum2.data_ptr() if full else None, B * h * w, C, 1e-5, int(full), 1, st) == _lib.VIG_OK
     assert lib.vig_dwconv3x3_fwd(p(normed), p(wt), p(bias), p(want), B, h, w, C, int(full), 1, st) == _lib.VIG_OK
     assert not full or torch.equal(total, sum2)
-    # a norm whose last fp32 bit differs moves a normed value by an ulp of bf16 now and then: 2^-7 of it at most, so of the taps' sum of
-    # magnitudes (SiLU's slope is below 1.1); the two results are rounded by half an ulp each
-    grid = normed.float().abs().view(B, h, w, C).permute(0, 3, 1, 2)
-    taps = torch.nn.functional.conv2d(grid, wt.abs().view(C, 1, 3, 3), padding=1, groups=C).permute(0, 2, 3, 1).reshape(B, h * w, C)
-    assert ((y.float() - want.float()).abs() <= 1.1 * 2.0 ** -7 * taps + 2.0 ** -7 * want.float().abs()).all()
-    assert (y != want).float().mean() < 0.02
+    assert torch.equal(y, want)  # the same sums in the same order
 
 
 def test_refused():

@@ -25,16 +25,7 @@ def test_against_two_kernels(rows, K, I):
     assert lib.vig_rmsnorm_fwd(x.data_ptr(), res.data_ptr(), nw.data_ptr(), normed.data_ptr(), sum2.data_ptr(), rows, K, 1e-5, 0, 1, st) == _lib.VIG_OK
     assert lib.vig_linear_swiglu_fwd(normed.data_ptr(), w.data_ptr(), want.data_ptr(), rows, K, I, 1, st) == _lib.VIG_OK
     assert torch.equal(total, sum2)
-    # a norm that differs in its last fp32 bit moves a value by an ulp of bf16 now and then, a pre-activation and the output likewise
-    s = x.double() + res.double()
-    n = s * torch.rsqrt(s.pow(2).mean(-1, keepdim=True) + 1e-5) * nw.double()
-    g, u = (n @ w.double().t()).chunk(2, 1)
-    exact = torch.nn.functional.silu(g) * u
-    spread = (n.abs() @ w.double().abs().t()).chunk(2, 1)
-    # inputs rounded to bf16 once (errors add up as the root of the terms: 8 sigma of 2^-9 relative), factors and product once each
-    bound = 8 * 2.0 ** -9 * K ** -0.5 * (spread[0] * u.abs() + spread[1] * g.abs()) + 2.0 ** -6 * exact.abs() + 2.0 ** -7 * (g.abs() + u.abs()) * 2.0 ** -2
-    assert ((y.double() - exact).abs() <= bound).all()
-    assert (y.double() - want.double()).abs().max() <= 2.0 ** -6 * want.double().abs().max() and (y != want).float().mean() < 0.02
+    assert torch.equal(y, want)  # the same sums in the same order
 
 
 def test_refused():

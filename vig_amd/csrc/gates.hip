@@ -673,7 +673,7 @@ __global__ __launch_bounds__(48 * LANES) void norm_stencil_kernel(NormStencilArg
     if (own) {
       const int p = 3 * k + pr;
       const bool in = inside(p);
-      float s[NV][8], ss = 0.f;
+      float s[NV][8], sq[NV] = {};
 #pragma unroll
       for (int i = 0; i < NV; ++i) {
         float b[8];
@@ -685,10 +685,11 @@ __global__ __launch_bounds__(48 * LANES) void norm_stencil_kernel(NormStencilArg
           res[i].store(a.sum + image + (size_t)((row0 - 1 + p) * a.w + c) * C + 8 * (sub + LANES * i));
         res[i].unpack(s[i]);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) ss = __builtin_fmaf(s[i][j], s[i][j], ss);
+        for (int j = 0; j < 8; ++j) sq[i] = __builtin_fmaf(s[i][j], s[i][j], sq[i]);
       }
+      float ss = (sq[0] + sq[2]) + sq[1];  // the order of rmsnorm_kernel's wave, so its bits
 #pragma unroll
-      for (int d = 1; d < LANES; d <<= 1) ss += __shfl_xor(ss, d);
+      for (int d = LANES / 2; d > 0; d >>= 1) ss += __shfl_xor(ss, d);
       const float rstd = 1.0f / sqrtf(ss / (float)C + a.eps);
       uint16_t* const cell = tile + ((p % kRing) * pw + pc) * C;
 #pragma unroll

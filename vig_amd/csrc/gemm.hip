@@ -202,17 +202,18 @@ __global__ __launch_bounds__(64 * NW) void gemm_norm_pair_kernel(NormPairArgs a)
     Raw8<uint16_t> x[NV], res[NV];
 #pragma unroll
     for (int i = 0; i < NV; ++i) x[i].load(a.x + base + 8 * (sub + kLanes * i)), res[i].load(a.residual + base + 8 * (sub + kLanes * i));
-    float s[NV][8], ss = 0.f;
+    float s[NV][8], sq[NV] = {};
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
       float b[8];
       x[i].unpack(s[i]);
       res[i].unpack(b);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) s[i][j] += b[j], ss = __builtin_fmaf(s[i][j], s[i][j], ss);
+      for (int j = 0; j < 8; ++j) s[i][j] += b[j], sq[i] = __builtin_fmaf(s[i][j], s[i][j], sq[i]);
     }
+    float ss = (sq[0] + sq[2]) + sq[1];  // the order of rmsnorm_kernel's wave, so its bits
 #pragma unroll
-    for (int d = 1; d < kLanes; d <<= 1) ss += __shfl_xor(ss, d);
+    for (int d = kLanes / 2; d > 0; d >>= 1) ss += __shfl_xor(ss, d);
     const float rstd = 1.0f / sqrtf(ss / (float)K + a.eps);
     const bool keep = blockIdx.x == 0 && m0 + row < a.M;
 #pragma unroll
