@@ -288,7 +288,7 @@ struct BlendFewArgs {
   const uint16_t *o, *loc, *glin;  // [B, H, L, 64]; [M, K]; rows of pitch ldg
   const float *wg, *wl;            // 64 each
   const uint16_t* w;               // [K, K]
-  uint16_t* y;                     // [M, K]
+  uint16_t *y, *kept;              // [M, K]; kept: the blended rows for a backward, or null
   long long ldg;
   int M, L, silu_out;
   float eps;
@@ -355,6 +355,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_blend_kernel(BlendFewArgs a) {
       for (int j = 0; j < 4; ++j) y[j] = pack_bf16x2(e[2 * j], e[2 * j + 1]);
       const int oct = oct0 + kLanes * i;
       *reinterpret_cast<u32x4_t*>(smem + (oct >> 2) * 2048 + row * 64 + 16 * ((oct & 3) ^ ((row >> 2) & 3))) = y;
+      if (a.kept && blockIdx.x == 0 && m0 + row < a.M) *reinterpret_cast<u32x4_t*>(a.kept + (size_t)m * K + 8 * oct) = y;
     }
   }
   wait_vmem<0>();
@@ -736,9 +737,9 @@ int launch_norm_swiglu(const void* x, const void* residual, const float* norm, c
 // 7.44 / 4.73 (four waves 5.17), 588 7.51 / 4.92, 784 (300 tiles, four waves) 7.48 / 7.09, 1176 7.54 / 7.41.
 bool few_blend_linear(long long T, int C) { return (C == 192 || C == 384) && (T + 31) / 32 * (C / 32) <= 256; }
 int launch_few_blend_linear(const void* o, const void* loc, const void* glin, const float* w_g, const float* w_l, const void* W, void* out,
-                            long long T, int L, int C, long long ldg, float eps, int silu_out, hipStream_t stream) {
+                            void* kept, long long T, int L, int C, long long ldg, float eps, int silu_out, hipStream_t stream) {
   const BlendFewArgs a{(const uint16_t*)o, (const uint16_t*)loc, (const uint16_t*)glin, w_g, w_l, (const uint16_t*)W, (uint16_t*)out,
-                       ldg, (int)T, L, silu_out, eps};
+                       (uint16_t*)kept, ldg, (int)T, L, silu_out, eps};
   const dim3 grid(C / 32, (unsigned)((T + 31) / 32));
   if (C == 192) hipLaunchKernelGGL(gemm_blend_kernel<4>, grid, dim3(256), 0, stream, a);
   else hipLaunchKernelGGL(gemm_blend_kernel<8>, grid, dim3(512), 0, stream, a);

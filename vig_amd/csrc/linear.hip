@@ -607,7 +607,7 @@ int launch_blend_linear(const void* o, const void* loc, const void* glin, const 
       ldg < C)
     return -95;
   const long long T = (long long)B * L;
-  if (!kept && few_blend_linear(T, C)) return launch_few_blend_linear(o, loc, glin, w_g, w_l, W, out, T, L, C, ldg, eps, silu_out, stream);
+  if (few_blend_linear(T, C)) return launch_few_blend_linear(o, loc, glin, w_g, w_l, W, out, kept, T, L, C, ldg, eps, silu_out, stream);
   const int num_cu = cu_count();
   if (!num_cu) return -5;
   // twelve waves with one weight tile each (three per SIMD at 168 registers) at the wider size, six at the narrower
