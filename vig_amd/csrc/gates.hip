@@ -620,9 +620,9 @@ int launch_locality_gate(const void* o, const float* wt, void* y, int B, int H, 
 // up to 14 columns of the grid, of one row or of a band that it walks three rows at a time (WALK): the sums and norms of these cells
 // and of those around them (LANES lanes a token), staged rounded in LDS between zeros, three rows or the five that three rows of taps
 // reach; then the taps.  One row is bound by latency (two launches with a chain of loads each became one; the taps' weights come by
-// way of LDS: fetched by the octets of 72 that a thread needs, as above, they cost 1.8 us at C 192 and 3 at 384), the walk by the
-// vector pipe: 115 registers leave C 384 one workgroup a CU (80 registers for two spill 35: 46 -> 61 us), its next rows are fetched
-// during the taps.  C 384, 256 x 14 x 14: 37.6 us = 4.1 TB/s of the two inputs and two outputs; the two kernels 46.4.
+// way of LDS: fetched by the octets of 72 that a thread needs, as above, they cost 1.8 us at C 192 and 3 at 384), the walk by
+// what one workgroup a CU has under way (vector pipe 46 %): 115 registers leave C 384 no second one (80 for two spill 35: 46 -> 61 us);
+// its next rows are fetched during the taps.  C 384, 256 x 14 x 14: 37.6 us = 4.1 TB/s of the two inputs and two outputs; the two kernels 46.4.
 // ---------------------------------------------------------------------------
 constexpr int kNormStencilCols = 14;  // with the two beside them in three rows: 48 tokens
 
