@@ -627,7 +627,7 @@ int vig_norm_dwconv3x3_fwd(const void* x, const void* residual, const float* nor
  * Residual add, RMS norm and the SwiGLU layer behind it in one kernel, bf16, packed rows:
  *   sum [rows, K] = x + residual (stored rounded; the norm is of the sum in fp32),  y [rows, I] = SwiGLU of rms(sum) * norm_weight . weight^T,
  * weight [2*I, K] with the gate rows first: what vig_rmsnorm_fwd (round_sum 0) and vig_linear_swiglu_fwd give one after the other.
- * K = 192 or 384, I % 32 == 0 and few rows (vig_norm_swiglu_preferred), else VIG_ENOTSUP.  sum is neither x nor residual.
+ * K = 192 or 384, I % 32 == 0 and few rows (vig_norm_swiglu_preferred), else VIG_ENOTSUP.  No output may be an input.
  *
  * Replaces: classification/models/vig.py:486-496,604-606 (prenorm add, mlp_norm, gate_proj, up_proj and their product).
  */

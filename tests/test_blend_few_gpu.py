@@ -38,3 +38,16 @@ def test_against_fp64(B, L, H, silu, pitch):
     many = 1 + 6000 // (B * L)  # copies of the batch, past the row count of the kernel of few rows
     ref = run(o.repeat(many, 1, 1, 1), loc.repeat(many, 1, 1), wide.repeat(many, 1, 1)[..., pitch:], many * B)[:B]
     assert (got != ref).float().mean() < 0.02 and (got.float() - ref.float()).abs().max() <= 2.0 ** -7 * ref.float().abs().max()
+
+
+def test_result_over_an_input():
+    gen = torch.Generator().manual_seed(1)
+    o, loc, g = torch.randn(1, 3, 196, 64, generator=gen).bfloat16().cuda(), *(torch.randn(1, 196, 192, generator=gen).bfloat16().cuda() for _ in range(2))
+    w, n = torch.randn(192, 192, generator=gen).bfloat16().cuda(), torch.ones(64, device="cuda")
+    lib, st = _lib.load(), torch.cuda.current_stream().cuda_stream
+    call = lambda out, x, y: lib.vig_locality_blend_linear_fwd(o.data_ptr(), x.data_ptr(), y.data_ptr(), n.data_ptr(), n.data_ptr(), w.data_ptr(),  # noqa: E731
+                                                               out.data_ptr(), 1, 3, 196, 64, 192, 192, 1e-5, 0, 1, st)
+    want, over_loc, over_g = torch.empty_like(loc), loc.clone(), g.clone()
+    assert call(want, loc, g) == call(over_loc, over_loc, g) == call(over_g, loc, over_g) == _lib.VIG_OK
+    for got in (over_loc, over_g):  # the kernel of whole rows: sums in another order, an ulp of bf16 now and then
+        assert (got != want).float().mean() < 0.02 and (got.float() - want.float()).abs().max() <= 2.0 ** -7 * want.float().abs().max()

@@ -29,11 +29,12 @@ def test_against_two_kernels(rows, K, I):
 
 
 def test_refused():
-    t = torch.zeros(4096, 384, dtype=torch.bfloat16, device="cuda")
+    x, res, w, out, total = (torch.zeros(2048, 384, dtype=torch.bfloat16, device="cuda") for _ in range(5))
     f, lib, st = torch.ones(384, device="cuda"), _lib.load(), torch.cuda.current_stream().cuda_stream
-    call = lambda x, s, rows, K, I: lib.vig_norm_swiglu_fwd(x, t.data_ptr(), f.data_ptr(), t.data_ptr(), s, t.data_ptr(), rows, K, I, 1e-5, st)  # noqa: E731
-    other = torch.zeros_like(t)
-    assert call(other.data_ptr(), other.data_ptr(), 32, 384, 32) == _lib.VIG_EINVAL  # the sum over its input
-    out = torch.zeros_like(t)
-    assert call(other.data_ptr(), out.data_ptr(), 4096, 384, 1024) == _lib.VIG_ENOTSUP  # many rows
-    assert call(other.data_ptr(), out.data_ptr(), 32, 256, 32) == _lib.VIG_ENOTSUP  # another width
+    call = lambda s, y, rows, K, I: lib.vig_norm_swiglu_fwd(x.data_ptr(), res.data_ptr(), f.data_ptr(), w.data_ptr(), s.data_ptr(), y.data_ptr(),  # noqa: E731
+                                                            rows, K, I, 1e-5, st)
+    assert call(total, out, 32, 384, 32) == _lib.VIG_OK
+    for s, y in ((x, out), (res, out), (total, x), (total, res), (total, total)):  # an output over an input or the other output
+        assert call(s, y, 32, 384, 32) == _lib.VIG_EINVAL
+    assert call(total, out, 2048, 384, 1024) == _lib.VIG_ENOTSUP  # many rows
+    assert call(total, out, 32, 256, 32) == _lib.VIG_ENOTSUP  # another width

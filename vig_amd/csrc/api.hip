@@ -508,7 +508,8 @@ int vig_norm_swiglu_preferred(long long rows, int K, int I) { return vig::norm_s
 
 int vig_norm_swiglu_fwd(const void* x, const void* residual, const float* norm_weight, const void* weight, void* sum, void* y,
                         long long rows, int K, int I, float eps, void* stream) {
-  if (!x || !residual || !norm_weight || !weight || !sum || !y || rows <= 0 || K <= 0 || I <= 0 || sum == x || sum == residual)
+  if (!x || !residual || !norm_weight || !weight || !sum || !y || rows <= 0 || K <= 0 || I <= 0 || sum == x || sum == residual ||
+      y == x || y == residual || y == sum)
     return VIG_EINVAL;
   if (!aligned16(x, residual, norm_weight, weight, sum, y)) return VIG_EINVAL;
   if (!vig::norm_swiglu_supported(rows, K, I)) return VIG_ENOTSUP;

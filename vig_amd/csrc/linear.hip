@@ -607,7 +607,13 @@ int launch_blend_linear(const void* o, const void* loc, const void* glin, const 
       ldg < C)
     return -95;
   const long long T = (long long)B * L;
-  if (few_blend_linear(T, C)) return launch_few_blend_linear(o, loc, glin, w_g, w_l, W, out, kept, T, L, C, ldg, eps, silu_out, stream);
+  // (there a row's inputs are read by several workgroups: a result over an input, which whole rows a workgroup allow, stays with those)
+  const auto over = [&](const void* p, const void* q, long long bytes) {
+    const uintptr_t a = (uintptr_t)p, b = (uintptr_t)q;
+    return p && a < b + (uintptr_t)bytes && b < a + (uintptr_t)(2 * T * C);
+  };
+  const auto apart = [&](const void* p) { return !over(p, o, 2 * T * C) && !over(p, loc, 2 * T * C) && !over(p, glin, 2 * ((T - 1) * ldg + C)); };
+  if (few_blend_linear(T, C) && apart(out) && apart(kept)) return launch_few_blend_linear(o, loc, glin, w_g, w_l, W, out, kept, T, L, C, ldg, eps, silu_out, stream);
   const int num_cu = cu_count();
   if (!num_cu) return -5;
   // twelve waves with one weight tile each (three per SIMD at 168 registers) at the wider size, six at the narrower
