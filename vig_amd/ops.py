@@ -571,8 +571,9 @@ def gla_bidir_locality_gate(q, k, v, g_fwd, g_bwd, weight: torch.Tensor, hw, sca
                             out_scale: float = 1.0) -> torch.Tensor:
     """locality_gate(gla_bidir_forward(q, k, v, g_fwd, g_bwd), weight, hw), bit for bit.
 
-    Shapes the one-kernel form is built for (bf16, Dk in {32,64}, Dv=64, L=h*w<=256) never write the ungated
-    output to memory; every other shape makes the two calls.  Inference only.
+    Shapes the one-kernel form is built for (bf16, Dk in {32,64}, Dv=64, L=h*w up to 512 at Dk 32 and 416 at Dk 64, a
+    grid whose padded rows fit LDS) never write the ungated output to memory; every other shape makes the two calls (and
+    without the native module every L past 256).  Inference only.
     """
     h, w = hw
     calls = _ext.calls()
