@@ -130,7 +130,9 @@ def emulate_tiles(q, k, v, gf, gb, tile=32):
     tile-local cumulative gates G (fp32), total T; a = f16(exp(G)), b = f16(exp(-G)), d = f16(exp(T));
     q^ = f16(q a), k' = f16(k b), k^ = f16(k' d); own tile: P = mask(k' q^T), rounded to fp16 per direction and the two
     directions added in fp16; another tile j walked outwards: q^ <- f16(q^ d_m) for every tile m passed, P = k^_j q^T
-    rounded once to fp16; O += P V with fp32 accumulation (chunk_util.py:37-78 with the anchors per tile)."""
+    rounded once to fp16; O += P V with fp32 accumulation (chunk_util.py:37-78 with the anchors per tile).
+    More than eight tiles: k^ = f16(k f16(exp(T - G))); q^ stays as it is, k^_j <- f16(k^_j f16(exp(the totals of the tiles
+    passed)))."""
     N, L, Dk = q.shape
     Dv = v.shape[-1]
     s = np.float32(Dk ** -0.5)
@@ -139,6 +141,7 @@ def emulate_tiles(q, k, v, gf, gb, tile=32):
     sl = [slice(i * tile, min(L, (i + 1) * tile)) for i in range(nt)]
     acc = np.zeros((N, L, Dv), np.float32)
     diag = [np.zeros((N, sl[i].stop - sl[i].start, sl[i].stop - sl[i].start), np.float32) for i in range(nt)]
+    many = nt > 8
     for direction in (0, 1):
         g = gf if direction == 0 else gb
         qh, kc, kh, d = [], [], [], []
@@ -155,19 +158,29 @@ def emulate_tiles(q, k, v, gf, gb, tile=32):
             qh.append(f16_round(q[:, sl[i]] * a16))
             kci = f16_round(k[:, sl[i]] * b16)
             kc.append(kci)
-            kh.append(f16_round(kci * d16))
-            d.append(d16)
+            if many:
+                kh.append(f16_round(k[:, sl[i]] * f16_round(np.exp(Tt - G))))
+                d.append(Tt)
+            else:
+                kh.append(f16_round(kci * d16))
+                d.append(d16)
         for i in range(nt):
             n = qh[i].shape[1]
             tri = np.tril(np.ones((n, n), np.float32)) if direction == 0 else np.triu(np.ones((n, n), np.float32))
             # own tile: P[i, j] over the pairs the direction keeps; the two directions meet in fp16
             diag[i] = f16_round(diag[i] + f16_round(_mm(qh[i], T_(kc[i])) * tri))
-            qw = qh[i]
+            qw, between = qh[i], np.float32(0.0)
             others = range(i - 1, -1, -1) if direction == 0 else range(i + 1, nt)
             for step, j in enumerate(others):
+                kj = kh[j]
                 if step > 0:
-                    qw = f16_round(qw * d[j + 1 if direction == 0 else j - 1])
-                acc[:, sl[i]] += _mm(f16_round(_mm(qw, T_(kh[j]))), v[:, sl[j]])
+                    last = d[j + 1 if direction == 0 else j - 1]
+                    if many:
+                        between = between + last
+                        kj = f16_round(kj * f16_round(np.exp(between)))
+                    else:
+                        qw = f16_round(qw * last)
+                acc[:, sl[i]] += _mm(f16_round(_mm(qw, T_(kj))), v[:, sl[j]])
     for i in range(nt):
         acc[:, sl[i]] += _mm(diag[i], v[:, sl[i]])
     return s * acc

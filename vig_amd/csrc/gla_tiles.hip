@@ -67,12 +67,20 @@ struct TileGeo {
   float inv_norm, clamp;
 };
 
+// Sequences of more tiles than this (MANY below): a far tile's q^ has picked up the decays of up to fifteen tiles, and a product
+// rounded to fp16 for each, by a rounded decay, would leave more error than segments linked by fp32 states do.  There k^ comes from
+// k at once and, on the walk, takes the decay of all tiles between, made from the fp32 totals: two roundings however far.
+// Error of the op in 1e-4 of its rms, output not yet rounded, segments / decays one by one in fp16 / this: 512 tokens, Dk 32, gate
+// logits around 0 4.72 / 4.76 / 4.51, around 5 5.55 / 7.27 / 4.75; 416, Dk 64 4.72 / 4.75 / 4.50, 5.80 / 6.89 / 4.70.  us, one by
+// one / this: 312 sequences of 512, Dk 32 33.9 / 36.6; 360 of 416, Dk 64 40.7 / 44.5.
+constexpr int kFewTiles = 8;
+
 // byte offsets of the workgroup's LDS areas
 template <int NG>
 struct TileLds {
   static constexpr int KB = NG * 1024;  // one k^ tile: NG units
   static constexpr int VB = 4096;       // one V tile: 4 units
-  int kf, kb, v, d, scratch, guard, total;
+  int kf, kb, v, d, scratch, scratch_b, guard, total;
   // gate_bytes: what the fused locality gate stages in the tile regions once they are dead (0: no gate)
   __host__ __device__ explicit TileLds(int NT, int gate_bytes = 0) {
     kf = 0;
@@ -81,7 +89,9 @@ struct TileLds {
     d = v + NT * VB;
     if (d < gate_bytes) d = gate_bytes;
     scratch = d + 2 * NT * 128;  // per wave: 64 floats (tile totals on their way from one lane pair to a lane per channel)
-    guard = scratch + NT * 256;
+    // (the reverse direction's; more than kFewTiles: both stay, everybody reads them)
+    scratch_b = NT > kFewTiles ? scratch + NT * 256 : scratch;
+    guard = scratch_b + NT * 256;
     total = guard + NT * 16;
   }
 };
@@ -212,16 +222,24 @@ __device__ __forceinline__ void park_totals(f32x16_t& C, float* sc, int r, int h
   wave_lds_sync();
 }
 
+// place of sc[lane]'s channel in a table of decays (a lane half's 8 NG channels as it reads them)
+template <int NG>
+__device__ __forceinline__ int table_channel(int lane) {
+  return 8 * NG * (lane >> 5) + 8 * ((lane >> 2) & 3) + 2 * (lane & 3) + ((lane >> 4) & 1);
+}
+template <int NG>
+__device__ __forceinline__ bool has_table_channel(int lane) { return ((lane >> 2) & 3) < NG; }
+
 // Operands of one direction for this wave's tile, the publication of what other tiles need from it, and the diagonal
 // score tile (masked to the pairs the direction sees and rounded to fp16 pairs: the B operand of the value product).
 //   qh: q^ = q exp(G)      (B operand of every score product of this wave; kept)
 //   k^ = k exp(T - G)      (published to kreg unless null, piece by piece)
-//   D  = exp(T)            (published to dtab, fp16, channel order)
+//   D  = exp(T)            (published to dtab, fp16, channel order; MANY: T to sc instead)
 // fp16 form (GENERAL false): the diagonal tile uses k' = k exp(-G) against q^; returns (wave-uniform) whether some
 // channel's tile total is outside the form's range.
 // General form: inputs carry the power-of-two scales 2^-eq, 2^-ek; the diagonal tile uses the half-anchored pair
 // q~ = q exp(G - T/2), k~ = k exp(T/2 - G) as bf16 hi + lo, three MFMA terms per k-step.
-template <int NG, bool FWD, bool GENERAL, bool LOW>
+template <int NG, bool FWD, bool GENERAL, bool LOW, bool MANY>
 __device__ __forceinline__ bool prepare_direction(const uint32_t (&gD)[2][8], const LowRank& low, float inv_norm, float clamp,
                                                   int nvalid, const u32x4_t (&rawq)[NG],
                                                   const u32x4_t (&rawk)[NG], float* sc, _Float16* dtab, char* kreg,
@@ -241,11 +259,8 @@ __device__ __forceinline__ bool prepare_direction(const uint32_t (&gD)[2][8], co
   if (!GENERAL) wide = __builtin_amdgcn_ballot_w64(!(fabsf(tl) <= kTileRange)) != 0;
   else tl = fmaxf(tl, kExpFloor);
   const float dT = exp2_fast(tl);
-  if (GENERAL) sc[lane] = tl;
-  {
-    const int p = (lane >> 4) & 1, g = (lane >> 2) & 3, m = lane & 3;
-    if (g < NG) dtab[HC * (lane >> 5) + 8 * g + 2 * m + p] = (_Float16)dT;
-  }
+  if (GENERAL || MANY) sc[lane] = tl;
+  if (!MANY && has_table_channel<NG>(lane)) dtab[table_channel<NG>(lane)] = (_Float16)dT;
   wave_lds_sync();
   const float* mine = sc + 32 * (lane >> 5);
   const u32x4_t* dmine = reinterpret_cast<const u32x4_t*>(dtab + HC * (lane >> 5));  // this lane half's decays as fp16 pairs
@@ -256,7 +271,7 @@ __device__ __forceinline__ bool prepare_direction(const uint32_t (&gD)[2][8], co
   for (int g = 0; g < NG; ++g) {
     u32x4_t kh;
     f32x4_t d0, d1;
-    if (GENERAL) {
+    if (GENERAL || MANY) {
       d0 = *reinterpret_cast<const f32x4_t*>(mine + 4 * g);
       d1 = *reinterpret_cast<const f32x4_t*>(mine + 16 + 4 * g);
     }
@@ -264,7 +279,8 @@ __device__ __forceinline__ bool prepare_direction(const uint32_t (&gD)[2][8], co
       // rawq / rawk hold fp16 pairs here; the decay factors are rounded to fp16 and applied as packed products
       // (the diagonal tile's products wait until the loop is through: their 16 accumulators would otherwise sit
       // beside the cumulative gates and the raw rows, which are at their fullest in the first pieces)
-      const u32x4_t d16 = dmine[g];
+      u32x4_t d16;
+      if (!MANY) d16 = dmine[g];
 #pragma unroll
       for (int m = 0; m < 4; ++m) {
         const int c = 4 * g + m;
@@ -273,7 +289,7 @@ __device__ __forceinline__ bool prepare_direction(const uint32_t (&gD)[2][8], co
         const uint32_t b16 = pack_f16x2(exp2_fast(-x0), exp2_fast(-x1));
         qh[g][m] = mul_f16x2(rawq[g][m], a16);
         kc[g][m] = mul_f16x2(rawk[g][m], b16);
-        kh[m] = mul_f16x2(kc[g][m], d16[m]);
+        kh[m] = MANY ? mul_f16x2(rawk[g][m], pack_f16x2(exp2_fast(d0[m] - x0), exp2_fast(d1[m] - x1))) : mul_f16x2(kc[g][m], d16[m]);
       }
     } else {
       u32x4_t qhi, qlo, khi, klo;
@@ -425,6 +441,56 @@ __device__ __forceinline__ void walk_tiles_ahead(char* lds, const TileLds<NG>& l
     for (int g = 0; g < NG; ++g)
 #pragma unroll
       for (int m = 0; m < 4; ++m) qh[g][m] = mul_f16x2(qh[g][m], s < n ? d[g][m] : 0x3C003C00u);
+    apply_values(P, vf, O);
+  }
+}
+
+// The same for many tiles: a tile's k^ takes the decay of the tiles between it and the wave's own.  A lane adds up one channel's totals
+// and leaves the factor for the step after this one in the wave's own two pieces of the table of decays.
+template <int NG, bool FWD>
+__device__ __forceinline__ void walk_many_tiles(char* lds, const TileLds<NG>& lay, int ti, int NT, int lane, const u32x4_t (&qh)[NG],
+                                                f32x16_t (&O)[2]) {
+  constexpr int KB = TileLds<NG>::KB;
+  constexpr bool kAhead = NG == 2;  // (a tile's keys fetched while the tile before is at work)
+  const int n = FWD ? ti : NT - 1 - ti;
+  if (n == 0) return;
+  const int kbase = FWD ? lay.kf : lay.kb - KB;  // reverse regions start at tile 1
+  const auto load_k = [&](int j, u32x4_t (&kf)[NG]) {
+#pragma unroll
+    for (int g = 0; g < NG; ++g) kf[g] = *reinterpret_cast<const u32x4_t*>(unit_ptr(lds + kbase + j * KB, g, lane));
+  };
+  const float* totals = reinterpret_cast<const float*>(lds + (FWD ? lay.scratch : lay.scratch_b)) + lane;
+  char* factors = lds + lay.d + ti * 256;
+  const int mine = 2 * table_channel<NG>(lane);
+  const auto leave = [&](int slot, float decay) {
+    if (has_table_channel<NG>(lane)) *reinterpret_cast<_Float16*>(factors + 128 * slot + mine) = (_Float16)decay;
+    asm volatile("" ::: "memory");  // (a wave's LDS accesses stay in order)
+  };
+  float sum = 0.f;
+  u32x4_t kf[NG];
+  if (kAhead) load_k(FWD ? ti - 1 : ti + 1, kf);
+  leave(1, 1.0f);
+#pragma unroll 1
+  for (int s = 1; s <= n; ++s) {
+    const int j = FWD ? ti - s : ti + s;
+    char* vreg = lds + lay.v + j * TileLds<NG>::VB;
+    if (!kAhead) load_k(j, kf);
+    const float total = totals[64 * j];
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+      const u32x4_t d = *reinterpret_cast<const u32x4_t*>(factors + 128 * (s & 1) + 16 * NG * (lane >> 5) + 16 * g);
+#pragma unroll
+      for (int m = 0; m < 4; ++m) kf[g][m] = mul_f16x2(kf[g][m], d[m]);
+    }
+    u32x4_t vf[2][2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int pv = 0; pv < 2; ++pv) vf[t][pv] = *reinterpret_cast<const u32x4_t*>(unit_ptr(vreg, 2 * t + pv, lane));
+    const f32x16_t P = score_tile16<NG>(kf, qh);
+    sum += total;
+    leave(~s & 1, exp2_fast(sum));
+    if (kAhead) load_k(FWD ? max(j - 1, 0) : min(j + 1, NT - 1), kf);
     apply_values(P, vf, O);
   }
 }
@@ -657,14 +723,14 @@ static_assert(offsetof(TileKernArgs, geo) == 6 * sizeof(void*) && offsetof(TileK
                   offsetof(TileKernArgs, gate_w) == 48 + sizeof(TileGeo) + 8 && alignof(TileGeo) == 8,
               "TileKernArgs has to mirror the parameter list of gla_tile_kernel");
 
-template <int NG, bool BIDIR, bool PITCHED, bool GATE, bool CHAIN, bool LOW>
+template <int NG, bool BIDIR, bool PITCHED, bool GATE, bool CHAIN, bool LOW, bool MANY>
 __device__ void tile_pass_general(const TileKernArgs* ka_in);
 
 // Everything one wave does for its slab.  When some tile of the slab is outside the fp16 form's range (GENERAL false), every wave
 // of the workgroup, before anything is stored, runs the general form (ka: the kernel's argument block) and ends there: a call
 // that came back would keep the accumulators alive across it, and the compiler then kept sixteen of them in per-lane memory
 // throughout, walks included (long sequences at Dk 32, 144 of 784 tokens: this kernel 38.7 -> 23.5 us).
-template <int NG, bool BIDIR, bool PITCHED, bool GENERAL, bool GATE, bool CHAIN, bool LOW>
+template <int NG, bool BIDIR, bool PITCHED, bool GENERAL, bool GATE, bool CHAIN, bool LOW, bool MANY>
 __device__ __forceinline__ void tile_pass(const TileCtx& cx, const TileKernArgs* ka) {
   const int lane = cx.lane, r = lane & 31, h = lane >> 5;
   const int ti = cx.ti, NT = cx.NT;
@@ -672,6 +738,7 @@ __device__ __forceinline__ void tile_pass(const TileCtx& cx, const TileKernArgs*
   char* lds = cx.lds;
   char* vregion = lds + lay.v + ti * TileLds<NG>::VB;
   float* sc = reinterpret_cast<float*>(lds + lay.scratch + ti * 256);
+  float* sc_b = reinterpret_cast<float*>(lds + lay.scratch_b + ti * 256);
   float* guard = reinterpret_cast<float*>(lds + lay.guard);
   _Float16* dtab_f = reinterpret_cast<_Float16*>(lds + lay.d + ti * 128);
   _Float16* dtab_b = reinterpret_cast<_Float16*>(lds + lay.d + (NT + ti) * 128);
@@ -771,7 +838,7 @@ __device__ __forceinline__ void tile_pass(const TileCtx& cx, const TileKernArgs*
   u32x4_t p16[2];
   {
     char* kreg = ti < NT - 1 ? lds + lay.kf + ti * TileLds<NG>::KB : nullptr;
-    if (prepare_direction<NG, true, GENERAL, LOW>(gDf, low, cx.inv_norm, cx.clamp, cx.nvalid, rawq, rawk, sc, dtab_f, kreg, lane, eq, ek, qhf, p16)) veto = true;
+    if (prepare_direction<NG, true, GENERAL, LOW, MANY>(gDf, low, cx.inv_norm, cx.clamp, cx.nvalid, rawq, rawk, sc, dtab_f, kreg, lane, eq, ek, qhf, p16)) veto = true;
   }
   VIG_PHASE();
   if (BIDIR) {
@@ -791,7 +858,7 @@ __device__ __forceinline__ void tile_pass(const TileCtx& cx, const TileKernArgs*
     // (lane-derived constants of this direction are built here, not carried from the top of the kernel)
     int lane_b = lane;
     asm volatile("" : "+v"(lane_b));
-    if (prepare_direction<NG, false, GENERAL, LOW>(gDb, low, cx.inv_norm, cx.clamp, cx.nvalid, rawq, rawk, sc, dtab_b, kreg, lane_b, eq, ek, qhb, pb)) veto = true;
+    if (prepare_direction<NG, false, GENERAL, LOW, MANY>(gDb, low, cx.inv_norm, cx.clamp, cx.nvalid, rawq, rawk, MANY ? sc_b : sc, dtab_b, kreg, lane_b, eq, ek, qhb, pb)) veto = true;
     // (the two directions meet on the pairs j = i only: one more fp16 rounding there)
 #pragma unroll
     for (int t = 0; t < 2; ++t)
@@ -816,7 +883,7 @@ __device__ __forceinline__ void tile_pass(const TileCtx& cx, const TileKernArgs*
   if (!GENERAL) {
     const float mine = lane < NT ? guard[4 * lane] : 0.0f;
     if (__builtin_amdgcn_ballot_w64(mine != 0.0f) != 0) {
-      tile_pass_general<NG, BIDIR, PITCHED, GATE, CHAIN, LOW>(ka);
+      tile_pass_general<NG, BIDIR, PITCHED, GATE, CHAIN, LOW, MANY>(ka);
       __builtin_amdgcn_endpgm();
     }
   }
@@ -827,13 +894,15 @@ __device__ __forceinline__ void tile_pass(const TileCtx& cx, const TileKernArgs*
   int lane_w = lane;
   asm volatile("" : "+v"(lane_w));
   constexpr bool kAhead = NG == 2 && !CHAIN;
-  if constexpr (kAhead) walk_tiles_ahead<NG, true>(lds, lay, ti, NT, lane_w, qhf, O);
+  if constexpr (MANY) walk_many_tiles<NG, true>(lds, lay, ti, NT, lane_w, qhf, O);
+  else if constexpr (kAhead) walk_tiles_ahead<NG, true>(lds, lay, ti, NT, lane_w, qhf, O);
   else walk_tiles<NG, true>(lds, lay, ti, NT, lane_w, qhf, O);
   // (general form: the state's term joins accumulators that carry 2^-(eq + ek + ev); q^ carries 2^-eq itself)
   if (CHAIN)
     apply_state<NG, true>(cx.state_in, shift_f, lds + lay.d + 16 * NG * (lane_w >> 5), ti > 0, lane_w,
                           GENERAL ? -(ek + ev) : 0, qhf, O);
-  if constexpr (BIDIR && kAhead) walk_tiles_ahead<NG, false>(lds, lay, ti, NT, lane_w, qhb, O);
+  if constexpr (BIDIR && MANY) walk_many_tiles<NG, false>(lds, lay, ti, NT, lane_w, qhb, O);
+  else if constexpr (BIDIR && kAhead) walk_tiles_ahead<NG, false>(lds, lay, ti, NT, lane_w, qhb, O);
   else if constexpr (BIDIR) walk_tiles<NG, false>(lds, lay, ti, NT, lane_w, qhb, O);
   if (CHAIN && BIDIR)
     apply_state<NG, false>(cx.state_in + kGlaStateFloats, shift_b,
@@ -914,7 +983,7 @@ __device__ __forceinline__ TileCtx make_tile_ctx(const uint16_t* q, const uint16
 // the kernel's arguments from the argument block itself (ka: the kernel's own kernarg segment pointer; the builtin
 // yields null inside a called function): handed over as parameters, the geometry would need a copy in per-lane
 // memory, and the compiler writes that copy at the top of the kernel, for every wave, redo or not.
-template <int NG, bool BIDIR, bool PITCHED, bool GATE, bool CHAIN, bool LOW>
+template <int NG, bool BIDIR, bool PITCHED, bool GATE, bool CHAIN, bool LOW, bool MANY>
 __device__ __noinline__ void tile_pass_general(const TileKernArgs* ka_in) {
 #if defined(__HIP_DEVICE_COMPILE__)  // (the host pass has no constant address space to copy the geometry from)
   // (a called function gets its arguments in vector registers: back to scalars, or every argument read through the
@@ -929,13 +998,13 @@ __device__ __noinline__ void tile_pass_general(const TileKernArgs* ka_in) {
   const TileGeo geo = ka->geo;
   const TileCtx cx = make_tile_ctx<NG, BIDIR, PITCHED, GATE, CHAIN, LOW>(ka->q, ka->k, ka->v, ka->gf, ka->gb, ka->o, geo,
                                                                      ka->oscale, ka->gate_w, lds);
-  tile_pass<NG, BIDIR, PITCHED, true, GATE, CHAIN, LOW>(cx, nullptr);
+  tile_pass<NG, BIDIR, PITCHED, true, GATE, CHAIN, LOW, MANY>(cx, nullptr);
 #endif
 }
 
 }  // namespace
 
-template <int NG, bool BIDIR, bool PITCHED, bool GATE, bool CHAIN = false, bool LOW = false>
+template <int NG, bool BIDIR, bool PITCHED, bool GATE, bool CHAIN = false, bool LOW = false, bool MANY = false>
 __global__ __launch_bounds__(1024, 4) void gla_tile_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
                                                           const uint16_t* __restrict__ v,
                                                           const uint16_t* __restrict__ gf,
@@ -945,7 +1014,7 @@ __global__ __launch_bounds__(1024, 4) void gla_tile_kernel(const uint16_t* __res
   extern __shared__ __align__(16) char lds[];
   const TileKernArgs* ka = (const TileKernArgs*)__builtin_amdgcn_kernarg_segment_ptr();
   const TileCtx cx = make_tile_ctx<NG, BIDIR, PITCHED, GATE, CHAIN, LOW>(q, k, v, gf, gb, o, geo, oscale, gate_w, lds);
-  tile_pass<NG, BIDIR, PITCHED, false, GATE, CHAIN, LOW>(cx, ka);
+  tile_pass<NG, BIDIR, PITCHED, false, GATE, CHAIN, LOW, MANY>(cx, ka);
 }
 
 // The general form alone, for launches whose caller knows the gates to be strong: with 256 registers per wave (one
@@ -961,15 +1030,15 @@ __global__ __launch_bounds__(512, 2) void gla_tile_wide_kernel(const uint16_t* _
                                                                const float* __restrict__ gate_w) {
   extern __shared__ __align__(16) char lds[];
   const TileCtx cx = make_tile_ctx<NG, BIDIR, PITCHED, GATE, CHAIN, LOW>(q, k, v, gf, gb, o, geo, oscale, gate_w, lds);
-  tile_pass<NG, BIDIR, PITCHED, true, GATE, CHAIN, LOW>(cx, nullptr);
+  tile_pass<NG, BIDIR, PITCHED, true, GATE, CHAIN, LOW, false>(cx, nullptr);
 }
 
 constexpr int kTileMaxLds = 160 * 1024;
 
 // Whole sequences up to 13 tiles (Dk 64: 158 KB of LDS) or 16 (Dk 32: sixteen waves of 128 registers, all that a CU holds) go
 // through one workgroup: k, v and the gates are read once instead of twice, no states pass through memory, one launch instead
-// of three.  us, one workgroup / segments linked by states: Dk 32: 3 sequences of 257 10.4 / 19.6, 480 of 300 29 / 75, 312 of 512
-// 38 / 81; Dk 64: 3 of 257 13.7 / 22.7, 6 of 400 18.8 / 24.0, 480 of 300 40 / 96, 360 of 416 49 / 76.
+// of three.  us, one workgroup / segments linked by states: Dk 32: 3 sequences of 257 9.7 / 20.3, 480 of 300 27.7 / 75, 312 of 512
+// 36.6 / 81; Dk 64: 3 of 257 13.6 / 23.1, 6 of 400 19.2 / 25.2, 480 of 300 38.8 / 96, 360 of 416 44.5 / 76.
 // The general form's own kernel has twice the registers per wave and takes eight.
 int gla_slab_tokens(int Dk) { return Dk == 64 ? 416 : 512; }
 
@@ -993,13 +1062,16 @@ bool gla_tiles_supported(const GlaArgs& a) {
   return true;
 }
 
-template <int NG, bool BIDIR, bool PITCHED, bool GATE, bool CHAIN = false, bool LOW = false>
+template <int NG, bool BIDIR, bool PITCHED, bool GATE, bool CHAIN = false, bool LOW = false, bool MANY = false>
 static int launch_tiles_t(const GlaArgs& a, const TileGeo& geo, int dev) {
+  if constexpr (!MANY && !CHAIN)
+    if (geo.NT > kFewTiles) return launch_tiles_t<NG, BIDIR, PITCHED, GATE, CHAIN, LOW, true>(a, geo, dev);
   constexpr int kMaxDevices = 64;
+  constexpr bool kWide = !LOW && !MANY;  // (gates known to be strong: whole sequences of few tiles and segments)
   static bool attr_done_dev[kMaxDevices] = {};
-  const void* kf = reinterpret_cast<const void*>(gla_tile_kernel<NG, BIDIR, PITCHED, GATE, CHAIN, LOW>);
+  const void* kf = reinterpret_cast<const void*>(gla_tile_kernel<NG, BIDIR, PITCHED, GATE, CHAIN, LOW, MANY>);
   const void* kw = nullptr;
-  if constexpr (!LOW) kw = reinterpret_cast<const void*>(gla_tile_wide_kernel<NG, BIDIR, PITCHED, GATE, CHAIN, LOW>);
+  if constexpr (kWide) kw = reinterpret_cast<const void*>(gla_tile_wide_kernel<NG, BIDIR, PITCHED, GATE, CHAIN, LOW>);
   if (!attr_done_dev[dev]) {
     if (hipFuncSetAttribute(kf, hipFuncAttributeMaxDynamicSharedMemorySize, kTileMaxLds) != hipSuccess) return -5;
     if (kw && hipFuncSetAttribute(kw, hipFuncAttributeMaxDynamicSharedMemorySize, kTileMaxLds) != hipSuccess) return -5;
@@ -1007,8 +1079,8 @@ static int launch_tiles_t(const GlaArgs& a, const TileGeo& geo, int dev) {
   }
   const TileLds<NG> lay(geo.NT, GATE ? gate_stage_bytes(geo.gw, geo.gh) : 0);
   if (lay.total > kTileMaxLds) return -95;
-  auto kernel = gla_tile_kernel<NG, BIDIR, PITCHED, GATE, CHAIN, LOW>;
-  if constexpr (!LOW)
+  auto kernel = gla_tile_kernel<NG, BIDIR, PITCHED, GATE, CHAIN, LOW, MANY>;
+  if constexpr (kWide)
     if (geo.wide) kernel = gla_tile_wide_kernel<NG, BIDIR, PITCHED, GATE, CHAIN, LOW>;
   hipLaunchKernelGGL(kernel, dim3(a.B * a.H, CHAIN ? geo.nseg : 1), dim3(64 * geo.NT), lay.total, a.stream, (const uint16_t*)a.q,
                      (const uint16_t*)a.k, (const uint16_t*)a.v, (const uint16_t*)a.g_fwd, (const uint16_t*)a.g_bwd, (uint16_t*)a.o, geo,
