@@ -125,8 +125,9 @@ int vig_gla_slab_fwd(const void* q, const void* k, const void* v, const void* g_
 /*
  * The bidirectional op with q, k, v read in place and the gates made on the way, as vig_dirgate_lowrank_fwd makes them (same
  * roundings), instead of read: low [B, L, 16] (rows low_row_stride elements apart), up_w [2*H*Dk, 16], up_b [2*H*Dk], clamp_min NaN
- * for none; all bf16.  Dk 32, Dv 64, all three strides given (as for _strided); VIG_ENOTSUP for anything else.  Any length; past
- * vig_gla_slab_tokens(32) tokens the workspace (vig_gla_lowrank_fwd_workspace bytes) holds the states that link the segments.
+ * for none; all bf16.  Dk 32, Dv 64, all three strides given (as for _strided; token stride 0: that tensor is plain); VIG_ENOTSUP for
+ * anything else.  Any length; past vig_gla_slab_tokens(32) tokens the workspace (vig_gla_lowrank_fwd_workspace bytes) holds the states
+ * that link the segments, and 2*B*H > 65535 is refused with VIG_ENOTSUP.
  *
  * Replaces: classification/models/vig.py:401-435 (head split, gate up-projection, log-sigmoid, direction split, the op).
  */

@@ -1179,9 +1179,14 @@ static int launch_gla_mfma_t(const GlaArgs& a, int num_cu, int dev) {
 }
 
 // a sequence of any length with its gates made on the way (GlaArgs::low)
-int launch_gla_lowrank(const GlaArgs& a) {
-  if (gla_tiles_supported(a)) return launch_gla_tiles(a);
-  if (!gla_tiles_chain_supported(a)) return -95;
+int launch_gla_lowrank(const GlaArgs& given) {
+  if (gla_tiles_supported(given)) return launch_gla_tiles(given);
+  // (the scan puts sequence x direction on grid.y; the state pass reads with the strides before the last kernel looks at them)
+  if (!gla_tiles_chain_supported(given) || (long long)given.B * given.H * 2 > 65535) return -95;
+  long long sq[3], sk[3], sv[3];
+  if (const int rc = gla_strides(given, sq, sk, sv)) return rc;
+  GlaArgs a = given;
+  a.q_strides = sq, a.k_strides = sk, a.v_strides = sv;
   if (!a.workspace || a.workspace_bytes < gla_mfma_workspace(a.B, a.H, a.L, a.Dk, a.Dv)) return -28;
   const Geometry geo = make_geometry(a.B * a.H, a.L, true);
   float* ws = (float*)a.workspace;

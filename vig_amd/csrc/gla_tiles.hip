@@ -1088,14 +1088,14 @@ static int launch_tiles_t(const GlaArgs& a, const TileGeo& geo, int dev) {
   return hipGetLastError() == hipSuccess ? 0 : -5;
 }
 
-// the caller's strides, plain ones where there are none: rows 16-byte aligned, pitches within the descriptors' 32-bit extents
-static int fill_strides(const GlaArgs& a, TileGeo& geo) {
+// the caller's strides (batch, head, token), plain ones where there are none: rows 16-byte aligned, pitches within the descriptors'
+// 32-bit extents
+int gla_strides(const GlaArgs& a, long long (&q)[3], long long (&k)[3], long long (&v)[3]) {
   const long long* given[3] = {a.q_strides, a.k_strides, a.v_strides};
-  long long* dst[3] = {geo.sq, geo.sk, geo.sv};
+  long long* dst[3] = {q, k, v};
   const int D[3] = {a.Dk, a.Dk, a.Dv};
   for (int i = 0; i < 3; ++i) {
     if (given[i] && given[i][2] != 0) {
-      // rows 16-byte aligned, pitches within the descriptors' 32-bit extents
       for (int j = 0; j < 3; ++j)
         if (given[i][j] <= 0 || given[i][j] % 8 != 0) return -22;
       if (given[i][2] > (1 << 20)) return -22;
@@ -1121,7 +1121,7 @@ int launch_gla_tiles(const GlaArgs& a) {
   geo.wide = a.wide_gates;
   const bool pitched = a.q_strides || a.k_strides || a.v_strides;
   if (pitched)
-    if (const int rc = fill_strides(a, geo)) return rc;
+    if (const int rc = gla_strides(a, geo.sq, geo.sk, geo.sv)) return rc;
   const bool bidir = a.g_bwd != nullptr;
   if (a.gate_w) {
     geo.gw = a.gate_cols, geo.gh = a.gate_rows, geo.heads = a.H;
@@ -1162,7 +1162,7 @@ int launch_gla_tiles_chain(const GlaArgs& a, const float* states, const float* m
   geo.states = states;
   geo.maxima = maxima;
   if (a.low) {
-    if (const int rc = fill_strides(a, geo)) return rc;
+    if (const int rc = gla_strides(a, geo.sq, geo.sk, geo.sv)) return rc;
     fill_lowrank(a, geo);
     return launch_tiles_t<2, true, true, false, true, true>(a, geo, dev);
   }

@@ -107,11 +107,12 @@ size_t gla_recurrent_workspace(int B, int H, int L, int Dv, int io_dtype);
 bool gla_mfma_supported(const GlaArgs& a);
 int launch_gla_mfma(const GlaArgs& a);
 int launch_gla_lowrank(const GlaArgs& a);
-// bf16 tile-pair path for whole-sequence slabs (L <= 256): one wave per 32-token tile, both directions per wave.
+int gla_strides(const GlaArgs& a, long long (&q)[3], long long (&k)[3], long long (&v)[3]);  // what q, k, v are read with; -22: none such
+// bf16 tile-pair path for whole sequences (up to gla_slab_tokens): one wave per 32-token tile, both directions per wave.
 bool gla_tiles_supported(const GlaArgs& a);
 int gla_slab_tokens(int Dk);  // longest sequence that one workgroup takes whole
 int launch_gla_tiles(const GlaArgs& a);
-// the same kernel as the output pass of a long sequence (L > 256): one workgroup per (sequence, segment), the states
+// the same kernel as the output pass of a longer sequence: one workgroup per (sequence, segment), the states
 // entering the segments (scanned slots, kGlaStateFloats floats per (sequence, segment, direction)) and their maxima
 // (kGlaScanMaxima floats per (sequence, direction)) in `states` / `maxima`
 bool gla_tiles_chain_supported(const GlaArgs& a);
