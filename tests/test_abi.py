@@ -92,3 +92,22 @@ def test_reference_signatures():
     sig = inspect.signature(vig_amd.bid_fused_recurrent_gla)
     assert list(sig.parameters) == ["q", "k", "v", "gk", "gv", "scale", "initial_state", "output_final_state", "causal"]
     assert sig.parameters["scale"].default == -1 and sig.parameters["causal"].default is True
+
+
+def test_token_rows_past_two_to_the_31():
+    """Elementwise passes over token rows take as many as 32 bits number (16 channels of them fit the card)."""
+    import torch
+
+    from vig_amd import _lib
+
+    if not os.path.exists(_lib.LIB_PATH):
+        pytest.skip("library not built here")
+    if torch.cuda.is_available():
+        pytest.skip("pointers to nothing: only where no launch can follow")
+    lib, p, nan = _lib.load(), 4096, float("nan")
+    refused = (_lib.VIG_EINVAL, _lib.VIG_ENOTSUP)
+    for B, L in ((2, 1 << 30), (60000, 70000)):
+        assert lib.vig_dirgate_fwd(p, p, B, L, 1, 8, 1.0, nan, 1, 1, None) not in refused
+        assert lib.vig_dirgate_bwd(p, p, p, B, L, 1, 8, 1.0, nan, 1, 1, None) not in refused
+        assert lib.vig_split_heads_fwd(p, p, p, p, B, L, 1, 8, 8, 0, 1, None) not in refused
+    assert lib.vig_dirgate_fwd(p, p, 65535, 70000, 1, 8, 1.0, nan, 1, 1, None) in refused

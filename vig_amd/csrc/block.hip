@@ -402,9 +402,10 @@ __global__ __launch_bounds__(256) void split_heads_kernel(typename std::conditio
 
 template <bool MERGE, typename Q, typename P>
 static int launch_heads(Q* qkv, P* q, P* k, P* v, int B, int L, int H, int Dk, int Dv, long long ld, int io_dtype, hipStream_t stream) {
-  if (Dk % 8 != 0 || Dv % 8 != 0 || B > 65535 || (long long)B * L > 0x7fffffffLL) return -95;
-  const int nv = H * (2 * Dk + Dv) / 8, each = octets_each((long long)B * L, nv), tokens = octet_tokens(nv, each);
-  const dim3 grid(((unsigned)B * L + tokens - 1) / tokens), block(256);
+  if (Dk % 8 != 0 || Dv % 8 != 0 || B > 65535 || !octet_rows_ok(B, L)) return -95;
+  const int nv = H * (2 * Dk + Dv) / 8, each = octets_each((long long)B * L, nv);
+  int tokens = octet_tokens(nv, each);
+  const dim3 grid(octet_grid((long long)B * L, tokens)), block(256);
 #define VIG_HEADS_CASE(T)                                                                                                              \
   hipLaunchKernelGGL((each == 4 ? split_heads_kernel<T, MERGE, 4> : split_heads_kernel<T, MERGE, 1>), grid, block, 0, stream,         \
                      (typename std::conditional<MERGE, T, const T>::type*)qkv, (typename std::conditional<MERGE, const T, T>::type*)q, \

@@ -130,9 +130,10 @@ __global__ __launch_bounds__(256) void dirgate_bwd_kernel(const TI* __restrict__
 int launch_dirgate_bwd(const void* in, const void* d_out, void* d_in, int B, int L, int H, int Dk, float inv_norm,
                        float clamp_min, int in_dtype, int out_dtype, hipStream_t stream) {
   const int use_clamp = clamp_min == clamp_min;  // NaN disables
-  if (B > 65535 || (long long)B * L > 0x7fffffffLL) return -22;
-  const int nv = 2 * H * Dk / 8, each = octets_each((long long)B * L, nv), tokens = octet_tokens(nv, each);
-  const dim3 grid(((unsigned)B * L + tokens - 1) / tokens), block(256);
+  if (B > 65535 || !octet_rows_ok(B, L)) return -22;
+  const int nv = 2 * H * Dk / 8, each = octets_each((long long)B * L, nv);
+  int tokens = octet_tokens(nv, each);
+  const dim3 grid(octet_grid((long long)B * L, tokens)), block(256);
 #define VIG_DGB_CASE(TI, TO)                                                                                                   \
   hipLaunchKernelGGL((each == 4 ? dirgate_bwd_kernel<TI, TO, 4> : dirgate_bwd_kernel<TI, TO, 1>), grid, block, 0, stream,     \
                      (const TI*)in, (const TO*)d_out, (TI*)d_in, B, L, H, Dk, inv_norm, clamp_min, use_clamp, tokens)
@@ -148,10 +149,11 @@ template <typename TI, typename TO>
 static int launch_dirgate_t(const void* in, void* out, int B, int L, int H, int Dk, float inv_norm,
                             float clamp_min, hipStream_t stream) {
   const int use_clamp = clamp_min == clamp_min;  // NaN disables
-  if (B > 65535 || (long long)B * L > 0x7fffffffLL) return -22;
-  const int nv = 2 * H * Dk / 8, each = octets_each((long long)B * L, nv), tokens = octet_tokens(nv, each);
-  hipLaunchKernelGGL((each == 4 ? dirgate_kernel<TI, TO, 4> : dirgate_kernel<TI, TO, 1>), dim3(((unsigned)B * L + tokens - 1) / tokens),
-                     dim3(256), 0, stream, (const TI*)in, (TO*)out, B, L, H, Dk, inv_norm, clamp_min, use_clamp, tokens);
+  if (B > 65535 || !octet_rows_ok(B, L)) return -22;
+  const int nv = 2 * H * Dk / 8, each = octets_each((long long)B * L, nv);
+  int tokens = octet_tokens(nv, each);
+  const dim3 grid(octet_grid((long long)B * L, tokens)), block(256);
+  hipLaunchKernelGGL((each == 4 ? dirgate_kernel<TI, TO, 4> : dirgate_kernel<TI, TO, 1>), grid, block, 0, stream, (const TI*)in, (TO*)out, B, L, H, Dk, inv_norm, clamp_min, use_clamp, tokens);
   return hipGetLastError() == hipSuccess ? 0 : -5;
 }
 
@@ -858,9 +860,10 @@ __global__ __launch_bounds__(256) void locality_blend_kernel(const T* __restrict
 int launch_locality_blend(const void* o, const void* loc, const void* glin, const float* wg, const float* wl, void* y,
                           int B, int H, int L, int Dv, long long ldg, float eps, int silu_out, int io_dtype,
                           hipStream_t stream) {
-  if (B > 65535 || (long long)B * L > 0x7fffffffLL) return -22;
-  const int nv = H * (Dv / 8), each = octets_each((long long)B * L, nv), tokens = octet_tokens(nv, each);
-  const dim3 grid(((unsigned)B * L + tokens - 1) / tokens), block(256);
+  if (B > 65535 || !octet_rows_ok(B, L)) return -22;
+  const int nv = H * (Dv / 8), each = octets_each((long long)B * L, nv);
+  int tokens = octet_tokens(nv, each);
+  const dim3 grid(octet_grid((long long)B * L, tokens)), block(256);
 #define VIG_BLEND_CASE(T)                                                                                                    \
   hipLaunchKernelGGL((each == 4 ? locality_blend_kernel<T, 4> : locality_blend_kernel<T, 1>), grid, block, 0, stream,       \
                      (const T*)o, (const T*)loc, (const T*)glin, wg, wl, (T*)y, B, H, L, Dv, ldg, eps, silu_out, tokens)
@@ -1214,7 +1217,7 @@ int launch_locality_blend_bwd(const void* o, const void* loc, const void* glin, 
                               const void* dy, void* d_o, void* d_loc, void* d_glin, float* dw, void* workspace, long long workspace_rows, int B,
                               int H, int L, int Dv, long long ldg, long long ldd, float eps, int silu_out, int io_dtype,
                               hipStream_t stream) {
-  if (B > 65535 || (long long)B * L > 0x7fffffffLL) return -22;
+  if (B > 65535 || !octet_rows_ok(B, L)) return -22;
   const int nv = H * (Dv / 8);
   const long long total = (long long)B * L, room = std::min<long long>(kBlendBwdBlocks, workspace_rows);
   // whole rounds of 256 octets, as few as the workgroups allow

@@ -162,6 +162,13 @@ int launch_few_swiglu(const void* x, const void* w, void* y, long long T, int K,
 
 // Tokens a workgroup of 256 threads owns where every thread takes `each` octets of rows of nv octets (OctetRows).
 inline int octet_tokens(int nv, int each) { return nv >= 256 * each ? 1 : 256 * each / nv; }
+// ... and their workgroups, as many as one launch takes threads for (a workgroup of more tokens goes round more often); token rows are
+// numbered in 32 bits
+inline bool octet_rows_ok(int B, int L) { return (long long)B * L <= 0xffffffffLL; }
+inline unsigned octet_grid(long long rows, int& tokens) {
+  while ((rows + tokens - 1) / tokens > 0xffffff) tokens *= 2;
+  return (unsigned)((rows + tokens - 1) / tokens);
+}
 // Octets a thread takes at once: four, whose loads are under way together, once that leaves four workgroups a compute unit.
 inline int octets_each(long long rows, int nv) { return rows / octet_tokens(nv, 4) >= 1024 ? 4 : 1; }
 
