@@ -1,4 +1,4 @@
-// Segment states of long sequences (gfx950), bf16, Dk in {32, 64}, Dv = 64: per (sequence, segment, direction) what the
+// Segment states of long sequences (gfx950), bf16, Dk = 32, Dv = 64: per (sequence, segment, direction) what the
 // segment's tokens contribute to the state that leaves it, U = sum_t w_t k_t v_t^T, and the segment's total decay; for the
 // backward also the gradient states, the same sums over (q, d_o).
 //   plain set:     forward  w_t = exp(gates of the tokens behind t),  reverse  w_t = exp(gates of the tokens before t)
@@ -8,10 +8,11 @@
 // One workgroup per (sequence, segment), each wave two 32-token tiles.  Everything is read with tokens in the contraction slots
 // (mfma_tiles.h), so a lane owns channels: a tile's cumulative gates come out of a triangular-ones product in the layout that
 // weights the keys and feeds the next product, and the tiles' totals, exchanged through LDS, anchor the weights at the segment's
-// edge as one addition per channel.  The waves' sums meet in LDS once per direction.  The weighted key goes in as two bf16
+// edge as one addition per channel.  The waves' sums meet in LDS.  The weighted key goes in as two bf16
 // pieces (17 bits) against v as it is: no range to guard, and the kernel waits for memory, not for the matrix pipe.
-// Dk 32: the lanes' upper half, which holds no channel, carries the other direction, one pass serves both.
-// Whole op at Dk 32, us, against the chunked kernel's state pass (one workgroup of eight waves per CU, four chunks walked each
+// The lanes' upper half, which holds no channel, carries the other direction: one pass serves both.  (64 channels, which fill the lanes,
+// have gla_mfma.hip's state pass.)
+// Whole op, us, against the chunked kernel's state pass (one workgroup of eight waves per CU, four chunks walked each
 // way): 24 sequences of 4096 tokens 47.5 -> 44.9, 45 of 1679 44.9 -> 41.7, 147 of 534 43.6 -> 40.5.
 #include "common.h"
 #include "launch.h"
@@ -35,7 +36,7 @@ struct StateArgs {
 
 constexpr int kStateTiles = 16;  // most tiles of a segment
 constexpr int kStateRedBytes = 64 * 64 * 4;
-constexpr int state_lds(int waves) { return 2 * kStateTiles * 64 * 4 + waves * kStateRedBytes; }
+constexpr int state_lds(int waves) { return kStateTiles * 64 * 4 + waves * kStateRedBytes; }
 
 // tokens j that row token i of the cumulative product adds up: before or behind i, with or without i itself
 __device__ __forceinline__ uint32_t token_bits(bool before, bool with_own, int i) {
@@ -66,7 +67,7 @@ __device__ __forceinline__ void add_tile(const u32x4_t (&kf)[2][2], const u32x4_
     }
 }
 
-// LOW (Dk 32): one matrix instruction per channel parity makes a tile's gates of both directions from its rank-16 rows, where the lanes
+// LOW: one matrix instruction per channel parity makes a tile's gates of both directions from its rank-16 rows, where the lanes
 // would have read them.
 __device__ __forceinline__ void lowrank_gates(u32x4_t x, u32x4_t w, float bias, float inv_norm, float clamp, int rows, int h,
                                               u32x4_t (&gate)[2]) {
@@ -77,24 +78,20 @@ __device__ __forceinline__ void lowrank_gates(u32x4_t x, u32x4_t w, float bias, 
 
 }  // namespace
 
-template <int NG, bool LOW = false>
+template <bool LOW>
 __global__ __launch_bounds__(512, 2) void gla_states_kernel(StateArgs a) {
   extern __shared__ __align__(16) char lds[];
-  constexpr int DK = 16 * NG;
-  constexpr bool kJoint = NG == 2;  // both directions in one pass
-  constexpr int NDIR = kJoint ? 1 : 2;
+  constexpr int NG = 2, DK = 16 * NG;
   const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), waves = (int)blockDim.x >> 6;
   const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
   const bool grad = !LOW && blockIdx.z != 0, bidir = LOW || a.gb != nullptr;
   const int seq = blockIdx.x, seg = blockIdx.y;
-  float* tot = reinterpret_cast<float*>(lds);  // [direction][tile][p][lane row]
-  char* red = lds + 2 * kStateTiles * 64 * 4;
+  float* tot = reinterpret_cast<float*>(lds);  // [tile][p][lane row]
+  char* red = lds + kStateTiles * 64 * 4;
 
   // ---- loads of both tiles ----
-  const int rho = kJoint ? r & 15 : r;
-  const unsigned ch2 = cpair<NG>(rho);
-  uint32_t gD[NDIR][2][2][8], kD[2][2][8], vD[2][2][8];
-  static_assert(!LOW || kJoint, "gates from rank-16 rows: 32 key channels");
+  const unsigned ch2 = cpair<NG>(r & 15);
+  uint32_t gD[2][2][8], kD[2][2][8], vD[2][2][8];
   const int batch = LOW ? seq / a.H : 0, head = LOW ? seq - batch * a.H : 0;
   u32x4_t lowx[2], loww[2];
   uint32_t lowb[2];
@@ -127,14 +124,10 @@ __global__ __launch_bounds__(512, 2) void gla_states_kernel(StateArgs a) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         const unsigned off = base + (unsigned)jmap(t, 0, e) * (2u * DK);
-        if (kJoint) {  // (a lane of the other half reads beyond the descriptor: zero)
-          const uint32_t f = __builtin_amdgcn_raw_buffer_load_b32(rf, r < 16 ? off : kOutOfRange, 0, 0);
-          const uint32_t b = __builtin_amdgcn_raw_buffer_load_b32(rb, r < 16 ? kOutOfRange : off, 0, 0);
-          gD[0][i][t][e] = f | b;
-        } else {
-          gD[0][i][t][e] = __builtin_amdgcn_raw_buffer_load_b32(rf, off, 0, 0);
-          gD[NDIR - 1][i][t][e] = __builtin_amdgcn_raw_buffer_load_b32(rb, off, 0, 0);
-        }
+        // (a lane of the other half reads beyond the descriptor: zero)
+        const uint32_t f = __builtin_amdgcn_raw_buffer_load_b32(rf, r < 16 ? off : kOutOfRange, 0, 0);
+        const uint32_t b = __builtin_amdgcn_raw_buffer_load_b32(rb, r < 16 ? kOutOfRange : off, 0, 0);
+        gD[i][t][e] = f | b;
       }
   }
 #pragma unroll
@@ -161,113 +154,91 @@ __global__ __launch_bounds__(512, 2) void gla_states_kernel(StateArgs a) {
   }
 
   // ---- the tiles' totals, to everybody ----
-  u32x4_t gfrag[NDIR][2][2][2];
-  float own[NDIR][2][2];
+  u32x4_t gfrag[2][2][2];
+  float own[2][2];
   const u32x4_t ones = {0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};
 #pragma unroll
-  for (int d = 0; d < NDIR; ++d)
+  for (int i = 0; i < 2; ++i) {
+    if constexpr (!LOW) finish_tfrags<2>(gD[i], gfrag[i]);
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      if constexpr (!LOW) finish_tfrags<2>(gD[d][i], gfrag[d][i]);
-#pragma unroll
-      for (int p = 0; p < 2; ++p) {
-        if constexpr (LOW) {
-          u32x4_t gate[2];
-          lowrank_gates(lowx[i], loww[p], __uint_as_float(lowb[p] << 16), a.inv_norm, a.clamp, rows[i], h, gate);
-          gfrag[d][i][0][p] = gate[0], gfrag[d][i][1][p] = gate[1];
-        }
-        f32x16_t T = {0.f};
-        T = mfma(ones, gfrag[d][i][0][p], T);
-        T = mfma(ones, gfrag[d][i][1][p], T);
-        own[d][i][p] = T[0];
-        if (h == 0) tot[(d * kStateTiles + 2 * w + i) * 64 + 32 * p + r] = T[0];
+    for (int p = 0; p < 2; ++p) {
+      if constexpr (LOW) {
+        u32x4_t gate[2];
+        lowrank_gates(lowx[i], loww[p], __uint_as_float(lowb[p] << 16), a.inv_norm, a.clamp, rows[i], h, gate);
+        gfrag[i][0][p] = gate[0], gfrag[i][1][p] = gate[1];
       }
+      f32x16_t T = {0.f};
+      T = mfma(ones, gfrag[i][0][p], T);
+      T = mfma(ones, gfrag[i][1][p], T);
+      own[i][p] = T[0];
+      if (h == 0) tot[(2 * w + i) * 64 + 32 * p + r] = T[0];
     }
+  }
   lds_barrier();
-  float before[NDIR][2], behind[NDIR][2];
-#pragma unroll
-  for (int d = 0; d < NDIR; ++d)
-#pragma unroll
-    for (int p = 0; p < 2; ++p) before[d][p] = behind[d][p] = 0.f;
+  float before[2] = {0.f, 0.f}, behind[2] = {0.f, 0.f};
   for (int t = 0; t < 2 * waves; ++t)
 #pragma unroll
-    for (int d = 0; d < NDIR; ++d)
-#pragma unroll
-      for (int p = 0; p < 2; ++p) {
-        const float x = tot[(d * kStateTiles + t) * 64 + 32 * p + r];
-        before[d][p] += t < 2 * w ? x : 0.f;
-        behind[d][p] += t > 2 * w + 1 ? x : 0.f;
-      }
+    for (int p = 0; p < 2; ++p) {
+      const float x = tot[t * 64 + 32 * p + r];
+      before[p] += t < 2 * w ? x : 0.f;
+      behind[p] += t > 2 * w + 1 ? x : 0.f;
+    }
 
   // ---- decays ----
   float* out = (grad ? a.grad_slots : a.slots) + ((size_t)seq * a.nseg + seg) * 2 * kGlaStateFloats;
   if (w == 0 && h == 0 && !grad) {
 #pragma unroll
-    for (int d = 0; d < NDIR; ++d)
-#pragma unroll
-      for (int p = 0; p < 2; ++p) {
-        const float all = before[d][p] + own[d][0][p] + own[d][1][p] + behind[d][p];
-        out[(kJoint ? r >> 4 : d) * kGlaStateFloats + 64 * 64 + 2 * ch2 + p] = exp2_fast(all * kLog2e);
-      }
+    for (int p = 0; p < 2; ++p) {
+      const float all = before[p] + own[0][p] + own[1][p] + behind[p];
+      out[(r >> 4) * kGlaStateFloats + 64 * 64 + 2 * ch2 + p] = exp2_fast(all * kLog2e);
+    }
   }
 
   // ---- weights, products, the waves' sums ----
+  f32x16_t U[2][2] = {{{0.f}, {0.f}}, {{0.f}, {0.f}}};
 #pragma unroll
-  for (int d = 0; d < NDIR; ++d) {
-    if (d == 1 && !bidir) break;
-    f32x16_t U[2][2] = {{{0.f}, {0.f}}, {{0.f}, {0.f}}};
+  for (int i = 0; i < 2; ++i) {
+    u32x4_t kf[2][2], vf[2][2];
+    finish_tfrags<2>(kD[i], kf);
+    finish_tfrags<2>(vD[i], vf);
+    f32x16_t G[2];
+    float off[2];
+    const bool up = grad;  // the lower lane half's (forward) direction adds up the tokens before
+    const uint32_t bits = token_bits(up, grad, r) >> (4 * h);
+    const u32x4_t tri0 = keep_masks<0>(bits) & 0x3F803F80u, tri1 = keep_masks<1>(bits) & 0x3F803F80u;
+    const uint32_t obits = token_bits(!up, grad, r) >> (4 * h);
+    const u32x4_t otri0 = keep_masks<0>(obits) & 0x3F803F80u, otri1 = keep_masks<1>(obits) & 0x3F803F80u;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      u32x4_t kf[2][2], vf[2][2];
-      finish_tfrags<2>(kD[i], kf);
-      finish_tfrags<2>(vD[i], vf);
-      f32x16_t G[2];
-      float off[2];
-      const bool up = (d == 0) == grad;  // this (lower lane half's) direction adds up the tokens before
-      const uint32_t bits = token_bits(up, grad, r) >> (4 * h);
-      const u32x4_t tri0 = keep_masks<0>(bits) & 0x3F803F80u, tri1 = keep_masks<1>(bits) & 0x3F803F80u;
-      const uint32_t obits = token_bits(!up, grad, r) >> (4 * h);
-      const u32x4_t otri0 = keep_masks<0>(obits) & 0x3F803F80u, otri1 = keep_masks<1>(obits) & 0x3F803F80u;
+    for (int p = 0; p < 2; ++p) {
+      f32x16_t g = {0.f}, o = {0.f};
+      g = mfma(tri0, gfrag[i][0][p], g);
+      G[p] = mfma(tri1, gfrag[i][1][p], g);
+      o = mfma(otri0, gfrag[i][0][p], o);
+      o = mfma(otri1, gfrag[i][1][p], o);
 #pragma unroll
-      for (int p = 0; p < 2; ++p) {
-        f32x16_t g = {0.f};
-        g = mfma(tri0, gfrag[d][i][0][p], g);
-        G[p] = mfma(tri1, gfrag[d][i][1][p], g);
-        if (kJoint) {
-          f32x16_t o = {0.f};
-          o = mfma(otri0, gfrag[d][i][0][p], o);
-          o = mfma(otri1, gfrag[d][i][1][p], o);
-#pragma unroll
-          for (int c = 0; c < 16; ++c) G[p][c] = r < 16 ? G[p][c] : o[c];
-        }
-        const float b = before[d][p] + (i == 1 ? own[d][0][p] : 0.f), e = behind[d][p] + (i == 0 ? own[d][1][p] : 0.f);
-        off[p] = (kJoint && r >= 16) != up ? b : e;
-      }
-      add_tile(kf, vf, G, off, U);
+      for (int c = 0; c < 16; ++c) G[p][c] = r < 16 ? G[p][c] : o[c];
+      const float b = before[p] + (i == 1 ? own[0][p] : 0.f), e = behind[p] + (i == 0 ? own[1][p] : 0.f);
+      off[p] = (r >= 16) != up ? b : e;
     }
-    char* mine = red + w * kStateRedBytes;
-    if (d > 0) lds_barrier();  // the sums of the direction before have been read
+    add_tile(kf, vf, G, off, U);
+  }
+  char* mine = red + w * kStateRedBytes;
 #pragma unroll
-    for (int pk = 0; pk < 2; ++pk)
+  for (int pk = 0; pk < 2; ++pk)
 #pragma unroll
-      for (int pv = 0; pv < 2; ++pv)
+    for (int pv = 0; pv < 2; ++pv)
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const f32x4_t x = {U[pk][pv][4 * g], U[pk][pv][4 * g + 1], U[pk][pv][4 * g + 2], U[pk][pv][4 * g + 3]};
-          *reinterpret_cast<f32x4_t*>(unit_ptr(mine, (pk * 2 + pv) * 4 + g, lane)) = x;
-        }
-    lds_barrier();
-    for (int i = threadIdx.x; i < 16 * 64; i += blockDim.x) {
-      f32x4_t x = *reinterpret_cast<const f32x4_t*>(red + 16 * i);
-      for (int o = 1; o < waves; ++o) x += *reinterpret_cast<const f32x4_t*>(red + o * kStateRedBytes + 16 * i);
-      // (joint: register quads 0, 1 are the forward direction's, 2, 3 the reverse one's)
-      const int u = i >> 6, g = u & 3;
-      if (kJoint) {
-        if (g < 2 || bidir) *reinterpret_cast<f32x4_t*>(out + (g >> 1) * kGlaStateFloats + (((u & ~3) | (g & 1)) * 64 + (i & 63)) * 4) = x;
-      } else {
-        *reinterpret_cast<f32x4_t*>(out + d * kGlaStateFloats + 4 * i) = x;
+      for (int g = 0; g < 4; ++g) {
+        const f32x4_t x = {U[pk][pv][4 * g], U[pk][pv][4 * g + 1], U[pk][pv][4 * g + 2], U[pk][pv][4 * g + 3]};
+        *reinterpret_cast<f32x4_t*>(unit_ptr(mine, (pk * 2 + pv) * 4 + g, lane)) = x;
       }
-    }
+  lds_barrier();
+  for (int i = threadIdx.x; i < 16 * 64; i += blockDim.x) {
+    f32x4_t x = *reinterpret_cast<const f32x4_t*>(red + 16 * i);
+    for (int o = 1; o < waves; ++o) x += *reinterpret_cast<const f32x4_t*>(red + o * kStateRedBytes + 16 * i);
+    // (register quads 0, 1 are the forward direction's, 2, 3 the reverse one's)
+    const int u = i >> 6, g = u & 3;
+    if (g < 2 || bidir) *reinterpret_cast<f32x4_t*>(out + (g >> 1) * kGlaStateFloats + (((u & ~3) | (g & 1)) * 64 + (i & 63)) * 4) = x;
   }
 }
 
@@ -280,20 +251,19 @@ int launch_gla_states(const GlaArgs& a, int seg_len, int nseg, float* slots, con
               (const uint16_t*)q, (const uint16_t*)d_o, slots, grad_slots, a.L, seg_len, nseg};
   const int waves = (NT + 1) / 2;
   const dim3 grid(a.B * a.H, nseg, q ? 2 : 1), block(64 * waves);
-  static bool done[3][64] = {};
+  static bool done[64] = {}, done_low[64] = {};
+  if (a.Dk != 32) return -95;
   if (a.low) {
-    if (a.Dk != 32 || q || !a.k_strides || !a.v_strides) return -22;
+    if (q || !a.k_strides || !a.v_strides) return -22;
     for (int j = 0; j < 3; ++j) s.sk[j] = a.k_strides[j], s.sv[j] = a.v_strides[j];
     s.low = (const uint16_t*)a.low, s.up_w = (const uint16_t*)a.up_w, s.up_b = (const uint16_t*)a.up_b;
     s.low_ld = a.low_ld, s.inv_norm = a.inv_norm, s.clamp = a.clamp, s.H = a.H;
-    if (!allow_lds(reinterpret_cast<const void*>(gla_states_kernel<2, true>), state_lds(kStateTiles / 2), done[2])) return -5;
-    hipLaunchKernelGGL((gla_states_kernel<2, true>), grid, block, state_lds(waves), a.stream, s);
-    return hipGetLastError() == hipSuccess ? 0 : -5;
+    if (!allow_lds(reinterpret_cast<const void*>(gla_states_kernel<true>), state_lds(kStateTiles / 2), done_low)) return -5;
+    hipLaunchKernelGGL(gla_states_kernel<true>, grid, block, state_lds(waves), a.stream, s);
+  } else {
+    if (!allow_lds(reinterpret_cast<const void*>(gla_states_kernel<false>), state_lds(kStateTiles / 2), done)) return -5;
+    hipLaunchKernelGGL(gla_states_kernel<false>, grid, block, state_lds(waves), a.stream, s);
   }
-  const void* kernel = a.Dk == 64 ? reinterpret_cast<const void*>(gla_states_kernel<4>) : reinterpret_cast<const void*>(gla_states_kernel<2>);
-  if (!allow_lds(kernel, state_lds(kStateTiles / 2), done[a.Dk == 64])) return -5;
-  if (a.Dk == 64) hipLaunchKernelGGL(gla_states_kernel<4>, grid, block, state_lds(waves), a.stream, s);
-  else hipLaunchKernelGGL(gla_states_kernel<2>, grid, block, state_lds(waves), a.stream, s);
   return hipGetLastError() == hipSuccess ? 0 : -5;
 }
 
