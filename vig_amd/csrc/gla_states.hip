@@ -176,6 +176,7 @@ __global__ __launch_bounds__(512, 2) void gla_states_kernel(StateArgs a) {
   }
   lds_barrier();
   float before[2] = {0.f, 0.f}, behind[2] = {0.f, 0.f};
+#pragma unroll 1
   for (int t = 0; t < 2 * waves; ++t)
 #pragma unroll
     for (int p = 0; p < 2; ++p) {

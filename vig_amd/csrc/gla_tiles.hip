@@ -81,16 +81,16 @@ struct TileLds {
   static constexpr int KB = NG * 1024;  // one k^ tile: NG units
   static constexpr int VB = 4096;       // one V tile: 4 units
   int kf, kb, v, d, scratch, scratch_b, guard, total;
-  // gate_bytes: what the fused locality gate stages in the tile regions once they are dead (0: no gate)
-  __host__ __device__ explicit TileLds(int NT, int gate_bytes = 0) {
+  // gate_bytes: what the fused locality gate stages in the tile regions once they are dead (0: no gate); many: more than kFewTiles
+  __host__ __device__ TileLds(int NT, int gate_bytes, bool many) {
     kf = 0;
     kb = (NT - 1) * KB;
     v = 2 * (NT - 1) * KB;
     d = v + NT * VB;
     if (d < gate_bytes) d = gate_bytes;
     scratch = d + 2 * NT * 128;  // per wave: 64 floats (tile totals on their way from one lane pair to a lane per channel)
-    // (the reverse direction's; more than kFewTiles: both stay, everybody reads them)
-    scratch_b = NT > kFewTiles ? scratch + NT * 256 : scratch;
+    // (the reverse direction's; many: both stay, everybody reads them)
+    scratch_b = many ? scratch + NT * 256 : scratch;
     guard = scratch_b + NT * 256;
     total = guard + NT * 16;
   }
@@ -222,14 +222,6 @@ __device__ __forceinline__ void park_totals(f32x16_t& C, float* sc, int r, int h
   wave_lds_sync();
 }
 
-// place of sc[lane]'s channel in a table of decays (a lane half's 8 NG channels as it reads them)
-template <int NG>
-__device__ __forceinline__ int table_channel(int lane) {
-  return 8 * NG * (lane >> 5) + 8 * ((lane >> 2) & 3) + 2 * (lane & 3) + ((lane >> 4) & 1);
-}
-template <int NG>
-__device__ __forceinline__ bool has_table_channel(int lane) { return ((lane >> 2) & 3) < NG; }
-
 // Operands of one direction for this wave's tile, the publication of what other tiles need from it, and the diagonal
 // score tile (masked to the pairs the direction sees and rounded to fp16 pairs: the B operand of the value product).
 //   qh: q^ = q exp(G)      (B operand of every score product of this wave; kept)
@@ -260,7 +252,10 @@ __device__ __forceinline__ bool prepare_direction(const uint32_t (&gD)[2][8], co
   else tl = fmaxf(tl, kExpFloor);
   const float dT = exp2_fast(tl);
   if (GENERAL || MANY) sc[lane] = tl;
-  if (!MANY && has_table_channel<NG>(lane)) dtab[table_channel<NG>(lane)] = (_Float16)dT;
+  if (!MANY) {
+    const int p = (lane >> 4) & 1, g = (lane >> 2) & 3, m = lane & 3;
+    if (g < NG) dtab[HC * (lane >> 5) + 8 * g + 2 * m + p] = (_Float16)dT;
+  }
   wave_lds_sync();
   const float* mine = sc + 32 * (lane >> 5);
   const u32x4_t* dmine = reinterpret_cast<const u32x4_t*>(dtab + HC * (lane >> 5));  // this lane half's decays as fp16 pairs
@@ -461,9 +456,10 @@ __device__ __forceinline__ void walk_many_tiles(char* lds, const TileLds<NG>& la
   };
   const float* totals = reinterpret_cast<const float*>(lds + (FWD ? lay.scratch : lay.scratch_b)) + lane;
   char* factors = lds + lay.d + ti * 256;
-  const int mine = 2 * table_channel<NG>(lane);
+  // (sc[lane]'s channel, as in prepare_direction)
+  const int g0 = (lane >> 2) & 3, mine = 2 * (8 * NG * (lane >> 5) + 8 * g0 + 2 * (lane & 3) + ((lane >> 4) & 1));
   const auto leave = [&](int slot, float decay) {
-    if (has_table_channel<NG>(lane)) *reinterpret_cast<_Float16*>(factors + 128 * slot + mine) = (_Float16)decay;
+    if (g0 < NG) *reinterpret_cast<_Float16*>(factors + 128 * slot + mine) = (_Float16)decay;
     asm volatile("" ::: "memory");  // (a wave's LDS accesses stay in order)
   };
   float sum = 0.f;
@@ -734,7 +730,7 @@ template <int NG, bool BIDIR, bool PITCHED, bool GENERAL, bool GATE, bool CHAIN,
 __device__ __forceinline__ void tile_pass(const TileCtx& cx, const TileKernArgs* ka) {
   const int lane = cx.lane, r = lane & 31, h = lane >> 5;
   const int ti = cx.ti, NT = cx.NT;
-  const TileLds<NG> lay(NT, GATE ? gate_stage_bytes(cx.gw, cx.gh) : 0);
+  const TileLds<NG> lay(NT, GATE ? gate_stage_bytes(cx.gw, cx.gh) : 0, MANY);
   char* lds = cx.lds;
   char* vregion = lds + lay.v + ti * TileLds<NG>::VB;
   float* sc = reinterpret_cast<float*>(lds + lay.scratch + ti * 256);
@@ -1057,7 +1053,7 @@ bool gla_tiles_supported(const GlaArgs& a) {
         (long long)a.gate_cols * a.gate_rows != a.L)
       return false;
     const int NT = (a.L + 31) / 32, stage = gate_stage_bytes(a.gate_cols, a.gate_rows);
-    if ((a.Dk == 64 ? TileLds<4>(NT, stage).total : TileLds<2>(NT, stage).total) > kTileMaxLds) return false;
+    if ((a.Dk == 64 ? TileLds<4>(NT, stage, NT > kFewTiles).total : TileLds<2>(NT, stage, NT > kFewTiles).total) > kTileMaxLds) return false;
   }
   return true;
 }
@@ -1077,7 +1073,7 @@ static int launch_tiles_t(const GlaArgs& a, const TileGeo& geo, int dev) {
     if (kw && hipFuncSetAttribute(kw, hipFuncAttributeMaxDynamicSharedMemorySize, kTileMaxLds) != hipSuccess) return -5;
     attr_done_dev[dev] = true;
   }
-  const TileLds<NG> lay(geo.NT, GATE ? gate_stage_bytes(geo.gw, geo.gh) : 0);
+  const TileLds<NG> lay(geo.NT, GATE ? gate_stage_bytes(geo.gw, geo.gh) : 0, MANY);
   if (lay.total > kTileMaxLds) return -95;
   auto kernel = gla_tile_kernel<NG, BIDIR, PITCHED, GATE, CHAIN, LOW, MANY>;
   if constexpr (kWide)
