@@ -143,7 +143,9 @@ int vig_gla_lowrank_fwd(const void* q, const void* k, const void* v, const void*
 size_t vig_gla_bidir_fwd_workspace(int B, int H, int L, int Dk, int Dv, int io_dtype);
 /* Workspace of exactly the kernel vig_gla_bidir_fwd / _wide dispatch to for these arguments (bidirectional: g_bwd
  * given): 0 for bf16 tensors and gates with Dk in {32, 64}, Dv = 64, L <= 256 (between 257 tokens and the one-launch
- * kernel's limit only _wide uses it, but both ask for it). */
+ * kernel's limit only _wide uses it, but both ask for it).  fp32 tensors take quicker forms in this much than in less: shorter
+ * segments, or whole sequences as two halves, the sums in another order (equal within fp32 rounding); with the same
+ * number of bytes a call gives the same bits. */
 size_t vig_gla_bidir_fwd_workspace_for(int B, int H, int L, int Dk, int Dv, int io_dtype, int gate_dtype,
                                        int bidirectional);
 
@@ -196,12 +198,12 @@ int vig_gla_bidir_fwd_wide(const void* q, const void* k, const void* v,
 /*
  * vig_gla_bidir_fwd without a workspace argument, for callers that cannot allocate device memory: code under
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc.  Same tensors, dispatch, kernels and
- * results (bit for bit) as vig_gla_bidir_fwd; the workspace is a device array inside the library,
+ * results (bit for bit) as vig_gla_bidir_fwd with vig_gla_bidir_fwd_workspace_for(...) bytes; the workspace is a device array inside the library,
  * VIG_GLA_NOALLOC_SCRATCH_BYTES per GPU, held from the first call on that GPU until the process ends.  A shape whose
  * vig_gla_bidir_fwd_workspace_for(...) exceeds that size returns VIG_ENOSPC and launches nothing (then use
  * vig_gla_bidir_fwd with a workspace of the caller's).  Calls no hipMalloc / hipFree and nothing else that allocates.
- * All calls on one GPU share the one array: calls that overlap in time on the same GPU (two streams, two threads)
- * race on it; serialise them.  The tensors must live on the current device (another device's pointers: VIG_EINVAL).
+ * All calls on one GPU share the one array, fp32 calls on whole sequences too: calls that overlap in time on the same GPU (two
+ * streams, two threads) race on it; serialise them.  The tensors must live on the current device (another device's pointers: VIG_EINVAL).
  * Under HIP graph capture: make one call per device and shape class outside the capture first.  The first call on a
  * device looks up the array's address and sets the kernels' shared-memory attribute (no stream work, but not capturable
  * either); every later call is kernel launches on `stream` only.  It has no counterpart in the reference, whose ops

@@ -301,7 +301,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_blend_kernel(BlendFewArgs a) {
   const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int m0 = blockIdx.y * 32, n0 = blockIdx.x * 32;
-  // ---- the weights of this wave's stages (wave, wave + 4, ..), all of them under way at once ----
+  // ---- the weights of this wave's stages (wave, wave + NW, ..), all of them under way at once ----
   const uint32_t w0 = lds_offset(smem) + kX + wave * (kMine * 2048);
 #pragma unroll
   for (int at = 0; at < kMine; ++at) {
@@ -668,9 +668,12 @@ static long long tiles_of(const GemmArgs& a, int tm, int tn) { return (long long
 //   up to 9 GFLOP:              64 x 64 tiles    (M 1568 N 1280 K 384 6.1 / 6.9; M 2500 N 384 K 1024 8.0 / 8.0)
 //                               or, past 512 of them, 128 x 128 tiles  (M 3136 N 1280 K 384 8.3 / 9.1, with 64 x 64 tiles 10.3; M 9216 17.6 /
 //                               21.8, 22.9; M 4000 N 768 K 768 11.1 / 10.1, 13.3; M 1000 N 4096 K 768 13.4 / 11.2, 19.7)
-//                               (between 2 and 9 GFLOP a few us slower than the library on some sizes, at worst 18 %; but the library's
-//                               front end takes 22 us of host time a call, this one 4, and models of such products wait for the host, whole forward:
-//                               ViG-B, 2 images of 288 px, 37 products: 1.81 -> 1.06 ms; 8 of 208 px 1.84 -> 1.19; 4 of 320 px 2.05 -> 1.36; ViG-S, 16 of 224 px 0.95 -> 0.85)
+//                               (between 2 and 9 GFLOP the device alone takes 0.41 to 1.35 of the library's time, 0.93 in the mean of 80 drawn
+//                               sizes; the worst where a second tile comes to some CUs only, M 5725 N 768 K 768 16.6 / 12.2, and at
+//                               M 409 N 4096 K 768 11.3 / 8.7.  But the library's front end takes 22 us of host time a call, this one 4, and models
+//                               of such products wait for the host.  Whole forward, ms, library past 2 GFLOP / this, and as captured graphs: ViG-B,
+//                               images of 224 px, 2 1.30 / 1.00, 0.78 / 0.78; 6 1.72 / 1.10, 1.02 / 1.08; 12 1.93 / 1.39, 1.45 / 1.42; 20 1.94 / 1.88, 1.87 /
+//                               1.87; 29 2.66 / 2.68, 2.63 / 2.66; ViG-S 16 0.83 / 0.80, 0.82 / 0.80; 40 1.20 / 1.18, 1.19 / 1.18)
 //   K 384 or 192, N % 64 == 0, 16384 rows and fewer for some N (regs_rows): weights in registers (linear.hip)
 //   K <= 256 with 512 tiles:    256 x 128 tiles  (M 65536 N 520 K 192: other column counts)
 // Beyond that the library's products win (M 50176 N 1280 K 512 and longer contractions).

@@ -83,8 +83,8 @@ bool aligned(const Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr())
 
 // out = A B^T (+ bias) (+ add) of fp32 rows, A [M, K] or its transpose lying as rows, B [N, K] or its transpose, on the matrix cores;
 // false where the library's product is to be taken.
-// Where the line lies: a call costs 4 us of host time here and 22 us there, and products of up to about 5e9 multiply-adds take as long or
-// less here as well (us, here / library; layer, input gradient, weight gradient with column sums): 400 x 2048 x 384 10 / 10, 18 / 17, 18 / 22;
+// Where the line lies: a call costs 4 us of host time here and 22 us there, and products of up to about 5e9 multiply-adds take 0.4 to
+// 1.24 of the library's time on the device (us, here / library; layer, input gradient, weight gradient with column sums): 400 x 2048 x 384 10 / 10, 18 / 17, 18 / 22;
 // 1960 x 768 x 768 28 / 26, 30 / 30, 34 / 42; 8100 x 192 x 512 21 / 17, 24 / 30, 29 / 71; 8100 x 768 x 768 87 / 80, 85 / 90, 106 / 117; beyond,
 // 8100 x 2048 x 384 117 / 103, 106 / 110, 146 / 121.  Training passes (ms, line here / library alone): 32 images of 224 px, ViG-T
 // 7.9 / 10.1; 30, ViG-S 13.3 / 15.0 (line at 2.5e9: 14.2; at 9e9: 13.5).
