@@ -1,5 +1,5 @@
-"""The locality gate inside the op's kernel against the two calls, bit for bit, where outputs of the op leave fp16's range (the kernel
-stages them as fp16 pairs while every one of them is an fp16 value) and at every length the kernel takes."""
+"""The locality gate inside the op's kernel against the two calls, bit for bit, where outputs of the op are beyond fp16's range, below its grid,
+around its limits, zero, or large enough for the sigmoid's tail, and at every length the kernel takes."""
 import pytest
 import torch
 
@@ -38,3 +38,18 @@ def test_equals_two_calls(hw, Dk, what):
     got = vig_amd.gla_bidir_locality_gate(q, k, v, gf, gb, w, hw)
     assert torch.isfinite(got).all()
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("top", [0.0, 2.0 ** -23, 300.0, 500.0, 1020.0, 1024.0, 65000.0])
+@pytest.mark.parametrize("Dk", [32, 64])
+def test_largest_output(Dk, top):
+    """All outputs scaled to a largest one; 0: a head without values, a channel without, a masked query."""
+    announce(f"gate range, largest output {top} Dk{Dk}")
+    B, H, hw = 2, 3, (14, 14)
+    q, k, v, gf, gb = (t.cuda() for t in make_gla_inputs(B, H, 196, Dk, 64, seed=3, dtype=torch.bfloat16))
+    if top == 0:
+        v[:, 1], v[:, :, :, 5], q[:, :, 7] = 0, 0, 0
+    factor = top / float(vig_amd.gla_bidir_forward(q, k, v, gf, gb).float().abs().max()) if top else 1.0
+    w = make_locality_weight(H * 64, 31).cuda()
+    want = vig_amd.locality_gate(vig_amd.gla_bidir_forward(q, k, v, gf, gb, -1, factor), w, hw)
+    assert torch.equal(vig_amd.gla_bidir_locality_gate(q, k, v, gf, gb, w, hw, -1, factor), want)

@@ -97,7 +97,7 @@ struct TileLds {
 };
 
 // Fused locality gate: the slab's rounded outputs as a zero-padded (gh + 2) x (gw + 2) grid of cells (64 channels as
-// fp16: 128 bytes, 144 bytes apart, so that eight lanes on neighbouring tokens cover every LDS bank once), then the
+// bf16: 128 bytes, 144 bytes apart, so that eight lanes on neighbouring tokens cover every LDS bank once), then the
 // 64 x 9 stencil weights of the slab's head.
 constexpr int kGateWeightBytes = 64 * 9 * 4;
 constexpr int kGateCell = 144;
@@ -558,47 +558,56 @@ __device__ __forceinline__ void apply_state(const float* slot, int shift, const 
 }
 
 // Fused locality gate: y = o * sigmoid(conv3x3(o)) per channel on the gw x gh token grid (zero padding), o being the
-// bf16-rounded output.  The whole slab's outputs are staged in LDS where the tiles lay.
-struct GateGrid {
-  char* cells;
-  int gw, gh, pw;
-  float inv_w;
-};
-
-// This wave's rounded outputs into their cells: as pairs of fp16, times kGateUnit (F16: returns whether one may be none) or as
-// they are.
-constexpr float kGateUnit = 64.0f;
-template <bool F16>
-__device__ __forceinline__ bool stage_cells(const f32x16_t (&O)[2], float os, const GateGrid& g, int ti, int lane) {
-  const int T = 32 * ti + (lane & 31);
-  u16x2_t top = {0, 0};
-  if (F16) os *= kGateUnit;  // (a power of two: the same rounding)
-  if (T < g.gw * g.gh) {
-    const int y = (int)(((float)T + 0.5f) * g.inv_w), x = T - __mul24(y, g.gw);
-    char* cell = g.cells + ((y + 1) * g.pw + x + 1) * kGateCell + 64 * (lane >> 5);
+// bf16-rounded output, which is staged whole in LDS where the tiles lay; the arithmetic of the kernel that reads o from memory.
+// (fp16 cells, which v_fma_mix_f32 reads in place, hold neither large nor small outputs: 768 slabs of 14 x 14, Dk 64, 40.1 us with them, with
+// a look at the values and these cells for slabs that need them 41.8, these alone 40.7; one image of ViG-T 10.43, 10.64, 10.36.)
+__device__ __forceinline__ void locality_gate_epilogue(f32x16_t O0, f32x16_t O1, float os, char* cells, const float* gate_w,
+                                                    rsrc_t o_rsrc, int gw, int gh, int ti, int NT, int lane_w) {
+  const f32x16_t O[2] = {O0, O1};
+  const int pw = gw + 2;
+  const float inv_w = 1.0f / (float)gw;
+  float* wlds = reinterpret_cast<float*>(cells + pw * (gh + 2) * kGateCell);
+  // the head's stencil weights, fetched by the first 144 threads while the other waves finish their walks
+  f32x4_t w4 = {0.f, 0.f, 0.f, 0.f};
+  const bool w_mine = ti * 64 + lane_w < 64 * 9 / 4;
+  if (w_mine) w4 = reinterpret_cast<const f32x4_t*>(gate_w)[ti * 64 + lane_w];
+  lds_barrier();  // every wave is done with the tiles
+  if (w_mine) reinterpret_cast<f32x4_t*>(wlds)[ti * 64 + lane_w] = w4;
+  // (workgroups of fewer than three waves: the rest of the 144 pieces)
+  for (int idx = ti * 64 + lane_w + 64 * NT; idx < 64 * 9 / 4; idx += 64 * NT)
+    reinterpret_cast<f32x4_t*>(wlds)[idx] = reinterpret_cast<const f32x4_t*>(gate_w)[idx];
+  {
+    const int T = 32 * ti + (lane_w & 31);
+    if (T < gw * gh) {
+      const int y = (int)(((float)T + 0.5f) * inv_w), x = T - __mul24(y, gw);
+      char* cell = cells + ((y + 1) * pw + x + 1) * kGateCell + 64 * (lane_w >> 5);
 #pragma unroll
-    for (int gq = 0; gq < 4; ++gq) {
-      u32x4_t w;
+      for (int gq = 0; gq < 4; ++gq) {
+        u32x4_t w;
 #pragma unroll
-      for (int m = 0; m < 4; ++m) {
-        w[m] = pack_bf16x2(O[0][4 * gq + m] * os, O[1][4 * gq + m] * os);
-        if (F16) {
-          // a magnitude from 2^-17 to 2^16 (exclusive) is an fp16 value; less, or zero, wraps around (twice the bits: no sign)
-          const uint32_t both = w[m];
-          top = __builtin_elementwise_max(top, (u16x2_t)(__builtin_bit_cast(u16x2_t, both) * (uint16_t)2 - (uint16_t)0x6e00));
-          w[m] = pack_f16x2(bf16lo_to_f32(w[m]), bf16hi_to_f32(w[m]));
-        }
+        for (int m = 0; m < 4; ++m) w[m] = pack_bf16x2(O[0][4 * gq + m] * os, O[1][4 * gq + m] * os);
+        *reinterpret_cast<u32x4_t*>(cell + 16 * gq) = w;
       }
-      *reinterpret_cast<u32x4_t*>(cell + 16 * gq) = w;
     }
   }
-  return F16 && (top[0] >= 0x8f00 - 0x6e00 || top[1] >= 0x8f00 - 0x6e00);
-}
-
-// The stencil over the staged cells: four passes of eight tokens, a lane eight channels (octet oct) of one token.
-template <bool F16>
-__device__ __forceinline__ void gate_stencil(const GateGrid& g, const float* wlds, rsrc_t out, int ti, int lane) {
-  const int oct = lane & 7, tl = lane >> 3;
+  const int oct = lane_w & 7, tl = lane_w >> 3;
+  {  // the border cells, by the whole workgroup: top row, bottom row, then the two ends of every other row
+    const int nborder = 2 * pw + 2 * gh;
+    const u32x4_t zero = {0u, 0u, 0u, 0u};
+    for (int bc = ti * 8 + tl; bc < nborder; bc += 8 * NT) {
+      int py, px;
+      if (bc < 2 * pw) {
+        py = bc < pw ? 0 : gh + 1;
+        px = bc < pw ? bc : bc - pw;
+      } else {
+        const int j = bc - 2 * pw;
+        py = 1 + (j >> 1);
+        px = (j & 1) ? pw - 1 : 0;
+      }
+      *reinterpret_cast<u32x4_t*>(cells + (py * pw + px) * kGateCell + 16 * oct) = zero;
+    }
+  }
+  lds_barrier();  // the slab's outputs, the zero border and the weights are staged
   float wreg[8][9];
   {
     const f32x4_t* wp = reinterpret_cast<const f32x4_t*>(wlds + oct * 72);
@@ -606,104 +615,39 @@ __device__ __forceinline__ void gate_stencil(const GateGrid& g, const float* wld
     for (int i = 0; i < 18; ++i) {
       const f32x4_t x = wp[i];
 #pragma unroll
-      for (int m = 0; m < 4; ++m) wreg[(4 * i + m) / 9][(4 * i + m) % 9] = F16 ? x[m] : x[m] * kGateUnit;
+      for (int m = 0; m < 4; ++m) wreg[(4 * i + m) / 9][(4 * i + m) % 9] = x[m];
     }
   }
+  // four passes of eight tokens, a lane eight channels (octet oct) of one token
 #pragma unroll 1
   for (int i = 0; i < 4; ++i) {
     const int row = tl + 8 * i;
     const int T = 32 * ti + row;
-    if (T < g.gw * g.gh) {
-      const int y = (int)(((float)T + 0.5f) * g.inv_w), x = T - __mul24(y, g.gw);
+    if (T < gw * gh) {
+      const int y = (int)(((float)T + 0.5f) * inv_w), x = T - __mul24(y, gw);
       float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
       u32x4_t ctr = {0u, 0u, 0u, 0u};
 #pragma unroll
       for (int di = 0; di < 3; ++di) {
-        const char* rowp = g.cells + ((y + di) * g.pw + x) * kGateCell + 16 * oct;  // padded cell of tap (di - 1, -1)
+        const char* rowp = cells + ((y + di) * pw + x) * kGateCell + 16 * oct;  // padded cell of tap (di - 1, -1)
 #pragma unroll
         for (int dj = 0; dj < 3; ++dj) {
           const u32x4_t w = *reinterpret_cast<const u32x4_t*>(rowp + dj * kGateCell);
 #pragma unroll
           for (int m = 0; m < 4; ++m) {
-            if (F16) {
-              asm("v_fma_mix_f32 %0, %1, %2, %0 op_sel:[0,0,0] op_sel_hi:[1,0,0]"
-                  : "+v"(acc[2 * m]) : "v"(w[m]), "v"(wreg[2 * m][di * 3 + dj]));
-              asm("v_fma_mix_f32 %0, %1, %2, %0 op_sel:[1,0,0] op_sel_hi:[1,0,0]"
-                  : "+v"(acc[2 * m + 1]) : "v"(w[m]), "v"(wreg[2 * m + 1][di * 3 + dj]));
-            } else {
-              acc[2 * m] = __builtin_fmaf(bf16lo_to_f32(w[m]), wreg[2 * m][di * 3 + dj], acc[2 * m]);
-              acc[2 * m + 1] = __builtin_fmaf(bf16hi_to_f32(w[m]), wreg[2 * m + 1][di * 3 + dj], acc[2 * m + 1]);
-            }
+            acc[2 * m] = __builtin_fmaf(bf16lo_to_f32(w[m]), wreg[2 * m][di * 3 + dj], acc[2 * m]);
+            acc[2 * m + 1] = __builtin_fmaf(bf16hi_to_f32(w[m]), wreg[2 * m + 1][di * 3 + dj], acc[2 * m + 1]);
           }
           if (di == 1 && dj == 1) ctr = w;
         }
       }
       u32x4_t o;
 #pragma unroll
-      for (int m = 0; m < 4; ++m) {
-        const uint32_t cw = ctr[m];
-        constexpr float unit = F16 ? kGateUnit : 1.0f;
-        const float s0 = __builtin_amdgcn_rcpf(__builtin_fmaf(exp_fast(-acc[2 * m]), unit, unit));  // the sigmoid, a unit-th of it
-        const float s1 = __builtin_amdgcn_rcpf(__builtin_fmaf(exp_fast(-acc[2 * m + 1]), unit, unit));
-        float y0 = bf16lo_to_f32(cw) * s0, y1 = bf16hi_to_f32(cw) * s1;
-        if (F16) {  // the centre values, read as fp16 halves in place
-          asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel:[0,0,0] op_sel_hi:[1,0,0]" : "=v"(y0) : "v"(cw), "v"(s0));
-          asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(y1) : "v"(cw), "v"(s1));
-        }
-        o[m] = pack_bf16x2(y0, y1);
-      }
-      __builtin_amdgcn_raw_buffer_store_b128(o, out, (unsigned)row * 128u + 16u * oct, 0, 0);
+      for (int m = 0; m < 4; ++m)
+        o[m] = pack_bf16x2(bf16lo_to_f32(ctr[m]) * sigmoidf_(acc[2 * m]), bf16hi_to_f32(ctr[m]) * sigmoidf_(acc[2 * m + 1]));
+      __builtin_amdgcn_raw_buffer_store_b128(o, o_rsrc, (unsigned)row * 128u + 16u * oct, 0, 0);
     }
   }
-}
-
-// The outputs are staged as fp16 pairs, so that the stencil's multiply-adds read them in place (v_fma_mix_f32: fp16 x fp32 + fp32,
-// the same fp32 arithmetic as on unpacked values, without the unpacking); 64 times as large, with weights a 64th, so that of bf16
-// values around one hardly any is too small for fp16.  A slab that has one all the same, or a value from 1024 on, a zero or what is no
-// number, is staged again as it is and unpacked.  768 slabs of 14 x 14, Dk 64: 41.2 us, without the look at the values 40.3.  flags: a float
-// per wave, 4 apart.
-__device__ __forceinline__ void locality_gate_epilogue(f32x16_t O0, f32x16_t O1, float os, char* lds, float* flags, const float* gate_w,
-                                                    rsrc_t o_rsrc, int gw, int gh, int ti, int NT, int lane_w) {
-  const f32x16_t O[2] = {O0, O1};
-  const GateGrid g{lds, gw, gh, gw + 2, 1.0f / (float)gw};
-  float* wlds = reinterpret_cast<float*>(lds + g.pw * (gh + 2) * kGateCell);
-  // the head's stencil weights, fetched by the first 144 threads while the other waves finish their walks
-  f32x4_t w4 = {0.f, 0.f, 0.f, 0.f};
-  const bool w_mine = ti * 64 + lane_w < 64 * 9 / 4;
-  if (w_mine) w4 = reinterpret_cast<const f32x4_t*>(gate_w)[ti * 64 + lane_w];
-  lds_barrier();  // every wave is done with the tiles
-  if (w_mine) reinterpret_cast<f32x4_t*>(wlds)[ti * 64 + lane_w] = w4 * (1.0f / kGateUnit);
-  // (workgroups of fewer than three waves: the rest of the 144 pieces)
-  for (int idx = ti * 64 + lane_w + 64 * NT; idx < 64 * 9 / 4; idx += 64 * NT)
-    reinterpret_cast<f32x4_t*>(wlds)[idx] = reinterpret_cast<const f32x4_t*>(gate_w)[idx] * (1.0f / kGateUnit);
-  const bool other = __builtin_amdgcn_ballot_w64(stage_cells<true>(O, os, g, ti, lane_w)) != 0;
-  if (lane_w == 0) flags[4 * ti] = other ? 1.0f : 0.0f;
-  const int oct = lane_w & 7, tl = lane_w >> 3;
-  {  // the border cells, by the whole workgroup: top row, bottom row, then the two ends of every other row
-    const int nborder = 2 * g.pw + 2 * gh;
-    const u32x4_t zero = {0u, 0u, 0u, 0u};
-    for (int bc = ti * 8 + tl; bc < nborder; bc += 8 * NT) {
-      int py, px;
-      if (bc < 2 * g.pw) {
-        py = bc < g.pw ? 0 : gh + 1;
-        px = bc < g.pw ? bc : bc - g.pw;
-      } else {
-        const int j = bc - 2 * g.pw;
-        py = 1 + (j >> 1);
-        px = (j & 1) ? g.pw - 1 : 0;
-      }
-      *reinterpret_cast<u32x4_t*>(g.cells + (py * g.pw + px) * kGateCell + 16 * oct) = zero;
-    }
-  }
-  lds_barrier();  // the slab's outputs, the zero border and the weights are staged
-  const float mine = lane_w < NT ? flags[4 * lane_w] : 0.0f;
-  if (__builtin_expect(__builtin_amdgcn_ballot_w64(mine != 0.0f) == 0, 1)) {
-    gate_stencil<true>(g, wlds, o_rsrc, ti, lane_w);
-    return;
-  }
-  stage_cells<false>(O, os, g, ti, lane_w);  // (nobody reads a cell before the barrier behind this)
-  lds_barrier();
-  gate_stencil<false>(g, wlds, o_rsrc, ti, lane_w);
 }
 
 // The kernel's argument block as the hardware lays it out (every argument at its natural alignment).
@@ -907,7 +851,7 @@ __device__ __forceinline__ void tile_pass(const TileCtx& cx, const TileKernArgs*
   float os = cx.oscale;
   if (GENERAL) os *= __builtin_amdgcn_exp2f((float)(eq + ek + ev));
   if (GATE) {
-    locality_gate_epilogue(O[0], O[1], os, lds, guard, cx.gate_w, cx.o, cx.gw, cx.gh, ti, NT, lane_w);
+    locality_gate_epilogue(O[0], O[1], os, lds, cx.gate_w, cx.o, cx.gw, cx.gh, ti, NT, lane_w);
     return;
   }
   // ---- store: lane (r, h) holds channels [32h, 32h + 32) of token r; rows beyond the sequence are dropped ----

@@ -195,7 +195,6 @@ __device__ __forceinline__ void store_kt(uint16_t* kt, int row, int h, const u32
 // ---- fp16 operands, magnitude guard, split-bf16 operands, LDS units (shared by the forward kernels) ----
 typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
-typedef uint16_t u16x2_t __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ f32x16_t mfma_f16(const u32x4_t& a, const u32x4_t& b, const f32x16_t& c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0,
                                                 0, 0);
