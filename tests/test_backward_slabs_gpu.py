@@ -58,3 +58,28 @@ def test_segments(B, H, L, Dk, both):
     got = vig_amd.gla_bidir_backward(q, k, v, gf, gb, do, out_scale=out)
     n = 5 if both else 4
     _check_mfma(got[:n], [f64(t) for t in want[:n]], q.cpu())
+
+
+@pytest.mark.parametrize("both", [True, False])
+@pytest.mark.parametrize("B,H,L,Dk", [(1, 2, 160, 64), (1, 2, 193, 32), (1, 2, 224, 64), (1, 2, 224, 32), (1, 2, 225, 64), (1, 3, 255, 32)])
+def test_seven_and_eight_tiles(B, H, L, Dk, both):
+    test_lengths(B, H, L, Dk, both)
+
+
+@pytest.mark.parametrize("B,H,L,Dk", [(90, 6, 70, 64), (87, 6, 197, 64), (87, 6, 197, 32), (90, 3, 230, 64), (90, 3, 230, 32)])
+def test_slabs_given_up_in_either_direction(B, H, L, Dk):
+    """Several slabs a workgroup, some beyond the range in their first direction, some in their second (whose loads are then
+    on their way already), some in both: those from the recurrent kernel bit for bit, the rest within the bound."""
+    announce(f"backward slabs, {B * H} of {L} tokens, Dk{Dk}, strong in either direction")
+    q, k, v, gf, gb = (t.cuda() for t in make_gla_inputs(B, H, L, Dk, 64, seed=8, dtype=torch.bfloat16))
+    slab = torch.arange(B * H, device="cuda").reshape(B, H)
+    first, second = slab % 7 == 2, slab % 5 == 1
+    gf = torch.where(first[:, :, None, None], torch.full_like(gf, -4.0), gf)
+    gb = torch.where(second[:, :, None, None], torch.full_like(gb, -4.0), gb)
+    do = _do(v.shape, 4, torch.bfloat16).cuda()
+    exact = vig_amd.gla_bidir_backward(q, k, v, gf, gb, do, out_scale=0.5, exact=True)
+    got = vig_amd.gla_bidir_backward(q, k, v, gf, gb, do, out_scale=0.5)
+    strong = first | second
+    for g, e in zip(got, exact):
+        assert torch.equal(g[strong], e[strong])
+    _check_mfma([g[~strong] for g in got], [f64(e[~strong]) for e in exact], q[~strong].cpu())

@@ -11,17 +11,24 @@
 // s = scale * out_scale.  This is the natural-order form of flash-linear-attention/fla/ops/gla/chunk_fuse.py:413-518
 // with one chunk per sequence; the flip-concat glue of classification/models/vig.py:407-426 never materialises.
 //
-// One persistent workgroup of 8 waves per CU (two of 4, four of 2 for short slabs) walks slabs; wave w owns the 32-token tile w.  Per direction the
-// workgroup stages q~, k~ (and once v, do) as bf16 rows in LDS; then wave w accumulates dq of its tile over the key
-// tiles the direction keeps, and dk, dv of its tile over the query tiles: score tiles P, A come out of the matrix
-// cores in the register layout that feeds the next product directly (mfma_tiles.h), operands with tokens in the
-// contraction slots are read from the LDS rows as dwords.  The two directions take turns in LDS; a tile that is heavy
-// in one direction is light in the other, so over both every wave does the same amount of work.  dg needs a running
-// sum over tokens: inside the tile the lanes (= tokens) add up q dq - k dk by lane shifts, the tile totals are
-// exchanged through LDS.  Loads of the next direction (or slab) are issued before that exchange, when the accumulators
-// are dead (its gates a phase earlier), and its cumulative gates and their tile totals are prepared there as well.
+// One persistent workgroup of 8 (or 7) waves per CU (two of 4, four of 2 for short slabs) walks slabs; wave w owns the 32-token tile w.
+// Per direction the workgroup stages q~, k~ (and once v, do) as bf16 rows in LDS; then wave w accumulates dk, dv of its tile over
+// the query tiles the direction keeps, and dq over the key tiles: score tiles P, A come out of the matrix cores in the
+// register layout that feeds the next product directly (mfma_tiles.h), operands with tokens in the contraction slots are
+// transposed by the LDS reads themselves.  The two directions take turns in LDS; a tile that is heavy in one direction is
+// light in the other, so over both every wave does the same amount of work.  dg needs a running sum over tokens: inside the
+// tile the lanes (= tokens) add up q dq - k dk by lane shifts, the tile totals are exchanged through LDS.  What the next
+// direction (or slab) reads is fetched before this one's results are stored, and its cumulative gates and their tile
+// totals are prepared before the second barrier.
 // Two barriers per direction: staged q~ / k~, and the totals of q dq - k dk together with the next direction's gate
 // totals; the second also tells that nobody reads this direction's staged rows any more.
+//
+// What bounds it (768 slabs of 196 tokens, Dk = 64): a slab's loads and stores come in bursts that all CUs make at the same time (1664
+// bytes a token in all, 49 us at the rate of a large copy), and its products wait for LDS reads with two waves a SIMD.  us, against
+// operands read as dwords and put together by v_perm, dq ahead of dk, dv in loops of their own and the first direction's
+// dq, dk parked in the output tensors: 768 x 196 Dk 64 102 -> 86, Dk 32 74 -> 57; 768 x 256 Dk 64 125 -> 107; 1200 x 128 84 -> 75;
+// 24 x 2305 with the state passes, Dk 32 56.5 -> 50, Dk 64 81 -> 75; 384 x 57, Dk 64 22.6 -> 23.1 (one round of short slabs:
+// 1 / e is made twice).
 //
 // Slabs whose gate totals exceed the anchor's range (|G_total| / 2 * log2(e) > 60 in some channel) are not computed
 // here: the workgroup raises the slab's flag and the token-recurrent kernel, launched afterwards with that flag
@@ -35,22 +42,64 @@ namespace vig {
 namespace {
 
 constexpr int kBwdTiles = 8;  // most 32-token tiles per slab
+// Staged rows are 128 bytes and lie without gaps; the 16-byte piece c of row i is found at place c ^ (i & 7), so that eight rows'
+// pieces c cover every bank (rows padded to 144 bytes do too, but leave no room for `turn`).
+constexpr int kRow = 64;
+__device__ __forceinline__ int row_piece(int row, int c) { return row * kRow + ((c ^ (row & 7)) << 3); }
 // LDS of a workgroup of TW tiles, one wave each
 template <int TW>
 struct BwdLds {
-  static constexpr int mat = TW * 32 * kKtStride * 2;  // one staged (32 TW) x 64 bf16 matrix, 144-byte rows
-  static constexpr int q = 0, k = mat, v = 2 * mat, d_o = 3 * mat;
+  static constexpr int mat = TW * 32 * kRow * 2;  // one staged (32 TW) x 64 bf16 matrix
+  static constexpr int q = 0, d_o = mat, k = 2 * mat, v = 3 * mat;  // (those read together within a 16-bit offset)
   static constexpr int tot = 4 * mat;               // [TW][64] f32: gate totals of the tiles
   static constexpr int off = tot + TW * 64 * 4;     // [TW][64] f32: per wave, (prefix - anchor) of its tile
   static constexpr int dgtot = off + TW * 64 * 4;   // [TW][64] f32: totals of q dq - k dk of the tiles
-  static constexpr int total = dgtot + TW * 64 * 4;
+  // [TW][parked units of 64 lanes x 16 B]: the first direction's dq (Dk = 64) while the second runs, where there is room for it
+  static constexpr int parked = TW == 7 ? 4 : 0;
+  static constexpr int park = dgtot + TW * 64 * 4;
+  static constexpr int turn = park + TW * parked * 1024;  // [TW][16 rows] of results on their way out (store_rows)
+  static constexpr bool turns(int ng) { return ng == 4 && TW >= 4; }
+  static constexpr int total = turn + (turns(4) ? TW * 16 * kRow * 2 : 0);
 };
 constexpr float kBwdHalfRange = 60.0f;
 
 
-// fragment of 8 consecutive channels (k-step ks, lane half h) of a staged row: contraction over channels
-__device__ __forceinline__ u32x4_t row_frag(const uint16_t* mat, int row, int ks, int h) {
-  return *reinterpret_cast<const u32x4_t*>(mat + row * kKtStride + 16 * ks + 8 * h);
+// A lane's row of a staged matrix, as operand fragments of 8 consecutive channels (k-step ks, lane half h): piece 2 ks + h.
+// The addresses stay in registers: what is read around them goes by instruction offsets.
+struct RowPtr {
+  lds_u16_t p[4];
+  __device__ __forceinline__ RowPtr(lds_u16_t mat, int row, int h) {
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      p[ks] = mat + row_piece(row, 2 * ks + h);
+      asm volatile("" : "+v"(p[ks]));
+    }
+  }
+  __device__ __forceinline__ u32x4_t frag(int ks, int off = 0) const {
+    typedef __attribute__((address_space(3))) const u32x4_t lds_u32x4_t;
+    return *(lds_u32x4_t*)(p[ks] + off);
+  }
+  __device__ __forceinline__ void advance(int by) {
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) p[ks] += by;
+  }
+};
+// A lane's address for transposed fragments (tr_frag) of the tile at `mat`: its piece holds one of 16 NG / 4 groups of four channels
+template <int NG>
+__device__ __forceinline__ lds_u16_t tr_ptr(lds_u16_t mat, int lane) {
+  const int row = 4 * (lane >> 5) + ((lane & 15) >> 2), ch = tr_row_channel<NG>(16 * ((lane >> 4) & 1) + 4 * (lane & 3));
+  lds_u16_t at = mat + row_piece(row, ch >> 3) + (ch & 7);
+  asm volatile("" : "+v"(at));
+  return at;
+}
+// the NG pieces of a lane's half row
+template <int NG>
+__device__ __forceinline__ void store_row(uint16_t* mat, int row, int h, const u32x4_t (&x)[NG]) {
+#pragma unroll
+  for (int g = 0; g < NG; ++g) *reinterpret_cast<u32x4_t*>(mat + row_piece(row, NG * h + g)) = x[g];
+}
+__device__ __forceinline__ u32x4_t load_piece(const uint16_t* mat, int row, int c) {
+  return *reinterpret_cast<const u32x4_t*>(mat + row_piece(row, c));
 }
 
 // accumulator tile (rows 8g+4h+m in registers, column = lane) -> operand fragments with its rows in the contraction
@@ -62,18 +111,71 @@ __device__ __forceinline__ void tile_frags(const f32x16_t& T, u32x4_t (&f)[2]) {
     for (int x = 0; x < 4; ++x) f[t][x] = pack_bf16x2(T[8 * t + 2 * x], T[8 * t + 2 * x + 1]);
 }
 
-// keeps the entries of a diagonal tile (diag) the direction uses, and all of any other tile; ROWS_ARE_QUERIES: rows
-// i, column j (else rows j, column i).  Selects, not a branch around them: a branch between the matrix instructions
-// and the first vector read of their result left that read without its wait states in one build of this kernel.
+// keeps the entries of a diagonal tile the direction uses, in its operand fragments; ROWS_ARE_QUERIES: rows i, column j (else rows j,
+// column i).  (On the packed values: a branch between the matrix instructions and the first vector read of their result
+// left that read without its wait states in one build of this kernel.)
 template <bool FWD, bool ROWS_ARE_QUERIES>
-__device__ __forceinline__ void mask_diag(f32x16_t& T, int r, int h, bool diag) {
+__device__ __forceinline__ void mask_diag(u32x4_t (&f)[2], int r, int h) {
+  const uint32_t kept = (FWD == ROWS_ARE_QUERIES ? ~0u << r : ~0u >> (31 - r)) >> (4 * h);  // rows r .. 31, or 0 .. r
+  f[0] &= keep_masks<0>(kept), f[1] &= keep_masks<1>(kept);
+}
+
+// accumulators of a tile's k channels and where channel c8 of octet gq lies in them (tr_row_channel)
+template <int NG>
+struct KeyAcc {
+  f32x16_t a[NG / 2];
+  __device__ __forceinline__ void zero() {
 #pragma unroll
-  for (int c = 0; c < 16; ++c) {
-    const int row = 8 * (c >> 2) + 4 * h + (c & 3);
-    const int i = ROWS_ARE_QUERIES ? row : r, j = ROWS_ARE_QUERIES ? r : row;
-    const bool keep = !diag || (FWD ? (j <= i) : (j >= i));
-    T[c] = keep ? T[c] : 0.f;
+    for (int p = 0; p < NG / 2; ++p) a[p] = f32x16_t{0.f};
   }
+  __device__ __forceinline__ float get(int gq, int c8) const { return NG == 4 ? a[c8 >> 2][4 * gq + (c8 & 3)] : a[0][8 * gq + c8]; }
+};
+
+// dq^ of tile w += the key tile at `v` (rows) and `k` (transposed): A^T = v do^T, rows j, columns i
+template <bool FWD, int NG>
+__device__ __forceinline__ void add_dq(bool diag, const RowPtr& v, lds_u16_t k, const u32x4_t (&doB)[4], int r, int h, KeyAcc<NG>& dq) {
+  f32x16_t T = {0.f};
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) T = mfma(v.frag(ks), doB[ks], T);
+  u32x4_t f[2];
+  tile_frags(T, f);
+  if (diag) mask_diag<FWD, false>(f, r, h);
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int p = 0; p < NG / 2; ++p) dq.a[p] = mfma(tr_frag<kRow>(k + 4 * p, t), f[t], dq.a[p]);
+}
+
+// dv, dk^ of tile w += the query tile at `q` (rows; do's lie `to_do` further), `qt` and `dt` (transposed): P = q~ k~^T,
+// A = do v^T, rows i, columns j
+template <bool FWD, int NG>
+__device__ __forceinline__ void add_dv_dk(bool diag, const RowPtr& q, int to_do, lds_u16_t qt, lds_u16_t dt, const u32x4_t (&kB)[NG],
+                                          const u32x4_t (&vB)[4], int r, int h, f32x16_t (&dv)[2], KeyAcc<NG>& dk) {
+  f32x16_t P = {0.f}, A = {0.f};
+#pragma unroll
+  for (int ks = 0; ks < NG; ++ks) P = mfma(q.frag(ks), kB[ks], P);
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) A = mfma(q.frag(ks, to_do), vB[ks], A);
+  u32x4_t f[2];
+  tile_frags(P, f);
+  if (diag) mask_diag<FWD, true>(f, r, h);
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int p = 0; p < 2; ++p) dv[p] = mfma(tr_frag<kRow>(dt + 4 * p, t), f[t], dv[p]);
+  tile_frags(A, f);
+  if (diag) mask_diag<FWD, true>(f, r, h);
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int p = 0; p < NG / 2; ++p) dk.a[p] = mfma(tr_frag<kRow>(qt + 4 * p, t), f[t], dk.a[p]);
+}
+
+// A copy of the lane id that the compiler does not connect with the others: what is derived from it (rows, offsets) is made
+// again where it is used and does not stay in registers across the phases between.
+__device__ __forceinline__ int fresh_lane(int lane) {
+  asm volatile("" : "+v"(lane));
+  return lane;
 }
 
 // Inclusive running sums over the 32 tokens of a lane half (lanes 32h .. 32h + 31, in lane order) for N values at
@@ -100,6 +202,38 @@ __device__ __forceinline__ void half_prefix_sums(float (&x)[N]) {
 #pragma unroll
   for (int i = 0; i < N; ++i)  // row_bcast:15 into rows 1 and 3 (row mask 0b1010); rows 0 and 2 keep the zero
     x[i] += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x[i]), 0x142, 0xa, 0xf, false));
+}
+
+// the running sum of the token before (lane - 1), nothing for the first of the half
+__device__ __forceinline__ float before_lane(float x, int r) {
+  const float y = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x138, 0xf, 0xf, true));  // wave_shr:1
+  return r == 0 ? 0.f : y;
+}
+
+// A wave's 32 result rows of 16 NG bf16 channels (lane: the NG 16-byte pieces of its half row).  At Dk = 64 16 rows at a time go
+// by way of `turn`, so that a store instruction writes one contiguous KB instead of 64 pieces of 16 bytes in as many 64-byte
+// blocks: 768 slabs of 196 tokens 96.1 -> 90.6 us, 1200 of 128 83.5 -> 77.  Dk = 32 gains nothing by it (58.5, 59.1) and slabs of one
+// or two tiles lose the latency (25.3 against 24.0).
+template <int NG, int TW>
+__device__ __forceinline__ void store_rows(uint16_t* turn, const u32x4_t (&x)[NG], rsrc_t out, int lane) {
+  const int r = lane & 31, h = lane >> 5;
+  if constexpr (!BwdLds<TW>::turns(NG)) {
+#pragma unroll
+    for (int g = 0; g < NG; ++g) __builtin_amdgcn_raw_buffer_store_b128(x[g], out, r * (32u * NG) + h * (16u * NG) + 16u * g, 0, 0);
+  } else {
+    lane = fresh_lane(lane);
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      wave_lds_sync();
+      if ((r >> 4) == half) store_row<NG>(turn, r & 15, h, x);
+      wave_lds_sync();
+#pragma unroll
+      for (int j = 0; j < NG / 2; ++j) {
+        const int piece = 64 * j + lane;
+        __builtin_amdgcn_raw_buffer_store_b128(load_piece(turn, piece / (2 * NG), piece % (2 * NG)), out, 512u * NG * half + 16u * piece, 0, 0);
+      }
+    }
+  }
 }
 
 struct BwdSlab {
@@ -129,17 +263,20 @@ __device__ __forceinline__ void issue_bwd_gate_loads(const BwdNext& n, int w, in
   const int rows = __builtin_amdgcn_readfirstlane(min(max(n.L - 32 * w, 0), 32));  // (scalar: descriptors stay in SGPRs)
   issue_tdwords<0, 2, NG>(chunk_rsrc(n.g + (size_t)32 * w * DK, rows, 2 * DK), r, h, ld.gD);
 }
-template <bool WITH_VDO, int NG>
-__device__ __forceinline__ void issue_bwd_row_loads(const BwdNext& n, int w, int r, int h, BwdLoads<NG>& ld) {
+template <int NG>
+__device__ __forceinline__ void issue_bwd_qk_loads(const BwdNext& n, int w, int r, int h, BwdLoads<NG>& ld) {
   constexpr int DK = 16 * NG;
   const int rows = __builtin_amdgcn_readfirstlane(min(max(n.L - 32 * w, 0), 32));
-  const size_t tk = (size_t)32 * w * DK, tv = (size_t)32 * w * 64;
+  const size_t tk = (size_t)32 * w * DK;
   issue_raw_tile<NG>(chunk_rsrc(n.sl.q + tk, rows, 2 * DK), 0, r, h, ld.rawq);
   issue_raw_tile<NG>(chunk_rsrc(n.sl.k + tk, rows, 2 * DK), 0, r, h, ld.rawk);
-  if (WITH_VDO) {
-    issue_raw_tile<4>(chunk_rsrc(n.sl.v + tv, rows, 128), 0, r, h, ld.rawv);
-    issue_raw_tile<4>(chunk_rsrc(n.sl.d_o + tv, rows, 128), 0, r, h, ld.rawd);
-  }
+}
+template <int NG>
+__device__ __forceinline__ void issue_bwd_vdo_loads(const BwdNext& n, int w, int r, int h, BwdLoads<NG>& ld) {
+  const int rows = __builtin_amdgcn_readfirstlane(min(max(n.L - 32 * w, 0), 32));
+  const size_t tv = (size_t)32 * w * 64;
+  issue_raw_tile<4>(chunk_rsrc(n.sl.v + tv, rows, 128), 0, r, h, ld.rawv);
+  issue_raw_tile<4>(chunk_rsrc(n.sl.d_o + tv, rows, 128), 0, r, h, ld.rawd);
 }
 
 // Tile-local cumulative gates of the direction whose gate dwords have arrived: G^T = g^T T, lane = token, registers =
@@ -168,33 +305,57 @@ __device__ __forceinline__ void bwd_cumulate_gates(const BwdLoads<NG>& ld, int w
   }
 }
 
+// Gates before tile w in walking order, minus the anchor (half the slab total), per channel, from the tile totals that the
+// previous direction's tail (or the kernel's head) left one barrier ago.  False, for every wave alike, where the gates
+// are out of range: same totals in every wave, and nothing has been stored yet.
+template <bool FWD, int NG, int TW>
+__device__ __forceinline__ bool bwd_anchor(int w, int lane, char* lds) {
+  const float* tot = reinterpret_cast<const float*>(lds + BwdLds<TW>::tot) + (lane & (16 * NG - 1));
+  float pre = 0.f, all = 0.f;
+#pragma unroll
+  for (int t = 0; t < TW; ++t) {
+    const float x = tot[t * 64];
+    all += x;
+    pre += (FWD ? (t < w) : (t > w)) ? x : 0.f;
+  }
+  reinterpret_cast<float*>(lds + BwdLds<TW>::off)[w * 64 + lane] = pre - 0.5f * all;
+  const bool in_range = __builtin_amdgcn_ballot_w64(fabsf(all) * (0.5f * kLog2e) > kBwdHalfRange) == 0;
+  wave_lds_sync();
+  return in_range;
+}
+
 // One direction of one slab, for wave w (tile w).  dv accumulates over both directions (raw, unscaled).  The first
-// direction (FIRST, not LAST) stages v and do and parks its dq and dk, rounded to bf16, in the output tensors; the
-// second (LAST, not FIRST) adds its own to them and stores dq, dk, dv.  A one-direction (causal) launch runs a single
-// direction that is both.  Returns false, for every wave alike and before it has stored anything,
-// when the gates are out of range.
+// direction (FIRST, not LAST) stages v and do and hands its dq and dk, rounded to bf16, to the second: in registers, or at
+// Dk = 64, where the loops in between leave no room for dq, in LDS (seven tiles) or parked in the output tensor.  The second
+// (LAST, not FIRST) adds its own to them and stores dq, dk, dv.  A one-direction (causal) launch runs a single direction that
+// is both.  Registers set the order of the phases: dk and dv end before dq begins, and only e of the two factors is kept.
 // SEG: the slab is a segment of a longer sequence.  With S_in the state entering it along the direction, R_out the
 // gradient of the state leaving it, a = half the segment's gate total and ' = times e^a per k channel:
 //   dq^_i += S_in' do_i,   dk^_j += R_out' v_j,   dv_j += R_out'^T k~_j
 // (the e^{G_i - a}, e^{a - G_j} factors applied to dq^, dk^ at the end turn e^a into e^{G_i}, e^{T - G_j}), and the
 // running sum of the gate gradient starts from the total of q dq - k dk over the segments walked later.
 template <bool FWD, bool FIRST, bool LAST, int NG, bool SEG, int TW>
-__device__ __forceinline__ bool bwd_direction(const BwdSlab& sl, int L, int ntiles, int w, int lane, char* lds,
+__device__ __forceinline__ void bwd_direction(const BwdSlab& sl, int L, int ntiles, int w, int lane, char* lds,
                                               float s, f32x16_t (&dv)[2], u32x4_t (&keepq)[NG], u32x4_t (&keepk)[NG],
                                               BwdLoads<NG>& ld, const BwdNext& nxt, f32x16_t (&G)[2]) {
-  // where the first direction's dq, dk (bf16) wait for the second: in registers when the kernel has them to spare
-  // (Dk = 32), else parked in the output tensors
-  constexpr bool kKeepInRegs = NG == 2;
   constexpr bool stage_vdo = FIRST;
+  constexpr int kParkLds = NG == 4 && !(FIRST && LAST) ? BwdLds<TW>::parked : 0;
+  constexpr bool kParkDq = NG == 4 && kParkLds == 0 && !(FIRST && LAST);
+  // Fetched ahead of the dq loop, or, where its registers do not hold that too (a fetched value that is spilled is waited
+  // for at once), behind it: 1200 slabs of 128 tokens, Dk = 64 75 against 82 us with the gates early; 768 of 256 109 against 113
+  // with the rows.
+  constexpr bool kEarlyGates = !(LAST && kParkDq && TW <= 4);
+  constexpr bool kEarlyRows = LAST && (NG == 2 || TW == 7);
   constexpr int DK = 16 * NG;   // channels of q, k and the gates
   constexpr int HC = 8 * NG;    // channels per lane half
-  asm volatile("" : "+v"(lane));  // per-lane constants are rebuilt per direction instead of living across the slab loop
-  const int r = lane & 31, h = lane >> 5;
+  const int lane0 = lane;
+  lane = fresh_lane(lane0);
+  int r = lane & 31, h = lane >> 5;
+  auto next_phase = [&] { lane = fresh_lane(lane0), r = lane & 31, h = lane >> 5; };
   uint16_t* Q = reinterpret_cast<uint16_t*>(lds + BwdLds<TW>::q);
   uint16_t* K = reinterpret_cast<uint16_t*>(lds + BwdLds<TW>::k);
   uint16_t* V = reinterpret_cast<uint16_t*>(lds + BwdLds<TW>::v);
   uint16_t* DO = reinterpret_cast<uint16_t*>(lds + BwdLds<TW>::d_o);
-  float* tot = reinterpret_cast<float*>(lds + BwdLds<TW>::tot);
   float* offs = reinterpret_cast<float*>(lds + BwdLds<TW>::off) + w * 64;
   float* dgtot = reinterpret_cast<float*>(lds + BwdLds<TW>::dgtot);
   const int rows = __builtin_amdgcn_readfirstlane(min(max(L - 32 * w, 0), 32));  // valid tokens of this wave's tile
@@ -203,32 +364,15 @@ __device__ __forceinline__ bool bwd_direction(const BwdSlab& sl, int L, int ntil
   // ---- this tile's loads were issued a phase ago; v and do rows go to LDS once per slab (nobody reads the previous
   // slab's any more; the next barrier makes them visible) ----
   if (stage_vdo) {
-    store_kt<4>(V, 32 * w + r, h, ld.rawv);
-    store_kt<4>(DO, 32 * w + r, h, ld.rawd);
+    store_row<4>(V, 32 * w + r, h, ld.rawv);
+    store_row<4>(DO, 32 * w + r, h, ld.rawd);
   }
   u32x4_t rawq[NG], rawk[NG];
 #pragma unroll
   for (int i = 0; i < NG; ++i) rawq[i] = ld.rawq[i], rawk[i] = ld.rawk[i];
 
-  // ---- the cumulative gates G of this tile and every tile's total were left by the previous direction's tail (or
-  // the kernel's head), one barrier ago ----
-  // lane = channel: gates before this tile in walking order, minus the anchor (half the slab total)
-  bool out_of_range;
-  {
-    float pre = 0.f, all = 0.f;
-#pragma unroll
-    for (int t = 0; t < TW; ++t) {
-      const float x = lane < DK ? tot[t * 64 + lane] : 0.f;
-      all += x;
-      pre += (FWD ? (t < w) : (t > w)) ? x : 0.f;
-    }
-    offs[lane] = pre - 0.5f * all;
-    out_of_range = __builtin_amdgcn_ballot_w64(fabsf(all) * (0.5f * kLog2e) > kBwdHalfRange) != 0;
-  }
-  if (out_of_range) return false;  // same totals in every wave: the whole workgroup leaves together
-  wave_lds_sync();
-  // x = (G - a) * log2(e) per (token, channel): q~ = q 2^x, k~ = k 2^-x
-  f32x16_t x[2] = {{0.f}, {0.f}};
+  // e = e^{G - a} per (token, channel): q~ = q e, k~ = k / e
+  float e[2][4 * NG];
 #pragma unroll
   for (int gq = 0; gq < NG; ++gq) {
     const f32x4_t o0 = *reinterpret_cast<const f32x4_t*>(offs + HC * h + 8 * gq);
@@ -237,7 +381,7 @@ __device__ __forceinline__ bool bwd_direction(const BwdSlab& sl, int L, int ntil
 #pragma unroll
     for (int m = 0; m < 4; ++m)
 #pragma unroll
-      for (int p = 0; p < 2; ++p) x[p][4 * gq + m] = (G[p][4 * gq + m] + o8[2 * m + p]) * kLog2e;
+      for (int p = 0; p < 2; ++p) e[p][4 * gq + m] = exp2_fast((G[p][4 * gq + m] + o8[2 * m + p]) * kLog2e);
   }
   {
     u32x4_t qt[NG], kt[NG];
@@ -246,222 +390,168 @@ __device__ __forceinline__ bool bwd_direction(const BwdSlab& sl, int L, int ntil
 #pragma unroll
       for (int m = 0; m < 4; ++m) {
         const int c = 4 * gq + m;
-        const float e0 = exp2_fast(x[0][c]), e1 = exp2_fast(x[1][c]);
         const uint32_t wq = rawq[gq][m], wk = rawk[gq][m];
-        qt[gq][m] = pack_bf16x2(bf16lo_to_f32(wq) * e0, bf16hi_to_f32(wq) * e1);
-        kt[gq][m] = pack_bf16x2(bf16lo_to_f32(wk) * exp2_fast(-x[0][c]), bf16hi_to_f32(wk) * exp2_fast(-x[1][c]));
+        qt[gq][m] = pack_bf16x2(bf16lo_to_f32(wq) * e[0][c], bf16hi_to_f32(wq) * e[1][c]);
+        kt[gq][m] = pack_bf16x2(bf16lo_to_f32(wk) * __builtin_amdgcn_rcpf(e[0][c]), bf16hi_to_f32(wk) * __builtin_amdgcn_rcpf(e[1][c]));
       }
-    store_kt<NG>(Q, 32 * w + r, h, qt);
-    store_kt<NG>(K, 32 * w + r, h, kt);
+    store_row<NG>(Q, 32 * w + r, h, qt);
+    store_row<NG>(K, 32 * w + r, h, kt);
   }
+  // (only e is kept, not also 1 / e, which is needed again at the end)
+#pragma unroll
+  for (int p = 0; p < 2; ++p)
+#pragma unroll
+    for (int c = 0; c < 4 * NG; ++c) asm volatile("" : "+v"(e[p][c]));
   lds_barrier();  // (2) q~, k~ of every tile visible
 
-  // ---- dq of tile w: over the key tiles J the direction keeps ----
-  f32x16_t dqh[2] = {{0.f}, {0.f}};
+  next_phase();
+  constexpr int kTile = 32 * kRow, kToDo = (BwdLds<TW>::d_o - BwdLds<TW>::q) / 2;
+  const lds_u16_t Qs = (lds_u16_t)Q, Ks = (lds_u16_t)K, Vs = (lds_u16_t)V, Ds = (lds_u16_t)DO;
+  // ---- dv and dk of tile w: over the query tiles I the direction keeps, both in one pass: the two score tiles of a step
+  // are independent, so one's packs run under the other's matrix instructions ----
+  KeyAcc<NG> dkh;
+  dkh.zero();
   if (w < ntiles) {
-    u32x4_t doB[4];
+    u32x4_t kB[NG], vB[4];
+    {
+      const RowPtr k(Ks + w * kTile, r, h);
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) doB[ks] = row_frag(DO, 32 * w + r, ks, h);
-    const int j0 = FWD ? 0 : w, j1 = FWD ? w : ntiles - 1;
-    // Two steps in flight: the score tile of the next key tile is on the matrix cores while this one is masked,
-    // packed and multiplied on (after the last tile the next one is that tile again, computed and dropped).
-    f32x16_t T = {0.f};  // A^T tile: rows j in J, columns i in tile w
+      for (int ks = 0; ks < NG; ++ks) kB[ks] = k.frag(ks);
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) T = mfma(row_frag(V, 32 * j0 + r, ks, h), doB[ks], T);
-#pragma unroll 1
-    for (int J = j0; J <= j1; ++J) {
-      const int Jn = min(J + 1, j1);
-      u32x4_t kf[2][2];
-#pragma unroll
-      for (int t = 0; t < 2; ++t) load_tfrag_lds<NG>(K + 32 * J * kKtStride, t, r, h, kf[t]);
-      f32x16_t Tn = {0.f};
-#pragma unroll
-      for (int ks = 0; ks < 4; ++ks) Tn = mfma(row_frag(V, 32 * Jn + r, ks, h), doB[ks], Tn);
-      mask_diag<FWD, false>(T, r, h, J == w);
-      u32x4_t f[2];
-      tile_frags(T, f);
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        dqh[0] = mfma(kf[t][0], f[t], dqh[0]);
-        dqh[1] = mfma(kf[t][1], f[t], dqh[1]);
-      }
-      T = Tn;
+      for (int ks = 0; ks < 4; ++ks) vB[ks] = k.frag(ks, (BwdLds<TW>::v - BwdLds<TW>::k) / 2);
     }
-    if (SEG) {  // the state entering the segment: rows = the k channels of this lane's accumulator rows, over v
-      const uint16_t* sp = sl.sp + (FWD ? 0 : DK * 64);
-      const bool row_ok = row_has_channel<NG>(r);
-      const int row0 = row_ok ? 2 * cpair<NG>(r) : 0;
-#pragma unroll
-      for (int p = 0; p < 2; ++p)
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-          u32x4_t a = *reinterpret_cast<const u32x4_t*>(sp + (row0 + p) * 64 + 16 * ks + 8 * h);
-          if (NG != 4 && !row_ok) a = u32x4_t{0u, 0u, 0u, 0u};
-          dqh[p] = mfma(a, doB[ks], dqh[p]);
-        }
-    }
-  }
-  // dq^ waits as bf16 pairs while the other accumulators are at work
-  uint32_t dqp[16];
-#pragma unroll
-  for (int c = 0; c < 16; ++c) dqp[c] = pack_bf16x2(dqh[0][c], dqh[1][c]);
-  // the first direction parked its dq and dk (rounded to bf16) in the output tensors; fetch them under the loops
-  const rsrc_t oq = chunk_rsrc(sl.dq + tk, rows, 2 * DK), okk = chunk_rsrc(sl.dk + tk, rows, 2 * DK);
-  u32x4_t prevq[NG], prevk[NG];
-  if (!FIRST && kKeepInRegs) {
-#pragma unroll
-    for (int gq = 0; gq < NG; ++gq) prevq[gq] = keepq[gq], prevk[gq] = keepk[gq];
-  }
-  if (!FIRST && !kKeepInRegs) {
-#pragma unroll
-    for (int gq = 0; gq < NG; ++gq) {
-      const unsigned off = (unsigned)r * (2u * DK) + (2u * HC) * h + 16u * gq;
-      prevq[gq] = __builtin_amdgcn_raw_buffer_load_b128(oq, off, 0, 0);
-      prevk[gq] = __builtin_amdgcn_raw_buffer_load_b128(okk, off, 0, 0);
-    }
-  }
-  // ---- dv and dk of tile w: over the query tiles I the direction keeps.  Dk = 32 has the registers to do both in
-  // one loop: the two score tiles of a step are independent, so one's masks and packs run under the other's matrix
-  // instructions.  Dk = 64: two loops (fewer live registers). ----
-  f32x16_t dkh[2] = {{0.f}, {0.f}};
-  if (w < ntiles) {
-    const int i0 = FWD ? w : 0, i1 = FWD ? ntiles - 1 : w;
-    if constexpr (NG == 2) {
+    const int i0 = FWD ? w : 0, i1 = FWD ? ntiles : w + 1;
+    RowPtr q(Qs + i0 * kTile, r, h);
+    lds_u16_t qt = tr_ptr<NG>(Qs + i0 * kTile, lane), dt = NG == 4 ? qt : tr_ptr<4>(Ds + i0 * kTile, lane);
 #pragma unroll 1
-      for (int I = i0; I <= i1; ++I) {
-        f32x16_t P = {0.f}, A = {0.f};  // rows i in I, columns j in tile w
-#pragma unroll
-        for (int ks = 0; ks < NG; ++ks) P = mfma(row_frag(Q, 32 * I + r, ks, h), row_frag(K, 32 * w + r, ks, h), P);
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) A = mfma(row_frag(DO, 32 * I + r, ks, h), row_frag(V, 32 * w + r, ks, h), A);
-        mask_diag<FWD, true>(P, r, h, I == w);
-        u32x4_t pf[2];
-        tile_frags(P, pf);
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          u32x4_t df[2];
-          load_tfrag_lds<4>(DO + 32 * I * kKtStride, t, r, h, df);
-          dv[0] = mfma(df[0], pf[t], dv[0]);
-          dv[1] = mfma(df[1], pf[t], dv[1]);
-        }
-        mask_diag<FWD, true>(A, r, h, I == w);
-        u32x4_t af[2];
-        tile_frags(A, af);
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          u32x4_t qf[2];
-          load_tfrag_lds<NG>(Q + 32 * I * kKtStride, t, r, h, qf);
-          dkh[0] = mfma(qf[0], af[t], dkh[0]);
-          dkh[1] = mfma(qf[1], af[t], dkh[1]);
-        }
-      }
-    } else {
-#pragma unroll 1
-      for (int I = i0; I <= i1; ++I) {
-        f32x16_t P = {0.f};  // rows i in I, columns j in tile w
-#pragma unroll
-        for (int ks = 0; ks < NG; ++ks) P = mfma(row_frag(Q, 32 * I + r, ks, h), row_frag(K, 32 * w + r, ks, h), P);
-        mask_diag<FWD, true>(P, r, h, I == w);
-        u32x4_t pf[2];
-        tile_frags(P, pf);
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          u32x4_t df[2];
-          load_tfrag_lds<4>(DO + 32 * I * kKtStride, t, r, h, df);
-          dv[0] = mfma(df[0], pf[t], dv[0]);
-          dv[1] = mfma(df[1], pf[t], dv[1]);
-        }
-      }
-#pragma unroll 1
-      for (int I = i0; I <= i1; ++I) {
-        f32x16_t A = {0.f};
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) A = mfma(row_frag(DO, 32 * I + r, ks, h), row_frag(V, 32 * w + r, ks, h), A);
-        mask_diag<FWD, true>(A, r, h, I == w);
-        u32x4_t af[2];
-        tile_frags(A, af);
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          u32x4_t qf[2];
-          load_tfrag_lds<NG>(Q + 32 * I * kKtStride, t, r, h, qf);
-          dkh[0] = mfma(qf[0], af[t], dkh[0]);
-          dkh[1] = mfma(qf[1], af[t], dkh[1]);
-        }
-      }
-    }
+    for (int I = i0; I < i1; ++I, q.advance(kTile), qt += kTile, dt += kTile)
+      add_dv_dk<FWD, NG>(I == w, q, kToDo, qt, NG == 4 ? qt + kToDo : dt, kB, vB, r, h, dv, dkh);
     if (SEG) {  // the gradient of the state leaving the segment, against this tile's k~ rows (dv) and v rows (dk)
-      const uint16_t* rpt = sl.rpt + (FWD ? 0 : DK * 64);
-      const int vrow = 2 * cpair<4>(r);
+      const uint16_t* rpt = sl.rpt + (FWD ? 0 : DK * 64) + tr_row_channel<4>(r) * DK + 8 * h;
 #pragma unroll
       for (int p = 0; p < 2; ++p)
 #pragma unroll
-        for (int ks = 0; ks < NG; ++ks) {
-          const u32x4_t a = *reinterpret_cast<const u32x4_t*>(rpt + (vrow + p) * DK + 16 * ks + 8 * h);
-          dv[p] = mfma(a, row_frag(K, 32 * w + r, ks, h), dv[p]);
-        }
-      const uint16_t* rp = sl.rp + (FWD ? 0 : DK * 64);
-      const bool row_ok = row_has_channel<NG>(r);
-      const int row0 = row_ok ? 2 * cpair<NG>(r) : 0;
+        for (int ks = 0; ks < NG; ++ks)
+          dv[p] = mfma(*reinterpret_cast<const u32x4_t*>(rpt + 4 * p * DK + 16 * ks), kB[ks], dv[p]);
+      const uint16_t* rp = sl.rp + (FWD ? 0 : DK * 64) + tr_row_channel<NG>(r) * 64 + 8 * h;
 #pragma unroll
-      for (int p = 0; p < 2; ++p)
+      for (int p = 0; p < NG / 2; ++p)
 #pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-          u32x4_t a = *reinterpret_cast<const u32x4_t*>(rp + (row0 + p) * 64 + 16 * ks + 8 * h);
-          if (NG != 4 && !row_ok) a = u32x4_t{0u, 0u, 0u, 0u};
-          dkh[p] = mfma(a, row_frag(V, 32 * w + r, ks, h), dkh[p]);
-        }
+        for (int ks = 0; ks < 4; ++ks)
+          dkh.a[p] = mfma(*reinterpret_cast<const u32x4_t*>(rp + 4 * p * 64 + 16 * ks), vB[ks], dkh.a[p]);
     }
   }
-  issue_bwd_gate_loads<NG>(nxt, w, r, h, ld);  // the next direction's gates travel under the rest of this one
-  // ---- scale back; X = q dq - k dk = s (q~ dq^ - k~ dk^): the exponentials cancel, and the staged rows serve ----
-  f32x16_t X[2];
+  next_phase();
+  // ---- dv and dk (which the first direction hands to the second); X = q dq - k dk = s (q~ dq^ - k~ dk^): the exponentials
+  // cancel, and the staged rows serve ----
+  float X[2][4 * NG];
+  uint16_t* turn = reinterpret_cast<uint16_t*>(lds + BwdLds<TW>::turn) + w * 16 * kRow;
+  u32x4_t outv[4];
+  if (LAST) {
+#pragma unroll
+    for (int gq = 0; gq < 4; ++gq)
+#pragma unroll
+      for (int m = 0; m < 4; ++m) outv[gq][m] = pack_bf16x2(dv[m >> 1][4 * gq + 2 * (m & 1)] * s, dv[m >> 1][4 * gq + 2 * (m & 1) + 1] * s);
+  }
   {
-    const rsrc_t ov = chunk_rsrc(sl.dv + tv, rows, 128);
-    if (LAST) {
-#pragma unroll
-      for (int gq = 0; gq < 4; ++gq) {
-        u32x4_t xv;
-#pragma unroll
-        for (int m = 0; m < 4; ++m) xv[m] = pack_bf16x2(dv[0][4 * gq + m] * s, dv[1][4 * gq + m] * s);
-        __builtin_amdgcn_raw_buffer_store_b128(xv, ov, (unsigned)r * 128u + 64u * h + 16u * gq, 0, 0);
-      }
-    }
 #pragma unroll
     for (int gq = 0; gq < NG; ++gq) {
-      const u32x4_t qrow = *reinterpret_cast<const u32x4_t*>(Q + (32 * w + r) * kKtStride + HC * h + 8 * gq);
-      const u32x4_t krow = *reinterpret_cast<const u32x4_t*>(K + (32 * w + r) * kKtStride + HC * h + 8 * gq);
-      u32x4_t xq, xk;
+      const u32x4_t krow = load_piece(K, 32 * w + r, NG * h + gq);
+      u32x4_t xk;
 #pragma unroll
       for (int m = 0; m < 4; ++m) {
         const int c = 4 * gq + m;
-        float a[2], b[2];
+        float b[2];
 #pragma unroll
         for (int p = 0; p < 2; ++p) {
-          const float dqc = p ? bf16hi_to_f32(dqp[c]) : bf16lo_to_f32(dqp[c]);
-          const float dkc = dkh[p][c];
-          const float qt = p ? bf16hi_to_f32(qrow[m]) : bf16lo_to_f32(qrow[m]);
-          const float kt = p ? bf16hi_to_f32(krow[m]) : bf16lo_to_f32(krow[m]);
-          X[p][c] = s * (qt * dqc - kt * dkc);
-          a[p] = s * exp2_fast(x[p][c]) * dqc;
-          b[p] = s * exp2_fast(-x[p][c]) * dkc;
-          if (!FIRST) {
-            a[p] += p ? bf16hi_to_f32(prevq[gq][m]) : bf16lo_to_f32(prevq[gq][m]);
-            b[p] += p ? bf16hi_to_f32(prevk[gq][m]) : bf16lo_to_f32(prevk[gq][m]);
-          }
+          const float dkc = dkh.get(gq, 2 * m + p);
+          X[p][c] = (p ? bf16hi_to_f32(krow[m]) : bf16lo_to_f32(krow[m])) * dkc;
+          b[p] = s * __builtin_amdgcn_rcpf(e[p][c]) * dkc;
+          if (!FIRST) b[p] += p ? bf16hi_to_f32(keepk[gq][m]) : bf16lo_to_f32(keepk[gq][m]);
         }
-        xq[m] = pack_bf16x2(a[0], a[1]);
         xk[m] = pack_bf16x2(b[0], b[1]);
       }
-      const unsigned off = (unsigned)r * (2u * DK) + (2u * HC) * h + 16u * gq;
-      if (!LAST && kKeepInRegs) {
-        keepq[gq] = xq;
-        keepk[gq] = xk;
-      } else {
-        __builtin_amdgcn_raw_buffer_store_b128(xq, oq, off, 0, 0);
-        __builtin_amdgcn_raw_buffer_store_b128(xk, okk, off, 0, 0);
-      }
+      keepk[gq] = xk;
     }
   }
+  __builtin_amdgcn_sched_barrier(0);
+  // The counter that a load is waited for with goes down in the order of issue, stores included: a load behind a store waits for
+  // that store.  So what is stored waits, packed, until what is fetched here is on its way.
+  if (kParkDq && !FIRST) {
+#pragma unroll
+    for (int g = 0; g < NG; ++g)
+      keepq[g] = __builtin_amdgcn_raw_buffer_load_b128(chunk_rsrc(sl.dq + tk, rows, 2 * DK), r * (32u * NG) + h * (16u * NG) + 16u * g, 0, 0);
+  }
+  if (kEarlyGates) issue_bwd_gate_loads<NG>(nxt, w, r, h, ld);
+  if (kEarlyRows) issue_bwd_qk_loads<NG>(nxt, w, r, h, ld);
+  __builtin_amdgcn_sched_barrier(0);
+  if (LAST) {
+    store_rows<4, TW>(turn, outv, chunk_rsrc(sl.dv + tv, rows, 128), lane);
+    store_rows<NG, TW>(turn, keepk, chunk_rsrc(sl.dk + tk, rows, 2 * DK), lane);
+  }
+  next_phase();
+  // ---- dq of tile w: over the key tiles J the direction keeps ----
+  KeyAcc<NG> dqh;
+  dqh.zero();
+  if (w < ntiles) {
+    u32x4_t doB[4];
+    {
+      const RowPtr d(Ds + w * kTile, r, h);
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) doB[ks] = d.frag(ks);
+    }
+    const int j0 = FWD ? 0 : w, j1 = FWD ? w + 1 : ntiles;
+    RowPtr v(Vs + j0 * kTile, r, h);
+    lds_u16_t k = tr_ptr<NG>(Ks + j0 * kTile, lane);
+#pragma unroll 1
+    for (int J = j0; J < j1; ++J, v.advance(kTile), k += kTile) add_dq<FWD, NG>(J == w, v, k, doB, r, h, dqh);
+    if (SEG) {  // the state entering the segment: rows = the k channels of this lane's accumulator rows, over v
+      const uint16_t* sp = sl.sp + (FWD ? 0 : DK * 64) + tr_row_channel<NG>(r) * 64 + 8 * h;
+#pragma unroll
+      for (int p = 0; p < NG / 2; ++p)
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks)
+          dqh.a[p] = mfma(*reinterpret_cast<const u32x4_t*>(sp + 4 * p * 64 + 16 * ks), doB[ks], dqh.a[p]);
+    }
+  }
+  next_phase();
+  if (!FIRST) {
+#pragma unroll
+    for (int g = 0; g < kParkLds; ++g) keepq[g] = *reinterpret_cast<const u32x4_t*>(unit_ptr(lds + BwdLds<TW>::park, w * kParkLds + g, lane));
+  }
+  {
+#pragma unroll
+    for (int gq = 0; gq < NG; ++gq) {
+      const u32x4_t qrow = load_piece(Q, 32 * w + r, NG * h + gq);
+      u32x4_t xq;
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        const int c = 4 * gq + m;
+        float a[2];
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+          const float dqc = dqh.get(gq, 2 * m + p);
+          X[p][c] = s * ((p ? bf16hi_to_f32(qrow[m]) : bf16lo_to_f32(qrow[m])) * dqc - X[p][c]);
+          a[p] = s * e[p][c] * dqc;
+          if (!FIRST) a[p] += p ? bf16hi_to_f32(keepq[gq][m]) : bf16lo_to_f32(keepq[gq][m]);
+        }
+        xq[m] = pack_bf16x2(a[0], a[1]);
+      }
+      keepq[gq] = xq;
+    }
+  }
+  // the next direction's rows travel while this one finishes
+  next_phase();
+  if (!kEarlyGates) issue_bwd_gate_loads<NG>(nxt, w, r, h, ld);
+  if (!kEarlyRows) issue_bwd_qk_loads<NG>(nxt, w, r, h, ld);
+  if (LAST) issue_bwd_vdo_loads<NG>(nxt, w, r, h, ld);
+  next_phase();
+  __builtin_amdgcn_sched_barrier(0);
+  if (!LAST) {
+#pragma unroll
+    for (int g = 0; g < kParkLds; ++g) *reinterpret_cast<u32x4_t*>(unit_ptr(lds + BwdLds<TW>::park, w * kParkLds + g, lane)) = keepq[g];
+  }
+  if (LAST || kParkDq) store_rows<NG, TW>(turn, keepq, chunk_rsrc(sl.dq + tk, rows, 2 * DK), lane);
   // ---- dg: the running sum of X over the tokens the gate acts on.  Inside the tile by lane shifts (lane = token),
   // across tiles through the tile totals in LDS: walking forward a token takes everything from itself to the end,
   // i.e. the totals of this and the later tiles minus what lies before it in the tile. ----
@@ -480,11 +570,10 @@ __device__ __forceinline__ bool bwd_direction(const BwdSlab& sl, int L, int ntil
         dgtot[w * 64 + ch + 1] = pfx[4 * NG + c];
       }
     }
-    // the next direction's rows travel while this one finishes; its cumulative gates and tile totals are prepared
-    // here, so that one barrier serves both exchanges
-    issue_bwd_row_loads<LAST, NG>(nxt, w, r, h, ld);
-    bwd_cumulate_gates<LAST, NG, TW>(ld, w, lane, lds, G);
+    // the next direction's cumulative gates and tile totals are prepared here, so that one barrier serves both exchanges
+    bwd_cumulate_gates<LAST, NG, TW>(ld, w, fresh_lane(lane0), lds, G);
     lds_barrier();  // (4) tile totals of X and of the next gates visible; nobody reads q~, k~, v, do of this direction
+    next_phase();
     {
       const int cl = lane < DK ? lane : 0;
       float run = 0.f;
@@ -501,26 +590,24 @@ __device__ __forceinline__ bool bwd_direction(const BwdSlab& sl, int L, int ntil
     }
     wave_lds_sync();
     uint16_t* dg = FWD ? sl.dgf : sl.dgb;
-    const rsrc_t rdg = chunk_rsrc(dg + tk, rows, 2 * DK);
+    u32x4_t out[NG];
 #pragma unroll
     for (int gq = 0; gq < NG; ++gq) {
       const f32x4_t o0 = *reinterpret_cast<const f32x4_t*>(offs + HC * h + 8 * gq);
       const f32x4_t o1 = *reinterpret_cast<const f32x4_t*>(offs + HC * h + 8 * gq + 4);
       const float o8[8] = {o0[0], o0[1], o0[2], o0[3], o1[0], o1[1], o1[2], o1[3]};
-      u32x4_t out;
 #pragma unroll
       for (int m = 0; m < 4; ++m) {
         const int c = 4 * gq + m;
         float d[2];
 #pragma unroll
         for (int p = 0; p < 2; ++p)
-          d[p] = FWD ? o8[2 * m + p] - (pfx[4 * NG * p + c] - X[p][c]) : o8[2 * m + p] + pfx[4 * NG * p + c];
-        out[m] = pack_bf16x2(d[0], d[1]);
+          d[p] = FWD ? o8[2 * m + p] - before_lane(pfx[4 * NG * p + c], r) : o8[2 * m + p] + pfx[4 * NG * p + c];
+        out[gq][m] = pack_bf16x2(d[0], d[1]);
       }
-      __builtin_amdgcn_raw_buffer_store_b128(out, rdg, (unsigned)r * (2u * DK) + (2u * HC) * h + 16u * gq, 0, 0);
     }
+    store_rows<NG, TW>(turn, out, chunk_rsrc(dg + tk, rows, 2 * DK), lane);
   }
-  return true;
 }
 
 }  // namespace
@@ -570,7 +657,8 @@ __global__ __launch_bounds__(64 * TW, 2) void gla_backward_mfma_kernel(
     const BwdSlab s0 = slab_of(blockIdx.x);
     const BwdNext first{s0, s0.gf, s0.L};
     issue_bwd_gate_loads<NG>(first, w, r, h, ld);
-    issue_bwd_row_loads<true, NG>(first, w, r, h, ld);
+    issue_bwd_qk_loads<NG>(first, w, r, h, ld);
+    issue_bwd_vdo_loads<NG>(first, w, r, h, ld);
     bwd_cumulate_gates<true, NG, TW>(ld, w, lane, lds, G);
     lds_barrier();
   }
@@ -581,25 +669,32 @@ __global__ __launch_bounds__(64 * TW, 2) void gla_backward_mfma_kernel(
     const BwdSlab sn = slab_of(following < nslabs ? following : slab);
     const BwdNext second{sl, sl.gb, sl.L}, next_first{sn, sn.gf, following < nslabs ? sn.L : 0};
     f32x16_t dvacc[2] = {{0.f}, {0.f}};
-    u32x4_t keepq[NG], keepk[NG];
-    bool ok;
-    if constexpr (BIDIR) {
-      ok = bwd_direction<true, true, false, NG, SEG, TW>(sl, sl.L, ntiles, w, lane, lds, s, dvacc, keepq, keepk, ld, second, G);
-      if (ok) {
-        ok = bwd_direction<false, false, true, NG, SEG, TW>(sl, sl.L, ntiles, w, lane, lds, s, dvacc, keepq, keepk, ld,
-                                                        next_first, G);
-      }
-    } else {  // the causal op: the forward direction alone, first and last at once
-      ok = bwd_direction<true, true, true, NG, SEG, TW>(sl, sl.L, ntiles, w, lane, lds, s, dvacc, keepq, keepk, ld,
-                                                    next_first, G);
-    }
-    // a direction that left early has neither issued the loads of the slab that follows nor prepared its gates
-    if (!ok) {
+    // a direction that is not run has neither issued the loads of the slab that follows nor prepared its gates
+    const auto skip = [&] {
+      const int ln = fresh_lane(lane);
       lds_barrier();  // a wave that has left must not touch the gate totals the others still read
-      issue_bwd_gate_loads<NG>(next_first, w, r, h, ld);
-      issue_bwd_row_loads<true, NG>(next_first, w, r, h, ld);
-      bwd_cumulate_gates<true, NG, TW>(ld, w, lane, lds, G);
+      issue_bwd_gate_loads<NG>(next_first, w, ln & 31, ln >> 5, ld);
+      issue_bwd_qk_loads<NG>(next_first, w, ln & 31, ln >> 5, ld);
+      issue_bwd_vdo_loads<NG>(next_first, w, ln & 31, ln >> 5, ld);
+      bwd_cumulate_gates<true, NG, TW>(ld, w, ln, lds, G);
       lds_barrier();
+    };
+    bool ok = bwd_anchor<true, NG, TW>(w, lane, lds);
+    if (ok) {
+      u32x4_t keepq[NG], keepk[NG];
+      if constexpr (BIDIR) {
+        bwd_direction<true, true, false, NG, SEG, TW>(sl, sl.L, ntiles, w, lane, lds, s, dvacc, keepq, keepk, ld, second, G);
+        ok = bwd_anchor<false, NG, TW>(w, lane, lds);
+        if (ok) {
+          bwd_direction<false, false, true, NG, SEG, TW>(sl, sl.L, ntiles, w, lane, lds, s, dvacc, keepq, keepk, ld, next_first, G);
+        } else {
+          skip();  // (in each branch, so that nothing of this slab's loads stays alive for it)
+        }
+      } else {  // the causal op: the forward direction alone, first and last at once
+        bwd_direction<true, true, true, NG, SEG, TW>(sl, sl.L, ntiles, w, lane, lds, s, dvacc, keepq, keepk, ld, next_first, G);
+      }
+    } else {
+      skip();
     }
     if (SEG) {  // one flag per sequence, cleared by the segment scan: any segment out of range gives the sequence away
       if (tid == 0 && !ok) flags[slab / sg.nseg] = 1;
@@ -756,13 +851,16 @@ static int launch_bwd_t(const BwdLaunch& l) {
   return hipGetLastError() == hipSuccess ? 0 : -5;
 }
 // Slabs of up to 64 and up to 128 tokens get workgroups of two and four waves, four and two of them to a CU: in one of eight, the
-// waves without a tile idle and nothing runs beside the loads.  us, eight waves / as many as the slab has tiles: Dk 64: 2010 slabs of
-// 57 tokens 119 / 62, 1200 of 128 113 / 83, 3 of 49 20 / 16; Dk 32: 91 / 37, 82 / 51, 16 / 13.
+// waves without a tile idle and nothing runs beside the loads.  us, eight waves / as many as the slab has tiles (dword operands): Dk 64:
+// 2010 slabs of 57 tokens 119 / 62, 1200 of 128 113 / 83, 3 of 49 20 / 16; Dk 32: 91 / 37, 82 / 51, 16 / 13.  Seven waves instead of
+// eight for 193 to 224 tokens: at Dk 64 the LDS of the eighth tile holds the first
+// direction's dq (768 slabs of 196 tokens, Dk 64 91.4 / 87.1, Dk 32 58.7 / 57.5; of 130, 74.7 / 70.6).
 template <int NG, bool BIDIR>
 static int launch_bwd(const BwdLaunch& l, bool seg, int tokens) {
   if (seg) return tokens <= 128 ? launch_bwd_t<NG, BIDIR, true, 4>(l) : launch_bwd_t<NG, BIDIR, true, 8>(l);
   if (tokens <= 64) return launch_bwd_t<NG, BIDIR, false, 2>(l);
-  return tokens <= 128 ? launch_bwd_t<NG, BIDIR, false, 4>(l) : launch_bwd_t<NG, BIDIR, false, 8>(l);
+  if (tokens <= 128) return launch_bwd_t<NG, BIDIR, false, 4>(l);
+  return tokens <= 224 ? launch_bwd_t<NG, BIDIR, false, 7>(l) : launch_bwd_t<NG, BIDIR, false, 8>(l);
 }
 
 // Where the segments of a call keep what links them: n slots, one per (sequence, segment, direction).
