@@ -74,6 +74,8 @@ SIGNATURES = {
     "vig_linear_bwd_weight_workspace": (_c_size_t, [_c_longlong, _c_int, _c_int]),
     "vig_linear_bwd_weight": (_c_int, [_c_void_p, _c_longlong, _c_void_p, _c_longlong] + [_c_void_p] * 3 +
                               [_c_size_t, _c_longlong, _c_int, _c_int, _c_void_p]),
+    "vig_linear_bwd_weight_many_workspace": (_c_size_t, [_c_longlong, _c_void_p, _c_void_p, _c_int]),
+    "vig_linear_bwd_weight_many": (_c_int, [_c_void_p] * 7 + [_c_size_t, _c_longlong, _c_void_p, _c_void_p, _c_int, _c_void_p]),
     "vig_dirgate_lowrank_bwd": (_c_int, [_c_void_p, _c_longlong] + [_c_void_p] * 6 + [_c_longlong] + [_c_int] * 5 +
                                 [_c_float, _c_float, _c_int, _c_int, _c_void_p]),
     "vig_linear_norm_preferred": (_c_int, [_c_longlong, _c_int, _c_int]),

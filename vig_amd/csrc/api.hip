@@ -76,9 +76,6 @@ int launch_gla_backward(const void* q, const void* k, const void* v, const void*
                         int gate_dtype, bool exact, size_t beyond, hipStream_t stream);
 size_t gla_backward_workspace(int B, int H, int L, int Dk, int Dv, int bidir);  // (launch_gla_backward's; `beyond`: bytes behind it)
 bool linear_wgrad_supported(long long T, int N, int K);
-size_t linear_wgrad_workspace(long long T, int N, int K);
-int launch_linear_wgrad(const void* dy, long long ldy, const void* x, long long ldx, long long T, int N, int K, float* dw,
-                        float* db, void* workspace, hipStream_t stream);
 size_t matmul_f32_workspace(long long M, int N, long long K);
 bool matmul_f32_supported(long long lda, bool ta, long long ldb, bool tb, long long M, int N, long long K);
 int launch_matmul_f32(const float* a, long long lda, bool ta, const float* b, long long ldb, bool tb, const float* bias, const float* add,
@@ -909,18 +906,44 @@ int vig_gla_bidir_bwd_exact(const void* q, const void* k, const void* v, const v
 }
 
 size_t vig_linear_bwd_weight_workspace(long long rows, int N, int K) {
-  return vig::linear_wgrad_supported(rows, N, K) ? vig::linear_wgrad_workspace(rows, N, K) : 0;
+  return vig_linear_bwd_weight_many_workspace(rows, &N, &K, 1);
+}
+
+size_t vig_linear_bwd_weight_many_workspace(long long rows, const int* N, const int* K, int count) {
+  if (!N || !K || count < 1 || count > vig::kWgradLayers) return 0;
+  vig::LinearWgrad l[vig::kWgradLayers] = {};
+  for (int i = 0; i < count; ++i) {
+    if (!vig::linear_wgrad_supported(rows, N[i], K[i])) return 0;
+    l[i].N = N[i], l[i].K = K[i];
+  }
+  return vig::linear_wgrad_workspace(rows, l, count);
 }
 
 int vig_linear_bwd_weight(const void* dy, long long dy_row_stride, const void* x, long long x_row_stride, float* dweight,
                           float* dbias, void* workspace, size_t workspace_bytes, long long rows, int N, int K, void* stream) {
-  if (!dy || !x || !dweight || rows <= 0 || N <= 0 || K <= 0 || dy_row_stride < N || x_row_stride < K) return VIG_EINVAL;
-  if (!vig::linear_wgrad_supported(rows, N, K)) return VIG_ENOTSUP;
-  if (!strided_rows_ok(dy, dy_row_stride, VIG_BF16) || !strided_rows_ok(x, x_row_stride, VIG_BF16) ||
-      !aligned16(dweight, workspace) || (dbias && reinterpret_cast<uintptr_t>(dbias) % 4))
-    return VIG_EINVAL;
-  if (!workspace || workspace_bytes < vig::linear_wgrad_workspace(rows, N, K)) return VIG_ENOSPC;
-  return vig::launch_linear_wgrad(dy, dy_row_stride, x, x_row_stride, rows, N, K, dweight, dbias, workspace, (hipStream_t)stream);
+  return vig_linear_bwd_weight_many(&dy, &dy_row_stride, &x, &x_row_stride, &dweight, &dbias, workspace, workspace_bytes, rows, &N, &K, 1,
+                                    stream);
+}
+
+int vig_linear_bwd_weight_many(const void* const* dy, const long long* dy_row_stride, const void* const* x, const long long* x_row_stride,
+                               float* const* dweight, float* const* dbias, void* workspace, size_t workspace_bytes, long long rows,
+                               const int* N, const int* K, int count, void* stream) {
+  if (!dy || !dy_row_stride || !x || !x_row_stride || !dweight || !N || !K || count < 1 || count > vig::kWgradLayers) return VIG_EINVAL;
+  vig::LinearWgrad l[vig::kWgradLayers] = {};
+  for (int i = 0; i < count; ++i)
+    if (!dy[i] || !x[i] || !dweight[i] || rows <= 0 || N[i] <= 0 || K[i] <= 0 || dy_row_stride[i] < N[i] || x_row_stride[i] < K[i])
+      return VIG_EINVAL;
+  for (int i = 0; i < count; ++i)
+    if (!vig::linear_wgrad_supported(rows, N[i], K[i])) return VIG_ENOTSUP;
+  for (int i = 0; i < count; ++i) {
+    float* const db = dbias ? dbias[i] : nullptr;
+    if (!strided_rows_ok(dy[i], dy_row_stride[i], VIG_BF16) || !strided_rows_ok(x[i], x_row_stride[i], VIG_BF16) ||
+        !aligned16(dweight[i], workspace) || (db && reinterpret_cast<uintptr_t>(db) % 4))
+      return VIG_EINVAL;
+    l[i] = {dy[i], x[i], dy_row_stride[i], x_row_stride[i], dweight[i], db, N[i], K[i]};
+  }
+  if (!workspace || workspace_bytes < vig::linear_wgrad_workspace(rows, l, count)) return VIG_ENOSPC;
+  return vig::launch_linear_wgrad(l, count, rows, workspace, (hipStream_t)stream);
 }
 
 }  // extern "C"

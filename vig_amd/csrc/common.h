@@ -118,6 +118,13 @@ __device__ __forceinline__ float logsigmoidf_(float x) {
 __device__ __forceinline__ void load_to_lds16(const void* p, uint32_t lds_base) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_base), "v"(p) : "memory");
 }
+// (base: wave-uniform; 32-bit byte offset a lane)
+__device__ __forceinline__ void load_to_lds16(const void* base, uint32_t offset, uint32_t lds_base) {
+  const uint64_t b = (uint64_t)base;  // (in scalar registers, also where the compiler worked the address out in vector ones)
+  const uint64_t sb = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b) |
+                      (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(b >> 32)) << 32;
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(offset), "s"(sb) : "memory");
+}
 // at most N vector memory operations (loads and stores, in the order of issue) still out
 template <int N>
 __device__ __forceinline__ void wait_vmem() {

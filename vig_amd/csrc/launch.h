@@ -96,6 +96,17 @@ int launch_gla_states(const GlaArgs& a, int seg_len, int nseg, float* slots, con
 // chains the slots of a state pass in place (gla_segment_scan_kernel, no state in or out), and those of another if there is one
 int launch_gla_segment_scan(float* slots, float* more, int nseq, int nseg, int ndir, int ng, hipStream_t stream);
 
+// Weight and bias gradients of up to kWgradLayers linear layers over the same T bf16 rows (wgrad.hip).
+constexpr int kWgradLayers = 4;
+struct LinearWgrad {
+  const void *dy, *x;
+  long long ldy, ldx;
+  float *dw, *db;  // db may be null
+  int N, K;
+};
+size_t linear_wgrad_workspace(long long T, const LinearWgrad* layers, int count);
+int launch_linear_wgrad(const LinearWgrad* layers, int count, long long T, void* workspace, hipStream_t stream);
+
 // Most tensors one launch_cast_many takes.
 constexpr int kMaxCastJobs = 16;
 

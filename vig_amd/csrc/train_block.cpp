@@ -10,7 +10,7 @@
 //   - q/k/v, gate and low-rank projection are one product over stacked weights (rows padded to a multiple of 128: 35 instead of
 //     62 us at 25088 x 384), their gradients gather into one matrix whose rows the kernels write in place, and one product
 //     returns the input gradient, added to the local branch's in fp32 before it is rounded;
-//   - weight and bias gradients leave vig_linear_bwd_weight as fp32, one launch for the three stacked layers;
+//   - weight and bias gradients leave vig_linear_bwd_weight_many as fp32, one launch for all of a node's layers;
 //   - the up-projection of the gates and its input gradient run inside the gate kernels (bf16), and the depthwise
 //     convolution's three gradients are one kernel.
 // ViG-S, B 128 at 224 px under bf16 autocast, forward and backward on one MI355X: 23.7 -> 12.1 ms.
@@ -103,28 +103,47 @@ bool matmul_f32(const Tensor& a, bool a_across, const Tensor& b, bool b_across, 
   return true;
 }
 
-// dy^T x in fp32 (and the column sums of dy); rows of both may lie in wider matrices
-Tensor weight_grad(const Tensor& dy, const Tensor& x, Tensor* bias_grad) {
-  const int64_t T = dy.size(0), N = dy.size(1), K = x.size(1);
-  if (dy.scalar_type() == at::kFloat) {
-    Tensor dw = at::empty({N, K}, dy.options()), db;
-    if (bias_grad) db = at::empty({N}, dy.options());
-    if (!matmul_f32(dy, true, x, true, nullptr, Tensor(), dw, bias_grad ? fptr(db) : nullptr)) {
-      if (bias_grad) db = dy.sum(0);
-      at::mm_out(dw, dy.t(), x);
+// Weight gradients dy^T x in fp32 (and the column sums of dy) of a node's layers; rows of both may lie in wider matrices.  Those of
+// bf16 rows are gathered and go out together (run), as many as the library takes at once; the tensors handed out are filled then.
+struct WeightGrads {
+  static constexpr int kMost = 4;
+  std::vector<Tensor> keep;
+  const void *dy[kMost], *x[kMost];
+  long long ldy[kMost], ldx[kMost], rows = 0;
+  float *dw[kMost], *db[kMost];
+  int N[kMost], K[kMost], count = 0;
+
+  Tensor add(const Tensor& d, const Tensor& in, Tensor* bias_grad) {
+    const int64_t n = d.size(1), k = in.size(1);
+    if (d.scalar_type() == at::kFloat) {
+      Tensor w = at::empty({n, k}, d.options()), b;
+      if (bias_grad) b = at::empty({n}, d.options());
+      if (!matmul_f32(d, true, in, true, nullptr, Tensor(), w, bias_grad ? fptr(b) : nullptr)) {
+        if (bias_grad) b = d.sum(0);
+        at::mm_out(w, d.t(), in);
+      }
+      if (bias_grad) *bias_grad = b;
+      return w;
     }
-    if (bias_grad) *bias_grad = db;
-    return dw;
+    if (count == kMost) run();
+    Tensor w = at::empty({n, k}, d.options().dtype(at::kFloat));
+    if (bias_grad) *bias_grad = at::empty({n}, w.options());
+    dy[count] = d.data_ptr(), ldy[count] = d.stride(0), x[count] = in.data_ptr(), ldx[count] = in.stride(0);
+    dw[count] = fptr(w), db[count] = bias_grad ? fptr(*bias_grad) : nullptr, N[count] = (int)n, K[count] = (int)k;
+    rows = d.size(0), ++count;
+    keep.insert(keep.end(), {d, in, w});
+    if (bias_grad) keep.push_back(*bias_grad);
+    return w;
   }
-  Tensor dw = at::empty({N, K}, dy.options().dtype(at::kFloat));
-  if (bias_grad) *bias_grad = at::empty({N}, dw.options());
-  const size_t need = vig_linear_bwd_weight_workspace(T, (int)N, (int)K);
-  Tensor ws = bytes_like(need, dy);
-  check_rc(vig_linear_bwd_weight(dy.data_ptr(), dy.stride(0), x.data_ptr(), x.stride(0), fptr(dw),
-                                 bias_grad ? fptr(*bias_grad) : nullptr, ws.data_ptr(), need, T, (int)N, (int)K, stream_of(dy)),
-           "vig_linear_bwd_weight");
-  return dw;
-}
+  void run() {
+    if (!count) return;
+    const size_t need = vig_linear_bwd_weight_many_workspace(rows, N, K, count);
+    Tensor ws = bytes_like(need, keep[0]);
+    check_rc(vig_linear_bwd_weight_many(dy, ldy, x, ldx, dw, db, ws.data_ptr(), need, rows, N, K, count, stream_of(keep[0])),
+             "vig_linear_bwd_weight_many");
+    keep.clear(), count = 0;
+  }
+};
 
 // x w^T (+ bias) for rows x [M, K] (packed ones in bf16), packed w [N, K]
 Tensor product(const Tensor& x, const Tensor& w, const Tensor& bias) {
@@ -327,7 +346,9 @@ struct MixNode : torch::autograd::Function<MixNode> {
     variable_list out(2 + kMixParams + 1);
 
     const Tensor da = grad_rows(grads[0], m.rows, m.C, xs, type);
-    if (wants(kOutW)) out[2 + kOutW] = like_param(weight_grad(da, blend.view({m.rows, m.V}), nullptr), out_w, {m.C, m.V});
+    WeightGrads weights;
+    Tensor dw_out, dw_up, db_up, dw_in, db_in;
+    if (wants(kOutW)) dw_out = weights.add(da, blend.view({m.rows, m.V}), nullptr);
     const Tensor d_blend = input_grad(da, w_out);
     // gradients of the stacked projection's columns, written in place by the three kernels that produce them
     Tensor dz = at::empty({m.rows, m.nz}, opts);
@@ -372,21 +393,19 @@ struct MixNode : torch::autograd::Function<MixNode> {
       Tensor d_low = dz.narrow(1, m.n1, kRank);
       if (!matmul_f32(dx, false, up_w, true, nullptr, Tensor(), d_low)) at::mm_out(d_low, dx, up_w);
     }
-    if (wants(kUpW) || wants(kUpB)) {
-      Tensor db;
-      const Tensor dw = weight_grad(dx, z.narrow(1, m.n1, kRank), &db);
-      out[2 + kUpW] = like_param(dw, up_w, {2 * m.K, kRank});
-      out[2 + kUpB] = like_param(db, up_w, {2 * m.K});
-    }
     const Tensor dzs = dz.narrow(1, 0, m.n2);
-    if (wants(kQkvW) || wants(kGateW) || wants(kGateB) || wants(kLowW)) {
-      Tensor db;
-      const bool bias = wants(kGateB);
-      const Tensor dw = weight_grad(dzs, xs.view({m.rows, m.C}), bias ? &db : nullptr);
-      out[2 + kQkvW] = like_param(dw.narrow(0, 0, m.n0), out_w, {m.n0, m.C});
-      out[2 + kGateW] = like_param(dw.narrow(0, m.n0, m.V), out_w, {m.V, m.C});
-      out[2 + kLowW] = like_param(dw.narrow(0, m.n1, kRank), out_w, {kRank, m.C});
-      if (bias) out[2 + kGateB] = like_param(db.narrow(0, m.n0, m.V), out_w, {m.V});
+    if (wants(kUpW) || wants(kUpB)) dw_up = weights.add(dx, z.narrow(1, m.n1, kRank), &db_up);
+    if (wants(kQkvW) || wants(kGateW) || wants(kGateB) || wants(kLowW))
+      dw_in = weights.add(dzs, xs.view({m.rows, m.C}), wants(kGateB) ? &db_in : nullptr);
+    weights.run();
+    out[2 + kOutW] = like_param(dw_out, out_w, {m.C, m.V});
+    out[2 + kUpW] = like_param(dw_up, up_w, {2 * m.K, kRank});
+    out[2 + kUpB] = like_param(db_up, up_w, {2 * m.K});
+    if (dw_in.defined()) {
+      out[2 + kQkvW] = like_param(dw_in.narrow(0, 0, m.n0), out_w, {m.n0, m.C});
+      out[2 + kGateW] = like_param(dw_in.narrow(0, m.n0, m.V), out_w, {m.V, m.C});
+      out[2 + kLowW] = like_param(dw_in.narrow(0, m.n1, kRank), out_w, {kRank, m.C});
+      if (db_in.defined()) out[2 + kGateB] = like_param(db_in.narrow(0, m.n0, m.V), out_w, {m.V});
     }
     if (m.bf16 || !matmul_f32(dzs, false, w_in, true, nullptr, d_xs, d_xs)) at::addmm_out(d_xs, d_xs, dzs, w_in);
     const bool conv_grads = wants(kConvW) || (off[10] && wants(kConvB));
@@ -461,7 +480,9 @@ struct MlpNode : torch::autograd::Function<MlpNode> {
     const Tensor wg = same ? gate_w : matrix(packed, off[0], 2 * I, C), wd = same ? down_w : matrix(packed, off[1], C, I);
     variable_list out(7);
     const Tensor d_out = grad_rows(grads[0], rows, C, y, type);
-    if (ctx->needs_input_grad(4)) out[4] = like_param(weight_grad(d_out, prod, nullptr), down_w, {C, I});
+    WeightGrads weights;
+    Tensor dw_gate, dw_down;
+    if (ctx->needs_input_grad(4)) dw_down = weights.add(d_out, prod, nullptr);
     Tensor dz = at::empty_like(z);
     // At any number of tokens (us, fused / input gradient and SwiGLU pass): C 192: 1 3.5 / 6.6, 1568 5.0 / 9.2, 25088 28 / 41; C 384: 1 3.9 / 5.8,
     // 1568 8.5 / 13.7, 25088 53 / 72.
@@ -474,7 +495,10 @@ struct MlpNode : torch::autograd::Function<MlpNode> {
       check_rc(vig_swiglu_bwd(z.data_ptr(), d_prod.data_ptr(), dz.data_ptr(), rows, (int)I, dtype_code(z), stream_of(z)),
                "vig_swiglu_bwd");
     }
-    if (ctx->needs_input_grad(3)) out[3] = like_param(weight_grad(dz, y.view({rows, C}), nullptr), gate_w, {2 * I, C});
+    if (ctx->needs_input_grad(3)) dw_gate = weights.add(dz, y.view({rows, C}), nullptr);
+    weights.run();
+    out[3] = like_param(dw_gate, gate_w, {2 * I, C});
+    out[4] = like_param(dw_down, down_w, {C, I});
     const Tensor d_y = type == at::kFloat ? input_grad(dz, wg) : at::mm(dz, wg);
     const auto g = norm_bwd(sum, wide ? fptr(norm_w) : fptr(small), d_y, grads[1], off[3], ctx->needs_input_grad(2),
                             ctx->saved_data["eps"].toDouble());
