@@ -713,25 +713,29 @@ __global__ __launch_bounds__(64 * TW, 2) void gla_backward_mfma_kernel(
 //   carry(s) = rowsum_v(S_out(s) R_out(s)): what q dq - k dk adds up to over the segments walked after s, since a segment's
 //              part, rowsum_v(S_in Q - R_out U), is the difference of two such products and R_out is zero behind the last
 // (bf16 matrices in plain row-major order; carry as two partial sums per channel, over 16 accumulator lanes each).
-// One wave per (sequence, direction, register quad cq, 16 lanes of the passes' register order).  The walks are serial and short,
-// so everything is fetched into LDS in one round trip and the loops stay small: unrolled over segments in registers this
-// kernel took 1 us a segment, its code being read once and cold.  A thread holds the four state elements (k channels c, c+1) x
-// (v columns x, x+1), so that its bf16 results leave as 4-byte words.  Chunks of kScanChunk segments; with more than one,
-// S_out waits in `term` between the walks.
+// One workgroup of two waves per (sequence, direction, register quad cq, 16 lanes of the passes' register order).  The walks are serial
+// and short, so everything is fetched into LDS in one round trip and the loops stay small: unrolled over segments in registers this
+// kernel took 1 us a segment, its code being read once and cold.  The first wave walks S, the second R at the same time, each with the
+// next segment's values on their way out of LDS; what needs both, the carries, comes last, from all threads.  A thread holds the four
+// state elements (k channels c, c+1) x (v columns x, x+1), so that its bf16 results leave as 4-byte words.  Chunks of kScanChunk
+// segments; with more than one the walks follow each other and S_out waits in `term` in between.
+// us, whole backward calls, one wave after the other walk / two: 24 sequences of 2305 tokens, Dk 32 49.2 / 46.6; 3 of 5000 46.5 / 38.5, of 9000, Dk 64
+// (two chunks) 93.3 / 85.3; 12 of 300 27.6 / 27.0.
 constexpr int kScanChunk = 48;
-constexpr int kScanSegFloats = 256 + 256 + 128 + 8;  // U or S_out, Q, products, decays
-__global__ __launch_bounds__(64) void gla_backward_segment_scan_kernel(
+constexpr int kScanSegFloats = 256 + 256 + 8;  // U or S_out, Q or R_out, decays
+__global__ __launch_bounds__(128) void gla_backward_segment_scan_kernel(
     const float* __restrict__ ws_fwd, const float* __restrict__ ws_grad, float* __restrict__ term, uint16_t* __restrict__ sp,
     uint16_t* __restrict__ rp, uint16_t* __restrict__ rpt, float* __restrict__ carry, int* __restrict__ flags, int nseq, int nseg,
     int ndir, int ng, int grad_swapped) {
   extern __shared__ __align__(16) float sh[];
-  const int t = threadIdx.x, cq = blockIdx.y >> 2, quarter = blockIdx.y & 3;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), t = threadIdx.x & 63;
+  const int cq = blockIdx.y >> 2, quarter = blockIdx.y & 3;
   const int seq = blockIdx.x / ndir, dir = blockIdx.x % ndir, gdir = grad_swapped ? 1 - dir : dir;
   if (seq >= nseq) return;
   const int chunk = min(nseg, kScanChunk), nchunks = (nseg + chunk - 1) / chunk;
-  float *F = sh, *Q = F + chunk * 256, *P = Q + chunk * 256, *D = P + chunk * 128;
+  float *F = sh, *Q = F + chunk * 256, *D = Q + chunk * 256;
   const size_t state_elems = 16 * ng * 64;
-  if (blockIdx.y == 0 && t == 0 && dir == 0) flags[seq] = 0;
+  if (blockIdx.y == 0 && threadIdx.x == 0 && dir == 0) flags[seq] = 0;
   const int m = t & 3, lane = 16 * quarter + (t >> 2), h = lane >> 5;
   const int cbase = 8 * ng * h + 8 * cq, ch0 = cbase + 2 * m;  // k channels ch0 (pk = 0), ch0 + 1 (pk = 1)
   const int v0 = 2 * cpair<4>(lane & 31);                        // v columns v0 (pv = 0), v0 + 1 (pv = 1)
@@ -739,77 +743,117 @@ __global__ __launch_bounds__(64) void gla_backward_segment_scan_kernel(
   // lane t fetches 16 bytes (four channels) of unit (pk, pv) = t >> 4: element (pk, pv) of thread t lies at 64 (2 pk + pv) + t
   const int fetched = ((((t >> 4) * 4 + cq) * 64) + 16 * quarter + (t & 15)) * 4;
   auto fetch = [&](const float* from, int d, int i0, int n, float* to) {
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // (what lay there has been read and written)
     for (int i = 0; i < n; ++i) load_to_lds16(from + slot(i0 + i, d) * kGlaStateFloats + fetched, lds_offset(to + i * 256));
   };
   auto fetch_decays = [&](int i0, int n) {
     for (int i = t >> 3; i < n; i += 8) D[8 * i + (t & 7)] = ws_fwd[slot(i0 + i, dir) * kGlaStateFloats + 64 * 64 + cbase + (t & 7)];
   };
   auto kept = [&](int i) { return term + ((slot(i, dir) * ng * 4 + blockIdx.y) * 64 + t) * 4; };
-  float S[4] = {0.f, 0.f, 0.f, 0.f};
-  for (int c = 0; c < nchunks; ++c) {
-    const int i0 = c * chunk, n = min(chunk, nseg - i0);
-    fetch(ws_fwd, dir, i0, n, F);
-    if (nchunks == 1) fetch(ws_grad, gdir, i0, n, Q);
-    fetch_decays(i0, n);
-    wait_vmem<0>();
-    wave_lds_sync();
+  struct Step {
+    float x[4], d[2];
+  };
+  auto step = [&](const float* from, int i) {
+    Step y;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) y.x[j] = from[256 * i + 64 * j + t];
+    y.d[0] = D[8 * i + 2 * m], y.d[1] = D[8 * i + 2 * m + 1];
+    return y;
+  };
+  float S[4] = {0.f, 0.f, 0.f, 0.f}, R[4] = {0.f, 0.f, 0.f, 0.f};
+  auto walk_states = [&](int i0, int n) {
+    Step next = step(F, 0);
+#pragma unroll 1
     for (int i = 0; i < n; ++i) {
+      const Step y = next;
+      next = step(F, min(i + 1, n - 1));
       uint16_t* out = sp + slot(i0 + i, dir) * state_elems + ch0 * 64 + v0;
 #pragma unroll
       for (int pk = 0; pk < 2; ++pk) {
-        const float d = D[8 * i + 2 * m + pk], rd = __builtin_amdgcn_sqrtf(d);
+        const float rd = __builtin_amdgcn_sqrtf(y.d[pk]);
         *reinterpret_cast<uint32_t*>(out + 64 * pk) = pack_bf16x2(rd * S[2 * pk], rd * S[2 * pk + 1]);
 #pragma unroll
         for (int pv = 0; pv < 2; ++pv) {
           const int x = 2 * pk + pv;
-          S[x] = __builtin_fmaf(d, S[x], F[256 * i + 64 * x + t]);
+          S[x] = __builtin_fmaf(y.d[pk], S[x], y.x[x]);
           F[256 * i + 64 * x + t] = S[x];
         }
       }
       if (nchunks > 1) *reinterpret_cast<f32x4_t*>(kept(i0 + i)) = f32x4_t{S[0], S[1], S[2], S[3]};
     }
-  }
-  float R[4] = {0.f, 0.f, 0.f, 0.f};
-  for (int c = nchunks - 1; c >= 0; --c) {
-    const int i0 = c * chunk, n = min(chunk, nseg - i0);
-    if (nchunks > 1) {
-      wave_lds_sync();  // (the chunk before has been read)
-      fetch(ws_grad, gdir, i0, n, Q);
-      fetch_decays(i0, n);
-      for (int i = 0; i < n; ++i) {
-        const f32x4_t x = *reinterpret_cast<const f32x4_t*>(kept(i0 + i));
-#pragma unroll
-        for (int j = 0; j < 4; ++j) F[256 * i + 64 * j + t] = x[j];
-      }
-      wait_vmem<0>();
-      wave_lds_sync();
-    }
+  };
+  auto walk_gradients = [&](int i0, int n) {  // (R_out of a segment takes the place of its Q)
+    Step next = step(Q, n - 1);
+#pragma unroll 1
     for (int i = n - 1; i >= 0; --i) {
+      const Step y = next;
+      next = step(Q, max(i - 1, 0));
       const size_t at = slot(i0 + i, dir) * state_elems;
-      float x[4], q[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) x[j] = F[256 * i + 64 * j + t], q[j] = Q[256 * i + 64 * j + t];
-      const float d[2] = {D[8 * i + 2 * m], D[8 * i + 2 * m + 1]};
-      const float rd[2] = {__builtin_amdgcn_sqrtf(d[0]), __builtin_amdgcn_sqrtf(d[1])};
-      P[128 * i + t] = x[0] * R[0] + x[1] * R[1];
-      P[128 * i + 64 + t] = x[2] * R[2] + x[3] * R[3];
+      const float rd[2] = {__builtin_amdgcn_sqrtf(y.d[0]), __builtin_amdgcn_sqrtf(y.d[1])};
 #pragma unroll
       for (int p = 0; p < 2; ++p) {
         *reinterpret_cast<uint32_t*>(rp + at + (ch0 + p) * 64 + v0) = pack_bf16x2(rd[p] * R[2 * p], rd[p] * R[2 * p + 1]);
         *reinterpret_cast<uint32_t*>(rpt + at + (v0 + p) * 16 * ng + ch0) = pack_bf16x2(rd[0] * R[p], rd[1] * R[2 + p]);
       }
 #pragma unroll
-      for (int j = 0; j < 4; ++j) R[j] = __builtin_fmaf(d[j >> 1], R[j], q[j]);
+      for (int j = 0; j < 4; ++j) {
+        Q[256 * i + 64 * j + t] = R[j];
+        R[j] = __builtin_fmaf(y.d[j >> 1], R[j], y.x[j]);
+      }
     }
-    wave_lds_sync();
-    for (int j = t; j < 8 * n; j += 64) {  // (segment, channel 2 mm + pk): the 16 lanes' products, in a fixed order
+  };
+  // (segment, channel 2 mm + pk): the products of the 16 lanes that hold it, in a fixed order
+  auto carries = [&](int i0, int n) {
+    for (int j = threadIdx.x; j < 8 * n; j += 128) {
       const int i = j >> 3, mm = (j >> 1) & 3, pk = j & 1;
       float acc = 0.f;
 #pragma unroll
-      for (int l = 0; l < 16; ++l) acc += P[128 * i + 64 * pk + 4 * l + mm];
+      for (int l = 0; l < 16; ++l) {
+        const int e = 256 * i + 128 * pk + 4 * ((l + i) & 15) + mm;  // (segments start in different banks)
+        acc += F[e] * Q[e] + F[e + 64] * Q[e + 64];
+      }
       carry[slot(i0 + i, dir) * 128 + 64 * (quarter & 1) + cbase + (j & 7)] = acc;
     }
+  };
+  if (nchunks == 1) {
+    if (wave == 0) fetch(ws_fwd, dir, 0, nseg, F);
+    else fetch(ws_grad, gdir, 0, nseg, Q), fetch_decays(0, nseg);
+    wait_vmem<0>();
+    lds_barrier();
+    if (wave == 0) walk_states(0, nseg);
+    else walk_gradients(0, nseg);
+    lds_barrier();
+    carries(0, nseg);
+    return;
+  }
+  for (int c = 0; c < nchunks; ++c) {
+    const int i0 = c * chunk, n = min(chunk, nseg - i0);
+    if (wave == 0) {
+      fetch(ws_fwd, dir, i0, n, F);
+      fetch_decays(i0, n);
+      wait_vmem<0>();
+      wave_lds_sync();
+      walk_states(i0, n);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // (what lies there has been read and written)
+    }
+  }
+  for (int c = nchunks - 1; c >= 0; --c) {
+    const int i0 = c * chunk, n = min(chunk, nseg - i0);
+    lds_barrier();  // (the chunk before has been read)
+    if (wave == 0) {
+      for (int i = 0; i < n; ++i) {
+        const f32x4_t x = *reinterpret_cast<const f32x4_t*>(kept(i0 + i));
+#pragma unroll
+        for (int j = 0; j < 4; ++j) F[256 * i + 64 * j + t] = x[j];
+      }
+    } else {
+      fetch(ws_grad, gdir, i0, n, Q);
+      fetch_decays(i0, n);
+      wait_vmem<0>();
+      wave_lds_sync();
+      walk_gradients(i0, n);
+    }
+    lds_barrier();
+    carries(i0, n);
   }
 }
 
@@ -947,7 +991,7 @@ int launch_gla_backward_mfma(const void* q, const void* k, const void* v, const 
     static bool done[64] = {};
     if (!allow_lds(reinterpret_cast<const void*>(gla_backward_segment_scan_kernel), kScanChunk * kScanSegFloats * sizeof(float), done)) return -5;
     const int held = sg.nseg < kScanChunk ? sg.nseg : kScanChunk;
-    hipLaunchKernelGGL(gla_backward_segment_scan_kernel, dim3((B * H * ndir + 7) / 8 * 8, 4 * ng), dim3(64),
+    hipLaunchKernelGGL(gla_backward_segment_scan_kernel, dim3((B * H * ndir + 7) / 8 * 8, 4 * ng), dim3(128),
                        held * kScanSegFloats * sizeof(float), stream, r.fwd, r.grad, r.term, r.sp, r.rp, r.rpt, r.carry, flags, B * H,
                        sg.nseg, ndir, ng, (int)(Dk == 64));
     sg.sp = r.sp, sg.rp = r.rp, sg.rpt = r.rpt, sg.carry = r.carry;
