@@ -586,7 +586,9 @@ int launch_blend_linear_t(const void* o, const void* loc, const void* glin, cons
   constexpr size_t lds = (size_t)2 * 32 * (K + 8) * sizeof(uint16_t) + 128 * sizeof(float) + (size_t)(32 * K / 8) * 3 * sizeof(u32x4_t);
   static_assert(lds >= (size_t)NW * kRing * 4096, "the weights' rings fit");
   const long long ntiles_t = (T + 31) / 32;
-  const int grid = ntiles_t < num_cu ? (int)ntiles_t : num_cu;
+  // K 192 leaves room for two workgroups to a CU, which blend and multiply at each other's loads (us, one / two: 32768 tokens 17.8 / 16.4,
+  // 12544 9.7 / 8.9, 25088 16.5 / 15.1, with y kept 17.1 / 15.8, 50176 24.9 / 21.2); at K 384 LDS holds one.
+  const int most = KS == 12 ? 2 * num_cu : num_cu, grid = ntiles_t < most ? (int)ntiles_t : most;
   static bool done[64] = {};
   if (!allow_lds((const void*)blend_linear_kernel<KS, NW, TPW, KEPT>, lds, done)) return -5;
   hipLaunchKernelGGL((blend_linear_kernel<KS, NW, TPW, KEPT>), dim3(grid), dim3(64 * NW), lds, stream, (const uint16_t*)o,
