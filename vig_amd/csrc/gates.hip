@@ -602,11 +602,139 @@ static int launch_stencil(const void* x, const float* wt, const float* bias, voi
   return hipGetLastError() == hipSuccess ? 0 : -5;
 }
 
+// ---------------------------------------------------------------------------
+// The depthwise convolution where there is not enough of it for the staged form above: a thread makes four channels of one column of a
+// band of rows.  It walks down the band with the three cells of a row (its own and the two beside it, which other threads fetch too:
+// the lines are in L1) and three rows of sums under way, the next three rows on their way from memory.  No cell passes LDS and no wave
+// waits for another, except once for the taps' weights, which come by way of LDS (a lane's 36 floats lie 144 bytes apart).  A
+// workgroup: 16 quads of channels (a line of bf16) by 16 columns, counted through bands and images.
+// Sums in the staged form's order, so its bits.
+// ---------------------------------------------------------------------------
+template <typename T> struct Quad;  // four values of a row
+template <> struct Quad<uint16_t> {
+  u32x2_t a;
+  __device__ __forceinline__ void zero() { a = u32x2_t{0u, 0u}; }
+  __device__ __forceinline__ void load(const uint16_t* p) { a = *reinterpret_cast<const u32x2_t*>(p); }
+  __device__ __forceinline__ void unpack(float (&v)[4]) const {
+    v[0] = bf16lo_to_f32(a[0]), v[1] = bf16hi_to_f32(a[0]), v[2] = bf16lo_to_f32(a[1]), v[3] = bf16hi_to_f32(a[1]);
+  }
+  static __device__ __forceinline__ void store(uint16_t* p, const float (&v)[4]) {
+    *reinterpret_cast<u32x2_t*>(p) = u32x2_t{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+  }
+};
+template <> struct Quad<float> {
+  f32x4_t a;
+  __device__ __forceinline__ void zero() { a = f32x4_t{0.f, 0.f, 0.f, 0.f}; }
+  __device__ __forceinline__ void load(const float* p) { a = *reinterpret_cast<const f32x4_t*>(p); }
+  __device__ __forceinline__ void unpack(float (&v)[4]) const { v[0] = a[0], v[1] = a[1], v[2] = a[2], v[3] = a[3]; }
+  static __device__ __forceinline__ void store(float* p, const float (&v)[4]) { *reinterpret_cast<f32x4_t*>(p) = f32x4_t{v[0], v[1], v[2], v[3]}; }
+};
+
+template <typename T>
+__global__ __launch_bounds__(256) void dwconv3x3_columns_kernel(const T* __restrict__ x, const float* __restrict__ wt,
+                                                                const float* __restrict__ bias, T* __restrict__ y, T* __restrict__ pre,
+                                                                int columns, int h, int w, int C, int bands, int band, int silu) {
+  __shared__ __align__(16) float wts[kStencilGroup * 9];
+  const int quad = threadIdx.x & 15, ch = blockIdx.y * kStencilGroup + 4 * quad;
+  const int column = blockIdx.x * 16 + (threadIdx.x >> 4);
+  const bool own = column < columns && ch < C;
+  const int line = column / w, c = column - line * w;  // (image, band)
+  const int img = line / bands, r0 = (line - img * bands) * band;
+  const int r1 = own ? min(r0 + band, h) : r0 - 2;  // (no rows for a thread without a column)
+  const size_t base = ((size_t)img * h * w + c) * C + ch, pitch = (size_t)w * C;
+  Quad<T> cell[3][3];
+  const auto fetch = [&](int row, Quad<T> (&to)[3]) {
+    const bool in = row >= 0 && row <= r1 && row < h;
+    const T* p = x + base + (in ? row * pitch : 0);
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      to[d].zero();
+      if (in && (d == 1 || (d == 0 ? c > 0 : c < w - 1))) to[d].load(p + (d - 1) * C);
+    }
+  };
+#pragma unroll
+  for (int u = 0; u < 3; ++u) fetch(r0 - 1 + u, cell[u]);
+  {
+    const int n = min(kStencilGroup, C - (int)blockIdx.y * kStencilGroup) * 9;  // (a multiple of 72)
+    const float* from = wt + (size_t)blockIdx.y * (kStencilGroup * 9);
+    for (int i = 4 * threadIdx.x; i < n; i += 1024) *reinterpret_cast<f32x4_t*>(wts + i) = *reinterpret_cast<const f32x4_t*>(from + i);
+  }
+  float b[4] = {0.f, 0.f, 0.f, 0.f};
+  if (bias && own) {
+    const f32x4_t v = *reinterpret_cast<const f32x4_t*>(bias + ch);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) b[j] = v[j];
+  }
+  __syncthreads();
+  float k[4][9];
+#pragma unroll
+  for (int i = 0; i < 9; ++i) {
+    const f32x4_t v = *reinterpret_cast<const f32x4_t*>(wts + 36 * quad + 4 * i);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) k[(4 * i + e) / 9][(4 * i + e) % 9] = v[e];
+  }
+  float s0[4] = {0.f, 0.f, 0.f, 0.f}, s1[4] = {b[0], b[1], b[2], b[3]};  // sums of the row above the one at hand, and of its own
+  for (int p0 = r0 - 1; p0 <= r1; p0 += 3) {
+#pragma unroll
+    for (int u = 0; u < 3; ++u) {
+      const int p = p0 + u;
+      if (p > r1) break;
+      float s2[4] = {b[0], b[1], b[2], b[3]};
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        float v[4];
+        cell[u][d].unpack(v);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          s0[j] = __builtin_fmaf(v[j], k[j][6 + d], s0[j]);
+          s1[j] = __builtin_fmaf(v[j], k[j][3 + d], s1[j]);
+          s2[j] = __builtin_fmaf(v[j], k[j][d], s2[j]);
+        }
+      }
+      fetch(p + 3, cell[u]);
+      if (p > r0) {
+        const size_t at = base + (p - 1) * pitch;
+        if (silu) {
+          if (pre) {  // kept for the backward; the activation reads the stored value
+            Quad<T>::store(pre + at, s0);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) s0[j] = Stored<T>::of(s0[j]);
+          }
+#pragma unroll
+          for (int j = 0; j < 4; ++j) s0[j] = s0[j] * sigmoidf_(s0[j]);
+        }
+        Quad<T>::store(y + at, s0);
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) s0[j] = s1[j], s1[j] = s2[j];
+    }
+  }
+}
+
+// The columns form while quads x columns of all images are no more than this.  Beyond, a thread to a column fills the chip without bands, the
+// form is bound by its vector work (a quad's row costs as much around its 36 products as in them) and the staged form's bands of a whole
+// image are quicker.  us, staged / columns, bf16 unless said: C 384 32 x 14 x 14 9.8 / 8.1, 64 images 13.2 / 10.6, 90 (120 k) 15.8 / 12.2, 128
+// (172 k) 17.3 / 19.5, 256 23.3 / 26.0; C 192 128 images (86 k) 11.6 / 9.0, 256 (172 k) 15.1 / 15.7, 8 x 64 x 64 12.8 / 10.3, 3 x 48 x 48 8.0 / 6.2;
+// C 768 64 x 14 x 14 (172 k) 14.8 / 16.0, 10 x 32 x 32 15.2 / 11.8; fp32 C 768 8 x 32 x 32 18.2 / 13.8, C 192 8 x 48 x 48 15.6 / 10.2; one image
+// 14 x 14 4.3 / 3.9.
+constexpr long long kColumnThreads = 150000;
+template <typename T>
+static int launch_dwconv3x3_t(const void* x, const float* wt, const float* bias, void* y, void* pre, int B, int h, int w, int C, int silu,
+                              hipStream_t stream) {
+  const long long threads = (long long)B * w * (C / 4), cells = (long long)B * h * w;
+  if (3 * (w + 2) * kStencilGroup * (int)sizeof(T) > 48 * 1024) return -95;
+  // every batch element is an image of C channels; all images share the C weight channels
+  if (threads > kColumnThreads || cells > (1 << 30)) return launch_stencil<T, false>(x, wt, bias, y, pre, B, h, w, C, 1, C, silu, stream);
+  // bands for two hundred thousand threads, as far as there are rows (8 x 64 x 64, C 192: for half or twice as many 11.2, 11.8 instead of 10.3)
+  const int want = (int)std::min<long long>(h, (200000 + threads - 1) / threads), band = (h + want - 1) / want, bands = (h + band - 1) / band;
+  const int columns = B * bands * w;
+  hipLaunchKernelGGL(dwconv3x3_columns_kernel<T>, dim3((columns + 15) / 16, (C + kStencilGroup - 1) / kStencilGroup), dim3(256), 0, stream,
+                     (const T*)x, wt, bias, (T*)y, (T*)pre, columns, h, w, C, bands, band, silu);
+  return hipGetLastError() == hipSuccess ? 0 : -5;
+}
 int launch_dwconv3x3(const void* x, const float* wt, const float* bias, void* y, void* pre, int B, int h, int w, int C,
                      int silu, int io_dtype, hipStream_t stream) {
-  // every batch element is an image of C channels; all images share the C weight channels
-  if (io_dtype == 0) return launch_stencil<float, false>(x, wt, bias, y, pre, B, h, w, C, 1, C, silu, stream);
-  return launch_stencil<uint16_t, false>(x, wt, bias, y, pre, B, h, w, C, 1, C, silu, stream);
+  return (io_dtype == 0 ? launch_dwconv3x3_t<float> : launch_dwconv3x3_t<uint16_t>)(x, wt, bias, y, pre, B, h, w, C, silu, stream);
 }
 
 int launch_locality_gate(const void* o, const float* wt, void* y, int B, int H, int h, int w, int Dv, int io_dtype,
