@@ -338,9 +338,11 @@ __global__ __launch_bounds__(256) void dirgate_lowrank_mfma_kernel(const uint16_
 // the elementwise pass moved the [B*L, 2*H*Dk] matrix five times.
 // us at 4 / 6 / 8 / 12 waves (a wave per channel tile at most): rows 784, 768 channels 12.5 / 10.7 / 9.1 / 8.4; 4704, 768 13.4 / 11.5 / 10.0 / 9.6;
 // 25088, 384 17.1 / 18.1 / 15.7 / 19.3; 11760, 768 18.7 / 18.9 / 16.0 / 17.5.
+// A form of its own where nothing is clamped, as in the models: whether a gate was, costs two of a value's four transcendental
+// instructions, which were what bound the kernel (25088 rows, 384 15.8 -> 13.0 us; 11760, 768 16.2 -> 12.5; 784, 768 9.1 -> 7.5).
 constexpr int kGateBwdWaves = 8;
 
-template <typename TO>
+template <typename TO, bool CLAMP>
 __global__ __launch_bounds__(64 * kGateBwdWaves) void dirgate_lowrank_bwd_kernel(const uint16_t* __restrict__ low, long long ld,
                                                                   const uint16_t* __restrict__ w1,
                                                                   const uint16_t* __restrict__ w1t,
@@ -392,8 +394,7 @@ __global__ __launch_bounds__(64 * kGateBwdWaves) void dirgate_lowrank_bwd_kernel
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         const float x = Stored<uint16_t>::of(acc[8 * p + j] + bias[p][j]);
-        // (no clamp: clamp_min is NaN and the comparison is false)
-        const bool clamped = logsigmoidf_(x) * inv_norm < clamp_min;
+        const bool clamped = CLAMP && logsigmoidf_(x) * inv_norm < clamp_min;
         e[j] = clamped ? 0.f : g[p][j] * inv_norm * sigmoidf_(-x);
       }
 #pragma unroll
@@ -423,7 +424,7 @@ int launch_dirgate_lowrank_bwd(const void* low, long long ld, const void* w1, co
   if (Dk % 16 != 0 || ntok >= 0x7fffffffLL - 64 || 2LL * H * Dk > (1 << 20)) return -95;
   const dim3 grid((unsigned)((ntok + 31) / 32)), block(64 * std::min(kGateBwdWaves, 2 * H * Dk / 32));
 #define VIG_DLB_CASE(TO)                                                                                             \
-  hipLaunchKernelGGL((dirgate_lowrank_bwd_kernel<TO>), grid, block, 0, stream, (const uint16_t*)low, ld,             \
+  hipLaunchKernelGGL((clamp_min == clamp_min ? dirgate_lowrank_bwd_kernel<TO, true> : dirgate_lowrank_bwd_kernel<TO, false>), grid, block, 0, stream, (const uint16_t*)low, ld,             \
                      (const uint16_t*)w1, (const uint16_t*)w1t, (const uint16_t*)b1, (const TO*)d_out, (uint16_t*)dx, \
                      (uint16_t*)d_low, ldd, ntok, B, L, H, Dk, inv_norm, clamp_min)
   if (out_dtype == 1) VIG_DLB_CASE(uint16_t);
