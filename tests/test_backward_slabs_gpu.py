@@ -66,6 +66,12 @@ def test_seven_and_eight_tiles(B, H, L, Dk, both):
     test_lengths(B, H, L, Dk, both)
 
 
+@pytest.mark.parametrize("both", [True, False])
+@pytest.mark.parametrize("B,H,L", [(1, 2, 65), (1, 1, 80), (2, 3, 96), (1, 2, 97), (90, 6, 95)])
+def test_three_tiles(B, H, L, both):
+    test_lengths(B, H, L, 64, both)
+
+
 @pytest.mark.parametrize("B,H,L,Dk", [(90, 6, 70, 64), (87, 6, 197, 64), (87, 6, 197, 32), (90, 3, 230, 64), (90, 3, 230, 32)])
 def test_slabs_given_up_in_either_direction(B, H, L, Dk):
     """Several slabs a workgroup, some beyond the range in their first direction, some in their second (whose loads are then

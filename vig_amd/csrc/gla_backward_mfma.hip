@@ -55,10 +55,10 @@ struct BwdLds {
   static constexpr int off = tot + TW * 64 * 4;     // [TW][64] f32: per wave, (prefix - anchor) of its tile
   static constexpr int dgtot = off + TW * 64 * 4;   // [TW][64] f32: totals of q dq - k dk of the tiles
   // [TW][parked units of 64 lanes x 16 B]: the first direction's dq (Dk = 64) while the second runs, where there is room for it
-  static constexpr int parked = TW == 7 ? 4 : 0;
+  static constexpr int parked = TW == 7 || TW == 3 ? 4 : 0;
   static constexpr int park = dgtot + TW * 64 * 4;
   static constexpr int turn = park + TW * parked * 1024;  // [TW][16 rows] of results on their way out (store_rows)
-  static constexpr bool turns(int ng) { return ng == 4 && TW >= 4; }
+  static constexpr bool turns(int ng) { return ng == 4 && TW >= 3; }
   static constexpr int total = turn + (turns(4) ? TW * 16 * kRow * 2 : 0);
 };
 constexpr float kBwdHalfRange = 60.0f;
@@ -345,7 +345,7 @@ __device__ __forceinline__ void bwd_direction(const BwdSlab& sl, int L, int ntil
   // for at once), behind it: 1200 slabs of 128 tokens, Dk = 64 75 against 82 us with the gates early; 768 of 256 109 against 113
   // with the rows.
   constexpr bool kEarlyGates = !(LAST && kParkDq && TW <= 4);
-  constexpr bool kEarlyRows = LAST && (NG == 2 || TW == 7);
+  constexpr bool kEarlyRows = LAST && (NG == 2 || TW == 7 || TW == 3);
   constexpr int DK = 16 * NG;   // channels of q, k and the gates
   constexpr int HC = 8 * NG;    // channels per lane half
   const int lane0 = lane;
@@ -898,11 +898,15 @@ static int launch_bwd_t(const BwdLaunch& l) {
 // waves without a tile idle and nothing runs beside the loads.  us, eight waves / as many as the slab has tiles (dword operands): Dk 64:
 // 2010 slabs of 57 tokens 119 / 62, 1200 of 128 113 / 83, 3 of 49 20 / 16; Dk 32: 91 / 37, 82 / 51, 16 / 13.  Seven waves instead of
 // eight for 193 to 224 tokens: at Dk 64 the LDS of the eighth tile holds the first
-// direction's dq (768 slabs of 196 tokens, Dk 64 91.4 / 87.1, Dk 32 58.7 / 57.5; of 130, 74.7 / 70.6).
+// direction's dq (768 slabs of 196 tokens, Dk 64 91.4 / 87.1, Dk 32 58.7 / 57.5; of 130, 74.7 / 70.6).  For the same room three waves
+// instead of four for 65 to 96 tokens at Dk 64: 768 slabs of 70 tokens 39.0 / 36.0, 1200 55.4 / 51.1, 297 27.3 / 26.3, 768 of 96 41.9 / 37.8 (Dk 32
+// has its dq in registers: 23.8 / 23.8).
 template <int NG, bool BIDIR>
 static int launch_bwd(const BwdLaunch& l, bool seg, int tokens) {
   if (seg) return tokens <= 128 ? launch_bwd_t<NG, BIDIR, true, 4>(l) : launch_bwd_t<NG, BIDIR, true, 8>(l);
   if (tokens <= 64) return launch_bwd_t<NG, BIDIR, false, 2>(l);
+  if constexpr (NG == 4)
+    if (tokens <= 96) return launch_bwd_t<NG, BIDIR, false, 3>(l);
   if (tokens <= 128) return launch_bwd_t<NG, BIDIR, false, 4>(l);
   return tokens <= 224 ? launch_bwd_t<NG, BIDIR, false, 7>(l) : launch_bwd_t<NG, BIDIR, false, 8>(l);
 }
