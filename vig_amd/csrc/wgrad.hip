@@ -14,9 +14,10 @@
 // tokens, so an operand fragment needs 8 tokens of one channel: ds_read_b64_tr_b16 hands every lane of a group of sixteen
 // four tokens of its channel out of a 4 x 16 block.  The 32-byte units of a row are swapped among themselves by the row
 // number (the loads fetch them that way), so that the four rows and two units that 32 lanes read lie in different banks.
-// What bounds it: a stage takes twice its matrix time, and neither the LDS (27 % busy), the L2's rate (10 TB/s; 256 x 192 tiles ask
-// for 0.6 of it and take as long), nor the memory's latency (lines touched 4 to 20 stages ahead by a fifth wave: no faster) is
-// what it waits for; fragments read a k-step ahead of their products gave 3 %.
+// What bounds it, at one layer of 2048 x 384 over 25088 rows (63 us): 31 us the loop (1.27 PFLOP/s, what a large product of the library
+// reaches), 11 until the pipes run full, 4 to 7 writing and 7 to 9 adding the partial tiles.  Fragments read a k-step ahead of their
+// products gave 3 %; 128 x 192 and 256 x 192 tiles, which ask the L2 for 0.8 and 0.6 of the operands, 57 to 60 us there and no better where
+// a node's layers share the launch; lines touched 4 to 20 stages ahead by a fifth wave were no faster.
 #include "common.h"
 #include "launch.h"
 #include "mfma_tiles.h"
