@@ -50,6 +50,24 @@ def test_layers_together(T, count):
     _check(dys, xs, *_call(dys, xs, [b for _, _, b in layers]))
 
 
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan")])
+@pytest.mark.parametrize("T", [20, 700])  # one range; several, whose partial sums are added
+@pytest.mark.parametrize("N", [8, 48, 136, 384])  # a part of a block of 32 channels, one and a half, a tile and a rest, whole tiles
+def test_a_channel_keeps_to_itself(N, T, value):
+    """Gradients that overflowed in one channel leave every other channel's sums bit for bit what they are without it."""
+    g = torch.Generator("cuda").manual_seed(N + T)
+    dy, x = (torch.randn(T, n, device="cuda", generator=g).bfloat16() for n in (N, 40))
+    (dw0,), (db0,) = _call([dy], [x], [True])
+    for n in sorted({0, 7, N // 2, N - 8, N - 1}):
+        bad = dy.clone()
+        bad[T // 3, n] = value
+        (dw,), (db,) = _call([bad], [x], [True])
+        others = torch.arange(N, device="cuda") != n
+        assert torch.equal(db[others], db0[others]) and torch.equal(dw[others], dw0[others])
+        assert torch.equal(db[n].nan_to_num(nan=7.0), torch.tensor(value, device="cuda").nan_to_num(nan=7.0))
+        assert not dw[n].isfinite().any()
+
+
 def test_rows_far_apart():  # past 32-bit byte offsets inside a stage
     T, ld, n, k = 40, (1 << 26) + 8, 136, 24
     dy = torch.empty(T * ld, dtype=torch.bfloat16, device="cuda").as_strided((T, n), (ld, 1))
