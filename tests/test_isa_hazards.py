@@ -4,7 +4,11 @@ instruction within a few issue slots of it on ANY control-flow path.
 One build of the backward kernel had a branch between the last matrix instruction of a score tile and the first read
 of its result; the compiler's wait states covered the fall-through path only, and the taken path read half-finished
 sums (wrong gradients for some shapes, no error).  The kernels avoid such branches; this test compiles them to
-assembly (no GPU needed) and walks every path behind every matrix instruction."""
+assembly (no GPU needed) and walks every path behind every matrix instruction.
+
+And no memory instruction may take its address from a scalar register that a vector instruction wrote less than five wait states
+before: the compiler sees to it, except in asm blocks, which it does not look into (load_to_lds16 of common.h)."""
+import functools
 import os
 import re
 import subprocess
@@ -14,7 +18,8 @@ import pytest
 
 from vig_amd import build as B
 
-SOURCES = ["gla_tiles.hip", "gla_mfma.hip", "gla_backward_mfma.hip", "gates.hip", "patch_conv.hip", "linear.hip", "gla_states.hip"]
+SOURCES = ["gla_tiles.hip", "gla_mfma.hip", "gla_backward_mfma.hip", "gates.hip", "patch_conv.hip", "linear.hip", "gla_states.hip",
+           "wgrad.hip"]
 WINDOW = 8  # issue slots behind a 32x32x16 matrix instruction in which its destination must not be read
 
 
@@ -72,6 +77,67 @@ def early_reads(asm: str, window: int = WINDOW):
     return found
 
 
+SCALAR_WAIT = 5  # wait states between a vector instruction's write of a scalar register and a memory instruction's read of it
+VMEM = ("buffer_", "global_", "scratch_", "flat_")
+
+
+def _sregs(text):
+    out = set()
+    for m in re.finditer(r"\bs\[(\d+):(\d+)\]", text):
+        out |= set(range(int(m.group(1)), int(m.group(2)) + 1))
+    for m in re.finditer(r"\bs(\d+)\b", text):
+        out.add(int(m.group(1)))
+    return out
+
+
+def stale_scalars(asm: str):
+    lines = asm.split("\n")
+    labels = {m.group(1): i for i, l in enumerate(lines) if (m := re.match(r"^(\.LBB\w+):", l))}
+    found = []
+    for i, l in enumerate(lines):
+        t = l.strip()
+        dst = _sregs(t.split(",")[0]) if t.startswith("v_") else set()
+        if not dst:
+            continue
+        stack, seen = [(i + 1, 0, frozenset(dst))], set()
+        while stack:
+            k, waited, live = stack.pop()
+            while k < len(lines) and waited < SCALAR_WAIT and live and (k, waited) not in seen:
+                seen.add((k, waited))
+                t = lines[k].split(";")[0].strip()
+                k += 1
+                if not t or t.startswith(".") or t.endswith(":"):
+                    continue
+                op = t.split()[0]
+                if op.startswith(VMEM) and _sregs(t) & live:
+                    found.append((i + 1, l.strip(), k, waited, t))
+                    break
+                if op == "s_endpgm":
+                    break
+                if op.startswith("s_cbranch") and t.split()[1] in labels:
+                    stack.append((labels[t.split()[1]], waited + 1, live))
+                if op == "s_branch":
+                    k = labels.get(t.split()[1], len(lines))
+                if "," in t and op.startswith("s_"):
+                    live = live - _sregs(t.split(",")[0])  # (written anew)
+                waited += int(t.split()[1]) + 1 if op == "s_nop" else 1
+    return found
+
+
+def test_checker_sees_stale_scalars():
+    asm = """
+\tv_readfirstlane_b32 s5, v1
+\tv_readfirstlane_b32 s4, v0
+\t;;#ASMSTART
+\ts_mov_b32 m0, s8
+\ts_nop %d
+\tglobal_load_lds_dwordx4 v3, s[4:5]
+\t;;#ASMEND
+"""
+    assert len(stale_scalars(asm % 0)) == 2 and len(stale_scalars(asm % 2)) == 1 and stale_scalars(asm % 3) == []
+    assert stale_scalars((asm % 0).replace("v_readfirstlane_b32 s5, v1", "s_mov_b32 s5, 0").replace("v_readfirstlane_b32 s4, v0", "s_mov_b32 s4, 0")) == []
+
+
 def test_checker_sees_the_pattern():
     asm = """
 .LBB0_1:
@@ -88,13 +154,31 @@ def test_checker_sees_the_pattern():
     assert early_reads(asm.replace("\ts_cbranch_scc1 .LBB0_3\n", "")) == []
 
 
-@pytest.mark.parametrize("src", SOURCES)
-def test_no_early_read_of_matrix_results(src):
+@functools.lru_cache(maxsize=None)
+def _assembly(src):
     with tempfile.TemporaryDirectory() as tmp:
         out = os.path.join(tmp, src + ".s")
         cmd = [B.HIPCC, *[f for f in B.FLAGS if f != "-fPIC"], "-S", "--cuda-device-only", "-I", B.CSRC,
                os.path.join(B.CSRC, src), "-o", out]
         r = subprocess.run(cmd, capture_output=True, text=True)
         assert r.returncode == 0, r.stderr[-2000:]
-        hits = early_reads(open(out).read())
-    assert hits == [], "\n".join(f"line {a}: {b}  ->  line {c} after {d} slots: {e}" for a, b, c, d, e in hits[:10])
+        return open(out).read()
+
+
+def _report(hits):
+    return "\n".join(f"line {a}: {b}  ->  line {c} after {d} slots: {e}" for a, b, c, d, e in hits[:10])
+
+
+@pytest.mark.parametrize("src", SOURCES)
+def test_no_early_read_of_matrix_results(src):
+    hits = early_reads(_assembly(src))
+    assert hits == [], _report(hits)
+
+
+LDS_LOADS = [f for f in B.SOURCES if "load_to_lds16(" in open(os.path.join(B.CSRC, f)).read()]
+
+
+@pytest.mark.parametrize("src", LDS_LOADS)
+def test_no_stale_scalar_address(src):
+    hits = stale_scalars(_assembly(src))
+    assert hits == [], _report(hits)

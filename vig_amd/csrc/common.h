@@ -118,12 +118,12 @@ __device__ __forceinline__ float logsigmoidf_(float x) {
 __device__ __forceinline__ void load_to_lds16(const void* p, uint32_t lds_base) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_base), "v"(p) : "memory");
 }
-// (base: wave-uniform; 32-bit byte offset a lane)
+// (base: wave-uniform; 32-bit byte offset a lane.)  The base has to come out of scalar arithmetic.  One in vector registers does not
+// assemble; one that v_readfirstlane has just brought over may be read as a load's address five wait states later at the earliest, which the
+// compiler sees to between its own instructions, but not into an asm block, where there are two: tests/test_isa_hazards.py goes through
+// the compiled callers for that.  (Five wait states in here cost the weight gradients 1 %: 25088 rows, 2048 x 384 67.2 -> 68.0 us.)
 __device__ __forceinline__ void load_to_lds16(const void* base, uint32_t offset, uint32_t lds_base) {
-  const uint64_t b = (uint64_t)base;  // (in scalar registers, also where the compiler worked the address out in vector ones)
-  const uint64_t sb = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b) |
-                      (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(b >> 32)) << 32;
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(offset), "s"(sb) : "memory");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(offset), "s"(base) : "memory");
 }
 // at most N vector memory operations (loads and stores, in the order of issue) still out
 template <int N>
