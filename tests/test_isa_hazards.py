@@ -7,7 +7,10 @@ sums (wrong gradients for some shapes, no error).  The kernels avoid such branch
 assembly (no GPU needed) and walks every path behind every matrix instruction.
 
 And no memory instruction may take its address from a scalar register that a vector instruction wrote less than five wait states
-before: the compiler sees to it, except in asm blocks, which it does not look into (load_to_lds16 of common.h)."""
+before: the compiler sees to it, except in asm blocks, which it does not look into (load_to_lds16 of common.h).
+
+And the bf16 backward reloads no spilled register between the end of a direction and the staging of the next: the counter a reload is
+waited for with goes down in the order of issue, so that it waits for everything the wave has just stored (3 to 6 % of a call)."""
 import functools
 import os
 import re
@@ -154,6 +157,17 @@ def test_checker_sees_the_pattern():
     assert early_reads(asm.replace("\ts_cbranch_scc1 .LBB0_3\n", "")) == []
 
 
+def reloads_while_staging(asm: str, kernels: str):
+    """(kernel, reload) for every reload between two barriers around a direction's factors, 32 exponentials and more."""
+    found, seen = [], 0
+    for name, body in re.findall(rf"^({kernels}\w*):[^\n]*\n(.*?)^\.Lfunc_end", asm, re.S | re.M):
+        for part in re.split(r"^\ts_barrier", body, flags=re.M):
+            if part.count("v_exp_f32") >= 32:
+                seen += 1
+                found += [(name, l.strip()) for l in part.split("\n") if "scratch_load" in l]
+    return found, seen
+
+
 @functools.lru_cache(maxsize=None)
 def _assembly(src):
     with tempfile.TemporaryDirectory() as tmp:
@@ -182,3 +196,9 @@ LDS_LOADS = [f for f in B.SOURCES if "load_to_lds16(" in open(os.path.join(B.CSR
 def test_no_stale_scalar_address(src):
     hits = stale_scalars(_assembly(src))
     assert hits == [], _report(hits)
+
+
+def test_no_reload_between_the_directions():
+    # whole sequences, 64 key channels, both directions: two to eight waves
+    found, seen = reloads_while_staging(_assembly("gla_backward_mfma.hip"), r"_ZN3vig24gla_backward_mfma_kernelILi4ELb1ELb0ELi[23478]E")
+    assert seen == 10 and found == []

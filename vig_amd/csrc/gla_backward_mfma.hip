@@ -11,7 +11,8 @@
 // s = scale * out_scale.  This is the natural-order form of flash-linear-attention/fla/ops/gla/chunk_fuse.py:413-518
 // with one chunk per sequence; the flip-concat glue of classification/models/vig.py:407-426 never materialises.
 //
-// One persistent workgroup of 8 (or 7) waves per CU (two of 4, four of 2 for short slabs) walks slabs; wave w owns the 32-token tile w.
+// One persistent workgroup of 8 or 7 waves per CU (for short slabs two of 4 or, at Dk 64, 3, four of 2) walks slabs; wave w owns the 32-token
+// tile w.
 // Per direction the workgroup stages q~, k~ (and once v, do) as bf16 rows in LDS; then wave w accumulates dk, dv of its tile over
 // the query tiles the direction keeps, and dq over the key tiles: score tiles P, A come out of the matrix cores in the
 // register layout that feeds the next product directly (mfma_tiles.h), operands with tokens in the contraction slots are
@@ -23,12 +24,12 @@
 // Two barriers per direction: staged q~ / k~, and the totals of q dq - k dk together with the next direction's gate
 // totals; the second also tells that nobody reads this direction's staged rows any more.
 //
-// What bounds it (768 slabs of 196 tokens, Dk = 64): a slab's loads and stores come in bursts that all CUs make at the same time (1664
-// bytes a token in all, 49 us at the rate of a large copy), and its products wait for LDS reads with two waves a SIMD.  us, against
-// operands read as dwords and put together by v_perm, dq ahead of dk, dv in loops of their own and the first direction's
-// dq, dk parked in the output tensors: 768 x 196 Dk 64 102 -> 86, Dk 32 74 -> 57; 768 x 256 Dk 64 125 -> 107; 1200 x 128 84 -> 75;
-// 24 x 2305 with the state passes, Dk 32 56.5 -> 50, Dk 64 81 -> 75; 384 x 57, Dk 64 22.6 -> 23.1 (one round of short slabs:
-// 1 / e is made twice).
+// What bounds it (768 slabs of 196 tokens, Dk = 64): a slab's loads and stores come in bursts that all CUs make at the same time (a token
+// asks for 1664 bytes, q and k in either direction, 49 us at the rate of a large copy; 1864 pass the memory, what fifteen spilled registers write
+// among them), and its products wait for LDS reads with two waves a SIMD.  us, whole calls one behind the other, the flag pass with them, against operands read as dwords and
+// put together by v_perm, dq ahead of dk, dv in loops of their own and the first direction's dq, dk parked in the output tensors:
+// 768 x 196 Dk 64 104 -> 87, Dk 32 74 -> 57; 768 x 256 Dk 64 124 -> 106; 1200 x 128 84 -> 71; 24 x 2305 with the state passes, Dk 32 57 -> 47.5,
+// Dk 64 82 -> 73; 384 x 57 Dk 64 23.7 -> 23.1, 600 x 64, where the second 1 / e tells most, 27.1 -> 27.4.
 //
 // Slabs whose gate totals exceed the anchor's range (|G_total| / 2 * log2(e) > 60 in some channel) are not computed
 // here: the workgroup raises the slab's flag and the token-recurrent kernel, launched afterwards with that flag
@@ -171,11 +172,22 @@ __device__ __forceinline__ void add_dv_dk(bool diag, const RowPtr& q, int to_do,
     for (int p = 0; p < NG / 2; ++p) dk.a[p] = mfma(tr_frag<kRow>(qt + 4 * p, t), f[t], dk.a[p]);
 }
 
-// A copy of the lane id that the compiler does not connect with the others: what is derived from it (rows, offsets) is made
-// again where it is used and does not stay in registers across the phases between.
-__device__ __forceinline__ int fresh_lane(int lane) {
+// The lane id, counted where it is asked for, in a copy that the compiler does not connect with the others: what is derived from it (rows,
+// offsets) does not stay in registers across the phases between, and neither does the id.  Kept, it was spilled, and reloaded behind the stores
+// that end a direction: the counter a load is waited for with goes down in the order of issue, so the wave waited for all it had just
+// stored.  (With tile_rows, us: 768 slabs of 49 tokens, Dk 64 27.4 -> 25.8, of 65 37.3 -> 36.1, of 128 51.5 -> 47.2; one of 128 20.0 -> 19.2.)
+__device__ __forceinline__ int fresh_lane() {
+  uint32_t lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0));
   asm volatile("" : "+v"(lane));
-  return lane;
+  return (int)lane;
+}
+
+// Valid tokens of tile w of a slab of L, by scalar instructions: a two-sided clamp becomes one vector instruction, whose result was kept from
+// slab to slab, spilled and reloaded like the lane id.
+__device__ __forceinline__ int tile_rows(int L, int w) {
+  int n = max(L - 32 * w, 0);
+  asm volatile("" : "+s"(n));
+  return min(n, 32);
 }
 
 // Inclusive running sums over the 32 tokens of a lane half (lanes 32h .. 32h + 31, in lane order) for N values at
@@ -221,7 +233,7 @@ __device__ __forceinline__ void store_rows(uint16_t* turn, const u32x4_t (&x)[NG
 #pragma unroll
     for (int g = 0; g < NG; ++g) __builtin_amdgcn_raw_buffer_store_b128(x[g], out, r * (32u * NG) + h * (16u * NG) + 16u * g, 0, 0);
   } else {
-    lane = fresh_lane(lane);
+    lane = fresh_lane();
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
       wave_lds_sync();
@@ -260,20 +272,20 @@ struct BwdNext {  // the direction whose loads are issued while this one finishe
 template <int NG>
 __device__ __forceinline__ void issue_bwd_gate_loads(const BwdNext& n, int w, int r, int h, BwdLoads<NG>& ld) {
   constexpr int DK = 16 * NG;
-  const int rows = __builtin_amdgcn_readfirstlane(min(max(n.L - 32 * w, 0), 32));  // (scalar: descriptors stay in SGPRs)
+  const int rows = tile_rows(n.L, w);
   issue_tdwords<0, 2, NG>(chunk_rsrc(n.g + (size_t)32 * w * DK, rows, 2 * DK), r, h, ld.gD);
 }
 template <int NG>
 __device__ __forceinline__ void issue_bwd_qk_loads(const BwdNext& n, int w, int r, int h, BwdLoads<NG>& ld) {
   constexpr int DK = 16 * NG;
-  const int rows = __builtin_amdgcn_readfirstlane(min(max(n.L - 32 * w, 0), 32));
+  const int rows = tile_rows(n.L, w);
   const size_t tk = (size_t)32 * w * DK;
   issue_raw_tile<NG>(chunk_rsrc(n.sl.q + tk, rows, 2 * DK), 0, r, h, ld.rawq);
   issue_raw_tile<NG>(chunk_rsrc(n.sl.k + tk, rows, 2 * DK), 0, r, h, ld.rawk);
 }
 template <int NG>
 __device__ __forceinline__ void issue_bwd_vdo_loads(const BwdNext& n, int w, int r, int h, BwdLoads<NG>& ld) {
-  const int rows = __builtin_amdgcn_readfirstlane(min(max(n.L - 32 * w, 0), 32));
+  const int rows = tile_rows(n.L, w);
   const size_t tv = (size_t)32 * w * 64;
   issue_raw_tile<4>(chunk_rsrc(n.sl.v + tv, rows, 128), 0, r, h, ld.rawv);
   issue_raw_tile<4>(chunk_rsrc(n.sl.d_o + tv, rows, 128), 0, r, h, ld.rawd);
@@ -309,7 +321,8 @@ __device__ __forceinline__ void bwd_cumulate_gates(const BwdLoads<NG>& ld, int w
 // previous direction's tail (or the kernel's head) left one barrier ago.  False, for every wave alike, where the gates
 // are out of range: same totals in every wave, and nothing has been stored yet.
 template <bool FWD, int NG, int TW>
-__device__ __forceinline__ bool bwd_anchor(int w, int lane, char* lds) {
+__device__ __forceinline__ bool bwd_anchor(int w, char* lds) {
+  const int lane = fresh_lane();
   const float* tot = reinterpret_cast<const float*>(lds + BwdLds<TW>::tot) + (lane & (16 * NG - 1));
   float pre = 0.f, all = 0.f;
 #pragma unroll
@@ -335,7 +348,7 @@ __device__ __forceinline__ bool bwd_anchor(int w, int lane, char* lds) {
 // (the e^{G_i - a}, e^{a - G_j} factors applied to dq^, dk^ at the end turn e^a into e^{G_i}, e^{T - G_j}), and the
 // running sum of the gate gradient starts from the total of q dq - k dk over the segments walked later.
 template <bool FWD, bool FIRST, bool LAST, int NG, bool SEG, int TW>
-__device__ __forceinline__ void bwd_direction(const BwdSlab& sl, int L, int ntiles, int w, int lane, char* lds,
+__device__ __forceinline__ void bwd_direction(const BwdSlab& sl, int L, int ntiles, int w, char* lds,
                                               float s, f32x16_t (&dv)[2], u32x4_t (&keepq)[NG], u32x4_t (&keepk)[NG],
                                               BwdLoads<NG>& ld, const BwdNext& nxt, f32x16_t (&G)[2]) {
   constexpr bool stage_vdo = FIRST;
@@ -348,17 +361,16 @@ __device__ __forceinline__ void bwd_direction(const BwdSlab& sl, int L, int ntil
   constexpr bool kEarlyRows = LAST && (NG == 2 || TW == 7 || TW == 3);
   constexpr int DK = 16 * NG;   // channels of q, k and the gates
   constexpr int HC = 8 * NG;    // channels per lane half
-  const int lane0 = lane;
-  lane = fresh_lane(lane0);
+  int lane = fresh_lane();
   int r = lane & 31, h = lane >> 5;
-  auto next_phase = [&] { lane = fresh_lane(lane0), r = lane & 31, h = lane >> 5; };
+  auto next_phase = [&] { lane = fresh_lane(), r = lane & 31, h = lane >> 5; };
   uint16_t* Q = reinterpret_cast<uint16_t*>(lds + BwdLds<TW>::q);
   uint16_t* K = reinterpret_cast<uint16_t*>(lds + BwdLds<TW>::k);
   uint16_t* V = reinterpret_cast<uint16_t*>(lds + BwdLds<TW>::v);
   uint16_t* DO = reinterpret_cast<uint16_t*>(lds + BwdLds<TW>::d_o);
   float* offs = reinterpret_cast<float*>(lds + BwdLds<TW>::off) + w * 64;
   float* dgtot = reinterpret_cast<float*>(lds + BwdLds<TW>::dgtot);
-  const int rows = __builtin_amdgcn_readfirstlane(min(max(L - 32 * w, 0), 32));  // valid tokens of this wave's tile
+  const int rows = tile_rows(L, w);  // valid tokens of this wave's tile
   const size_t tk = (size_t)32 * w * DK, tv = (size_t)32 * w * 64;
 
   // ---- this tile's loads were issued a phase ago; v and do rows go to LDS once per slab (nobody reads the previous
@@ -571,7 +583,7 @@ __device__ __forceinline__ void bwd_direction(const BwdSlab& sl, int L, int ntil
       }
     }
     // the next direction's cumulative gates and tile totals are prepared here, so that one barrier serves both exchanges
-    bwd_cumulate_gates<LAST, NG, TW>(ld, w, fresh_lane(lane0), lds, G);
+    bwd_cumulate_gates<LAST, NG, TW>(ld, w, fresh_lane(), lds, G);
     lds_barrier();  // (4) tile totals of X and of the next gates visible; nobody reads q~, k~, v, do of this direction
     next_phase();
     {
@@ -627,9 +639,7 @@ __global__ __launch_bounds__(64 * TW, 2) void gla_backward_mfma_kernel(
     uint16_t* __restrict__ dq, uint16_t* __restrict__ dk, uint16_t* __restrict__ dv, uint16_t* __restrict__ dgf,
     uint16_t* __restrict__ dgb, int* __restrict__ flags, int nslabs, int L, float s, BwdSegments sg) {
   extern __shared__ __align__(16) char lds[];
-  const int tid = threadIdx.x;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   // slab i: a whole sequence, or (SEG) segment i % nseg of sequence i / nseg
   auto slab_of = [&](int i) {
     size_t t0 = (size_t)i * L;
@@ -650,10 +660,10 @@ __global__ __launch_bounds__(64 * TW, 2) void gla_backward_mfma_kernel(
     sl.L = len;
     return sl;
   };
-  const int r = lane & 31, h = lane >> 5;
   BwdLoads<NG> ld;
   f32x16_t G[2];  // cumulative gates of the direction about to run, prepared one barrier ahead of it
   if ((int)blockIdx.x < nslabs) {
+    const int lane = fresh_lane(), r = lane & 31, h = lane >> 5;
     const BwdSlab s0 = slab_of(blockIdx.x);
     const BwdNext first{s0, s0.gf, s0.L};
     issue_bwd_gate_loads<NG>(first, w, r, h, ld);
@@ -671,7 +681,7 @@ __global__ __launch_bounds__(64 * TW, 2) void gla_backward_mfma_kernel(
     f32x16_t dvacc[2] = {{0.f}, {0.f}};
     // a direction that is not run has neither issued the loads of the slab that follows nor prepared its gates
     const auto skip = [&] {
-      const int ln = fresh_lane(lane);
+      const int ln = fresh_lane();
       lds_barrier();  // a wave that has left must not touch the gate totals the others still read
       issue_bwd_gate_loads<NG>(next_first, w, ln & 31, ln >> 5, ld);
       issue_bwd_qk_loads<NG>(next_first, w, ln & 31, ln >> 5, ld);
@@ -679,27 +689,26 @@ __global__ __launch_bounds__(64 * TW, 2) void gla_backward_mfma_kernel(
       bwd_cumulate_gates<true, NG, TW>(ld, w, ln, lds, G);
       lds_barrier();
     };
-    bool ok = bwd_anchor<true, NG, TW>(w, lane, lds);
+    bool ok = bwd_anchor<true, NG, TW>(w, lds);
     if (ok) {
       u32x4_t keepq[NG], keepk[NG];
       if constexpr (BIDIR) {
-        bwd_direction<true, true, false, NG, SEG, TW>(sl, sl.L, ntiles, w, lane, lds, s, dvacc, keepq, keepk, ld, second, G);
-        ok = bwd_anchor<false, NG, TW>(w, lane, lds);
+        bwd_direction<true, true, false, NG, SEG, TW>(sl, sl.L, ntiles, w, lds, s, dvacc, keepq, keepk, ld, second, G);
+        ok = bwd_anchor<false, NG, TW>(w, lds);
         if (ok) {
-          bwd_direction<false, false, true, NG, SEG, TW>(sl, sl.L, ntiles, w, lane, lds, s, dvacc, keepq, keepk, ld, next_first, G);
+          bwd_direction<false, false, true, NG, SEG, TW>(sl, sl.L, ntiles, w, lds, s, dvacc, keepq, keepk, ld, next_first, G);
         } else {
           skip();  // (in each branch, so that nothing of this slab's loads stays alive for it)
         }
       } else {  // the causal op: the forward direction alone, first and last at once
-        bwd_direction<true, true, true, NG, SEG, TW>(sl, sl.L, ntiles, w, lane, lds, s, dvacc, keepq, keepk, ld, next_first, G);
+        bwd_direction<true, true, true, NG, SEG, TW>(sl, sl.L, ntiles, w, lds, s, dvacc, keepq, keepk, ld, next_first, G);
       }
     } else {
       skip();
     }
-    if (SEG) {  // one flag per sequence, cleared by the segment scan: any segment out of range gives the sequence away
-      if (tid == 0 && !ok) flags[slab / sg.nseg] = 1;
-    } else if (tid == 0) {
-      flags[slab] = ok ? 0 : 1;
+    if (w == 0 && fresh_lane() == 0) {
+      if (!SEG) flags[slab] = ok ? 0 : 1;
+      else if (!ok) flags[slab / sg.nseg] = 1;  // one flag per sequence, cleared by the segment scan: any segment out of range gives it away
     }
   }
 }
@@ -896,11 +905,15 @@ static int launch_bwd_t(const BwdLaunch& l) {
 }
 // Slabs of up to 64 and up to 128 tokens get workgroups of two and four waves, four and two of them to a CU: in one of eight, the
 // waves without a tile idle and nothing runs beside the loads.  us, eight waves / as many as the slab has tiles (dword operands): Dk 64:
-// 2010 slabs of 57 tokens 119 / 62, 1200 of 128 113 / 83, 3 of 49 20 / 16; Dk 32: 91 / 37, 82 / 51, 16 / 13.  Seven waves instead of
-// eight for 193 to 224 tokens: at Dk 64 the LDS of the eighth tile holds the first
-// direction's dq (768 slabs of 196 tokens, Dk 64 91.4 / 87.1, Dk 32 58.7 / 57.5; of 130, 74.7 / 70.6).  For the same room three waves
-// instead of four for 65 to 96 tokens at Dk 64: 768 slabs of 70 tokens 39.0 / 36.0, 1200 55.4 / 51.1, 297 27.3 / 26.3, 768 of 96 41.9 / 37.8 (Dk 32
-// has its dq in registers: 23.8 / 23.8).
+// 2010 slabs of 57 tokens 119 / 62, 1200 of 128 113 / 83, 3 of 49 20 / 16; Dk 32: 91 / 37, 82 / 51, 16 / 13.
+// Seven waves instead of eight for 129 to 224 tokens.  Both directions at Dk 64, where the LDS of the eighth tile also holds the first
+// direction's dq: 768 slabs of 129 tokens 74.6 / 71.1, of 145 77.3 / 72.9, of 180 87.1 / 81.7, of 192 88.5 / 82.9, of 196 91.4 / 87.1, 300 of 160 52.2 / 50.4,
+// one of 160 26.4 / 26.2.  The rest by the wave that idles: the forward direction alone, Dk 64 768 of 129 45.4 / 42.0, of 192 52.9 / 50.1, of 210 55.8 / 53.1, 300
+// of 145 30.3 / 29.5; Dk 32, both directions 768 of 160 49.7 / 48.9, 1200 of 180 83.3 / 82.1, one 18.1 / 18.0, forward 768 of 129 30.2 / 30.0, 1200 of 160 45.5 /
+// 44.7.
+// Three waves instead of four for 65 to 96 tokens at Dk 64, again with room for that dq: both directions 768 slabs of 70 tokens 39.0 / 36.0, 1200 55.4 /
+// 51.1, 297 27.3 / 26.3, 768 of 96 41.9 / 37.8; forward alone 768 of 65 24.1 / 23.8, of 96 26.3 / 25.6, 1200 of 80 34.9 / 34.0, 300 of 65 17.5 / 16.9, one 11.6 /
+// 11.5.  (Dk 32 has its dq in registers: 768 of 96 27.1 / 26.8, 1200 35.3 / 35.3; four.)
 template <int NG, bool BIDIR>
 static int launch_bwd(const BwdLaunch& l, bool seg, int tokens) {
   if (seg) return tokens <= 128 ? launch_bwd_t<NG, BIDIR, true, 4>(l) : launch_bwd_t<NG, BIDIR, true, 8>(l);
