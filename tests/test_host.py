@@ -45,6 +45,24 @@ def test_workspace_sizes():
     assert wb(2, 3, 600, 64, 32, 1) == (3 * n_qk + n_v // 2) * 4 + 2 * 3 * 4  # Dv = 32: recurrent kernel only
 
 
+@pytest.mark.parametrize("rows", [9568, 12544])
+@pytest.mark.parametrize("C,inner,stacked", [(192, 512, 592), (384, 1024, 1168), (768, 2048, 2320)])  # ViG-T, -S, -B
+def test_weight_gradients_of_a_node_fill_the_chip(rows, C, inner, stacked):
+    """Token ranges times 128 x 128 tiles come near a whole number of workgroups for each of the 256 compute units."""
+    import ctypes
+
+    from vig_amd import _lib
+
+    if not os.path.exists(_lib.LIB_PATH):
+        pytest.skip("library not built here")
+    for layers in (((C, inner), (2 * inner, C)), ((C, C), (C, 16), (stacked, C))):
+        N, K = ((ctypes.c_int * len(layers))(*x) for x in zip(*layers))
+        need = _lib.load().vig_linear_bwd_weight_many_workspace(rows, N, K, len(layers))
+        ranges = need // (4 * sum(n * k + n for n, k in layers))
+        groups = ranges * sum(-(-n // 128) * -(-k // 128) for n, k in layers)
+        assert groups >= 0.7 * 256 * -(-groups // 256), (layers, ranges)
+
+
 def test_wrappers_reject_what_is_not_built():
     import vig_amd
 

@@ -68,6 +68,13 @@ def test_a_channel_keeps_to_itself(N, T, value):
         assert not dw[n].isfinite().any()
 
 
+@pytest.mark.parametrize("T", [16384, 16385])  # 274 tiles: in one launch, and a layer behind the other
+def test_many_tiles(T):
+    g = torch.Generator("cuda").manual_seed(T)
+    dys, xs = zip(*([torch.randn(T, n, device="cuda", generator=g).bfloat16() for n in nk] for nk in ((2048, 2056), (136, 24))))
+    _check(dys, xs, *_call(dys, xs, [True, True]))
+
+
 def test_rows_far_apart():  # past 32-bit byte offsets inside a stage
     T, ld, n, k = 40, (1 << 26) + 8, 136, 24
     dy = torch.empty(T * ld, dtype=torch.bfloat16, device="cuda").as_strided((T, n), (ld, 1))

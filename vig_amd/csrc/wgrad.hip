@@ -18,6 +18,10 @@
 // reaches), 11 until the pipes run full, 4 to 7 writing and 7 to 9 adding the partial tiles.  Fragments read a k-step ahead of their
 // products gave 3 %; 128 x 192 and 256 x 192 tiles, which ask the L2 for 0.8 and 0.6 of the operands, 57 to 60 us there and no better where
 // a node's layers share the launch; lines touched 4 to 20 stages ahead by a fifth wave were no faster.
+#include <math.h>
+
+#include <algorithm>
+
 #include "common.h"
 #include "launch.h"
 #include "mfma_tiles.h"
@@ -258,16 +262,38 @@ __global__ __launch_bounds__(256) void wgrad_sum_kernel(WgradSums a) {
 
 long long wgrad_tiles(int N, int K) { return (long long)((N + kWgTile - 1) / kWgTile) * ((K + kWgTile - 1) / kWgTile); }
 
-// Token ranges of layers of that many tiles in all.  A multiple of eight keeps a range's tiles on one XCD; it is taken where it leaves
-// no more than an eighth of the places empty (T 25088, us: 768 x 768, 14 ranges or 8: 47 / 58; 384 x 1024, 21 or 16: 38 / 41;
-// 1232 x 384, 17 or 16: 47 / 46).
-int wgrad_splits(long long T, long long tiles) {
-  long long s = 512 / tiles;                       // two workgroups per CU
-  const long long most = (T + 255) / 256;          // at least eight stages each
-  if (s > most) s = most;
-  if (s > 128) s = 128;
-  if (s / 8 * 8 * 8 >= s * 7) s = s / 8 * 8;
-  return s < 1 ? 1 : (int)s;
+// Token ranges of some layers that go out together: the number with the least estimated time, from what was measured for 1 to 128 ranges of
+// 19 layers and nodes of ViG-T, -S and -B at 100 to 50 176 rows, inputs in the caches and not.  A workgroup alone on its CU takes 11 ns a row, two on
+// one CU 14.2; three make a pair and one behind it, with 2.3 us to fill the pipes again, and every round behind
+// the first adds 12 % to all of it: the ranges no longer walk in step through what the caches hold.  Partial tiles cost a launch, the result written and, for
+// what is written and read back between the two, 2.5 us times the 3/4th power of the millions of them (the more there are, the more of that hides
+// under the loops).  Beyond eight ranges a multiple of eight keeps a range's tiles on one XCD: 6 %.
+// 1 % off the best of all counts on average and 5 % at most, where "as many as fill the chip in one round" was 9 % off.  us, that rule / this one: both
+// MLP layers of ViG-B, 288 tiles, 12 544 rows (one range: 288 of 512 places) 197 / 178; of ViG-S, 784 rows (4 ranges) 21 / 14.5; 2320 x 768, 784 rows
+// 24 / 16; 1000 x 192, 4 888 rows (20 ranges) 20.1 / 18.6; 2048 x 384, 25 088 rows 67 / 67.
+float wgrad_estimate(long long T, long long tiles, float melems, int s) {
+  const long long per = ((T + s - 1) / s + kWgStage - 1) / kWgStage * kWgStage;
+  const long long deep = (tiles * ((T + per - 1) / per) + 255) / 256;  // workgroups a CU has to do
+  const long long rounds = (deep + 1) >> 1;
+  float us = ((deep >> 1) * 0.0142f + (deep & 1) * 0.011f) * per * (0.88f + 0.12f * rounds) + 2.3f * rounds;
+  if (s > 1) {
+    const float x = s * melems;
+    us += 0.8f + 0.47f * melems + 2.5f * sqrtf(x * sqrtf(x));
+  }
+  return s > 8 && s % 8 ? 1.06f * us : us;
+}
+int wgrad_splits(long long T, const LinearWgrad* layers, int count) {
+  long long tiles = 0;
+  float melems = 0.f;
+  for (int i = 0; i < count; ++i) tiles += wgrad_tiles(layers[i].N, layers[i].K), melems += 1e-6f * layers[i].N * layers[i].K;
+  const long long most = std::min<long long>(128, std::min((T + 63) / 64, 2048 / tiles));
+  int best = 1;
+  float least = wgrad_estimate(T, tiles, melems, 1);
+  for (int s = 2; s <= most; s += s < 24 ? 1 : 4) {
+    const float us = wgrad_estimate(T, tiles, melems, s);
+    if (us < least) least = us, best = s;
+  }
+  return best;
 }
 
 }  // namespace
@@ -275,25 +301,40 @@ int wgrad_splits(long long T, long long tiles) {
 bool linear_wgrad_supported(long long T, int N, int K) {
   return T > 0 && T < 0x7fffffffLL - 4096 && N > 0 && K > 0 && N % 8 == 0 && K % 8 == 0 && N <= (1 << 20) && K <= (1 << 20);
 }
-size_t linear_wgrad_workspace(long long T, const LinearWgrad* layers, int count) {
+// Past 256 tiles a layer's own number of ranges fits the chip better than one number for all, and from here on the loops are all that counts: both MLP
+// layers of ViG-B, us, together / one behind the other: 6 272 rows 99 / 108, 12 544 174 / 181, 16 384 220 / 226, 18 000 245 / 239, 25 088 348 / 326, 50 176 722 / 656.
+static bool wgrad_together(long long T, const LinearWgrad* layers, int count) {
   long long tiles = 0;
   for (int i = 0; i < count; ++i) tiles += wgrad_tiles(layers[i].N, layers[i].K);
+  return count == 1 || tiles <= 256 || T <= 16384;
+}
+size_t linear_wgrad_workspace(long long T, const LinearWgrad* layers, int count) {
+  if (!wgrad_together(T, layers, count)) {
+    size_t most = 0;
+    for (int i = 0; i < count; ++i) most = std::max(most, linear_wgrad_workspace(T, layers + i, 1));
+    return most;
+  }
   size_t floats = 0;
   for (int i = 0; i < count; ++i) floats += ((size_t)layers[i].N * layers[i].K + layers[i].N + 3) / 4 * 4;
-  return wgrad_splits(T, tiles) * floats * sizeof(float);
+  return wgrad_splits(T, layers, count) * floats * sizeof(float);
 }
 
 int launch_linear_wgrad(const LinearWgrad* layers, int count, long long T, void* workspace, hipStream_t stream) {
   static bool done[64] = {};
   constexpr int lds = kWgBuffers * 2 * kWgHalf;
   if (count < 1 || count > kWgradLayers) return -22;
+  if (!wgrad_together(T, layers, count)) {
+    int rc = 0;
+    for (int i = 0; i < count && rc == 0; ++i) rc = launch_linear_wgrad(layers + i, 1, T, workspace, stream);
+    return rc;
+  }
   if (!allow_lds(reinterpret_cast<const void*>(linear_wgrad_kernel), lds, done)) return -5;
   WgradArgs a{};
   WgradSums b{};
   long long tiles = 0, blocks = 0;
   for (int i = 0; i < count; ++i) tiles += wgrad_tiles(layers[i].N, layers[i].K);
   if (tiles > 0x7fffffffLL / 256) return -22;
-  const int want = wgrad_splits(T, tiles);
+  const int want = wgrad_splits(T, layers, count);
   a.T = (int)T, a.layers = b.layers = count, a.tiles = (int)tiles;
   a.per = (int)(((T + want - 1) / want + kWgStage - 1) / kWgStage * kWgStage);
   a.splits = b.splits = (int)((T + a.per - 1) / a.per);
