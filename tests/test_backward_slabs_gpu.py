@@ -1,5 +1,5 @@
-"""The matrix-core backward's workgroups of two, four and eight tiles at the edges of their ranges, and with more slabs than
-workgroups (each walks several)."""
+"""The matrix-core backward's workgroups of two, three (64 key channels only), four, seven and eight tiles at the edges of their
+ranges, and with more slabs than workgroups (each walks several)."""
 import pytest
 import torch
 
@@ -72,6 +72,13 @@ def test_three_tiles(B, H, L, both):
     test_lengths(B, H, L, 64, both)
 
 
+@pytest.mark.parametrize("both", [True, False])
+@pytest.mark.parametrize("B,H,L", [(1, 1, 1), (1, 2, 32), (1, 1, 33), (2, 3, 64), (180, 6, 49)])
+def test_two_tiles(B, H, L, both):
+    """64 key channels: of the first direction's dq three units of four wait in LDS, one in the output tensor."""
+    test_lengths(B, H, L, 64, both)
+
+
 @pytest.mark.parametrize("B,H,L,Dk", [(90, 6, 70, 64), (87, 6, 197, 64), (87, 6, 197, 32), (90, 3, 230, 64), (90, 3, 230, 32)])
 def test_slabs_given_up_in_either_direction(B, H, L, Dk):
     """Several slabs a workgroup, some beyond the range in their first direction, some in their second (whose loads are then
@@ -89,3 +96,7 @@ def test_slabs_given_up_in_either_direction(B, H, L, Dk):
     for g, e in zip(got, exact):
         assert torch.equal(g[strong], e[strong])
     _check_mfma([g[~strong] for g in got], [f64(e[~strong]) for e in exact], q[~strong].cpu())
+
+
+def test_two_tile_slabs_given_up_in_either_direction():
+    test_slabs_given_up_in_either_direction(360, 3, 60, 64)

@@ -10,7 +10,8 @@ And no memory instruction may take its address from a scalar register that a vec
 before: the compiler sees to it, except in asm blocks, which it does not look into (load_to_lds16 of common.h).
 
 And the bf16 backward reloads no spilled register between the end of a direction and the staging of the next: the counter a reload is
-waited for with goes down in the order of issue, so that it waits for everything the wave has just stored (3 to 6 % of a call)."""
+waited for with goes down in the order of issue, so that it waits for everything the wave has just stored (3 to 6 % of a call).  Its
+workgroups of two tiles send no more through memory than LDS has no room for."""
 import functools
 import os
 import re
@@ -202,3 +203,11 @@ def test_no_reload_between_the_directions():
     # whole sequences, 64 key channels, both directions: two to eight waves
     found, seen = reloads_while_staging(_assembly("gla_backward_mfma.hip"), r"_ZN3vig24gla_backward_mfma_kernelILi4ELb1ELb0ELi[23478]E")
     assert seen == 10 and found == []
+
+
+def test_two_tiles_park_one_unit_of_four_in_memory():
+    # 64 key channels, both directions, two waves: dv, dk, dq and either gate's gradient in four stores each, and what is left of the
+    # first direction's dq (all four units through memory: 600 slabs of 64 tokens 27.6 us instead of 26.9)
+    name, = re.findall(r"^(_ZN3vig24gla_backward_mfma_kernelILi4ELb1ELb0ELi2E\w*):", _assembly("gla_backward_mfma.hip"), re.M)
+    body = re.search(rf"^{name}:.*?^\.Lfunc_end", _assembly("gla_backward_mfma.hip"), re.S | re.M).group(0)
+    assert body.count("buffer_store_dwordx4") == 5 * 4 + 1

@@ -29,7 +29,8 @@
 // among them), and its products wait for LDS reads with two waves a SIMD.  us, whole calls one behind the other, the flag pass with them, against operands read as dwords and
 // put together by v_perm, dq ahead of dk, dv in loops of their own and the first direction's dq, dk parked in the output tensors:
 // 768 x 196 Dk 64 104 -> 87, Dk 32 74 -> 57; 768 x 256 Dk 64 124 -> 106; 1200 x 128 84 -> 71; 24 x 2305 with the state passes, Dk 32 57 -> 47.5,
-// Dk 64 82 -> 73; 384 x 57 Dk 64 23.7 -> 23.1, 600 x 64, where the second 1 / e tells most, 27.1 -> 27.4.
+// Dk 64 82 -> 73; 384 x 57 Dk 64 23.4 -> 22.9, 600 x 64 27.0 -> 27.2, 1200 x 64 42.4 -> 39.7, 768 x 49
+// 26.7 -> 26.4, forward alone 18.0 -> 18.4.
 //
 // Slabs whose gate totals exceed the anchor's range (|G_total| / 2 * log2(e) > 60 in some channel) are not computed
 // here: the workgroup raises the slab's flag and the token-recurrent kernel, launched afterwards with that flag
@@ -55,8 +56,10 @@ struct BwdLds {
   static constexpr int tot = 4 * mat;               // [TW][64] f32: gate totals of the tiles
   static constexpr int off = tot + TW * 64 * 4;     // [TW][64] f32: per wave, (prefix - anchor) of its tile
   static constexpr int dgtot = off + TW * 64 * 4;   // [TW][64] f32: totals of q dq - k dk of the tiles
-  // [TW][parked units of 64 lanes x 16 B]: the first direction's dq (Dk = 64) while the second runs, where there is room for it
-  static constexpr int parked = TW == 7 || TW == 3 ? 4 : 0;
+  // [TW][parked units of 64 lanes x 16 B]: the first direction's dq (Dk = 64) while the second runs, where there is room for it.  Two tiles:
+  // three of its four units, which leave four workgroups to a CU; the last one goes by way of the output tensor.  us, all four that
+  // way / one / none, with three workgroups: 600 slabs of 64 tokens 27.6 / 26.9 / 26.8, 768 29.4 / 28.9 / 28.6, 1024 34.5 / 33.7 / 40.4; one 15.0 / 15.1 / 15.0.
+  static constexpr int parked = TW == 7 || TW == 3 ? 4 : TW == 2 ? 3 : 0;
   static constexpr int park = dgtot + TW * 64 * 4;
   static constexpr int turn = park + TW * parked * 1024;  // [TW][16 rows] of results on their way out (store_rows)
   static constexpr bool turns(int ng) { return ng == 4 && TW >= 3; }
@@ -339,7 +342,7 @@ __device__ __forceinline__ bool bwd_anchor(int w, char* lds) {
 
 // One direction of one slab, for wave w (tile w).  dv accumulates over both directions (raw, unscaled).  The first
 // direction (FIRST, not LAST) stages v and do and hands its dq and dk, rounded to bf16, to the second: in registers, or at
-// Dk = 64, where the loops in between leave no room for dq, in LDS (seven tiles) or parked in the output tensor.  The second
+// Dk = 64, where the loops in between leave no room for dq, in LDS as far as there is room, else parked in the output tensor.  The second
 // (LAST, not FIRST) adds its own to them and stores dq, dk, dv.  A one-direction (causal) launch runs a single direction that
 // is both.  Registers set the order of the phases: dk and dv end before dq begins, and only e of the two factors is kept.
 // SEG: the slab is a segment of a longer sequence.  With S_in the state entering it along the direction, R_out the
@@ -353,7 +356,7 @@ __device__ __forceinline__ void bwd_direction(const BwdSlab& sl, int L, int ntil
                                               BwdLoads<NG>& ld, const BwdNext& nxt, f32x16_t (&G)[2]) {
   constexpr bool stage_vdo = FIRST;
   constexpr int kParkLds = NG == 4 && !(FIRST && LAST) ? BwdLds<TW>::parked : 0;
-  constexpr bool kParkDq = NG == 4 && kParkLds == 0 && !(FIRST && LAST);
+  constexpr bool kParkDq = NG == 4 && kParkLds < NG && !(FIRST && LAST);
   // Fetched ahead of the dq loop, or, where its registers do not hold that too (a fetched value that is spilled is waited
   // for at once), behind it: 1200 slabs of 128 tokens, Dk = 64 75 against 82 us with the gates early; 768 of 256 109 against 113
   // with the rows.
@@ -491,7 +494,7 @@ __device__ __forceinline__ void bwd_direction(const BwdSlab& sl, int L, int ntil
   // that store.  So what is stored waits, packed, until what is fetched here is on its way.
   if (kParkDq && !FIRST) {
 #pragma unroll
-    for (int g = 0; g < NG; ++g)
+    for (int g = kParkLds; g < NG; ++g)
       keepq[g] = __builtin_amdgcn_raw_buffer_load_b128(chunk_rsrc(sl.dq + tk, rows, 2 * DK), r * (32u * NG) + h * (16u * NG) + 16u * g, 0, 0);
   }
   if (kEarlyGates) issue_bwd_gate_loads<NG>(nxt, w, r, h, ld);
@@ -563,7 +566,13 @@ __device__ __forceinline__ void bwd_direction(const BwdSlab& sl, int L, int ntil
 #pragma unroll
     for (int g = 0; g < kParkLds; ++g) *reinterpret_cast<u32x4_t*>(unit_ptr(lds + BwdLds<TW>::park, w * kParkLds + g, lane)) = keepq[g];
   }
-  if (LAST || kParkDq) store_rows<NG, TW>(turn, keepq, chunk_rsrc(sl.dq + tk, rows, 2 * DK), lane);
+  if (LAST || (kParkDq && kParkLds == 0)) {
+    store_rows<NG, TW>(turn, keepq, chunk_rsrc(sl.dq + tk, rows, 2 * DK), lane);
+  } else if (kParkDq) {
+#pragma unroll
+    for (int g = kParkLds; g < NG; ++g)
+      __builtin_amdgcn_raw_buffer_store_b128(keepq[g], chunk_rsrc(sl.dq + tk, rows, 2 * DK), r * (32u * NG) + h * (16u * NG) + 16u * g, 0, 0);
+  }
   // ---- dg: the running sum of X over the tokens the gate acts on.  Inside the tile by lane shifts (lane = token),
   // across tiles through the tile totals in LDS: walking forward a token takes everything from itself to the end,
   // i.e. the totals of this and the later tiles minus what lies before it in the tile. ----
@@ -895,6 +904,7 @@ template <int NG, bool BIDIR, bool SEG, int TW>
 static int launch_bwd_t(const BwdLaunch& l) {
   static bool done[64] = {};
   auto* kernel = gla_backward_mfma_kernel<NG, BIDIR, SEG, TW>;
+  static_assert(kBwdTiles / TW * BwdLds<TW>::total <= 160 * 1024, "the workgroups of a CU fit its LDS");
   if (!allow_lds(reinterpret_cast<const void*>(kernel), BwdLds<TW>::total, done)) return -5;
   const int most = l.num_cu * (kBwdTiles / TW);
   hipLaunchKernelGGL(kernel, dim3(l.nslabs < most ? l.nslabs : most), dim3(64 * TW), BwdLds<TW>::total, l.stream,
