@@ -77,6 +77,7 @@ __global__ __launch_bounds__(256, 2) void linear_wgrad_kernel(WgradArgs a) {
   const int t0 = split * a.per, t1 = min(a.T, t0 + a.per);
   const int nstage = (t1 - t0 + kWgStage - 1) / kWgStage;
   const int wn = 64 * (wave & 1), wk = 64 * (wave >> 1);  // this wave's 64 x 64 of the tile
+  const int flip = wave >> 1;  // block of 32 channels of dY that comes first: the one whose bias is this wave's
 
   // a wave's share of a stage: rows 8*wave .. +8 of both operands, four rows (1 KB) per load.  Rows and channels past the
   // end are read from the last row and from channel 0 (every load is issued: the waits below count them); such rows are
@@ -125,20 +126,23 @@ __global__ __launch_bounds__(256, 2) void linear_wgrad_kernel(WgradArgs a) {
 #pragma unroll
   for (int b = 0; b < 2; ++b) {
     const int tok = 8 * h + ((lane >> 2) & 3), half = (lane >> 4) & 1;
-    atn[b] = tok * kWgRow + 32 * (((wn >> 4) + 2 * b + half) ^ unit_swap(tok)) + 8 * (lane & 3);
+    atn[b] = tok * kWgRow + 32 * (((wn >> 4) + 2 * (b ^ flip) + half) ^ unit_swap(tok)) + 8 * (lane & 3);
     atk[b] = kWgHalf + tok * kWgRow + 32 * (((wk >> 4) + 2 * b + half) ^ unit_swap(tok)) + 8 * (lane & 3);
   }
-  f32x16_t acc[2][2], accb[2];
+  f32x16_t acc[2][2];
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    accb[i] = f32x16_t{0.f};
+  for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) acc[i][j] = f32x16_t{0.f};
-  }
-  const bool with_bias = y.bpart && k0 == 0 && wk == 0;
-  // (A 16x16x32 product would take 24 registers less, but contracts over two channels at once, told apart by zeros in the other operand:
-  // 0 x Inf and 0 x NaN are NaN, and a channel that overflowed would take the other one's sum with it.)
-  const u32x4_t ones = {0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};
+  // The bias by sixteen 4x4x4 products against ones at a time: a row is four tokens of one channel, a lane's own, so that a channel that
+  // overflowed keeps to itself (a 16x16x32 product has two channels in a row, told apart by zeros in the other operand: 0 x Inf is NaN).
+  // Of the two waves that read the same channels either takes one block of 32.  A workgroup that does the bias takes longer than the others
+  // and the launch waits for it; us, 32x32x16 products in one wave of the two / this: 25088 x 2048 x 384 63.4 / 58.5, 768 x 2048 106 / 100.5, 1168 x 384 43.5
+  // / 40.6; lane sums by v_dot2 59.9, 101, 41.4.
+  const bool with_bias = y.bpart && k0 == 0;
+  f32x4acc_t accb[2] = {f32x4acc_t{0.f}, f32x4acc_t{0.f}};
+  s16x4_t ones = {0x3F80, 0x3F80, 0x3F80, 0x3F80};
+  asm volatile("" : "+v"(ones));  // (in registers: made anew in every k-step otherwise)
   struct Frags {
     u32x4_t n[2], k[2];
   };
@@ -157,8 +161,10 @@ __global__ __launch_bounds__(256, 2) void linear_wgrad_kernel(WgradArgs a) {
 #pragma unroll
       for (int i = 0; i < 2; ++i) acc[i][j] = mfma(f.n[i], f.k[j], acc[i][j]);
     if (with_bias) {
+      const u32x4_t y = f.n[0];
 #pragma unroll
-      for (int i = 0; i < 2; ++i) accb[i] = mfma(f.n[i], ones, accb[i]);
+      for (int q = 0; q < 2; ++q)
+        accb[q] = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(__builtin_bit_cast(s16x4_t, u32x2_t{y[2 * q], y[2 * q + 1]}), ones, accb[q], 0, 0, 0);
     }
   };
   for (int s = 0; s < kWgBuffers - 1; ++s)
@@ -199,23 +205,21 @@ __global__ __launch_bounds__(256, 2) void linear_wgrad_kernel(WgradArgs a) {
         const int k = k0 + wk + 32 * j + r;
 #pragma unroll
         for (int c = 0; c < 16; ++c) {
-          const int n = n0 + wn + 32 * i + 8 * (c >> 2) + 4 * h + (c & 3);
+          const int n = n0 + wn + 32 * (i ^ flip) + 8 * (c >> 2) + 4 * h + (c & 3);
           if (whole || (n < N && k < K)) part[(size_t)n * K + k] = acc[i][j][c];
         }
       }
   };
   if (n0 + kWgTile <= N && k0 + kWgTile <= K) store(true);
   else store(false);
-  if (with_bias) {  // (all columns of accb are alike: lane r of a half stores what row r of its registers holds.  Stored by two
-    // lanes one value after the other: 49 tokens 384 x 16 5.8 instead of 5.3 us, 25088 16.7 instead of 16.3)
+  if (with_bias) {
+    const f32x4acc_t both = accb[0] + accb[1];
+    float sum = both[0];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      float sum = accb[i][0];
-#pragma unroll
-      for (int c = 1; c < 16; ++c) sum = r == c ? accb[i][c] : sum;
-      const int n = n0 + wn + 32 * i + 8 * (r >> 2) + 4 * h + (r & 3);
-      if (r < 16 && n < N) y.bpart[(size_t)split * N + n] = sum;
-    }
+    for (int c = 1; c < 4; ++c) sum = (lane & 3) == c ? both[c] : sum;
+    sum += __shfl_xor(sum, 32);
+    const int n = n0 + wn + 32 * flip + r;
+    if (h == 0 && n < N) y.bpart[(size_t)split * N + n] = sum;
   }
 }
 
