@@ -63,6 +63,20 @@ def test_weight_gradients_of_a_node_fill_the_chip(rows, C, inner, stacked):
         assert groups >= 0.7 * 256 * -(-groups // 256), (layers, ranges)
 
 
+@pytest.mark.parametrize("rows,N,K,least,most", [(16384, 384, 16, 48, 80), (6272, 1000, 384, 9, 21), (6272, 384, 1024, 7, 21), (2352, 2320, 768, 4, 4),
+                                                 (784, 2320, 768, 1, 1), (25088, 2048, 384, 8, 10)])
+def test_token_ranges_near_the_best(rows, N, K, least, most):
+    """Counts of ranges whose times lie within 5 % of the best one's as measured over all of 1 to 128."""
+    import ctypes
+
+    from vig_amd import _lib
+
+    if not os.path.exists(_lib.LIB_PATH):
+        pytest.skip("library not built here")
+    need = _lib.load().vig_linear_bwd_weight_many_workspace(rows, (ctypes.c_int * 1)(N), (ctypes.c_int * 1)(K), 1)
+    assert least <= need // (4 * (N * K + N)) <= most
+
+
 def test_wrappers_reject_what_is_not_built():
     import vig_amd
 

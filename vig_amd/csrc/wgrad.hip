@@ -267,24 +267,21 @@ __global__ __launch_bounds__(256) void wgrad_sum_kernel(WgradSums a) {
 long long wgrad_tiles(int N, int K) { return (long long)((N + kWgTile - 1) / kWgTile) * ((K + kWgTile - 1) / kWgTile); }
 
 // Token ranges of some layers that go out together: the number with the least estimated time, from what was measured for 1 to 128 ranges of
-// 19 layers and nodes of ViG-T, -S and -B at 100 to 50 176 rows, inputs in the caches and not.  A workgroup alone on its CU takes 11 ns a row, two on
-// one CU 14.2; three make a pair and one behind it, with 2.3 us to fill the pipes again, and every round behind
-// the first adds 12 % to all of it: the ranges no longer walk in step through what the caches hold.  Partial tiles cost a launch, the result written and, for
-// what is written and read back between the two, 2.5 us times the 3/4th power of the millions of them (the more there are, the more of that hides
-// under the loops).  Beyond eight ranges a multiple of eight keeps a range's tiles on one XCD: 6 %.
-// 1 % off the best of all counts on average and 5 % at most, where "as many as fill the chip in one round" was 9 % off.  us, that rule / this one: both
-// MLP layers of ViG-B, 288 tiles, 12 544 rows (one range: 288 of 512 places) 197 / 178; of ViG-S, 784 rows (4 ranges) 21 / 14.5; 2320 x 768, 784 rows
-// 24 / 16; 1000 x 192, 4 888 rows (20 ranges) 20.1 / 18.6; 2048 x 384, 25 088 rows 67 / 67.
+// 23 layers and nodes of ViG-T, -S and -B at 100 to 50 176 rows, inputs in the L2s and not.  A workgroup alone on its CU takes 8.8 ns a row, two on
+// one CU 11.6; three make a pair and one behind it, with 1.4 us to fill the pipes again, and every round behind
+// the first adds 7 % to all of it: the ranges no longer walk in step through what the caches hold.  Partial tiles cost a launch, the result written, a
+// pass of the adding kernel for eight ranges and, for what is written and read back between the two, 3.1 us times the 0.56th power of the millions of them
+// (the more there are, the more of that hides under the loops).  Beyond eight ranges a multiple of eight keeps a range's tiles on one XCD: 3.6 %.
+// 0.7 % off the best of all counts on average, where "as many as fill the chip in one round" was 6.4 % off; more than 2 % behind that rule at 12 of 736 points, by
+// 0.4 us at most.  us, that rule / this one: both MLP layers of ViG-S, 784 rows (4 ranges) 21 / 14.5; 2320 x 768, 784 rows 24.6 / 15.6; 1024 x 192, 4 704 rows (19
+// ranges) 19.1 / 17.4; 384 x 16, 784 rows (4) 9.3 / 7.7; 2048 x 384, 25 088 rows 58.7 / 58.4.
 float wgrad_estimate(long long T, long long tiles, float melems, int s) {
   const long long per = ((T + s - 1) / s + kWgStage - 1) / kWgStage * kWgStage;
   const long long deep = (tiles * ((T + per - 1) / per) + 255) / 256;  // workgroups a CU has to do
   const long long rounds = (deep + 1) >> 1;
-  float us = ((deep >> 1) * 0.0142f + (deep & 1) * 0.011f) * per * (0.88f + 0.12f * rounds) + 2.3f * rounds;
-  if (s > 1) {
-    const float x = s * melems;
-    us += 0.8f + 0.47f * melems + 2.5f * sqrtf(x * sqrtf(x));
-  }
-  return s > 8 && s % 8 ? 1.06f * us : us;
+  float us = ((deep >> 1) * 0.0116f + (deep & 1) * 0.0088f) * per * (0.93f + 0.07f * rounds) + 1.4f * rounds;
+  if (s > 1) us += 0.3f + 0.55f * melems + 0.1f * ((s + 7) / 8) + 3.1f * powf(s * melems, 0.56f);
+  return s > 8 && s % 8 ? 1.036f * us : us;
 }
 int wgrad_splits(long long T, const LinearWgrad* layers, int count) {
   long long tiles = 0;
