@@ -144,7 +144,7 @@ __device__ __forceinline__ void load_tfrag_lds(const uint16_t* kt, int t, int r,
 // token fetched, for all four tokens.  Which four channels a piece holds is the address's to say: accumulator rows 4Q .. 4Q + 3
 // (Q = 2g + h) take channels 32h + 8g + 4p + m (NG = 4, p = 0, 1: two fragments span the 64 channels) or
 // 16h + 4g + m (NG = 2: one fragment spans the 32), so register 4g + m of lane half h ends up with that channel of the
-// half's 8 NG contiguous ones.  Against the dword form below: half the LDS instructions, no v_perm, and at 32 channels
+// half's 8 NG contiguous ones.  Against the dword form above: half the LDS instructions, no v_perm, and at 32 channels
 // no accumulator rows without a channel.
 typedef short s16x4_t __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) const uint16_t* lds_u16_t;
@@ -153,13 +153,10 @@ __device__ __forceinline__ int tr_row_channel(int rho) {  // of accumulator row 
   const int Q = rho >> 2;
   return 8 * NG * (Q & 1) + 2 * NG * (Q >> 1) + (rho & 3);
 }
-template <int NG, int STRIDE>
-__device__ __forceinline__ int tr_lane_offset(int lane) {  // elements from the tile's first row
-  const int a = lane & 3, b = (lane >> 4) & 1;
-  return (4 * (lane >> 5) + ((lane & 15) >> 2)) * STRIDE + tr_row_channel<NG>(4 * (4 * b + a));
-}
+// `at`: the lane's own piece (four channels from tr_row_channel's on) of row 4 (lane / 32) + (lane & 15) / 4 of the tile, or 4 elements on for p = 1.  Rows
+// 8 apart are read from the same place of theirs: pieces may be swapped within a row by the row number's three lowest bits.
 template <int STRIDE>
-__device__ __forceinline__ u32x4_t tr_frag(lds_u16_t at, int t) {  // k-step t; `at`: the tile's first row + tr_lane_offset (+ 4p)
+__device__ __forceinline__ u32x4_t tr_frag(lds_u16_t at, int t) {  // k-step t
   typedef __attribute__((address_space(3))) s16x4_t lds_s16x4_t;
   typedef short s16x8_t __attribute__((ext_vector_type(8)));
   const s16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)(at + 16 * t * STRIDE));
