@@ -698,8 +698,8 @@ int vig_linear_bwd_weight(const void* dy, long long dy_row_stride, const void* x
                           float* dbias, void* workspace, size_t workspace_bytes, long long rows, int N, int K, void* stream);
 
 /*
- * The same of up to four layers over the same number of rows, in one launch and one that adds the partial sums: arrays of `count`
- * entries, each as above; dbias may be NULL, and so may its entries.
+ * The same of up to four layers over the same number of rows, in one launch and one that adds the partial sums, or, where that is quicker (many
+ * tiles and rows), in a pair of launches a layer: arrays of `count` entries, each as above; dbias may be NULL, and so may its entries.
  */
 size_t vig_linear_bwd_weight_many_workspace(long long rows, const int* N, const int* K, int count);
 int vig_linear_bwd_weight_many(const void* const* dy, const long long* dy_row_stride, const void* const* x,

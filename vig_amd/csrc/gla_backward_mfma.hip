@@ -28,7 +28,7 @@
 // asks for 1664 bytes, q and k in either direction, 49 us at the rate of a large copy; 1864 pass the memory, what fifteen spilled registers write
 // among them), and its products wait for LDS reads with two waves a SIMD.  us, whole calls one behind the other, the flag pass with them, against operands read as dwords and
 // put together by v_perm, dq ahead of dk, dv in loops of their own and the first direction's dq, dk parked in the output tensors:
-// 768 x 196 Dk 64 104 -> 87, Dk 32 74 -> 57; 768 x 256 Dk 64 124 -> 106; 1200 x 128 84 -> 71; 24 x 2305 with the state passes, Dk 32 57 -> 47.5,
+// 768 x 196 Dk 64 103 to 105 -> 86 to 90, Dk 32 74 to 76 -> 57 to 60; 768 x 256 Dk 64 124 to 129 -> 106 to 112; 1200 x 128 84 -> 71; 24 x 2305 with the state passes, Dk 32 57 -> 47.5,
 // Dk 64 82 -> 73; 384 x 57 Dk 64 23.4 -> 22.9, 600 x 64 27.0 -> 27.2, 1200 x 64 42.4 -> 39.7, 768 x 49
 // 26.7 -> 26.4, forward alone 18.0 -> 18.4.
 //

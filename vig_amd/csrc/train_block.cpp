@@ -10,10 +10,10 @@
 //   - q/k/v, gate and low-rank projection are one product over stacked weights (rows padded to a multiple of 128: 35 instead of
 //     62 us at 25088 x 384), their gradients gather into one matrix whose rows the kernels write in place, and one product
 //     returns the input gradient, added to the local branch's in fp32 before it is rounded;
-//   - weight and bias gradients leave vig_linear_bwd_weight_many as fp32, one launch for all of a node's layers;
+//   - weight and bias gradients leave vig_linear_bwd_weight_many as fp32, a node's layers together;
 //   - the up-projection of the gates and its input gradient run inside the gate kernels (bf16), and the depthwise
 //     convolution's three gradients are one kernel.
-// ViG-S, B 128 at 224 px under bf16 autocast, forward and backward on one MI355X: 23.7 -> 12.1 ms.
+// ViG-S, B 128 at 224 px under bf16 autocast, forward and backward on one MI355X: 23.7 -> 11.0 ms.
 #include <ATen/autocast_mode.h>
 
 #include "host_calls.h"
