@@ -36,3 +36,10 @@ def test_forms(B, h, w, C, silu, keep, biased, dtype, eps):
     if silu:
         want = want * torch.sigmoid(want)  # (its slope stays below 1.1)
     assert ((grid(y) - want).abs() <= 1.2 * eps * size).all()
+
+
+@pytest.mark.parametrize("dtype,eps", [(torch.float32, 2.0 ** -20), (torch.bfloat16, 2.0 ** -8)])
+@pytest.mark.parametrize("B,h,w,C", [(390, 7, 14, 64), (391, 7, 14, 64), (585, 9, 14, 64), (586, 16, 14, 64), (586, 17, 14, 64)])
+def test_bands_that_fit_a_round(B, h, w, C, dtype, eps):
+    """Both sides of the lines between three, two and one band: 87 360 and 87 584 columns of quads, 131 040 and 131 264."""
+    test_forms(B, h, w, C, 1, True, True, dtype, eps)

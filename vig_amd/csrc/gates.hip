@@ -726,8 +726,12 @@ static int launch_dwconv3x3_t(const void* x, const float* wt, const float* bias,
   if (3 * (w + 2) * kStencilGroup * (int)sizeof(T) > 48 * 1024) return -95;
   // every batch element is an image of C channels; all images share the C weight channels
   if (threads > kColumnThreads || cells > (1 << 30)) return launch_stencil<T, false>(x, wt, bias, y, pre, B, h, w, C, 1, C, silu, stream);
-  // bands for two hundred thousand threads, as far as there are rows (8 x 64 x 64, C 192: for half or twice as many 11.2, 11.8 instead of 10.3)
-  const int want = (int)std::min<long long>(h, (200000 + threads - 1) / threads), band = (h + want - 1) / want, bands = (h + band - 1) / band;
+  // Bands for two hundred thousand threads, as far as there are rows (8 x 64 x 64, C 192: for half or twice as many 11.2, 11.8 instead of 10.3), but
+  // no more threads than the chip takes at once, four workgroups to a CU: a band less where the last one would begin a second round, unless that
+  // leaves one long band (us, inputs from memory, staged / with that band / without; C 192: 170 x 11 x 11 10.3 / 11.7 / 9.8, 231 x 8 x 8 9.7 / 10.3 / 8.1, 255 x 11 x 11 13.1 / 14.1 / 13.1,
+  // 350 x 8 x 8 13.1 / 11.8 / 10.9, 200 x 14 x 14 16.2 / 15.5 / 15.3; 116 x 24 x 24 21.3 / 20.6 / 21.7; fp32 170 x 11 x 11 12.4 / 13.1 / 10.8)
+  const int fill = (int)((200000 + threads - 1) / threads), fit = (int)std::max<long long>(1, 4 * 256 * 256 / threads);
+  const int want = std::min(h, fit > 1 || h <= 16 ? std::min(fill, fit) : fill), band = (h + want - 1) / want, bands = (h + band - 1) / band;
   const int columns = B * bands * w;
   hipLaunchKernelGGL(dwconv3x3_columns_kernel<T>, dim3((columns + 15) / 16, (C + kStencilGroup - 1) / kStencilGroup), dim3(256), 0, stream,
                      (const T*)x, wt, bias, (T*)y, (T*)pre, columns, h, w, C, bands, band, silu);
