@@ -712,9 +712,10 @@ __global__ __launch_bounds__(256) void dwconv3x3_columns_kernel(const T* __restr
   }
 }
 
-// The columns form while quads x columns of all images are no more than this.  Beyond, a thread to a column fills the chip without bands, the
+// The columns form while quads x columns of all images are no more than this.  Beyond, two bands are more threads than the chip takes at once, the
 // form is bound by its vector work (a quad's row costs as much around its 36 products as in them) and the staged form's bands of a whole
-// image are quicker.  us, staged / columns, bf16 unless said: C 384 32 x 14 x 14 9.8 / 8.1, 64 images 13.2 / 10.6, 90 (120 k) 15.8 / 12.2, 128
+// image are quicker than two of its bands (than one only where images are tall: inputs from memory, us, staged / one / two: C 192 172 k columns 14 x 14 16.7 / 15.8 / 16.7,
+// 198 k 48 x 48 52.0 / 53.8 / 48.7).  us, staged / columns, bf16 unless said: C 384 32 x 14 x 14 9.8 / 8.1, 64 images 13.2 / 10.6, 90 (120 k) 15.8 / 12.2, 128
 // (172 k) 17.3 / 19.5, 256 23.3 / 26.0; C 192 128 images (86 k) 11.6 / 9.0, 256 (172 k) 15.1 / 15.7, 8 x 64 x 64 12.8 / 10.3, 3 x 48 x 48 8.0 / 6.2;
 // C 768 64 x 14 x 14 (172 k) 14.8 / 16.0, 10 x 32 x 32 15.2 / 11.8; fp32 C 768 8 x 32 x 32 18.2 / 13.8, C 192 8 x 48 x 48 15.6 / 10.2; one image
 // 14 x 14 4.3 / 3.9.
