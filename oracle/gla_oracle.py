@@ -1,8 +1,8 @@
 """CPU oracle for ViG's bidirectional gated-linear-attention (GLA) forward path.
 
 TEST INFRASTRUCTURE ONLY.  Nothing in the shipped package imports this module; it
-is the checker used by tests/, by __graft_entry__.smoke() and by the cpu_baseline
-leg of bench.py.  The product path is the HIP library and fails loudly without it.
+is what tests/ and __graft_entry__.smoke() compare with, and the cpu_baseline leg
+of bench.py.  The product path is the HIP library and fails loudly without it.
 
 Every function restates, in float64 numpy (or float32 torch for the timed CPU
 baseline), the arithmetic of one reference routine; the reference file:line it

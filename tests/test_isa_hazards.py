@@ -128,7 +128,7 @@ def stale_scalars(asm: str):
     return found
 
 
-def test_checker_sees_stale_scalars():
+def test_walk_sees_stale_scalars():
     asm = """
 \tv_readfirstlane_b32 s5, v1
 \tv_readfirstlane_b32 s4, v0

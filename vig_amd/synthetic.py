@@ -3,7 +3,7 @@
 The distributions mirror what ViG's block feeds the op
 (classification/models/vig.py:432-441): q, k, v ~ N(0,1) with k pre-scaled by
 Dk^-0.5, and per-direction log-gates logsigmoid(N(0,1))/16.  Everything is drawn
-on the CPU from one torch.Generator so the GPU box and the CPU checker see the
+on the CPU from one torch.Generator so that a GPU run and the oracle see the
 same numbers; draw order is q, k, v, g_fwd, g_bwd.
 """
 from __future__ import annotations
@@ -57,7 +57,7 @@ def torch_dtype(name: str) -> torch.dtype:
 def make_gla_inputs(B, H, L, Dk, Dv, seed, dtype=torch.float32, gate_scale=1.0 / 16.0):
     """Returns (q, k, v, g_fwd, g_bwd) as CPU tensors of `dtype`.
 
-    Generated in float32 and rounded once to `dtype`; a checker must consume the
+    Generated in float32 and rounded once to `dtype`; the oracle must consume the
     rounded tensors (input rounding alone moves bf16 outputs by ~1e-2).
     """
     gen = torch.Generator(device="cpu").manual_seed(seed)
