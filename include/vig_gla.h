@@ -594,7 +594,7 @@ int vig_locality_blend_linear_kept_fwd(const void* o, const void* local, const v
  *   w_packed [Cout, Cin*KH, 16] bf16: the kernel rows of the [Cout, Cin, KH, KW] weight, each padded with zeros to
  *   16 columns.
  * Built for the reference's stem: stride 8, padding 1, KW <= 16 (9 where W > 248), Cin*KH = 27 (3 channels x 9 rows),
- * W % 8 == 0, Cout a multiple of 32 from 64 to 256; anything else returns VIG_ENOTSUP (use a library convolution).
+ * W % 8 == 0, Cout a multiple of 32 from 64 to 256, or 384; anything else returns VIG_ENOTSUP (use a library convolution).
  *
  * Replaces: the first nn.Conv2d of V2PatchEmbed (classification/models/vig.py:651) and the layout change a
  * channels-last convolution library needs in front of it.

@@ -429,7 +429,7 @@ PyObject* run_plan(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const int64_t B = images.size(0), S = images.size(2), W = images.size(3), half = st.w1.size(0);
   const int64_t oh1 = (S + 2 - st.KH) / 8 + 1, ow1 = (W + 2 - st.KW) / 8 + 1;
   // the stem's shape, and the grid the position table is for
-  if (B > 65535 || images.size(1) * st.KH != 27 || st.KW > 16 || (W > 248 && st.KW > 9) || S + 2 < st.KH || W % 8 || W + 2 < st.KW || half % 32 || half < 64 || half > 256 ||
+  if (B > 65535 || images.size(1) * st.KH != 27 || st.KW > 16 || (W > 248 && st.KW > 9) || S + 2 < st.KH || W % 8 || W + 2 < st.KW || half % 32 || half < 64 || (half > 256 && half != 384) ||
       (oh1 + 1) / 2 != st.gh || (ow1 + 1) / 2 != st.gw || B * oh1 * ow1 > 0x7fffffff - 8192)
     Py_RETURN_NONE;
   if (!still_valid(*p)) Py_RETURN_FALSE;

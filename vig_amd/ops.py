@@ -896,7 +896,7 @@ def patch_conv_supported(x: torch.Tensor, weight: torch.Tensor, stride: int, pad
     Cout, Cin, KH, KW = weight.shape
     return (x.dtype == torch.bfloat16 and x.is_cuda and x.dim() == 4 and stride == 8 and padding == 1 and KW <= 16
             and Cin * KH == 27 and x.shape[1] == Cin and x.shape[3] % 8 == 0
-            and (x.shape[3] <= 248 or KW <= 9) and Cout % 32 == 0 and 64 <= Cout <= 256)
+            and (x.shape[3] <= 248 or KW <= 9) and Cout % 32 == 0 and (64 <= Cout <= 256 or Cout == 384))
 
 
 def patch_conv(x: torch.Tensor, w_packed: torch.Tensor, kernel_hw, stride: int = 8, padding: int = 1) -> torch.Tensor:
