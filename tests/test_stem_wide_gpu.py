@@ -38,3 +38,15 @@ def test_planned_forward_768(B, side):
         modules = net.head(net.forward_features(images))
     err = (planned.float() - modules.float()).norm() / modules.float().norm()
     assert err.item() <= 2e-2, err.item()  # bf16 activations of two blocks, products in another order
+
+
+# one size for each tile shape of the rule, ragged rows and columns (64 x 192, 128 x 128, 128 x 192 in turn)
+@pytest.mark.parametrize("B,H,W,Cin,Cout", [(33, 28, 27, 64, 760), (47, 28, 28, 64, 760), (63, 27, 28, 64, 760)])
+def test_conv3x3s2_tiles(B, H, W, Cin, Cout):
+    announce(f"3x3 stride-2 convolution B{B} {H}x{W} {Cin}->{Cout}")
+    g = torch.Generator().manual_seed(12)
+    x, w = torch.randn(B, Cin, H, W, generator=g).bfloat16(), (torch.randn(Cout, Cin, 3, 3, generator=g) * (9 * Cin) ** -0.5).bfloat16()
+    got = ops.conv3x3s2(x.cuda().contiguous(memory_format=torch.channels_last), w.cuda().contiguous(memory_format=torch.channels_last))
+    want = torch.nn.functional.conv2d(x.double(), w.double(), None, 2, 1)
+    err = (got.double().cpu() - want).abs() / want.abs().clamp_min(1.0)
+    assert err.max().item() <= 2.0 ** -7, err.max().item()

@@ -750,8 +750,27 @@ int launch_few_blend_linear(const void* o, const void* loc, const void* glin, co
 }
 
 // The convolution library took 12 to 138 us where these take 4.3 to 96: B 1, 28 x 28 x 96 -> 192 4.3 / 12.3; B 32, 192 -> 384
-// 26 / 54; B 256 96 / 137.  Long contractions (27 to 108 stages) want eight waves a tile while tiles are fewer than CUs, and
-// 192-column tiles once there is a tile for every CU.
+// 26 / 54; B 256 96 / 137.  Long contractions (27 to 108 stages) want eight waves a tile while tiles are fewer than CUs.
+// Past 640 tiles of 32 x 32 the tile of least estimated time: what it takes alone on its CU a stage, two of them on one CU `pair`
+// times that (64 x 64: five fit, half a tile's time each from the third on).  28 x 28 inputs, us, "64 x 64 tiles, 128 x 192 once there is one
+// for every CU" / this: 192 -> 384 32 images 26.5 / 23.8, 64 42.4 / 31.4, 96 46.8 / 39.4; 384 -> 768 24 61.6 / 54, 32 81.8 / 55.6, 40 93 / 65, 48
+// 85.8 / 72.8, 96 152 / 143; 96 -> 192 96 20.1 / 18.2, 128 24.1 / 19.2; the rest as before.
+struct TapsTile {
+  int tm, tn;
+  float stage, pair;
+};
+constexpr TapsTile kTapsTiles[] = {{64, 64, 0.26f, 1.23f}, {64, 192, 0.37f, 1.35f}, {128, 128, 0.47f, 1.3f}, {128, 192, 0.535f, 1.42f}};
+static int taps_tile(const GemmArgs& a) {
+  int best = 0;
+  float least = 0.f;
+  for (int i = 0; i < 4; ++i) {
+    const TapsTile& t = kTapsTiles[i];
+    const long long deep = (tiles_of(a, t.tm, t.tn) + 255) / 256;
+    const float rounds = i == 0 && deep > 2 ? 0.5f * deep : (deep >> 1) * t.pair + (deep & 1);
+    if (i == 0 || t.stage * rounds < least) least = t.stage * rounds, best = i;
+  }
+  return best;
+}
 int launch_conv3x3s2(const void* x, const void* w, void* y, int B, int H, int W, int Cin, int Cout, hipStream_t stream) {
   const int oh = (H + 1) / 2, ow = (W + 1) / 2;
   const long long M = (long long)B * oh * ow;
@@ -760,7 +779,11 @@ int launch_conv3x3s2(const void* x, const void* w, void* y, int B, int H, int W,
   if (tiles_of(a, 64, 64) > 0x7fffffffLL - 8) return -95;
   if (tiles_of(a, 32, 32) <= 256) return launch_few<8, kTaps>(a, stream);
   if (tiles_of(a, 32, 32) <= kFewTiles) return launch_few<4, kTaps>(a, stream);
-  if (tiles_of(a, 128, 192) >= 256) return launch_many<2, 3, 4, true>(a, stream);
+  switch (taps_tile(a)) {
+    case 1: return launch_many<1, 3, 4, true>(a, stream);
+    case 2: return launch_many<2, 2, 4, true>(a, stream);
+    case 3: return launch_many<2, 3, 4, true>(a, stream);
+  }
   return launch_many<1, 1, 4, true>(a, stream);
 }
 
