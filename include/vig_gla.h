@@ -627,6 +627,18 @@ int vig_norm_dwconv3x3_fwd(const void* x, const void* residual, const float* nor
                            void* sum, void* y, int B, int h, int w, int C, float eps, int silu, void* stream);
 
 /*
+ * The same with a row product behind the convolution: sum as above (may be NULL), conv [B, h*w, C] the convolution's result,
+ * y [B, h*w, N] = conv . weight [N, C]^T (+ bias [N] bf16, or NULL), as vig_norm_dwconv3x3_fwd and vig_linear_fwd give one after the other.
+ * C = 192 or 384, N % 64 == 0 and few images (vig_norm_dwconv3x3_linear_preferred), else VIG_ENOTSUP.  No output may be an input.
+ *
+ * Replaces: classification/models/vig.py:291-294,364-369,598-606 (attn_norm, local convolution, projections).
+ */
+int vig_norm_dwconv3x3_linear_preferred(int B, int h, int w, int C, int N);
+int vig_norm_dwconv3x3_linear_fwd(const void* x, const void* residual, const float* norm_weight, const float* conv_weight,
+                                  const float* conv_bias, const void* weight, const void* bias, void* sum, void* conv, void* y, int B,
+                                  int h, int w, int C, int N, float eps, int silu, void* stream);
+
+/*
  * Residual add, RMS norm and the SwiGLU layer behind it in one kernel, bf16, packed rows:
  *   sum [rows, K] = x + residual (stored rounded; the norm is of the sum in fp32),  y [rows, I] = SwiGLU of rms(sum) * norm_weight . weight^T,
  * weight [2*I, K] with the gate rows first: what vig_rmsnorm_fwd (round_sum 0) and vig_linear_swiglu_fwd give one after the other.

@@ -597,6 +597,24 @@ int vig_norm_dwconv3x3_fwd(const void* x, const void* residual, const float* nor
   return vig::launch_norm_dwconv3x3(x, residual, norm_weight, weight, bias, sum, y, B, h, w, C, eps, silu, (hipStream_t)stream);
 }
 
+int vig_norm_dwconv3x3_linear_preferred(int B, int h, int w, int C, int N) {
+  return B > 0 && h > 0 && w > 0 && N > 0 && vig::norm_conv_linear_supported(B, h, w, C, N);
+}
+
+int vig_norm_dwconv3x3_linear_fwd(const void* x, const void* residual, const float* norm_weight, const float* conv_weight,
+                                  const float* conv_bias, const void* weight, const void* bias, void* sum, void* conv, void* y, int B,
+                                  int h, int w, int C, int N, float eps, int silu, void* stream) {
+  if (!x || !norm_weight || !conv_weight || !weight || !conv || !y || B <= 0 || h <= 0 || w <= 0 || C <= 0 || N <= 0) return VIG_EINVAL;
+  // (a workgroup reads its neighbours' rows: nothing may be written over an input)
+  for (const void* out : {(const void*)sum, (const void*)conv, (const void*)y})
+    if (out && (out == x || out == residual || out == weight)) return VIG_EINVAL;
+  if (conv == y || conv == sum || y == sum) return VIG_EINVAL;
+  if (!aligned16(x, residual, norm_weight, conv_weight, sum, conv) || !aligned16(conv_bias, weight, bias, y)) return VIG_EINVAL;
+  if (!vig::norm_conv_linear_supported(B, h, w, C, N)) return VIG_ENOTSUP;
+  return vig::launch_norm_conv_linear(x, residual, norm_weight, conv_weight, conv_bias, weight, bias, sum, conv, y, B, h, w, C, N, eps, silu,
+                                      (hipStream_t)stream);
+}
+
 size_t vig_dwconv3x3_bwd_weight_workspace(int B, int C) {
   if (B <= 0 || C <= 0) return 0;
   return vig::dwconv3x3_wgrad_workspace(B, C);

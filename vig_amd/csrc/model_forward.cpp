@@ -201,16 +201,23 @@ Tensor run(const Plan& p, const Tensor& images) {
     const bool sums = !normed && residual >= 0;
     if (normed) hidden = residual;
     else if (sums) hidden = residual == res0 ? res1 : res0;
-    if (!normed && vig_norm_dwconv3x3_preferred((int)B, st.gh, st.gw, (int)C)) {
-      check_rc(vig_norm_dwconv3x3_fwd(k.at(branch0), sums ? k.at(residual) : nullptr, f32(b.norm1), f32(b.conv_w), f32(b.conv_b),
-                                      sums ? k.at(hidden) : nullptr, k.at(xs), (int)B, st.gh, st.gw, (int)C, (float)b.eps1, b.act, k.stream),
-               "vig_norm_dwconv3x3_fwd");
+    if (!normed && vig_norm_dwconv3x3_linear_preferred((int)B, st.gh, st.gw, (int)C, (int)ld)) {
+      check_rc(vig_norm_dwconv3x3_linear_fwd(k.at(branch0), sums ? k.at(residual) : nullptr, f32(b.norm1), f32(b.conv_w), f32(b.conv_b),
+                                             b.w_in.data_ptr(), b.b_in.data_ptr(), sums ? k.at(hidden) : nullptr, k.at(xs), k.at(z), (int)B,
+                                             st.gh, st.gw, (int)C, (int)ld, (float)b.eps1, b.act, k.stream),
+               "vig_norm_dwconv3x3_linear_fwd");
     } else {
-      if (!normed) k.norm(branch0, sums ? residual : -1, b.norm1, b.eps1, sums, y, sums ? hidden : -1, T);
-      check_rc(vig_dwconv3x3_fwd(k.at(y), f32(b.conv_w), f32(b.conv_b), k.at(xs), (int)B, st.gh, st.gw, (int)C, b.act, VIG_BF16, k.stream),
-               "vig_dwconv3x3_fwd");
+      if (!normed && vig_norm_dwconv3x3_preferred((int)B, st.gh, st.gw, (int)C)) {
+        check_rc(vig_norm_dwconv3x3_fwd(k.at(branch0), sums ? k.at(residual) : nullptr, f32(b.norm1), f32(b.conv_w), f32(b.conv_b),
+                                        sums ? k.at(hidden) : nullptr, k.at(xs), (int)B, st.gh, st.gw, (int)C, (float)b.eps1, b.act, k.stream),
+                 "vig_norm_dwconv3x3_fwd");
+      } else {
+        if (!normed) k.norm(branch0, sums ? residual : -1, b.norm1, b.eps1, sums, y, sums ? hidden : -1, T);
+        check_rc(vig_dwconv3x3_fwd(k.at(y), f32(b.conv_w), f32(b.conv_b), k.at(xs), (int)B, st.gh, st.gw, (int)C, b.act, VIG_BF16, k.stream),
+                 "vig_dwconv3x3_fwd");
+      }
+      k.linear(xs, b.w_in, b.b_in, z, T);
     }
-    k.linear(xs, b.w_in, b.b_in, z, T);
     const float scale = 1.0f / std::sqrt((float)b.Dk);
     const long long sqk[3] = {(long long)(L * ld), b.Dk, ld}, sv[3] = {(long long)(L * ld), b.Dv, ld};
     if (lowrank(b)) {
