@@ -65,6 +65,7 @@ struct TileGeo {
   const uint16_t *low, *up_w, *up_b;
   long long low_ld;
   float inv_norm, clamp;
+  int spread;               // nonzero: grid (sequence, query tile), gla_spread_kernel
 };
 
 // Sequences of more tiles than this (MANY below): a far tile's q^ has picked up the decays of up to fifteen tiles, and a product
@@ -119,6 +120,7 @@ struct TileCtx {
   const uint16_t *up_w[2], *up_b[2];
   int nvalid;  // tokens of the tile
   float inv_norm, clamp;
+  bool silent;  // another workgroup stores this tile's outputs
 };
 
 // What a wave fetches to make its tile's gates: its tokens' rank-16 rows and, per direction, the weights and the bias of a lane's
@@ -850,6 +852,7 @@ __device__ __forceinline__ void tile_pass(const TileCtx& cx, const TileKernArgs*
                            GENERAL ? -(ek + ev) : 0, qhb, O);
   float os = cx.oscale;
   if (GENERAL) os *= __builtin_amdgcn_exp2f((float)(eq + ek + ev));
+  if (GENERAL && cx.silent) return;
   if (GATE) {
     locality_gate_epilogue(O[0], O[1], os, lds, cx.gate_w, cx.o, cx.gw, cx.gh, ti, NT, lane_w);
     return;
@@ -864,17 +867,20 @@ __device__ __forceinline__ void tile_pass(const TileCtx& cx, const TileKernArgs*
   }
 }
 
+__device__ __forceinline__ int own_tile() { return __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6); }
+
 template <int NG, bool BIDIR, bool PITCHED, bool GATE, bool CHAIN, bool LOW>
 __device__ __forceinline__ TileCtx make_tile_ctx(const uint16_t* q, const uint16_t* k, const uint16_t* v,
                                                  const uint16_t* gf, const uint16_t* gb, uint16_t* o,
-                                                 const TileGeo& geo, float oscale, const float* gate_w, char* lds) {
+                                                 const TileGeo& geo, float oscale, const float* gate_w, char* lds, int ti) {
   constexpr int DK = 16 * NG;
   TileCtx cx;
   cx.lds = lds;
   cx.gw = GATE ? geo.gw : 0, cx.gh = GATE ? geo.gh : 0;
   // (slab = batch element * heads + head)
   cx.gate_w = GATE ? gate_w + (size_t)((int)blockIdx.x % geo.heads) * (64 * 9) : nullptr;
-  cx.ti = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  cx.ti = ti;
+  cx.silent = !CHAIN && geo.spread && ti != (int)blockIdx.y;
   cx.lane = threadIdx.x & 63;
   cx.NT = geo.NT;
   cx.oscale = oscale;
@@ -937,7 +943,7 @@ __device__ __noinline__ void tile_pass_general(const TileKernArgs* ka_in) {
                                      (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)kp));
   const TileGeo geo = ka->geo;
   const TileCtx cx = make_tile_ctx<NG, BIDIR, PITCHED, GATE, CHAIN, LOW>(ka->q, ka->k, ka->v, ka->gf, ka->gb, ka->o, geo,
-                                                                     ka->oscale, ka->gate_w, lds);
+                                                                     ka->oscale, ka->gate_w, lds, own_tile());
   tile_pass<NG, BIDIR, PITCHED, true, GATE, CHAIN, LOW, MANY>(cx, nullptr);
 #endif
 }
@@ -953,7 +959,7 @@ __global__ __launch_bounds__(1024, 4) void gla_tile_kernel(const uint16_t* __res
                                                           const float* __restrict__ gate_w) {
   extern __shared__ __align__(16) char lds[];
   const TileKernArgs* ka = (const TileKernArgs*)__builtin_amdgcn_kernarg_segment_ptr();
-  const TileCtx cx = make_tile_ctx<NG, BIDIR, PITCHED, GATE, CHAIN, LOW>(q, k, v, gf, gb, o, geo, oscale, gate_w, lds);
+  const TileCtx cx = make_tile_ctx<NG, BIDIR, PITCHED, GATE, CHAIN, LOW>(q, k, v, gf, gb, o, geo, oscale, gate_w, lds, own_tile());
   tile_pass<NG, BIDIR, PITCHED, false, GATE, CHAIN, LOW, MANY>(cx, ka);
 }
 
@@ -969,8 +975,271 @@ __global__ __launch_bounds__(512, 2) void gla_tile_wide_kernel(const uint16_t* _
                                                                TileGeo geo, float oscale,
                                                                const float* __restrict__ gate_w) {
   extern __shared__ __align__(16) char lds[];
-  const TileCtx cx = make_tile_ctx<NG, BIDIR, PITCHED, GATE, CHAIN, LOW>(q, k, v, gf, gb, o, geo, oscale, gate_w, lds);
+  const TileCtx cx = make_tile_ctx<NG, BIDIR, PITCHED, GATE, CHAIN, LOW>(q, k, v, gf, gb, o, geo, oscale, gate_w, lds, own_tile());
   tile_pass<NG, BIDIR, PITCHED, true, GATE, CHAIN, LOW, false>(cx, nullptr);
+}
+
+// ---------------------------------------------------------------------------
+// Few sequences of five to eight tiles: a workgroup per query tile instead of one per sequence.  What a lone workgroup of the kernel above waits
+// for is its own CU: of 14.7 thousand clocks at seven tiles, Dk 32, 2.3 go by until the rows are there, 7 until every wave has prepared
+// its tile in both directions (two waves to a SIMD), 3.5 for six steps of the walk, whose operands are 6 KB of LDS a wave and step.
+// Here wave j has key tile j against the workgroup's one query tile i: one direction (forward before i, reverse behind it), keys alone, in
+// registers from the load to the product, no walk; the tile's own pairs are wave i's (forward) and one wave's more (reverse).
+//   1. cumulative gates and totals of the wave's tile and direction; totals to LDS, barrier
+//   2. key waves: k^ = k exp(T + totals of the tiles between - G), rounded once; query waves: q^ to LDS and their half of the diagonal; barrier
+//   3. key waves: P = k^ q^, O = V^T P; every wave leaves its 32 x 64 partial sums in LDS, barrier, the workgroup adds them up and stores.
+// Keys, values and gates are read by every workgroup of the sequence, out of the L2.  us, workgroup a sequence / this: 3
+// sequences of 49 tokens, Dk 32 4.2 / 3.8, of 100 5.0 / 4.4, of 196 7.2 / 5.0, of 256 7.6 / 5.5; Dk 64, of 196 9.5 / 6.3, of 256 10.3 / 6.9.
+// Outside the fp16 form's range a workgroup runs the general form of the whole sequence and stores its own tile of it.
+// ---------------------------------------------------------------------------
+template <int NG>
+struct SpreadLds {
+  static constexpr int kQuery = NG * 1024;  // q^ of one direction
+  int totals, scratch, part, guard, total;
+  __host__ __device__ explicit SpreadLds(int NT) {
+    totals = 2 * kQuery;
+    scratch = totals + (NT + 1) * 256;
+    part = scratch + (NT + 1) * 256;
+    guard = part + (NT + 1) * 8192;
+    const int general = TileLds<NG>(NT, 0, false).total;  // (whose waves may write while others still read the guard)
+    if (guard < general) guard = general;
+    total = guard + 64;
+  }
+};
+
+template <int NG, bool PITCHED, bool LOW>
+__global__ __launch_bounds__(576, 3) void gla_spread_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
+                                                            const uint16_t* __restrict__ v, const uint16_t* __restrict__ gf,
+                                                            const uint16_t* __restrict__ gb, uint16_t* __restrict__ o, TileGeo geo,
+                                                            float oscale, const float* __restrict__ gate_w) {
+  extern __shared__ __align__(16) char lds[];
+  const TileKernArgs* ka = (const TileKernArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+  const int NT = geo.NT, qi = blockIdx.y, wave = own_tile();
+  const bool query = wave == qi || wave == NT, fwd = wave <= qi;
+  const TileCtx cx = make_tile_ctx<NG, true, PITCHED, false, false, LOW>(q, k, v, gf, gb, o, geo, oscale, gate_w, lds, wave == NT ? qi : wave);
+  const SpreadLds<NG> lay(NT);
+  const int lane = cx.lane, r = lane & 31, h = lane >> 5;
+  // ---- loads ----
+  uint32_t gD[2][8], vD[2][8];
+  u32x4_t rawq[NG], rawk[NG], lowx, loww;
+  uint32_t lowb = 0;
+  if (LOW) {
+    const int c = 2 * cpair<2>(r & 15) + (r >> 4);
+    lowx = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(cx.low, (unsigned)r * cx.low_pitch + 16u * h, 0, 0));
+    loww = *reinterpret_cast<const u32x4_t*>((fwd ? cx.up_w[0] : cx.up_w[1]) + 16 * c + 8 * h);
+    lowb = (fwd ? cx.up_b[0] : cx.up_b[1])[c];
+  } else {
+    const size_t off = ((size_t)blockIdx.x * geo.L + 32 * cx.ti) * (16 * NG);
+    issue_tdwords<0, 2, NG>(chunk_rsrc((fwd ? gf : gb) + off, min(32, geo.L - 32 * cx.ti), 32 * NG), r, h, gD);
+  }
+  if (PITCHED) issue_raw_tile_pitched<NG>(cx.k, 0, r, h, cx.k_pitch, rawk);
+  else issue_raw_tile<NG>(cx.k, 0, r, h, rawk);
+  if (query) {
+    if (PITCHED) issue_raw_tile_pitched<NG>(cx.q, 0, r, h, cx.q_pitch, rawq);
+    else issue_raw_tile<NG>(cx.q, 0, r, h, rawq);
+  } else {
+#pragma unroll
+    for (int g = 0; g < NG; ++g) rawq[g] = u32x4_t{0u, 0u, 0u, 0u};
+  }
+  if (PITCHED) issue_tdwords_pitched<0, 2, 4>(cx.v, r, h, cx.v_pitch, vD);
+  else issue_tdwords<0, 2, 4>(cx.v, r, h, vD);
+  // ---- 1: cumulative gates G[p][4g+m] = channel 8*NG*h + 8g + 2m + p of token r; totals ----
+  const uint32_t keep = (fwd ? (2u << r) - 1u : 0xFFFFFFFFu << r) >> (4 * h);
+  float* const totals = reinterpret_cast<float*>(lds + lay.totals);
+  f32x16_t G[2];
+  {
+    const u32x4_t tri0 = keep_masks<0>(keep) & 0x3F803F80u, tri1 = keep_masks<1>(keep) & 0x3F803F80u;
+    if constexpr (LOW) {
+      f32x16_t acc = {0.f};
+      acc = mfma(lowx, loww, acc);
+      u32x4_t gate[2];
+      lowrank_to_gates(acc, __uint_as_float(lowb << 16), cx.inv_norm, cx.clamp, cx.nvalid, h, gate);
+      f32x16_t c = {0.f};
+      c = mfma(gate[0], tri0, c);
+      c = mfma(gate[1], tri1, c);
+      G[0] = c;
+    } else {
+      u32x4_t gfrag[2][2];
+      finish_tfrags<2>(gD, gfrag);
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        f32x16_t c = {0.f};
+        c = mfma(gfrag[0][p], tri0, c);
+        c = mfma(gfrag[1][p], tri1, c);
+        G[p] = c;
+      }
+    }
+  }
+  const auto gates = [&](int p, int c) { return LOW ? G[0][8 * p + c] : G[p][c]; };
+  {
+    float* const sc = totals + 64 * wave;
+    if constexpr (LOW) asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 3" : "+v"(G[0]));  // (as in park_totals)
+    else asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 3" : "+v"(G[0]), "+v"(G[1]));
+    if (r == (fwd ? 31 : 0)) {
+#pragma unroll
+      for (int p = 0; p < 2; ++p)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          *reinterpret_cast<f32x4_t*>(sc + 32 * h + 16 * p + 4 * g) =
+              g < (LOW ? 2 : 4) ? f32x4_t{gates(p, 4 * g), gates(p, 4 * g + 1), gates(p, 4 * g + 2), gates(p, 4 * g + 3)} : f32x4_t{0.f, 0.f, 0.f, 0.f};
+    }
+    wave_lds_sync();
+  }
+  // ---- magnitudes, as in tile_pass; fp16 operands ----
+  float* const guard = reinterpret_cast<float*>(lds + lay.guard);
+  u32x4_t vf[2][2];
+  {
+    finish_tfrags<2>(vD, vf);
+    f32x4acc_t gq = {0.f, 0.f, 0.f, 0.f}, gk = gq, gv = gq;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int p = 0; p < 2; ++p) gram_acc(vf[t][p], gv);
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+      gram_acc(rawq[g], gq);
+      gram_acc(rawk[g], gk);
+    }
+    const float mq = fmaxf(fmaxf(fabsf(gq[0]), fabsf(gq[1])), fmaxf(fabsf(gq[2]), fabsf(gq[3])));
+    const float mk = fmaxf(fmaxf(fabsf(gk[0]), fabsf(gk[1])), fmaxf(fabsf(gk[2]), fabsf(gk[3])));
+    const float mv = fmaxf(fmaxf(fabsf(gv[0]), fabsf(gv[1])), fmaxf(fabsf(gv[2]), fabsf(gv[3])));
+    const float tl = totals[64 * wave + lane] * kLog2e;
+    const bool veto = __builtin_amdgcn_ballot_w64(!(mq < kMaxSquaresQ) || !(mk < kMaxSquaresK) || !(mv < kMaxSquaresV) || !(fabsf(tl) <= kTileRange)) != 0;
+    if (lane == 0) guard[wave] = veto ? 1.0f : 0.0f;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int p = 0; p < 2; ++p)
+#pragma unroll
+        for (int x = 0; x < 4; ++x) vf[t][p][x] = pack_f16x2(bf16lo_to_f32(vf[t][p][x]), bf16hi_to_f32(vf[t][p][x]));
+#pragma unroll
+    for (int g = 0; g < NG; ++g)
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        rawq[g][m] = pack_f16x2(bf16lo_to_f32(rawq[g][m]), bf16hi_to_f32(rawq[g][m]));
+        rawk[g][m] = pack_f16x2(bf16lo_to_f32(rawk[g][m]), bf16hi_to_f32(rawk[g][m]));
+      }
+  }
+  lds_barrier();  // the totals are visible
+  {
+    const float mine = lane <= NT ? guard[lane] : 0.0f;
+    if (__builtin_amdgcn_ballot_w64(mine != 0.0f) != 0) {
+      if (wave < NT) tile_pass_general<NG, true, PITCHED, false, false, LOW, false>(ka);
+      __builtin_amdgcn_endpgm();
+    }
+  }
+  // ---- 2 ----
+  f32x16_t O[2] = {f32x16_t{0.f}, f32x16_t{0.f}};
+  u32x4_t kf[NG];
+  char* const qreg = lds + (fwd ? 0 : SpreadLds<NG>::kQuery);
+  if (query) {
+    u32x4_t qh[NG];
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        const float x0 = gates(0, 4 * g + m) * kLog2e, x1 = gates(1, 4 * g + m) * kLog2e;
+        qh[g][m] = mul_f16x2(rawq[g][m], pack_f16x2(exp2_fast(x0), exp2_fast(x1)));
+        kf[g][m] = mul_f16x2(rawk[g][m], pack_f16x2(exp2_fast(-x0), exp2_fast(-x1)));  // k' = k exp(-G)
+      }
+      *reinterpret_cast<u32x4_t*>(unit_ptr(qreg, g, lane)) = qh[g];
+    }
+    const f32x16_t P = score_tile16<NG>(kf, qh);
+    const u32x4_t m0 = keep_masks<0>(keep), m1 = keep_masks<1>(keep);
+    u32x4_t p16[2];
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+      const int c = 4 * (x >> 1) + 2 * (x & 1);
+      p16[0][x] = pack_f16x2(P[c], P[c + 1]) & m0[x];
+      p16[1][x] = pack_f16x2(P[8 + c], P[8 + c + 1]) & m1[x];
+    }
+    apply_values16(p16, vf, O);
+  } else {
+    float sum = 0.f;
+    const int near = fwd ? wave : qi + 1, far = fwd ? qi - 1 : wave;  // the wave's own tile and those between
+    for (int t = near; t <= far; ++t) sum += totals[64 * t + lane];
+    float* const sc = reinterpret_cast<float*>(lds + lay.scratch) + 64 * wave;
+    sc[lane] = sum * kLog2e;
+    wave_lds_sync();
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+      const f32x4_t d0 = *reinterpret_cast<const f32x4_t*>(sc + 32 * h + 4 * g), d1 = *reinterpret_cast<const f32x4_t*>(sc + 32 * h + 16 + 4 * g);
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        const float x0 = gates(0, 4 * g + m) * kLog2e, x1 = gates(1, 4 * g + m) * kLog2e;
+        kf[g][m] = mul_f16x2(rawk[g][m], pack_f16x2(exp2_fast(d0[m] - x0), exp2_fast(d1[m] - x1)));
+      }
+    }
+  }
+  lds_barrier();  // q^ of both directions is visible
+  // ---- 3 ----
+  if (!query) {
+    u32x4_t qh[NG];
+#pragma unroll
+    for (int g = 0; g < NG; ++g) qh[g] = *reinterpret_cast<const u32x4_t*>(unit_ptr(qreg, g, lane));
+    apply_values(score_tile16<NG>(kf, qh), vf, O);
+  }
+  f32x4_t* const part = reinterpret_cast<f32x4_t*>(lds + lay.part);  // [wave][half of the channels' pairs][quarter][lane]
+#pragma unroll
+  for (int p = 0; p < 2; ++p)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) part[(8 * wave + 4 * p + g) * 64 + lane] = f32x4_t{O[p][4 * g], O[p][4 * g + 1], O[p][4 * g + 2], O[p][4 * g + 3]};
+  lds_barrier();
+  const rsrc_t out = chunk_rsrc(o + ((size_t)blockIdx.x * geo.L + 32 * qi) * 64, min(32, geo.L - 32 * qi), 128);
+  for (int g = wave; g < 4; g += NT + 1) {
+    f32x4_t a = part[g * 64 + lane], b = part[(4 + g) * 64 + lane];
+    for (int w = 1; w <= NT; ++w) a += part[(8 * w + g) * 64 + lane], b += part[(8 * w + 4 + g) * 64 + lane];
+    u32x4_t x;
+#pragma unroll
+    for (int m = 0; m < 4; ++m) x[m] = pack_bf16x2(a[m] * oscale, b[m] * oscale);
+    __builtin_amdgcn_raw_buffer_store_b128(x, out, (unsigned)r * 128u + 64u * h + 16u * g, 0, 0);
+  }
+}
+
+// The locality gate behind it, in place (there is no other room for the op's outputs): the convolution is a channel's own, so a workgroup has all tokens
+// of a sequence's sixteen channels, staged in LDS as a zero-padded grid before the first store.  A thread takes one octet of one token;
+// sums, sigmoid and rounding as in locality_gate_epilogue.
+constexpr int kSpreadGateChannels = 16;
+__global__ __launch_bounds__(512) void spread_gate_kernel(uint16_t* __restrict__ o, const float* __restrict__ weight, int L, int gw, int gh, int heads) {
+  extern __shared__ __align__(16) char lds[];
+  const int oct = threadIdx.x & 1, first = threadIdx.x >> 1, ch = blockIdx.y * kSpreadGateChannels + 8 * oct, pw = gw + 2;
+  uint16_t* const rows = o + (size_t)blockIdx.x * L * 64 + ch;
+  const f32x4_t* const wp = reinterpret_cast<const f32x4_t*>(weight + ((size_t)((int)blockIdx.x % heads) * 64 + ch) * 9);
+  float wreg[8][9];
+#pragma unroll
+  for (int i = 0; i < 18; ++i) {
+    const f32x4_t x = wp[i];
+#pragma unroll
+    for (int m = 0; m < 4; ++m) wreg[(4 * i + m) / 9][(4 * i + m) % 9] = x[m];
+  }
+  for (int c = first; c < pw * (gh + 2); c += 256) {
+    const int y = c / pw - 1, x = c - c / pw * pw - 1;
+    u32x4_t v = {0u, 0u, 0u, 0u};
+    if (y >= 0 && y < gh && x >= 0 && x < gw) v = *reinterpret_cast<const u32x4_t*>(rows + (size_t)(y * gw + x) * 64);
+    *reinterpret_cast<u32x4_t*>(lds + 2 * kSpreadGateChannels * c + 16 * oct) = v;
+  }
+  __syncthreads();
+  for (int T = first; T < L; T += 256) {
+    const int y = T / gw, x = T - y * gw;
+    float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    u32x4_t ctr = {0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int di = 0; di < 3; ++di)
+#pragma unroll
+      for (int dj = 0; dj < 3; ++dj) {
+        const u32x4_t w = *reinterpret_cast<const u32x4_t*>(lds + 2 * kSpreadGateChannels * ((y + di) * pw + x + dj) + 16 * oct);
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+          acc[2 * m] = __builtin_fmaf(bf16lo_to_f32(w[m]), wreg[2 * m][di * 3 + dj], acc[2 * m]);
+          acc[2 * m + 1] = __builtin_fmaf(bf16hi_to_f32(w[m]), wreg[2 * m + 1][di * 3 + dj], acc[2 * m + 1]);
+        }
+        if (di == 1 && dj == 1) ctr = w;
+      }
+    u32x4_t out;
+#pragma unroll
+    for (int m = 0; m < 4; ++m) out[m] = pack_bf16x2(bf16lo_to_f32(ctr[m]) * sigmoidf_(acc[2 * m]), bf16hi_to_f32(ctr[m]) * sigmoidf_(acc[2 * m + 1]));
+    *reinterpret_cast<u32x4_t*>(rows + (size_t)T * 64) = out;
+  }
 }
 
 constexpr int kTileMaxLds = 160 * 1024;
@@ -1000,6 +1269,29 @@ bool gla_tiles_supported(const GlaArgs& a) {
     if ((a.Dk == 64 ? TileLds<4>(NT, stage, NT > kFewTiles).total : TileLds<2>(NT, stage, NT > kFewTiles).total) > kTileMaxLds) return false;
   }
   return true;
+}
+
+// Whether a workgroup for each query tile is the quicker form: while there is a CU for each.  us, a workgroup a sequence / a query tile: Dk 32: 36
+// sequences of 196 (252 tiles) 7.4 / 5.4, 42 (294) 7.5 / 8.1, 96 (672) 7.8 / 11.7; 48 of 160 (240) 6.7 / 5.0, 60 (300) 6.7 / 7.8; Dk 64: 36 of
+// 196 9.7 / 6.7, 42 9.8 / 10.2; 24 of 256 (192) 10.5 / 7.2, 36 (288) 10.5 / 12.4.  From five tiles on, because the op with the locality gate
+// gives the plain op's bits and so takes the same form, with the gate behind it: 3 of 14 x 14, Dk 32 10.4 / 9.2, Dk 64 12.8 / 10.3, 36 of 12 x 13
+// 10.0 / 9.3; but 12 of 10 x 12 7.8 / 8.4, where the plain op alone would gain too (60 of 128 5.5 / 4.8).
+static bool spread_preferred(const GlaArgs& a, int NT) {
+  return NT >= 5 && NT <= kFewTiles && (long long)a.B * a.H * NT <= 256 && !a.wide_gates;
+}
+template <int NG, bool PITCHED, bool LOW>
+static int launch_spread(const GlaArgs& a, TileGeo geo, int dev) {
+  static bool done[64] = {};
+  const auto kernel = gla_spread_kernel<NG, PITCHED, LOW>;
+  const SpreadLds<NG> lay(geo.NT);
+  if (!done[dev]) {
+    if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, SpreadLds<NG>(kFewTiles).total) != hipSuccess) return -5;
+    done[dev] = true;
+  }
+  geo.spread = 1;
+  hipLaunchKernelGGL(kernel, dim3(a.B * a.H, geo.NT), dim3(64 * (geo.NT + 1)), lay.total, a.stream, (const uint16_t*)a.q, (const uint16_t*)a.k,
+                     (const uint16_t*)a.v, (const uint16_t*)a.g_fwd, (const uint16_t*)a.g_bwd, (uint16_t*)a.o, geo, a.scale * a.out_scale, a.gate_w);
+  return hipGetLastError() == hipSuccess ? 0 : -5;
 }
 
 template <int NG, bool BIDIR, bool PITCHED, bool GATE, bool CHAIN = false, bool LOW = false, bool MANY = false>
@@ -1064,13 +1356,25 @@ int launch_gla_tiles(const GlaArgs& a) {
     if (const int rc = gla_strides(a, geo.sq, geo.sk, geo.sv)) return rc;
   const bool bidir = a.g_bwd != nullptr;
   if (a.gate_w) {
+    if (spread_preferred(a, geo.NT)) {
+      if (const int rc = a.Dk == 64 ? launch_spread<4, false, false>(a, geo, dev) : launch_spread<2, false, false>(a, geo, dev)) return rc;
+      const int cells = (a.gate_cols + 2) * (a.gate_rows + 2);  // (at most 3 x 258)
+      hipLaunchKernelGGL(spread_gate_kernel, dim3(a.B * a.H, 64 / kSpreadGateChannels), dim3(512), 2 * kSpreadGateChannels * cells, a.stream,
+                         (uint16_t*)a.o, a.gate_w, a.L, a.gate_cols, a.gate_rows, a.H);
+      return hipGetLastError() == hipSuccess ? 0 : -5;
+    }
     geo.gw = a.gate_cols, geo.gh = a.gate_rows, geo.heads = a.H;
     return a.Dk == 64 ? launch_tiles_t<4, true, false, true>(a, geo, dev) : launch_tiles_t<2, true, false, true>(a, geo, dev);
   }
   geo.heads = 1;
   if (a.low) {
     fill_lowrank(a, geo);
+    if (spread_preferred(a, geo.NT)) return launch_spread<2, true, true>(a, geo, dev);
     return launch_tiles_t<2, true, true, false, false, true>(a, geo, dev);
+  }
+  if (bidir && spread_preferred(a, geo.NT)) {
+    if (pitched) return a.Dk == 64 ? launch_spread<4, true, false>(a, geo, dev) : launch_spread<2, true, false>(a, geo, dev);
+    return a.Dk == 64 ? launch_spread<4, false, false>(a, geo, dev) : launch_spread<2, false, false>(a, geo, dev);
   }
   if (a.Dk == 64) {
     if (pitched)
