@@ -615,6 +615,19 @@ int vig_linear_fwd(const void* x, long long x_row_stride, const void* weight, co
                    long long rows, int N, int K, void* stream);
 
 /*
+ * The middle of a block in one kernel, bf16, few rows of C = 192 channels (vig_locality_blend_swiglu_preferred), else VIG_ENOTSUP: what
+ * vig_locality_blend_linear_fwd (out_weight [C, C]; its result is not stored) and vig_norm_swiglu_fwd (weight [2*I, C], I % 64 == 0) give one
+ * after the other, bit for bit: sum [B*L, C], y [B*L, I].  No output may be an input.
+ *
+ * Replaces: classification/models/vig.py:444-463,606-608 and :492-497 (head norms, sigmoid blend, out_act, o_proj, mlp_norm, SwiGLU layer).
+ */
+int vig_locality_blend_swiglu_preferred(long long rows, int C, int I);
+int vig_locality_blend_swiglu_fwd(const void* o, const void* local, const void* g_lin, const float* w_g, const float* w_l,
+                                  const void* out_weight, const void* residual, const float* norm_weight, const void* weight, void* sum,
+                                  void* y, int B, int H, int L, int Dv, int C, int I, long long g_row_stride, float eps, int silu_out,
+                                  float norm_eps, void* stream);
+
+/*
  * Residual add, RMS norm and the depthwise 3x3 convolution behind it in one kernel, bf16:
  *   sum [B, h*w, C] = x + residual (rounded; residual NULL: x),  y = conv3x3(rms(sum) * norm_weight) (+ bias, SiLU): what
  * vig_rmsnorm_fwd (round_sum 1) and vig_dwconv3x3_fwd give one after the other.  weight [C, 9], bias [C] or NULL; sum may be NULL.

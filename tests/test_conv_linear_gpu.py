@@ -26,16 +26,13 @@ def test_against_separate_kernels(B, h, w, C, N, full):
     total, conv, y = (torch.full((rows, n), float("nan"), dtype=torch.bfloat16, device="cuda") for n in (C, C, N))
     assert lib.vig_norm_dwconv3x3_linear_fwd(p(x), p(res), p(nw), p(taps), p(cb), p(wt), p(b), p(total) if full else None, p(conv), p(y), B, h, w,
                                              C, N, 1e-5, full, st) == _lib.VIG_OK
-    normed, total2, conv2 = (torch.empty(rows, C, dtype=torch.bfloat16, device="cuda") for _ in range(3))
+    normed, total2, conv2, y2 = (torch.empty(rows, n, dtype=torch.bfloat16, device="cuda") for n in (C, C, C, N))
     assert lib.vig_rmsnorm_fwd(p(x), p(res), p(nw), p(normed), p(total2), rows, C, 1e-5, 1, 1, st) == _lib.VIG_OK
     assert lib.vig_dwconv3x3_fwd(p(normed), p(taps), p(cb), p(conv2), B, h, w, C, full, 1, st) == _lib.VIG_OK
     if full:
         assert torch.equal(total, total2)
-    # the same sums in the same order (vig_dwconv3x3_fwd may start its sum from the taps: one rounding of bf16 apart at most)
-    assert ((conv.float() - conv2.float()).abs() <= 2.0 ** -7 * conv2.float().abs().clamp_min(2.0 ** -6)).all()
-    want = conv.double() @ wt.double().t() + (b.double() if full else 0)
-    err = (y.double() - want).abs() / want.abs().clamp_min(1.0)
-    assert err.max().item() <= 2.0 ** -8, err.max().item()  # one rounding of the output, and fp32 sums
+    assert lib.vig_linear_fwd(p(conv2), C, p(wt), p(b), p(y2), N, rows, N, C, st) == _lib.VIG_OK
+    assert torch.equal(conv, conv2) and torch.equal(y, y2)  # the same sums in the same order
 
 
 def test_refused():

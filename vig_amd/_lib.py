@@ -87,6 +87,8 @@ SIGNATURES = {
     "vig_norm_dwconv3x3_fwd": (_c_int, [_c_void_p] * 7 + [_c_int] * 4 + [_c_float, _c_int, _c_void_p]),
     "vig_norm_dwconv3x3_linear_preferred": (_c_int, [_c_int] * 5),
     "vig_norm_dwconv3x3_linear_fwd": (_c_int, [_c_void_p] * 10 + [_c_int] * 5 + [_c_float, _c_int, _c_void_p]),
+    "vig_locality_blend_swiglu_preferred": (_c_int, [_c_longlong, _c_int, _c_int]),
+    "vig_locality_blend_swiglu_fwd": (_c_int, [_c_void_p] * 11 + [_c_int] * 6 + [_c_longlong, _c_float, _c_int, _c_float, _c_void_p]),
     "vig_norm_swiglu_preferred": (_c_int, [_c_longlong, _c_int, _c_int]),
     "vig_norm_swiglu_fwd": (_c_int, [_c_void_p] * 6 + [_c_longlong, _c_int, _c_int, _c_float, _c_void_p]),
     "vig_matmul_f32_workspace": (_c_size_t, [_c_longlong, _c_int, _c_longlong]),

@@ -760,6 +760,26 @@ int vig_locality_blend_linear_kept_fwd(const void* o, const void* local, const v
                                   (hipStream_t)stream);
 }
 
+int vig_locality_blend_swiglu_preferred(long long rows, int C, int I) { return vig::blend_swiglu_supported(rows, C, I); }
+
+int vig_locality_blend_swiglu_fwd(const void* o, const void* local, const void* g_lin, const float* w_g, const float* w_l,
+                                  const void* out_weight, const void* residual, const float* norm_weight, const void* weight, void* sum,
+                                  void* y, int B, int H, int L, int Dv, int C, int I, long long g_row_stride, float eps, int silu_out,
+                                  float norm_eps, void* stream) {
+  if (!o || !local || !g_lin || !w_g || !w_l || !out_weight || !residual || !norm_weight || !weight || !sum || !y || B <= 0 || H <= 0 || L <= 0)
+    return VIG_EINVAL;
+  // (a row is read by every workgroup of its tile: nothing may be written over an input)
+  for (const void* in : {o, local, g_lin, out_weight, residual, weight})
+    if (in == sum || in == y) return VIG_EINVAL;
+  if (sum == y) return VIG_EINVAL;
+  if (!aligned16(o, local, w_g, w_l, out_weight, residual) || !aligned16(norm_weight, weight, sum, y)) return VIG_EINVAL;
+  if (Dv != 64 || (long long)H * Dv != C || !vig::blend_swiglu_supported((long long)B * L, C, I)) return VIG_ENOTSUP;
+  const long long ldg = g_row_stride > 0 ? g_row_stride : C;
+  if (ldg < C || !strided_rows_ok(g_lin, ldg, VIG_BF16)) return VIG_EINVAL;
+  return vig::launch_blend_swiglu(o, local, g_lin, w_g, w_l, out_weight, residual, norm_weight, weight, sum, y, (long long)B * L, L, C, I, ldg,
+                                  eps, silu_out, norm_eps, (hipStream_t)stream);
+}
+
 int vig_linear_swiglu_fwd(const void* x, const void* weight, void* y, long long rows, int K, int I, int io_dtype,
                           void* stream) {
   if (!x || !weight || !y || rows <= 0 || K <= 0 || I <= 0) return VIG_EINVAL;

@@ -152,13 +152,16 @@ __global__ __launch_bounds__(C == 192 ? 512 : 1024) void conv_linear_kernel(Conv
   lds_barrier();
   // ---- the product ----
   if (wave < 8) {
-    f32x4_t sum = f32x4_t{0.f};
+    f32x4_t part[4];  // (every fourth stage a sum of its own: gemm_few_kernel's order, so its bits)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) part[k] = f32x4_t{0.f};
 #pragma unroll
     for (int k = 0; k < kStages; ++k) {
       const int off = 1024 * k + 64 * r + 16 * (quarter ^ ((r >> 2) & 3));
-      sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8_t*>(smem + weights + off),
-                                                    *reinterpret_cast<const bf16x8_t*>(smem + Lds::kRowsAt + off), sum, 0, 0, 0);
+      part[k & 3] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8_t*>(smem + weights + off),
+                                                            *reinterpret_cast<const bf16x8_t*>(smem + Lds::kRowsAt + off), part[k & 3], 0, 0, 0);
     }
+    f32x4_t sum = ((part[0] + part[1]) + part[2]) + part[3];
     // register m of lane (r, quarter) is channel 4 quarter + m of token r
     const int gy = y0 + r / kPatchW, gx = x0 + r % kPatchW;
     if (gy < a.h && gx < a.w_cells) {

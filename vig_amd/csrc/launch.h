@@ -166,6 +166,10 @@ bool norm_conv_linear_supported(int B, int h, int w, int C, int N);
 int launch_norm_conv_linear(const void* x, const void* residual, const float* norm, const float* taps, const float* conv_bias, const void* w,
                             const void* bias, void* sum, void* conv, void* y, int B, int h, int width, int C, int N, float eps, int silu,
                             hipStream_t stream);
+bool blend_swiglu_supported(long long T, int C, int N);
+int launch_blend_swiglu(const void* o, const void* loc, const void* glin, const float* w_g, const float* w_l, const void* w_out,
+                        const void* residual, const float* norm, const void* w, void* sum, void* y, long long T, int L, int C, int N,
+                        long long ldg, float eps, int silu_out, float norm_eps, hipStream_t stream);
 bool norm_swiglu_supported(long long T, int K, int I);
 int launch_norm_swiglu(const void* x, const void* residual, const float* norm, const void* w, void* sum, void* y, long long T, int K, int I,
                        float eps, hipStream_t stream);

@@ -167,8 +167,15 @@ Tensor run(const Plan& p, const Tensor& images) {
   if (!all_in_place) q = k.take(T * K2 / 2), kk = k.take(T * K2 / 2), v = k.take(T * C);
   int64_t most = k.used;
   k.used = region;
-  const int64_t mid = k.take(T * I), wide = swiglu_kernel ? 0 : k.take(T * 2 * I);
+  int64_t mid = k.take(T * I);
+  const int64_t wide = swiglu_kernel ? 0 : k.take(T * 2 * I);
   most = std::max(most, k.used);
+  const auto one_middle = [&](const Block& b) { return b.Dv == 64 && vig_locality_blend_swiglu_preferred(T, (int)C, (int)b.w_down.size(1)); };
+  if (std::any_of(p.blocks.begin(), p.blocks.end(), one_middle)) {  // (reads z while it writes mid)
+    k.used = most;
+    mid = k.take(T * I);
+    most = k.used;
+  }
   k.used = region;
   const int64_t c1 = k.take(n1 * half), c1n = k.take(n1 * half);
   most = std::max(most, k.used);
@@ -242,31 +249,38 @@ Tensor run(const Plan& p, const Tensor& images) {
                  "vig_gla_bidir_fwd");
       }
     }
-    if (b.Dv == 64 && (C == 384 || C == 192)) {
-      check_rc(vig_locality_blend_linear_fwd(k.at(o), k.at(xs), k.at(z + n0), f32(b.gn), f32(b.ln), b.w_o.data_ptr(), k.at(branch1), (int)B,
-                                             b.H, (int)L, b.Dv, (int)C, ld, (float)b.eps, b.out_act, VIG_BF16, k.stream),
-               "vig_locality_blend_linear_fwd");
-    } else {
-      check_rc(vig_locality_blend_fwd(k.at(o), k.at(xs), k.at(z + n0), f32(b.gn), f32(b.ln), k.at(y), (int)B, b.H, (int)L, b.Dv, ld,
-                                      (float)b.eps, b.out_act, VIG_BF16, k.stream),
-               "vig_locality_blend_fwd");
-      k.linear(y, b.w_o, Tensor(), branch1, T);
-    }
     const int64_t next = hidden == res0 ? res1 : res0;
     residual = next;
     const int64_t width = b.w_down.size(1);
-    const bool with_norm = swiglu_kernel && vig_norm_swiglu_preferred(T, (int)C, (int)width);
-    if (!with_norm) k.norm(branch1, hidden, b.norm2, b.eps2, false, y, next, T);
-    if (with_norm) {
-      check_rc(vig_norm_swiglu_fwd(k.at(branch1), k.at(hidden), f32(b.norm2), b.w_gate.data_ptr(), k.at(next), k.at(mid), T, (int)C, (int)width,
-                                   (float)b.eps2, k.stream),
-               "vig_norm_swiglu_fwd");
-    } else if (swiglu_kernel) {
-      check_rc(vig_linear_swiglu_fwd(k.at(y), b.w_gate.data_ptr(), k.at(mid), T, (int)C, (int)width, VIG_BF16, k.stream),
-               "vig_linear_swiglu_fwd");
+    if (one_middle(b)) {
+      check_rc(vig_locality_blend_swiglu_fwd(k.at(o), k.at(xs), k.at(z + n0), f32(b.gn), f32(b.ln), b.w_o.data_ptr(), k.at(hidden), f32(b.norm2),
+                                             b.w_gate.data_ptr(), k.at(next), k.at(mid), (int)B, b.H, (int)L, b.Dv, (int)C, (int)width, ld,
+                                             (float)b.eps, b.out_act, (float)b.eps2, k.stream),
+               "vig_locality_blend_swiglu_fwd");
     } else {
-      k.linear(y, b.w_gate, Tensor(), wide, T);
-      check_rc(vig_swiglu_fwd(k.at(wide), k.at(mid), T, (int)width, VIG_BF16, k.stream), "vig_swiglu_fwd");
+      if (b.Dv == 64 && (C == 384 || C == 192)) {
+        check_rc(vig_locality_blend_linear_fwd(k.at(o), k.at(xs), k.at(z + n0), f32(b.gn), f32(b.ln), b.w_o.data_ptr(), k.at(branch1), (int)B,
+                                               b.H, (int)L, b.Dv, (int)C, ld, (float)b.eps, b.out_act, VIG_BF16, k.stream),
+                 "vig_locality_blend_linear_fwd");
+      } else {
+        check_rc(vig_locality_blend_fwd(k.at(o), k.at(xs), k.at(z + n0), f32(b.gn), f32(b.ln), k.at(y), (int)B, b.H, (int)L, b.Dv, ld,
+                                        (float)b.eps, b.out_act, VIG_BF16, k.stream),
+                 "vig_locality_blend_fwd");
+        k.linear(y, b.w_o, Tensor(), branch1, T);
+      }
+      const bool with_norm = swiglu_kernel && vig_norm_swiglu_preferred(T, (int)C, (int)width);
+      if (!with_norm) k.norm(branch1, hidden, b.norm2, b.eps2, false, y, next, T);
+      if (with_norm) {
+        check_rc(vig_norm_swiglu_fwd(k.at(branch1), k.at(hidden), f32(b.norm2), b.w_gate.data_ptr(), k.at(next), k.at(mid), T, (int)C, (int)width,
+                                     (float)b.eps2, k.stream),
+                 "vig_norm_swiglu_fwd");
+      } else if (swiglu_kernel) {
+        check_rc(vig_linear_swiglu_fwd(k.at(y), b.w_gate.data_ptr(), k.at(mid), T, (int)C, (int)width, VIG_BF16, k.stream),
+                 "vig_linear_swiglu_fwd");
+      } else {
+        k.linear(y, b.w_gate, Tensor(), wide, T);
+        check_rc(vig_swiglu_fwd(k.at(wide), k.at(mid), T, (int)width, VIG_BF16, k.stream), "vig_swiglu_fwd");
+      }
     }
     normed = i + 1 < p.blocks.size() && vig_linear_norm_preferred(T, (int)C, (int)width);
     if (normed) {
