@@ -603,6 +603,15 @@ int vig_patch_conv_fwd(const void* x, const void* w_packed, void* y, int B, int 
                        int stride, int padding, int Cout, int io_dtype, void* stream);
 
 /*
+ * vig_patch_conv_fwd and vig_layernorm_fwd on its rows (pre_bias [Cout] or NULL, silu, no post_add) in one kernel, bit for bit; the
+ * convolution's own result is not stored.  Built for the same shapes up to Cout = 256, bf16.
+ *
+ * Replaces: the first nn.Conv2d, LayerNorm2d and SiLU of V2PatchEmbed (classification/models/vig.py:651-653).
+ */
+int vig_patch_conv_norm_fwd(const void* x, const void* w_packed, const float* norm_weight, const float* norm_bias, const float* pre_bias, void* y,
+                            int B, int Cin, int H, int W, int KH, int KW, int stride, int padding, int Cout, float eps, int silu, void* stream);
+
+/*
  * y [rows, N] = x [rows, K] . weight [N, K]^T (+ bias [N]), bf16, fp32 accumulation, the bias added before the one rounding;
  * rows of x and y x_row_stride / y_row_stride elements apart.  N % 8 == 0, K % 32 == 0.
  * vig_linear_preferred: whether this entry point is the better choice for a size (short of large products, where the BLAS

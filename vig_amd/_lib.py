@@ -61,6 +61,7 @@ SIGNATURES = {
     "vig_linear_bwd_input": (_c_int, [_c_void_p] * 3 + [_c_longlong, _c_int, _c_int, _c_int, _c_void_p]),
     "vig_linear_swiglu_fwd": (_c_int, [_c_void_p] * 3 + [_c_longlong, _c_int, _c_int, _c_int, _c_void_p]),
     "vig_patch_conv_fwd": (_c_int, [_c_void_p] * 3 + [_c_int] * 10 + [_c_void_p]),
+    "vig_patch_conv_norm_fwd": (_c_int, [_c_void_p] * 6 + [_c_int] * 9 + [_c_float, _c_int, _c_void_p]),
     "vig_locality_blend_bwd_workspace": (_c_size_t, [_c_int] * 3),
     "vig_locality_blend_bwd": (_c_int, [_c_void_p] * 11 + [_c_size_t] + [_c_int] * 4 + [_c_longlong, _c_float, _c_int,
                                                                                         _c_int, _c_void_p]),

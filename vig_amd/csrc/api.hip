@@ -67,6 +67,8 @@ int launch_linear_swiglu(const void* A, const void* W, void* out, void* kept, lo
 bool patch_conv_supported(int Cin, int H, int W, int KH, int KW, int stride, int padding, int Cout);
 int launch_patch_conv(const void* x, const void* w_packed, void* y, int B, int Cin, int H, int W, int KH, int KW,
                       int Cout, hipStream_t stream);
+int launch_patch_conv_norm(const void* x, const void* w_packed, const float* weight, const float* bias, const float* pre_bias, void* y, int B,
+                           int Cin, int H, int W, int KH, int KW, int Cout, float eps, int silu, hipStream_t stream);
 int launch_pad_channels(const void* src, void* dst, long long rows, int src_c, int dst_c, hipStream_t stream);
 int launch_pad_channels_multi(const void* const* src, void* const* dst, const int* src_c, const int* dst_c, int n,
                               long long rows, hipStream_t stream);
@@ -734,6 +736,15 @@ int vig_patch_conv_fwd(const void* x, const void* w_packed, void* y, int B, int 
   if (!strided_rows_ok(x, W, io_dtype) || !strided_rows_ok(w_packed, 16, io_dtype) || !strided_rows_ok(y, Cout, io_dtype))
     return VIG_EINVAL;
   return vig::launch_patch_conv(x, w_packed, y, B, Cin, H, W, KH, KW, Cout, (hipStream_t)stream);
+}
+
+int vig_patch_conv_norm_fwd(const void* x, const void* w_packed, const float* norm_weight, const float* norm_bias, const float* pre_bias, void* y,
+                            int B, int Cin, int H, int W, int KH, int KW, int stride, int padding, int Cout, float eps, int silu, void* stream) {
+  if (!x || !w_packed || !norm_weight || !norm_bias || !y || B <= 0 || Cin <= 0 || H <= 0 || W <= 0 || KH <= 0 || KW <= 0 || Cout <= 0)
+    return VIG_EINVAL;
+  if (!vig::patch_conv_supported(Cin, H, W, KH, KW, stride, padding, Cout)) return VIG_ENOTSUP;
+  if (!strided_rows_ok(x, W, VIG_BF16) || !strided_rows_ok(w_packed, 16, VIG_BF16) || !strided_rows_ok(y, Cout, VIG_BF16)) return VIG_EINVAL;
+  return vig::launch_patch_conv_norm(x, w_packed, norm_weight, norm_bias, pre_bias, y, B, Cin, H, W, KH, KW, Cout, eps, silu, (hipStream_t)stream);
 }
 
 int vig_locality_blend_linear_fwd(const void* o, const void* local, const void* g_lin, const float* w_g,

@@ -177,7 +177,7 @@ Tensor run(const Plan& p, const Tensor& images) {
     most = k.used;
   }
   k.used = region;
-  const int64_t c1 = k.take(n1 * half), c1n = k.take(n1 * half);
+  const int64_t c1 = k.take(n1 * half), c1n = half > 256 ? k.take(n1 * half) : c1;  // (beyond: two kernels)
   most = std::max(most, k.used);
   k.used = region;
   const size_t pool_ws = vig_rmsnorm_pool_workspace((int)B, (int)L, (int)C);
@@ -186,13 +186,19 @@ Tensor run(const Plan& p, const Tensor& images) {
   k.space = at::empty({most}, images.options());
 
   // ---- stem: convolution, norm + SiLU, convolution, norm + position table (each convolution's bias rides in the norm behind) ----
-  check_rc(vig_patch_conv_fwd(images.data_ptr(), st.w1.data_ptr(), k.at(c1), (int)B, (int)cin, (int)S, (int)W, st.KH, st.KW, 8, 1,
-                              (int)half, VIG_BF16, k.stream),
-           "vig_patch_conv_fwd");
-  check_rc(vig_layernorm_fwd(k.at(c1), f32(st.ln1w), f32(st.ln1b), k.at(c1n), n1, (int)half, (float)st.eps1, 1, f32(st.b1), nullptr, 0,
-                             VIG_BF16, k.stream),
-           "vig_layernorm_fwd");
-  check_rc(vig_conv3x3s2_fwd(k.at(c1n), st.w2.data_ptr(), k.at(y), (int)B, (int)oh1, (int)ow1, (int)half, (int)C, k.stream),
+  int64_t stem = c1;
+  int rc = vig_patch_conv_norm_fwd(images.data_ptr(), st.w1.data_ptr(), f32(st.ln1w), f32(st.ln1b), f32(st.b1), k.at(c1), (int)B, (int)cin, (int)S, (int)W,
+                                   st.KH, st.KW, 8, 1, (int)half, (float)st.eps1, 1, k.stream);
+  if (rc == VIG_ENOTSUP) {
+    check_rc(vig_patch_conv_fwd(images.data_ptr(), st.w1.data_ptr(), k.at(c1), (int)B, (int)cin, (int)S, (int)W, st.KH, st.KW, 8, 1,
+                                (int)half, VIG_BF16, k.stream),
+             "vig_patch_conv_fwd");
+    stem = c1n;
+    rc = vig_layernorm_fwd(k.at(c1), f32(st.ln1w), f32(st.ln1b), k.at(c1n), n1, (int)half, (float)st.eps1, 1, f32(st.b1), nullptr, 0, VIG_BF16,
+                           k.stream);
+  }
+  check_rc(rc, "the stem's first norm");
+  check_rc(vig_conv3x3s2_fwd(k.at(stem), st.w2.data_ptr(), k.at(y), (int)B, (int)oh1, (int)ow1, (int)half, (int)C, k.stream),
            "vig_conv3x3s2_fwd");
   check_rc(vig_layernorm_fwd(k.at(y), f32(st.ln2w), f32(st.ln2b), k.at(branch0), T, (int)C, (float)st.eps2, 0, f32(st.b2),
                              st.pos.data_ptr(), (int)L, VIG_BF16, k.stream),

@@ -24,15 +24,53 @@ constexpr int kPcStride = 8;       // convolution stride = elements per pixel st
 constexpr int kPcRowElems = 272;   // staged row: 32 chunks of 8 elements written per step, 16 more that stay zero
 constexpr int kPcKW = 16;          // kernel columns per contraction step (weights beyond the real width are zero)
 
-template <int KS, int NW>  // KS = Cin * KH contraction steps, NW = Cout / 32 waves
+// The layer norm behind it (NORM), as layernorm_kernel gives it for the stored rows, bit for bit: + pre_bias (rounded), norm, SiLU.
+struct PcNorm {
+  const float *weight, *bias, *pre_bias;  // [Cout]; pre_bias may be null
+  float eps;
+  int silu;
+};
+// the sum that layernorm_kernel's lanes, one to an octet, come to by exchange
+template <int N>
+__device__ __forceinline__ float octet_tree(const float* row) {
+  constexpr int G = 32;
+  static_assert(N <= G, "one octet to a lane of the kernel behind");
+  float a[G];
+#pragma unroll
+  for (int i = 0; i < N; i += 4) {
+    const f32x4_t v = *reinterpret_cast<const f32x4_t*>(row + i);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) a[i + j] = v[j];
+  }
+#pragma unroll
+  for (int i = N; i < G; ++i) a[i] = 0.f;
+#pragma unroll
+  for (int off = G / 2; off > 0; off >>= 1)
+#pragma unroll
+    for (int i = 0; i < off; ++i) a[i] += a[i + off];
+  return a[0];
+}
+
+// NORM: the workgroup has whole rows of channels, so their norm needs two exchanges of octet sums through LDS (a barrier each, one of
+// which takes the place of the one in front of the next staging) instead of a pass over memory.  us, two kernels / this: 96 channels, one image of
+// 224 px 8.5 / 6.7, 8 9.6 / 6.9, 256 74 / 54, 8 of 1024 px 50 / 35; 192, 1 9.4 / 7.9, 32 28 / 22, 64 37 / 32, 256 99.6 / 97.2 (one workgroup to a CU: its 191
+// registers brought down to 168 for a second one spill 13 to 18, 124).  At 384 channels the 48 octets spill (60 images 55 / 73): two kernels.
+template <int KS, int NW, bool NORM>  // KS = Cin * KH contraction steps, NW = Cout / 32 waves
 __global__ __launch_bounds__(NW > 8 ? 64 * NW : 512) void patch_conv_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ wp,
                                                          uint16_t* __restrict__ y, int Cin, int H, int W, int KH, int OH,
-                                                         int OW, int Cout, int pieces, int nitems) {
+                                                         int OW, int Cout, int pieces, int nitems, PcNorm norm) {
+  constexpr int kPitch = 4 * NW + 4;  // floats between two pixels' octet sums
   extern __shared__ __align__(16) char smem[];
   uint16_t* slab = reinterpret_cast<uint16_t*>(smem);  // [KS][kPcRowElems]
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   constexpr int nwaves = NW;
   const int r = lane & 31, h = lane >> 5;
+  float* const stats = reinterpret_cast<float*>(smem + KS * kPcRowElems * 2);  // [sums, squares][32 pixels][octets]
+  float* const params = stats + 2 * 32 * kPitch;                              // weight, bias, pre_bias [32 NW]
+  if constexpr (NORM) {
+    for (int i = threadIdx.x; i < 32 * NW; i += blockDim.x)
+      params[i] = norm.weight[i], params[32 * NW + i] = norm.bias[i], params[64 * NW + i] = norm.pre_bias ? norm.pre_bias[i] : 0.f;
+  }
   // the columns no step writes (and, until the first step, everything) read as zero
   for (int i = threadIdx.x; i < KS * kPcRowElems / 8; i += blockDim.x)
     reinterpret_cast<u32x4_t*>(slab)[i] = u32x4_t{0u, 0u, 0u, 0u};
@@ -97,10 +135,52 @@ __global__ __launch_bounds__(NW > 8 ? 64 * NW : 512) void patch_conv_kernel(cons
                                                     __builtin_bit_cast(bf16x8_t, px), acc, 0, 0, 0);
     }
     u32x4_t lo, hi;
+    const auto pack = [&](const auto& v) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      lo[j] = pack_bf16x2(acc[2 * j], acc[2 * j + 1]);
-      hi[j] = pack_bf16x2(acc[8 + 2 * j], acc[8 + 2 * j + 1]);
+      for (int j = 0; j < 4; ++j) {
+        lo[j] = pack_bf16x2(v[2 * j], v[2 * j + 1]);
+        hi[j] = pack_bf16x2(v[8 + 2 * j], v[8 + 2 * j + 1]);
+      }
+    };
+    pack(acc);
+    if constexpr (NORM) {
+      float s[16];
+      const auto unpack = [&] {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          s[2 * j] = bf16lo_to_f32(lo[j]), s[2 * j + 1] = bf16hi_to_f32(lo[j]);
+          s[8 + 2 * j] = bf16lo_to_f32(hi[j]), s[9 + 2 * j] = bf16hi_to_f32(hi[j]);
+        }
+      };
+      const float* const mine = params + 32 * wave + 16 * h;
+      unpack();
+      if (norm.pre_bias) {
+#pragma unroll
+        for (int j = 0; j < 16; ++j) s[j] += mine[64 * NW + j];
+        pack(s);
+        unpack();
+      }
+      float* const place = stats + r * kPitch + 4 * wave + 2 * h;
+      float sum[2] = {0.f, 0.f}, sq[2] = {0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < 16; ++j) sum[j >> 3] += s[j];
+      *reinterpret_cast<u32x2_t*>(place) = u32x2_t{__float_as_uint(sum[0]), __float_as_uint(sum[1])};
+      __syncthreads();  // (and nobody reads the slab any more)
+      const float mean = octet_tree<4 * NW>(stats + r * kPitch) / (float)(32 * NW);
+#pragma unroll
+      for (int j = 0; j < 16; ++j) s[j] -= mean, sq[j >> 3] = __builtin_fmaf(s[j], s[j], sq[j >> 3]);
+      *reinterpret_cast<u32x2_t*>(place + 32 * kPitch) = u32x2_t{__float_as_uint(sq[0]), __float_as_uint(sq[1])};
+      __syncthreads();
+      const float rstd = 1.0f / sqrtf(octet_tree<4 * NW>(stats + (32 + r) * kPitch) / (float)(32 * NW) + norm.eps);
+#pragma unroll
+      for (int j = 0; j < 16; ++j) s[j] = __builtin_fmaf(s[j] * rstd, mine[j], mine[32 * NW + j]);
+      pack(s);
+      if (norm.silu) {
+        unpack();
+#pragma unroll
+        for (int j = 0; j < 16; ++j) s[j] = s[j] * sigmoidf_(s[j]);
+        pack(s);
+      }
     }
     const int row = item / pieces, ox = (item - row * pieces) * 32 + r;
     if (ox < OW) {
@@ -108,7 +188,7 @@ __global__ __launch_bounds__(NW > 8 ? 64 * NW : 512) void patch_conv_kernel(cons
       *reinterpret_cast<u32x4_t*>(dst) = lo;
       *reinterpret_cast<u32x4_t*>(dst + 8) = hi;
     }
-    __syncthreads();  // the next step's staging overwrites the slab
+    if (!NORM) __syncthreads();  // the next step's staging overwrites the slab
   }
 }
 
@@ -122,19 +202,20 @@ bool patch_conv_supported(int Cin, int H, int W, int KH, int KW, int stride, int
   return OW >= 1 && Cout % 32 == 0 && ((Cout >= 64 && Cout <= 256) || Cout == 384);
 }
 
-int launch_patch_conv(const void* x, const void* w_packed, void* y, int B, int Cin, int H, int W, int KH, int KW,
-                      int Cout, hipStream_t stream) {
+static int launch(const void* x, const void* w_packed, void* y, int B, int Cin, int H, int W, int KH, int KW, int Cout, const PcNorm* norm,
+                  hipStream_t stream) {
   if (!patch_conv_supported(Cin, H, W, KH, KW, kPcStride, 1, Cout)) return -95;
   const int OH = (H + 2 - KH) / kPcStride + 1, OW = (W + 2 - KW) / kPcStride + 1;
   const int pieces = (OW + 31) / 32;
   if (OH < 1 || (long long)B * OH * pieces > 0x7fffffffLL - 4096 || Cout / 32 < 2) return -95;
   const int nitems = B * OH * pieces;
   const int grid = nitems < 512 ? nitems : 512;  // two workgroups a CU; each walks pieces grid apart
-  const size_t lds = (size_t)27 * kPcRowElems * sizeof(uint16_t);
+  const size_t lds = (size_t)27 * kPcRowElems * sizeof(uint16_t) + (norm ? 4 * (2 * 32 * (Cout / 8 + 4) + 3 * Cout) : 0);
 #define VIG_PC_CASE(NW)                                                                                            \
   case NW:                                                                                                         \
-    hipLaunchKernelGGL((patch_conv_kernel<27, NW>), dim3(grid), dim3(64 * NW), lds, stream, (const uint16_t*)x, \
-                       (const uint16_t*)w_packed, (uint16_t*)y, Cin, H, W, KH, OH, OW, Cout, pieces, nitems);              \
+    hipLaunchKernelGGL((norm ? patch_conv_kernel<27, NW, (NW <= 8)> : patch_conv_kernel<27, NW, false>), dim3(grid), dim3(64 * NW), lds, stream, \
+                       (const uint16_t*)x, (const uint16_t*)w_packed, (uint16_t*)y, Cin, H, W, KH, OH, OW, Cout, pieces, nitems,          \
+                       norm ? *norm : PcNorm{});                                                                                        \
     break
   switch (Cout / 32) {
     VIG_PC_CASE(2);
@@ -150,6 +231,15 @@ int launch_patch_conv(const void* x, const void* w_packed, void* y, int B, int C
   }
 #undef VIG_PC_CASE
   return hipGetLastError() == hipSuccess ? 0 : -5;
+}
+int launch_patch_conv(const void* x, const void* w_packed, void* y, int B, int Cin, int H, int W, int KH, int KW, int Cout, hipStream_t stream) {
+  return launch(x, w_packed, y, B, Cin, H, W, KH, KW, Cout, nullptr, stream);
+}
+int launch_patch_conv_norm(const void* x, const void* w_packed, const float* weight, const float* bias, const float* pre_bias, void* y, int B,
+                           int Cin, int H, int W, int KH, int KW, int Cout, float eps, int silu, hipStream_t stream) {
+  if (Cout > 256) return -95;
+  const PcNorm norm{weight, bias, pre_bias, eps, silu};
+  return launch(x, w_packed, y, B, Cin, H, W, KH, KW, Cout, &norm, stream);
 }
 
 }  // namespace vig
