@@ -740,6 +740,38 @@ int vig_linear_bwd_weight_many(const void* const* dy, const long long* dy_row_st
                                const long long* x_row_stride, float* const* dweight, float* const* dbias, void* workspace,
                                size_t workspace_bytes, long long rows, const int* N, const int* K, int count, void* stream);
 
+/*
+ * Several backward kernels leave partial rows in their workspace that a sum over the rows finishes, a launch each.  The _later forms put
+ * that sum off (`later` NULL: they do not): they enter it in `later` (zero before the first one), the gradients concerned (dw_db, dw, dweight, dbias) are filled by
+ * vig_sum_jobs_run, one launch for all, on the same stream, and until then every workspace and every output has to stay.  Results bit
+ * for bit as without.  A full list is refused with VIG_EINVAL (a form enters up to one, one, one and 2 * count of them).
+ * vig_sum_jobs_run empties the list.
+ */
+#define VIG_SUM_JOBS 12
+typedef struct {
+  const float* part; /* [rows, cols] */
+  float* out;        /* [cols] */
+  long long cols;
+  int rows, fours;   /* fours: few rows, columns taken four at a time */
+} vig_sum_job;
+typedef struct {
+  vig_sum_job job[VIG_SUM_JOBS];
+  int count;
+} vig_sum_jobs;
+int vig_dwconv3x3_bwd_later(const void* x, const void* dy, const void* pre, const float* weight, void* dx, float* dw_db,
+                      void* workspace, size_t workspace_bytes, int B, int h, int w, int C, int io_dtype, vig_sum_jobs* later, void* stream);
+int vig_locality_blend_bwd_strided_later(const void* o, const void* local, const void* g_lin, const float* w_g, const float* w_l,
+                                   const void* dy, void* d_o, void* d_local, void* d_glin, float* dw, void* workspace,
+                                   size_t workspace_bytes, int B, int H, int L, int Dv, long long g_row_stride,
+                                   long long d_glin_row_stride, float eps, int silu_out, int io_dtype, vig_sum_jobs* later, void* stream);
+int vig_rmsnorm_mixed_bwd_later(const void* sum, const float* weight, const void* dy, const void* d_sum, void* ds, void* dx,
+                          float* dweight, void* workspace, size_t workspace_bytes, long long rows, int C, float eps,
+                          int sum_dtype, int y_dtype, vig_sum_jobs* later, void* stream);
+int vig_linear_bwd_weight_many_later(const void* const* dy, const long long* dy_row_stride, const void* const* x,
+                               const long long* x_row_stride, float* const* dweight, float* const* dbias, void* workspace,
+                               size_t workspace_bytes, long long rows, const int* N, const int* K, int count, vig_sum_jobs* later, void* stream);
+int vig_sum_jobs_run(vig_sum_jobs* jobs, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

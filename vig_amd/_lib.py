@@ -106,6 +106,12 @@ SIGNATURES = {
     "vig_rmsnorm_mixed_fwd": (_c_int, [_c_void_p] * 5 + [_c_longlong, _c_int, _c_float] + [_c_int] * 4 + [_c_void_p]),
     "vig_rmsnorm_mixed_bwd": (_c_int, [_c_void_p] * 8 + [_c_size_t, _c_longlong, _c_int, _c_float, _c_int, _c_int, _c_void_p]),
     "vig_swiglu_fwd": (_c_int, [_c_void_p, _c_void_p, ctypes.c_longlong, _c_int, _c_int, _c_void_p]),
+    "vig_dwconv3x3_bwd_later": (_c_int, [_c_void_p] * 7 + [_c_size_t] + [_c_int] * 5 + [_c_void_p] + [_c_void_p]),
+    "vig_locality_blend_bwd_strided_later": (_c_int, [_c_void_p] * 11 + [_c_size_t] + [_c_int] * 4 +
+                                       [_c_longlong, _c_longlong, _c_float, _c_int, _c_int, _c_void_p] + [_c_void_p]),
+    "vig_rmsnorm_mixed_bwd_later": (_c_int, [_c_void_p] * 8 + [_c_size_t, _c_longlong, _c_int, _c_float, _c_int, _c_int, _c_void_p] + [_c_void_p]),
+    "vig_linear_bwd_weight_many_later": (_c_int, [_c_void_p] * 7 + [_c_size_t, _c_longlong, _c_void_p, _c_void_p, _c_int, _c_void_p] + [_c_void_p]),
+    "vig_sum_jobs_run": (_c_int, [_c_void_p, _c_void_p]),
 }
 
 _lib = None

@@ -15,7 +15,7 @@ int launch_merge_heads(const void* dq, const void* dk, const void* dv, void* dqk
 size_t dwconv3x3_wgrad_workspace(int B, int C);
 size_t dwconv3x3_wgrad_least_workspace(int B, int C);
 int launch_dwconv3x3_bwd(const void* x, const void* dy, const void* pre, const float* wt, void* dx, float* dw_db,
-                         void* workspace, size_t workspace_bytes, int B, int h, int w, int C, int io_dtype, hipStream_t stream);
+                         void* workspace, size_t workspace_bytes, int B, int h, int w, int C, int io_dtype, vig_sum_jobs* later, hipStream_t stream);
 int launch_dirgate_lowrank_bwd(const void* low, long long ld, const void* w1, const void* w1t, const void* b1,
                                const void* d_out, void* dx, void* d_low, long long ldd, int B, int L, int H, int Dk,
                                float inv_norm, float clamp_min, int out_dtype, hipStream_t stream);
@@ -43,7 +43,7 @@ size_t locality_blend_bwd_least_workspace(int B, int L, int Dv);
 int launch_locality_blend_bwd(const void* o, const void* loc, const void* glin, const float* wg, const float* wl,
                               const void* dy, void* d_o, void* d_loc, void* d_glin, float* dw, void* workspace, long long workspace_rows, int B,
                               int H, int L, int Dv, long long ldg, long long ldd, float eps, int silu_out, int io_dtype,
-                              hipStream_t stream);
+                              vig_sum_jobs* later, hipStream_t stream);
 bool rmsnorm_types_ok(int x_dtype, int sum_dtype, int y_dtype);
 int launch_rmsnorm(const void* x, const void* residual, const float* weight, void* y, void* residual_out, int rows,
                    int C, float eps, int round_sum, int x_dtype, int sum_dtype, int y_dtype, hipStream_t stream);
@@ -57,7 +57,7 @@ int launch_swiglu_bwd(const void* in, const void* dy, void* din, long long rows,
                       hipStream_t stream);
 size_t rmsnorm_bwd_workspace(long long rows, int C);
 int launch_rmsnorm_bwd(const void* s, const float* weight, const void* dy, const void* d_sum, void* ds, void* dx, float* dweight,
-                       void* workspace, long long rows, int C, float eps, int sum_dtype, int y_dtype, hipStream_t stream);
+                       void* workspace, long long rows, int C, float eps, int sum_dtype, int y_dtype, vig_sum_jobs* later, hipStream_t stream);
 bool blend_linear_supported(int H, int Dv, int C);
 int launch_blend_linear(const void* o, const void* loc, const void* glin, const float* w_g, const float* w_l,
                         const void* W, void* out, void* kept, int B, int H, int L, int Dv, int C, long long ldg, float eps,
@@ -92,6 +92,8 @@ static bool strided_rows_ok(const void* base, long long ld_elems, int dtype) {
   const long long elem = dtype == VIG_BF16 ? 2 : 4;
   return (reinterpret_cast<uintptr_t>(base) % 16) == 0 && (ld_elems * elem) % 16 == 0;
 }
+// whether a list of sums put off (none: they run at once) takes n more
+static bool room_for(const vig_sum_jobs* later, int n) { return !later || (later->count >= 0 && later->count <= VIG_SUM_JOBS - n); }
 // every tensor is moved 16 bytes per access: a pointer off that boundary is refused (null, for an optional tensor, passes)
 template <typename... P>
 static bool aligned16(P... p) {
@@ -622,14 +624,19 @@ size_t vig_dwconv3x3_bwd_weight_workspace(int B, int C) {
   return vig::dwconv3x3_wgrad_workspace(B, C);
 }
 
-int vig_dwconv3x3_bwd(const void* x, const void* dy, const void* pre, const float* weight, void* dx, float* dw_db,
-                      void* workspace, size_t workspace_bytes, int B, int h, int w, int C, int io_dtype, void* stream) {
+int vig_dwconv3x3_bwd_later(const void* x, const void* dy, const void* pre, const float* weight, void* dx, float* dw_db,
+                      void* workspace, size_t workspace_bytes, int B, int h, int w, int C, int io_dtype, vig_sum_jobs* later, void* stream) {
   if (!x || !dy || (!dx && !dw_db) || (dx && !weight) || B <= 0 || h <= 0 || w <= 0 || C <= 0 || dx == dy || (dx && dx == x))
     return VIG_EINVAL;
   if (!aligned16(x, dy, pre, dx, dw_db, workspace)) return VIG_EINVAL;
   if (!dtype_ok(io_dtype) || (C % 8) != 0) return VIG_ENOTSUP;
   if (dw_db && (!workspace || workspace_bytes < vig::dwconv3x3_wgrad_least_workspace(B, C))) return VIG_ENOSPC;
-  return vig::launch_dwconv3x3_bwd(x, dy, pre, weight, dx, dw_db, workspace, workspace_bytes, B, h, w, C, io_dtype, (hipStream_t)stream);
+  if (!room_for(later, dw_db ? 1 : 0)) return VIG_EINVAL;
+  return vig::launch_dwconv3x3_bwd(x, dy, pre, weight, dx, dw_db, workspace, workspace_bytes, B, h, w, C, io_dtype, later, (hipStream_t)stream);
+}
+int vig_dwconv3x3_bwd(const void* x, const void* dy, const void* pre, const float* weight, void* dx, float* dw_db,
+                      void* workspace, size_t workspace_bytes, int B, int h, int w, int C, int io_dtype, void* stream) {
+  return vig_dwconv3x3_bwd_later(x, dy, pre, weight, dx, dw_db, workspace, workspace_bytes, B, h, w, C, io_dtype, nullptr, stream);
 }
 
 int vig_dwconv3x3_bwd_weight(const void* x, const void* dy, float* dw_db, void* workspace, size_t workspace_bytes,
@@ -663,10 +670,10 @@ size_t vig_locality_blend_bwd_workspace(int B, int L, int Dv) {
   return vig::locality_blend_bwd_workspace(B, L, Dv);
 }
 
-int vig_locality_blend_bwd_strided(const void* o, const void* local, const void* g_lin, const float* w_g, const float* w_l,
+int vig_locality_blend_bwd_strided_later(const void* o, const void* local, const void* g_lin, const float* w_g, const float* w_l,
                                    const void* dy, void* d_o, void* d_local, void* d_glin, float* dw, void* workspace,
                                    size_t workspace_bytes, int B, int H, int L, int Dv, long long g_row_stride,
-                                   long long d_glin_row_stride, float eps, int silu_out, int io_dtype, void* stream) {
+                                   long long d_glin_row_stride, float eps, int silu_out, int io_dtype, vig_sum_jobs* later, void* stream) {
   if (!o || !local || !g_lin || !w_g || !w_l || !dy || !d_o || !d_local || !d_glin || !dw || B <= 0 || H <= 0 ||
       L <= 0)
     return VIG_EINVAL;
@@ -678,8 +685,16 @@ int vig_locality_blend_bwd_strided(const void* o, const void* local, const void*
     return VIG_EINVAL;
   if (!workspace || workspace_bytes < vig::locality_blend_bwd_least_workspace(B, L, Dv)) return VIG_ENOSPC;
   const long long rows = (long long)(std::min(workspace_bytes, vig::locality_blend_bwd_workspace(B, L, Dv)) / (2 * Dv * sizeof(float)));
+  if (!room_for(later, 1)) return VIG_EINVAL;
   return vig::launch_locality_blend_bwd(o, local, g_lin, w_g, w_l, dy, d_o, d_local, d_glin, dw, workspace, rows, B, H, L, Dv,
-                                        ldg, ldd, eps, silu_out, io_dtype, (hipStream_t)stream);
+                                        ldg, ldd, eps, silu_out, io_dtype, later, (hipStream_t)stream);
+}
+int vig_locality_blend_bwd_strided(const void* o, const void* local, const void* g_lin, const float* w_g, const float* w_l,
+                                   const void* dy, void* d_o, void* d_local, void* d_glin, float* dw, void* workspace,
+                                   size_t workspace_bytes, int B, int H, int L, int Dv, long long g_row_stride,
+                                   long long d_glin_row_stride, float eps, int silu_out, int io_dtype, void* stream) {
+  return vig_locality_blend_bwd_strided_later(o, local, g_lin, w_g, w_l, dy, d_o, d_local, d_glin, dw, workspace, workspace_bytes, B, H, L,
+                                              Dv, g_row_stride, d_glin_row_stride, eps, silu_out, io_dtype, nullptr, stream);
 }
 
 int vig_locality_blend_bwd(const void* o, const void* local, const void* g_lin, const float* w_g, const float* w_l,
@@ -849,17 +864,23 @@ size_t vig_rmsnorm_bwd_workspace(long long rows, int C) {
   return vig::rmsnorm_bwd_workspace(rows, C);
 }
 
-int vig_rmsnorm_mixed_bwd(const void* sum, const float* weight, const void* dy, const void* d_sum, void* ds, void* dx,
+int vig_rmsnorm_mixed_bwd_later(const void* sum, const float* weight, const void* dy, const void* d_sum, void* ds, void* dx,
                           float* dweight, void* workspace, size_t workspace_bytes, long long rows, int C, float eps,
-                          int sum_dtype, int y_dtype, void* stream) {
+                          int sum_dtype, int y_dtype, vig_sum_jobs* later, void* stream) {
   if (!sum || !weight || !dy || !ds || rows <= 0 || C <= 0 || rows > 0x7fffffffLL) return VIG_EINVAL;
   if (!aligned16(sum, weight, dy, d_sum, ds, dx, dweight, workspace)) return VIG_EINVAL;
   if (!dtype_ok(sum_dtype) || !dtype_ok(y_dtype) || (C % 8) != 0 || C > 1024 ||
       !vig::rmsnorm_types_ok(sum_dtype, sum_dtype, y_dtype))
     return VIG_ENOTSUP;
   if (dweight && (!workspace || workspace_bytes < vig::rmsnorm_bwd_workspace(rows, C))) return VIG_ENOSPC;
+  if (!room_for(later, dweight ? 1 : 0)) return VIG_EINVAL;
   return vig::launch_rmsnorm_bwd(sum, weight, dy, d_sum, ds, dx, dweight, workspace, rows, C, eps, sum_dtype, y_dtype,
-                                 (hipStream_t)stream);
+                                 later, (hipStream_t)stream);
+}
+int vig_rmsnorm_mixed_bwd(const void* sum, const float* weight, const void* dy, const void* d_sum, void* ds, void* dx,
+                          float* dweight, void* workspace, size_t workspace_bytes, long long rows, int C, float eps,
+                          int sum_dtype, int y_dtype, void* stream) {
+  return vig_rmsnorm_mixed_bwd_later(sum, weight, dy, d_sum, ds, dx, dweight, workspace, workspace_bytes, rows, C, eps, sum_dtype, y_dtype, nullptr, stream);
 }
 
 int vig_rmsnorm_bwd(const void* sum, const float* weight, const void* dy, const void* d_sum, void* ds, float* dweight,
@@ -974,9 +995,9 @@ int vig_linear_bwd_weight(const void* dy, long long dy_row_stride, const void* x
                                     stream);
 }
 
-int vig_linear_bwd_weight_many(const void* const* dy, const long long* dy_row_stride, const void* const* x, const long long* x_row_stride,
+int vig_linear_bwd_weight_many_later(const void* const* dy, const long long* dy_row_stride, const void* const* x, const long long* x_row_stride,
                                float* const* dweight, float* const* dbias, void* workspace, size_t workspace_bytes, long long rows,
-                               const int* N, const int* K, int count, void* stream) {
+                               const int* N, const int* K, int count, vig_sum_jobs* later, void* stream) {
   if (!dy || !dy_row_stride || !x || !x_row_stride || !dweight || !N || !K || count < 1 || count > vig::kWgradLayers) return VIG_EINVAL;
   vig::LinearWgrad l[vig::kWgradLayers] = {};
   for (int i = 0; i < count; ++i)
@@ -992,7 +1013,20 @@ int vig_linear_bwd_weight_many(const void* const* dy, const long long* dy_row_st
     l[i] = {dy[i], x[i], dy_row_stride[i], x_row_stride[i], dweight[i], db, N[i], K[i]};
   }
   if (!workspace || workspace_bytes < vig::linear_wgrad_workspace(rows, l, count)) return VIG_ENOSPC;
-  return vig::launch_linear_wgrad(l, count, rows, workspace, (hipStream_t)stream);
+  if (!room_for(later, 2 * count)) return VIG_EINVAL;
+  return vig::launch_linear_wgrad(l, count, rows, workspace, later, (hipStream_t)stream);
+}
+int vig_linear_bwd_weight_many(const void* const* dy, const long long* dy_row_stride, const void* const* x, const long long* x_row_stride,
+                               float* const* dweight, float* const* dbias, void* workspace, size_t workspace_bytes, long long rows,
+                               const int* N, const int* K, int count, void* stream) {
+  return vig_linear_bwd_weight_many_later(dy, dy_row_stride, x, x_row_stride, dweight, dbias, workspace, workspace_bytes, rows, N, K, count, nullptr, stream);
+}
+
+int vig_sum_jobs_run(vig_sum_jobs* jobs, void* stream) {
+  if (!jobs || jobs->count < 0 || jobs->count > VIG_SUM_JOBS) return VIG_EINVAL;
+  const int rc = vig::launch_sum_jobs(*jobs, (hipStream_t)stream);
+  if (rc == VIG_OK) jobs->count = 0;
+  return rc;
 }
 
 }  // extern "C"

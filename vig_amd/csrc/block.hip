@@ -590,34 +590,10 @@ __global__ __launch_bounds__(64 * kRmsBwdWaves) void rmsnorm_bwd_kernel(const TS
   }
 }
 
-// out[c] = sum over the n rows of partials [n, C].  The rows were written by every XCD, so a load is a trip to memory: a workgroup takes
-// 16 columns, a thread every 64th row of one, eight loads under way at a time.  Measured with the
-// kernel in front of it, 512 to 1024 rows of 128: 3.7 us less than with 64 columns a workgroup and four loads.
 __global__ __launch_bounds__(1024) void column_sum_kernel(const float* __restrict__ partials, float* __restrict__ out,
                                                           int n, int C) {
   __shared__ float red[64][17];
-  const int col = threadIdx.x & 15, slice = threadIdx.x >> 4;
-  const int c = blockIdx.x * 16 + col;
-  float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  if (c < C) {
-    for (int i = slice; i < n; i += 512) {
-      float x[8];
-#pragma unroll
-      for (int k = 0; k < 8; ++k) x[k] = i + 64 * k < n ? partials[(size_t)(i + 64 * k) * C + c] : 0.f;
-#pragma unroll
-      for (int k = 0; k < 8; ++k) acc[k] += x[k];
-    }
-  }
-  red[slice][col] = ((acc[0] + acc[1]) + (acc[2] + acc[3])) + ((acc[4] + acc[5]) + (acc[6] + acc[7]));
-  __syncthreads();
-  if (threadIdx.x < 64) {  // four threads a column, 16 slices each
-    float t = 0.f;
-#pragma unroll
-    for (int k = 0; k < 16; ++k) t += red[4 * k + (threadIdx.x >> 4)][col];
-    t += __shfl_xor(t, 16);
-    t += __shfl_xor(t, 32);
-    if (threadIdx.x < 16 && c < C) out[c] = t;
-  }
+  sum_columns(partials, out, n, C, blockIdx.x, red);
 }
 
 int launch_column_sum(const float* partials, float* out, int n, int C, hipStream_t stream) {
@@ -634,7 +610,7 @@ size_t rmsnorm_bwd_workspace(long long rows, int C) { return (size_t)rmsnorm_bwd
 
 template <typename TS, typename TY, typename TX>
 static int launch_rmsnorm_bwd_t(const void* s, const float* weight, const void* dy, const void* d_sum, void* ds, void* dx,
-                                float* dweight, float* partials, int rows, int C, float eps, hipStream_t stream) {
+                                float* dweight, float* partials, int rows, int C, float eps, vig_sum_jobs* later, hipStream_t stream) {
   const int grid = rmsnorm_bwd_grid(rows);
   const size_t lds = dweight ? (size_t)kRmsBwdWaves * C * sizeof(float) : 0;
   float* part = dweight ? partials : nullptr;
@@ -646,20 +622,19 @@ static int launch_rmsnorm_bwd_t(const void* s, const float* weight, const void* 
   else VIG_RMSB_CASE(2);
 #undef VIG_RMSB_CASE
   if (hipGetLastError() != hipSuccess) return -5;
-  if (dweight) {
-    return launch_column_sum(partials, dweight, grid, C, stream);
-  }
-  return 0;
+  if (!dweight) return 0;
+  if (later) return put_off(*later, partials, dweight, grid, C, false) ? 0 : -22;
+  return launch_column_sum(partials, dweight, grid, C, stream);
 }
 
 int launch_rmsnorm_bwd(const void* s, const float* weight, const void* dy, const void* d_sum, void* ds, void* dx, float* dweight,
-                       void* workspace, long long rows, int C, float eps, int sum_dtype, int y_dtype, hipStream_t stream) {
+                       void* workspace, long long rows, int C, float eps, int sum_dtype, int y_dtype, vig_sum_jobs* later, hipStream_t stream) {
   if (C % 8 != 0 || C > 1024 || rows > 0x7fffffffLL - 8192) return -95;  // 16 rows of C floats in 64 KB of LDS
   if (!rmsnorm_types_ok(sum_dtype, sum_dtype, y_dtype)) return -95;
   auto fn = sum_dtype == 1 ? launch_rmsnorm_bwd_t<uint16_t, uint16_t, uint16_t>
             : y_dtype == 0 ? launch_rmsnorm_bwd_t<float, float, float>
                            : launch_rmsnorm_bwd_t<float, uint16_t, uint16_t>;
-  return fn(s, weight, dy, d_sum, ds, dx, dweight, (float*)workspace, (int)rows, C, eps, stream);
+  return fn(s, weight, dy, d_sum, ds, dx, dweight, (float*)workspace, (int)rows, C, eps, later, stream);
 }
 
 // ---------------------------------------------------------------------------

@@ -110,6 +110,34 @@ __device__ __forceinline__ float logsigmoidf_(float x) {
   return fminf(x, 0.f) - 0.6931471805599453f * __builtin_amdgcn_logf(1.f + exp_fast(-fabsf(x)));
 }
 
+// out[c] = sum over the n rows of partials [n, C].  The rows were written by every XCD, so a load is a trip to memory: a workgroup of 1024 takes
+// 16 columns, a thread every 64th row of one, eight loads under way at a time.  Measured with the
+// kernel in front of it, 512 to 1024 rows of 128: 3.7 us less than with 64 columns a workgroup and four loads.
+__device__ __forceinline__ void sum_columns(const float* partials, float* out, int n, long long C, int block, float (*red)[17]) {
+  const int col = threadIdx.x & 15, slice = threadIdx.x >> 4;
+  const long long c = (long long)block * 16 + col;
+  float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  if (c < C) {
+    for (int i = slice; i < n; i += 512) {
+      float x[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) x[k] = i + 64 * k < n ? partials[(size_t)(i + 64 * k) * C + c] : 0.f;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) acc[k] += x[k];
+    }
+  }
+  red[slice][col] = ((acc[0] + acc[1]) + (acc[2] + acc[3])) + ((acc[4] + acc[5]) + (acc[6] + acc[7]));
+  __syncthreads();
+  if (threadIdx.x < 64) {  // four threads a column, 16 slices each
+    float t = 0.f;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) t += red[4 * k + (threadIdx.x >> 4)][col];
+    t += __shfl_xor(t, 16);
+    t += __shfl_xor(t, 32);
+    if (threadIdx.x < 16 && c < C) out[c] = t;
+  }
+}
+
 // 16 bytes per lane from memory straight into LDS: lane i lands 16 i bytes behind lds_base (wave-uniform byte offset in the
 // workgroup's LDS).  In assembly, because the compiler answers the builtin of this load with waits of its own in front of
 // every later LDS read it cannot tell apart from the destination, down to vmcnt(0), which also drains the stores and the

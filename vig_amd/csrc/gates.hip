@@ -1188,7 +1188,7 @@ size_t dwconv3x3_wgrad_least_workspace(int B, int C) { return (size_t)B * kWgrad
 
 template <typename T, bool SILU>
 static int launch_dwconv3x3_bwd_t(const void* x, const void* dy, const void* pre, const float* wt, void* dx, float* dw_db,
-                                  float* partials, int most_split, int B, int h, int w, int C, hipStream_t stream) {
+                                  float* partials, int most_split, int B, int h, int w, int C, vig_sum_jobs* later, hipStream_t stream) {
   constexpr int kCells = 48 * 1024 / (kStencilGroup * (int)sizeof(T));  // three workgroups' tiles fit a CU's LDS
   const int band_cols = w < kCells / 6 - 2 ? w : kCells / 6 - 2;        // four rows at least
   const int rows = kCells / (band_cols + 2) - 2;
@@ -1209,11 +1209,13 @@ static int launch_dwconv3x3_bwd_t(const void* x, const void* dy, const void* pre
                      (const T*)x, (const T*)dy, (const T*)pre, wt, (T*)dx, dw_db ? partials : nullptr, h, w, C, groups,
                      band_rows, band_cols, col_bands, nbands);
   if (hipGetLastError() != hipSuccess) return -5;
+  if (dw_db && later) return put_off(*later, partials, dw_db, split * B, C * 10, false) ? 0 : -22;
   return dw_db ? launch_column_sum(partials, dw_db, split * B, C * 10, stream) : 0;
 }
 
 int launch_dwconv3x3_bwd(const void* x, const void* dy, const void* pre, const float* wt, void* dx, float* dw_db,
-                         void* workspace, size_t workspace_bytes, int B, int h, int w, int C, int io_dtype, hipStream_t stream) {
+                         void* workspace, size_t workspace_bytes, int B, int h, int w, int C, int io_dtype, vig_sum_jobs* later,
+                         hipStream_t stream) {
   if (B > 65535 || C % 8 != 0 || (long long)h * w > 0x7fffffffLL - 64 || (long long)C * 10 > 0x7fffffffLL ||
       (long long)B * ((C + 63) / 64) > 0x7fffffffLL)
     return -22;
@@ -1221,7 +1223,7 @@ int launch_dwconv3x3_bwd(const void* x, const void* dy, const void* pre, const f
                           : (pre ? launch_dwconv3x3_bwd_t<uint16_t, true> : launch_dwconv3x3_bwd_t<uint16_t, false>);
   // (without weight gradients nobody's partial sums need room)
   const int most = dw_db ? (int)std::min<size_t>(wgrad_split(B, C), workspace_bytes / ((size_t)B * C * 10 * sizeof(float))) : wgrad_split(B, C);
-  return fn(x, dy, pre, wt, dx, dw_db, static_cast<float*>(workspace), most, B, h, w, C, stream);
+  return fn(x, dy, pre, wt, dx, dw_db, static_cast<float*>(workspace), most, B, h, w, C, later, stream);
 }
 
 // ---------------------------------------------------------------------------
@@ -1351,7 +1353,7 @@ size_t locality_blend_bwd_least_workspace(int B, int L, int Dv) { return (size_t
 int launch_locality_blend_bwd(const void* o, const void* loc, const void* glin, const float* wg, const float* wl,
                               const void* dy, void* d_o, void* d_loc, void* d_glin, float* dw, void* workspace, long long workspace_rows, int B,
                               int H, int L, int Dv, long long ldg, long long ldd, float eps, int silu_out, int io_dtype,
-                              hipStream_t stream) {
+                              vig_sum_jobs* later, hipStream_t stream) {
   if (B > 65535 || !octet_rows_ok(B, L)) return -22;
   const int nv = H * (Dv / 8);
   const long long total = (long long)B * L, room = std::min<long long>(kBlendBwdBlocks, workspace_rows);
@@ -1369,6 +1371,7 @@ int launch_locality_blend_bwd(const void* o, const void* loc, const void* glin, 
                        (const uint16_t*)loc, (const uint16_t*)glin, wg, wl, (const uint16_t*)dy, (uint16_t*)d_o,
                        (uint16_t*)d_loc, (uint16_t*)d_glin, partials, B, H, L, Dv, ldg, ldd, eps, silu_out, tokens);
   if (hipGetLastError() != hipSuccess) return -5;
+  if (later) return put_off(*later, partials, dw, (int)grid.x, 2 * Dv, false) ? 0 : -22;
   return launch_column_sum(partials, dw, (int)grid.x, 2 * Dv, stream);
 }
 

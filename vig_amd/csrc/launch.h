@@ -3,6 +3,8 @@
 #include <hip/hip_runtime.h>
 #include <stddef.h>
 
+#include "../../include/vig_gla.h"
+
 namespace vig {
 
 struct GlaArgs {
@@ -96,6 +98,14 @@ int launch_gla_states(const GlaArgs& a, int seg_len, int nseg, float* slots, con
 // chains the slots of a state pass in place (gla_segment_scan_kernel, no state in or out), and those of another if there is one
 int launch_gla_segment_scan(float* slots, float* more, int nseq, int nseg, int ndir, int ng, hipStream_t stream);
 
+// Sums that kernels put off (wgrad.hip): false where the list is full.
+inline bool put_off(vig_sum_jobs& jobs, const float* part, float* out, int rows, long long cols, bool fours) {
+  if (jobs.count < 0 || jobs.count >= VIG_SUM_JOBS) return false;
+  jobs.job[jobs.count++] = {part, out, cols, rows, fours};
+  return true;
+}
+int launch_sum_jobs(const vig_sum_jobs& jobs, hipStream_t stream);
+
 // Weight and bias gradients of up to kWgradLayers linear layers over the same T bf16 rows (wgrad.hip).
 constexpr int kWgradLayers = 4;
 struct LinearWgrad {
@@ -105,7 +115,7 @@ struct LinearWgrad {
   int N, K;
 };
 size_t linear_wgrad_workspace(long long T, const LinearWgrad* layers, int count);
-int launch_linear_wgrad(const LinearWgrad* layers, int count, long long T, void* workspace, hipStream_t stream);
+int launch_linear_wgrad(const LinearWgrad* layers, int count, long long T, void* workspace, vig_sum_jobs* later, hipStream_t stream);
 
 // Most tensors one launch_cast_many takes.
 constexpr int kMaxCastJobs = 16;

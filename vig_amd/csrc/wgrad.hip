@@ -223,45 +223,48 @@ __global__ __launch_bounds__(256, 2) void linear_wgrad_kernel(WgradArgs a) {
   }
 }
 
-struct WgradSum {
-  const float *part, *bpart;
-  float *dw, *db;
-  long long n4;     // fours of dW
-  int N, first;     // the layer's first block
-};
-struct WgradSums {
-  WgradSum layer[kWgradLayers];
-  int layers, splits;
+// A launch for the sums that several kernels have left partial rows of.  Behind each of them a launch of its own took 4.7 us, most of it the launch: 72 of a
+// training pass of twelve blocks are 24, or 48 with large partial tiles, which are added up at once (train_block.cpp).  Sums in the order they had there.
+struct SumLaunch {
+  vig_sum_jobs jobs;
+  int first[VIG_SUM_JOBS];  // a job's first block
 };
 
-// sums of the splits' partial results: 32 columns of four values by eight groups of splits per block, the groups' sums
-// added in LDS in order; a layer's last blocks do the bias (one value a column)
-__global__ __launch_bounds__(256) void wgrad_sum_kernel(WgradSums a) {
-  __shared__ f32x4_t sums[8][32];
-  int which = 0;
-  for (int i = 1; i < a.layers; ++i) which = (int)blockIdx.x >= a.layer[i].first ? i : which;
-  const WgradSum& y = a.layer[which];
-  const long long n4 = y.n4;
-  const int splits = a.splits, N = y.N;
-  const int col = threadIdx.x & 31, grp = threadIdx.x >> 5;
-  const long long i = (long long)((int)blockIdx.x - y.first) * 32 + col;
-  const bool bias = i >= n4;
-  const long long j = i - n4;
+// fours: a block has as many columns of four values as an eighth of its threads and eight groups of rows, whose sums are added in LDS in order
+template <int THREADS>
+__device__ __forceinline__ void sum_fours(const vig_sum_job& y, int block, f32x4_t (*sums)[THREADS / 8]) {
+  const int col = threadIdx.x % (THREADS / 8), grp = threadIdx.x / (THREADS / 8);
+  const long long n4 = y.cols / 4, i = (long long)block * (THREADS / 8) + col;
   f32x4_t s = {0.f, 0.f, 0.f, 0.f};
-  if (!bias) {
+  if (i < n4) {
     const f32x4_t* p = reinterpret_cast<const f32x4_t*>(y.part) + i;
 #pragma unroll 4
-    for (int k = grp; k < splits; k += 8) s += p[(long long)k * n4];
-  } else if (y.db && j < N) {
-    for (int k = grp; k < splits; k += 8) s[0] += y.bpart[(long long)k * N + j];
+    for (int k = grp; k < y.rows; k += 8) s += p[(long long)k * n4];
   }
   sums[grp][col] = s;
   __syncthreads();
-  if (grp != 0) return;
+  if (grp != 0 || i >= n4) return;
 #pragma unroll
   for (int k = 1; k < 8; ++k) s += sums[k][col];
-  if (!bias) reinterpret_cast<f32x4_t*>(y.dw)[i] = s;
-  else if (y.db && j < N) y.db[j] = s[0];
+  if ((reinterpret_cast<uintptr_t>(y.out) & 15) == 0) {
+    reinterpret_cast<f32x4_t*>(y.out)[i] = s;
+  } else {  // (a caller's bias gradient may start anywhere)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) y.out[4 * i + k] = s[k];
+  }
+}
+
+// 1024 threads where there are sums of few columns, which have all rows of a column under way (four slices of rows to each of 256 take 138 registers,
+// and the other form from eight waves a SIMD to three: a node's sums of ViG-S at 25 088 rows 19 us, with these 13 to 14); 256 where there are none.
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) void sum_jobs_kernel(SumLaunch a) {
+  __shared__ __align__(16) char room[THREADS * 16];
+  int which = 0;
+  for (int i = 1; i < a.jobs.count; ++i) which = (int)blockIdx.x >= a.first[i] ? i : which;
+  const vig_sum_job& y = a.jobs.job[which];
+  const int block = (int)blockIdx.x - a.first[which];
+  if (THREADS == 256 || y.fours) sum_fours<THREADS>(y, block, reinterpret_cast<f32x4_t(*)[THREADS / 8]>(room));
+  else if constexpr (THREADS == 1024) sum_columns(y.part, y.out, y.rows, y.cols, block, reinterpret_cast<float(*)[17]>(room));
 }
 
 long long wgrad_tiles(int N, int K) { return (long long)((N + kWgTile - 1) / kWgTile) * ((K + kWgTile - 1) / kWgTile); }
@@ -320,45 +323,64 @@ size_t linear_wgrad_workspace(long long T, const LinearWgrad* layers, int count)
   return wgrad_splits(T, layers, count) * floats * sizeof(float);
 }
 
-int launch_linear_wgrad(const LinearWgrad* layers, int count, long long T, void* workspace, hipStream_t stream) {
+int launch_sum_jobs(const vig_sum_jobs& jobs, hipStream_t stream) {
+  if (jobs.count < 1) return 0;
+  if (jobs.count > VIG_SUM_JOBS) return -22;
+  SumLaunch a{};
+  a.jobs = jobs;
+  long long blocks = 0;
+  bool only_fours = true;
+  for (int i = 0; i < jobs.count; ++i) only_fours = only_fours && jobs.job[i].fours;
+  const int four_columns = only_fours ? 32 : 128;
+  for (int i = 0; i < jobs.count; ++i) {
+    const vig_sum_job& y = jobs.job[i];
+    if (!y.part || !y.out || y.cols <= 0 || y.rows <= 0 || (y.fours && (y.cols % 4 || (reinterpret_cast<uintptr_t>(y.part) & 15)))) return -22;
+    a.first[i] = (int)blocks;
+    blocks += y.fours ? (y.cols / 4 + four_columns - 1) / four_columns : (y.cols + 15) / 16;
+    if (blocks > 0x7fffffffLL / 256) return -22;
+  }
+  hipLaunchKernelGGL((only_fours ? sum_jobs_kernel<256> : sum_jobs_kernel<1024>), dim3((unsigned)blocks), dim3(only_fours ? 256 : 1024), 0, stream, a);
+  return hipGetLastError() == hipSuccess ? 0 : -5;
+}
+
+// later: the sums over token ranges are left to it, where the layers go out together
+int launch_linear_wgrad(const LinearWgrad* layers, int count, long long T, void* workspace, vig_sum_jobs* later, hipStream_t stream) {
   static bool done[64] = {};
   constexpr int lds = kWgBuffers * 2 * kWgHalf;
   if (count < 1 || count > kWgradLayers) return -22;
   if (!wgrad_together(T, layers, count)) {
     int rc = 0;
-    for (int i = 0; i < count && rc == 0; ++i) rc = launch_linear_wgrad(layers + i, 1, T, workspace, stream);
+    for (int i = 0; i < count && rc == 0; ++i) rc = launch_linear_wgrad(layers + i, 1, T, workspace, nullptr, stream);  // (one workspace for all)
     return rc;
   }
   if (!allow_lds(reinterpret_cast<const void*>(linear_wgrad_kernel), lds, done)) return -5;
   WgradArgs a{};
-  WgradSums b{};
-  long long tiles = 0, blocks = 0;
+  vig_sum_jobs own{}, &sums = later ? *later : own;
+  long long tiles = 0;
   for (int i = 0; i < count; ++i) tiles += wgrad_tiles(layers[i].N, layers[i].K);
   if (tiles > 0x7fffffffLL / 256) return -22;
   const int want = wgrad_splits(T, layers, count);
-  a.T = (int)T, a.layers = b.layers = count, a.tiles = (int)tiles;
+  a.T = (int)T, a.layers = count, a.tiles = (int)tiles;
   a.per = (int)(((T + want - 1) / want + kWgStage - 1) / kWgStage * kWgStage);
-  a.splits = b.splits = (int)((T + a.per - 1) / a.per);
+  a.splits = (int)((T + a.per - 1) / a.per);
   const bool sum = a.splits > 1;
   float* ws = (float*)workspace;
   tiles = 0;
   for (int i = 0; i < count; ++i) {
     const LinearWgrad& l = layers[i];
     WgradLayer& y = a.layer[i];
-    WgradSum& z = b.layer[i];
     const size_t weights = (size_t)a.splits * l.N * l.K;
     y.dy = (const uint16_t*)l.dy, y.x = (const uint16_t*)l.x, y.ldy = l.ldy, y.ldx = l.ldx, y.N = l.N, y.K = l.K;
     y.part = sum ? ws : l.dw;
     y.bpart = l.db ? (sum ? ws + weights : l.db) : nullptr;
     y.tn = (l.N + kWgTile - 1) / kWgTile, y.first = (int)tiles;
-    z.part = y.part, z.bpart = y.bpart, z.dw = l.dw, z.db = l.db, z.n4 = (long long)l.N * l.K / 4, z.N = l.N, z.first = (int)blocks;
+    if (sum && !(put_off(sums, y.part, l.dw, a.splits, (long long)l.N * l.K, true) && (!l.db || put_off(sums, y.bpart, l.db, a.splits, l.N, true)))) return -22;
     ws += (weights + (l.db ? (size_t)a.splits * l.N : 0) + 3) / 4 * 4;
     tiles += wgrad_tiles(l.N, l.K);
-    blocks += (z.n4 + (l.db ? l.N : 0) + 31) / 32;
   }
   hipLaunchKernelGGL(linear_wgrad_kernel, dim3(8 * ((a.splits * a.tiles + 7) / 8)), dim3(256), lds, stream, a);
-  if (sum) hipLaunchKernelGGL(wgrad_sum_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, b);
-  return hipGetLastError() == hipSuccess ? 0 : -5;
+  if (hipGetLastError() != hipSuccess) return -5;
+  return later ? 0 : launch_sum_jobs(own, stream);
 }
 
 }  // namespace vig
