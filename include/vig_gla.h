@@ -741,6 +741,21 @@ int vig_linear_bwd_weight_many(const void* const* dy, const long long* dy_row_st
                                size_t workspace_bytes, long long rows, const int* N, const int* K, int count, void* stream);
 
 /*
+ * The layer norms of the patch embedding for training: y [rows, C] = layernorm(x + pre_bias) * weight + bias, through SiLU if silu, x [rows, C]
+ * and y bf16 or fp32 (fp32 x: fp32 y), all between them fp32; pre_bias [C] or NULL.  C % 8 == 0, C <= 1024.
+ * _bwd: dx [rows, C] in x's type (NULL: not wanted) and dparams [3, C]: the gradients of weight, bias and pre_bias; dy in y's type.
+ *
+ * Replaces: LayerNorm2d and nn.SiLU of V2PatchEmbed (classification/models/vig.py:619-624,651-656), the convolutions' bias adds, and what
+ * autograd derives for them.
+ */
+int vig_stem_norm_fwd(const void* x, const float* pre_bias, const float* weight, const float* bias, void* y, long long rows, int C, float eps,
+                      int silu, int x_dtype, int y_dtype, void* stream);
+size_t vig_stem_norm_bwd_workspace(long long rows, int C);
+int vig_stem_norm_bwd(const void* x, const float* pre_bias, const float* weight, const float* bias, const void* dy, void* dx, float* dparams,
+                      void* workspace, size_t workspace_bytes, long long rows, int C, float eps, int silu, int x_dtype, int y_dtype,
+                      void* stream);
+
+/*
  * Several backward kernels leave partial rows in their workspace that a sum over the rows finishes, a launch each.  The _later forms put
  * that sum off (`later` NULL: they do not): they enter it in `later` (zero before the first one), the gradients concerned (dw_db, dw, dweight, dbias) are filled by
  * vig_sum_jobs_run, one launch for all, on the same stream, and until then every workspace and every output has to stay.  Results bit

@@ -111,6 +111,9 @@ SIGNATURES = {
                                        [_c_longlong, _c_longlong, _c_float, _c_int, _c_int, _c_void_p] + [_c_void_p]),
     "vig_rmsnorm_mixed_bwd_later": (_c_int, [_c_void_p] * 8 + [_c_size_t, _c_longlong, _c_int, _c_float, _c_int, _c_int, _c_void_p] + [_c_void_p]),
     "vig_linear_bwd_weight_many_later": (_c_int, [_c_void_p] * 7 + [_c_size_t, _c_longlong, _c_void_p, _c_void_p, _c_int, _c_void_p] + [_c_void_p]),
+    "vig_stem_norm_fwd": (_c_int, [_c_void_p] * 5 + [_c_longlong, _c_int, _c_float, _c_int, _c_int, _c_int, _c_void_p]),
+    "vig_stem_norm_bwd_workspace": (_c_size_t, [_c_longlong, _c_int]),
+    "vig_stem_norm_bwd": (_c_int, [_c_void_p] * 8 + [_c_size_t, _c_longlong, _c_int, _c_float, _c_int, _c_int, _c_int, _c_void_p]),
     "vig_sum_jobs_run": (_c_int, [_c_void_p, _c_void_p]),
 }
 

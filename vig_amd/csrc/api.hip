@@ -67,6 +67,12 @@ int launch_linear_swiglu(const void* A, const void* W, void* out, void* kept, lo
 bool patch_conv_supported(int Cin, int H, int W, int KH, int KW, int stride, int padding, int Cout);
 int launch_patch_conv(const void* x, const void* w_packed, void* y, int B, int Cin, int H, int W, int KH, int KW,
                       int Cout, hipStream_t stream);
+bool stem_norm_supported(long long rows, int C, int x_dtype, int y_dtype);
+size_t stem_norm_bwd_workspace(long long rows, int C);
+int launch_stem_norm(const void* x, const float* pre, const float* w, const float* b, void* y, long long rows, int C, float eps, int silu,
+                     int x_dtype, int y_dtype, hipStream_t stream);
+int launch_stem_norm_bwd(const void* x, const float* pre, const float* w, const float* b, const void* dy, void* dx, float* dparams, void* workspace,
+                         long long rows, int C, float eps, int silu, int x_dtype, int y_dtype, hipStream_t stream);
 int launch_patch_conv_norm(const void* x, const void* w_packed, const float* weight, const float* bias, const float* pre_bias, void* y, int B,
                            int Cin, int H, int W, int KH, int KW, int Cout, float eps, int silu, hipStream_t stream);
 int launch_pad_channels(const void* src, void* dst, long long rows, int src_c, int dst_c, hipStream_t stream);
@@ -731,6 +737,26 @@ int vig_layernorm_fwd(const void* x, const float* weight, const float* bias, voi
   if (!dtype_ok(io_dtype) || (C % 8) != 0 || C > 4096) return VIG_ENOTSUP;
   return vig::launch_layernorm(x, weight, bias, y, rows, C, eps, silu, pre_bias, post_add, post_rows, io_dtype,
                                (hipStream_t)stream);
+}
+
+int vig_stem_norm_fwd(const void* x, const float* pre_bias, const float* weight, const float* bias, void* y, long long rows, int C, float eps,
+                      int silu, int x_dtype, int y_dtype, void* stream) {
+  if (!x || !weight || !bias || !y || rows <= 0 || C <= 0) return VIG_EINVAL;
+  if (!aligned16(x, pre_bias, weight, bias, y)) return VIG_EINVAL;
+  if (!dtype_ok(x_dtype) || !dtype_ok(y_dtype) || !vig::stem_norm_supported(rows, C, x_dtype, y_dtype)) return VIG_ENOTSUP;
+  return vig::launch_stem_norm(x, pre_bias, weight, bias, y, rows, C, eps, silu, x_dtype, y_dtype, (hipStream_t)stream);
+}
+
+size_t vig_stem_norm_bwd_workspace(long long rows, int C) { return rows <= 0 || C <= 0 ? 0 : vig::stem_norm_bwd_workspace(rows, C); }
+
+int vig_stem_norm_bwd(const void* x, const float* pre_bias, const float* weight, const float* bias, const void* dy, void* dx, float* dparams,
+                      void* workspace, size_t workspace_bytes, long long rows, int C, float eps, int silu, int x_dtype, int y_dtype,
+                      void* stream) {
+  if (!x || !weight || !bias || !dy || !dparams || rows <= 0 || C <= 0) return VIG_EINVAL;
+  if (!aligned16(x, pre_bias, weight, bias, dy, dx) || !aligned16(dparams, workspace)) return VIG_EINVAL;
+  if (!dtype_ok(x_dtype) || !dtype_ok(y_dtype) || !vig::stem_norm_supported(rows, C, x_dtype, y_dtype)) return VIG_ENOTSUP;
+  if (!workspace || workspace_bytes < vig::stem_norm_bwd_workspace(rows, C)) return VIG_ENOSPC;
+  return vig::launch_stem_norm_bwd(x, pre_bias, weight, bias, dy, dx, dparams, workspace, rows, C, eps, silu, x_dtype, y_dtype, (hipStream_t)stream);
 }
 
 int vig_split_heads_fwd(const void* qkv, void* q, void* k, void* v, int B, int L, int H, int Dk, int Dv,

@@ -16,6 +16,8 @@
 // ViG-S, B 128 at 224 px under bf16 autocast, forward and backward on one MI355X: 23.7 -> 11.0 ms.
 #include <ATen/autocast_mode.h>
 
+#include <torch/csrc/autograd/autograd.h>
+
 #include "host_calls.h"
 
 namespace vig_host {
@@ -535,6 +537,68 @@ struct MlpNode : torch::autograd::Function<MlpNode> {
   }
 };
 
+// A layer norm of the patch embedding with the bias of the convolution in front and, if asked for, the SiLU behind it.  x [B, C, h, w] in
+// channels-last memory.
+struct StemNormNode : torch::autograd::Function<StemNormNode> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, const std::optional<Tensor>& pre_arg, const Tensor& weight, const Tensor& bias,
+                        double eps, bool silu, bool narrow) {
+    const c10::DeviceGuard guard(x.device());
+    const Tensor pre = pre_arg ? *pre_arg : Tensor();
+    const int64_t C = x.size(1), rows = x.numel() / C;
+    Tensor y = at::empty(x.sizes(), x.options().dtype(scalar_type(narrow)).memory_format(at::MemoryFormat::ChannelsLast));
+    check_rc(vig_stem_norm_fwd(x.data_ptr(), pre.defined() ? fptr(pre) : nullptr, fptr(weight), fptr(bias), y.data_ptr(), rows, (int)C, (float)eps,
+                               silu, dtype_code(x), dtype_code(y), stream_of(x)),
+             "vig_stem_norm_fwd");
+    ctx->save_for_backward({x, pre, weight, bias});
+    ctx->saved_data["eps"] = eps;
+    ctx->saved_data["silu"] = silu;
+    return y;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const NoAutocast no_autocast;
+    const auto s = ctx->get_saved_variables();
+    const Tensor &x = s[0], &pre = s[1], &weight = s[2], &bias = s[3];
+    const double eps = ctx->saved_data["eps"].toDouble();
+    const bool silu = ctx->saved_data["silu"].toBool();
+    variable_list out(7);
+    // (an absent bias has no edge)
+    const int first = pre.defined() ? 2 : 1;
+    const bool wants[4] = {ctx->needs_input_grad(0), pre.defined() && ctx->needs_input_grad(1), ctx->needs_input_grad(first),
+                           ctx->needs_input_grad(first + 1)};
+    if (at::GradMode::is_enabled()) {  // a graph of the gradients is wanted: the same from operators that have one
+      Tensor z = x.permute({0, 2, 3, 1}).to(at::kFloat);
+      if (pre.defined()) z = z + pre;
+      z = at::layer_norm(z, {x.size(1)}, weight, bias, eps);
+      if (silu) z = at::silu(z);
+      z = z.to(grads[0].scalar_type()).permute({0, 3, 1, 2});
+      variable_list in;
+      for (int i = 0; i < 4; ++i)
+        if (wants[i]) in.push_back(s[i]);
+      const auto g = torch::autograd::grad({z}, in, {grads[0]}, true, true, true);
+      for (int i = 0, at = 0; i < 4; ++i)
+        if (wants[i]) out[i] = g[at++];
+      return out;
+    }
+    const c10::DeviceGuard guard(x.device());
+    Tensor dy = grads[0].contiguous(at::MemoryFormat::ChannelsLast);
+    if (!dy.permute({0, 2, 3, 1}).is_contiguous() || !aligned(dy)) dy = dy.permute({0, 2, 3, 1}).clone(at::MemoryFormat::Contiguous).permute({0, 3, 1, 2});
+    const int64_t C = x.size(1), rows = x.numel() / C;
+    Tensor dx, dparams = at::empty({3, C}, weight.options());
+    if (wants[0]) dx = at::empty_like(x);
+    const size_t need = vig_stem_norm_bwd_workspace(rows, (int)C);
+    Tensor ws = bytes_like(need, x);
+    check_rc(vig_stem_norm_bwd(x.data_ptr(), pre.defined() ? fptr(pre) : nullptr, fptr(weight), fptr(bias), dy.data_ptr(),
+                               dx.defined() ? dx.data_ptr() : nullptr, fptr(dparams), ws.data_ptr(), need, rows, (int)C, (float)eps, silu,
+                               dtype_code(x), dtype_code(dy), stream_of(x)),
+             "vig_stem_norm_bwd");
+    out[0] = dx;
+    if (wants[1]) out[1] = dparams.select(0, 2);
+    if (wants[2]) out[2] = dparams.select(0, 0);
+    if (wants[3]) out[3] = dparams.select(0, 1);
+    return out;
+  }
+};
+
 // Whether branch and residual are rows the nodes take and the weights share one usable type; sets the products' type.
 bool stream_ok(const Tensor& branch, const Tensor& residual, const Tensor* const* params, int n, bool& bf16) {
   if (!branch.defined() || !branch.is_cuda() || branch.dim() != 3 || branch.numel() == 0 || observed()) return false;
@@ -618,6 +682,38 @@ PyObject* block_mlp(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (I <= 0 || I % 8 || !is_shape(norm_w, {C}) || !is_shape(gate_w, {2 * I, C})) Py_RETURN_NONE;
   auto r = MlpNode::apply(branch, residual, norm_w, gate_w, down_w, eps, bf16);
   return Py_BuildValue("(NN)", THPVariable_Wrap(r[0]), THPVariable_Wrap(r[1]));
+  END_HANDLE_TH_ERRORS
+}
+
+// stem_norm(x, convolution's bias or None, weight, bias, eps, silu, last) -> the norm of the map (in the products' type, the last one in fp32), or
+// None for a call the node does not take
+PyObject* stem_norm(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK_TYPE(n == 7, "stem_norm takes 7 arguments");
+  for (int i = 0; i < 4; ++i)
+    if (!is_tensor(a[i]) && !(i == 1 && a[i] == Py_None)) Py_RETURN_NONE;
+  const Tensor &x = THPVariable_Unpack(a[0]), &weight = THPVariable_Unpack(a[2]), &bias = THPVariable_Unpack(a[3]);
+  const Tensor pre = tensor_arg(a[1]);
+  const double eps = PyFloat_AsDouble(a[4]);
+  if (PyErr_Occurred()) return nullptr;
+  const bool silu = PyObject_IsTrue(a[5]), last = PyObject_IsTrue(a[6]);
+  if (!x.defined() || !x.is_cuda() || x.dim() != 4 || x.numel() == 0 || observed() ||
+      c10::impl::tls_local_dispatch_key_set().included_.has(c10::DispatchKey::FuncTorchDynamicLayerFrontMode))
+    Py_RETURN_NONE;
+  const auto dev = x.device();
+  if (x.unsafeGetTensorImpl()->is_python_dispatch() || x.layout() != at::kStrided || !x.is_contiguous(at::MemoryFormat::ChannelsLast) ||
+      !x.permute({0, 2, 3, 1}).is_contiguous() || !aligned(x))
+    Py_RETURN_NONE;
+  const int64_t C = x.size(1), rows = x.numel() / C;
+  for (const Tensor* t : {&weight, &bias, &pre})
+    if (t->defined() && (!plain(*t, dev) || t->scalar_type() != at::kFloat || !is_shape(*t, {C}))) Py_RETURN_NONE;
+  for (const Tensor* t : {&x, &weight, &bias, &pre})
+    if (t->defined() && t->_fw_grad(0).defined()) Py_RETURN_NONE;  // (forward-mode derivatives: the operators have them)
+  const bool mixed = at::autocast::is_autocast_enabled(at::kCUDA);
+  // the norm under autocast is one in fp32 whatever it reads, and the next convolution casts; without, map and parameters are of one type
+  if (x.scalar_type() != (mixed ? at::kBFloat16 : at::kFloat) || (mixed && at::autocast::get_autocast_dtype(at::kCUDA) != at::kBFloat16)) Py_RETURN_NONE;
+  if (C % 8 || C > 1024 || rows > 0x7fffffff - 8192) Py_RETURN_NONE;
+  return THPVariable_Wrap(StemNormNode::apply(x, pre.defined() ? std::optional<Tensor>(pre) : std::nullopt, weight, bias, eps, silu, mixed && !last));
   END_HANDLE_TH_ERRORS
 }
 

@@ -602,8 +602,8 @@ class V2PatchEmbed(_CacheMixin, nn.Module):
         inside the last norm's kernel."""
         # channels-last throughout: the convolutions run in that layout, the norms see row matrices, and the final
         # 'b c h w -> b (h w) c' is a view; each convolution's bias add rides in the norm kernel behind it
-        if _recording(self):  # plain modules, differentiable (LayerNorm2d and the convolutions record their graph)
-            x = self.proj(x)
+        if _recording(self):  # differentiable: convolutions of torch, each norm with its neighbours one native node where that takes it
+            x = self._recorded(x)
             hw = tuple(x.shape[-2:])
             x = x.flatten(2).transpose(1, 2)
             if pos_embed is not None:
@@ -627,6 +627,28 @@ class V2PatchEmbed(_CacheMixin, nn.Module):
             pos_embed = resize_pos_embed(pos_embed, pos_shape, hw).to(x.dtype)
         x = norm2(x, pre_bias=_f32(self, "b2", conv2.bias), post_add=pos_embed)
         return x.flatten(2).transpose(1, 2), hw
+
+    def _recorded(self, x):
+        """self.proj(x): the convolutions without their biases, each norm one autograd node (csrc/train_block.cpp) with the bias in front of
+        it and the activation behind it.  Modules of other types or with something hanging on their calls run as modules, and so does
+        what the node does not take."""
+        calls, proj = _ext.calls(), self.proj
+        if (calls is None or type(proj) is not nn.Sequential or [type(m) for m in proj] != [nn.Conv2d, LayerNorm2d, nn.SiLU, nn.Conv2d, LayerNorm2d]
+                or not _direct(proj, *proj) or any(m.padding_mode != "zeros" for m in (proj[0], proj[3]))):
+            return proj(x)
+        for conv, norm, act, last in ((proj[0], proj[1], proj[2], False), (proj[3], proj[4], None, True)):
+            rows = norm.elementwise_affine and norm.bias is not None and norm.normalized_shape == (conv.out_channels,)
+            if not rows or not x.is_cuda or conv.weight.dtype != torch.float32:
+                x = norm(conv(x))
+                x = x if act is None else act(x)
+                continue
+            x = F.conv2d(x, conv.weight, None, conv.stride, conv.padding, conv.dilation, conv.groups)
+            y = calls.stem_norm(x, conv.bias, norm.weight, norm.bias, norm.eps, act is not None, last)
+            if y is None:
+                x = norm(x if conv.bias is None else x + conv.bias.to(x.dtype).view(1, -1, 1, 1))
+                y = x if act is None else act(x)
+            x = y
+        return x
 
     def _packed_w1(self):
         """The first convolution's weight in the kernel's packed form, rebuilt when the parameter changes."""
