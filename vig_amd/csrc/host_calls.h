@@ -97,6 +97,7 @@ inline bool is_tensor(PyObject* o) { return THPVariable_Check(o); }
 // the methods of train_block.cpp
 PyObject* block_mix(PyObject*, PyObject* const* a, Py_ssize_t n);
 PyObject* block_mlp(PyObject*, PyObject* const* a, Py_ssize_t n);
+PyObject* stem_conv(PyObject*, PyObject* const* a, Py_ssize_t n);
 PyObject* stem_norm(PyObject*, PyObject* const* a, Py_ssize_t n);
 
 // the methods of model_forward.cpp

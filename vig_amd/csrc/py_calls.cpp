@@ -163,6 +163,7 @@ PyMethodDef kMethods[] = {
     {"gla_gate", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(gla_gate)), METH_FASTCALL, nullptr},
     {"block_mix", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(block_mix)), METH_FASTCALL, nullptr},
     {"block_mlp", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(block_mlp)), METH_FASTCALL, nullptr},
+    {"stem_conv", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(stem_conv)), METH_FASTCALL, nullptr},
     {"stem_norm", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(stem_norm)), METH_FASTCALL, nullptr},
     {"make_plan", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(make_plan)), METH_FASTCALL, nullptr},
     {"plan_describes", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(plan_describes)), METH_FASTCALL, nullptr},

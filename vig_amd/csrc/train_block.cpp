@@ -599,6 +599,37 @@ struct StemNormNode : torch::autograd::Function<StemNormNode> {
   }
 };
 
+// A convolution of the patch embedding without its bias: the library's kernel forward, torch's operator for the gradients.  x bf16, as it arrives
+// ([B, Cin, H, W] in memory) in front of the first one, channels-last for the second; w bf16 in channels-last memory.
+struct StemConvNode : torch::autograd::Function<StemConvNode> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w, int64_t stride) {
+    const NoAutocast no_autocast;
+    const c10::DeviceGuard guard(x.device());
+    const int B = (int)x.size(0), Cin = (int)x.size(1), H = (int)x.size(2), W = (int)x.size(3), Cout = (int)w.size(0), KH = (int)w.size(2),
+              KW = (int)w.size(3);
+    Tensor y = at::empty({B, Cout, (H + 2 - KH) / stride + 1, (W + 2 - KW) / stride + 1}, x.options().memory_format(at::MemoryFormat::ChannelsLast));
+    if (stride == 2) {
+      check_rc(vig_conv3x3s2_fwd(x.data_ptr(), w.data_ptr(), y.data_ptr(), B, H, W, Cin, Cout, stream_of(x)), "vig_conv3x3s2_fwd");
+    } else {
+      Tensor packed = at::zeros({Cout, Cin, KH, 16}, w.options().memory_format(at::MemoryFormat::Contiguous));
+      packed.narrow(3, 0, KW).copy_(w);
+      check_rc(vig_patch_conv_fwd(x.data_ptr(), packed.data_ptr(), y.data_ptr(), B, Cin, H, W, KH, KW, (int)stride, 1, Cout, VIG_BF16, stream_of(x)),
+               "vig_patch_conv_fwd");
+    }
+    ctx->save_for_backward({x, w});
+    ctx->saved_data["stride"] = stride;
+    return y;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const NoAutocast no_autocast;
+    const auto s = ctx->get_saved_variables();
+    const int64_t stride = ctx->saved_data["stride"].toInt();
+    const auto g = at::convolution_backward(grads[0], s[0], s[1], c10::nullopt, {stride, stride}, {1, 1}, {1, 1}, false, {0, 0}, 1,
+                                            {ctx->needs_input_grad(0), ctx->needs_input_grad(1), false});
+    return {std::get<0>(g), std::get<1>(g), Tensor()};
+  }
+};
+
 // Whether branch and residual are rows the nodes take and the weights share one usable type; sets the products' type.
 bool stream_ok(const Tensor& branch, const Tensor& residual, const Tensor* const* params, int n, bool& bf16) {
   if (!branch.defined() || !branch.is_cuda() || branch.dim() != 3 || branch.numel() == 0 || observed()) return false;
@@ -682,6 +713,42 @@ PyObject* block_mlp(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (I <= 0 || I % 8 || !is_shape(norm_w, {C}) || !is_shape(gate_w, {2 * I, C})) Py_RETURN_NONE;
   auto r = MlpNode::apply(branch, residual, norm_w, gate_w, down_w, eps, bf16);
   return Py_BuildValue("(NN)", THPVariable_Wrap(r[0]), THPVariable_Wrap(r[1]));
+  END_HANDLE_TH_ERRORS
+}
+
+// stem_conv(x, weight, stride) -> the convolution with padding 1 and without a bias, under bf16 autocast, or None for a call the node does not take: the
+// kernels' shapes (the first convolution of images three channels deep, 9 x 9 at stride 8; 3 x 3 at stride 2), as in evaluation.
+// us, 128 images of 224 px, the convolution library's (the first with the layout change in front of it) / here: 192 channels 93 / 40, 384 98 / 55; a training
+// pass of ViG-S under autocast 10.37 -> 10.25 ms.  (As in evaluation, a pixel that is not finite also reaches the window that ends in front of it: the zeros that fill
+// a kernel row up to 16 columns multiply it.)
+PyObject* stem_conv(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK_TYPE(n == 3, "stem_conv takes 3 arguments");
+  if (!is_tensor(a[0]) || !is_tensor(a[1])) Py_RETURN_NONE;
+  const Tensor &x = THPVariable_Unpack(a[0]), &weight = THPVariable_Unpack(a[1]);
+  const int64_t stride = PyLong_AsLong(a[2]);
+  if (PyErr_Occurred()) return nullptr;
+  if ((stride != 2 && stride != 8) || !x.defined() || !x.is_cuda() || x.dim() != 4 || weight.dim() != 4 || x.numel() == 0 || weight.numel() == 0 || observed() ||
+      !at::autocast::is_autocast_enabled(at::kCUDA) || at::autocast::get_autocast_dtype(at::kCUDA) != at::kBFloat16 ||
+      c10::impl::tls_local_dispatch_key_set().included_.has(c10::DispatchKey::FuncTorchDynamicLayerFrontMode))
+    Py_RETURN_NONE;
+  for (const Tensor* t : {&x, &weight})
+    if (t->unsafeGetTensorImpl()->is_python_dispatch() || t->layout() != at::kStrided || t->device() != x.device() || t->_fw_grad(0).defined() ||
+        (t->scalar_type() != at::kFloat && t->scalar_type() != at::kBFloat16))
+      Py_RETURN_NONE;
+  const int64_t Cout = weight.size(0), Cin = weight.size(1), KH = weight.size(2), KW = weight.size(3), H = x.size(2), W = x.size(3);
+  if (x.size(1) != Cin || x.numel() > 0x7fffffff || x.size(0) * Cout > 0x7fffffff / ((H / stride + 1) * (W / stride + 1)) ||
+      !weight.permute({0, 2, 3, 1}).is_contiguous())
+    Py_RETURN_NONE;
+  if (stride == 2) {
+    if (KH != 3 || KW != 3 || Cin % 32 || Cout % 8 || !x.permute({0, 2, 3, 1}).is_contiguous()) Py_RETURN_NONE;
+  } else if (KW > 16 || Cin * KH != 27 || H + 2 < KH || W + 2 < KW || W % 8 || (W > 248 && KW > 9) || Cout % 32 ||
+             !((Cout >= 64 && Cout <= 256) || Cout == 384) || !x.is_contiguous()) {
+    Py_RETURN_NONE;
+  }
+  const Tensor xb = at::autocast::cached_cast(at::kBFloat16, x, at::kCUDA), wb = at::autocast::cached_cast(at::kBFloat16, weight, at::kCUDA);
+  if (!aligned(xb) || !aligned(wb) || !wb.permute({0, 2, 3, 1}).is_contiguous()) Py_RETURN_NONE;
+  return THPVariable_Wrap(StemConvNode::apply(xb, wb, stride));
   END_HANDLE_TH_ERRORS
 }
 

@@ -629,7 +629,7 @@ class V2PatchEmbed(_CacheMixin, nn.Module):
         return x.flatten(2).transpose(1, 2), hw
 
     def _recorded(self, x):
-        """self.proj(x): the convolutions without their biases, each norm one autograd node (csrc/train_block.cpp) with the bias in front of
+        """self.proj(x): the convolutions without their biases (under autocast the library's kernels forward), each norm one autograd node (csrc/train_block.cpp) with the bias in front of
         it and the activation behind it.  Modules of other types or with something hanging on their calls run as modules, and so does
         what the node does not take."""
         calls, proj = _ext.calls(), self.proj
@@ -642,7 +642,9 @@ class V2PatchEmbed(_CacheMixin, nn.Module):
                 x = norm(conv(x))
                 x = x if act is None else act(x)
                 continue
-            x = F.conv2d(x, conv.weight, None, conv.stride, conv.padding, conv.dilation, conv.groups)
+            plain = (conv.stride in ((2, 2), (8, 8)) and conv.padding == conv.dilation == (1, 1) and conv.groups == 1)
+            y = calls.stem_conv(x, conv.weight, conv.stride[0]) if plain else None
+            x = F.conv2d(x, conv.weight, None, conv.stride, conv.padding, conv.dilation, conv.groups) if y is None else y
             y = calls.stem_norm(x, conv.bias, norm.weight, norm.bias, norm.eps, act is not None, last)
             if y is None:
                 x = norm(x if conv.bias is None else x + conv.bias.to(x.dtype).view(1, -1, 1, 1))
