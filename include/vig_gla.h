@@ -271,6 +271,17 @@ size_t vig_gla_bidir_bwd_workspace(int B, int H, int L, int Dk, int Dv, int bidi
 size_t vig_gla_bidir_bwd_workspace_for(int B, int H, int L, int Dk, int Dv, int io_dtype, int gate_dtype,
                                        int bidirectional);
 
+/*
+ * vig_gla_bidir_bwd for q, k, v in the columns of a matrix [B * L, row_stride], head h's channels at q + h*Dk, k + h*Dk and v + h*Dv of a token's
+ * row, and dq, dk, dv likewise in one of d_row_stride; the other tensors and the workspace as there, and the same results.  Both directions,
+ * bf16 tensors and gates, Dk in {32, 64}, Dv = 64, L <= 256; VIG_ENOTSUP otherwise.  Row strides are multiples of 8 up to 2^20 elements.
+ *
+ * Replaces: the backward of the head split (classification/models/vig.py:401-409) around that of the op.
+ */
+int vig_gla_bidir_bwd_rows(const void* q, const void* k, const void* v, long long row_stride, const void* g_fwd, const void* g_bwd, const void* d_o,
+                           void* dq, void* dk, void* dv, long long d_row_stride, void* dg_fwd, void* dg_bwd, void* workspace, size_t workspace_bytes,
+                           int B, int H, int L, int Dk, int Dv, float scale, float out_scale, int io_dtype, int gate_dtype, void* stream);
+
 /* Same contract as vig_gla_bidir_bwd, always the fp32-arithmetic token-recurrent kernel (the exact path). */
 int vig_gla_bidir_bwd_exact(const void* q, const void* k, const void* v,
                             const void* g_fwd, const void* g_bwd, const void* d_o,

@@ -81,7 +81,8 @@ int launch_pad_channels_multi(const void* const* src, void* const* dst, const in
 int launch_gla_backward(const void* q, const void* k, const void* v, const void* g_fwd, const void* g_bwd,
                         const void* d_o, void* dq, void* dk, void* dv, void* dg_fwd, void* dg_bwd, void* workspace,
                         int B, int H, int L, int Dk, int Dv, float scale, float out_scale, int io_dtype,
-                        int gate_dtype, bool exact, size_t beyond, hipStream_t stream);
+                        int gate_dtype, bool exact, size_t beyond, hipStream_t stream, long long ld_in = 0, long long ld_out = 0);
+bool gla_backward_in_place(int L, int Dk, int Dv, int io_dtype, int gate_dtype, bool bidir);
 size_t gla_backward_workspace(int B, int H, int L, int Dk, int Dv, int bidir);  // (launch_gla_backward's; `beyond`: bytes behind it)
 bool linear_wgrad_supported(long long T, int N, int K);
 size_t matmul_f32_workspace(long long M, int N, long long K);
@@ -990,6 +991,20 @@ int vig_gla_bidir_bwd(const void* q, const void* k, const void* v, const void* g
                       int io_dtype, int gate_dtype, void* stream) {
   return gla_bidir_bwd(q, k, v, g_fwd, g_bwd, d_o, dq, dk, dv, dg_fwd, dg_bwd, workspace, workspace_bytes, B, H, L, Dk,
                        Dv, scale, out_scale, io_dtype, gate_dtype, false, stream);
+}
+
+int vig_gla_bidir_bwd_rows(const void* q, const void* k, const void* v, long long row_stride, const void* g_fwd, const void* g_bwd, const void* d_o,
+                           void* dq, void* dk, void* dv, long long d_row_stride, void* dg_fwd, void* dg_bwd, void* workspace, size_t workspace_bytes,
+                           int B, int H, int L, int Dk, int Dv, float scale, float out_scale, int io_dtype, int gate_dtype, void* stream) {
+  if (!q || !k || !v || !g_fwd || !g_bwd || !d_o || !dq || !dk || !dv || !dg_fwd || !dg_bwd || B <= 0 || H <= 0 || L <= 0) return VIG_EINVAL;
+  if (!aligned16(q, k, v, g_fwd, g_bwd, d_o, dq, dk, dv, dg_fwd, dg_bwd, workspace)) return VIG_EINVAL;
+  if (!vig::gla_backward_in_place(L, Dk, Dv, io_dtype, gate_dtype, true) || (long long)B * H > 2147483647LL) return VIG_ENOTSUP;
+  for (const long long ld : {row_stride, d_row_stride})
+    if (ld < (long long)H * std::max(Dk, Dv) || ld % 8 != 0 || ld > (1 << 20)) return VIG_EINVAL;
+  const size_t need = vig::gla_backward_workspace(B, H, L, Dk, Dv, 1);
+  if (!workspace || workspace_bytes < need) return VIG_ENOSPC;
+  return vig::launch_gla_backward(q, k, v, g_fwd, g_bwd, d_o, dq, dk, dv, dg_fwd, dg_bwd, workspace, B, H, L, Dk, Dv, scale, out_scale, io_dtype,
+                                  gate_dtype, false, workspace_bytes - need, (hipStream_t)stream, row_stride, d_row_stride);
 }
 
 // Same contract, always the fp32-arithmetic token-recurrent kernel.

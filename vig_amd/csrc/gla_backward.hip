@@ -31,6 +31,7 @@ struct GlaBwdArgs {
   hipStream_t stream;
   int* only_flagged;  // null: every slab; else one int per (batch, head): slabs with 0 are skipped
   bool split;         // the two directions in workgroups of their own (fp32 tensors, flagged slabs)
+  long long ld_in, ld_out;  // q, k, v (their gradients) in rows of a matrix, elements apart; 0: head-major tensors
 };
 
 // Stores and loads of what the two workgroups of a split slab hand each other: through to memory, past the L2 of their own chiplet
@@ -41,11 +42,13 @@ __device__ __forceinline__ void store_shared(float* p, float x, bool shared) {
 }
 __device__ __forceinline__ float load_shared(const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
-template <typename TIO, typename TG, int DK, int DV, int TB>
+// PITCHED: q, k, v and their gradients lie in the rows of two matrices, ld_in and ld_out elements apart (H heads)
+template <typename TIO, typename TG, int DK, int DV, int TB, bool PITCHED>
 __global__ __launch_bounds__(256) void gla_backward_kernel(
     const TIO* __restrict__ q, const TIO* __restrict__ k, const TIO* __restrict__ v, const TG* __restrict__ gf,
     const TG* __restrict__ gb, const TIO* __restrict__ d_o, TIO* dq, TIO* dk, TIO* dv, TG* dgf, TG* dgb,
-    float* ws_dq, float* ws_acc_k, float* ws_acc_v, int L, float scale, float out_scale, int* only_flagged, int split) {
+    float* ws_dq, float* ws_acc_k, float* ws_acc_v, int L, float scale, float out_scale, int* only_flagged, int split, int H,
+    long long ld_in, long long ld_out) {
   // second pass behind the matrix-core kernel: only the slabs it left out (uniform per workgroup, before any barrier)
   if (only_flagged && only_flagged[blockIdx.x] == 0) return;
   constexpr bool kSplit = sizeof(TIO) == 4;
@@ -64,6 +67,13 @@ __global__ __launch_bounds__(256) void gla_backward_kernel(
   const size_t bh = blockIdx.x;
   const size_t qk_base = bh * (size_t)L * DK;
   const size_t vo_base = bh * (size_t)L * DV;
+  const size_t b = PITCHED ? bh / H : 0, head = PITCHED ? bh - b * H : 0;
+  const size_t in = PITCHED ? (size_t)ld_in : 0, out = PITCHED ? (size_t)ld_out : 0;
+  // where channel 0 of a token's q and k, v, dq and dk, dv lies
+  const auto qk_in = [&](int tok) { return PITCHED ? (b * L + tok) * in + head * DK : qk_base + (size_t)tok * DK; };
+  const auto v_in = [&](int tok) { return PITCHED ? (b * L + tok) * in + head * DV : vo_base + (size_t)tok * DV; };
+  const auto qk_out = [&](int tok) { return PITCHED ? (b * L + tok) * out + head * DK : qk_base + (size_t)tok * DK; };
+  const auto v_out = [&](int tok) { return PITCHED ? (b * L + tok) * out + head * DV : vo_base + (size_t)tok * DV; };
   const int nblk = (L + TB - 1) / TB;
   const int ndir = gb ? 2 : 1;
   const bool row_ok = lane < DK;  // layout B lanes that own a state row
@@ -76,8 +86,8 @@ __global__ __launch_bounds__(256) void gla_backward_kernel(
       float fq = 0.f, fk = 0.f, fa = 1.f;
       if (tok < L) {
         const size_t off = qk_base + (size_t)tok * DK + d;
-        if (with_q) fq = Elem<TIO>::load(q + off) * scale;
-        fk = Elem<TIO>::load(k + off);
+        if (with_q) fq = Elem<TIO>::load(q + qk_in(tok) + d) * scale;
+        fk = Elem<TIO>::load(k + qk_in(tok) + d);
         fa = __expf(Elem<TG>::load(g + off));
       }
       sq[t][d] = fq;
@@ -89,7 +99,7 @@ __global__ __launch_bounds__(256) void gla_backward_kernel(
       const int tok = t0 + t;
       float fv = 0.f, fd = 0.f;
       if (tok < L) {
-        fv = Elem<TIO>::load(v + vo_base + (size_t)tok * DV + c);
+        fv = Elem<TIO>::load(v + v_in(tok) + c);
         fd = Elem<TIO>::load(d_o + vo_base + (size_t)tok * DV + c) * out_scale;
       }
       sv[t][c] = fv;
@@ -196,7 +206,7 @@ __global__ __launch_bounds__(256) void gla_backward_kernel(
                 continue;
               }
               if (ndir == 2) s += ws_acc_v[off];
-              Elem<TIO>::store(dv + off, s);
+              Elem<TIO>::store(dv + v_out(tok) + c, s);
             }
           }
         }
@@ -211,7 +221,7 @@ __global__ __launch_bounds__(256) void gla_backward_kernel(
             // this direction's part of the gate gradient below (unscaled q: my_dq already carries the scale), taken here by all
             // threads: the running sum's own loop waited for two rows from memory per token, one after the other (fp32, L 196:
             // 384 sequences of 32 key channels 493 -> 426 us, 768 of 64 745 -> 678)
-            pk[0][t][d] = Elem<TIO>::load(q + off) * sq_ - sk[t][d] * s;
+            pk[0][t][d] = Elem<TIO>::load(q + qk_in(tok) + d) * sq_ - sk[t][d] * s;
             if (ndir == 2 && !last_dir) {
               store_shared(ws_acc_k + off, s, split);
             } else {
@@ -223,8 +233,8 @@ __global__ __launch_bounds__(256) void gla_backward_kernel(
                 s += ws_acc_k[off];
                 sq_ += ws_dq[bh * (size_t)L * DK + (size_t)tok * DK + d];  // the first direction's dq
               }
-              Elem<TIO>::store(dk + off, s);
-              Elem<TIO>::store(dq + off, sq_);
+              Elem<TIO>::store(dk + qk_out(tok) + d, s);
+              Elem<TIO>::store(dq + qk_out(tok) + d, sq_);
             }
           }
         }
@@ -274,10 +284,16 @@ static int launch_bwd_t(const GlaBwdArgs& a) {
   float* ws_acc_k = ws + (size_t)ndir * n_qk;
   float* ws_acc_v = ws_acc_k + n_qk;
   (void)n_v;
-  hipLaunchKernelGGL((gla_backward_kernel<TIO, TG, DK, DV, TB>), dim3(a.B * a.H, a.split ? 2 : 1), dim3(256), 0, a.stream,
+  constexpr bool kPitched = sizeof(TIO) == 2 && sizeof(TG) == 2 && DK >= 32 && DV == 64;
+  auto* kernel = gla_backward_kernel<TIO, TG, DK, DV, TB, false>;
+  if (a.ld_in) {
+    if constexpr (kPitched) kernel = gla_backward_kernel<TIO, TG, DK, DV, TB, true>;
+    else return -95;
+  }
+  hipLaunchKernelGGL(kernel, dim3(a.B * a.H, a.split ? 2 : 1), dim3(256), 0, a.stream,
                      (const TIO*)a.q, (const TIO*)a.k, (const TIO*)a.v, (const TG*)a.g_fwd, (const TG*)a.g_bwd,
                      (const TIO*)a.d_o, (TIO*)a.dq, (TIO*)a.dk, (TIO*)a.dv, (TG*)a.dg_fwd, (TG*)a.dg_bwd, ws_dq,
-                     ws_acc_k, ws_acc_v, a.L, a.scale, a.out_scale, a.only_flagged, (int)a.split);
+                     ws_acc_k, ws_acc_v, a.L, a.scale, a.out_scale, a.only_flagged, (int)a.split, a.H, a.ld_in, a.ld_out);
   return hipGetLastError() == hipSuccess ? 0 : -5;
 }
 
@@ -310,18 +326,24 @@ size_t gla_backward_workspace(int B, int H, int L, int Dk, int Dv, int bidir) {
   return flags_end(B, H, L, Dk, Dv, bidir) + seg;
 }
 
+// q, k, v in the rows of a matrix and their gradients into those of another: whole sequences on the matrix cores
+bool gla_backward_in_place(int L, int Dk, int Dv, int io_dtype, int gate_dtype, bool bidir) {
+  return bidir && L <= 256 && (Dk == 32 || Dk == 64) && Dv == 64 && io_dtype == 1 && gate_dtype == 1;
+}
+
 int launch_gla_backward(const void* q, const void* k, const void* v, const void* g_fwd, const void* g_bwd,
                         const void* d_o, void* dq, void* dk, void* dv, void* dg_fwd, void* dg_bwd, void* workspace,
                         int B, int H, int L, int Dk, int Dv, float scale, float out_scale, int io_dtype,
-                        int gate_dtype, bool exact, size_t beyond, hipStream_t stream) {
+                        int gate_dtype, bool exact, size_t beyond, hipStream_t stream, long long ld_in, long long ld_out) {
   GlaBwdArgs a{q, k, v, g_fwd, g_bwd, d_o, dq, dk, dv, dg_fwd, dg_bwd, workspace, B, H, L, Dk, Dv,
-               scale, out_scale, io_dtype, gate_dtype, stream, nullptr, false};
+               scale, out_scale, io_dtype, gate_dtype, stream, nullptr, false, ld_in, ld_out};
+  if (ld_in && (exact || !gla_backward_in_place(L, Dk, Dv, io_dtype, gate_dtype, g_bwd != nullptr))) return -95;
   if (!exact && gla_backward_mfma_supported(B, H, L, Dk, Dv, io_dtype, gate_dtype, g_bwd != nullptr)) {
     int* flags = reinterpret_cast<int*>((float*)workspace + recurrent_floats(B, H, L, Dk, Dv, g_bwd != nullptr));
     void* seg_ws = (char*)workspace + flags_end(B, H, L, Dk, Dv, g_bwd != nullptr);
     const int rc = launch_gla_backward_mfma(q, k, v, g_fwd, g_bwd, d_o, dq, dk, dv, dg_fwd, dg_bwd, flags, workspace,
                                             recurrent_floats(B, H, L, Dk, Dv, g_bwd != nullptr) * sizeof(float), seg_ws,
-                                            gla_backward_mfma_workspace(B, H, L, Dk, Dv), B, H, L, Dk, scale * out_scale, stream);
+                                            gla_backward_mfma_workspace(B, H, L, Dk, Dv), B, H, L, Dk, scale * out_scale, ld_in, ld_out, stream);
     if (rc != 0) return rc;
     a.only_flagged = flags;  // slabs with gates beyond the matrix-core kernel's range
   }

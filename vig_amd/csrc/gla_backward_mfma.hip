@@ -229,12 +229,13 @@ __device__ __forceinline__ float before_lane(float x, int r) {
 // by way of `turn`, so that a store instruction writes one contiguous KB instead of 64 pieces of 16 bytes in as many 64-byte
 // blocks: 768 slabs of 196 tokens 96.1 -> 90.6 us, 1200 of 128 83.5 -> 77.  Dk = 32 gains nothing by it (58.5, 59.1) and slabs of one
 // or two tiles lose the latency (25.3 against 24.0).
-template <int NG, int TW>
-__device__ __forceinline__ void store_rows(uint16_t* turn, const u32x4_t (&x)[NG], rsrc_t out, int lane) {
+template <int NG, int TW, bool PITCHED = false>
+__device__ __forceinline__ void store_rows(uint16_t* turn, const u32x4_t (&x)[NG], rsrc_t out, int lane, unsigned pitch = 32u * NG) {
   const int r = lane & 31, h = lane >> 5;
   if constexpr (!BwdLds<TW>::turns(NG)) {
 #pragma unroll
-    for (int g = 0; g < NG; ++g) __builtin_amdgcn_raw_buffer_store_b128(x[g], out, r * (32u * NG) + h * (16u * NG) + 16u * g, 0, 0);
+    for (int g = 0; g < NG; ++g)
+      __builtin_amdgcn_raw_buffer_store_b128(x[g], out, r * (PITCHED ? pitch : 32u * NG) + h * (16u * NG) + 16u * g, 0, 0);
   } else {
     lane = fresh_lane();
 #pragma unroll
@@ -245,7 +246,9 @@ __device__ __forceinline__ void store_rows(uint16_t* turn, const u32x4_t (&x)[NG
 #pragma unroll
       for (int j = 0; j < NG / 2; ++j) {
         const int piece = 64 * j + lane;
-        __builtin_amdgcn_raw_buffer_store_b128(load_piece(turn, piece / (2 * NG), piece % (2 * NG)), out, 512u * NG * half + 16u * piece, 0, 0);
+        const int row = piece / (2 * NG), at = piece % (2 * NG);
+        const unsigned to = PITCHED ? (16u * half + row) * pitch + 16u * at : 512u * NG * half + 16u * piece;
+        __builtin_amdgcn_raw_buffer_store_b128(load_piece(turn, row, at), out, to, 0, 0);
       }
     }
   }
@@ -258,6 +261,8 @@ struct BwdSlab {
   const uint16_t *sp, *rp, *rpt;  // sqrt(D) S_in as [k channel][v], sqrt(D) R_out as [k channel][v] and as [v][k channel]
   const float* carry;             // [2 directions][2 partial sums][64]: q dq - k dk summed over the segments walked later
   int L;                          // tokens of this slab / segment
+  // PITCHED: a token's q, k and v lie in one row of a matrix, their gradients in one of another; bytes from row to row
+  unsigned in, out;
 };
 
 // What a wave loads for one direction of one slab (its own 32-token tile), issued one phase ahead.
@@ -278,19 +283,26 @@ __device__ __forceinline__ void issue_bwd_gate_loads(const BwdNext& n, int w, in
   const int rows = tile_rows(n.L, w);
   issue_tdwords<0, 2, NG>(chunk_rsrc(n.g + (size_t)32 * w * DK, rows, 2 * DK), r, h, ld.gD);
 }
-template <int NG>
+template <int NG, bool PITCHED>
 __device__ __forceinline__ void issue_bwd_qk_loads(const BwdNext& n, int w, int r, int h, BwdLoads<NG>& ld) {
   constexpr int DK = 16 * NG;
   const int rows = tile_rows(n.L, w);
+  if constexpr (PITCHED) {
+    const size_t t = (size_t)(16 * w) * n.sl.in;
+    issue_raw_tile_pitched<NG>(chunk_rsrc(n.sl.q + t, rows, n.sl.in), 0, r, h, n.sl.in, ld.rawq);
+    issue_raw_tile_pitched<NG>(chunk_rsrc(n.sl.k + t, rows, n.sl.in), 0, r, h, n.sl.in, ld.rawk);
+    return;
+  }
   const size_t tk = (size_t)32 * w * DK;
   issue_raw_tile<NG>(chunk_rsrc(n.sl.q + tk, rows, 2 * DK), 0, r, h, ld.rawq);
   issue_raw_tile<NG>(chunk_rsrc(n.sl.k + tk, rows, 2 * DK), 0, r, h, ld.rawk);
 }
-template <int NG>
+template <int NG, bool PITCHED>
 __device__ __forceinline__ void issue_bwd_vdo_loads(const BwdNext& n, int w, int r, int h, BwdLoads<NG>& ld) {
   const int rows = tile_rows(n.L, w);
   const size_t tv = (size_t)32 * w * 64;
-  issue_raw_tile<4>(chunk_rsrc(n.sl.v + tv, rows, 128), 0, r, h, ld.rawv);
+  if constexpr (PITCHED) issue_raw_tile_pitched<4>(chunk_rsrc(n.sl.v + (size_t)(16 * w) * n.sl.in, rows, n.sl.in), 0, r, h, n.sl.in, ld.rawv);
+  else issue_raw_tile<4>(chunk_rsrc(n.sl.v + tv, rows, 128), 0, r, h, ld.rawv);
   issue_raw_tile<4>(chunk_rsrc(n.sl.d_o + tv, rows, 128), 0, r, h, ld.rawd);
 }
 
@@ -350,7 +362,7 @@ __device__ __forceinline__ bool bwd_anchor(int w, char* lds) {
 //   dq^_i += S_in' do_i,   dk^_j += R_out' v_j,   dv_j += R_out'^T k~_j
 // (the e^{G_i - a}, e^{a - G_j} factors applied to dq^, dk^ at the end turn e^a into e^{G_i}, e^{T - G_j}), and the
 // running sum of the gate gradient starts from the total of q dq - k dk over the segments walked later.
-template <bool FWD, bool FIRST, bool LAST, int NG, bool SEG, int TW>
+template <bool FWD, bool FIRST, bool LAST, int NG, bool SEG, int TW, bool PITCHED>
 __device__ __forceinline__ void bwd_direction(const BwdSlab& sl, int L, int ntiles, int w, char* lds,
                                               float s, f32x16_t (&dv)[2], u32x4_t (&keepq)[NG], u32x4_t (&keepk)[NG],
                                               BwdLoads<NG>& ld, const BwdNext& nxt, f32x16_t (&G)[2]) {
@@ -375,6 +387,9 @@ __device__ __forceinline__ void bwd_direction(const BwdSlab& sl, int L, int ntil
   float* dgtot = reinterpret_cast<float*>(lds + BwdLds<TW>::dgtot);
   const int rows = tile_rows(L, w);  // valid tokens of this wave's tile
   const size_t tk = (size_t)32 * w * DK, tv = (size_t)32 * w * 64;
+  // where the tile's rows of dq and dk start (dv), and how far apart they are
+  const size_t to_k = PITCHED ? (size_t)(16 * w) * sl.out : tk, to_v = PITCHED ? to_k : tv;
+  const unsigned out_k = PITCHED ? sl.out : 2 * DK, out_v = PITCHED ? sl.out : 128;
 
   // ---- this tile's loads were issued a phase ago; v and do rows go to LDS once per slab (nobody reads the previous
   // slab's any more; the next barrier makes them visible) ----
@@ -495,14 +510,14 @@ __device__ __forceinline__ void bwd_direction(const BwdSlab& sl, int L, int ntil
   if (kParkDq && !FIRST) {
 #pragma unroll
     for (int g = kParkLds; g < NG; ++g)
-      keepq[g] = __builtin_amdgcn_raw_buffer_load_b128(chunk_rsrc(sl.dq + tk, rows, 2 * DK), r * (32u * NG) + h * (16u * NG) + 16u * g, 0, 0);
+      keepq[g] = __builtin_amdgcn_raw_buffer_load_b128(chunk_rsrc(sl.dq + to_k, rows, out_k), r * out_k + h * (16u * NG) + 16u * g, 0, 0);
   }
   if (kEarlyGates) issue_bwd_gate_loads<NG>(nxt, w, r, h, ld);
-  if (kEarlyRows) issue_bwd_qk_loads<NG>(nxt, w, r, h, ld);
+  if (kEarlyRows) issue_bwd_qk_loads<NG, PITCHED>(nxt, w, r, h, ld);
   __builtin_amdgcn_sched_barrier(0);
   if (LAST) {
-    store_rows<4, TW>(turn, outv, chunk_rsrc(sl.dv + tv, rows, 128), lane);
-    store_rows<NG, TW>(turn, keepk, chunk_rsrc(sl.dk + tk, rows, 2 * DK), lane);
+    store_rows<4, TW, PITCHED>(turn, outv, chunk_rsrc(sl.dv + to_v, rows, out_v), lane, out_v);
+    store_rows<NG, TW, PITCHED>(turn, keepk, chunk_rsrc(sl.dk + to_k, rows, out_k), lane, out_k);
   }
   next_phase();
   // ---- dq of tile w: over the key tiles J the direction keeps ----
@@ -558,8 +573,8 @@ __device__ __forceinline__ void bwd_direction(const BwdSlab& sl, int L, int ntil
   // the next direction's rows travel while this one finishes
   next_phase();
   if (!kEarlyGates) issue_bwd_gate_loads<NG>(nxt, w, r, h, ld);
-  if (!kEarlyRows) issue_bwd_qk_loads<NG>(nxt, w, r, h, ld);
-  if (LAST) issue_bwd_vdo_loads<NG>(nxt, w, r, h, ld);
+  if (!kEarlyRows) issue_bwd_qk_loads<NG, PITCHED>(nxt, w, r, h, ld);
+  if (LAST) issue_bwd_vdo_loads<NG, PITCHED>(nxt, w, r, h, ld);
   next_phase();
   __builtin_amdgcn_sched_barrier(0);
   if (!LAST) {
@@ -567,11 +582,11 @@ __device__ __forceinline__ void bwd_direction(const BwdSlab& sl, int L, int ntil
     for (int g = 0; g < kParkLds; ++g) *reinterpret_cast<u32x4_t*>(unit_ptr(lds + BwdLds<TW>::park, w * kParkLds + g, lane)) = keepq[g];
   }
   if (LAST || (kParkDq && kParkLds == 0)) {
-    store_rows<NG, TW>(turn, keepq, chunk_rsrc(sl.dq + tk, rows, 2 * DK), lane);
+    store_rows<NG, TW, PITCHED>(turn, keepq, chunk_rsrc(sl.dq + to_k, rows, out_k), lane, out_k);
   } else if (kParkDq) {
 #pragma unroll
     for (int g = kParkLds; g < NG; ++g)
-      __builtin_amdgcn_raw_buffer_store_b128(keepq[g], chunk_rsrc(sl.dq + tk, rows, 2 * DK), r * (32u * NG) + h * (16u * NG) + 16u * g, 0, 0);
+      __builtin_amdgcn_raw_buffer_store_b128(keepq[g], chunk_rsrc(sl.dq + to_k, rows, out_k), r * out_k + h * (16u * NG) + 16u * g, 0, 0);
   }
   // ---- dg: the running sum of X over the tokens the gate acts on.  Inside the tile by lane shifts (lane = token),
   // across tiles through the tile totals in LDS: walking forward a token takes everything from itself to the end,
@@ -641,12 +656,21 @@ struct BwdSegments {
   int nseg, seg_len;
 };
 
-template <int NG, bool BIDIR, bool SEG, int TW>
+// PITCHED: q, k and v are read out of the rows of a stacked projection and dq, dk and dv written into the rows of its gradient, where passes over memory would
+// split and gather them (`BwdPitch`: elements from row to row, heads).  Rows of 64 or 128 bytes either way; the kernel itself takes 1 to 4 % longer.  us, splitting pass,
+// op, its backward and gathering pass / op and backward on rows: Dk 32, 768 sequences of 196 tokens 107 / 85, 384 66 / 55 and 64 / 54 (3 and 12 heads), 48 33 / 29, 384 of
+// 100 37 / 29, 1200 of 49 44 / 33, 240 of 256 48 / 38; Dk 64, 768 of 196 149 / 113, 1800 of 128 202 / 152.
+struct BwdPitch {
+  long long in, out;
+  int H;
+};
+
+template <int NG, bool BIDIR, bool SEG, int TW, bool PITCHED>
 __global__ __launch_bounds__(64 * TW, 2) void gla_backward_mfma_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
     const uint16_t* __restrict__ gf, const uint16_t* __restrict__ gb, const uint16_t* __restrict__ d_o,
     uint16_t* __restrict__ dq, uint16_t* __restrict__ dk, uint16_t* __restrict__ dv, uint16_t* __restrict__ dgf,
-    uint16_t* __restrict__ dgb, int* __restrict__ flags, int nslabs, int L, float s, BwdSegments sg) {
+    uint16_t* __restrict__ dgb, int* __restrict__ flags, int nslabs, int L, float s, BwdSegments sg, BwdPitch rows) {
   extern __shared__ __align__(16) char lds[];
   const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   // slab i: a whole sequence, or (SEG) segment i % nseg of sequence i / nseg
@@ -666,6 +690,14 @@ __global__ __launch_bounds__(64 * TW, 2) void gla_backward_mfma_kernel(
     const size_t bk = t0 * (16 * NG), bv = t0 * 64;
     sl.q = q + bk, sl.k = k + bk, sl.v = v + bv, sl.gf = gf + bk, sl.gb = BIDIR ? gb + bk : nullptr, sl.d_o = d_o + bv;
     sl.dq = dq + bk, sl.dk = dk + bk, sl.dv = dv + bv, sl.dgf = dgf + bk, sl.dgb = BIDIR ? dgb + bk : nullptr;
+    if constexpr (PITCHED) {
+      static_assert(!SEG, "whole sequences");
+      const int b = i / rows.H, head = i - b * rows.H;
+      const size_t from = (size_t)b * L * rows.in, to = (size_t)b * L * rows.out;
+      sl.q = q + from + head * (16 * NG), sl.k = k + from + head * (16 * NG), sl.v = v + from + head * 64;
+      sl.dq = dq + to + head * (16 * NG), sl.dk = dk + to + head * (16 * NG), sl.dv = dv + to + head * 64;
+      sl.in = 2u * (unsigned)rows.in, sl.out = 2u * (unsigned)rows.out;
+    }
     sl.L = len;
     return sl;
   };
@@ -676,8 +708,8 @@ __global__ __launch_bounds__(64 * TW, 2) void gla_backward_mfma_kernel(
     const BwdSlab s0 = slab_of(blockIdx.x);
     const BwdNext first{s0, s0.gf, s0.L};
     issue_bwd_gate_loads<NG>(first, w, r, h, ld);
-    issue_bwd_qk_loads<NG>(first, w, r, h, ld);
-    issue_bwd_vdo_loads<NG>(first, w, r, h, ld);
+    issue_bwd_qk_loads<NG, PITCHED>(first, w, r, h, ld);
+    issue_bwd_vdo_loads<NG, PITCHED>(first, w, r, h, ld);
     bwd_cumulate_gates<true, NG, TW>(ld, w, lane, lds, G);
     lds_barrier();
   }
@@ -693,8 +725,8 @@ __global__ __launch_bounds__(64 * TW, 2) void gla_backward_mfma_kernel(
       const int ln = fresh_lane();
       lds_barrier();  // a wave that has left must not touch the gate totals the others still read
       issue_bwd_gate_loads<NG>(next_first, w, ln & 31, ln >> 5, ld);
-      issue_bwd_qk_loads<NG>(next_first, w, ln & 31, ln >> 5, ld);
-      issue_bwd_vdo_loads<NG>(next_first, w, ln & 31, ln >> 5, ld);
+      issue_bwd_qk_loads<NG, PITCHED>(next_first, w, ln & 31, ln >> 5, ld);
+      issue_bwd_vdo_loads<NG, PITCHED>(next_first, w, ln & 31, ln >> 5, ld);
       bwd_cumulate_gates<true, NG, TW>(ld, w, ln, lds, G);
       lds_barrier();
     };
@@ -702,15 +734,15 @@ __global__ __launch_bounds__(64 * TW, 2) void gla_backward_mfma_kernel(
     if (ok) {
       u32x4_t keepq[NG], keepk[NG];
       if constexpr (BIDIR) {
-        bwd_direction<true, true, false, NG, SEG, TW>(sl, sl.L, ntiles, w, lds, s, dvacc, keepq, keepk, ld, second, G);
+        bwd_direction<true, true, false, NG, SEG, TW, PITCHED>(sl, sl.L, ntiles, w, lds, s, dvacc, keepq, keepk, ld, second, G);
         ok = bwd_anchor<false, NG, TW>(w, lds);
         if (ok) {
-          bwd_direction<false, false, true, NG, SEG, TW>(sl, sl.L, ntiles, w, lds, s, dvacc, keepq, keepk, ld, next_first, G);
+          bwd_direction<false, false, true, NG, SEG, TW, PITCHED>(sl, sl.L, ntiles, w, lds, s, dvacc, keepq, keepk, ld, next_first, G);
         } else {
           skip();  // (in each branch, so that nothing of this slab's loads stays alive for it)
         }
       } else {  // the causal op: the forward direction alone, first and last at once
-        bwd_direction<true, true, true, NG, SEG, TW>(sl, sl.L, ntiles, w, lds, s, dvacc, keepq, keepk, ld, next_first, G);
+        bwd_direction<true, true, true, NG, SEG, TW, PITCHED>(sl, sl.L, ntiles, w, lds, s, dvacc, keepq, keepk, ld, next_first, G);
       }
     } else {
       skip();
@@ -897,20 +929,23 @@ struct BwdLaunch {
   int nslabs, L;
   float s;
   BwdSegments sg;
+  BwdPitch rows;  // (in = 0: head-major tensors)
   int num_cu;
   hipStream_t stream;
 };
-template <int NG, bool BIDIR, bool SEG, int TW>
+template <int NG, bool BIDIR, bool SEG, int TW, bool PITCHED = false>
 static int launch_bwd_t(const BwdLaunch& l) {
+  if constexpr (BIDIR && !SEG && !PITCHED)
+    if (l.rows.in) return launch_bwd_t<NG, BIDIR, SEG, TW, true>(l);
   static bool done[64] = {};
-  auto* kernel = gla_backward_mfma_kernel<NG, BIDIR, SEG, TW>;
+  auto* kernel = gla_backward_mfma_kernel<NG, BIDIR, SEG, TW, PITCHED>;
   static_assert(kBwdTiles / TW * BwdLds<TW>::total <= 160 * 1024, "the workgroups of a CU fit its LDS");
   if (!allow_lds(reinterpret_cast<const void*>(kernel), BwdLds<TW>::total, done)) return -5;
   const int most = l.num_cu * (kBwdTiles / TW);
   hipLaunchKernelGGL(kernel, dim3(l.nslabs < most ? l.nslabs : most), dim3(64 * TW), BwdLds<TW>::total, l.stream,
                      (const uint16_t*)l.q, (const uint16_t*)l.k, (const uint16_t*)l.v, (const uint16_t*)l.gf, (const uint16_t*)l.gb,
                      (const uint16_t*)l.d_o, (uint16_t*)l.dq, (uint16_t*)l.dk, (uint16_t*)l.dv, (uint16_t*)l.dgf, (uint16_t*)l.dgb,
-                     l.flags, l.nslabs, l.L, l.s, l.sg);
+                     l.flags, l.nslabs, l.L, l.s, l.sg, l.rows);
   return hipGetLastError() == hipSuccess ? 0 : -5;
 }
 // Slabs of up to 64 and up to 128 tokens get workgroups of two and four waves, four and two of them to a CU: in one of eight, the
@@ -969,7 +1004,7 @@ static bool short_segments(int B, int H, int L, int Dk) { return Dk == 32 || (lo
 int launch_gla_backward_mfma(const void* q, const void* k, const void* v, const void* gf, const void* gb,
                              const void* d_o, void* dq, void* dk, void* dv, void* dgf, void* dgb, int* flags,
                              void* scratch, size_t scratch_bytes, void* seg_workspace, size_t seg_bytes, int B, int H, int L,
-                             int Dk, float s, hipStream_t stream) {
+                             int Dk, float s, long long ld_in, long long ld_out, hipStream_t stream) {
   constexpr int kMaxDevices = 64;
   static bool attr_done_dev[kMaxDevices] = {};
   static int num_cu_dev[kMaxDevices] = {};
@@ -982,6 +1017,7 @@ int launch_gla_backward_mfma(const void* q, const void* k, const void* v, const 
     attr_done_dev[dev] = true;
   }
   const bool seg = L > 32 * kBwdTiles;
+  if (ld_in && (seg || !gb)) return -95;
   BwdSegments sg{};
   int nslabs = B * H;
   if (seg) {
@@ -1024,7 +1060,7 @@ int launch_gla_backward_mfma(const void* q, const void* k, const void* v, const 
     sg.sp = r.sp, sg.rp = r.rp, sg.rpt = r.rpt, sg.carry = r.carry;
     nslabs = B * H * sg.nseg;
   }
-  const BwdLaunch l{q, k, v, gf, gb, d_o, dq, dk, dv, dgf, dgb, flags, nslabs, L, s, sg, num_cu_dev[dev], stream};
+  const BwdLaunch l{q, k, v, gf, gb, d_o, dq, dk, dv, dgf, dgb, flags, nslabs, L, s, sg, BwdPitch{ld_in, ld_out, H}, num_cu_dev[dev], stream};
   const int tokens = seg ? sg.seg_len : L;
   if (gb) return Dk == 64 ? launch_bwd<4, true>(l, seg, tokens) : launch_bwd<2, true>(l, seg, tokens);
   return Dk == 64 ? launch_bwd<4, false>(l, seg, tokens) : launch_bwd<2, false>(l, seg, tokens);

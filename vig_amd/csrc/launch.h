@@ -150,7 +150,7 @@ size_t gla_backward_mfma_workspace(int B, int H, int L, int Dk, int Dv);
 int launch_gla_backward_mfma(const void* q, const void* k, const void* v, const void* gf, const void* gb,
                              const void* d_o, void* dq, void* dk, void* dv, void* dgf, void* dgb, int* flags,
                              void* scratch, size_t scratch_bytes, void* seg_workspace, size_t seg_bytes, int B, int H, int L,
-                             int Dk, float s, hipStream_t stream);
+                             int Dk, float s, long long ld_in, long long ld_out, hipStream_t stream);
 
 // allows a kernel its LDS, once per device (concurrent first calls only repeat an idempotent setting)
 inline bool allow_lds(const void* kernel, size_t bytes, bool (&done)[64]) {

@@ -13,7 +13,7 @@
 //   - weight and bias gradients leave vig_linear_bwd_weight_many as fp32, a node's layers together;
 //   - the up-projection of the gates and its input gradient run inside the gate kernels (bf16), and the depthwise
 //     convolution's three gradients are one kernel.
-// ViG-S, B 128 at 224 px under bf16 autocast, forward and backward on one MI355X: 23.7 -> 11.0 ms.
+// ViG-S, B 128 at 224 px under bf16 autocast, forward and backward on one MI355X: 23.7 -> 9.9 ms.
 #include <ATen/autocast_mode.h>
 
 #include <torch/csrc/autograd/autograd.h>
@@ -41,6 +41,9 @@ struct Mix {
     m.n0 = 2 * m.K + m.V, m.n1 = m.n0 + m.V, m.n2 = m.n1 + kRank, m.nz = (m.n2 + 127) / 128 * 128;
     return m;
   }
+  // whether the op reads q, k and v out of the projection's rows and writes their gradients into those of its gradient: wherever its kernels can, the passes
+  // that split and gather them cost more at any size (gla_backward_mfma.hip)
+  bool in_place() const { return bf16 && Dv == 64 && Dk >= 32 && L <= 256 && nz <= (1 << 20); }
   at::ScalarType type() const { return bf16 ? at::kBFloat16 : at::kFloat; }
   int code() const { return bf16 ? VIG_BF16 : VIG_F32; }
 };
@@ -301,10 +304,13 @@ struct MixNode : torch::autograd::Function<MixNode> {
                                    m.act ? pre.data_ptr() : nullptr, (int)m.B, (int)m.h, (int)m.w, (int)m.C, m.act, m.code(), stream),
              "vig_dwconv3x3_fwd_pre");
     const Tensor z = product(xs.view({m.rows, m.C}), w_in, b_in);
-    Tensor q = at::empty({m.B, m.H, m.L, m.Dk}, opts), k = at::empty_like(q), v = at::empty({m.B, m.H, m.L, m.Dv}, opts);
-    check_rc(vig_split_heads_fwd(z.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), (int)m.B, (int)m.L, (int)m.H, (int)m.Dk,
-                                 (int)m.Dv, m.nz, m.code(), stream),
-             "vig_split_heads_fwd");
+    Tensor q, k, v;  // head-major copies, where the op does not take its operands out of z
+    if (!m.in_place()) {
+      q = at::empty({m.B, m.H, m.L, m.Dk}, opts), k = at::empty_like(q), v = at::empty({m.B, m.H, m.L, m.Dv}, opts);
+      check_rc(vig_split_heads_fwd(z.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), (int)m.B, (int)m.L, (int)m.H, (int)m.Dk,
+                                   (int)m.Dv, m.nz, m.code(), stream),
+               "vig_split_heads_fwd");
+    }
     Tensor gates = at::empty({2 * m.B, m.H, m.L, m.Dk}, opts), gate_lin;
     if (m.bf16) {
       check_rc(vig_dirgate_lowrank_fwd(at_elem(z, m.n1), m.nz, same ? up_w.data_ptr() : at_elem(packed, up_off),
@@ -319,7 +325,15 @@ struct MixNode : torch::autograd::Function<MixNode> {
     }
     Call c{(int)m.B, (int)m.H, (int)m.L, (int)m.Dk, (int)m.Dv, m.code(), m.code(), (float)std::pow((double)m.Dk, -0.5), 0.5f};
     Tensor o;
-    check_rc(run_forward(q, k, v, gates, Tensor(), true, kDefault, c, o), "vig_gla_bidir_fwd");
+    if (m.in_place()) {
+      o = at::empty({m.B, m.H, m.L, m.Dv}, opts);
+      const long long sk[3] = {m.L * m.nz, m.Dk, m.nz}, sv[3] = {m.L * m.nz, m.Dv, m.nz};
+      check_rc(vig_gla_bidir_fwd_strided(z.data_ptr(), at_elem(z, m.K), at_elem(z, 2 * m.K), gates.data_ptr(), at_elem(gates, gates.numel() / 2),
+                                         o.data_ptr(), c.B, c.H, c.L, c.Dk, c.Dv, sk, sk, sv, c.scale, c.out_scale, c.io, c.gd, stream),
+               "vig_gla_bidir_fwd_strided");
+    } else {
+      check_rc(run_forward(q, k, v, gates, Tensor(), true, kDefault, c, o), "vig_gla_bidir_fwd");
+    }
     Tensor blend = at::empty_like(xs);
     Tensor a;
     // At any number of tokens (us, fused / blend and product): C 192: 49 4.8 / 10.7, 1568 5.3 / 12.4, 25088 16 / 29; C 384: 49 7.7 / 11.2,
@@ -388,8 +402,18 @@ struct MixNode : torch::autograd::Function<MixNode> {
                                               (float)m.eps, m.out_act, m.code(), &sums.jobs, stream),
                "vig_locality_blend_bwd_strided");
     }
-    Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v), dg = at::empty_like(gates);
-    {
+    Tensor dg = at::empty_like(gates);
+    if (m.in_place()) {
+      const size_t need = vig_gla_bidir_bwd_workspace_for((int)m.B, (int)m.H, (int)m.L, (int)m.Dk, (int)m.Dv, m.code(), m.code(), 1);
+      Tensor ws = bytes_like(need, sum);
+      const int64_t half = gates.numel() / 2;
+      check_rc(vig_gla_bidir_bwd_rows(z.data_ptr(), at_elem(z, m.K), at_elem(z, 2 * m.K), m.nz, gates.data_ptr(), at_elem(gates, half),
+                                      d_o.data_ptr(), dz.data_ptr(), at_elem(dz, m.K), at_elem(dz, 2 * m.K), m.nz, dg.data_ptr(),
+                                      at_elem(dg, half), ws.data_ptr(), need, (int)m.B, (int)m.H, (int)m.L, (int)m.Dk, (int)m.Dv,
+                                      (float)std::pow((double)m.Dk, -0.5), 0.5f, m.code(), m.code(), stream),
+               "vig_gla_bidir_bwd_rows");
+    } else {
+      Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
       const size_t need = vig_gla_bidir_bwd_workspace_for((int)m.B, (int)m.H, (int)m.L, (int)m.Dk, (int)m.Dv, m.code(), m.code(), 1);
       Tensor ws = bytes_like(need, sum);
       const int64_t half = gates.numel() / 2;
@@ -398,10 +422,10 @@ struct MixNode : torch::autograd::Function<MixNode> {
                                  (int)m.B, (int)m.H, (int)m.L, (int)m.Dk, (int)m.Dv, (float)std::pow((double)m.Dk, -0.5), 0.5f,
                                  m.code(), m.code(), stream),
                "vig_gla_bidir_bwd");
+      check_rc(vig_split_heads_bwd_strided(dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dz.data_ptr(), m.nz, (int)m.B, (int)m.L,
+                                           (int)m.H, (int)m.Dk, (int)m.Dv, m.code(), stream),
+               "vig_split_heads_bwd_strided");
     }
-    check_rc(vig_split_heads_bwd_strided(dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dz.data_ptr(), m.nz, (int)m.B, (int)m.L,
-                                         (int)m.H, (int)m.Dk, (int)m.Dv, m.code(), stream),
-             "vig_split_heads_bwd_strided");
     Tensor dx = at::empty({m.rows, 2 * m.K}, opts);
     if (m.bf16) {
       check_rc(vig_dirgate_lowrank_bwd(at_elem(z, m.n1), m.nz, same ? up_w.data_ptr() : at_elem(packed, off[2]),
