@@ -112,7 +112,7 @@ int vig_gla_bidir_fwd_strided(const void* q, const void* k, const void* v,
 int vig_gla_slab_tokens(int Dk);
 
 /*
- * The one-launch kernel behind vig_gla_bidir_fwd, _strided and vig_gla_bidir_locgate_fwd at every length it takes
+ * The kernel behind vig_gla_bidir_fwd, _strided and vig_gla_bidir_locgate_fwd at every length one launch takes
  * (L <= vig_gla_slab_tokens(Dk); those two stop at 256): strides as for _strided, each NULL for a plain tensor; with
  * gate_weight [H*Dv, 3, 3] f32 (NULL: none) the locality gate of vig_gla_bidir_locgate_fwd on a grid_h x grid_w token grid
  * (both directions, plain tensors, grid_w <= 126, a grid whose padded rows fit LDS).  VIG_ENOTSUP for anything else.  No workspace.
@@ -393,9 +393,10 @@ int vig_locality_gate_fwd(const void* o, const float* weight, void* y,
                           int B, int H, int h, int w, int Dv, int io_dtype, void* stream);
 
 /*
- * vig_gla_bidir_fwd and vig_locality_gate_fwd in one kernel: the GLA output o = out_scale * (o_fwd + o_bwd) is
+ * vig_gla_bidir_fwd and vig_locality_gate_fwd in one call: the GLA output o = out_scale * (o_fwd + o_bwd) is
  * rounded to bf16, staged on chip, and y = o * sigmoid(dwconv3x3(o)) is what reaches memory (bit-identical to the
- * two calls in a row).  Same tensors as vig_gla_bidir_fwd; weight [H*Dv, 3, 3] f32; L = grid_h * grid_w.
+ * two calls in a row); of few sequences of 129 to 256 tokens, which the op spreads over the chip, the op's output does, and a second
+ * launch gates it in place.  Same tensors as vig_gla_bidir_fwd; weight [H*Dv, 3, 3] f32; L = grid_h * grid_w.
  * Built for bf16 tensors and gates, Dk in {32, 64}, Dv = 64, L <= 256, both directions, and token grids with
  * grid_w <= 62 and grid_h + 2 <= 8 * floor(64 / (grid_w + 2)) (14x14 and 16x16 are); VIG_ENOTSUP otherwise
  * (the caller then makes the two calls).  No workspace.

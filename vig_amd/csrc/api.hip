@@ -405,7 +405,7 @@ int vig_gla_bidir_fwd_noalloc(const void* q, const void* k, const void* v, const
 }
 
 // vig_gla_bidir_fwd followed by vig_locality_gate_fwd in one kernel: y = o * sigmoid(conv3x3(o)) with o the rounded
-// GLA output, never written to memory.  Only shapes of the bf16 MFMA path with the whole sequence in one slab.
+// GLA output, never written to memory (but for few sequences: gla_tiles.hip, spread_gate_kernel).  Only shapes of the bf16 MFMA path with the whole sequence in one slab.
 int vig_gla_bidir_locgate_fwd(const void* q, const void* k, const void* v, const void* g_fwd, const void* g_bwd,
                               const float* gate_weight, void* y, int B, int H, int L, int Dk, int Dv, int grid_h,
                               int grid_w, float scale, float out_scale, int io_dtype, int gate_dtype, void* stream) {

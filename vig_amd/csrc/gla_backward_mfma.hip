@@ -666,11 +666,11 @@ struct BwdPitch {
 };
 
 template <int NG, bool BIDIR, bool SEG, int TW, bool PITCHED>
-__global__ __launch_bounds__(64 * TW, 2) void gla_backward_mfma_kernel(
+__device__ __forceinline__ void gla_backward_slabs(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
     const uint16_t* __restrict__ gf, const uint16_t* __restrict__ gb, const uint16_t* __restrict__ d_o,
     uint16_t* __restrict__ dq, uint16_t* __restrict__ dk, uint16_t* __restrict__ dv, uint16_t* __restrict__ dgf,
-    uint16_t* __restrict__ dgb, int* __restrict__ flags, int nslabs, int L, float s, BwdSegments sg, BwdPitch rows) {
+    uint16_t* __restrict__ dgb, int* __restrict__ flags, int nslabs, int L, float s, const BwdSegments& sg, const BwdPitch& rows) {
   extern __shared__ __align__(16) char lds[];
   const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   // slab i: a whole sequence, or (SEG) segment i % nseg of sequence i / nseg
@@ -752,6 +752,23 @@ __global__ __launch_bounds__(64 * TW, 2) void gla_backward_mfma_kernel(
       else if (!ok) flags[slab / sg.nseg] = 1;  // one flag per sequence, cleared by the segment scan: any segment out of range gives it away
     }
   }
+}
+
+template <int NG, bool BIDIR, bool SEG, int TW>
+__global__ __launch_bounds__(64 * TW, 2) void gla_backward_mfma_kernel(
+    const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
+    const uint16_t* __restrict__ gf, const uint16_t* __restrict__ gb, const uint16_t* __restrict__ d_o,
+    uint16_t* __restrict__ dq, uint16_t* __restrict__ dk, uint16_t* __restrict__ dv, uint16_t* __restrict__ dgf,
+    uint16_t* __restrict__ dgb, int* __restrict__ flags, int nslabs, int L, float s, BwdSegments sg) {
+  gla_backward_slabs<NG, BIDIR, SEG, TW, false>(q, k, v, gf, gb, d_o, dq, dk, dv, dgf, dgb, flags, nslabs, L, s, sg, BwdPitch{});
+}
+template <int NG, int TW>
+__global__ __launch_bounds__(64 * TW, 2) void gla_backward_rows_kernel(
+    const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
+    const uint16_t* __restrict__ gf, const uint16_t* __restrict__ gb, const uint16_t* __restrict__ d_o,
+    uint16_t* __restrict__ dq, uint16_t* __restrict__ dk, uint16_t* __restrict__ dv, uint16_t* __restrict__ dgf,
+    uint16_t* __restrict__ dgb, int* __restrict__ flags, int nslabs, int L, float s, BwdPitch rows) {
+  gla_backward_slabs<NG, true, false, TW, true>(q, k, v, gf, gb, d_o, dq, dk, dv, dgf, dgb, flags, nslabs, L, s, BwdSegments{}, rows);
 }
 
 // Links the segments of every (sequence, direction) for the backward.  Per segment s (walked in the direction's order)
@@ -933,20 +950,24 @@ struct BwdLaunch {
   int num_cu;
   hipStream_t stream;
 };
-template <int NG, bool BIDIR, bool SEG, int TW, bool PITCHED = false>
+template <int NG, bool BIDIR, bool SEG, int TW>
 static int launch_bwd_t(const BwdLaunch& l) {
-  if constexpr (BIDIR && !SEG && !PITCHED)
-    if (l.rows.in) return launch_bwd_t<NG, BIDIR, SEG, TW, true>(l);
-  static bool done[64] = {};
-  auto* kernel = gla_backward_mfma_kernel<NG, BIDIR, SEG, TW, PITCHED>;
   static_assert(kBwdTiles / TW * BwdLds<TW>::total <= 160 * 1024, "the workgroups of a CU fit its LDS");
-  if (!allow_lds(reinterpret_cast<const void*>(kernel), BwdLds<TW>::total, done)) return -5;
   const int most = l.num_cu * (kBwdTiles / TW);
-  hipLaunchKernelGGL(kernel, dim3(l.nslabs < most ? l.nslabs : most), dim3(64 * TW), BwdLds<TW>::total, l.stream,
-                     (const uint16_t*)l.q, (const uint16_t*)l.k, (const uint16_t*)l.v, (const uint16_t*)l.gf, (const uint16_t*)l.gb,
-                     (const uint16_t*)l.d_o, (uint16_t*)l.dq, (uint16_t*)l.dk, (uint16_t*)l.dv, (uint16_t*)l.dgf, (uint16_t*)l.dgb,
-                     l.flags, l.nslabs, l.L, l.s, l.sg, l.rows);
-  return hipGetLastError() == hipSuccess ? 0 : -5;
+  const auto launch = [&](auto* kernel, bool (&done)[64], const auto& last) {
+    if (!allow_lds(reinterpret_cast<const void*>(kernel), BwdLds<TW>::total, done)) return -5;
+    hipLaunchKernelGGL(kernel, dim3(l.nslabs < most ? l.nslabs : most), dim3(64 * TW), BwdLds<TW>::total, l.stream,
+                       (const uint16_t*)l.q, (const uint16_t*)l.k, (const uint16_t*)l.v, (const uint16_t*)l.gf, (const uint16_t*)l.gb,
+                       (const uint16_t*)l.d_o, (uint16_t*)l.dq, (uint16_t*)l.dk, (uint16_t*)l.dv, (uint16_t*)l.dgf, (uint16_t*)l.dgb,
+                       l.flags, l.nslabs, l.L, l.s, last);
+    return hipGetLastError() == hipSuccess ? 0 : -5;
+  };
+  if constexpr (BIDIR && !SEG) {
+    static bool done_rows[64] = {};
+    if (l.rows.in) return launch(gla_backward_rows_kernel<NG, TW>, done_rows, l.rows);
+  }
+  static bool done[64] = {};
+  return launch(gla_backward_mfma_kernel<NG, BIDIR, SEG, TW>, done, l.sg);
 }
 // Slabs of up to 64 and up to 128 tokens get workgroups of two and four waves, four and two of them to a CU: in one of eight, the
 // waves without a tile idle and nothing runs beside the loads.  us, eight waves / as many as the slab has tiles (dword operands): Dk 64:

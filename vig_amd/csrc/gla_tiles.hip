@@ -1,5 +1,6 @@
 // Bidirectional GLA forward on MFMA tiles (gfx950), Dk in {32, 64}, Dv = 64, bf16 in and out: one workgroup per
 // (batch, head) slab of up to 512 tokens (Dk 64: 416), one wave per 32-token query tile, both directions in the same wave.
+// Few sequences of five to eight tiles, both directions, get a workgroup for each query tile instead (gla_spread_kernel).
 // A longer sequence is cut into segments of at most seven tiles, each handled like a slab plus the products with the states
 // that enter it from either side (apply_state; the states come from a state pass and a scan, gla_mfma.hip).
 //

@@ -572,8 +572,8 @@ def gla_bidir_locality_gate(q, k, v, g_fwd, g_bwd, weight: torch.Tensor, hw, sca
     """locality_gate(gla_bidir_forward(q, k, v, g_fwd, g_bwd), weight, hw), bit for bit.
 
     Shapes the one-kernel form is built for (bf16, Dk in {32,64}, Dv=64, L=h*w up to 512 at Dk 32 and 416 at Dk 64, a
-    grid whose padded rows fit LDS) never write the ungated output to memory; every other shape makes the two calls (and
-    without the native module every L past 256).  Inference only.
+    grid whose padded rows fit LDS) never write the ungated output to memory, few sequences of 129 to 256 tokens apart, whose
+    gate is a launch in place behind the op; every other shape makes the two calls (and without the native module every L past 256).  Inference only.
     """
     h, w = hw
     calls = _ext.calls()
