@@ -53,7 +53,7 @@ __device__ __forceinline__ float octet_tree(const float* row) {
 
 // NORM: the workgroup has whole rows of channels, so their norm needs two exchanges of octet sums through LDS (a barrier each, one of
 // which takes the place of the one in front of the next staging) instead of a pass over memory.  us, two kernels / this: 96 channels, one image of
-// 224 px 8.5 / 6.7, 8 9.6 / 6.9, 256 74 / 54, 8 of 1024 px 50 / 35; 192, 1 9.4 / 7.9, 32 28 / 22, 64 37 / 32, 256 99.6 / 97.2 (one workgroup to a CU: its 191
+// 224 px 8.5 / 6.7, 8 9.6 / 6.9, 256 74 / 54, 8 of 1024 px 50 / 35; 192, 1 9.4 / 7.9, 32 25 / 19, 64 34 / 29, 256 96 / 94 (one workgroup to a CU: its 191
 // registers brought down to 168 for a second one spill 13 to 18, 124).  At 384 channels the 48 octets spill (60 images 55 / 73): two kernels.
 template <int KS, int NW, bool NORM>  // KS = Cin * KH contraction steps, NW = Cout / 32 waves
 __global__ __launch_bounds__(NW > 8 ? 64 * NW : 512) void patch_conv_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ wp,
@@ -198,7 +198,7 @@ bool patch_conv_supported(int Cin, int H, int W, int KH, int KW, int stride, int
   if (stride != kPcStride || padding != 1 || KW < 1 || KW > kPcKW || Cin * KH != 27) return false;
   if (W % 8 != 0 || H < 1 || (W > 248 && KW > 9)) return false;  // (a piece holds nine columns of its last pixel)
   const int OW = (W + 2 - KW) / stride + 1;
-  // (twelve waves, one workgroup a CU: 384 channels, 224 px, 1 image 12.4 us, 32 24.9, where the library took 39.7 for 32 and 21 beside it)
+  // (twelve waves, one workgroup a CU: 384 channels, 224 px, 1 image 12.4 us, 40 21.3, where the library took 39.7 for 32 and 21 beside it)
   return OW >= 1 && Cout % 32 == 0 && ((Cout >= 64 && Cout <= 256) || Cout == 384);
 }
 
@@ -209,7 +209,10 @@ static int launch(const void* x, const void* w_packed, void* y, int B, int Cin, 
   const int pieces = (OW + 31) / 32;
   if (OH < 1 || (long long)B * OH * pieces > 0x7fffffffLL - 4096 || Cout / 32 < 2) return -95;
   const int nitems = B * OH * pieces;
-  const int grid = nitems < 512 ? nitems : 512;  // two workgroups a CU; each walks pieces grid apart
+  // As many workgroups as the chip holds, two to a CU of up to four waves and one of more; each walks pieces grid apart.  (A second one of more waves runs
+  // behind the first and fetches the weights again; us, two to a CU / one: 192 channels, 16 images of 224 px 12.4 / 9.1, 32 16.5 / 13.5, 256 61 / 57.5, with the
+  // norm 97.7 / 94.2; 256 channels, 20 15.4 / 11.7; 384, 16 18.9 / 13.4, 128 50.8 / 42.5.)
+  const int most = Cout > 128 ? 256 : 512, grid = nitems < most ? nitems : most;
   const size_t lds = (size_t)27 * kPcRowElems * sizeof(uint16_t) + (norm ? 4 * (2 * 32 * (Cout / 8 + 4) + 3 * Cout) : 0);
 #define VIG_PC_CASE(NW)                                                                                            \
   case NW:                                                                                                         \
