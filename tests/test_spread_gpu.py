@@ -88,14 +88,18 @@ def test_gates_made_inside(B, H, L):
     assert torch.equal(o.float(), _run(lib.vig_gla_bidir_fwd, q, k, v, g))  # the same operands, one form
 
 
-def test_one_sequence_in_a_batch():
-    """A sequence's outputs as a workgroup a query tile gives them and as a workgroup a sequence does."""
-    q, k, v, g = _inputs(1, 2, 196, 64, torch.Generator().manual_seed(9))
-    one = vig_amd.batch_bid_fused_chunk_gla(q, k, v, g.flatten(0, 1))[0].float()
+@pytest.mark.parametrize("L,Dk,keys", [(129, 32, 1.0), (160, 64, 1.0), (196, 32, 1.0), (197, 64, 1.0), (225, 32, 1.0), (256, 64, 1.0), (256, 32, 30.0), (196, 32, 1e-3),
+                                       (196, 32, 1e-4), (256, 64, 3e-4)])
+def test_one_sequence_in_a_batch(L, Dk, keys):
+    """A sequence's outputs as a workgroup a query tile gives them and as a workgroup a sequence does: the same bits, keys in fp16's subnormals
+    once decayed among them."""
+    announce(f"spread forward, one sequence and sixty L{L} Dk{Dk} keys x {keys}")
+    q, k, v, g = _inputs(1, 2, L, Dk, torch.Generator().manual_seed(9))
+    k = k * keys
+    one = vig_amd.batch_bid_fused_chunk_gla(q, k, v, g.flatten(0, 1))[0]
     many = [t.repeat(30, 1, 1, 1) for t in (q, k, v)]
-    batch = vig_amd.batch_bid_fused_chunk_gla(*many, g.repeat_interleave(30, 1).flatten(0, 1))[0].float()
-    assert torch.equal(batch[0], batch[29])
-    _close(one[0], batch[0])
+    batch = vig_amd.batch_bid_fused_chunk_gla(*many, g.repeat_interleave(30, 1).flatten(0, 1))[0]
+    assert torch.equal(batch[0], batch[29]) and torch.equal(one[0], batch[0])
 
 
 @pytest.mark.parametrize("B,H,hw,Dk", [(1, 3, (14, 14), 32), (2, 2, (2, 126), 64), (1, 2, (256, 1), 32), (3, 1, (11, 12), 64)])

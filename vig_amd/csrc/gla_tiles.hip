@@ -985,23 +985,30 @@ __global__ __launch_bounds__(512, 2) void gla_tile_wide_kernel(const uint16_t* _
 // for is its own CU: of 14.7 thousand clocks at seven tiles, Dk 32, 2.3 go by until the rows are there, 7 until every wave has prepared
 // its tile in both directions (two waves to a SIMD), 3.5 for six steps of the walk, whose operands are 6 KB of LDS a wave and step.
 // Here wave j has key tile j against the workgroup's one query tile i: one direction (forward before i, reverse behind it), keys alone, in
-// registers from the load to the product, no walk; the tile's own pairs are wave i's (forward) and one wave's more (reverse).
-//   1. cumulative gates and totals of the wave's tile and direction; totals to LDS, barrier
-//   2. key waves: k^ = k exp(T + totals of the tiles between - G), rounded once; query waves: q^ to LDS and their half of the diagonal; barrier
-//   3. key waves: P = k^ q^, O = V^T P; every wave leaves its 32 x 64 partial sums in LDS, barrier, the workgroup adds them up and stores.
-// Keys, values and gates are read by every workgroup of the sequence, out of the L2.  us, workgroup a sequence / this: 3
-// sequences of 49 tokens, Dk 32 4.2 / 3.8, of 100 5.0 / 4.4, of 196 7.2 / 5.0, of 256 7.6 / 5.5; Dk 64, of 196 9.5 / 6.3, of 256 10.3 / 6.9.
+// registers from the load to the product; the tile's own pairs are wave i's (forward) and one wave's more (reverse), the query waves.
+//   1. gates, operands, values and decays as in prepare_direction, each wave for its tile and direction; query waves: q^ and their half of
+//      the diagonal's scores; all but k^ to LDS, barrier
+//   2. key waves: q^ takes the decays of the tiles between, nearest first, as on the walk; P = k^ q^, rounded, to LDS; barrier
+//   3. query waves, one for each half of the value channels: the walk's chain of value products, diagonal first, then outwards, forward
+//      before reverse; the halves meet in LDS, wave i stores.
+// Every rounding and every sum is the walk's, so inside the fp16 form's range a sequence has the same bits in a call of any size.  (Keys that
+// take all decays between at once, and partial sums of each key tile added up by the workgroup, are 2 to 8 % quicker, but round
+// otherwise and lose more of small keys to fp16's subnormals: 256 tokens, Dk 64, keys of rms 3.7e-5, error 9.5e-4 of the rms against 7.0e-4.)
+// Keys, values and gates are read by every workgroup of the sequence, out of the L2.  us on the device, workgroup a sequence / this: 3
+// sequences of 129 tokens, Dk 32 6.1 / 4.6, of 196 7.1 / 5.0, of 256 7.5 / 5.6; Dk 64, of 129 8.0 / 5.8, of 196 9.4 / 6.3, of 256 10.2 / 7.3.
 // Outside the fp16 form's range a workgroup runs the general form of the whole sequence and stores its own tile of it.
 // ---------------------------------------------------------------------------
 template <int NG>
 struct SpreadLds {
-  static constexpr int kQuery = NG * 1024;  // q^ of one direction
-  int totals, scratch, part, guard, total;
+  static constexpr int kQuery = NG * 1024;  // q^ of one direction; later the second half of the sums
+  static_assert(2 * kQuery >= 4096, "the second query wave's sums");
+  int scratch, d, v, p, guard, total;
   __host__ __device__ explicit SpreadLds(int NT) {
-    totals = 2 * kQuery;
-    scratch = totals + (NT + 1) * 256;
-    part = scratch + (NT + 1) * 256;
-    guard = part + (NT + 1) * 8192;
+    scratch = 2 * kQuery;
+    d = scratch + (NT + 1) * 256;
+    v = d + (NT + 1) * 128;
+    p = v + NT * 4096;
+    guard = p + (NT + 1) * 2048;
     const int general = TileLds<NG>(NT, 0, false).total;  // (whose waves may write while others still read the guard)
     if (guard < general) guard = general;
     total = guard + 64;
@@ -1046,7 +1053,8 @@ __global__ __launch_bounds__(576, 3) void gla_spread_kernel(const uint16_t* __re
   else issue_tdwords<0, 2, 4>(cx.v, r, h, vD);
   // ---- 1: cumulative gates G[p][4g+m] = channel 8*NG*h + 8g + 2m + p of token r; totals ----
   const uint32_t keep = (fwd ? (2u << r) - 1u : 0xFFFFFFFFu << r) >> (4 * h);
-  float* const totals = reinterpret_cast<float*>(lds + lay.totals);
+  float* const sc = reinterpret_cast<float*>(lds + lay.scratch) + 64 * wave;
+  _Float16* const decays = reinterpret_cast<_Float16*>(lds + lay.d + 128 * wave);
   f32x16_t G[2];
   {
     const u32x4_t tri0 = keep_masks<0>(keep) & 0x3F803F80u, tri1 = keep_masks<1>(keep) & 0x3F803F80u;
@@ -1073,7 +1081,6 @@ __global__ __launch_bounds__(576, 3) void gla_spread_kernel(const uint16_t* __re
   }
   const auto gates = [&](int p, int c) { return LOW ? G[0][8 * p + c] : G[p][c]; };
   {
-    float* const sc = totals + 64 * wave;
     if constexpr (LOW) asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 3" : "+v"(G[0]));  // (as in park_totals)
     else asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 3" : "+v"(G[0]), "+v"(G[1]));
     if (r == (fwd ? 31 : 0)) {
@@ -1104,7 +1111,11 @@ __global__ __launch_bounds__(576, 3) void gla_spread_kernel(const uint16_t* __re
     const float mq = fmaxf(fmaxf(fabsf(gq[0]), fabsf(gq[1])), fmaxf(fabsf(gq[2]), fabsf(gq[3])));
     const float mk = fmaxf(fmaxf(fabsf(gk[0]), fabsf(gk[1])), fmaxf(fabsf(gk[2]), fabsf(gk[3])));
     const float mv = fmaxf(fmaxf(fabsf(gv[0]), fabsf(gv[1])), fmaxf(fabsf(gv[2]), fabsf(gv[3])));
-    const float tl = totals[64 * wave + lane] * kLog2e;
+    const float tl = sc[lane] * kLog2e;
+    {
+      const int p = (lane >> 4) & 1, g = (lane >> 2) & 3, m = lane & 3;
+      if (g < NG) decays[8 * NG * (lane >> 5) + 8 * g + 2 * m + p] = (_Float16)exp2_fast(tl);
+    }
     const bool veto = __builtin_amdgcn_ballot_w64(!(mq < kMaxSquaresQ) || !(mk < kMaxSquaresK) || !(mv < kMaxSquaresV) || !(fabsf(tl) <= kTileRange)) != 0;
     if (lane == 0) guard[wave] = veto ? 1.0f : 0.0f;
 #pragma unroll
@@ -1121,7 +1132,46 @@ __global__ __launch_bounds__(576, 3) void gla_spread_kernel(const uint16_t* __re
         rawk[g][m] = pack_f16x2(bf16lo_to_f32(rawk[g][m]), bf16hi_to_f32(rawk[g][m]));
       }
   }
-  lds_barrier();  // the totals are visible
+  char* const values = lds + lay.v;
+  char* const scores = lds + lay.p;
+  if (wave < NT) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int p = 0; p < 2; ++p) *reinterpret_cast<u32x4_t*>(unit_ptr(values, 4 * wave + 2 * t + p, lane)) = vf[t][p];
+  }
+  wave_lds_sync();
+  // ---- operands; the diagonal ----
+  u32x4_t kc[NG], p16[2];  // k' = k exp(-G), then k^
+  char* const qreg = lds + (fwd ? 0 : SpreadLds<NG>::kQuery);
+#pragma unroll
+  for (int g = 0; g < NG; ++g) {
+    const u32x4_t d16 = reinterpret_cast<const u32x4_t*>(decays + 8 * NG * h)[g];
+    u32x4_t qh;
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      const float x0 = gates(0, 4 * g + m) * kLog2e, x1 = gates(1, 4 * g + m) * kLog2e;
+      kc[g][m] = mul_f16x2(rawk[g][m], pack_f16x2(exp2_fast(-x0), exp2_fast(-x1)));
+      if (query) qh[m] = mul_f16x2(rawq[g][m], pack_f16x2(exp2_fast(x0), exp2_fast(x1)));
+      else kc[g][m] = mul_f16x2(kc[g][m], d16[m]);
+    }
+    if (query) {
+      *reinterpret_cast<u32x4_t*>(unit_ptr(qreg, g, lane)) = qh;
+      rawq[g] = qh;
+    }
+  }
+  const auto leave_scores = [&](const f32x16_t& P, const u32x4_t& m0, const u32x4_t& m1) {
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+      const int c = 4 * (x >> 1) + 2 * (x & 1);
+      p16[0][x] = pack_f16x2(P[c], P[c + 1]) & m0[x];
+      p16[1][x] = pack_f16x2(P[8 + c], P[8 + c + 1]) & m1[x];
+    }
+#pragma unroll
+    for (int t = 0; t < 2; ++t) *reinterpret_cast<u32x4_t*>(unit_ptr(scores, 2 * wave + t, lane)) = p16[t];
+  };
+  if (query) leave_scores(score_tile16<NG>(kc, rawq), keep_masks<0>(keep), keep_masks<1>(keep));
+  lds_barrier();  // values, decays, q^ and the diagonal are visible
   {
     const float mine = lane <= NT ? guard[lane] : 0.0f;
     if (__builtin_amdgcn_ballot_w64(mine != 0.0f) != 0) {
@@ -1130,69 +1180,75 @@ __global__ __launch_bounds__(576, 3) void gla_spread_kernel(const uint16_t* __re
     }
   }
   // ---- 2 ----
-  f32x16_t O[2] = {f32x16_t{0.f}, f32x16_t{0.f}};
-  u32x4_t kf[NG];
-  char* const qreg = lds + (fwd ? 0 : SpreadLds<NG>::kQuery);
-  if (query) {
-    u32x4_t qh[NG];
-#pragma unroll
-    for (int g = 0; g < NG; ++g) {
-#pragma unroll
-      for (int m = 0; m < 4; ++m) {
-        const float x0 = gates(0, 4 * g + m) * kLog2e, x1 = gates(1, 4 * g + m) * kLog2e;
-        qh[g][m] = mul_f16x2(rawq[g][m], pack_f16x2(exp2_fast(x0), exp2_fast(x1)));
-        kf[g][m] = mul_f16x2(rawk[g][m], pack_f16x2(exp2_fast(-x0), exp2_fast(-x1)));  // k' = k exp(-G)
-      }
-      *reinterpret_cast<u32x4_t*>(unit_ptr(qreg, g, lane)) = qh[g];
-    }
-    const f32x16_t P = score_tile16<NG>(kf, qh);
-    const u32x4_t m0 = keep_masks<0>(keep), m1 = keep_masks<1>(keep);
-    u32x4_t p16[2];
-#pragma unroll
-    for (int x = 0; x < 4; ++x) {
-      const int c = 4 * (x >> 1) + 2 * (x & 1);
-      p16[0][x] = pack_f16x2(P[c], P[c + 1]) & m0[x];
-      p16[1][x] = pack_f16x2(P[8 + c], P[8 + c + 1]) & m1[x];
-    }
-    apply_values16(p16, vf, O);
-  } else {
-    float sum = 0.f;
-    const int near = fwd ? wave : qi + 1, far = fwd ? qi - 1 : wave;  // the wave's own tile and those between
-    for (int t = near; t <= far; ++t) sum += totals[64 * t + lane];
-    float* const sc = reinterpret_cast<float*>(lds + lay.scratch) + 64 * wave;
-    sc[lane] = sum * kLog2e;
-    wave_lds_sync();
-#pragma unroll
-    for (int g = 0; g < NG; ++g) {
-      const f32x4_t d0 = *reinterpret_cast<const f32x4_t*>(sc + 32 * h + 4 * g), d1 = *reinterpret_cast<const f32x4_t*>(sc + 32 * h + 16 + 4 * g);
-#pragma unroll
-      for (int m = 0; m < 4; ++m) {
-        const float x0 = gates(0, 4 * g + m) * kLog2e, x1 = gates(1, 4 * g + m) * kLog2e;
-        kf[g][m] = mul_f16x2(rawk[g][m], pack_f16x2(exp2_fast(d0[m] - x0), exp2_fast(d1[m] - x1)));
-      }
-    }
-  }
-  lds_barrier();  // q^ of both directions is visible
-  // ---- 3 ----
   if (!query) {
     u32x4_t qh[NG];
 #pragma unroll
     for (int g = 0; g < NG; ++g) qh[g] = *reinterpret_cast<const u32x4_t*>(unit_ptr(qreg, g, lane));
-    apply_values(score_tile16<NG>(kf, qh), vf, O);
+    const int between = fwd ? qi - 1 - wave : wave - qi - 1;
+    for (int s = 1; s <= between; ++s) {
+      const u32x4_t* const d = reinterpret_cast<const u32x4_t*>(lds + lay.d + 128 * (fwd ? qi - s : qi + s) + 16 * NG * h);
+#pragma unroll
+      for (int g = 0; g < NG; ++g) {
+        const u32x4_t x = d[g];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) qh[g][m] = mul_f16x2(qh[g][m], x[m]);
+      }
+    }
+    const u32x4_t all = {~0u, ~0u, ~0u, ~0u};
+    leave_scores(score_tile16<NG>(kc, qh), all, all);
+    lds_barrier();
+    return;
   }
-  f32x4_t* const part = reinterpret_cast<f32x4_t*>(lds + lay.part);  // [wave][half of the channels' pairs][quarter][lane]
+  // ---- 3 ----
+  const bool second = wave == NT;
+  f32x16_t O = {0.f};
 #pragma unroll
-  for (int p = 0; p < 2; ++p)
+  for (int t = 0; t < 2; ++t) {
+    const u32x4_t other = *reinterpret_cast<const u32x4_t*>(unit_ptr(scores, 2 * (second ? qi : NT) + t, lane));
 #pragma unroll
-    for (int g = 0; g < 4; ++g) part[(8 * wave + 4 * p + g) * 64 + lane] = f32x4_t{O[p][4 * g], O[p][4 * g + 1], O[p][4 * g + 2], O[p][4 * g + 3]};
-  lds_barrier();
+    for (int x = 0; x < 4; ++x) p16[t][x] = add_f16x2(p16[t][x], other[x]);
+    O = mfma_f16(second ? vf[t][1] : vf[t][0], p16[t], O);
+  }
+  const auto tile_of = [&](int s) { return s < qi ? qi - 1 - s : s + 1; };  // outwards, forward first
+  const auto load_values = [&](int s, u32x4_t (&x)[2]) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) x[t] = *reinterpret_cast<const u32x4_t*>(unit_ptr(values, 4 * tile_of(s) + 2 * t + second, lane));
+  };
+  const auto load_scores = [&](int s, u32x4_t (&x)[2]) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) x[t] = *reinterpret_cast<const u32x4_t*>(unit_ptr(scores, 2 * tile_of(s) + t, lane));
+  };
+  u32x4_t va[2], pa[2], vb[2], pb[2];
+  load_values(0, va);
+  load_values(1, vb);
+  lds_barrier();  // every tile's scores are visible
+  load_scores(0, pa);
+  const int last = NT - 2;  // (the loads of a step travel during the one before)
+  for (int s = 0; s <= last; s += 2) {
+    load_scores(min(s + 1, last), pb);
+    O = mfma_f16(va[0], pa[0], O);
+    O = mfma_f16(va[1], pa[1], O);
+    if (s == last) break;
+    load_values(min(s + 2, last), va);
+    load_scores(min(s + 2, last), pa);
+    O = mfma_f16(vb[0], pb[0], O);
+    O = mfma_f16(vb[1], pb[1], O);
+    load_values(min(s + 3, last), vb);
+  }
+  f32x4_t* const half = reinterpret_cast<f32x4_t*>(lds);
+  if (second) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) half[64 * g + lane] = f32x4_t{O[4 * g], O[4 * g + 1], O[4 * g + 2], O[4 * g + 3]};
+  }
+  lds_barrier();  // (of the two query waves)
+  if (second) return;
   const rsrc_t out = chunk_rsrc(o + ((size_t)blockIdx.x * geo.L + 32 * qi) * 64, min(32, geo.L - 32 * qi), 128);
-  for (int g = wave; g < 4; g += NT + 1) {
-    f32x4_t a = part[g * 64 + lane], b = part[(4 + g) * 64 + lane];
-    for (int w = 1; w <= NT; ++w) a += part[(8 * w + g) * 64 + lane], b += part[(8 * w + 4 + g) * 64 + lane];
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    const f32x4_t b = half[64 * g + lane];
     u32x4_t x;
 #pragma unroll
-    for (int m = 0; m < 4; ++m) x[m] = pack_bf16x2(a[m] * oscale, b[m] * oscale);
+    for (int m = 0; m < 4; ++m) x[m] = pack_bf16x2(O[4 * g + m] * oscale, b[m] * oscale);
     __builtin_amdgcn_raw_buffer_store_b128(x, out, (unsigned)r * 128u + 64u * h + 16u * g, 0, 0);
   }
 }
@@ -1273,10 +1329,10 @@ bool gla_tiles_supported(const GlaArgs& a) {
 }
 
 // Whether a workgroup for each query tile is the quicker form: while there is a CU for each.  us, a workgroup a sequence / a query tile: Dk 32: 36
-// sequences of 196 (252 tiles) 7.4 / 5.4, 42 (294) 7.5 / 8.1, 96 (672) 7.8 / 11.7; 48 of 160 (240) 6.7 / 5.0, 60 (300) 6.7 / 7.8; Dk 64: 36 of
-// 196 9.7 / 6.7, 42 9.8 / 10.2; 24 of 256 (192) 10.5 / 7.2, 36 (288) 10.5 / 12.4.  From five tiles on, because the op with the locality gate
-// gives the plain op's bits and so takes the same form, with the gate behind it: 3 of 14 x 14, Dk 32 10.4 / 9.2, Dk 64 12.8 / 10.3, 36 of 12 x 13
-// 10.0 / 9.3; but 12 of 10 x 12 7.8 / 8.4, where the plain op alone would gain too (60 of 128 5.5 / 4.8).
+// sequences of 196 (252 tiles) 7.2 / 5.2, 42 (294) 7.3 / 8.0, 96 (672) 7.6 / 11.3; 48 of 160 (240) 6.5 / 4.9, 60 (300) 6.5 / 7.6; Dk 64: 36 of
+// 196 9.6 / 6.7, 42 9.6 / 10.5; 32 of 256 (256) 10.4 / 7.7, 36 (288) 10.4 / 12.8.  From five tiles on, where the op with the locality gate, which
+// takes the same form with the gate behind it, gains too: 3 of 14 x 14, Dk 32 10.4 / 8.8, Dk 64 12.8 / 10.2, 36 of 12 x 13
+// 9.7 / 9.1; but 12 of 10 x 12 7.6 / 8.2, where the plain op alone would gain (60 of 128 5.2 / 4.6).
 static bool spread_preferred(const GlaArgs& a, int NT) {
   return NT >= 5 && NT <= kFewTiles && (long long)a.B * a.H * NT <= 256 && !a.wide_gates;
 }
