@@ -102,6 +102,40 @@ def test_one_sequence_in_a_batch(L, Dk, keys):
     assert torch.equal(batch[0], batch[29]) and torch.equal(one[0], batch[0])
 
 
+@pytest.mark.parametrize("L,Dk,over", [(129, 32, "v"), (196, 32, "v"), (256, 32, "v"), (196, 64, "q"), (197, 64, "k"), (256, 64, "v"), (225, 64, "gf"), (160, 64, "gb")])
+def test_output_over_an_input(L, Dk, over):
+    """A sequence's outputs written over one of its inputs, as a workgroup that has read the sequence may."""
+    announce(f"few sequences, output over {over} L{L} Dk{Dk}")
+    q, k, v, g = _inputs(1, 3, L, Dk, torch.Generator().manual_seed(L + 1))
+    want = vig_amd.gla_bidir_forward(q, k, v, g[0], g[1])
+    names = dict(q=q, k=k, v=v, gf=g[0].clone(), gb=g[1].clone())
+    o = vig_amd.gla_bidir_forward(*names.values(), out=names[over])
+    assert o.data_ptr() == names[over].data_ptr() and torch.equal(o, want)
+
+
+@pytest.mark.parametrize("Dk", [32, 64])
+def test_gated_output_over_the_values(Dk):
+    announce(f"few sequences, gated output over v Dk{Dk}")
+    gen = torch.Generator().manual_seed(Dk)
+    (q, k, v, g), w = _inputs(2, 3, 196, Dk, gen), (torch.randn(192, 9, generator=gen) / 3).cuda()
+    want = vig_amd.gla_bidir_locality_gate(q, k, v, g[0], g[1], w.view(-1, 1, 3, 3), (14, 14))
+    rc = _lib.load().vig_gla_bidir_locgate_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), g[0].data_ptr(), g[1].data_ptr(), w.data_ptr(), v.data_ptr(), 2, 3, 196,
+                                               Dk, 64, 14, 14, Dk ** -0.5, 1.0, 1, 1, torch.cuda.current_stream().cuda_stream)
+    assert rc == _lib.VIG_OK and torch.equal(v, want)
+
+
+def test_output_over_the_rows_of_the_values():
+    """One sequence whose values lie in wider rows, the output inside their span."""
+    announce("one sequence, output over the values' rows")
+    q, k, v, g = _inputs(1, 1, 196, 64, torch.Generator().manual_seed(5))
+    want = vig_amd.gla_bidir_forward(q, k, v, g[0], g[1])
+    rows = torch.cat([v[0, 0], v[0, 0]], 1).contiguous()
+    s, sv = (ctypes.c_longlong * 3)(196 * 64, 196 * 64, 64), (ctypes.c_longlong * 3)(196 * 128, 64, 128)
+    rc = _lib.load().vig_gla_bidir_fwd_strided(q.data_ptr(), k.data_ptr(), rows.data_ptr() + 128, g[0].data_ptr(), g[1].data_ptr(), rows.data_ptr(), 1, 1, 196, 64,
+                                               64, s, s, sv, 0.125, 1.0, 1, 1, torch.cuda.current_stream().cuda_stream)
+    assert rc == _lib.VIG_OK and torch.equal(rows.view(-1)[:196 * 64].view(196, 64), want[0, 0])
+
+
 @pytest.mark.parametrize("B,H,hw,Dk", [(1, 3, (14, 14), 32), (2, 2, (2, 126), 64), (1, 2, (256, 1), 32), (3, 1, (11, 12), 64)])
 def test_locality_gate_behind_it(B, H, hw, Dk):
     announce(f"spread forward with the locality gate B{B} H{H} {hw} Dk{Dk}")

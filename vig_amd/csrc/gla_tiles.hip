@@ -1328,13 +1328,27 @@ bool gla_tiles_supported(const GlaArgs& a) {
   return true;
 }
 
+// Whether the output lies anywhere over q, k, v or what the gates come from.  A workgroup a sequence has read all of it before it stores, so a caller
+// may give a sequence's v (at Dk 64 any input) as its output; workgroups a query tile read each other's rows.
+static bool over_an_input(const GlaArgs& a) {
+  const char *o = (const char*)a.o, *end = o + 2 * (size_t)a.B * a.H * a.L * 64;
+  const auto meets = [&](const void* p, size_t elements) { return p && (const char*)p < end && o < (const char*)p + 2 * elements; };
+  const auto extent = [&](const long long* s, int D) {  // first element to one past the last
+    const size_t n = (size_t)a.B * a.H * a.L * D;
+    return s && s[2] != 0 ? (size_t)((a.B - 1) * s[0] + (a.H - 1) * s[1] + (a.L - 1) * s[2]) + D : n;
+  };
+  const size_t gates = a.low ? 0 : (size_t)a.B * a.H * a.L * a.Dk;
+  return meets(a.q, extent(a.q_strides, a.Dk)) || meets(a.k, extent(a.k_strides, a.Dk)) || meets(a.v, extent(a.v_strides, 64)) ||
+         meets(a.g_fwd, gates) || meets(a.g_bwd, gates) || meets(a.low, a.low ? ((size_t)a.B * a.L - 1) * a.low_ld + 16 : 0);
+}
+
 // Whether a workgroup for each query tile is the quicker form: while there is a CU for each.  us, a workgroup a sequence / a query tile: Dk 32: 36
 // sequences of 196 (252 tiles) 7.2 / 5.2, 42 (294) 7.3 / 8.0, 96 (672) 7.6 / 11.3; 48 of 160 (240) 6.5 / 4.9, 60 (300) 6.5 / 7.6; Dk 64: 36 of
 // 196 9.6 / 6.7, 42 9.6 / 10.5; 32 of 256 (256) 10.4 / 7.7, 36 (288) 10.4 / 12.8.  From five tiles on, where the op with the locality gate, which
 // takes the same form with the gate behind it, gains too: 3 of 14 x 14, Dk 32 10.4 / 8.8, Dk 64 12.8 / 10.2, 36 of 12 x 13
 // 9.7 / 9.1; but 12 of 10 x 12 7.6 / 8.2, where the plain op alone would gain (60 of 128 5.2 / 4.6).
 static bool spread_preferred(const GlaArgs& a, int NT) {
-  return NT >= 5 && NT <= kFewTiles && (long long)a.B * a.H * NT <= 256 && !a.wide_gates;
+  return NT >= 5 && NT <= kFewTiles && (long long)a.B * a.H * NT <= 256 && !a.wide_gates && !over_an_input(a);
 }
 template <int NG, bool PITCHED, bool LOW>
 static int launch_spread(const GlaArgs& a, TileGeo geo, int dev) {
