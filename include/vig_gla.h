@@ -754,12 +754,13 @@ int vig_linear_bwd_weight_many(const void* const* dy, const long long* dy_row_st
 
 /*
  * The layer norms of the patch embedding for training: y [rows, C] = layernorm(x + pre_bias) * weight + bias, through SiLU if silu, x [rows, C]
- * and y bf16 or fp32 (fp32 x: fp32 y), all between them fp32; pre_bias [C] or NULL.  C % 8 == 0, C <= 1024.
+ * and y bf16 or fp32 (fp32 x: fp32 y), all between them fp32; pre_bias [C] or NULL.  C % 8 == 0, C <= 1024, at most VIG_STEM_NORM_ROWS rows.
  * _bwd: dx [rows, C] in x's type (NULL: not wanted) and dparams [3, C]: the gradients of weight, bias and pre_bias; dy in y's type.
  *
  * Replaces: LayerNorm2d and nn.SiLU of V2PatchEmbed (classification/models/vig.py:619-624,651-656), the convolutions' bias adds, and what
  * autograd derives for them.
  */
+#define VIG_STEM_NORM_ROWS (0x7fffffffLL - 16384)
 int vig_stem_norm_fwd(const void* x, const float* pre_bias, const float* weight, const float* bias, void* y, long long rows, int C, float eps,
                       int silu, int x_dtype, int y_dtype, void* stream);
 size_t vig_stem_norm_bwd_workspace(long long rows, int C);

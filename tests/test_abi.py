@@ -111,3 +111,20 @@ def test_token_rows_past_two_to_the_31():
         assert lib.vig_dirgate_bwd(p, p, p, B, L, 1, 8, 1.0, nan, 1, 1, None) not in refused
         assert lib.vig_split_heads_fwd(p, p, p, p, B, L, 1, 8, 8, 0, 1, None) not in refused
     assert lib.vig_dirgate_fwd(p, p, 65535, 70000, 1, 8, 1.0, nan, 1, 1, None) in refused
+
+
+def test_stem_norm_rows_a_walk_can_step_past():
+    """The backward walks rows in steps of up to 16384 (8 to 128 channels) and counts them as ints: rows that a step could carry past 2^31 - 1 are refused."""
+    import torch
+
+    from vig_amd import _lib
+
+    if torch.cuda.is_available() or not os.path.exists(_lib.LIB_PATH):
+        pytest.skip("pointers to nothing: only where no launch can follow")
+    lib, p, last = _lib.load(), 4096, 2 ** 31 - 1 - 512 * (512 // 16)
+    fwd = lambda rows, C: lib.vig_stem_norm_fwd(p, None, p, p, p, rows, C, 1e-5, 1, 1, 1, None)  # noqa: E731
+    bwd = lambda rows, C: lib.vig_stem_norm_bwd(p, None, p, p, p, p, p, p, 2 ** 40, rows, C, 1e-5, 1, 1, 1, None)  # noqa: E731
+    for C in (8, 128, 1024):
+        for rows in (last + 1, 2 ** 31 - 8192, 2 ** 31 - 1, 2 ** 31):
+            assert fwd(rows, C) == bwd(rows, C) == _lib.VIG_ENOTSUP, (rows, C)
+        assert fwd(last, C) not in (_lib.VIG_ENOTSUP, _lib.VIG_EINVAL) and bwd(last, C) not in (_lib.VIG_ENOTSUP, _lib.VIG_EINVAL)  # (no device here)

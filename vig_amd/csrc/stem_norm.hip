@@ -108,6 +108,7 @@ __global__ __launch_bounds__(256) void stem_norm_kernel(const TX* __restrict__ x
 // Workgroups walk the rows a grid apart and keep their shares of the three parameters' gradients in registers; the waves of a workgroup combine
 // through LDS, one parameter after the other, into one row of partials [grid, 3 C], which a column sum finishes (no atomics).
 constexpr int kStemThreads = 512, kStemBlocks = 512;  // two workgroups a CU
+static_assert(kStemBlocks * (kStemThreads / 16) <= 0x7fffffffLL - VIG_STEM_NORM_ROWS, "a walk's step behind the last row is still an int");
 template <typename TX, typename TY, int NV, int GROUP>
 __global__ __launch_bounds__(kStemThreads, NV == 1 ? 4 : 2) void stem_norm_bwd_kernel(const TX* __restrict__ x, const float* __restrict__ pre_bias,
                                                                        const float* __restrict__ weight, const float* __restrict__ bias,
@@ -193,7 +194,7 @@ int stem_grid(long long rows) { return (int)std::min<long long>(kStemBlocks, (ro
 int launch_column_sum(const float* partials, float* out, int n, int C, hipStream_t stream);
 
 bool stem_norm_supported(long long rows, int C, int x_dtype, int y_dtype) {
-  return C % 8 == 0 && C > 0 && C <= 1024 && rows > 0 && rows <= 0x7fffffffLL - 8192 && (x_dtype == 1 || (x_dtype == 0 && y_dtype == 0));
+  return C % 8 == 0 && C > 0 && C <= 1024 && rows > 0 && rows <= VIG_STEM_NORM_ROWS && (x_dtype == 1 || (x_dtype == 0 && y_dtype == 0));
 }
 size_t stem_norm_bwd_workspace(long long rows, int C) { return (size_t)stem_grid(rows) * 3 * C * sizeof(float); }
 

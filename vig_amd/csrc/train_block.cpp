@@ -803,7 +803,7 @@ PyObject* stem_norm(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const bool mixed = at::autocast::is_autocast_enabled(at::kCUDA);
   // the norm under autocast is one in fp32 whatever it reads, and the next convolution casts; without, map and parameters are of one type
   if (x.scalar_type() != (mixed ? at::kBFloat16 : at::kFloat) || (mixed && at::autocast::get_autocast_dtype(at::kCUDA) != at::kBFloat16)) Py_RETURN_NONE;
-  if (C % 8 || C > 1024 || rows > 0x7fffffff - 8192) Py_RETURN_NONE;
+  if (C % 8 || C > 1024 || rows > VIG_STEM_NORM_ROWS) Py_RETURN_NONE;
   return THPVariable_Wrap(StemNormNode::apply(x, pre.defined() ? std::optional<Tensor>(pre) : std::nullopt, weight, bias, eps, silu, mixed && !last));
   END_HANDLE_TH_ERRORS
 }
