@@ -42,6 +42,21 @@ def test_values_and_gradients(B, Cin, Cout, k, H, W):
         assert a.dtype == b.dtype and (a - b).norm() <= 1e-2 * b.norm()  # torch's operator for both (its sums need not have one order)
 
 
+@pytest.mark.parametrize("kw,W", [(9, 40), (9, 264), (3, 24), (16, 40)])
+def test_a_pixel_that_is_not_finite(kw, W):
+    """One in each image, at every column and a third of the rows: it reaches the windows that hold it and no other."""
+    announce(f"stem conv, pixels that are not finite, {kw} columns of {W}")
+    g = torch.Generator().manual_seed(kw)
+    x, w = torch.randn(W, 3, 25, W, generator=g).bfloat16(), (torch.randn(64, 3, 9, kw, generator=g) / 9).bfloat16()
+    at = torch.arange(W)
+    x[at, at % 3, at % 25, at] = torch.tensor([float("inf"), float("-inf"), float("nan")], dtype=torch.bfloat16)[at % 3]
+    want = F.conv2d(x.float(), w.float(), None, 8, 1)
+    got = _amp(_ext.calls().stem_conv, x.cuda(), w.float().cuda().contiguous(memory_format=torch.channels_last), 8).float().cpu()
+    assert 0 < want.isfinite().float().mean() < 1 and torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+    held = want.isfinite()
+    assert torch.equal(got[want.isinf()], want[want.isinf()]) and ((got - want)[held].abs() <= 2.0 ** -8 * want[held].abs() + 1e-5).all()
+
+
 def test_stays_with_torch():
     announce("stem conv: calls that stay with torch")
     take = _ext.calls().stem_conv

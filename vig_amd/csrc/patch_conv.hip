@@ -4,8 +4,11 @@
 //
 // One workgroup produces up to 32 pixels of one output row (b, oy), all Cout channels.  Its input is the slab of
 // Cin * KH image rows (27 for 3 channels x 9 kernel rows), 256 columns of them; each goes to LDS shifted by one element, so
-// that input column ix of the piece sits at element ix + 1 and element 0 is the column in front (the left padding): pixel ox then finds its 16 kernel columns
-// (9 real ones, the weights of the others are zero) at elements 8*ox .. 8*ox+15, two aligned 16-byte reads.  The
+// that input column ix of the piece sits at element ix + 1 and element 0 is the column in front (the left padding): pixel ox then finds its first eight kernel
+// columns at elements 8*ox .. 8*ox+7, and the rest of 16 (9 real ones, the weights of the others are zero) in a second copy of the row, eight elements on: two aligned
+// 16-byte reads.  Either copy has zeros for the columns that the kernel does not have, as the weights do: they belong to the next window, and a pixel that is not
+// finite stays out of a window it is not in.  us, one row without zeros / this / masks at the reads, 256 images of 224 px: 96 channels 37.3 / 38.2 / 39.3, with the norm
+// 54.6 / 57.9 / 58.1; 192 57.9 / 59.5 / 58.5, 94.7 / 97.5 / 102.9; 384 81.1 / 82.3 / 89.5.  The
 // contraction runs over (channel, kernel row) steps of 16 kernel columns: one v_mfma_f32_32x32x16_bf16 per step with
 // the weights (matrix rows = output channels) in registers for the life of the workgroup and the pixels as columns.
 // Matrix rows are assigned channels so that a lane ends with 16 consecutive channels of one pixel (32 contiguous
@@ -21,7 +24,7 @@ namespace vig {
 namespace {
 
 constexpr int kPcStride = 8;       // convolution stride = elements per pixel step in a staged row
-constexpr int kPcRowElems = 272;   // staged row: 32 chunks of 8 elements written per step, 16 more that stay zero
+constexpr int kPcRowElems = 512;   // staged row: 32 chunks of 8 elements, and the 32 behind each
 constexpr int kPcKW = 16;          // kernel columns per contraction step (weights beyond the real width are zero)
 
 // The layer norm behind it (NORM), as layernorm_kernel gives it for the stored rows, bit for bit: + pre_bias (rounded), norm, SiLU.
@@ -53,12 +56,12 @@ __device__ __forceinline__ float octet_tree(const float* row) {
 
 // NORM: the workgroup has whole rows of channels, so their norm needs two exchanges of octet sums through LDS (a barrier each, one of
 // which takes the place of the one in front of the next staging) instead of a pass over memory.  us, two kernels / this: 96 channels, one image of
-// 224 px 8.5 / 6.7, 8 9.6 / 6.9, 256 74 / 54, 8 of 1024 px 50 / 35; 192, 1 9.4 / 7.9, 32 25 / 19, 64 34 / 29, 256 96 / 94 (one workgroup to a CU: its 191
+// 224 px 8.5 / 6.7, 8 9.6 / 6.9, 256 75 / 58, 8 of 1024 px 50 / 36; 192, 1 9.4 / 7.8, 32 25 / 19, 64 34 / 30, 256 98 / 97 (one workgroup to a CU: its 191
 // registers brought down to 168 for a second one spill 13 to 18, 124).  At 384 channels the 48 octets spill (60 images 55 / 73): two kernels.
 template <int KS, int NW, bool NORM>  // KS = Cin * KH contraction steps, NW = Cout / 32 waves
 __global__ __launch_bounds__(NW > 8 ? 64 * NW : 512) void patch_conv_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ wp,
-                                                         uint16_t* __restrict__ y, int Cin, int H, int W, int KH, int OH,
-                                                         int OW, int Cout, int pieces, int nitems, PcNorm norm) {
+                                                         uint16_t* __restrict__ y, int Cin, int H, int W, int KH, int KW,
+                                                         int OH, int OW, int Cout, int pieces, int nitems, PcNorm norm) {
   constexpr int kPitch = 4 * NW + 4;  // floats between two pixels' octet sums
   extern __shared__ __align__(16) char smem[];
   uint16_t* slab = reinterpret_cast<uint16_t*>(smem);  // [KS][kPcRowElems]
@@ -71,9 +74,6 @@ __global__ __launch_bounds__(NW > 8 ? 64 * NW : 512) void patch_conv_kernel(cons
     for (int i = threadIdx.x; i < 32 * NW; i += blockDim.x)
       params[i] = norm.weight[i], params[32 * NW + i] = norm.bias[i], params[64 * NW + i] = norm.pre_bias ? norm.pre_bias[i] : 0.f;
   }
-  // the columns no step writes (and, until the first step, everything) read as zero
-  for (int i = threadIdx.x; i < KS * kPcRowElems / 8; i += blockDim.x)
-    reinterpret_cast<u32x4_t*>(slab)[i] = u32x4_t{0u, 0u, 0u, 0u};
   // this wave's 32 output channels: matrix row i holds channel 16*((i>>2)&1) + 4*(i>>3) + (i&3) of the tile, which
   // leaves lane (r, h) with channels 16h .. 16h+15 of pixel r in its accumulator registers
   const int chan_of_row = 16 * ((r >> 2) & 1) + 4 * (r >> 3) + (r & 3);
@@ -81,7 +81,14 @@ __global__ __launch_bounds__(NW > 8 ? 64 * NW : 512) void patch_conv_kernel(cons
 #pragma unroll
   for (int t = 0; t < KS; ++t)
     wf[t] = *reinterpret_cast<const u32x4_t*>(wp + ((size_t)(32 * wave + chan_of_row) * KS + t) * kPcKW + 8 * h);
-  __syncthreads();
+  // the kernel's columns among the first eight and the second
+  u32x4_t first, second;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int n0 = KW - 2 * j, n1 = n0 - 8;
+    first[j] = n0 >= 2 ? ~0u : n0 == 1 ? 0xFFFFu : 0u;
+    second[j] = n1 >= 2 ? ~0u : n1 == 1 ? 0xFFFFu : 0u;
+  }
   // image rows of the slab a thread fetches: half-wave (wave, h) takes slab rows 2*p + h, p = wave, wave + nwaves, ..;
   // the chunks of the next output row are in flight while the current one is multiplied
   constexpr int kMaxP = ((KS + 1) / 2 + NW - 1) / NW;  // row pairs per wave
@@ -110,7 +117,8 @@ __global__ __launch_bounds__(NW > 8 ? 64 * NW : 512) void patch_conv_kernel(cons
 #pragma unroll
     for (int i = 0; i < kMaxP; ++i) {
       const int t = 2 * (wave + i * nwaves) + h;
-      uint32_t prev = __shfl_up(v[i][3], 1, 32);  // the left neighbour's last pair; chunk 0 has the column in front there
+      uint32_t prev = __shfl(v[i][3], (r + 31) & 31, 32);  // the left neighbour's last pair; chunk 0 has the column in front there
+      const uint32_t last = prev >> 16;                    // (chunk 0: the last chunk's)
       if (r == 0) prev = front[i];
       u32x4_t o;
       o[0] = __builtin_amdgcn_alignbit(v[i][0], prev, 16);
@@ -118,8 +126,10 @@ __global__ __launch_bounds__(NW > 8 ? 64 * NW : 512) void patch_conv_kernel(cons
       o[2] = __builtin_amdgcn_alignbit(v[i][2], v[i][1], 16);
       o[3] = __builtin_amdgcn_alignbit(v[i][3], v[i][2], 16);
       if (t < KS) {
-        *reinterpret_cast<u32x4_t*>(slab + t * kPcRowElems + r * 8) = o;
-        if (r == 31) slab[t * kPcRowElems + 256] = (uint16_t)(v[i][3] >> 16);  // the last pixel's ninth column
+        *reinterpret_cast<u32x4_t*>(slab + t * kPcRowElems + r * 8) = o & first;
+        // chunk r is what follows chunk r - 1; behind the last one there is its pixel's ninth column
+        if (r == 0) o = u32x4_t{last, 0u, 0u, 0u};
+        *reinterpret_cast<u32x4_t*>(slab + t * kPcRowElems + 256 + 8 * ((r + 31) & 31)) = o & second;
       }
     }
     __syncthreads();
@@ -130,7 +140,7 @@ __global__ __launch_bounds__(NW > 8 ? 64 * NW : 512) void patch_conv_kernel(cons
     for (int j = 0; j < 16; ++j) acc[j] = 0.f;
 #pragma unroll
     for (int t = 0; t < KS; ++t) {
-      const u32x4_t px = *reinterpret_cast<const u32x4_t*>(slab + t * kPcRowElems + r * kPcStride + 8 * h);
+      const u32x4_t px = *reinterpret_cast<const u32x4_t*>(slab + t * kPcRowElems + r * kPcStride + 256 * h);
       acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, wf[t]),
                                                     __builtin_bit_cast(bf16x8_t, px), acc, 0, 0, 0);
     }
@@ -217,7 +227,7 @@ static int launch(const void* x, const void* w_packed, void* y, int B, int Cin, 
 #define VIG_PC_CASE(NW)                                                                                            \
   case NW:                                                                                                         \
     hipLaunchKernelGGL((norm ? patch_conv_kernel<27, NW, (NW <= 8)> : patch_conv_kernel<27, NW, false>), dim3(grid), dim3(64 * NW), lds, stream, \
-                       (const uint16_t*)x, (const uint16_t*)w_packed, (uint16_t*)y, Cin, H, W, KH, OH, OW, Cout, pieces, nitems,          \
+                       (const uint16_t*)x, (const uint16_t*)w_packed, (uint16_t*)y, Cin, H, W, KH, KW, OH, OW, Cout, pieces, nitems,          \
                        norm ? *norm : PcNorm{});                                                                                        \
     break
   switch (Cout / 32) {

@@ -742,9 +742,8 @@ PyObject* block_mlp(PyObject*, PyObject* const* a, Py_ssize_t n) {
 
 // stem_conv(x, weight, stride) -> the convolution with padding 1 and without a bias, under bf16 autocast, or None for a call the node does not take: the
 // kernels' shapes (the first convolution of images three channels deep, 9 x 9 at stride 8; 3 x 3 at stride 2), as in evaluation.
-// us, 128 images of 224 px, the convolution library's (the first with the layout change in front of it) / here: 192 channels 93 / 40, 384 98 / 55; a training
-// pass of ViG-S under autocast 10.37 -> 10.25 ms.  (As in evaluation, a pixel that is not finite also reaches the window that ends in front of it: the zeros that fill
-// a kernel row up to 16 columns multiply it.)
+// us, 128 images of 224 px, the convolution library's (the first with the layout change in front of it) / here: 192 channels 93 / 41, 384 98 / 55; a training
+// pass of ViG-S under autocast 10.37 -> 10.25 ms.
 PyObject* stem_conv(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   TORCH_CHECK_TYPE(n == 3, "stem_conv takes 3 arguments");
