@@ -8,7 +8,7 @@
 // columns at elements 8*ox .. 8*ox+7, and the rest of 16 (9 real ones, the weights of the others are zero) in a second copy of the row, eight elements on: two aligned
 // 16-byte reads.  Either copy has zeros for the columns that the kernel does not have, as the weights do: they belong to the next window, and a pixel that is not
 // finite stays out of a window it is not in.  us, one row without zeros / this / masks at the reads, 256 images of 224 px: 96 channels 37.3 / 38.2 / 39.3, with the norm
-// 54.6 / 57.9 / 58.1; 192 57.9 / 59.5 / 58.5, 94.7 / 97.5 / 102.9; 384 81.1 / 82.3 / 89.5.  The
+// 54.6 / 57.9 / 58.1 (55.0 with its sums' present pitch); 192 57.9 / 59.5 / 58.5, 94.7 / 97.5 / 102.9; 384 81.1 / 82.3 / 89.5.  The
 // contraction runs over (channel, kernel row) steps of 16 kernel columns: one v_mfma_f32_32x32x16_bf16 per step with
 // the weights (matrix rows = output channels) in registers for the life of the workgroup and the pixels as columns.
 // Matrix rows are assigned channels so that a lane ends with 16 consecutive channels of one pixel (32 contiguous
@@ -56,13 +56,16 @@ __device__ __forceinline__ float octet_tree(const float* row) {
 
 // NORM: the workgroup has whole rows of channels, so their norm needs two exchanges of octet sums through LDS (a barrier each, one of
 // which takes the place of the one in front of the next staging) instead of a pass over memory.  us, two kernels / this: 96 channels, one image of
-// 224 px 8.5 / 6.7, 8 9.6 / 6.9, 256 75 / 58, 8 of 1024 px 50 / 36; 192, 1 9.4 / 7.8, 32 25 / 19, 64 34 / 30, 256 98 / 97 (one workgroup to a CU: its 191
+// 224 px 8.5 / 6.7, 8 9.5 / 6.9, 256 76 / 55, 8 of 1024 px 50 / 35; 192, 1 9.4 / 7.7, 32 24 / 19, 256 100 / 97, 224, 256 103 / 95, 256, 256 110 / 95 (one workgroup to a CU: its 191
 // registers brought down to 168 for a second one spill 13 to 18, 124).  At 384 channels the 48 octets spill (60 images 55 / 73): two kernels.
 template <int KS, int NW, bool NORM>  // KS = Cin * KH contraction steps, NW = Cout / 32 waves
 __global__ __launch_bounds__(NW > 8 ? 64 * NW : 512) void patch_conv_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ wp,
                                                          uint16_t* __restrict__ y, int Cin, int H, int W, int KH, int KW,
                                                          int OH, int OW, int Cout, int pieces, int nitems, PcNorm norm) {
-  constexpr int kPitch = 4 * NW + 4;  // floats between two pixels' octet sums
+  // floats between two pixels' octet sums: an odd number of fours, so that 16 pixels meet every bank once (seven waves, 32 floats, all pixels in the same four
+  // banks: 224 channels, 256 images of 224 px, 133 us for 95)
+  constexpr int kPitch = 4 * (NW | 1);
+  static_assert(kPitch >= 4 * NW && kPitch % 8 == 4, "pixels spread over the banks");
   extern __shared__ __align__(16) char smem[];
   uint16_t* slab = reinterpret_cast<uint16_t*>(smem);  // [KS][kPcRowElems]
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -223,7 +226,7 @@ static int launch(const void* x, const void* w_packed, void* y, int B, int Cin, 
   // behind the first and fetches the weights again; us, two to a CU / one: 192 channels, 16 images of 224 px 12.4 / 9.1, 32 16.5 / 13.5, 256 61 / 57.5, with the
   // norm 97.7 / 94.2; 256 channels, 20 15.4 / 11.7; 384, 16 18.9 / 13.4, 128 50.8 / 42.5.)
   const int most = Cout > 128 ? 256 : 512, grid = nitems < most ? nitems : most;
-  const size_t lds = (size_t)27 * kPcRowElems * sizeof(uint16_t) + (norm ? 4 * (2 * 32 * (Cout / 8 + 4) + 3 * Cout) : 0);
+  const size_t lds = (size_t)27 * kPcRowElems * sizeof(uint16_t) + (norm ? 4 * (2 * 32 * 4 * (Cout / 32 | 1) + 3 * Cout) : 0);
 #define VIG_PC_CASE(NW)                                                                                            \
   case NW:                                                                                                         \
     hipLaunchKernelGGL((norm ? patch_conv_kernel<27, NW, (NW <= 8)> : patch_conv_kernel<27, NW, false>), dim3(grid), dim3(64 * NW), lds, stream, \
