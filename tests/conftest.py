@@ -17,3 +17,18 @@ def rng():
     import numpy as np
 
     return np.random.default_rng(1234)
+
+
+@pytest.fixture(autouse=True)
+def _repeatable_library(request):
+    """One test asks two runs of torch's own convolutions for the same bits; their library adds a weight gradient up in any order
+    unless it is told to repeat itself (proj.0.weight of 2 x 3 x 64 x 48: 61 of 300 pairs of runs differ, none with this)."""
+    if (request.module.__name__.rpartition(".")[2], request.node.name) != ("test_stem_norm_gpu", "test_stays_with_the_modules"):
+        yield
+        return
+    import torch
+
+    before = torch.backends.cudnn.deterministic
+    torch.backends.cudnn.deterministic = True
+    yield
+    torch.backends.cudnn.deterministic = before
