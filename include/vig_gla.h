@@ -663,7 +663,7 @@ int vig_norm_dwconv3x3_fwd(const void* x, const void* residual, const float* nor
 /*
  * The same with a row product behind the convolution: sum as above (may be NULL), conv [B, h*w, C] the convolution's result,
  * y [B, h*w, N] = conv . weight [N, C]^T (+ bias [N] bf16, or NULL), as vig_norm_dwconv3x3_fwd and vig_linear_fwd give one after the other.
- * C = 192 or 384, N % 64 == 0 and few images (vig_norm_dwconv3x3_linear_preferred), else VIG_ENOTSUP.  No output may be an input.
+ * C = 192 or 384, N % 128 == 0 and few images (vig_norm_dwconv3x3_linear_preferred), else VIG_ENOTSUP.  No output may be an input.
  *
  * Replaces: classification/models/vig.py:291-294,364-369,598-606 (attn_norm, local convolution, projections).
  */

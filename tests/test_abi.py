@@ -128,3 +128,17 @@ def test_stem_norm_rows_a_walk_can_step_past():
         for rows in (last + 1, 2 ** 31 - 8192, 2 ** 31 - 1, 2 ** 31):
             assert fwd(rows, C) == bwd(rows, C) == _lib.VIG_ENOTSUP, (rows, C)
         assert fwd(last, C) not in (_lib.VIG_ENOTSUP, _lib.VIG_EINVAL) and bwd(last, C) not in (_lib.VIG_ENOTSUP, _lib.VIG_EINVAL)  # (no device here)
+
+
+def test_columns_of_the_norm_convolution_and_product():
+    """Its column tiles are 128 wide: the widths it takes, and the ones the header names."""
+    from vig_amd import _lib
+
+    if not os.path.exists(_lib.LIB_PATH):
+        pytest.skip("library not built")
+    takes, p = _lib.load().vig_norm_dwconv3x3_linear_preferred, 4096
+    for C in (192, 384):
+        assert [N for N in range(8, 641, 8) if takes(1, 4, 8, C, N)] == list(range(128, 641, 128))
+        assert _lib.load().vig_norm_dwconv3x3_linear_fwd(p, None, p, p, None, p, None, None, 2 * p, 3 * p, 1, 4, 8, C, 192, 1e-6, 1, None) == _lib.VIG_ENOTSUP
+    text = " ".join(open(os.path.join(ROOT, "include", "vig_gla.h")).read().split())
+    assert re.search(r"N % (\d+) == 0 and few images \(vig_norm_dwconv3x3_linear_preferred\)", text).group(1) == "128"
