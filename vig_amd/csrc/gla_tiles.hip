@@ -66,7 +66,6 @@ struct TileGeo {
   const uint16_t *low, *up_w, *up_b;
   long long low_ld;
   float inv_norm, clamp;
-  int spread;               // nonzero: grid (sequence, query tile), gla_spread_kernel
 };
 
 // Sequences of more tiles than this (MANY below): a far tile's q^ has picked up the decays of up to fifteen tiles, and a product
@@ -121,7 +120,6 @@ struct TileCtx {
   const uint16_t *up_w[2], *up_b[2];
   int nvalid;  // tokens of the tile
   float inv_norm, clamp;
-  bool silent;  // another workgroup stores this tile's outputs
 };
 
 // What a wave fetches to make its tile's gates: its tokens' rank-16 rows and, per direction, the weights and the bias of a lane's
@@ -666,14 +664,16 @@ static_assert(offsetof(TileKernArgs, geo) == 6 * sizeof(void*) && offsetof(TileK
                   offsetof(TileKernArgs, gate_w) == 48 + sizeof(TileGeo) + 8 && alignof(TileGeo) == 8,
               "TileKernArgs has to mirror the parameter list of gla_tile_kernel");
 
-template <int NG, bool BIDIR, bool PITCHED, bool GATE, bool CHAIN, bool LOW, bool MANY>
+template <int NG, bool BIDIR, bool PITCHED, bool GATE, bool CHAIN, bool LOW, bool MANY, bool SPREAD = false>
 __device__ void tile_pass_general(const TileKernArgs* ka_in);
 
 // Everything one wave does for its slab.  When some tile of the slab is outside the fp16 form's range (GENERAL false), every wave
 // of the workgroup, before anything is stored, runs the general form (ka: the kernel's argument block) and ends there: a call
 // that came back would keep the accumulators alive across it, and the compiler then kept sixteen of them in per-lane memory
 // throughout, walks included (long sequences at Dk 32, 144 of 784 tokens: this kernel 38.7 -> 23.5 us).
-template <int NG, bool BIDIR, bool PITCHED, bool GENERAL, bool GATE, bool CHAIN, bool LOW, bool MANY>
+// SPREAD: the general form of gla_spread_kernel, whose workgroups store one tile each.  (A template's argument, not a field of the geometry, which
+// would move the registers of every kernel: nine to thirteen tiles at Dk 64 reloaded seven more, 33 sequences of 275 tokens 14.6 -> 16.7 us.)
+template <int NG, bool BIDIR, bool PITCHED, bool GENERAL, bool GATE, bool CHAIN, bool LOW, bool MANY, bool SPREAD = false>
 __device__ __forceinline__ void tile_pass(const TileCtx& cx, const TileKernArgs* ka) {
   const int lane = cx.lane, r = lane & 31, h = lane >> 5;
   const int ti = cx.ti, NT = cx.NT;
@@ -853,7 +853,7 @@ __device__ __forceinline__ void tile_pass(const TileCtx& cx, const TileKernArgs*
                            GENERAL ? -(ek + ev) : 0, qhb, O);
   float os = cx.oscale;
   if (GENERAL) os *= __builtin_amdgcn_exp2f((float)(eq + ek + ev));
-  if (GENERAL && cx.silent) return;
+  if (SPREAD && ti != (int)blockIdx.y) return;
   if (GATE) {
     locality_gate_epilogue(O[0], O[1], os, lds, cx.gate_w, cx.o, cx.gw, cx.gh, ti, NT, lane_w);
     return;
@@ -881,7 +881,6 @@ __device__ __forceinline__ TileCtx make_tile_ctx(const uint16_t* q, const uint16
   // (slab = batch element * heads + head)
   cx.gate_w = GATE ? gate_w + (size_t)((int)blockIdx.x % geo.heads) * (64 * 9) : nullptr;
   cx.ti = ti;
-  cx.silent = !CHAIN && geo.spread && ti != (int)blockIdx.y;
   cx.lane = threadIdx.x & 63;
   cx.NT = geo.NT;
   cx.oscale = oscale;
@@ -930,7 +929,7 @@ __device__ __forceinline__ TileCtx make_tile_ctx(const uint16_t* q, const uint16
 // the kernel's arguments from the argument block itself (ka: the kernel's own kernarg segment pointer; the builtin
 // yields null inside a called function): handed over as parameters, the geometry would need a copy in per-lane
 // memory, and the compiler writes that copy at the top of the kernel, for every wave, redo or not.
-template <int NG, bool BIDIR, bool PITCHED, bool GATE, bool CHAIN, bool LOW, bool MANY>
+template <int NG, bool BIDIR, bool PITCHED, bool GATE, bool CHAIN, bool LOW, bool MANY, bool SPREAD>
 __device__ __noinline__ void tile_pass_general(const TileKernArgs* ka_in) {
 #if defined(__HIP_DEVICE_COMPILE__)  // (the host pass has no constant address space to copy the geometry from)
   // (a called function gets its arguments in vector registers: back to scalars, or every argument read through the
@@ -945,7 +944,7 @@ __device__ __noinline__ void tile_pass_general(const TileKernArgs* ka_in) {
   const TileGeo geo = ka->geo;
   const TileCtx cx = make_tile_ctx<NG, BIDIR, PITCHED, GATE, CHAIN, LOW>(ka->q, ka->k, ka->v, ka->gf, ka->gb, ka->o, geo,
                                                                      ka->oscale, ka->gate_w, lds, own_tile());
-  tile_pass<NG, BIDIR, PITCHED, true, GATE, CHAIN, LOW, MANY>(cx, nullptr);
+  tile_pass<NG, BIDIR, PITCHED, true, GATE, CHAIN, LOW, MANY, SPREAD>(cx, nullptr);
 #endif
 }
 
@@ -1175,7 +1174,7 @@ __global__ __launch_bounds__(576, 3) void gla_spread_kernel(const uint16_t* __re
   {
     const float mine = lane <= NT ? guard[lane] : 0.0f;
     if (__builtin_amdgcn_ballot_w64(mine != 0.0f) != 0) {
-      if (wave < NT) tile_pass_general<NG, true, PITCHED, false, false, LOW, false>(ka);
+      if (wave < NT) tile_pass_general<NG, true, PITCHED, false, false, LOW, false, true>(ka);
       __builtin_amdgcn_endpgm();
     }
   }
@@ -1359,7 +1358,6 @@ static int launch_spread(const GlaArgs& a, TileGeo geo, int dev) {
     if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, SpreadLds<NG>(kFewTiles).total) != hipSuccess) return -5;
     done[dev] = true;
   }
-  geo.spread = 1;
   hipLaunchKernelGGL(kernel, dim3(a.B * a.H, geo.NT), dim3(64 * (geo.NT + 1)), lay.total, a.stream, (const uint16_t*)a.q, (const uint16_t*)a.k,
                      (const uint16_t*)a.v, (const uint16_t*)a.g_fwd, (const uint16_t*)a.g_bwd, (uint16_t*)a.o, geo, a.scale * a.out_scale, a.gate_w);
   return hipGetLastError() == hipSuccess ? 0 : -5;
