@@ -56,7 +56,7 @@ __device__ __forceinline__ float octet_tree(const float* row) {
 
 // NORM: the workgroup has whole rows of channels, so their norm needs two exchanges of octet sums through LDS (a barrier each, one of
 // which takes the place of the one in front of the next staging) instead of a pass over memory.  us, two kernels / this: 96 channels, one image of
-// 224 px 8.5 / 6.7, 8 9.5 / 6.9, 256 76 / 55, 8 of 1024 px 50 / 35; 192, 1 9.4 / 7.7, 32 24 / 19, 256 100 / 97, 224, 256 103 / 95, 256, 256 110 / 95 (one workgroup to a CU: its 191
+// 224 px 8.5 / 6.7, 8 9.5 / 6.9, 256 76 / 55, 8 of 1024 px 50 / 35; 192, 1 9.4 / 7.7, 32 24 / 19, 256 100 / 97, 224, 256 103 / 95, 256, 256 110 / 95 (one workgroup to a CU: its 190
 // registers brought down to 168 for a second one spill 13 to 18, 124).  At 384 channels the 48 octets spill (60 images 55 / 73): two kernels.
 template <int KS, int NW, bool NORM>  // KS = Cin * KH contraction steps, NW = Cout / 32 waves
 __global__ __launch_bounds__(NW > 8 ? 64 * NW : 512) void patch_conv_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ wp,
@@ -222,9 +222,10 @@ static int launch(const void* x, const void* w_packed, void* y, int B, int Cin, 
   const int pieces = (OW + 31) / 32;
   if (OH < 1 || (long long)B * OH * pieces > 0x7fffffffLL - 4096 || Cout / 32 < 2) return -95;
   const int nitems = B * OH * pieces;
-  // As many workgroups as the chip holds, two to a CU of up to four waves and one of more; each walks pieces grid apart.  (A second one of more waves runs
-  // behind the first and fetches the weights again; us, two to a CU / one: 192 channels, 16 images of 224 px 12.4 / 9.1, 32 16.5 / 13.5, 256 61 / 57.5, with the
-  // norm 97.7 / 94.2; 256 channels, 20 15.4 / 11.7; 384, 16 18.9 / 13.4, 128 50.8 / 42.5.)
+  // Two workgroups to a CU of up to four waves, one of more; each walks pieces grid apart.  Of more waves one has enough under way, and a second one a CU, whether it
+  // fits beside the first (up to 192 channels without the norm: 168 registers) or not, only fetches the weights again, 3 us a launch at any size: us, two to a CU / one, 16
+  // and 256 images of 224 px: 160 channels 11.4 / 8.6, 61.4 / 58.4, with the norm 14.3 / 11.4, 98.8 / 95.5; 192 12.1 / 8.9, 62.4 / 59.0, 15.1 / 11.6, 100.6 / 97.0; 224 12.2 /
+  // 8.9, 62.4 / 58.5; 256 13.1 / 9.5, 65.6 / 62.2, 16.4 / 12.3, 99.5 / 94.9; 384, 16 18.9 / 13.4, 128 50.8 / 42.5.
   const int most = Cout > 128 ? 256 : 512, grid = nitems < most ? nitems : most;
   const size_t lds = (size_t)27 * kPcRowElems * sizeof(uint16_t) + (norm ? 4 * (2 * 32 * 4 * (Cout / 32 | 1) + 3 * Cout) : 0);
 #define VIG_PC_CASE(NW)                                                                                            \
