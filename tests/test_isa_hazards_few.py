@@ -27,3 +27,10 @@ def test_many_tiles_send_no_more_through_memory():
     name, = re.findall(r"^(_ZN3vig15gla_tile_kernelILi4ELb1ELb0ELb0ELb0ELb0ELb1E\w*):", asm, re.M)
     body = re.search(rf"^{name}:.*?^\.Lfunc_end", asm, re.S | re.M).group(0)
     assert body.count("scratch_load") <= 20 and body.count("scratch_store") <= 20
+
+
+def test_recurrent_backward_of_16_channels_leaves_room_for_six_waves():
+    # 512 registers a SIMD, whole eights a wave (with 96: 3072 sequences of 98 tokens 411 -> 456 us)
+    asm = _assembly("gla_backward.hip")
+    counts = re.findall(r"\.name:\s+_ZN3vig19gla_backward_kernelI\w\wLi16E.*?\.vgpr_count:\s+(\d+)", asm, re.S)
+    assert len(counts) == 4 and all(int(n) <= 80 for n in counts), counts
