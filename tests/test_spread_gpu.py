@@ -88,9 +88,19 @@ def test_gates_made_inside(B, H, L):
     assert torch.equal(o.float(), _run(lib.vig_gla_bidir_fwd, q, k, v, g))  # the same operands, one form
 
 
+def test_one_sequence_in_a_batch():
+    """A sequence's outputs as a workgroup a query tile gives them and as a workgroup a sequence does."""
+    q, k, v, g = _inputs(1, 2, 196, 64, torch.Generator().manual_seed(9))
+    one = vig_amd.batch_bid_fused_chunk_gla(q, k, v, g.flatten(0, 1))[0].float()
+    many = [t.repeat(30, 1, 1, 1) for t in (q, k, v)]
+    batch = vig_amd.batch_bid_fused_chunk_gla(*many, g.repeat_interleave(30, 1).flatten(0, 1))[0].float()
+    assert torch.equal(batch[0], batch[29])
+    _close(one[0], batch[0])
+
+
 @pytest.mark.parametrize("L,Dk,keys", [(129, 32, 1.0), (160, 64, 1.0), (196, 32, 1.0), (197, 64, 1.0), (225, 32, 1.0), (256, 64, 1.0), (256, 32, 30.0), (196, 32, 1e-3),
                                        (196, 32, 1e-4), (256, 64, 3e-4)])
-def test_one_sequence_in_a_batch(L, Dk, keys):
+def test_one_sequence_among_sixty(L, Dk, keys):
     """A sequence's outputs as a workgroup a query tile gives them and as a workgroup a sequence does: the same bits, keys in fp16's subnormals
     once decayed among them."""
     announce(f"spread forward, one sequence and sixty L{L} Dk{Dk} keys x {keys}")
